@@ -157,43 +157,87 @@ __global__ __launch_bounds__(256) void moe_identity_kernel(float* __restrict__ x
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int PLAN_MAX_EXPERTS = 512;
-constexpr int PREFETCH_SETS = 3;   // sets of operand registers in flight in the grouped products
+constexpr int PLAN_BATCH = 8;      // choices a thread of the plan has in flight
+constexpr int PREFETCH_SETS = 3;   // sets of operand registers in flight in the kernels of few rows
+
+__device__ __forceinline__ uint2 pack4(const f32x4& a) {
+  return make_uint2(static_cast<uint32_t>(f32_to_bf16(a[0])) | (static_cast<uint32_t>(f32_to_bf16(a[1])) << 16),
+                    static_cast<uint32_t>(f32_to_bf16(a[2])) | (static_cast<uint32_t>(f32_to_bf16(a[3])) << 16));
+}
 
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ sel, int pairs, int E,
                                                         int* __restrict__ where, int* __restrict__ order,
                                                         int* __restrict__ tiles, int* __restrict__ num_tiles,
                                                         int max_tiles, int tile_rows) {
-  __shared__ int cnt[PLAN_MAX_EXPERTS], off[PLAN_MAX_EXPERTS];
+  __shared__ int cnt[PLAN_MAX_EXPERTS], off[PLAN_MAX_EXPERTS], first_tile[PLAN_MAX_EXPERTS];
   const int tid = threadIdx.x;
-  for (int e = tid; e < E; e += blockDim.x) cnt[e] = 0;
+  for (int e = tid; e < PLAN_MAX_EXPERTS; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
-  for (int p = tid; p < pairs; p += blockDim.x) {
-    const int e = sel[p];
-    where[p] = (e >= 0 && e < E) ? atomicAdd(&cnt[e], 1) : -1;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int o = 0, nt = 0;
-    for (int e = 0; e < E; ++e) {
-      off[e] = o;
-      const int c = cnt[e];
-      for (int r0 = 0; r0 < c && nt < max_tiles; r0 += tile_rows) {
-        tiles[3 * nt] = e;
-        tiles[3 * nt + 1] = o + r0;
-        tiles[3 * nt + 2] = min(tile_rows, c - r0);
-        ++nt;
-      }
-      o += c;
+  // a thread's choices are asked for together: one trip to memory for PLAN_BATCH of them
+  for (int p0 = tid; p0 < pairs; p0 += PLAN_BATCH * blockDim.x) {
+    int e[PLAN_BATCH];
+#pragma unroll
+    for (int i = 0; i < PLAN_BATCH; ++i) e[i] = sel[min(p0 + i * static_cast<int>(blockDim.x), pairs - 1)];
+#pragma unroll
+    for (int i = 0; i < PLAN_BATCH; ++i) {
+      const int p = p0 + i * blockDim.x;
+      if (p < pairs) where[p] = (e[i] >= 0 && e[i] < E) ? atomicAdd(&cnt[e[i]], 1) : -1;
     }
-    *num_tiles = nt;
   }
   __syncthreads();
-  for (int p = tid; p < pairs; p += blockDim.x) {
-    const int e = sel[p];
-    if (e >= 0 && e < E) {
-      const int pos = off[e] + where[p];
-      where[p] = pos;
-      order[pos] = p;
+  if (tid < KVF_WAVE) {   // where every expert's rows and tiles begin: sums over the lanes before
+    constexpr int PER = PLAN_MAX_EXPERTS / KVF_WAVE;
+    int rows = 0, nt = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      rows += cnt[PER * tid + i];
+      nt += (cnt[PER * tid + i] + tile_rows - 1) / tile_rows;
+    }
+    int rows_upto = rows, nt_upto = nt;
+#pragma unroll
+    for (int o = 1; o < KVF_WAVE; o *= 2) {
+      const int r = __shfl_up(rows_upto, o, KVF_WAVE), t = __shfl_up(nt_upto, o, KVF_WAVE);
+      if (tid >= o) {
+        rows_upto += r;
+        nt_upto += t;
+      }
+    }
+    if (tid == KVF_WAVE - 1) *num_tiles = min(nt_upto, max_tiles);
+    rows_upto -= rows;
+    nt_upto -= nt;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      off[PER * tid + i] = rows_upto;
+      first_tile[PER * tid + i] = nt_upto;
+      rows_upto += cnt[PER * tid + i];
+      nt_upto += (cnt[PER * tid + i] + tile_rows - 1) / tile_rows;
+    }
+  }
+  __syncthreads();
+  if (tid < E && cnt[tid] > 0) {   // an expert's tiles hold about equally many rows, in whole sixteens
+    const int c = cnt[tid], nt = (c + tile_rows - 1) / tile_rows, per = ((c + nt - 1) / nt + 15) / 16 * 16;
+    for (int i = 0; i < nt && first_tile[tid] + i < max_tiles; ++i) {
+      int* t = tiles + 3 * (first_tile[tid] + i);
+      t[0] = tid;
+      t[1] = off[tid] + i * per;
+      t[2] = min(per, c - i * per);
+    }
+  }
+  for (int p0 = tid; p0 < pairs; p0 += PLAN_BATCH * blockDim.x) {
+    int e[PLAN_BATCH], at[PLAN_BATCH];
+#pragma unroll
+    for (int i = 0; i < PLAN_BATCH; ++i) {
+      const int p = min(p0 + i * static_cast<int>(blockDim.x), pairs - 1);
+      e[i] = sel[p];
+      at[i] = where[p];
+    }
+#pragma unroll
+    for (int i = 0; i < PLAN_BATCH; ++i) {
+      const int p = p0 + i * blockDim.x;
+      if (p < pairs && e[i] >= 0 && e[i] < E) {
+        where[p] = off[e[i]] + at[i];
+        order[off[e[i]] + at[i]] = p;
+      }
     }
   }
 }
@@ -203,12 +247,35 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
 // A is a tile of the weight (1 KB in lane order, as ``StreamedWeight`` keeps it), B the tile's 16
 // rows: a lane ends with four neighbouring output columns of one row.
 //
+// The kernels of few rows (a decode step): a wave takes 16 rows of one expert and 16 weight rows, so that
+// the experts' matrices, which bound it, come in through as many workgroups as there are.  A step's two
+// fragments are asked for two steps ahead of the matrix instruction that uses them: PREFETCH_SETS sets
+// of registers take turns.
+template <class Load>
+__device__ __forceinline__ f32x4 narrow_product(int S, const Load& load) {
+  constexpr int NB = PREFETCH_SETS;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  bf16x8 x[NB], w[NB];
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i)
+    if (i < S) load(i, x[i], w[i]);
+  for (int s = 0; s < S; s += NB) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      if (s + i < S) {
+        if (s + i + NB - 1 < S) load(s + i + NB - 1, x[(i + NB - 1) % NB], w[(i + NB - 1) % NB]);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], x[i], acc, 0, 0, 0);
+      }
+    }
+  }
+  return acc;
+}
+
 // moe_up: act[place, :] = silu(gate) * up for the tile's rows with their expert's matrices; the
 // weight holds every expert's gate and up rows interleaved (gate_j, up_j neighbours), so a lane's
-// four columns are two whole pairs.  Grid (column blocks, tiles); a wave takes GW groups of 16
-// weight rows.  in_wgt (or null): the choice's weight belongs to the expert's input; gate and up are
-// linear in it, so it is multiplied into both sums ahead of the activation.
-template <int RT, int GW>
+// four columns are two whole pairs.  Grid (column blocks, tiles).  in_wgt (or null): the choice's weight
+// belongs to the expert's input; gate and up are linear in it, so it is multiplied into both sums ahead
+// of the activation.
 __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* __restrict__ x, int ldx, int K,
                                                      const uint4* __restrict__ wt, int S,
                                                      const int* __restrict__ order,
@@ -221,73 +288,26 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* __restrict__ 
   const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
   const int lane = threadIdx.x % KVF_WAVE, wave = threadIdx.x / KVF_WAVE;
   const int j = lane % 16, c = lane / 16;
-  const int groups = ff / 8;   // groups of 16 interleaved rows per expert
-  const int g_first = (blockIdx.x * 4 + wave) * GW;
-  if (g_first >= groups) return;
-  // a tile holds RT sub-tiles of 16 rows; a weight fragment is loaded once for all of them
-  const bf16_t* xr[RT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-    xr[r] = 16 * r + j < rows ? x + static_cast<size_t>(order[row0 + 16 * r + j] / top) * ldx + 8 * c : nullptr;
-  f32x4 acc[RT][GW];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int g = 0; g < GW; ++g) acc[r][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const uint4* wbase = wt + (static_cast<size_t>(e) * groups + g_first) * S * KVF_WAVE + lane;
+  const int groups = ff / 8, g = blockIdx.x * 4 + wave;   // groups of 16 interleaved rows per expert
+  if (g >= groups) return;
+  const bf16_t* xr = j < rows ? x + static_cast<size_t>(order[row0 + j] / top) * ldx + 8 * c : nullptr;
+  const uint4* wbase = wt + (static_cast<size_t>(e) * groups + g) * S * KVF_WAVE + lane;
   const int s_full = K / 32;   // steps whose 32 elements all lie inside a row
-  // the fragments of a step are asked for NB - 1 steps ahead of the matrix instructions that use
-  // them: NB sets of registers take turns
-  constexpr int NB = PREFETCH_SETS;
-  bf16x8 xb[NB][RT], wb[NB][GW];
-  auto load = [&](int s, bf16x8 (&xs)[RT], bf16x8 (&ws)[GW]) {
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-      uint4 xf = make_uint4(0u, 0u, 0u, 0u);
-      if (xr[r] && (s < s_full || 32 * s + 8 * c + 8 <= K)) xf = *reinterpret_cast<const uint4*>(xr[r] + 32 * s);
-      xs[r] = __builtin_bit_cast(bf16x8, xf);
-    }
-#pragma unroll
-    for (int g = 0; g < GW; ++g)   // ff is a multiple of 32, so the groups come in whole fours
-      ws[g] = __builtin_bit_cast(bf16x8, wbase[(static_cast<size_t>(g) * S + s) * KVF_WAVE]);
-  };
-  auto mma = [&](const bf16x8 (&xs)[RT], const bf16x8 (&ws)[GW]) {
-#pragma unroll
-    for (int g = 0; g < GW; ++g)
-#pragma unroll
-      for (int r = 0; r < RT; ++r) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[g], xs[r], acc[r][g], 0, 0, 0);
-  };
-#pragma unroll
-  for (int i = 0; i < NB - 1; ++i)
-    if (i < S) load(i, xb[i], wb[i]);
-  for (int s = 0; s < S; s += NB) {
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      if (s + i < S) {
-        if (s + i + NB - 1 < S) load(s + i + NB - 1, xb[(i + NB - 1) % NB], wb[(i + NB - 1) % NB]);
-        mma(xb[i], wb[i]);
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    if (16 * r + j >= rows) continue;
-    bf16_t* out = act + static_cast<size_t>(row0 + 16 * r + j) * ff;
-    const float w = in_wgt ? in_wgt[order[row0 + 16 * r + j]] : 1.f;
-#pragma unroll
-    for (int g = 0; g < GW; ++g) {
-      if (g_first + g >= groups) continue;
-      const int col = (g_first + g) * 8 + 2 * c;
-      const float y0 = joined(f, w * acc[r][g][0], w * acc[r][g][1]), y1 = joined(f, w * acc[r][g][2], w * acc[r][g][3]);
-      *reinterpret_cast<uint32_t*>(out + col) =
-          static_cast<uint32_t>(f32_to_bf16(y0)) | (static_cast<uint32_t>(f32_to_bf16(y1)) << 16);
-    }
-  }
+  const f32x4 acc = narrow_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
+    uint4 xf = make_uint4(0u, 0u, 0u, 0u);
+    if (xr && (s < s_full || 32 * s + 8 * c + 8 <= K)) xf = *reinterpret_cast<const uint4*>(xr + 32 * s);
+    xs = __builtin_bit_cast(bf16x8, xf);
+    ws = __builtin_bit_cast(bf16x8, wbase[static_cast<size_t>(s) * KVF_WAVE]);
+  });
+  if (j >= rows) return;
+  const float w = in_wgt ? in_wgt[order[row0 + j]] : 1.f;
+  const float y0 = joined(f, w * acc[0], w * acc[1]), y1 = joined(f, w * acc[2], w * acc[3]);
+  *reinterpret_cast<uint32_t*>(act + static_cast<size_t>(row0 + j) * ff + g * 8 + 2 * c) =
+      static_cast<uint32_t>(f32_to_bf16(y0)) | (static_cast<uint32_t>(f32_to_bf16(y1)) << 16);
 }
 
 // moe_down: y[place, :] = act[place, :] W_down[expert]^T (bf16, not yet weighted).  The weight
 // holds the experts' down matrices side by side along K: expert e owns the steps e ff/32 ...
-template <int RT, int GW>
 __global__ __launch_bounds__(256) void moe_down_kernel(const bf16_t* __restrict__ act, int ff,
                                                        const uint4* __restrict__ wt, int S_all,
                                                        const int* __restrict__ tiles,
@@ -298,67 +318,237 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const bf16_t* __restrict_
   const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
   const int lane = threadIdx.x % KVF_WAVE, wave = threadIdx.x / KVF_WAVE;
   const int j = lane % 16, c = lane / 16;
-  const int groups = (hidden + 15) / 16;
-  const int g_first = (blockIdx.x * 4 + wave) * GW;
-  if (g_first >= groups) return;
-  const bf16_t* ar[RT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-    ar[r] = 16 * r + j < rows ? act + static_cast<size_t>(row0 + 16 * r + j) * ff + 8 * c : nullptr;
-  f32x4 acc[RT][GW];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int g = 0; g < GW; ++g) acc[r][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int groups = (hidden + 15) / 16, g = blockIdx.x * 4 + wave;
+  if (g >= groups) return;
+  const bf16_t* ar = j < rows ? act + static_cast<size_t>(row0 + j) * ff + 8 * c : nullptr;
   const int S = ff / 32;
-  const uint4* wbase = wt + (static_cast<size_t>(g_first) * S_all + static_cast<size_t>(e) * S) * KVF_WAVE + lane;
-  int goff[GW];
+  const uint4* wbase = wt + (static_cast<size_t>(g) * S_all + static_cast<size_t>(e) * S) * KVF_WAVE + lane;
+  const f32x4 acc = narrow_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
+    uint4 af = make_uint4(0u, 0u, 0u, 0u);
+    if (ar) af = *reinterpret_cast<const uint4*>(ar + 32 * s);
+    xs = __builtin_bit_cast(bf16x8, af);
+    ws = __builtin_bit_cast(bf16x8, wbase[static_cast<size_t>(s) * KVF_WAVE]);
+  });
+  const int col = g * 16 + 4 * c;
+  if (j >= rows || col >= hidden) return;   // hidden is a multiple of 8
+  *reinterpret_cast<uint2*>(y + static_cast<size_t>(row0 + j) * hidden + col) = pack4(acc);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same two products for more rows: tiles of up to 128 rows of one expert against 128 of its weight
+// rows, four waves of 32 weight rows each.
+//
+// What bounds it: the experts' matrices come from memory once (32 experts of 2,048 x 1,024: 403 MB, 80 us
+// at the 5 TB/s of a large copy), the other tiles of an expert find them in their XCD's L2 (see
+// wide_item).  A wave needs its own weight fragments only, so they go straight into registers; the rows,
+// which all four waves need, are gathered through LDS, 64 elements of K at a time in two buffers.  Both
+// are asked for one pass ahead, and three workgroups a compute unit cover what that leaves of the way to
+// memory.  Rows past an expert's last are read as its last and not stored; tiles of up to 96, 64 and 32
+// rows leave the other matrix instructions out.
+//
+// Up and down together with plan and sum, 2,048 tokens, 4 of 32 experts (ff 1,024 / 2,048): 200 / 358 us,
+// where tiles of 64 rows with every fragment straight from memory took 354 / 621.  On the way: 256
+// weight rows a workgroup, two of them a compute unit 215 / 364 (512 equal workgroups leave 40 for a
+// second round); 256 rows and 256 weight rows, eight waves 245 / 390; fragments read from LDS where they
+// are needed instead of two ahead 230 / 380.
+constexpr int WIDE_ROWS = 128, WIDE_GW = 2;
+
+// What a workgroup takes: tile and block of columns.  Workgroups go to the eight XCDs in turn, and each
+// XCD gets an unbroken eighth of the (tile, block) pairs, the blocks of a tile side by side and the tiles of an
+// expert next to each other: an expert's rows and its matrices are then read into one XCD's L2 each.
+__device__ __forceinline__ bool wide_item(int num_tiles, int blocks, int& tile, int& block) {
+  const int total = num_tiles * blocks, share = (total + 7) / 8, at = blockIdx.x / 8;
+  const int item = static_cast<int>(blockIdx.x % 8) * share + at;
+  tile = item / blocks;
+  block = item % blocks;
+  return at < share && item < total;
+}
+template <int N> struct Rows { static constexpr int value = N; };
+template <class F> __device__ __forceinline__ void wide_rows(int rows, const F& go) {
+  if (rows > 96) go(Rows<8>{});
+  else if (rows > 64) go(Rows<6>{});
+  else if (rows > 32) go(Rows<4>{});
+  else go(Rows<2>{});
+}
+
+template <int RT> struct WideAcc { f32x4 v[RT][WIDE_GW]; };
+
+// row_of(r): where row r of the tile starts (r below 16 RT).  wbase, goff: the
+// fragment of group g and step s begins at wbase + goff[g] + s * KVF_WAVE (the same for the whole wave).
+template <int RT, class RowOf>
+__device__ __forceinline__ void wide_product(const RowOf& row_of, int K, const uint4* __restrict__ wbase,
+                                             const size_t (&goff)[WIDE_GW], int S, uint4* lds, WideAcc<RT>& acc) {
+  constexpr int PASSES = RT / 2;                     // 32 rows of 128 bytes are staged at a time
+  const int tid = threadIdx.x, lane = tid % KVF_WAVE;
+  const int ch = tid % 8, sr = tid / 8;              // staged: the 8 elements at 8 ch of rows sr + 32 p
+  const bf16_t* src[PASSES];
 #pragma unroll
-  for (int g = 0; g < GW; ++g) goff[g] = min(g, groups - 1 - g_first);
-  constexpr int NB = PREFETCH_SETS;
-  bf16x8 xb[NB][RT], wb[NB][GW];
-  auto load = [&](int s, bf16x8 (&xs)[RT], bf16x8 (&ws)[GW]) {
+  for (int p = 0; p < PASSES; ++p) src[p] = row_of(sr + 32 * p) + 8 * ch;
+  // A fragment (16 rows x 32 elements) is 64 pieces of 16 bytes.  Piece (row j, c) lies at 4 j + c, c turned
+  // over for rows 8..15: a 16-byte access serves lanes 0-3, 12-15 and 20-27 together, then 4-11, 16-19 and
+  // 28-31, and either sixteen then fall on all banks, read (row lane % 16) or written (row lane / 8).
+  auto place = [](int j, int c) { return 4 * j + (c ^ (j >= 8 ? 3 : 0)); };
+  const int put_at = ((sr / 16) * 2 + ch / 4) * KVF_WAVE + place(sr % 16, ch % 4);
+  const int get_at = place(lane % 16, lane / 16);
+  // No load stands under a condition: where paths with and without one meet, the compiler waits for the
+  // newest loads before the first product, and nothing is ahead of anything any more.
+  uint4 stage[PASSES];
+  auto fetch = [&](int it) {
+    const int k = min(64 * it, K - 8 - 8 * ch);      // K is a multiple of 8: past it a row's last 8, see put
 #pragma unroll
-    for (int r = 0; r < RT; ++r) {
-      uint4 af = make_uint4(0u, 0u, 0u, 0u);
-      if (ar[r]) af = *reinterpret_cast<const uint4*>(ar[r] + 32 * s);
-      xs[r] = __builtin_bit_cast(bf16x8, af);
-    }
-#pragma unroll
-    for (int g = 0; g < GW; ++g)   // a group past the last is read as the last and not stored
-      ws[g] = __builtin_bit_cast(bf16x8, wbase[(static_cast<size_t>(goff[g]) * S_all + s) * KVF_WAVE]);
+    for (int p = 0; p < PASSES; ++p) stage[p] = *reinterpret_cast<const uint4*>(src[p] + k);
   };
-  auto mma = [&](const bf16x8 (&xs)[RT], const bf16x8 (&ws)[GW]) {
+  auto put = [&](int it) {
+    const bool in = 64 * it + 8 * ch < K;
+    uint4* to = lds + (it & 1) * RT * 2 * KVF_WAVE + put_at;
 #pragma unroll
-    for (int g = 0; g < GW; ++g)
+    for (int p = 0; p < PASSES; ++p) to[p * 4 * KVF_WAVE] = in ? stage[p] : make_uint4(0u, 0u, 0u, 0u);
+  };
+  using Weights = uint4[2][WIDE_GW];
+  auto weights = [&](int it, Weights& w) {
 #pragma unroll
-      for (int r = 0; r < RT; ++r) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[g], xs[r], acc[r][g], 0, 0, 0);
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int g = 0; g < WIDE_GW; ++g) w[h][g] = (wbase + goff[g] + static_cast<size_t>(min(2 * it + h, S - 1)) * KVF_WAVE)[lane];
+  };
+  // The products of a pass's first `halves` 32 elements.  Row fragments are read two ahead of the one in
+  // use; left alone the compiler reads each where it is needed, and every four products wait for LDS.
+  auto product = [&](int it, auto halves, const Weights& w) {
+    constexpr int N = RT * decltype(halves)::value;
+    const uint4* frag = lds + (it & 1) * RT * 2 * KVF_WAVE + get_at;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int h = i / RT, r = i % RT;
+      const bf16x8 x = __builtin_bit_cast(bf16x8, frag[(2 * r + h) * KVF_WAVE]);
+#pragma unroll
+      for (int g = 0; g < WIDE_GW; ++g)
+        acc.v[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[h][g]), x, acc.v[r][g], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+    for (int i = 0; i < N - 2; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, WIDE_GW, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 2 * WIDE_GW, 0);
   };
 #pragma unroll
-  for (int i = 0; i < NB - 1; ++i)
-    if (i < S) load(i, xb[i], wb[i]);
-  for (int s = 0; s < S; s += NB) {
+  for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      if (s + i < S) {
-        if (s + i + NB - 1 < S) load(s + i + NB - 1, xb[(i + NB - 1) % NB], wb[(i + NB - 1) % NB]);
-        mma(xb[i], wb[i]);
-      }
-    }
+    for (int g = 0; g < WIDE_GW; ++g) acc.v[r][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Weights now, next;
+  fetch(0);
+  weights(0, now);
+  put(0);
+  fetch(1);
+  const int passes = S / 2;                          // whole ones; an odd step is left over
+#pragma unroll 1
+  for (int it = 0; it < passes; ++it) {
+    __syncthreads();                                 // this pass's rows are there, the other buffer is free
+    put(it + 1);
+    fetch(it + 2);
+    weights(it + 1, next);
+    __builtin_amdgcn_sched_barrier(0);               // all loads first, and no sums held elsewhere
+    product(it, Rows<2>{}, now);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int g = 0; g < WIDE_GW; ++g) now[h][g] = next[h][g];
   }
+  if (S % 2) {
+    __syncthreads();
+    product(passes, Rows<1>{}, now);
+  }
+}
+
+// A lane holds four neighbouring weight rows' products of row lane % 16 of every sub-tile.
+template <int RT>
+__device__ __forceinline__ void wide_up_tile(const bf16_t* __restrict__ x, int ldx, int K, const uint4* __restrict__ wt,
+                                             int S, const int* __restrict__ order, int e, int row0, int rows, int block,
+                                             int top, int ff, const float* __restrict__ in_wgt, const GateForm& f,
+                                             bf16_t* __restrict__ act, uint4* lds) {
+  const int lane = threadIdx.x % KVF_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVF_WAVE);
+  const int j = lane % 16, c = lane / 16;
+  const int groups = ff / 8, g_first = (block * 4 + wave) * WIDE_GW;
+  const int g_read = min(g_first, groups - WIDE_GW);   // groups come in whole fours: all of a wave's or none
+  size_t goff[WIDE_GW];
+#pragma unroll
+  for (int g = 0; g < WIDE_GW; ++g) goff[g] = static_cast<size_t>(g) * S * KVF_WAVE;
+  WideAcc<RT> acc;
+  wide_product<RT>([&](int r) { return x + static_cast<size_t>(order[row0 + min(r, rows - 1)] / top) * ldx; }, K,
+                   wt + (static_cast<size_t>(e) * groups + g_read) * S * KVF_WAVE, goff, S, lds, acc);
+  if (g_first >= groups) return;
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    if (16 * r + j >= rows) continue;
-    bf16_t* out = y + static_cast<size_t>(row0 + 16 * r + j) * hidden;
+    const int row = 16 * r + j;
+    if (row >= rows) continue;
+    bf16_t* out = act + static_cast<size_t>(row0 + row) * ff;
+    const float w = in_wgt ? in_wgt[order[row0 + row]] : 1.f;
 #pragma unroll
-    for (int g = 0; g < GW; ++g) {
-      if (g_first + g >= groups) continue;
-      const int col = (g_first + g) * 16 + 4 * c;
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (col + v < hidden) out[col + v].bits = f32_to_bf16(acc[r][g][v]);
+    for (int g = 0; g < WIDE_GW; ++g) {
+      const f32x4 a = acc.v[r][g];
+      const float y0 = joined(f, w * a[0], w * a[1]), y1 = joined(f, w * a[2], w * a[3]);
+      *reinterpret_cast<uint32_t*>(out + (g_first + g) * 8 + 2 * c) =
+          static_cast<uint32_t>(f32_to_bf16(y0)) | (static_cast<uint32_t>(f32_to_bf16(y1)) << 16);
     }
   }
+}
+
+__global__ __launch_bounds__(256, 3) void moe_up_wide_kernel(const bf16_t* __restrict__ x, int ldx, int K,
+                                                             const uint4* __restrict__ wt, int S,
+                                                             const int* __restrict__ order,
+                                                             const int* __restrict__ tiles,
+                                                             const int* __restrict__ num_tiles, int top, int ff,
+                                                             const float* __restrict__ in_wgt, GateForm f,
+                                                             bf16_t* __restrict__ act) {
+  __shared__ uint4 lds[2 * WIDE_ROWS * 8];
+  int tile, block;
+  if (!wide_item(*num_tiles, (ff / 8 + 4 * WIDE_GW - 1) / (4 * WIDE_GW), tile, block)) return;
+  const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  auto go = [&](auto rt) { wide_up_tile<decltype(rt)::value>(x, ldx, K, wt, S, order, e, row0, rows, block, top, ff, in_wgt, f, act, lds); };
+  wide_rows(rows, go);
+}
+
+template <int RT>
+__device__ __forceinline__ void wide_down_tile(const bf16_t* __restrict__ act, int ff, const uint4* __restrict__ wt,
+                                               int S_all, int e, int row0, int rows, int block,
+                                               bf16_t* __restrict__ y, int hidden,
+                                               uint4* lds) {
+  const int lane = threadIdx.x % KVF_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVF_WAVE);
+  const int j = lane % 16, c = lane / 16;
+  const int groups = (hidden + 15) / 16, g_first = (block * 4 + wave) * WIDE_GW, S = ff / 32;
+  size_t goff[WIDE_GW];   // a group past the last is read as the last and not stored
+#pragma unroll
+  for (int g = 0; g < WIDE_GW; ++g) goff[g] = static_cast<size_t>(min(g_first + g, groups - 1)) * S_all * KVF_WAVE;
+  WideAcc<RT> acc;
+  wide_product<RT>([&](int r) { return act + static_cast<size_t>(row0 + min(r, rows - 1)) * ff; }, ff,
+                   wt + static_cast<size_t>(e) * S * KVF_WAVE, goff, S, lds, acc);
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int row = 16 * r + j;
+    if (row >= rows) continue;
+    bf16_t* out = y + static_cast<size_t>(row0 + row) * hidden;
+#pragma unroll
+    for (int g = 0; g < WIDE_GW; ++g) {
+      const int col = (g_first + g) * 16 + 4 * c;
+      if (col >= hidden) continue;                     // hidden is a multiple of 8
+      *reinterpret_cast<uint2*>(out + col) = pack4(acc.v[r][g]);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256, 3) void moe_down_wide_kernel(const bf16_t* __restrict__ act, int ff,
+                                                               const uint4* __restrict__ wt, int S_all,
+                                                               const int* __restrict__ tiles,
+                                                               const int* __restrict__ num_tiles,
+                                                               bf16_t* __restrict__ y, int hidden) {
+  __shared__ uint4 lds[2 * WIDE_ROWS * 8];
+  int tile, block;
+  if (!wide_item(*num_tiles, ((hidden + 15) / 16 + 4 * WIDE_GW - 1) / (4 * WIDE_GW), tile, block)) return;
+  const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  auto go = [&](auto rt) { wide_down_tile<decltype(rt)::value>(act, ff, wt, S_all, e, row0, rows, block, y, hidden, lds); };
+  wide_rows(rows, go);
 }
 
 // x[n, :] += sum over the token's choices, in their order, of weight * (the expert's row of y, or
@@ -483,9 +673,12 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int
                                hipStream_t s) {
   if (n <= 0) return 0;
   const int pairs = n * top;
-  // many rows: tiles of 64 rows (four sub-tiles share every weight fragment); few: tiles of 16
-  const bool many = pairs >= 1024;
-  const int tile_rows = many ? 64 : 16;
+  // Six rows an expert on average are where the kernels of more rows begin to pay: 192 pairs over 32
+  // experts 84 against 91 us (ff 1,024) and 160 against 162 (ff 2,048), 128 pairs 87 against 92 and 159
+  // against 154, 752 pairs 87 against 142 and 167 against 262 (where an expert's rows pass 16, tiles of
+  // 16 read its matrices again).
+  const bool many = pairs >= 6 * E;
+  const int tile_rows = many ? WIDE_ROWS : 16;
   const GateForm f{form, limit, 1.f};
   if (!form_ok(form, limit) || E <= 0 || E > PLAN_MAX_EXPERTS || K % 8 != 0 || ff % 32 != 0 || ldx % 8 != 0 || max_tiles > 65535 ||
       max_tiles < (pairs + 15) / 16 + E)
@@ -493,21 +686,23 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int
   hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel, pairs, E, where, order, tiles, num_tiles,
                      max_tiles, tile_rows);
   const int S = (K + 31) / 32, up_groups = ff / 8, down_groups = (K + 15) / 16;
-  const int gw = many ? 4 : 1;
-  const int grid_tiles = many ? (pairs + 63) / 64 + E : max_tiles;
-  const dim3 up_grid((up_groups + 4 * gw - 1) / (4 * gw), grid_tiles), down_grid((down_groups + 4 * gw - 1) / (4 * gw), grid_tiles);
   const bf16_t* xb = static_cast<const bf16_t*>(x);
+  const uint4 *up = static_cast<const uint4*>(w_gate_up), *down = static_cast<const uint4*>(w_down);
   const float* in_wgt = weigh_input ? wgt : nullptr;
-  if (many) {
-    hipLaunchKernelGGL((moe_up_kernel<4, 4>), up_grid, dim3(256), 0, s, xb, ldx, K, static_cast<const uint4*>(w_gate_up), S,
-                       order, tiles, num_tiles, top, ff, in_wgt, f, static_cast<bf16_t*>(act));
-    hipLaunchKernelGGL((moe_down_kernel<4, 4>), down_grid, dim3(256), 0, s, static_cast<const bf16_t*>(act), ff,
-                       static_cast<const uint4*>(w_down), E * (ff / 32), tiles, num_tiles, static_cast<bf16_t*>(y), K);
+  bf16_t *a = static_cast<bf16_t*>(act), *out = static_cast<bf16_t*>(y);
+  const int gw = many ? 4 * WIDE_GW : 4;   // groups a workgroup takes
+  const unsigned up_blocks = (up_groups + gw - 1) / gw, down_blocks = (down_groups + gw - 1) / gw;
+  if (many) {   // (tile, block) pairs in one dimension, whole eighths of them
+    const unsigned most = (pairs + WIDE_ROWS - 1) / WIDE_ROWS + E;
+    hipLaunchKernelGGL(moe_up_wide_kernel, dim3((up_blocks * most + 7) / 8 * 8), dim3(256), 0, s, xb, ldx, K, up, S, order,
+                       tiles, num_tiles, top, ff, in_wgt, f, a);
+    hipLaunchKernelGGL(moe_down_wide_kernel, dim3((down_blocks * most + 7) / 8 * 8), dim3(256), 0, s, a, ff, down,
+                       E * (ff / 32), tiles, num_tiles, out, K);
   } else {
-    hipLaunchKernelGGL((moe_up_kernel<1, 1>), up_grid, dim3(256), 0, s, xb, ldx, K, static_cast<const uint4*>(w_gate_up), S,
-                       order, tiles, num_tiles, top, ff, in_wgt, f, static_cast<bf16_t*>(act));
-    hipLaunchKernelGGL((moe_down_kernel<1, 1>), down_grid, dim3(256), 0, s, static_cast<const bf16_t*>(act), ff,
-                       static_cast<const uint4*>(w_down), E * (ff / 32), tiles, num_tiles, static_cast<bf16_t*>(y), K);
+    hipLaunchKernelGGL(moe_up_kernel, dim3(up_blocks, max_tiles), dim3(256), 0, s, xb, ldx, K, up, S, order, tiles,
+                       num_tiles, top, ff, in_wgt, f, a);
+    hipLaunchKernelGGL(moe_down_kernel, dim3(down_blocks, max_tiles), dim3(256), 0, s, a, ff, down, E * (ff / 32), tiles,
+                       num_tiles, out, K);
   }
   hipLaunchKernelGGL(moe_combine_kernel<bf16_t>, dim3(n), dim3(256), 0, s, residual, static_cast<const bf16_t*>(y),
                      static_cast<const bf16_t*>(h), sel, weigh_input ? nullptr : wgt, where, K, top, E, fresh);

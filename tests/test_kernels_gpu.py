@@ -1173,3 +1173,47 @@ def test_sample_frequencies_follow_softmax():
     freq = torch.bincount(toks.cpu().long(), minlength=5).double() / n
     want = torch.softmax(logits.double() / 0.8, -1)
     assert (freq - want).abs().max() < 0.03
+
+
+@pytest.mark.parametrize("counts,K,ff", [([1, 16, 32, 33], 64, 32), ([64, 65, 96, 97], 8, 96), ([127, 128, 129, 0], 200, 64),
+                                         ([256, 257, 0, 500], 72, 32), ([9, 0, 9, 6], 40, 64), ([5, 6, 7, 6], 2048, 160),
+                                         ([5, 6, 7, 5], 2048, 160)])
+@pytest.mark.parametrize("weigh_input", [False, True])
+def test_grouped_experts_at_the_edges_of_their_tiles(counts, K, ff, weigh_input):
+    """``counts[e]`` rows choose expert ``e`` and as many again an output that names no expert: tiles of
+    every size, widths with an odd step and with part of one, and both sides of the line between the
+    kernels of few and of more rows (six rows an expert).  The reference rounds where the kernels
+    store bf16 (the joined pairs, an expert's row); a sum in another order may fall to the other side of
+    either rounding, 2^-8 of its value at most."""
+    E = len(counts)
+    g = torch.Generator().manual_seed(K + sum(counts))
+    chosen = torch.tensor([e for e, c in enumerate(counts) for _ in range(c)], dtype=torch.int32)
+    chosen = chosen[torch.randperm(len(chosen), generator=g)]
+    n = len(chosen)
+    chosen = torch.stack([chosen, torch.full((n,), -1 if weigh_input else E, dtype=torch.int32)], 1).contiguous()
+    chosen = chosen[:, :1].contiguous() if weigh_input else chosen
+    top = chosen.shape[1]
+    x = torch.randn(n, K, generator=g).to(torch.bfloat16)
+    up, down = torch.randn(E, 2 * ff, K, generator=g) * K ** -0.5, torch.randn(K, E, ff, generator=g) * ff ** -0.5
+    up, down = up.to(torch.bfloat16), down.to(torch.bfloat16)
+    w, res = torch.rand(n, top, generator=g), torch.randn(n, K, generator=g)
+    o, tiles = ops(), ops().moe_grouped_tiles(n, top, E)
+    ints = {k: torch.empty(s, dtype=torch.int32, device=DEV) for k, s in (("where", n * top), ("order", n * top),
+                                                                          ("tiles", 3 * tiles), ("num_tiles", 1))}
+    rows = {k: torch.full((n * top, s), math.nan, dtype=torch.bfloat16, device=DEV) for k, s in (("act", ff), ("y", K))}
+    got = res.to(DEV)
+    o.moe_grouped(x.to(DEV), o.streamed(up.reshape(E * 2 * ff, K).to(DEV)), o.streamed(down.reshape(K, E * ff).to(DEV)),
+                  chosen.to(DEV), w.to(DEV), got, E, ff, {**ints, **rows}, weigh_input=weigh_input)
+    want, slack = res.double(), torch.zeros(n, K, dtype=torch.float64)
+    for e in range(E):
+        at = (chosen[:, 0] == e).nonzero()[:, 0]
+        h = torch.einsum("nk,fk->nf", x[at].double(), up[e].double()) * (w[at, :1].double() if weigh_input else 1.0)
+        a = (torch.nn.functional.silu(h[:, 0::2]) * h[:, 1::2]).to(torch.bfloat16).double()
+        y = (a @ down[:, e].double().T).to(torch.bfloat16).double()
+        by = 1.0 if weigh_input else w[at, :1].double()
+        want[at] += by * y
+        slack[at] = by * (y.abs() + a.abs() @ down[:, e].double().abs().T) * 2.0 ** -8
+    if not weigh_input:
+        want += w[:, 1:].double() * x.double()
+    err = (got.cpu().double() - want).abs()
+    assert bool((err <= slack + 1e-5 * (1 + want.abs())).all()), float((err - slack).max())
