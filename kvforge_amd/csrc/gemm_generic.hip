@@ -4,7 +4,7 @@
 // activations are bf16).  No reduced-precision matrix instruction is used: operands stored in
 // bf16 are widened (exactly) before they are multiplied.
 //
-// Many rows (a portion of a prompt), rows of K that start on 16 bytes: tiles of 128 x 128
+// Many rows (a portion of a prompt), rows of K that start on 16 bytes: tiles of 64 x 64 or 128 x 128
 // outputs on the matrix cores with v_mfma_f32_32x32x2_f32, which multiplies and adds in fp32
 // (gemm_mfma32_kernel below).  Many rows otherwise, and kept for comparison: tiles of 64 x 64
 // outputs on the vector ALUs, every output summed
@@ -166,35 +166,46 @@ template <> struct Quad<bf16_t> {
 };
 
 // ---- many rows on the matrix cores, true fp32.
-// A workgroup of four waves owns 128 x XN outputs; a wave owns 64 x (XN / 2) of them as 32 x 32
+// A workgroup of four waves owns XM x XN outputs; a wave owns a quarter of them, XM / 2 x XN / 2, as 32 x 32
 // tiles of v_mfma_f32_32x32x2_f32 (lane l supplies A[row l % 32][k = l / 32] and
 // W[column l % 32][k = l / 32], and holds 16 outputs of column l % 32).  K is walked in tiles of
-// 32: the tile after the current one travels from memory to registers while the matrix cores work
-// on the current one from LDS.  Within a tile of 32 the two halves of the wave take k = 8u + e
+// 32.  Within a tile of 32 the two halves of the wave take k = 8u + e
 // and k = 8u + 4 + e in instruction (u, e), so that a lane reads its operands from LDS 16 bytes
-// at a time; the order of the sums is fixed by K alone.  Rows of A and W start on 16 bytes
-// (8 for bf16) and K is a multiple of 4: the caller checks.
-constexpr int XM = 128, XK = 32, XLD = XK + 4;   // LDS rows 144 bytes apart
+// at a time; the order of the sums is fixed by K alone, whatever the tile.  Rows of A and W start on 16
+// bytes (8 for bf16) and K is a multiple of 4: the caller checks.
+//
+// What bounds it: the matrix cores (64 cycles an instruction) once several tiles share a compute unit, a
+// tile's walk along K otherwise.  The k-tile after the next is on its way into registers, two k-tiles lie
+// in LDS, and one barrier a k-tile is left: 0.66 us a k-tile of 64 x 64 alone, 0.98 with one k-tile ahead
+// and two barriers.  At 777 rows and a 16,384 / 3,072 / 2,048 x 2,048 and a 2,048 x 8,192 weight: 467, 110,
+// 81 and 302 us (112, 89, 81 and 86 TFLOP/s), 782, 224, 131 and 479 before.  Rows and columns past the end are read as the last and not stored, and what lies past K is
+// read inside the row and replaced by zero on its way into LDS: a load that stood against a zero under
+// a condition had become four loads of 4 bytes from a chosen address each, and half of the kernel's
+// time.  Consecutive workgroups go to the eight XCDs in turn; each XCD gets an unbroken eighth of the tiles,
+// the tiles that share columns of W side by side.
+constexpr int XK = 32, XLD = XK + 4;   // LDS rows 144 bytes apart
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-template <typename TA, typename TW, typename TO, int MODE, int XN>
+template <typename TA, typename TW, typename TO, int MODE, int XM, int XN>
 __global__ __launch_bounds__(256) void gemm_mfma32_kernel(const TA* __restrict__ A,
                                                           const TW* __restrict__ W,
                                                           TO* __restrict__ C, int M, int N, int K,
                                                           int lda, int ldc) {
-  constexpr int CT = XN / 64;          // 32-column tiles per wave
-  constexpr int WQ = XN / 32;          // float4 of W a thread stages per k-tile
-  __shared__ __align__(16) float As[XM][XLD];
-  __shared__ __align__(16) float Ws[XN][XLD];
+  constexpr int RT = XM / 64, CT = XN / 64;          // 32-row and 32-column tiles per wave
+  constexpr int AQ = XM / 32, WQ = XN / 32;          // float4 of A and W a thread stages per k-tile
+  __shared__ __align__(16) float As[2][XM][XLD];
+  __shared__ __align__(16) float Ws[2][XN][XLD];
+  const int down = (M + XM - 1) / XM, total = down * ((N + XN - 1) / XN), share = (total + 7) / 8;
+  const int at = static_cast<int>(blockIdx.x / 8), item = static_cast<int>(blockIdx.x % 8) * share + at;
+  if (at >= share || item >= total) return;
   const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE;
-  const int m0 = blockIdx.y * XM, n0 = blockIdx.x * XN;
-  const int wm = (wave / 2) * 64, wn = (wave % 2) * (XN / 2);
+  const int m0 = item % down * XM, n0 = item / down * XN;
+  const int wm = (wave / 2) * (XM / 2), wn = (wave % 2) * (XN / 2);
   const int r32 = lane % 32, half = lane / 32;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 
-  f32x16 acc[2][CT];
+  f32x16 acc[RT][CT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < CT; ++j)
 #pragma unroll
@@ -202,44 +213,43 @@ __global__ __launch_bounds__(256) void gemm_mfma32_kernel(const TA* __restrict__
 
   // what this thread stages: row srow + 32 i, elements skq .. skq + 3 of the k-tile
   const int srow = tid / 8, skq = (tid % 8) * 4;
-  float4 ra[4], rw[WQ];
-  auto fetch = [&](int k0) {
-    const int k = k0 + skq;
+  const TA* arow[AQ];
+  const TW* wrow[WQ];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + srow + 32 * i;
-      ra[i] = (m < M && k < K) ? Quad<TA>::load(A + static_cast<size_t>(m) * lda + k) : zero;
-    }
+  for (int i = 0; i < AQ; ++i) arow[i] = A + static_cast<size_t>(min(m0 + srow + 32 * i, M - 1)) * lda;
 #pragma unroll
-    for (int i = 0; i < WQ; ++i) {
-      const int n = n0 + srow + 32 * i;
-      rw[i] = (n < N && k < K) ? Quad<TW>::load(W + static_cast<size_t>(n) * K + k) : zero;
-    }
+  for (int i = 0; i < WQ; ++i) wrow[i] = W + static_cast<size_t>(min(n0 + srow + 32 * i, N - 1)) * K;
+  struct Staged { float4 a[AQ], w[WQ]; };
+  auto fetch = [&](int k0, Staged& f) {
+    const int k = min(k0 + skq, K - 4);
+#pragma unroll
+    for (int i = 0; i < AQ; ++i) f.a[i] = Quad<TA>::load(arow[i] + k);
+#pragma unroll
+    for (int i = 0; i < WQ; ++i) f.w[i] = Quad<TW>::load(wrow[i] + k);
   };
-  auto stage = [&]() {
+  auto stage = [&](int k0, const Staged& f, int buf) {
+    const bool in = k0 + skq < K;
+    auto kept = [&](const float4& v) { return make_float4(in ? v.x : 0.f, in ? v.y : 0.f, in ? v.z : 0.f, in ? v.w : 0.f); };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(&As[srow + 32 * i][skq]) = ra[i];
+    for (int i = 0; i < AQ; ++i) *reinterpret_cast<float4*>(&As[buf][srow + 32 * i][skq]) = kept(f.a[i]);
 #pragma unroll
-    for (int i = 0; i < WQ; ++i) *reinterpret_cast<float4*>(&Ws[srow + 32 * i][skq]) = rw[i];
+    for (int i = 0; i < WQ; ++i) *reinterpret_cast<float4*>(&Ws[buf][srow + 32 * i][skq]) = kept(f.w[i]);
   };
-
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += XK) {
-    __syncthreads();   // the tile before has been read by every wave
-    stage();
+  auto tile = [&](int k0, Staged& f, int buf) {
+    stage(k0, f, buf);       // its readers two tiles ago are past the barrier of the last one
+    fetch(k0 + 2 * XK, f);   // past the end: the row's last elements, not used
     __syncthreads();
-    if (k0 + XK < K) fetch(k0 + XK);
 #pragma unroll
     for (int u = 0; u < XK / 8; ++u) {
-      float4 a[2], w[CT];
+      float4 a[RT], w[CT];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const float4*>(&As[wm + 32 * i + r32][8 * u + 4 * half]);
+      for (int i = 0; i < RT; ++i) a[i] = *reinterpret_cast<const float4*>(&As[buf][wm + 32 * i + r32][8 * u + 4 * half]);
 #pragma unroll
-      for (int j = 0; j < CT; ++j) w[j] = *reinterpret_cast<const float4*>(&Ws[wn + 32 * j + r32][8 * u + 4 * half]);
+      for (int j = 0; j < CT; ++j) w[j] = *reinterpret_cast<const float4*>(&Ws[buf][wn + 32 * j + r32][8 * u + 4 * half]);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < RT; ++i)
 #pragma unroll
           for (int j = 0; j < CT; ++j) {
             const float av = e == 0 ? a[i].x : e == 1 ? a[i].y : e == 2 ? a[i].z : a[i].w;
@@ -247,10 +257,20 @@ __global__ __launch_bounds__(256) void gemm_mfma32_kernel(const TA* __restrict__
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, wv, acc[i][j], 0, 0, 0);
           }
     }
+  };
+
+  Staged f0, f1;
+  fetch(0, f0);
+  fetch(XK, f1);
+  int k0 = 0;
+  for (; k0 + XK < K; k0 += 2 * XK) {
+    tile(k0, f0, 0);
+    tile(k0 + XK, f1, 1);
   }
+  if (k0 < K) tile(k0, f0, 0);
   // output v of a lane: row 8 (v / 4) + 4 (lane / 32) + v % 4 of the tile, column lane % 32
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
       const int n = n0 + wn + 32 * j + r32;
@@ -412,19 +432,23 @@ int launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, 
     return kvf_last_error();
   }
   if (quads && !g_vector_alus_only) {
-    // tiles of 128 columns where they still give every compute unit two workgroups, of 64 else
-    const int wide = ((N + 127) / 128) * ((M + XM - 1) / XM);
-    if (wide >= 2 * compute_units()) {
-      dim3 mgrid((N + 127) / 128, (M + XM - 1) / XM);
-      hipLaunchKernelGGL((gemm_mfma32_kernel<TA, TW, TO, MODE, 128>), mgrid, dim3(256), 0, s,
-                         static_cast<const TA*>(A), static_cast<const TW*>(W), static_cast<TO*>(C),
-                         M, N, K, lda, ldc);
-    } else {
-      dim3 mgrid((N + 63) / 64, (M + XM - 1) / XM);
-      hipLaunchKernelGGL((gemm_mfma32_kernel<TA, TW, TO, MODE, 64>), mgrid, dim3(256), 0, s,
-                         static_cast<const TA*>(A), static_cast<const TW*>(W), static_cast<TO*>(C),
-                         M, N, K, lda, ldc);
-    }
+#define TILES(XM, XN)                                                                            \
+  do {                                                                                           \
+    const int total = ((N + XN - 1) / XN) * ((M + XM - 1) / XM);                                 \
+    hipLaunchKernelGGL((gemm_mfma32_kernel<TA, TW, TO, MODE, XM, XN>), dim3((total + 7) / 8 * 8), \
+                       dim3(256), 0, s, static_cast<const TA*>(A), static_cast<const TW*>(W),    \
+                       static_cast<TO*>(C), M, N, K, lda, ldc);                                  \
+  } while (0)
+    // Tiles of 64 x 64 unless tiles of 128 x 128 give every compute unit three or more to go through and
+    // leave the busiest one no more to do, by the 6% that they are faster once many are under way:
+    // 16,384 columns of 2,048 elements, 2,048 rows 1,123 against 1,198 us, 1,000 rows 534 against 563, but
+    // 777 rows 606 against 467 and 512 rows 294 against 287; 2,048 columns, 2,048 rows 163 against 148.
+    const long cus = compute_units();
+    auto tiles = [&](long side) { return ((N + side - 1) / side) * ((M + side - 1) / side); };
+    auto rounds = [&](long side) { return (tiles(side) + cus - 1) / cus; };
+    if (tiles(128) >= 3 * cus && 15 * 4 * rounds(128) <= 16 * rounds(64)) TILES(128, 128);
+    else TILES(64, 64);
+#undef TILES
     return kvf_last_error();
   }
   dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);

@@ -652,6 +652,29 @@ def test_gemm_generic_many_rows_on_the_matrix_cores(ta, tw, mnk):
     assert torch.equal(again, out)
 
 
+@pytest.mark.parametrize("tw", DTYPES)
+@pytest.mark.parametrize("k", [4, 36, 68, 128])
+def test_gemm_generic_tiles_of_both_sizes(tw, k):
+    """1,000 rows by 12,260 columns go through tiles of 128 x 128 with partial ones on both edges, 40 of
+    the rows through tiles of 64 x 64: one to four tiles along K, a part of one at its end, against a
+    64-bit product and bit against bit, for the order of the sums is K's alone."""
+    g = torch.Generator().manual_seed(k)
+    a = torch.randn(1000, k, generator=g).to(DEV)
+    w = (torch.randn(12260, k, generator=g) * 0.1).to(tw).to(DEV)
+    out = torch.full((1000, 12260), 7.0, device=DEV)
+    ops().gemm(a, w, out)
+    want = a.double() @ w.double().T
+    # every sum adds k terms: k 2^-24 of the sum of their magnitudes at most
+    bound = k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 1e-30
+    assert bool(((out.double() - want).abs() <= bound).all())
+    part = torch.empty(40, 12260, device=DEV)
+    ops().gemm(a[960:], w, part)
+    assert torch.equal(part, out[960:])
+    acc = torch.ones(1000, 12260, device=DEV)
+    ops().gemm(a, w, acc, accumulate=True)
+    assert torch.equal(acc, out + 1.0)
+
+
 @pytest.mark.parametrize("m", [1, 4, 8, 16, 32])
 @pytest.mark.parametrize("n,k", [(6150, 516), (16390, 260)])
 @pytest.mark.parametrize("tw", DTYPES)
