@@ -265,8 +265,9 @@ template <int RT> struct Rows {
 // the scores are then brought to log2 units before the maximum is taken.  BIAS 2: the scaled
 // score s becomes cap * tanh(s / cap), likewise before the maximum.  BIAS 4: a score also gets its head's
 // entry for the key's distance, likewise.
-template <int DT, int RT, int BIAS>
-__device__ __forceinline__ void block_update(const bf16x8 (&kf)[2][(DT + 1) / 2], const bf16x8 (&vf)[DT],
+// vf(t): the value fragment of element tile t.
+template <int DT, int RT, int BIAS, class Values>
+__device__ __forceinline__ void block_update(const bf16x8 (&kf)[2][(DT + 1) / 2], const Values& vf,
                                              const bf16x8 (&qf)[RT][(DT + 1) / 2], const Rows<RT>& rows,
                                              int kb, int kg, bool edge, float scale_log2, float (&m_ref)[RT], float (&l_run)[RT],
                                              f32x4 (&acc)[RT][DT], float cap = 0.f,
@@ -364,7 +365,7 @@ __device__ __forceinline__ void block_update(const bf16x8 (&kf)[2][(DT + 1) / 2]
     const bf16x8 pf = __builtin_convertvector(p, bf16x8);
 #pragma unroll
     for (int t = 0; t < DT; ++t)
-      acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], pf, acc[rt][t], 0, 0, 0);
+      acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf(t), pf, acc[rt][t], 0, 0, 0);
   }
 }
 
@@ -430,11 +431,14 @@ __device__ __forceinline__ void setup_rows(const bf16_t* q, const MArgs& a, int 
 }
 
 // ------------------------------------------------------------------------------------ query runs
-// SHARE: the waves stage the fragments of each key block in LDS for each other; otherwise every
-// wave loads all of them itself.
+constexpr bool runs_pair(int dt) { return dt > 8; }
+// The waves stage the fragments of each key block in LDS for each other.
 // SINK: the softmax has a sink (a.sinks); a kernel without is the code it was before sinks came
-template <int DT, int RT, bool SHARE, int BIAS, bool SINK>
-__global__ __launch_bounds__(256) KVF_VGPR_FORM(DT <= 8) void attn_mfma_runs_kernel(
+// NW: waves of the workgroup.  Eight stage half as much each as four do, and a key block is brought in for
+// twice the rows.  Heads wider than 128 have two items a work row, four waves each, side by side over the
+// keys that either sees; narrower ones one item of all the waves at a time.
+template <int DT, int RT, int NW, int BIAS, bool SINK>
+__global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) void attn_mfma_runs_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
     const bf16_t* __restrict__ vt_pages, const int* __restrict__ block_table,
     const int* __restrict__ work, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
@@ -444,12 +448,12 @@ __global__ __launch_bounds__(256) KVF_VGPR_FORM(DT <= 8) void attn_mfma_runs_ker
   constexpr int SCORE = CHUNK ? 0 : BIAS;
   constexpr int DC = (DT + 1) / 2;
   constexpr int N_K = 2 * DC, N_FRAG = N_K + DT;          // fragments of a key block
-  constexpr int FPW = (N_FRAG + WAVES - 1) / WAVES;       // fragments a wave stages per block
+  constexpr int FPW = (N_FRAG + NW - 1) / NW;       // fragments a wave stages per block
   // Fragments asked for two blocks ahead (two sets of staging registers) where the registers
   // that takes do not cost a wave per SIMD: measured at head size 128 with one row tile, 2,048
   // queries take 75.7 us with one set (three waves per SIMD) and 87.8 with two (two waves).
   constexpr bool DEEP = RT == 2 || DT <= 4;
-  extern __shared__ uint4 frag_lds[];                     // SHARE: [2][N_FRAG][64]
+  extern __shared__ uint4 frag_lds[];                     // [2][N_FRAG][64]
 
   const int lane = threadIdx.x % KVF_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVF_WAVE);  // the same in all lanes
@@ -465,22 +469,24 @@ __global__ __launch_bounds__(256) KVF_VGPR_FORM(DT <= 8) void attn_mfma_runs_ker
   const bool seq_ok = qlen > 0 && start >= 0;
   const Pages pg{k_pages, vt_pages, block_table + static_cast<size_t>(seq) * a.table_stride, kvh, ctx,
                  j16, kg};
-  float* dist_space = reinterpret_cast<float*>(frag_lds + (SHARE ? 2 * N_FRAG * KVF_WAVE : 0));
+  float* dist_space = reinterpret_cast<float*>(frag_lds + 2 * N_FRAG * KVF_WAVE);
   if (SCORE == 4 && a.dist_lds) {
     stage_dist(a, kvh * G, G, dist_space);
     __syncthreads();
   }
   const DistTable dist{SCORE == 4 && a.dist_lds ? dist_space : nullptr, a.dist, a.n_dist};
-  for (int part = 0; part < 2; ++part) {
-  const int item = work[3 * wrow + 1 + part];
-  if (item < 0) continue;
-  const int wg_tile = item * WAVES * RT;
+  constexpr bool PAIR = runs_pair(DT);
+  constexpr int IW = PAIR ? 4 : NW;   // waves of an item
+  static_assert(!PAIR || (NW == 8 && RT == 1), "pairs of items go to eight waves");
+  for (int part = 0; part < (PAIR ? 1 : 2); ++part) {
+  const int item = work[3 * wrow + 1 + (PAIR ? wave / IW : part)];
+  if (!PAIR && item < 0) continue;
 
   Rows<RT> rows;
   bf16x8 qf[RT][DC];
   int pos_min, pos_max;
-  setup_rows<DT, RT, CHUNK>(q, a, q0, qlen, start, kvh, wg_tile + wave * RT, j16, kg, seq_ok, rows, qf, pos_min,
-                     pos_max);
+  setup_rows<DT, RT, CHUNK>(q, a, q0, qlen, start, kvh, (max(item, 0) * IW + wave % IW) * RT, j16, kg,
+                            seq_ok && item >= 0, rows, qf, pos_min, pos_max);
   if constexpr (SCORE == 4) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -489,22 +495,25 @@ __global__ __launch_bounds__(256) KVF_VGPR_FORM(DT <= 8) void attn_mfma_runs_ker
       rows.far[rt] = a.dist[static_cast<size_t>(rows.head[rt]) * a.n_dist + a.n_dist - 1] * LOG2E;
     }
   }
-  // key range of this wave, and of the workgroup (tiles wg_tile .. wg_tile + 4*RT - 1)
+  // key range of this wave, and of the workgroup
   int lo_w = 0, hi_w = -1;
   if (pos_max >= 0) {
     hi_w = pos_max < ctx - 1 ? pos_max : ctx - 1;
     if (CHUNK) lo_w = chunk_first(a, pos_min);
     else if (a.window > 0 && pos_min - a.window + 1 > 0) lo_w = pos_min - a.window + 1;
   }
-  int lo_g = 0, hi_g = -1;
-  if (seq_ok && wg_tile * 16 < qlen * G) {
-    int t_hi = ((wg_tile + WAVES * RT) * 16 - 1) / G;
+  int lo_g = 0x7fffffff, hi_g = -1;
+#pragma unroll
+  for (int h = 0; h < (PAIR ? 2 : 1); ++h) {
+    const int at = PAIR ? work[3 * wrow + 1 + h] : item, tile = at * IW * RT;
+    if (!seq_ok || at < 0 || tile * 16 >= qlen * G) continue;
+    int t_hi = ((tile + IW * RT) * 16 - 1) / G;
     if (t_hi > qlen - 1) t_hi = qlen - 1;
-    hi_g = start + t_hi < ctx - 1 ? start + t_hi : ctx - 1;
-    const int p_lo = start + wg_tile * 16 / G;
-    if (CHUNK) lo_g = chunk_first(a, p_lo);
-    else if (a.window > 0 && p_lo - a.window + 1 > 0) lo_g = p_lo - a.window + 1;
+    hi_g = max(hi_g, start + t_hi < ctx - 1 ? start + t_hi : ctx - 1);
+    const int p_lo = start + tile * 16 / G;
+    lo_g = min(lo_g, CHUNK ? chunk_first(a, p_lo) : a.window > 0 && p_lo - a.window + 1 > 0 ? p_lo - a.window + 1 : 0);
   }
+  if (hi_g < 0) lo_g = 0;
   const float scale2 = a.scale * LOG2E;
   const int keep_w = a.window > 0 ? a.keep : 0;
 
@@ -518,171 +527,150 @@ __global__ __launch_bounds__(256) KVF_VGPR_FORM(DT <= 8) void attn_mfma_runs_ker
     for (int t = 0; t < DT; ++t) acc[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  if (SHARE) {
-    // fragment f of a block: K (tile f / DC, step f % DC) for f < N_K, then V^T element tiles;
-    // wave w stages fragments w, w + 4, ...
-    // What does not change from block to block is worked out once per fragment: the key a lane
-    // reads relative to the block's start, and its offset inside a page apart from the key's slot
-    // (in fragments of 16 bytes).
-    // Two sets of staging registers and of page lookups, named apart (an index chosen at run
-    // time would put them in scratch memory).  While the waves work on block p from LDS, the
-    // fragments of block p + 1 are on their way in one set (asked for a whole block ago, put
-    // into LDS at the end of this one), those of block p + 2 are asked for into the other, and
-    // the pages of block p + 3 are looked up.  Lookups are issued before the fragment loads of
-    // the same block: the load counter runs in order, so waiting for a lookup then does not
-    // also wait for fragments that were asked for after it.
-    struct Stage {
-      uint4 frag[FPW];
-      int live[FPW];
-    };
-    struct Lookup {
-      PageRef page[FPW];
-    };
-    int key_off[FPW];
-    unsigned lane_off[FPW];
-    bool is_k[FPW], whole[FPW];
-    const unsigned page_stride = static_cast<unsigned>(a.KV) * a.bs * (D / 8);
+  // fragment f of a block: K (tile f / DC, step f % DC) for f < N_K, then V^T element tiles;
+  // wave w stages fragments w, w + 4, ...
+  // What does not change from block to block is worked out once per fragment: the key a lane
+  // reads relative to the block's start, and its offset inside a page apart from the key's slot
+  // (in fragments of 16 bytes).
+  // Two sets of staging registers and of page lookups, named apart (an index chosen at run
+  // time would put them in scratch memory).  While the waves work on block p from LDS, the
+  // fragments of block p + 1 are on their way in one set (asked for a whole block ago, put
+  // into LDS at the end of this one), those of block p + 2 are asked for into the other, and
+  // the pages of block p + 3 are looked up.  Lookups are issued before the fragment loads of
+  // the same block: the load counter runs in order, so waiting for a lookup then does not
+  // also wait for fragments that were asked for after it.
+  struct Stage {
+    uint4 frag[FPW];
+    int live[FPW];
+  };
+  struct Lookup {
+    PageRef page[FPW];
+  };
+  int key_off[FPW];
+  unsigned lane_off[FPW];
+  bool is_k[FPW], whole[FPW];
+  const unsigned page_stride = static_cast<unsigned>(a.KV) * a.bs * (D / 8);
+#pragma unroll
+  for (int i = 0; i < FPW; ++i) {
+    const int f = min(wave + i * NW, N_FRAG - 1);        // past the last: read as the last, not kept
+    is_k[i] = f < N_K;
+    if (is_k[i]) {
+      const int t = f / DC, c = f % DC;
+      key_off[i] = 8 * (j16 >> 2) + 4 * t + (j16 & 3);
+      whole[i] = !((DT % 2) && c == DT / 2 && kg >= 2);  // a step that reaches past d
+      lane_off[i] = static_cast<unsigned>(kvh) * a.bs * (D / 8) + (whole[i] ? c * 4 + kg : 0);
+    } else {
+      key_off[i] = 8 * kg;
+      whole[i] = true;
+      lane_off[i] = (static_cast<unsigned>(kvh) * D + (f - N_K) * 16 + j16) * (a.bs / 8);
+    }
+  }
+  // Every load below reads a valid address whatever the block (a key past the context reads
+  // the table's last entry and page 0, and counts for nothing), so none of them sits in a
+  // branch and the compiler can count them.
+  const Walk wk = walk_of(a, lo_g, hi_g);
+  auto locate = [&](int kb, Lookup& l) {
+    kb = wk.at(kb);
+#pragma unroll
+    for (int i = 0; i < FPW; ++i) l.page[i] = page_of_key(pg, a, kb + key_off[i]);
+  };
+  auto fetch = [&](int kb, const Lookup& l, Stage& st) {
+    kb = wk.at(kb);
 #pragma unroll
     for (int i = 0; i < FPW; ++i) {
-      const int f = wave + i * WAVES;
-      is_k[i] = f < N_K;
-      if (is_k[i]) {
-        const int t = f / DC, c = f % DC;
-        key_off[i] = 8 * (j16 >> 2) + 4 * t + (j16 & 3);
-        whole[i] = !((DT % 2) && c == DT / 2 && kg >= 2);  // a step that reaches past d
-        lane_off[i] = static_cast<unsigned>(kvh) * a.bs * (D / 8) + (whole[i] ? c * 4 + kg : 0);
-      } else {
-        key_off[i] = 8 * kg;
-        whole[i] = f < N_FRAG;
-        lane_off[i] = (static_cast<unsigned>(kvh) * D + (f - N_K) * 16 + j16) * (a.bs / 8);
+      const int key = kb + key_off[i];
+      const unsigned slot = static_cast<unsigned>(key - block_of(a, key) * a.bs);
+      const bool ok = l.page[i].ok(a.nb) && whole[i];
+      st.live[i] = !ok ? 0 : is_k[i] ? 8 : min(ctx - key, 8);
+      const unsigned off = __umul24(ok ? l.page[i].page : 0, page_stride) + lane_off[i] +
+                           (is_k[i] ? __umul24(slot, D / 8) : slot >> 3);
+      st.frag[i] = ld16((is_k[i] ? k_pages : vt_pages) + static_cast<size_t>(off) * 8);
+    }
+  };
+  auto put = [&](int buf, const Stage& st) {
+#pragma unroll
+    for (int i = 0; i < FPW; ++i) {
+      const int f = wave + i * NW;
+      if (f < N_FRAG) frag_lds[(buf * N_FRAG + f) * KVF_WAVE + lane] = keep_first(st.frag[i], st.live[i]);
+    }
+  };
+  auto work_on = [&](int kb, int buf) {
+    kb = wk.at(kb);
+    if (kb <= hi_w && (kb + 31 >= lo_w || kb < keep_w)) {
+      bf16x8 kf[2][DC];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+          kf[t][c] = as_frag(frag_lds[(buf * N_FRAG + t * DC + c) * KVF_WAVE + lane]);
+      const uint4* values = frag_lds + (buf * N_FRAG + N_K) * KVF_WAVE + lane;
+      const bool edge = kb + 31 > pos_min || kb + 32 > ctx || a.window > 0 || CHUNK;
+      if constexpr (DT <= 14) {
+        bf16x8 vf[DT];
+#pragma unroll
+        for (int t = 0; t < DT; ++t) vf[t] = as_frag(values[t * KVF_WAVE]);
+        block_update<DT, RT, SCORE>(kf, [&](int t) { return vf[t]; }, qf, rows, kb, kg, edge, scale2, m_ref, l_run, acc,
+                                    a.cap, dist, pos_min);
+      } else {   // wide heads: a value fragment is read where it is used and holds no registers before
+        block_update<DT, RT, SCORE>(kf, [&](int t) { return as_frag(values[t * KVF_WAVE]); }, qf, rows, kb, kg, edge,
+                                    scale2, m_ref, l_run, acc, a.cap, dist, pos_min);
       }
     }
-    // Every load below reads a valid address whatever the block (a key past the context reads
-    // the table's last entry and page 0, and counts for nothing), so none of them sits in a
-    // branch and the compiler can count them.
-    const Walk wk = walk_of(a, lo_g, hi_g);
-    auto locate = [&](int kb, Lookup& l) {
-      kb = wk.at(kb);
-#pragma unroll
-      for (int i = 0; i < FPW; ++i) l.page[i] = page_of_key(pg, a, kb + key_off[i]);
-    };
-    auto fetch = [&](int kb, const Lookup& l, Stage& st) {
-      kb = wk.at(kb);
-#pragma unroll
-      for (int i = 0; i < FPW; ++i) {
-        const int key = kb + key_off[i];
-        const unsigned slot = static_cast<unsigned>(key - block_of(a, key) * a.bs);
-        const bool ok = l.page[i].ok(a.nb) && whole[i];
-        st.live[i] = !ok ? 0 : is_k[i] ? 8 : min(ctx - key, 8);
-        const unsigned off = __umul24(ok ? l.page[i].page : 0, page_stride) + lane_off[i] +
-                             (is_k[i] ? __umul24(slot, D / 8) : slot >> 3);
-        st.frag[i] = ld16((is_k[i] ? k_pages : vt_pages) + static_cast<size_t>(off) * 8);
-      }
-    };
-    auto put = [&](int buf, const Stage& st) {
-#pragma unroll
-      for (int i = 0; i < FPW; ++i) {
-        const int f = wave + i * WAVES;
-        if (f < N_FRAG) frag_lds[(buf * N_FRAG + f) * KVF_WAVE + lane] = keep_first(st.frag[i], st.live[i]);
-      }
-    };
-    auto work_on = [&](int kb, int buf) {
-      kb = wk.at(kb);
-      if (kb <= hi_w && (kb + 31 >= lo_w || kb < keep_w)) {
-        bf16x8 kf[2][DC], vf[DT];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int c = 0; c < DC; ++c)
-            kf[t][c] = as_frag(frag_lds[(buf * N_FRAG + t * DC + c) * KVF_WAVE + lane]);
-#pragma unroll
-        for (int t = 0; t < DT; ++t) vf[t] = as_frag(frag_lds[(buf * N_FRAG + N_K + t) * KVF_WAVE + lane]);
-        const bool edge = kb + 31 > pos_min || kb + 32 > ctx || a.window > 0 || CHUNK;
-        block_update<DT, RT, SCORE>(kf, vf, qf, rows, kb, kg, edge, scale2, m_ref, l_run, acc, a.cap, dist, pos_min);
-      }
-    };
-    const int kb_first = wk.first;
-    hi_g = wk.last;
-    Stage sa;
-    Lookup la;
-    if constexpr (DEEP) {
-      Stage sb;
-      Lookup lb;
-      if (kb_first <= hi_g) {
-        locate(kb_first, la);
-        locate(kb_first + 32, lb);
-        fetch(kb_first, la, sa);
-        locate(kb_first + 64, la);
-        fetch(kb_first + 32, lb, sb);
-        put(0, sa);
-      }
-      // Everything loaded so far (the query fragments among it) has to be there before the loop:
-      // otherwise the compiler, not knowing how many loads a first pass through the loop still
-      // has ahead of them, waits for all loads before the first product of every pass.
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  };
+  const int kb_first = wk.first;
+  hi_g = wk.last;
+  Stage sa;
+  Lookup la;
+  if constexpr (DEEP) {
+    Stage sb;
+    Lookup lb;
+    if (kb_first <= hi_g) {
+      locate(kb_first, la);
+      locate(kb_first + 32, lb);
+      fetch(kb_first, la, sa);
+      locate(kb_first + 64, la);
+      fetch(kb_first + 32, lb, sb);
+      put(0, sa);
+    }
+    // Everything loaded so far (the query fragments among it) has to be there before the loop:
+    // otherwise the compiler, not knowing how many loads a first pass through the loop still
+    // has ahead of them, waits for all loads before the first product of every pass.
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __syncthreads();
+    // at the top of a pass: LDS half 0 holds block kb, `sb` block kb + 32, `la` the pages of
+    // block kb + 64
+    for (int kb = kb_first; kb <= hi_g; kb += 64) {
+      locate(kb + 96, lb);
+      fetch(kb + 64, la, sa);
+      work_on(kb, 0);
+      put(1, sb);
       __syncthreads();
-      // at the top of a pass: LDS half 0 holds block kb, `sb` block kb + 32, `la` the pages of
-      // block kb + 64
-      for (int kb = kb_first; kb <= hi_g; kb += 64) {
-        locate(kb + 96, lb);
-        fetch(kb + 64, la, sa);
-        work_on(kb, 0);
-        put(1, sb);
-        __syncthreads();
-        if (kb + 32 > hi_g) break;
-        locate(kb + 128, la);
-        fetch(kb + 96, lb, sb);
-        work_on(kb + 32, 1);
-        put(0, sa);
-        __syncthreads();
-      }
-    } else {
-      // one set: the fragments of block p + 1 are asked for at the top of block p and put into
-      // LDS at its end; the pages of block p + 2 are looked up meanwhile
-      if (kb_first <= hi_g) {
-        locate(kb_first, la);
-        fetch(kb_first, la, sa);
-        locate(kb_first + 32, la);
-        put(0, sa);
-      }
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as above
+      if (kb + 32 > hi_g) break;
+      locate(kb + 128, la);
+      fetch(kb + 96, lb, sb);
+      work_on(kb + 32, 1);
+      put(0, sa);
       __syncthreads();
-      int buf = 0;
-      for (int kb = kb_first; kb <= hi_g; kb += 32) {
-        fetch(kb + 32, la, sa);
-        locate(kb + 64, la);
-        work_on(kb, buf);
-        put(buf ^ 1, sa);
-        __syncthreads();
-        buf ^= 1;
-      }
     }
   } else {
-    const Walk wk = walk_of(a, lo_w, hi_w);
-    PageRef pk[2] = {k_page(pg, a, wk.at(wk.first), 0), k_page(pg, a, wk.at(wk.first), 1)};
-    PageRef pv = v_page(pg, a, wk.at(wk.first));
-    for (int kc = wk.first; kc <= wk.last; kc += 32) {
-      const int kb = wk.at(kc);
-      uint4 kr[2][DC], vr[DT];
-      int kl[2][DC], vl;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int c = 0; c < DC; ++c) kr[t][c] = k_fragment<DT>(pg, a, kb, t, c, pk[t], kl[t][c]);
-#pragma unroll
-      for (int t = 0; t < DT; ++t) vr[t] = v_fragment(pg, a, kb, t, pv, vl);
-      pk[0] = k_page(pg, a, wk.at(kc + 32), 0);
-      pk[1] = k_page(pg, a, wk.at(kc + 32), 1);
-      pv = v_page(pg, a, wk.at(kc + 32));
-      bf16x8 kf[2][DC], vf[DT];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int c = 0; c < DC; ++c) kf[t][c] = as_frag(keep_first(kr[t][c], kl[t][c]));
-#pragma unroll
-      for (int t = 0; t < DT; ++t) vf[t] = as_frag(keep_first(vr[t], vl));
-      const bool edge = kb + 31 > pos_min || kb + 32 > ctx || a.window > 0 || CHUNK;
-      block_update<DT, RT, SCORE>(kf, vf, qf, rows, kb, kg, edge, scale2, m_ref, l_run, acc, a.cap, dist, pos_min);
+    // one set: the fragments of block p + 1 are asked for at the top of block p and put into
+    // LDS at its end; the pages of block p + 2 are looked up meanwhile
+    if (kb_first <= hi_g) {
+      locate(kb_first, la);
+      fetch(kb_first, la, sa);
+      locate(kb_first + 32, la);
+      put(0, sa);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as above
+    __syncthreads();
+    int buf = 0;
+    for (int kb = kb_first; kb <= hi_g; kb += 32) {
+      fetch(kb + 32, la, sa);
+      locate(kb + 64, la);
+      work_on(kb, buf);
+      put(buf ^ 1, sa);
+      __syncthreads();
+      buf ^= 1;
     }
   }
 
@@ -810,7 +798,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
 #pragma unroll
     for (int t = 0; t < DT; ++t) vf[t] = as_frag(keep_first(r.v[t], r.vl));
     const bool edge = kb + 31 > pos_min || kb + 32 > ctx || a.window != 0;
-    block_update<DT, 1, BIAS>(kf, vf, qf, rows, kb, kg, edge, scale2, m_ref, l_run, acc, a.cap, dist, pos_min);
+    block_update<DT, 1, BIAS>(kf, [&](int t) { return vf[t]; }, qf, rows, kb, kg, edge, scale2, m_ref, l_run, acc, a.cap, dist, pos_min);
   };
   // Without a window the page lookups of the first blocks are asked for together with the
   // query and the context length, not after them: one round trip to memory less.
@@ -974,30 +962,43 @@ unsigned chunk_magic_of(int window) {
   return m > 0xffffffffull ? 0xffffffffu : static_cast<unsigned>(m);
 }
 
-// Row tiles per wave and LDS sharing by head size: what fits the registers and 64 KB of LDS.
-// One tile per wave keeps more workgroups in flight; two halve what a key block costs per row
+// Row tiles per wave and waves by head size.  Up to 128 a workgroup is four waves.  One tile per wave (64
+// rows an item) keeps more workgroups in flight; two halve what a key block costs per row
 // (looking its pages up, staging it, the barrier) and pay when the work fills the chip anyway
 // (measured at 32 heads of size 64, one item per workgroup: 8,192 tokens 444 to 385 us, 4,096
 // tokens 143 to 114; 2,048 tokens 47 to 54 the other way): the caller chooses by the rows it
-// has and by kvf_attn_mfma_prefill_blocks_per_cu.
+// has and by kvf_attn_mfma_prefill_blocks_per_cu.  (One tile for each of eight waves in the place of two
+// for each of four: 2,048 queries behind 4,096 keys 175 to 162, but 4,096 queries 116 to 130.)
+// Wider heads have one tile per wave and two items of 64 rows to a workgroup of eight waves (PAIR), which
+// halves the fragments a wave stages and what is brought in per row: 32 heads of size 224 over one kv
+// head, 2,048 queries 105 us, 2,048 behind 4,096 keys 435; with four waves and one item 132 and 546; with
+// every wave loading all 28 fragments of a block by itself, in so many registers that a SIMD held one wave,
+// 300 and 1,385.  What bounds it now: a fragment read from LDS for each matrix instruction (448 TFLOP/s and
+// 671 of them; two tiles a wave would halve the reads but leave one wave a SIMD: 182 and 782 us).
 constexpr int runs_max_rt(int dt) { return dt <= 8 ? 2 : 1; }
-constexpr bool runs_share(int dt) { return dt <= 12; }
 constexpr size_t DIST_LDS_MOST = 64 * 1024;   // LDS a launch may ask for together with its table of biases
 
-template <int DT, int RT>
+template <int N> struct Count { static constexpr int value = N; };
+// calls go(tiles per wave, waves) for items of `row_tiles` times 64 rows
+template <int DT, class Go> void runs_shape(int row_tiles, const Go& go) {
+  if constexpr (runs_pair(DT)) go(Count<1>{}, Count<8>{});
+  else if (row_tiles < 2) go(Count<1>{}, Count<4>{});
+  else go(Count<2>{}, Count<4>{});
+}
+
+template <int DT, int RT, int NW>
 void launch_runs_rt(dim3 grid, hipStream_t s, const void* q, const void* k_pages, const void* vt_pages,
                     const int* block_table, const int* work, const int* cu_q, const int* ctx_lens, void* out,
                     const MArgs& a) {
-  constexpr bool SHARE = runs_share(DT);
   constexpr int N_FRAG = 2 * ((DT + 1) / 2) + DT;
-  const size_t lds = SHARE ? static_cast<size_t>(2) * N_FRAG * KVF_WAVE * sizeof(uint4) : 0;
+  const size_t lds = static_cast<size_t>(2) * N_FRAG * KVF_WAVE * sizeof(uint4);
   if (a.window < 0)   // (never with a cap, sinks or slopes: the exported entry refuses the pairs)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, SHARE, 3, false>), grid, dim3(256), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 3, false>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
   else if (a.cap > 0.f)   // (never with sinks or slopes: the exported entry refuses the pairs)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, SHARE, 2, false>), grid, dim3(256), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 2, false>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
@@ -1005,22 +1006,22 @@ void launch_runs_rt(dim3 grid, hipStream_t s, const void* q, const void* k_pages
     MArgs b = a;
     const size_t table = static_cast<size_t>(a.H / a.KV) * dist_row(a.n_dist) * sizeof(float);
     b.dist_lds = lds + table <= DIST_LDS_MOST;
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, SHARE, 4, false>), grid, dim3(256), b.dist_lds ? lds + table : lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 4, false>), grid, dim3(NW * KVF_WAVE), b.dist_lds ? lds + table : lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), b);
   } else if (a.sinks)   // (never with slopes: the exported entry refuses the pair)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, SHARE, 0, true>), grid, dim3(256), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 0, true>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
   else if (a.slopes)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, SHARE, 1, false>), grid, dim3(256), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 1, false>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
   else
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, SHARE, 0, false>), grid, dim3(256), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 0, false>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
@@ -1030,13 +1031,11 @@ template <int DT>
 void launch_runs(int row_tiles, dim3 grid, hipStream_t s, const void* q, const void* k_pages,
                  const void* vt_pages, const int* block_table, const int* work, const int* cu_q,
                  const int* ctx_lens, void* out, const MArgs& a) {
-  if constexpr (runs_max_rt(DT) >= 2) {
-    if (row_tiles == 2) {
-      launch_runs_rt<DT, 2>(grid, s, q, k_pages, vt_pages, block_table, work, cu_q, ctx_lens, out, a);
-      return;
-    }
-  }
-  launch_runs_rt<DT, 1>(grid, s, q, k_pages, vt_pages, block_table, work, cu_q, ctx_lens, out, a);
+  auto go = [&](auto rt, auto nw) {
+    launch_runs_rt<DT, decltype(rt)::value, decltype(nw)::value>(grid, s, q, k_pages, vt_pages, block_table, work, cu_q,
+                                                                 ctx_lens, out, a);
+  };
+  runs_shape<DT>(row_tiles, go);
 }
 
 template <int DT, int NW>
@@ -1107,33 +1106,30 @@ KVF_EXPORT int kvf_attn_mfma_rows_per_item(int d, int row_tiles) {
   return WAVES * (row_tiles >= 2 ? most : 1) * 16;
 }
 
+// Whether a work row's two items are taken side by side by one workgroup: a caller then makes rows of
+// neighbouring items.
+KVF_EXPORT int kvf_attn_mfma_prefill_pairs(int d) { return runs_pair((d + 15) / 16) ? 1 : 0; }
+
 // Workgroups of the kernel for query runs that a compute unit holds at once, by its registers
 // and LDS: what a caller weighs rows per item against (0 if the head size is not taken).
-template <int DT, int RT>
-int runs_blocks_per_cu() {
-  constexpr bool SHARE = runs_share(DT);
-  constexpr int N_FRAG = 2 * ((DT + 1) / 2) + DT;
-  const size_t lds = SHARE ? static_cast<size_t>(2) * N_FRAG * KVF_WAVE * sizeof(uint4) : 0;
-  int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_mfma_runs_kernel<DT, RT, SHARE, 0, false>, 256, lds) !=
-      hipSuccess)
-    return 0;
-  return n;
-}
 KVF_EXPORT int kvf_attn_mfma_prefill_blocks_per_cu(int d, int row_tiles) {
   if (d <= 0 || d % 16 != 0 || d > 256) return 0;
-  const bool two = row_tiles >= 2 && d <= 128;
+  int n = 0;
   switch (d / 16) {
-#define GO(DT)                                                              \
-  case DT:                                                                  \
-    if constexpr (runs_max_rt(DT) >= 2) {                                   \
-      if (two) return runs_blocks_per_cu<DT, 2>();                          \
-    }                                                                       \
-    return runs_blocks_per_cu<DT, 1>();
+#define GO(DT)                                                                                       \
+  case DT:                                                                                           \
+    runs_shape<DT>(row_tiles, [&](auto rt, auto nw) {                                                \
+      constexpr int NW = decltype(nw)::value;                                                        \
+      const size_t lds = static_cast<size_t>(2) * (2 * ((DT + 1) / 2) + DT) * KVF_WAVE * sizeof(uint4); \
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(                                              \
+              &n, attn_mfma_runs_kernel<DT, decltype(rt)::value, NW, 0, false>, NW * KVF_WAVE, lds) != hipSuccess) \
+        n = 0;                                                                                       \
+    });                                                                                              \
+    break;
     KVF_EACH_DT(GO)
 #undef GO
   }
-  return 0;
+  return n;
 }
 
 // Query runs: `work` holds num_work rows (sequence, item, item or -1) where item i covers rows

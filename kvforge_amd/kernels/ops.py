@@ -1269,11 +1269,18 @@ def attention_on_matrix_cores(dtype: torch.dtype, block_size: int, head_dim: int
 
 def prefill_rows_per_item(dtype: torch.dtype, head_dim: int, block_size: int, row_tiles: int = 1) -> int:
     """Rows of (query token, head in group) that one entry of a prefill work list covers.
-    ``row_tiles``: 1 or 2 tiles of 16 rows per wave of the matrix-core kernel (two where the head
-    size allows them; they pay when the work fills the chip anyway, see ``attn_mfma.hip``)."""
+    ``row_tiles``: 64 or 128 rows on the matrix cores, four waves times 1 or 2 tiles of 16 rows (two where the
+    head size allows them; they pay when the work fills the chip anyway, see ``attn_mfma.hip``)."""
     if attention_on_matrix_cores(dtype, block_size, head_dim):
         return int(_fn("attn_mfma", "kvf_attn_mfma_rows_per_item", [c_int, c_int])(int(head_dim), int(row_tiles)))
     return int(_fn("attn_generic", "kvf_attn_generic_rows_per_item", [])())
+
+
+def prefill_takes_pairs(dtype: torch.dtype, head_dim: int, block_size: int) -> bool:
+    """Whether the kernel for query runs takes the two items of a work row side by side, so that rows are best made
+    of neighbouring items (heads wider than 128 on the matrix cores)."""
+    return (attention_on_matrix_cores(dtype, block_size, head_dim)
+            and bool(_fn("attn_mfma", "kvf_attn_mfma_prefill_pairs", [c_int])(int(head_dim))))
 
 
 _blocks_per_cu: dict[tuple, int] = {}

@@ -51,7 +51,7 @@ def skew_cuts(max_ctx: int, sum_ctx: int, n: int) -> int:
 
 
 def prefill_work_rows(q_lens, prefill_seqs, group_size: int, rows_per_item: int,
-                      start_pos=None) -> list[tuple]:
+                      start_pos=None, pairs: bool = False) -> list[tuple]:
     """Rows (sequence row, item, -1) for every query run longer than one token: a run of ``q``
     tokens has ``q * group_size`` rows per kv head, an item covers ``rows_per_item`` of them, and
     a workgroup takes one item.  Under the causal mask an item walks the keys up to its last
@@ -61,14 +61,19 @@ def prefill_work_rows(q_lens, prefill_seqs, group_size: int, rows_per_item: int,
     one, which balances the workgroups among themselves; measured once the kv heads were spread
     over the XCDs it lost to this order, which keeps twice the workgroups in flight: 2,048
     queries of 32 heads of size 64 take 58 us in pairs and 47 us one by one, 2,048 at the end
-    of 8,192 keys 398 and 301.)"""
+    of 8,192 keys 398 and 301.)  ``pairs``: the kernel takes a row's two items side by side
+    (``ops.prefill_takes_pairs``), so a row holds two neighbouring ones, (sequence row, item, item before it or -1)."""
     rows = []
     for b in prefill_seqs:
         n = -(-q_lens[b] * group_size // rows_per_item)
         before = start_pos[b] if start_pos is not None else 0
-        rows += [(before + min(q_lens[b], -(-(i + 1) * rows_per_item // group_size)), b, i) for i in range(n)]
+        step = 2 if pairs else 1
+        for first in range(0, n, step):
+            last = min(first + step, n) - 1
+            end = before + min(q_lens[b], -(-(last + 1) * rows_per_item // group_size))
+            rows.append((end, b, last, first if first < last else -1))
     rows.sort(key=lambda r: -r[0])        # stable: equal walks stay in sequence and item order
-    return [(b, i, -1) for _, b, i in rows]
+    return [row[1:] for row in rows]
 
 
 def distance_bucket(n: int, buckets: int, far: float) -> int:
@@ -430,13 +435,13 @@ class PagedAttention(Mixer):
 
     def _prefill_work(self, step, act: torch.dtype, block_size: int):
         """(work rows on the device, rows per item) of the step's query runs, or ``(None, 0)``.
-        Items of two row tiles per wave halve what a key block costs per row (its page lookups,
+        Items of 128 rows halve what a key block costs per row (its page lookups,
         staging and barrier) and halve the workgroups.  They are taken where the kernel has them
         and their workgroups alone are as many as the chip holds of the one-tile kernel at a
         time (so that short items are left to fill in behind the long ones), or give every
         compute unit two while every run starts at least its own length into its sequence (then
         all items walk long and nothing needs filling in).  Measured at 32 heads over 8 kv heads,
-        one against two tiles: 2,048 queries from position 0, 47 against 55 us at head size 64
+        64 against 128 rows (as two row tiles a wave): 2,048 queries from position 0, 47 against 55 us at head size 64
         and 70 against 82 at 128; 4,096 queries, 140 against 114 and 231 against 196; 2,048
         queries behind 2,048 keys, 106 against 100 and 209 against 151.  The layers of a model
         that agree on group size and item share the rows through the step's scratch."""
@@ -447,12 +452,13 @@ class PagedAttention(Mixer):
         found = step.scratch.get(key)
         if found is None:
             units = compute_units(step.device)
+            pairs = ops.prefill_takes_pairs(act, self.d, block_size)
             per_item = ops.prefill_rows_per_item(act, self.d, block_size, 2)
-            rows = prefill_work_rows(step.q_lens, step.prefill_seqs, G, per_item, step.start_pos)
+            rows = prefill_work_rows(step.q_lens, step.prefill_seqs, G, per_item, step.start_pos, pairs)
             groups = len(rows) * self.KV
             fills = groups >= ops.prefill_blocks_per_cu(act, self.d, block_size, 1) * units
             deep = groups >= 2 * units and all(step.start_pos[b] >= step.q_lens[b] for b in step.prefill_seqs)
-            if not (fills or deep):
+            if not (fills or deep or pairs):     # where items go in pairs they have one size
                 per_item = ops.prefill_rows_per_item(act, self.d, block_size, 1)
                 rows = prefill_work_rows(step.q_lens, step.prefill_seqs, G, per_item, step.start_pos)
             found = (step.upload_ints([x for row in rows for x in row]).view(-1, 3), per_item)

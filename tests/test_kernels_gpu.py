@@ -794,6 +794,40 @@ def test_attn_prefill(dtype, seq_lens, q_lens, H, KV, d, bs, window):
         torch.testing.assert_close(out.float().cpu(), want, **tol(dtype))
 
 
+@pytest.mark.parametrize("d", [144, 208, 224, 240, 256])
+@pytest.mark.parametrize("H,KV", [(32, 1), (3, 1), (6, 2)])
+@pytest.mark.parametrize("window", [0, 11])
+def test_attn_prefill_of_wide_heads_takes_items_in_pairs(d, H, KV, window):
+    """Heads wider than 128: two items of a work row side by side.  Neighbours as the planner makes them (an odd one
+    left alone), an early one with a late one, a lone item in either place, and a row of a sequence without
+    one, on runs that end inside an item, inside a page and inside a block of keys."""
+    from kvforge_amd.parts.attention import prefill_work_rows
+    seq_lens, q_lens = [200, 131, 33, 77], [67, 131, 33, 2]
+    paged = Paged(seq_lens, KV, d, 16, torch.bfloat16, seed=d)
+    g = torch.Generator().manual_seed(d + H)
+    n, G = sum(q_lens), H // KV
+    q = torch.randn(n, H * d, generator=g).to(torch.bfloat16)
+    want = attn_reference(paged, q.view(n, H, d), seq_lens, q_lens, 1 / math.sqrt(d), window or None).reshape(n, H * d)
+    cu = torch.tensor([0] + list(torch.tensor(q_lens).cumsum(0)), dtype=torch.int32).to(DEV)
+    ctx = torch.tensor(seq_lens, dtype=torch.int32).to(DEV)
+    per = ops().prefill_rows_per_item(torch.bfloat16, d, 16)
+    assert ops().prefill_takes_pairs(torch.bfloat16, d, 16) and per == 64
+    planned = prefill_work_rows(q_lens, range(4), G, per, [s - m for s, m in zip(seq_lens, q_lens)], pairs=True)
+    assert sorted((b, i) for b, hi, lo in planned for i in (hi, lo) if i >= 0) == [
+        (b, i) for b, m in enumerate(q_lens) for i in range(-(-m * G // per))]
+    apart = prefill_work(q_lens, G, torch.bfloat16, d, 16).tolist()
+    alone = [(b, i, -1) if i % 2 else (b, -1, i) for b, m in enumerate(q_lens) for i in range(-(-m * G // per))]
+    got = []
+    for work in (planned, apart, alone + [(0, -1, -1)]):
+        out = torch.full((n, H * d), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops().attn_prefill(q.to(DEV), paged.k.to(DEV), paged.v.to(DEV), paged.table.to(DEV), cu, ctx,
+                           torch.tensor(work, dtype=torch.int32, device=DEV), out, H, KV, d, 1 / math.sqrt(d), window,
+                           rows_per_item=per)
+        torch.testing.assert_close(out.float().cpu(), want, **tol(torch.bfloat16))
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
 def test_prefill_kernel_says_how_many_workgroups_a_compute_unit_holds():
     """What the planner of query runs weighs rows per item against: asked of the runtime for the
     kernel that would run, at least one, never more with two row tiles than with one; sizes the
