@@ -475,14 +475,22 @@ __global__ __launch_bounds__(KVF_WAVE) void mlstm_gates_kernel(const float* __re
   const int t0 = cu_q[seq], t1 = cu_q[seq + 1];
   float* st = state + (static_cast<size_t>(slot) * a.H + head) * (static_cast<size_t>(a.dk) * a.dv + a.dk + 1);
   float m_c = positions[t0] == 0 ? 0.f : st[static_cast<size_t>(a.dk) * a.dv + a.dk];
+  // a chunk's gates are asked for while the chunk before is worked on: each would else wait for its own
+  // trip to memory (21 chunks 31 us, 29 now: the scans over the wave are the rest)
+  const float bias_i = bias_if[head], bias_f = bias_if[a.H + head];
+  float next_i, next_f;
+  auto ask = [&](int token) {
+    const float* z = zif + static_cast<size_t>(min(token, t1 - 1)) * a.gate_stride;
+    next_i = z[head];
+    next_f = z[a.H + head];
+  };
+  ask(t0 + lane);
   for (int j = 0; j < nc; ++j) {
     const int tb = t0 + j * CL, cnt = min(CL, t1 - tb), t = lane;
-    float i_gate = 0.f, f_gate = 0.f;
-    if (t < cnt) {
-      const float* z = zif + static_cast<size_t>(tb + t) * a.gate_stride;
-      i_gate = capped(z[head] + bias_if[head], a.cap);
-      f_gate = log_sigmoid(capped(z[a.H + head] + bias_if[a.H + head], a.cap));
-    }
+    const float z_i = next_i, z_f = next_f;
+    ask(tb + CL + lane);
+    const float i_gate = t < cnt ? capped(z_i + bias_i, a.cap) : 0.f;
+    const float f_gate = t < cnt ? log_sigmoid(capped(z_f + bias_f, a.cap)) : 0.f;
     double b = static_cast<double>(f_gate);
 #pragma unroll
     for (int o = 1; o < KVF_WAVE; o <<= 1) {
@@ -514,66 +522,60 @@ __global__ __launch_bounds__(KVF_WAVE) void mlstm_gates_kernel(const float* __re
   if (lane == 0) st[static_cast<size_t>(a.dk) * a.dv + a.dk] = m_c;
 }
 
-// K (token-major) and the block's columns of V (column-major) of one chunk into LDS, as the
-// chunk kernel keeps them; rows past the chunk's tokens and elements past dk, dv are zero.
-template <typename T, int DKP, int CL>
-__device__ __forceinline__ void stage_kv(const T* __restrict__ qkv, const ScanArgs& a, int head, int tb, int cnt,
-                                         int col0, float* Qs, float* Ks, float* Vt, bool vec8) {
-  constexpr int QLD = DKP + 4, VLD = CL + 4;
-  const int tid = threadIdx.x, dk = a.dk, dv = a.dv;
-  if (vec8) {
-    for (int i = tid; i < CL * (DKP / 8); i += blockDim.x) {
-      const int t = i / (DKP / 8), e = 8 * (i - t * (DKP / 8));
-      float qv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, kv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (t < cnt && e < dk) {
-        const T* row = qkv + static_cast<size_t>(tb + t) * a.row_len;
-        if (Qs) load8(row + a.q_off + head * dk + e, qv);
-        load8(row + a.k_off + head * dk + e, kv);
-      }
-#pragma unroll
-      for (int x = 0; x < 8; ++x) {
-        if (Qs) Qs[t * QLD + e + x] = qv[x] * a.q_scale;
-        Ks[t * QLD + e + x] = kv[x];
-      }
-    }
+// What the matrix instructions take is read straight from memory, four elements a lane at a time: the
+// working set of a (chunk, head) is a few times 32 KB that the waves and the workgroups of its column blocks find in
+// their caches.  (Staged in LDS it filled 114 KB, one workgroup a compute unit whose four waves waited for
+// every load in turn.)
+constexpr int PCOLS = 64;    // columns of S a workgroup of the passes takes
+
+__device__ __forceinline__ f32x4 load4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 load4(const bf16_t* p) {
+  const uint2 r = *reinterpret_cast<const uint2*>(p);
+  return f32x4{__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u), __uint_as_float(r.y << 16),
+               __uint_as_float(r.y & 0xffff0000u)};
+}
+// elements e .. e + 3 of a row of dk; zeros past its end.  `quads`: rows start on four elements and dk is a
+// multiple of four.
+template <typename T>
+__device__ __forceinline__ f32x4 row4(const T* row, int e, int dk, bool quads) {
+  f32x4 v;
+  if (quads) {
+    v = load4(row + min(e, dk - 4));
   } else {
-    for (int i = tid; i < CL * DKP; i += blockDim.x) {
-      const int t = i / DKP, e = i - t * DKP;
-      float qv = 0.f, kv = 0.f;
-      if (t < cnt && e < dk) {
-        const T* row = qkv + static_cast<size_t>(tb + t) * a.row_len;
-        if (Qs) qv = Elem<T>::load(row + a.q_off + head * dk + e) * a.q_scale;
-        kv = Elem<T>::load(row + a.k_off + head * dk + e);
-      }
-      if (Qs) Qs[t * QLD + e] = qv;
-      Ks[t * QLD + e] = kv;
-    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = Elem<T>::load(row + min(e + i, dk - 1));
   }
-  for (int i = tid; i < CL * CCOLS; i += blockDim.x) {
-    const int t = i / CCOLS, cl = i % CCOLS, c = col0 + cl;
-    Vt[cl * VLD + t] = (t < cnt && c < dv)
-                           ? Elem<T>::load(qkv + static_cast<size_t>(tb + t) * a.row_len + a.v_off + head * dv + c)
-                           : 0.f;
-  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = e + i < dk ? v[i] : 0.f;
+  return v;
+}
+template <typename T> __device__ __forceinline__ bool rows_of_quads(const T* qkv, const ScanArgs& a) {
+  return a.dk % 4 == 0 && a.row_len % 4 == 0 && a.q_off % 4 == 0 && a.k_off % 4 == 0 &&
+         reinterpret_cast<uintptr_t>(qkv) % (4 * sizeof(T)) == 0;
+}
+// four neighbouring tokens' elements at one column; tokens past the chunk's last read the last
+template <typename T>
+__device__ __forceinline__ f32x4 column4(const T* first, int token, int last, int row_len) {
+  f32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = Elem<T>::load(first + static_cast<size_t>(min(token + i, last)) * row_len);
+  return v;
 }
 
+// U = K^T diag(D[L]) V (30 us at the sizes given at mlstm_output_kernel, 37 before): a wave takes 16 columns,
+// its share of V (weighted, zero past the chunk's tokens) stays in registers, and K comes in 16 of its
+// columns at a time.  Bound by the trips of those tiles to memory and the 17 MB of sums it writes.
 template <typename T, int DKP, int CL>
 __global__ __launch_bounds__(256) void mlstm_local_kernel(const T* __restrict__ qkv, const int* __restrict__ slot_ids,
                                                           ScanArgs a, MultiArgs w) {
-  extern __shared__ __align__(16) float lds[];
-  constexpr int QLD = DKP + 4, VLD = CL + 4;
-  float* Ks = lds;                 // [CL][QLD]
-  float* Vt = Ks + CL * QLD;       // [CCOLS][VLD]
-  float* wl = Vt + CCOLS * VLD;    // [CL]
-  const int chunk = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * CCOLS;
+  __shared__ __align__(16) float wl[CL];
+  const int chunk = blockIdx.z, head = blockIdx.y;
   const int seq = w.chunks[4 * chunk], tb = w.chunks[4 * chunk + 1], cnt = w.chunks[4 * chunk + 2];
   const int slot = slot_ids[seq];
   if (slot < 0 || slot >= a.n_slots) return;
   const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE, l16 = lane % 16, lq = lane / 16;
-  const int dk = a.dk, dv = a.dv;
-  const bool vec8 = dk % 8 == 0 && a.row_len % 8 == 0 && a.k_off % 8 == 0 &&
-                    reinterpret_cast<uintptr_t>(qkv) % (8 * sizeof(T)) == 0;
-  stage_kv<T, DKP, CL>(qkv, a, head, tb, cnt, col0, nullptr, Ks, Vt, vec8);
+  const int dk = a.dk, dv = a.dv, c = blockIdx.x * PCOLS + 16 * wave + l16;
+  const T* rows = qkv + static_cast<size_t>(tb) * a.row_len;
   if (tid < CL) {
     float v = 0.f;
     if (tid < cnt) {
@@ -582,20 +584,29 @@ __global__ __launch_bounds__(256) void mlstm_local_kernel(const T* __restrict__ 
     }
     wl[tid] = v;
   }
-  __syncthreads();
-  float* U = w.W + (static_cast<size_t>(chunk) * a.H + head) * dk * dv;
-  for (int tile = wave; tile < (DKP / 16) * (CCOLS / 16); tile += 4) {
-    const int kt = tile / (CCOLS / 16), ct = tile - kt * (CCOLS / 16);
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float* ka = Ks + (4 * lq) * QLD + 16 * kt + l16;
-    const float* vb = Vt + (16 * ct + l16) * VLD + 4 * lq;
-#pragma unroll 2
-    for (int k0 = 0; k0 < CL; k0 += 16) {
-      const f32x4 b4 = *reinterpret_cast<const f32x4*>(vb + k0) * *reinterpret_cast<const f32x4*>(wl + k0 + 4 * lq);
+  const T* v_at = rows + a.v_off + head * dv + min(c, dv - 1);
+  f32x4 vw[CL / 16];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[(k0 + e) * QLD], b4[e], acc, 0, 0, 0);
+  for (int i = 0; i < CL / 16; ++i) {
+    const f32x4 v = column4(v_at, 16 * i + 4 * lq, cnt - 1, a.row_len);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) vw[i][e] = 16 * i + 4 * lq + e < cnt ? v[e] : 0.f;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < CL / 16; ++i) vw[i] *= *reinterpret_cast<const f32x4*>(wl + 16 * i + 4 * lq);
+  float* U = w.W + (static_cast<size_t>(chunk) * a.H + head) * dk * dv;
+#pragma unroll 2
+  for (int kt = 0; kt < DKP / 16; ++kt) {
+    const T* k_at = rows + a.k_off + head * dk + min(16 * kt + l16, dk - 1);
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < CL / 16; ++i) {
+      const f32x4 k4 = column4(k_at, 16 * i + 4 * lq, cnt - 1, a.row_len);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(16 * i + 4 * lq + e < cnt ? k4[e] : 0.f, vw[i][e], acc, 0, 0, 0);
     }
-    const int c = col0 + 16 * ct + l16;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int k = 16 * kt + 4 * lq + v;
@@ -606,7 +617,9 @@ __global__ __launch_bounds__(256) void mlstm_local_kernel(const T* __restrict__ 
     float* u = w.un + (static_cast<size_t>(chunk) * a.H + head) * dk;
     for (int k = tid; k < dk; k += blockDim.x) {
       float nk = 0.f;
-      for (int s2 = 0; s2 < cnt; ++s2) nk = fmaf(wl[s2], Ks[s2 * QLD + k], nk);
+#pragma unroll 8
+      for (int s2 = 0; s2 < cnt; ++s2)
+        nk = fmaf(wl[s2], Elem<T>::load(rows + static_cast<size_t>(s2) * a.row_len + a.k_off + head * dk + k), nk);
       u[k] = nk;
     }
   }
@@ -635,157 +648,155 @@ __global__ __launch_bounds__(256) void mlstm_carry_kernel(const int* __restrict_
   st[e] = S;
 }
 
+// A = (Q K^T) * D, O = A V + diag(g) Q S_c: a wave owns 16 tokens of the chunk (two waves share them where a
+// chunk has two such tiles only, each every other tile of columns).  Its q rows stay in registers, its rows
+// of A pass through LDS once, from the layout of sums to that of operands, and a tile of 16 columns of V
+// and S_c feeds them.  1,301 and 741 tokens, 8 heads of 128 x 256: 82 us where workgroups of 32 columns
+// that staged everything in LDS took 198.  What bounds it now: four trips to memory in a row a wave (q, the tiles of
+// k, the tiles of columns) at two waves a SIMD, which the registers of q and of 16 columns leave.  Measured
+// and left: S by columns and V through LDS, a quarter of the load instructions, 5 us more; addresses
+// without clamps for whole chunks 14 more; a tile of columns ahead 12; registers for four waves a SIMD spill, 46.
 template <typename T, int DKP, int CL>
 __global__ __launch_bounds__(256) void mlstm_output_kernel(const T* __restrict__ qkv, const int* __restrict__ slot_ids,
                                                            float* __restrict__ out, ScanArgs a, MultiArgs w) {
-  extern __shared__ __align__(16) float lds[];
-  constexpr int QLD = DKP + 4, ALD = CL + 4, VLD = CL + 4, SLD = DKP + 4;
-  double* bc = reinterpret_cast<double*>(lds);   // [CL]
-  float* Qs = lds + 2 * CL;
-  float* Ks = Qs + CL * QLD;
-  float* Vt = Ks + CL * QLD;
-  float* As = Vt + CCOLS * VLD;
-  float* St = As + CL * ALD;
-  float* ns = St + CCOLS * SLD;
-  float* li = ns + DKP;
-  float* mt = li + CL;
-  float* gt = mt + CL;
-  float* den = gt + CL;
-  float* part = den + CL;   // [256 / CL][CL]
-  const int chunk = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * CCOLS;
+  constexpr int RT = CL / 16, WPR = 4 / RT, KQ = DKP / 16, ALD = CL + 4, SH = 256 / CL;
+  static_assert(SH % 4 == 0, "a lane takes whole shares");
+  __shared__ double bc[CL];
+  __shared__ float li[CL], mt[CL], gt[CL];
+  __shared__ __align__(16) float As[4][16][ALD];
+  const int chunk = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * PCOLS;
   const int seq = w.chunks[4 * chunk], tb = w.chunks[4 * chunk + 1], cnt = w.chunks[4 * chunk + 2];
-  const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE, l16 = lane % 16, lq = lane / 16;
-  const int dk = a.dk, dv = a.dv;
+  const int tid = threadIdx.x, lane = tid % KVF_WAVE, l16 = lane % 16, lq = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / KVF_WAVE), rt = wave / WPR;
+  const int dk = a.dk, dv = a.dv, last = cnt - 1;
   const int slot = slot_ids[seq];
   if (slot < 0 || slot >= a.n_slots) {
-    for (int i = tid; i < cnt * CCOLS; i += blockDim.x) {
-      const int t = i / CCOLS, c = col0 + i % CCOLS;
+    for (int i = tid; i < cnt * PCOLS; i += blockDim.x) {
+      const int t = i / PCOLS, c = col0 + i % PCOLS;
       if (c < dv) out[static_cast<size_t>(tb + t) * a.H * dv + head * dv + c] = 0.f;
     }
     return;
   }
-  const bool vec8 = dk % 8 == 0 && a.row_len % 8 == 0 && a.q_off % 8 == 0 && a.k_off % 8 == 0 &&
-                    reinterpret_cast<uintptr_t>(qkv) % (8 * sizeof(T)) == 0;
-  stage_kv<T, DKP, CL>(qkv, a, head, tb, cnt, col0, Qs, Ks, Vt, vec8);
+  const bool quads = rows_of_quads(qkv, a);
   const size_t ch = static_cast<size_t>(chunk) * a.H + head;
-  const float* Sc = w.W + ch * dk * dv;
-  for (int i = tid; i < DKP * CCOLS; i += blockDim.x) {
-    const int r = i / CCOLS, cl = i % CCOLS, c = col0 + cl;
-    St[cl * SLD + r] = (r < dk && c < dv) ? Sc[static_cast<size_t>(r) * dv + c] : 0.f;
-  }
-  for (int r = tid; r < DKP; r += blockDim.x) ns[r] = r < dk ? w.un[ch * dk + r] : 0.f;
-  const int last = cnt - 1;
+  const T* rows = qkv + static_cast<size_t>(tb) * a.row_len;
   if (tid < CL) {
-    const int t = min(tid, last);
-    const size_t at = static_cast<size_t>(tb + t) * a.H + head;
+    const size_t at = static_cast<size_t>(tb + min(tid, last)) * a.H + head;
     const float m_c = w.mc[ch];
     li[tid] = w.li[at];
     bc[tid] = w.bc[at];
     mt[tid] = w.mt[at];
     gt[tid] = tid < cnt ? expf(static_cast<float>(w.bc[at] + static_cast<double>(m_c) - static_cast<double>(w.mt[at]))) : 0.f;
   }
-  __syncthreads();
-  constexpr int RT = CL / 16;
-  for (int tile = wave; tile < RT * RT; tile += 4) {
-    const int rt = tile / RT, ct = tile - rt * RT;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (ct <= rt) {
-      const float* qa = Qs + (16 * rt + l16) * QLD + 4 * lq;
-      const float* kb = Ks + (16 * ct + l16) * QLD + 4 * lq;
-#pragma unroll 4
-      for (int k0 = 0; k0 < DKP; k0 += 16) {
-        const f32x4 a4 = *reinterpret_cast<const f32x4*>(qa + k0), b4 = *reinterpret_cast<const f32x4*>(kb + k0);
+  const T* q_row = rows + static_cast<size_t>(min(16 * rt + l16, last)) * a.row_len + a.q_off + head * dk;
+  const float* n_c = w.un + ch * dk;
+  f32x4 q[KQ];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], b4[e], acc, 0, 0, 0);
+  for (int i = 0; i < KQ; ++i) q[i] = row4(q_row, 16 * i + 4 * lq, dk, quads) * a.q_scale;
+  // a row's sums, of q n and of A, are taken in SH strided shares, SH / 4 of them a lane: the order of the
+  // chunk kernel's (8 us more than sums as the registers hold them, and the same bits from both routes)
+  float nq[SH / 4];
+#pragma unroll
+  for (int x = 0; x < SH / 4; ++x) nq[x] = 0.f;
+#pragma unroll
+  for (int i0 = 0; i0 < KQ; i0 += RT) {
+#pragma unroll
+    for (int i = 0; i < RT && i0 + i < KQ; ++i) *reinterpret_cast<f32x4*>(&As[wave][l16][16 * i + 4 * lq]) = q[i0 + i];
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < SH / 4; ++x)
+#pragma unroll
+      for (int k = lq + 4 * x; k < min(CL, DKP - 16 * i0); k += SH) {
+        const int at = 16 * i0 + k;
+        const float n = n_c[min(at, dk - 1)];
+        nq[x] = fmaf(As[wave][l16][k], at < dk ? n : 0.f, nq[x]);
       }
+    __syncthreads();
+  }
+  for (int ct = 0; ct <= rt; ++ct) {
+    const T* k_row = rows + static_cast<size_t>(min(16 * ct + l16, last)) * a.row_len + a.k_off + head * dk;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) {
+      const f32x4 k4 = row4(k_row, 16 * i + 4 * lq, dk, quads);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i][e], k4[e], acc, 0, 0, 0);
     }
     const int s = 16 * ct + l16;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int t = 16 * rt + 4 * lq + v;
       const bool vis = s <= t && t < cnt;
-      As[t * ALD + s] = vis ? acc[v] * expf(static_cast<float>(bc[t] - bc[s]) + li[s] - mt[t]) : 0.f;
+      As[wave][4 * lq + v][s] = vis ? acc[v] * expf(static_cast<float>(bc[t] - bc[s]) + li[s] - mt[t]) : 0.f;
     }
   }
-  __syncthreads();
-  {
-    const int t = tid % CL, share = tid / CL;
-    constexpr int SH = 256 / CL;
+  __syncthreads();   // (a wave reads its own rows of A alone)
+  const float g = gt[16 * rt + l16];
+#pragma unroll
+  for (int x = 0; x < SH / 4; ++x) {
     float sum = 0.f;
-    for (int s2 = share; s2 < CL; s2 += SH) sum += As[t * ALD + s2];
-    float dot = 0.f;
-    for (int k = share; k < DKP; k += SH) dot = fmaf(Qs[t * QLD + k], ns[k], dot);
-    part[share * CL + t] = fmaf(gt[t], dot, sum);
+    for (int s = lq + 4 * x; s < 16 * (rt + 1); s += SH) sum += As[wave][l16][s];
+    nq[x] = fmaf(g, nq[x], sum);
   }
-  __syncthreads();
-  if (tid < CL) {
-    constexpr int SH = 256 / CL;
-    float nq = 0.f;
-    for (int sh = 0; sh < SH; ++sh) nq += part[sh * CL + tid];
-    den[tid] = fmaxf(fabsf(nq), expf(-mt[tid])) + 1e-6f;
-  }
-  __syncthreads();
-  for (int tile = wave; tile < RT * (CCOLS / 16); tile += 4) {
-    const int rt = tile / (CCOLS / 16), ct = tile - rt * (CCOLS / 16);
+  float whole = 0.f;
+#pragma unroll
+  for (int sh = 0; sh < SH; ++sh) whole += __shfl(nq[sh / 4], l16 + 16 * (sh % 4), KVF_WAVE);
+  whole = fmaxf(fabsf(whole), expf(-mt[16 * rt + l16])) + 1e-6f;
+  float den[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) den[v] = __shfl(whole, 4 * lq + v, KVF_WAVE);
+  f32x4 af[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) af[i] = *reinterpret_cast<const f32x4*>(&As[wave][l16][16 * min(i, rt) + 4 * lq]);
+#pragma unroll
+  for (int i = 0; i < KQ; ++i) q[i] *= g;
+  if (16 * rt >= cnt) return;
+  const float* Sc = w.W + ch * dk * dv;
+  for (int ct = wave % WPR; ct < PCOLS / 16; ct += WPR) {
+    const int c = col0 + 16 * ct + l16, cc = min(c, dv - 1);
+    const T* v_at = rows + a.v_off + head * dv + cc;
+    const float* s_at = Sc + cc;
+    f32x4 sv[KQ];
+#pragma unroll
+    for (int i = 0; i < KQ; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sv[i][e] = s_at[static_cast<size_t>(min(16 * i + 4 * lq + e, dk - 1)) * dv];
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float* aa = As + (16 * rt + l16) * ALD + 4 * lq;
-    const float* vb = Vt + (16 * ct + l16) * VLD + 4 * lq;
-    for (int k0 = 0; k0 < 16 * (rt + 1); k0 += 16) {
-      const f32x4 a4 = *reinterpret_cast<const f32x4*>(aa + k0), b4 = *reinterpret_cast<const f32x4*>(vb + k0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], b4[e], acc, 0, 0, 0);
-    }
-    const float g = gt[16 * rt + l16];
-    const float* qa = Qs + (16 * rt + l16) * QLD + 4 * lq;
-    const float* sb = St + (16 * ct + l16) * SLD + 4 * lq;
-#pragma unroll 4
-    for (int k0 = 0; k0 < DKP; k0 += 16) {
-      const f32x4 a4 = *reinterpret_cast<const f32x4*>(qa + k0) * g, b4 = *reinterpret_cast<const f32x4*>(sb + k0);
+    for (int i = 0; i < RT; ++i) {
+      if (i > rt) break;
+      const int t = 16 * i + 4 * lq;
+      const f32x4 v4 = column4(v_at, t, last, a.row_len);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], b4[e], acc, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][e], t + e < cnt ? v4[e] : 0.f, acc, 0, 0, 0);
     }
-    const int c = col0 + 16 * ct + l16;
+#pragma unroll
+    for (int i = 0; i < KQ; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i][e], 16 * i + 4 * lq + e < dk ? sv[i][e] : 0.f, acc, 0, 0, 0);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int t = 16 * rt + 4 * lq + v;
-      if (t < cnt && c < dv) out[static_cast<size_t>(tb + t) * a.H * dv + head * dv + c] = acc[v] / den[t];
+      if (t < cnt && c < dv) out[static_cast<size_t>(tb + t) * a.H * dv + head * dv + c] = acc[v] / den[v];
     }
   }
-}
-
-template <int DKP, int CL> constexpr size_t output_lds() {
-  return sizeof(float) * (2 * CL + 2 * CL * (DKP + 4) + CCOLS * (CL + 4) + CL * (CL + 4) + CCOLS * (DKP + 4) + DKP +
-                          4 * CL + 256);
-}
-template <int DKP, int CL> constexpr size_t local_lds() {
-  return sizeof(float) * (CL * (DKP + 4) + CCOLS * (CL + 4) + CL);
 }
 
 template <typename T, int DKP, int CL>
 int multi_go(const void* qkv, const float* zif, const float* bias_if, const int* cu_q, const int* positions,
              const int* slot_ids, float* state, float* out, int n_chunks, int n_runs, ScanArgs a, MultiArgs w,
              hipStream_t s) {
-  static bool allowed = false;
-  if (!allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&mlstm_output_kernel<T, DKP, CL>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(output_lds<DKP, CL>()));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&mlstm_local_kernel<T, DKP, CL>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(local_lds<DKP, CL>()));
-    if (e != hipSuccess) return static_cast<int>(e);
-    allowed = true;
-  }
   const T* rows = static_cast<const T*>(qkv);
-  constexpr size_t lds_local = local_lds<DKP, CL>(), lds_output = output_lds<DKP, CL>();
-  const int slices = (a.dv + CCOLS - 1) / CCOLS;
+  const int slices = (a.dv + PCOLS - 1) / PCOLS;
   hipLaunchKernelGGL(mlstm_gates_kernel<CL>, dim3(a.H, n_runs), dim3(KVF_WAVE), 0, s, zif, bias_if, cu_q, positions,
                      slot_ids, state, a, w);
-  hipLaunchKernelGGL((mlstm_local_kernel<T, DKP, CL>), dim3(slices, a.H, n_chunks), dim3(256), lds_local, s,
+  hipLaunchKernelGGL((mlstm_local_kernel<T, DKP, CL>), dim3(slices, a.H, n_chunks), dim3(256), 0, s,
                      rows, slot_ids, a, w);
   const unsigned per_head = static_cast<unsigned>((static_cast<size_t>(a.dk) * a.dv + a.dk + 255) / 256);
   hipLaunchKernelGGL(mlstm_carry_kernel, dim3(per_head, a.H, n_runs), dim3(256), 0, s, cu_q, positions, slot_ids, state,
                      a, w);
-  hipLaunchKernelGGL((mlstm_output_kernel<T, DKP, CL>), dim3(slices, a.H, n_chunks), dim3(256), lds_output, s,
+  hipLaunchKernelGGL((mlstm_output_kernel<T, DKP, CL>), dim3(slices, a.H, n_chunks), dim3(256), 0, s,
                      rows, slot_ids, out, a, w);
   return kvf_last_error();
 }

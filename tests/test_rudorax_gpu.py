@@ -287,6 +287,33 @@ def test_matrix_memory_with_all_chunks_at_once(dtype, H, dk, dv):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 65), (1, 64, 256), (3, 37, 31), (1, 4, 17), (1, 255, 64)])
+@pytest.mark.parametrize("n", [64, 65, 128, 143, 192])
+def test_matrix_memory_passes_at_the_edges_of_their_tiles(dtype, H, dk, dv, n):
+    """The passes over all chunks on one run: chunks that are whole, hold one token or end inside a tile; heads
+    that fill the kernels' size, are no multiple of four and hence read element by element, or are
+    smaller than a tile; columns that end inside a tile and inside a workgroup's."""
+    cap, cols = 12.0, 2 * H * dk + H * dv
+    rows, z = rand(n, cols, seed=n + dk).to(dtype), rand(n, 2 * H, seed=n, scale=3.0)
+    bias = torch.cat([torch.full((H,), -1.0), torch.full((H,), 4.0)])
+    x = rows.float()
+    want = scan_reference(x[:, :H * dk], x[:, H * dk:2 * H * dk], x[:, 2 * H * dk:], z[:, :H], z[:, H:], bias, cap, H, dk, dv)
+    chunks, runs = ops().mlstm_multi_plan([n], dk, 1)
+    multi = {"chunks": i32(chunks).view(-1, 4), "runs": i32(runs).view(-1, 3)}
+    for name, (shape, dt) in ops().mlstm_multi_scratch(n, len(chunks) // 4, H, dk, dv).items():
+        multi[name] = torch.full(shape, float("nan"), dtype=dt, device=DEV)
+    state = torch.full((2, ops().mlstm_state_floats(H, dk, dv)), 3.0, device=DEV)
+    by_token, short = state.clone(), torch.empty(n, H * dv, device=DEV)
+    out = torch.full((n, H * dv), 5.0, device=DEV)
+    args = (rows.to(DEV), z.to(DEV), bias.to(DEV), i32([0, n]), torch.arange(n).int().to(DEV), i32([1]))
+    tail = (1, H, dk, dv, 0, H * dk, 2 * H * dk, cap, dk ** -0.5)
+    ops().mlstm_scan(*args, state, out, *tail, chunk_from=1, multi_from=1, multi=multi)
+    ops().mlstm_scan(*args, by_token, short, *tail, chunk_from=1000)
+    torch.testing.assert_close(out.cpu(), want, atol=3e-4, rtol=3e-4)      # the bounds of the tests above
+    torch.testing.assert_close(state, by_token, atol=3e-4, rtol=3e-4)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_heads_normed_weighted_and_gated(dtype):
     H, dv, n, eps = 3, 40, 5, 1e-3
     raw, w = rand(n, H * dv, seed=1, scale=4.0), 1.0 + rand(H * dv, seed=2, scale=0.2)
