@@ -208,44 +208,6 @@ __device__ __forceinline__ PageRef page_of_key(const Pages& pg, const MArgs& a, 
   r.asked = key < pg.ctx && blk < a.table_stride;
   return r;
 }
-// Page that holds the keys of K tile t for this lane (row i = j16 is key kb + 8*(i/4) + 4*t + i%4)
-__device__ __forceinline__ PageRef k_page(const Pages& pg, const MArgs& a, int kb, int t) {
-  return page_of_key(pg, a, kb + 8 * (pg.j16 >> 2) + 4 * t + (pg.j16 & 3));
-}
-// Page of the keys kb + 8*kg + 0..7 (one page: the page size is a multiple of 8)
-__device__ __forceinline__ PageRef v_page(const Pages& pg, const MArgs& a, int kb) {
-  return page_of_key(pg, a, kb + 8 * pg.kg);
-}
-
-// K fragment of tile t, contraction step c, and how many of its eight elements count: none
-// without a page or where the step reaches past d (head sizes that are odd multiples of 16).
-// Offsets into the pages are counted in fragments of 16 bytes and fit 32 bits (the host checks).
-template <int DT>
-__device__ __forceinline__ uint4 k_fragment(const Pages& pg, const MArgs& a, int kb, int t, int c,
-                                            const PageRef& ref, int& live) {
-  const int key = kb + 8 * (pg.j16 >> 2) + 4 * t + (pg.j16 & 3);
-  const int slot = key - block_of(a, key) * a.bs;
-  const bool over = (DT % 2) && c == DT / 2 && pg.kg >= 2;
-  const bool ok = ref.ok(a.nb) && !over;
-  live = ok ? 8 : 0;
-  const unsigned row = (static_cast<unsigned>(ok ? ref.page : 0) * a.KV + pg.kvh) * a.bs + slot;
-  const unsigned off = row * (a.d / 8) + (over ? 0 : c * 4 + pg.kg);
-  return ld16(pg.k_pages + static_cast<size_t>(off) * 8);
-}
-// V^T fragment of element tile dt (row i = j16 is element dt*16 + i), slots are keys
-// kb + 8*kg + 0..7.  Keys at or past the context length hold whatever an earlier owner of the
-// page left there: they do not count.
-__device__ __forceinline__ uint4 v_fragment(const Pages& pg, const MArgs& a, int kb, int dt,
-                                            const PageRef& ref, int& live) {
-  const int key = kb + 8 * pg.kg;
-  const int slot = key - block_of(a, key) * a.bs;
-  const bool ok = ref.ok(a.nb);
-  live = ok ? min(pg.ctx - key, 8) : 0;
-  const unsigned row = (static_cast<unsigned>(ok ? ref.page : 0) * a.KV + pg.kvh) * a.d + dt * 16 + pg.j16;
-  const unsigned off = row * (a.bs / 8) + slot / 8;
-  return ld16(pg.vt_pages + static_cast<size_t>(off) * 8);
-}
-
 // The rows a lane works for: one per row tile.
 template <int RT> struct Rows {
   bool ok[RT];
@@ -694,9 +656,9 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
 }
 
 // ------------------------------------------------------------------------- few rows, split keys
-// TWO: a wave holds the fragments of two blocks, loading one while it consumes the other.
+// DEPTH 2: a wave holds the fragments of two blocks, loading one while it consumes the other.
 // NW: waves of the workgroup; more of them shorten each wave's walk over its cut of the keys.
-template <int DT, bool TWO, int NW, int BIAS, bool SINK>
+template <int DT, int DEPTH, int NW, int BIAS, bool SINK>
 __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfma_split_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
     const bf16_t* __restrict__ vt_pages, const int* __restrict__ block_table,
@@ -769,34 +731,76 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
   // scratch); the pages of a block are looked up one block before its fragments are loaded.
   struct Raw {
     uint4 k[2][DC], v[DT];
-    int kl[2][DC], vl;
+    bool k_ok[2], v_ok;
   };
-  Raw A, B;
-  PageRef pA[3], pB[3];
-  auto locate = [&](int kb, PageRef (&p)[3]) {
-    kb = wk.at(kb);
-    p[0] = k_page(pg, a, kb, 0);
-    p[1] = k_page(pg, a, kb, 1);
-    p[2] = v_page(pg, a, kb);
+  // a page lookup, and where in the page the lane's first fragment lies: of the key of K tile t (row
+  // i = j16 is key kb + 8*(i/4) + 4*t + i%4), or of V^T (row i is element i, slots are keys kb + 8*kg + 0..7:
+  // one page, whose size is a multiple of 8).  Offsets count fragments of 16 bytes and fit 32 bits, a page's
+  // size in fragments 24 (the host checks).
+  struct Spot {
+    PageRef page;
+    unsigned off;
   };
-  auto fetch = [&](int kb, const PageRef (&p)[3], Raw& r) {
+  Raw R[DEPTH];
+  Spot P[DEPTH][3];
+  const unsigned page_size = static_cast<unsigned>(a.KV) * a.bs * (D / 8);
+  const unsigned k_lane = static_cast<unsigned>(kvh) * a.bs * (D / 8) + kg;
+  const unsigned v_lane = (static_cast<unsigned>(kvh) * D + j16) * (a.bs / 8);
+  const int k_key = 8 * (j16 >> 2) + (j16 & 3);
+  auto locate = [&](int kb, Spot (&p)[3]) {
     kb = wk.at(kb);
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int i = 0; i < 3; ++i) {
+      const int key = kb + (i < 2 ? k_key + 4 * i : 8 * kg);
+      const unsigned slot = static_cast<unsigned>(key - block_of(a, key) * a.bs);
+      p[i].page = page_of_key(pg, a, key);
+      p[i].off = i < 2 ? k_lane + __umul24(slot, D / 8) : v_lane + (slot >> 3);
+    }
+  };
+  // a lane without a page reads page 0; its keys do not count
+  auto address = [&](const bf16_t* pages, const Spot& at, bool& ok) {
+    ok = at.page.ok(a.nb);
+    return pages + static_cast<size_t>(__umul24(ok ? at.page.page : 0, page_size) + at.off) * 8;
+  };
+  const bool over = DT % 2 != 0 && kg >= 2;   // of the last step along d, where it reaches past d
+  auto fetch = [&](const Spot (&p)[3], Raw& r) {
 #pragma unroll
-      for (int c = 0; c < DC; ++c) r.k[t][c] = k_fragment<DT>(pg, a, kb, t, c, p[t], r.kl[t][c]);
+    for (int t = 0; t < 2; ++t) {
+      const bf16_t* k = address(k_pages, p[t], r.k_ok[t]);
 #pragma unroll
-    for (int t = 0; t < DT; ++t) r.v[t] = v_fragment(pg, a, kb, t, p[2], r.vl);
+      for (int c = 0; c < DC; ++c)
+        r.k[t][c] = ld16(DT % 2 != 0 && c == DC - 1 ? k + (over ? 0 : 32 * c) : k + 32 * c);
+    }
+    const bf16_t* v = address(vt_pages, p[2], r.v_ok);
+#pragma unroll
+    for (int t = 0; t < DT; ++t, v += 16 * a.bs) r.v[t] = ld16(v);
   };
   auto consume = [&](int kb, const Raw& r) {
     kb = wk.at(kb);
+    Raw w = r;
+    if (DT % 2 != 0) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        w.k[t][DC - 1] = make_uint4(over ? 0 : r.k[t][DC - 1].x, over ? 0 : r.k[t][DC - 1].y,
+                                    over ? 0 : r.k[t][DC - 1].z, over ? 0 : r.k[t][DC - 1].w);
+    }
+    // Keys without a page do not count, nor do those at or past the context length, which hold whatever an
+    // earlier owner of the page left there.  Nearly every block is whole: one question for all its fragments.
+    if (kb + 32 > ctx || __any(!(r.k_ok[0] && r.k_ok[1] && r.v_ok))) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < DC; ++c) w.k[t][c] = keep_first(w.k[t][c], r.k_ok[t] ? 8 : 0);
+#pragma unroll
+      for (int t = 0; t < DT; ++t) w.v[t] = keep_first(w.v[t], r.v_ok ? min(ctx - kb - 8 * kg, 8) : 0);
+    }
     bf16x8 kf[2][DC], vf[DT];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int c = 0; c < DC; ++c) kf[t][c] = as_frag(keep_first(r.k[t][c], r.kl[t][c]));
+      for (int c = 0; c < DC; ++c) kf[t][c] = as_frag(w.k[t][c]);
 #pragma unroll
-    for (int t = 0; t < DT; ++t) vf[t] = as_frag(keep_first(r.v[t], r.vl));
+    for (int t = 0; t < DT; ++t) vf[t] = as_frag(w.v[t]);
     const bool edge = kb + 31 > pos_min || kb + 32 > ctx || a.window != 0;
     block_update<DT, 1, BIAS>(kf, [&](int t) { return vf[t]; }, qf, rows, kb, kg, edge, scale2, m_ref, l_run, acc, a.cap, dist, pos_min);
   };
@@ -804,37 +808,41 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
   // query and the context length, not after them: one round trip to memory less.
   const bool early = a.window == 0;
   if (early) {
-    locate(turn, pA);
-    if (TWO) locate(turn + STEP, pB);
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) locate(turn + i * STEP, P[i]);
   }
   // the query fragments have to be there before the loops (see the note in the runs kernel)
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  if (TWO) {
-    if (kb_begin < kb_end) {
-      if (!early) {
-        locate(kb_begin, pA);
-        locate(kb_begin + STEP, pB);
+  constexpr int AHEAD = DEPTH - 1;
+  if (kb_begin < kb_end) {
+    // A stage looks up the pages of the block DEPTH ahead, then asks for the fragments of the one before
+    // it, whose pages were looked up before the last fragments were asked for: the load counter runs in
+    // order, and no wait drains what was asked for after what it waits for.  For the same reason no load
+    // sits in a branch; past its last block a wave asks for its first again, and the blocks that nothing
+    // follows are taken behind the loop.
+    auto in = [&](int kb) { return kb < kb_end ? kb : kb_begin; };
+    if (!early) {
+#pragma unroll
+      for (int i = 0; i < DEPTH; ++i) locate(in(kb_begin + i * STEP), P[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) fetch(P[i], R[i]);
+    int kb = kb_begin;
+    for (; kb + AHEAD * STEP < kb_end; kb += DEPTH * STEP) {
+#pragma unroll
+      for (int i = 0; i < DEPTH; ++i) {
+        if (DEPTH > 1) locate(in(kb + (i + DEPTH) * STEP), P[i]);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(P[(i + AHEAD) % DEPTH], R[(i + AHEAD) % DEPTH]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (DEPTH == 1) locate(in(kb + STEP), P[i]);
+        consume(kb + i * STEP, R[i]);
       }
-      fetch(kb_begin, pA, A);
     }
-    for (int kb = kb_begin; kb < kb_end; kb += 2 * STEP) {
-      const bool second = kb + STEP < kb_end;
-      if (second) fetch(kb + STEP, pB, B);
-      locate(kb + 2 * STEP, pA);
-      consume(kb, A);
-      if (second) {
-        if (kb + 2 * STEP < kb_end) fetch(kb + 2 * STEP, pA, A);
-        locate(kb + 3 * STEP, pB);
-        consume(kb + STEP, B);
-      }
-    }
-  } else {
-    if (!early) locate(kb_begin, pA);
-    for (int kb = kb_begin; kb < kb_end; kb += STEP) {
-      fetch(kb, pA, A);
-      locate(kb + STEP, pA);
-      consume(kb, A);
-    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (kb + i * STEP < kb_end) consume(kb + i * STEP, R[i]);
   }
 
   // ---- merge the waves, then store or hand on the partial result
@@ -1038,13 +1046,22 @@ void launch_runs(int row_tiles, dim3 grid, hipStream_t s, const void* q, const v
   runs_shape<DT>(row_tiles, go);
 }
 
+// What bounds it: bytes where the workgroups are many and alike, else the longest wave's walk, a block at a
+// time.  32 heads over 8 kv heads, ragged contexts of 60 to 2,900 keys, before (lookups behind the fragments
+// they wait with, a branch round the loads, addresses and masks anew for each fragment) and after: 41
+// sequences of head size 64, 38.0 and 34.6 us (24 at the rate of a copy); of 128, 58.5 and 49.5; 128 sequences of
+// 128, 173 and 155; 256 of 64 with 128 keys each, 24.5 and 20.3.  Three blocks in flight at head sizes up to 64: 35.4
+// for the first, 24.9 for the last and 9.7 instead of 7.8 for 8 sequences of 600 keys, for 3 per cent at 64 and more long
+// sequences.
+constexpr int split_depth(int DT) { return DT <= 8 ? 2 : 1; }
+
 template <int DT, int NW>
 void launch_split_waves(dim3 grid, hipStream_t s, const void* q, const void* k_pages, const void* vt_pages,
                         const int* block_table, const int* seq_ids, const int* cu_q, const int* ctx_lens,
                         void* out, float* part_acc, float* part_ml, const MArgs& a) {
   const size_t lds = (static_cast<size_t>(NW) * DT * KVF_WAVE * 4 + NW * 16 * 2) * sizeof(float);
   if (a.cap > 0.f)
-    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, (DT <= 8), NW, 2, false>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, split_depth(DT), NW, 2, false>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, seq_ids, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), part_acc, part_ml, a);
@@ -1053,22 +1070,22 @@ void launch_split_waves(dim3 grid, hipStream_t s, const void* q, const void* k_p
     const int G = a.H / a.KV;
     const size_t table = static_cast<size_t>(G < 16 ? G : 16) * dist_row(a.n_dist) * sizeof(float);
     b.dist_lds = lds + table <= DIST_LDS_MOST;
-    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, (DT <= 8), NW, 4, false>), grid, dim3(NW * KVF_WAVE),
+    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, split_depth(DT), NW, 4, false>), grid, dim3(NW * KVF_WAVE),
                        b.dist_lds ? lds + table : lds, s, static_cast<const bf16_t*>(q),
                        static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(vt_pages), block_table, seq_ids,
                        cu_q, ctx_lens, static_cast<bf16_t*>(out), part_acc, part_ml, b);
   } else if (a.sinks)
-    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, (DT <= 8), NW, 0, true>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, split_depth(DT), NW, 0, true>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, seq_ids, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), part_acc, part_ml, a);
   else if (a.slopes)
-    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, (DT <= 8), NW, 1, false>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, split_depth(DT), NW, 1, false>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, seq_ids, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), part_acc, part_ml, a);
   else
-    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, (DT <= 8), NW, 0, false>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_split_kernel<DT, split_depth(DT), NW, 0, false>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, seq_ids, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), part_acc, part_ml, a);

@@ -883,6 +883,33 @@ def test_attn_decode(dtype, H, KV, d, bs, splits, window):
     assert (got[[0, 2, 3, 5]] == 5.0).all()
 
 
+@pytest.mark.parametrize("d,bs", [(16, 8), (64, 16), (80, 24), (112, 16), (128, 16), (144, 16), (256, 32)])
+@pytest.mark.parametrize("KV", [1, 16])
+@pytest.mark.parametrize("splits,window", [(1, 0), (2, 0), (1, 70), (2, 300)])
+def test_attn_decode_walks_of_few_and_odd_blocks(d, bs, KV, splits, window):
+    """Waves of four and of eight to a workgroup (by the grid) that find no block of keys, one, or an odd or
+    even number of them, the last cut short.  Whatever no sequence owns, in its last page and in the others, is NaN."""
+    dtype, G = torch.bfloat16, 3
+    seq_lens = [1, 31, 32, 33, 128, 129, 161, 255, 256, 257, 289, 384, 385, 500, 513, 640, 777, 1023]
+    n, H = len(seq_lens), G * KV
+    paged = Paged(seq_lens, KV, d, bs, dtype, seed=d + KV)
+    owned = torch.zeros(paged.nb, bs, dtype=torch.bool)
+    for s, m in enumerate(seq_lens):
+        for b in range(-(-m // bs)):
+            owned[paged.table[s, b], :min(bs, m - b * bs)] = True
+    k = paged.k.masked_fill(~owned[:, None, :, None], float("nan"))
+    v = paged.v.masked_fill(~owned[:, None, None, :], float("nan"))
+    q = torch.randn(n, H * d, generator=torch.Generator().manual_seed(d)).to(dtype)
+    scale = 1 / math.sqrt(d)
+    want = attn_reference(paged, q.view(n, H, d), seq_lens, [1] * n, scale, window or None).reshape(n, H * d)
+    ws = (torch.empty(n * H * splits * d, device=DEV), torch.empty(n * H * splits * 2, device=DEV))
+    out = torch.full((n, H * d), 7.0, dtype=dtype, device=DEV)
+    ops().attn_decode(q.to(DEV), k.to(DEV), v.to(DEV), paged.table.to(DEV), None, n,
+                      torch.arange(n + 1, dtype=torch.int32, device=DEV),
+                      torch.tensor(seq_lens, dtype=torch.int32, device=DEV), out, H, KV, d, scale, window, splits, ws)
+    torch.testing.assert_close(out.float().cpu(), want, **tol(dtype))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("splits", [1, 4])
 def test_attn_decode_clears_the_rows_of_empty_sequences(dtype, splits):
