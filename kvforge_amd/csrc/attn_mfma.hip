@@ -193,6 +193,13 @@ struct Pages {
   int kvh, ctx, j16, kg;
 };
 
+// The fragment of 16 bytes of a key's row (it has 2 DT of them) that lane group kg reads in step c along d.  The
+// last step of an odd DT reaches past the row: groups 2 and 3 read fragments 0 and 1 there, which are
+// cleared before they are used.
+template <int DT> constexpr int key_fragment(int c, int kg) {
+  return DT % 2 != 0 && c == DT / 2 && kg >= 2 ? kg - 2 : 4 * c + kg;
+}
+
 // A page lookup: the table entry as loaded, and whether the key it was asked for exists.  The
 // two are only combined where the page is used, so that nothing waits for the load before then;
 // the lookup is issued one block before the fragment loads that need it.
@@ -520,7 +527,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
       const int t = f / DC, c = f % DC;
       key_off[i] = 8 * (j16 >> 2) + 4 * t + (j16 & 3);
       whole[i] = !((DT % 2) && c == DT / 2 && kg >= 2);  // a step that reaches past d
-      lane_off[i] = static_cast<unsigned>(kvh) * a.bs * (D / 8) + (whole[i] ? c * 4 + kg : 0);
+      lane_off[i] = static_cast<unsigned>(kvh) * a.bs * (D / 8) + key_fragment<DT>(c, kg);
     } else {
       key_off[i] = 8 * kg;
       whole[i] = true;
@@ -768,8 +775,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
     for (int t = 0; t < 2; ++t) {
       const bf16_t* k = address(k_pages, p[t], r.k_ok[t]);
 #pragma unroll
-      for (int c = 0; c < DC; ++c)
-        r.k[t][c] = ld16(DT % 2 != 0 && c == DC - 1 ? k + (over ? 0 : 32 * c) : k + 32 * c);
+      for (int c = 0; c < DC; ++c) r.k[t][c] = ld16(k + 8 * (key_fragment<DT>(c, kg) - kg));   // (kg is in k_lane)
     }
     const bf16_t* v = address(vt_pages, p[2], r.v_ok);
 #pragma unroll
@@ -1121,6 +1127,16 @@ KVF_EXPORT void kvf_attn_mfma_set_split_waves(int waves) { g_split_waves = waves
 KVF_EXPORT int kvf_attn_mfma_rows_per_item(int d, int row_tiles) {
   const int most = d > 0 && d <= 128 ? 2 : 1;   // runs_max_rt(d / 16)
   return WAVES * (row_tiles >= 2 ? most : 1) * 16;
+}
+
+// For tests: the fragment of 16 bytes of a key's row that lane group 0..3 reads in step 0..(d/16+1)/2 - 1 along d.
+KVF_EXPORT int kvf_attn_mfma_key_fragment(int d, int step, int lane_group) {
+  switch (d / 16) {
+#define GO(DT) case DT: return key_fragment<DT>(step, lane_group);
+    KVF_EACH_DT(GO)
+#undef GO
+  }
+  return -1;
 }
 
 // Whether a work row's two items are taken side by side by one workgroup: a caller then makes rows of
