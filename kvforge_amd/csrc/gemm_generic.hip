@@ -431,7 +431,7 @@ int launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, 
                        N, K, lda, ldc);
     return kvf_last_error();
   }
-  if (quads && !g_vector_alus_only) {
+  if (quads && K > 0 && !g_vector_alus_only) {   // (its loads need an element of K to be clamped to)
 #define TILES(XM, XN)                                                                            \
   do {                                                                                           \
     const int total = ((N + XN - 1) / XN) * ((M + XM - 1) / XM);                                 \

@@ -675,6 +675,19 @@ def test_gemm_generic_tiles_of_both_sizes(tw, k):
     assert torch.equal(acc, out + 1.0)
 
 
+@pytest.mark.parametrize("tw", DTYPES)
+@pytest.mark.parametrize("m", [1, 17, 33, 130, 1000])
+def test_gemm_generic_over_no_elements(tw, m):
+    """Rows of a wider tensor cut down to no columns, on 16 bytes like those of any product: the sum over nothing
+    is zero, and added to what is there it changes nothing."""
+    a, w = torch.ones(m, 8, device=DEV)[:, 4:4], torch.empty(70, 0, dtype=tw, device=DEV)
+    out = torch.full((m, 70), 7.0, device=DEV)
+    ops().gemm(a, w, out, accumulate=True)
+    assert bool((out == 7.0).all())
+    ops().gemm(a, w, out)
+    assert bool((out == 0.0).all())
+
+
 @pytest.mark.parametrize("m", [1, 4, 8, 16, 32])
 @pytest.mark.parametrize("n,k", [(6150, 516), (16390, 260)])
 @pytest.mark.parametrize("tw", DTYPES)
