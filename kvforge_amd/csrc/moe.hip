@@ -660,24 +660,38 @@ KVF_EXPORT int kvf_moe_identity(int dtype, float* x, const void* h, const int* s
   return kvf_last_error();
 }
 
+// Whether kvf_moe_grouped takes the kernels of more rows.  Those of few rows bring an expert's 6 ff K bytes in anew
+// for every tile of 16 rows, in all about pairs / 16 + E / 2 tiles, at 7 TB/s where the matrices lie in the caches;
+// the others walk along K and ff in passes of 64 elements, 0.7 us each however few workgroups there are.  The
+// line is where the first takes longer than the second,
+//   (pairs / 16 + E / 2) 6 ff K / 7 TB/s > (K + ff) / 64 * 0.7 us, fitted: pairs / 16 + E / 2 >= 15,500 (1 / ff + 1 / K),
+// and six rows an expert, for below that either is bound by the matrices' way from memory.  Plan to sum, us, few
+// against more (experts, ff, K):
+//   4, 512, 1,024: 64 rows an expert 26 / 31, 192 41 / 35       8, 1,024, 1,024: 40 rows 36 / 42, 64 50 / 46
+//   8, 3,584, 2,048: 12 rows 92 / 100, 20 108 / 101             16, 512, 1,024: 32 rows 34 / 35, 48 42 / 37
+//   32, 1,024, 2,048: 6 rows 89 / 83, 32 163 / 87               64, 256, 1,024: 6 rows 33 / 36, 20 45 / 39
+// over 19 shapes and 2 to 512 rows an expert at most 10% off the better one.  (Six rows an expert alone sent the few
+// and small experts' steps to the wrong side, up to 33% slower.)  Pairs that name no expert are counted like
+// the others: the device alone knows them, and a router with such outputs changes sides that much early.
+KVF_EXPORT int kvf_moe_grouped_many_rows(int pairs, int E, int ff, int K) {
+  return pairs >= 6ll * E && (pairs + 8ll * E) * ff * K >= 248000ll * (ff + K);
+}
+
 // The routed experts of a bf16 step without the rows that did not choose them.  x [n, K] (row
 // stride ldx), w_gate_up / w_down: the tiled forms of [E 2 ff, K] (gate and up rows interleaved)
 // and [K, E ff]; sel / wgt [n, top]; scratch: where, order [n top], tiles [3 max_tiles],
 // num_tiles [1], act [n top, ff], y [n top, K].  Needs K % 8 == 0 and ff % 32 == 0.  weigh_input: the
 // weights go into the experts' inputs instead of the sum over their outputs.  fresh: residual is
-// written, not added to.  form, limit: how an expert's pairs are joined (GateForm's act 0 or 2).
+// written, not added to.  form, limit: how an expert's pairs are joined (GateForm's act 0 or 2).  many_rows: below
+// 0, or which kernels are taken whatever the sizes (0: those of few rows, else those of more).
 KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int K, int E, int ff, int top,
                                const void* w_gate_up, const void* w_down, const int* sel, const float* wgt,
                                int* where, int* order, int* tiles, int* num_tiles, int max_tiles, void* act,
                                void* y, float* residual, int weigh_input, int fresh, int form, float limit,
-                               hipStream_t s) {
+                               int many_rows, hipStream_t s) {
   if (n <= 0) return 0;
   const int pairs = n * top;
-  // Six rows an expert on average are where the kernels of more rows begin to pay: 192 pairs over 32
-  // experts 84 against 91 us (ff 1,024) and 160 against 162 (ff 2,048), 128 pairs 87 against 92 and 159
-  // against 154, 752 pairs 87 against 142 and 167 against 262 (where an expert's rows pass 16, tiles of
-  // 16 read its matrices again).
-  const bool many = pairs >= 6 * E;
+  const bool many = many_rows < 0 ? kvf_moe_grouped_many_rows(pairs, E, ff, K) != 0 : many_rows != 0;
   const int tile_rows = many ? WIDE_ROWS : 16;
   const GateForm f{form, limit, 1.f};
   if (!form_ok(form, limit) || E <= 0 || E > PLAN_MAX_EXPERTS || K % 8 != 0 || ff % 32 != 0 || ldx % 8 != 0 || max_tiles > 65535 ||

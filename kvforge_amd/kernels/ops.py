@@ -1891,10 +1891,10 @@ def moe_grouped_tiles(rows: int, top: int, experts: int) -> int:
 def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedWeight", chosen: torch.Tensor,
                 weights: torch.Tensor, residual: torch.Tensor, experts: int, ff: int,
                 scratch: dict[str, torch.Tensor], weigh_input: bool = False, fresh: bool = False,
-                form: str = "silu", limit: float | None = None) -> None:
+                form: str = "silu", limit: float | None = None, many_rows: bool | None = None) -> None:
     """``residual[n] += sum_k weights[n, k] * expert_{chosen[n, k]}(x[n])`` (a choice ``>= experts``
     stands for ``x[n]`` itself) with every expert's products taken over only the rows that chose
-    it: the pairs are grouped by expert on the device, tiles of 16 rows go through the
+    it: the pairs are grouped by expert on the device, tiles of up to 16 or up to 128 rows go through the
     matrix cores against the expert's tiles of ``w_gate_up`` (``[experts * 2 ff, K]``, gate and
     up rows interleaved) and ``w_down`` (``[K, experts * ff]``), an expert's output row is stored
     in bf16 and the weighted sum over a token's choices is taken in fp32 in their order.
@@ -1902,7 +1902,8 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
     ``act [n top, ff]``, ``y [n top, K]`` (bf16).  ``weigh_input``: every chosen expert reads its
     weight times the row, ``expert(weights[n, k] * x[n])``, and the outputs are summed as they are.
     ``fresh``: ``residual`` is written instead of added to.  ``form``, ``limit``: how an expert joins its
-    pairs (``MOE_FORMS``)."""
+    pairs (``MOE_FORMS``).  ``many_rows``: for tests, which of the two tile sizes is taken; the sizes
+    decide otherwise (``kvf_moe_grouped_many_rows`` in ``moe.hip``).  The results are the same bits."""
     code, lim = _moe_form(form, limit, "moe_grouped")
     n, k = x.shape
     top = chosen.shape[1]
@@ -1919,12 +1920,13 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
                                ("num_tiles", I32, (1,)), ("act", BF16, (pairs, ff)), ("y", BF16, (pairs, k))):
         _check(scratch[name], name, dtype, shape)
     f = _fn("moe", "kvf_moe_grouped", [c_void_p, c_int, c_void_p] + [c_int] * 5 + [c_void_p] * 8 + [c_int]
-            + [c_void_p] * 3 + [c_int, c_int, c_int, c_float, c_void_p])
+            + [c_void_p] * 3 + [c_int, c_int, c_int, c_float, c_int, c_void_p])
     _ok(f(x.data_ptr(), x.stride(0) if n > 1 else k, x.data_ptr(), n, k, int(experts), int(ff), top,
           w_gate_up.tiles.data_ptr(), w_down.tiles.data_ptr(), chosen.data_ptr(), weights.data_ptr(),
           scratch["where"].data_ptr(), scratch["order"].data_ptr(), scratch["tiles"].data_ptr(),
           scratch["num_tiles"].data_ptr(), max_tiles, scratch["act"].data_ptr(), scratch["y"].data_ptr(),
-          residual.data_ptr(), 1 if weigh_input else 0, 1 if fresh else 0, code, lim, _stream()), "moe_grouped")
+          residual.data_ptr(), 1 if weigh_input else 0, 1 if fresh else 0, code, lim,
+          -1 if many_rows is None else int(many_rows), _stream()), "moe_grouped")
 
 
 

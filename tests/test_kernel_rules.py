@@ -1,5 +1,5 @@
-"""Where the matrix-core attention kernels read a key's row, walked over on the CPU: the offsets come from the
-compiled module, which needs no GPU to be asked for them."""
+"""What the compiled modules say of themselves without a GPU: where the matrix-core attention kernels read a key's
+row, and which kernels the routed experts' sizes choose."""
 
 from __future__ import annotations
 
@@ -26,3 +26,13 @@ def test_every_fragment_of_a_key_lies_in_its_row(d, pages, KV, bs):
                 read = [base + fragment(d, c, group) for c in range(steps) for group in range(4)]
                 assert all(base <= at < base + row and at < size for at in read)
                 assert read[:row] == list(range(base, base + row))
+
+
+@pytest.mark.parametrize("experts,ff,k,few,more", [
+    (4, 512, 1024, 64, 192), (8, 1024, 1024, 40, 64), (8, 3584, 2048, 12, 20), (8, 2048, 4096, 12, 16), (16, 512, 1024, 32, 48),
+    (32, 1024, 2048, 5, 6), (64, 256, 1024, 6, 20), (512, 2048, 4096, 5, 6)])
+def test_routed_experts_change_kernels_where_tiles_of_many_rows_pay(experts, ff, k, few, more):
+    """``few`` and ``more`` rows an expert, either side of where the two take the same time: few or small experts, which
+    leave most of the chip to tiles of many rows idle, change late.  Sizes whose products pass 32 bits too."""
+    many = ctypes.CDLL(library.build_module("moe")).kvf_moe_grouped_many_rows
+    assert [many(rows * experts, experts, ff, k) for rows in (2, few, more, 4096)] == [0, 0, 1, 1]

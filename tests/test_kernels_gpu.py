@@ -1274,12 +1274,13 @@ def test_sample_frequencies_follow_softmax():
 
 @pytest.mark.parametrize("counts,K,ff", [([1, 16, 32, 33], 64, 32), ([64, 65, 96, 97], 8, 96), ([127, 128, 129, 0], 200, 64),
                                          ([256, 257, 0, 500], 72, 32), ([9, 0, 9, 6], 40, 64), ([5, 6, 7, 6], 2048, 160),
-                                         ([5, 6, 7, 5], 2048, 160)])
+                                         ([5, 6, 7, 5], 2048, 160), ([3, 0, 1, 17], 8, 96), ([2, 5, 1, 0], 72, 32),
+                                         ([4, 15, 1, 2], 200, 160)])
 @pytest.mark.parametrize("weigh_input", [False, True])
 def test_grouped_experts_at_the_edges_of_their_tiles(counts, K, ff, weigh_input):
     """``counts[e]`` rows choose expert ``e`` and as many again an output that names no expert: tiles of
-    every size, widths with an odd step and with part of one, and both sides of the line between the
-    kernels of few and of more rows (six rows an expert).  The reference rounds where the kernels
+    every size, widths with an odd step and with part of one, through the kernels of few rows, those of more
+    and the ones that the sizes choose, which give the same bits.  The reference rounds where the kernels
     store bf16 (the joined pairs, an expert's row); a sum in another order may fall to the other side of
     either rounding, 2^-8 of its value at most."""
     E = len(counts)
@@ -1298,9 +1299,15 @@ def test_grouped_experts_at_the_edges_of_their_tiles(counts, K, ff, weigh_input)
     ints = {k: torch.empty(s, dtype=torch.int32, device=DEV) for k, s in (("where", n * top), ("order", n * top),
                                                                           ("tiles", 3 * tiles), ("num_tiles", 1))}
     rows = {k: torch.full((n * top, s), math.nan, dtype=torch.bfloat16, device=DEV) for k, s in (("act", ff), ("y", K))}
-    got = res.to(DEV)
-    o.moe_grouped(x.to(DEV), o.streamed(up.reshape(E * 2 * ff, K).to(DEV)), o.streamed(down.reshape(K, E * ff).to(DEV)),
-                  chosen.to(DEV), w.to(DEV), got, E, ff, {**ints, **rows}, weigh_input=weigh_input)
+    outs = []
+    for many in (False, True, None):
+        for t in rows.values():
+            t.fill_(math.nan)
+        got = res.to(DEV)
+        o.moe_grouped(x.to(DEV), o.streamed(up.reshape(E * 2 * ff, K).to(DEV)), o.streamed(down.reshape(K, E * ff).to(DEV)),
+                      chosen.to(DEV), w.to(DEV), got, E, ff, {**ints, **rows}, weigh_input=weigh_input, many_rows=many)
+        outs.append(got)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
     want, slack = res.double(), torch.zeros(n, K, dtype=torch.float64)
     for e in range(E):
         at = (chosen[:, 0] == e).nonzero()[:, 0]
