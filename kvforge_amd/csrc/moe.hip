@@ -151,9 +151,12 @@ __global__ __launch_bounds__(256) void moe_identity_kernel(float* __restrict__ x
 //
 // moe_plan: the (token, choice) pairs are grouped by expert: where[pair] is the pair's place in
 // that order (-1 for a choice that names no expert), order[place] the pair; every expert's rows
-// are cut into tiles of tile_rows: tiles[t] = (expert, first place, rows).  One workgroup; the order of
+// are cut into tiles of up to 2^tile_shift: tiles[t] = (expert, first place, rows).  One workgroup; the order of
 // an expert's rows among themselves is whatever the atomics give, which no result depends on
-// (a row's products do not depend on its neighbours).
+// (a row's products do not depend on its neighbours).  What bounds it is one workgroup's chain of trips: choices,
+// counters in LDS, sums over the experts, stores.  Up to 8,192 pairs the choices and their places stay in
+// registers in between, and a lane adds up no more experts than there are; plan to sum at 4 experts (512 x 1,024)
+// and 24 pairs 19.4 us (20.3 with both passes over memory and sums over all 512 places).
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int PLAN_MAX_EXPERTS = 512;
@@ -168,30 +171,41 @@ __device__ __forceinline__ uint2 pack4(const f32x4& a) {
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ sel, int pairs, int E,
                                                         int* __restrict__ where, int* __restrict__ order,
                                                         int* __restrict__ tiles, int* __restrict__ num_tiles,
-                                                        int max_tiles, int tile_rows) {
+                                                        int max_tiles, int tile_shift) {
   __shared__ int cnt[PLAN_MAX_EXPERTS], off[PLAN_MAX_EXPERTS], first_tile[PLAN_MAX_EXPERTS];
-  const int tid = threadIdx.x;
-  for (int e = tid; e < PLAN_MAX_EXPERTS; e += blockDim.x) cnt[e] = 0;
+  const int tid = threadIdx.x, step = static_cast<int>(blockDim.x);
+  const int per = (E + KVF_WAVE - 1) / KVF_WAVE;   // experts a lane of the first wave adds up
+  auto tiles_of = [&](int rows) { return (rows + (1 << tile_shift) - 1) >> tile_shift; };
+  for (int e = tid; e < per * KVF_WAVE; e += step) cnt[e] = 0;
+  // A thread's choices are asked for together: one trip to memory for PLAN_BATCH of them.  One round of
+  // them stays in registers up to the end, more are read again.
+  int e[PLAN_BATCH], at[PLAN_BATCH];
+  const bool once = pairs <= PLAN_BATCH * step;
+  auto ask = [&](int p0) {
+#pragma unroll
+    for (int i = 0; i < PLAN_BATCH; ++i)
+      if (i * step < pairs) e[i] = sel[min(p0 + i * step, pairs - 1)];
+  };
+  auto each = [&](int p0, auto&& go) {
+#pragma unroll
+    for (int i = 0; i < PLAN_BATCH; ++i)
+      if (i * step < pairs && p0 + i * step < pairs) go(p0 + i * step, e[i], at[i]);
+  };
+  if (tid < pairs) ask(tid);
   __syncthreads();
-  // a thread's choices are asked for together: one trip to memory for PLAN_BATCH of them
-  for (int p0 = tid; p0 < pairs; p0 += PLAN_BATCH * blockDim.x) {
-    int e[PLAN_BATCH];
-#pragma unroll
-    for (int i = 0; i < PLAN_BATCH; ++i) e[i] = sel[min(p0 + i * static_cast<int>(blockDim.x), pairs - 1)];
-#pragma unroll
-    for (int i = 0; i < PLAN_BATCH; ++i) {
-      const int p = p0 + i * blockDim.x;
-      if (p < pairs) where[p] = (e[i] >= 0 && e[i] < E) ? atomicAdd(&cnt[e[i]], 1) : -1;
-    }
+  for (int p0 = tid; p0 < pairs; p0 += PLAN_BATCH * step) {
+    if (p0 != tid) ask(p0);
+    each(p0, [&](int p, int expert, int& place) {
+      place = expert >= 0 && expert < E ? atomicAdd(&cnt[expert], 1) : -1;
+      if (!once) where[p] = place;
+    });
   }
   __syncthreads();
   if (tid < KVF_WAVE) {   // where every expert's rows and tiles begin: sums over the lanes before
-    constexpr int PER = PLAN_MAX_EXPERTS / KVF_WAVE;
     int rows = 0, nt = 0;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      rows += cnt[PER * tid + i];
-      nt += (cnt[PER * tid + i] + tile_rows - 1) / tile_rows;
+    for (int i = 0; i < per; ++i) {
+      rows += cnt[per * tid + i];
+      nt += tiles_of(cnt[per * tid + i]);
     }
     int rows_upto = rows, nt_upto = nt;
 #pragma unroll
@@ -205,40 +219,36 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     if (tid == KVF_WAVE - 1) *num_tiles = min(nt_upto, max_tiles);
     rows_upto -= rows;
     nt_upto -= nt;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      off[PER * tid + i] = rows_upto;
-      first_tile[PER * tid + i] = nt_upto;
-      rows_upto += cnt[PER * tid + i];
-      nt_upto += (cnt[PER * tid + i] + tile_rows - 1) / tile_rows;
+    for (int i = 0; i < per; ++i) {
+      off[per * tid + i] = rows_upto;
+      first_tile[per * tid + i] = nt_upto;
+      rows_upto += cnt[per * tid + i];
+      nt_upto += tiles_of(cnt[per * tid + i]);
     }
   }
   __syncthreads();
   if (tid < E && cnt[tid] > 0) {   // an expert's tiles hold about equally many rows, in whole sixteens
-    const int c = cnt[tid], nt = (c + tile_rows - 1) / tile_rows, per = ((c + nt - 1) / nt + 15) / 16 * 16;
+    const int c = cnt[tid], nt = tiles_of(c);
+    int each_has = c;
+    if (nt > 1) each_has = ((c + nt - 1) / nt + 15) / 16 * 16;
     for (int i = 0; i < nt && first_tile[tid] + i < max_tiles; ++i) {
       int* t = tiles + 3 * (first_tile[tid] + i);
       t[0] = tid;
-      t[1] = off[tid] + i * per;
-      t[2] = min(per, c - i * per);
+      t[1] = off[tid] + i * each_has;
+      t[2] = min(each_has, c - i * each_has);
     }
   }
-  for (int p0 = tid; p0 < pairs; p0 += PLAN_BATCH * blockDim.x) {
-    int e[PLAN_BATCH], at[PLAN_BATCH];
+  for (int p0 = tid; p0 < pairs; p0 += PLAN_BATCH * step) {
+    if (!once) {
+      ask(p0);
 #pragma unroll
-    for (int i = 0; i < PLAN_BATCH; ++i) {
-      const int p = min(p0 + i * static_cast<int>(blockDim.x), pairs - 1);
-      e[i] = sel[p];
-      at[i] = where[p];
+      for (int i = 0; i < PLAN_BATCH; ++i) at[i] = where[min(p0 + i * step, pairs - 1)];
     }
-#pragma unroll
-    for (int i = 0; i < PLAN_BATCH; ++i) {
-      const int p = p0 + i * blockDim.x;
-      if (p < pairs && e[i] >= 0 && e[i] < E) {
-        where[p] = off[e[i]] + at[i];
-        order[off[e[i]] + at[i]] = p;
-      }
-    }
+    each(p0, [&](int p, int expert, int place) {
+      const bool named = expert >= 0 && expert < E;
+      if (named) order[off[expert] + place] = p;
+      if (named || once) where[p] = named ? off[expert] + place : -1;
+    });
   }
 }
 
@@ -351,7 +361,7 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const bf16_t* __restrict_
 // weight rows a workgroup, two of them a compute unit 215 / 364 (512 equal workgroups leave 40 for a
 // second round); 256 rows and 256 weight rows, eight waves 245 / 390; fragments read from LDS where they
 // are needed instead of two ahead 230 / 380.
-constexpr int WIDE_ROWS = 128, WIDE_GW = 2;
+constexpr int WIDE_SHIFT = 7, WIDE_ROWS = 1 << WIDE_SHIFT, WIDE_GW = 2;
 
 // What a workgroup takes: tile and block of columns.  Workgroups go to the eight XCDs in turn, and each
 // XCD gets an unbroken eighth of the (tile, block) pairs, the blocks of a tile side by side and the tiles of an
@@ -692,13 +702,12 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int
   if (n <= 0) return 0;
   const int pairs = n * top;
   const bool many = many_rows < 0 ? kvf_moe_grouped_many_rows(pairs, E, ff, K) != 0 : many_rows != 0;
-  const int tile_rows = many ? WIDE_ROWS : 16;
   const GateForm f{form, limit, 1.f};
   if (!form_ok(form, limit) || E <= 0 || E > PLAN_MAX_EXPERTS || K % 8 != 0 || ff % 32 != 0 || ldx % 8 != 0 || max_tiles > 65535 ||
       max_tiles < (pairs + 15) / 16 + E)
     return static_cast<int>(hipErrorInvalidValue);
   hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel, pairs, E, where, order, tiles, num_tiles,
-                     max_tiles, tile_rows);
+                     max_tiles, many ? WIDE_SHIFT : 4);
   const int S = (K + 31) / 32, up_groups = ff / 8, down_groups = (K + 15) / 16;
   const bf16_t* xb = static_cast<const bf16_t*>(x);
   const uint4 *up = static_cast<const uint4*>(w_gate_up), *down = static_cast<const uint4*>(w_down);

@@ -1275,11 +1275,12 @@ def test_sample_frequencies_follow_softmax():
 @pytest.mark.parametrize("counts,K,ff", [([1, 16, 32, 33], 64, 32), ([64, 65, 96, 97], 8, 96), ([127, 128, 129, 0], 200, 64),
                                          ([256, 257, 0, 500], 72, 32), ([9, 0, 9, 6], 40, 64), ([5, 6, 7, 6], 2048, 160),
                                          ([5, 6, 7, 5], 2048, 160), ([3, 0, 1, 17], 8, 96), ([2, 5, 1, 0], 72, 32),
-                                         ([4, 15, 1, 2], 200, 160)])
+                                         ([4, 15, 1, 2], 200, 160), ([3000, 1, 4500, 1700], 8, 32),
+                                         ([e % 7 for e in range(130)], 40, 32)])
 @pytest.mark.parametrize("weigh_input", [False, True])
 def test_grouped_experts_at_the_edges_of_their_tiles(counts, K, ff, weigh_input):
     """``counts[e]`` rows choose expert ``e`` and as many again an output that names no expert: tiles of
-    every size, widths with an odd step and with part of one, through the kernels of few rows, those of more
+    every size, more pairs than the plan holds in registers, more experts than a wave has lanes, widths with an odd step and with part of one, through the kernels of few rows, those of more
     and the ones that the sizes choose, which give the same bits.  The reference rounds where the kernels
     store bf16 (the joined pairs, an expert's row); a sum in another order may fall to the other side of
     either rounding, 2^-8 of its value at most."""
