@@ -166,12 +166,16 @@ __device__ __forceinline__ int block_of(const MArgs& a, int key) {
 __device__ __forceinline__ uint4 ld16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ bf16x8 as_frag(const uint4& r) { return __builtin_bit_cast(bf16x8, r); }
 
+// The part of word e (0..3) of a fragment that its first `live` (8 at most) bf16 take up.
+__device__ __forceinline__ uint32_t first_mask(int e, int live) {
+  return 2 * e + 1 < live ? 0xffffffffu : (2 * e < live ? 0xffffu : 0u);
+}
 // Keeps the first `live` (0..8) bf16 of a fragment, clears the rest.
 __device__ __forceinline__ uint4 keep_first(const uint4& r, int live) {
   if (!__any(live < 8)) return r;  // nearly every fragment is whole in every lane
   uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
-  for (int e = 0; e < 4; ++e) w[e] &= 2 * e + 1 < live ? 0xffffffffu : (2 * e < live ? 0xffffu : 0u);
+  for (int e = 0; e < 4; ++e) w[e] &= first_mask(e, live);
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
@@ -665,8 +669,10 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
 // ------------------------------------------------------------------------- few rows, split keys
 // DEPTH 2: a wave holds the fragments of two blocks, loading one while it consumes the other.
 // NW: waves of the workgroup; more of them shorten each wave's walk over its cut of the keys.
+// Two waves a SIMD where a wave's fragments leave room for them, two blocks of up to 96 elements or one of up
+// to 192 (head size 192, 41 ragged contexts: 34.0 us with one wave, 29.6 with two; at 256 two spill).
 template <int DT, int DEPTH, int NW, int BIAS, bool SINK>
-__global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfma_split_kernel(
+__global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6 || (DT > 8 && DT <= 12)) void attn_mfma_split_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
     const bf16_t* __restrict__ vt_pages, const int* __restrict__ block_table,
     const int* __restrict__ seq_ids, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
@@ -735,7 +741,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
   for (int t = 0; t < DT; ++t) acc[0][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // The register buffers are named apart (an index chosen at run time would put them in
-  // scratch); the pages of a block are looked up one block before its fragments are loaded.
+  // scratch); the pages of a block are looked up a stage before its fragments are loaded.
   struct Raw {
     uint4 k[2][DC], v[DT];
     bool k_ok[2], v_ok;
@@ -791,14 +797,28 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
                                     over ? 0 : r.k[t][DC - 1].z, over ? 0 : r.k[t][DC - 1].w);
     }
     // Keys without a page do not count, nor do those at or past the context length, which hold whatever an
-    // earlier owner of the page left there.  Nearly every block is whole: one question for all its fragments.
+    // earlier owner of the page left there.  Nearly every block is whole: one question for all its fragments,
+    // and no further one behind it (a question for each made the last block of a walk the slowest: one of 60
+    // keys at head size 256 8.2 us, 7.0 now).
     if (kb + 32 > ctx || __any(!(r.k_ok[0] && r.k_ok[1] && r.v_ok))) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t) {
+        const uint32_t m = r.k_ok[t] ? 0xffffffffu : 0u;
 #pragma unroll
-        for (int c = 0; c < DC; ++c) w.k[t][c] = keep_first(w.k[t][c], r.k_ok[t] ? 8 : 0);
+        for (int c = 0; c < DC; ++c) {
+          const uint4 f = w.k[t][c];
+          w.k[t][c] = make_uint4(f.x & m, f.y & m, f.z & m, f.w & m);
+        }
+      }
+      const int live = r.v_ok ? min(ctx - kb - 8 * kg, 8) : 0;
+      uint32_t m[4];
 #pragma unroll
-      for (int t = 0; t < DT; ++t) w.v[t] = keep_first(w.v[t], r.v_ok ? min(ctx - kb - 8 * kg, 8) : 0);
+      for (int e = 0; e < 4; ++e) m[e] = first_mask(e, live);
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        const uint4 f = w.v[t];
+        w.v[t] = make_uint4(f.x & m[0], f.y & m[1], f.z & m[2], f.w & m[3]);
+      }
     }
     bf16x8 kf[2][DC], vf[DT];
 #pragma unroll
@@ -824,12 +844,13 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
     // A stage looks up the pages of the block DEPTH ahead, then asks for the fragments of the one before
     // it, whose pages were looked up before the last fragments were asked for: the load counter runs in
     // order, and no wait drains what was asked for after what it waits for.  For the same reason no load
-    // sits in a branch; past its last block a wave asks for its first again, and the blocks that nothing
-    // follows are taken behind the loop.
-    auto in = [&](int kb) { return kb < kb_end ? kb : kb_begin; };
+    // sits in a branch; past its last block a wave asks for that block again, which its caches still hold
+    // (the first one again, which they do not, cost 64 walks of 8 blocks a wave at head size 96 9%), and the blocks
+    // that nothing follows are taken behind the loop.
+    auto in = [&](int kb, int last) { return kb < kb_end ? kb : last; };
     if (!early) {
 #pragma unroll
-      for (int i = 0; i < DEPTH; ++i) locate(in(kb_begin + i * STEP), P[i]);
+      for (int i = 0; i < DEPTH; ++i) locate(in(kb_begin + i * STEP, kb_begin), P[i]);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -838,11 +859,13 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6) void attn_mfm
     for (; kb + AHEAD * STEP < kb_end; kb += DEPTH * STEP) {
 #pragma unroll
       for (int i = 0; i < DEPTH; ++i) {
-        if (DEPTH > 1) locate(in(kb + (i + DEPTH) * STEP), P[i]);
-        __builtin_amdgcn_sched_barrier(0);
+        if (DEPTH > 1) {
+          locate(in(kb + (i + DEPTH) * STEP, kb + AHEAD * STEP), P[i]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
         fetch(P[(i + AHEAD) % DEPTH], R[(i + AHEAD) % DEPTH]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (DEPTH == 1) locate(in(kb + STEP), P[i]);
+        if (DEPTH > 1) __builtin_amdgcn_sched_barrier(0);   // one block at a time has nothing to keep apart
+        if (DEPTH == 1) locate(in(kb + STEP, kb), P[i]);
         consume(kb + i * STEP, R[i]);
       }
     }
