@@ -526,7 +526,6 @@ __global__ __launch_bounds__(KVF_WAVE) void mlstm_gates_kernel(const float* __re
 // working set of a (chunk, head) is a few times 32 KB that the waves and the workgroups of its column blocks find in
 // their caches.  (Staged in LDS it filled 114 KB, one workgroup a compute unit whose four waves waited for
 // every load in turn.)
-constexpr int PCOLS = 64;    // columns of S a workgroup of the passes takes
 
 __device__ __forceinline__ f32x4 load4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ f32x4 load4(const bf16_t* p) {
@@ -564,17 +563,17 @@ __device__ __forceinline__ f32x4 column4(const T* first, int token, int last, in
 
 // U = K^T diag(D[L]) V (30 us at the sizes given at mlstm_output_kernel, 37 before): a wave takes 16 columns,
 // its share of V (weighted, zero past the chunk's tokens) stays in registers, and K comes in 16 of its
-// columns at a time.  Bound by the trips of those tiles to memory and the 17 MB of sums it writes.
+// columns at a time; waves that have the same columns of V take the tiles of K in turn.  Bound by the trips of those tiles to memory and the 17 MB of sums it writes.
 template <typename T, int DKP, int CL>
 __global__ __launch_bounds__(256) void mlstm_local_kernel(const T* __restrict__ qkv, const int* __restrict__ slot_ids,
-                                                          ScanArgs a, MultiArgs w) {
+                                                          ScanArgs a, MultiArgs w, int cols) {
   __shared__ __align__(16) float wl[CL];
-  const int chunk = blockIdx.z, head = blockIdx.y;
+  const int chunk = blockIdx.z, head = blockIdx.y, groups = cols / 16;
   const int seq = w.chunks[4 * chunk], tb = w.chunks[4 * chunk + 1], cnt = w.chunks[4 * chunk + 2];
   const int slot = slot_ids[seq];
   if (slot < 0 || slot >= a.n_slots) return;
   const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE, l16 = lane % 16, lq = lane / 16;
-  const int dk = a.dk, dv = a.dv, c = blockIdx.x * PCOLS + 16 * wave + l16;
+  const int dk = a.dk, dv = a.dv, c = blockIdx.x * cols + 16 * (wave % groups) + l16;
   const T* rows = qkv + static_cast<size_t>(tb) * a.row_len;
   if (tid < CL) {
     float v = 0.f;
@@ -597,7 +596,7 @@ __global__ __launch_bounds__(256) void mlstm_local_kernel(const T* __restrict__ 
   for (int i = 0; i < CL / 16; ++i) vw[i] *= *reinterpret_cast<const f32x4*>(wl + 16 * i + 4 * lq);
   float* U = w.W + (static_cast<size_t>(chunk) * a.H + head) * dk * dv;
 #pragma unroll 2
-  for (int kt = 0; kt < DKP / 16; ++kt) {
+  for (int kt = wave / groups; kt < DKP / 16; kt += 4 / groups) {
     const T* k_at = rows + a.k_off + head * dk + min(16 * kt + l16, dk - 1);
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -658,21 +657,21 @@ __global__ __launch_bounds__(256) void mlstm_carry_kernel(const int* __restrict_
 // without clamps for whole chunks 14 more; a tile of columns ahead 12; registers for four waves a SIMD spill, 46.
 template <typename T, int DKP, int CL>
 __global__ __launch_bounds__(256) void mlstm_output_kernel(const T* __restrict__ qkv, const int* __restrict__ slot_ids,
-                                                           float* __restrict__ out, ScanArgs a, MultiArgs w) {
+                                                           float* __restrict__ out, ScanArgs a, MultiArgs w, int cols) {
   constexpr int RT = CL / 16, WPR = 4 / RT, KQ = DKP / 16, ALD = CL + 4, SH = 256 / CL;
   static_assert(SH % 4 == 0, "a lane takes whole shares");
   __shared__ double bc[CL];
   __shared__ float li[CL], mt[CL], gt[CL];
   __shared__ __align__(16) float As[4][16][ALD];
-  const int chunk = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * PCOLS;
+  const int chunk = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * cols;
   const int seq = w.chunks[4 * chunk], tb = w.chunks[4 * chunk + 1], cnt = w.chunks[4 * chunk + 2];
   const int tid = threadIdx.x, lane = tid % KVF_WAVE, l16 = lane % 16, lq = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / KVF_WAVE), rt = wave / WPR;
   const int dk = a.dk, dv = a.dv, last = cnt - 1;
   const int slot = slot_ids[seq];
   if (slot < 0 || slot >= a.n_slots) {
-    for (int i = tid; i < cnt * PCOLS; i += blockDim.x) {
-      const int t = i / PCOLS, c = col0 + i % PCOLS;
+    for (int i = tid; i < cnt * cols; i += blockDim.x) {
+      const int t = i / cols, c = col0 + i % cols;
       if (c < dv) out[static_cast<size_t>(tb + t) * a.H * dv + head * dv + c] = 0.f;
     }
     return;
@@ -752,7 +751,7 @@ __global__ __launch_bounds__(256) void mlstm_output_kernel(const T* __restrict__
   for (int i = 0; i < KQ; ++i) q[i] *= g;
   if (16 * rt >= cnt) return;
   const float* Sc = w.W + ch * dk * dv;
-  for (int ct = wave % WPR; ct < PCOLS / 16; ct += WPR) {
+  for (int ct = wave % WPR; ct < cols / 16; ct += WPR) {
     const int c = col0 + 16 * ct + l16, cc = min(c, dv - 1);
     const T* v_at = rows + a.v_off + head * dv + cc;
     const float* s_at = Sc + cc;
@@ -788,16 +787,30 @@ int multi_go(const void* qkv, const float* zif, const float* bias_if, const int*
              const int* slot_ids, float* state, float* out, int n_chunks, int n_runs, ScanArgs a, MultiArgs w,
              hipStream_t s) {
   const T* rows = static_cast<const T*>(qkv);
-  const int slices = (a.dv + PCOLS - 1) / PCOLS;
+  // Columns a workgroup takes: 64, or fewer (at least 16; of outputs what its waves have a tile each of) where the
+  // workgroups leave compute units idle, for then a wave's trips to memory in a row are what a pass takes: 4
+  // heads of 128 x 256 and one run of 200 tokens, all passes 42.4 us with 64 columns, 33.6 with fewer, 39.4 where
+  // everything went through LDS.  With all of them busy the products of q and k, which every block of columns
+  // makes anew, cost more than that hides: two runs of 256 tokens 38.1 us at 256 workgroups of outputs, 40.6 at
+  // 512; keys of more than 128, one workgroup a compute unit by their registers, must not come to a second round:
+  // 4 heads of 256 x 512, 200 tokens, 62 us with 64 columns (224 workgroups), 78 with 32.
+  auto cols_of = [&](int least) {
+    auto groups = [&](int cols) { return static_cast<long>((a.dv + cols - 1) / cols) * a.H * n_chunks; };
+    int cols = 64;
+    while (cols > least && (DKP > 128 ? groups(cols / 2) <= 256 : groups(cols) < 256)) cols /= 2;
+    return cols;
+  };
+  const int cols_local = cols_of(16), cols = cols_of(CL == 64 ? 16 : 32);
+  const int slices_local = (a.dv + cols_local - 1) / cols_local, slices = (a.dv + cols - 1) / cols;
   hipLaunchKernelGGL(mlstm_gates_kernel<CL>, dim3(a.H, n_runs), dim3(KVF_WAVE), 0, s, zif, bias_if, cu_q, positions,
                      slot_ids, state, a, w);
-  hipLaunchKernelGGL((mlstm_local_kernel<T, DKP, CL>), dim3(slices, a.H, n_chunks), dim3(256), 0, s,
-                     rows, slot_ids, a, w);
+  hipLaunchKernelGGL((mlstm_local_kernel<T, DKP, CL>), dim3(slices_local, a.H, n_chunks), dim3(256), 0, s,
+                     rows, slot_ids, a, w, cols_local);
   const unsigned per_head = static_cast<unsigned>((static_cast<size_t>(a.dk) * a.dv + a.dk + 255) / 256);
   hipLaunchKernelGGL(mlstm_carry_kernel, dim3(per_head, a.H, n_runs), dim3(256), 0, s, cu_q, positions, slot_ids, state,
                      a, w);
   hipLaunchKernelGGL((mlstm_output_kernel<T, DKP, CL>), dim3(slices, a.H, n_chunks), dim3(256), 0, s,
-                     rows, slot_ids, out, a, w);
+                     rows, slot_ids, out, a, w, cols);
   return kvf_last_error();
 }
 

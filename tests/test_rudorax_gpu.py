@@ -314,6 +314,39 @@ def test_matrix_memory_passes_at_the_edges_of_their_tiles(dtype, H, dk, dv, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,dk,dv", [(3, 37, 100), (2, 128, 65), (2, 200, 130), (1, 64, 256)])
+def test_matrix_memory_passes_whatever_the_columns_of_a_workgroup(dtype, H, dk, dv):
+    """The columns a workgroup takes follow from how many workgroups there are: runs of several lengths all in one
+    step, in steps of four and each alone give the same bits, and a run without a slot zeros."""
+    cap, cols, lens = 12.0, 2 * H * dk + H * dv, [64, 130, 200, 97] * 16
+    first = [0] + list(np.cumsum(lens))
+    n = first[-1]
+    rows, z = rand(n, cols, seed=dk).to(dtype).to(DEV), rand(n, 2 * H, seed=dv, scale=3.0).to(DEV)
+    bias = torch.cat([torch.full((H,), -1.0), torch.full((H,), 4.0)]).to(DEV)
+    slots = [s if s != 6 else -1 for s in range(len(lens))]
+
+    def run(at_once, upto):
+        state = torch.full((len(lens), ops().mlstm_state_floats(H, dk, dv)), 3.0, device=DEV)
+        out = torch.full((first[upto], H * dv), 5.0, device=DEV)
+        for s in range(0, upto, at_once):
+            a, b, q = first[s], first[s + at_once], lens[s:s + at_once]
+            chunks, runs = ops().mlstm_multi_plan(q, dk, 1)
+            multi = {"chunks": i32(chunks).view(-1, 4), "runs": i32(runs).view(-1, 3)}
+            for name, (shape, dt) in ops().mlstm_multi_scratch(b - a, len(chunks) // 4, H, dk, dv).items():
+                multi[name] = torch.full(shape, float("nan"), dtype=dt, device=DEV)
+            ops().mlstm_scan(rows[a:b], z[a:b], bias, i32([f - a for f in first[s:s + at_once + 1]]),
+                             torch.cat([torch.arange(m) for m in q]).int().to(DEV), i32(slots[s:s + at_once]), state, out[a:b],
+                             at_once, H, dk, dv, 0, H * dk, 2 * H * dk, cap, dk ** -0.5, chunk_from=1, multi_from=1, multi=multi)
+        return out, state
+
+    out, state = run(len(lens), len(lens))
+    for at_once, upto in ((4, len(lens)), (1, 8)):
+        some, some_state = run(at_once, upto)
+        assert torch.equal(some, out[:first[upto]]) and torch.equal(some_state[:upto], state[:upto])
+    assert bool((out[first[6]:first[7]] == 0.0).all()) and bool((state[6] == 3.0).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_heads_normed_weighted_and_gated(dtype):
     H, dv, n, eps = 3, 40, 5, 1e-3
     raw, w = rand(n, H * dv, seed=1, scale=4.0), 1.0 + rand(H * dv, seed=2, scale=0.2)
