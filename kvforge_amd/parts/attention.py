@@ -443,7 +443,11 @@ class PagedAttention(Mixer):
         all items walk long and nothing needs filling in).  Measured at 32 heads over 8 kv heads,
         64 against 128 rows (as two row tiles a wave): 2,048 queries from position 0, 47 against 55 us at head size 64
         and 70 against 82 at 128; 4,096 queries, 140 against 114 and 231 against 196; 2,048
-        queries behind 2,048 keys, 106 against 100 and 209 against 151.  The layers of a model
+        queries behind 2,048 keys, 106 against 100 and 209 against 151.  Heads wider than 128, whose
+        items a workgroup takes in pairs, go one by one while every item finds a compute unit of its own: with one
+        item the waves beside it only help to bring keys in.  16 heads of 256 over one kv head, 256 queries 20.6 us in
+        pairs and 16.1 one by one, 33 queries 10.4 and 7.5; with 512 items, four runs of 256 queries of 32 heads of 192,
+        19.2 and 20.7.  The layers of a model
         that agree on group size and item share the rows through the step's scratch."""
         if not step.prefill_seqs:
             return None, 0
@@ -452,15 +456,22 @@ class PagedAttention(Mixer):
         found = step.scratch.get(key)
         if found is None:
             units = compute_units(step.device)
-            pairs = ops.prefill_takes_pairs(act, self.d, block_size)
-            per_item = ops.prefill_rows_per_item(act, self.d, block_size, 2)
-            rows = prefill_work_rows(step.q_lens, step.prefill_seqs, G, per_item, step.start_pos, pairs)
-            groups = len(rows) * self.KV
-            fills = groups >= ops.prefill_blocks_per_cu(act, self.d, block_size, 1) * units
-            deep = groups >= 2 * units and all(step.start_pos[b] >= step.q_lens[b] for b in step.prefill_seqs)
-            if not (fills or deep or pairs):     # where items go in pairs they have one size
-                per_item = ops.prefill_rows_per_item(act, self.d, block_size, 1)
-                rows = prefill_work_rows(step.q_lens, step.prefill_seqs, G, per_item, step.start_pos)
+
+            def rows_of(tiles: int, pairs: bool = False):
+                per_item = ops.prefill_rows_per_item(act, self.d, block_size, tiles)
+                return prefill_work_rows(step.q_lens, step.prefill_seqs, G, per_item, step.start_pos, pairs), per_item
+
+            if ops.prefill_takes_pairs(act, self.d, block_size):     # items of one size
+                rows, per_item = rows_of(1)
+                if len(rows) * self.KV > units:
+                    rows, per_item = rows_of(1, True)
+            else:
+                rows, per_item = rows_of(2)
+                groups = len(rows) * self.KV
+                fills = groups >= ops.prefill_blocks_per_cu(act, self.d, block_size, 1) * units
+                deep = groups >= 2 * units and all(step.start_pos[b] >= step.q_lens[b] for b in step.prefill_seqs)
+                if not (fills or deep):
+                    rows, per_item = rows_of(1)
             found = (step.upload_ints([x for row in rows for x in row]).view(-1, 3), per_item)
             step.scratch[key] = found
         return found

@@ -1,13 +1,17 @@
-"""What the compiled modules say of themselves without a GPU: where the matrix-core attention kernels read a key's
-row, and which kernels the routed experts' sizes choose."""
+"""What the compiled modules say of themselves without a GPU, and what is planned from it: where the matrix-core
+attention kernels read a key's row, how items of wide heads are put together, and which kernels the routed experts'
+sizes choose."""
 
 from __future__ import annotations
 
 import ctypes
+from types import SimpleNamespace
 
 import pytest
+import torch
 
 from kvforge_amd.kernels import library
+from kvforge_amd.parts import attention
 
 
 @pytest.mark.parametrize("d", range(16, 257, 16))
@@ -36,3 +40,17 @@ def test_routed_experts_change_kernels_where_tiles_of_many_rows_pay(experts, ff,
     leave most of the chip to tiles of many rows idle, change late.  Sizes whose products pass 32 bits too."""
     many = ctypes.CDLL(library.build_module("moe")).kvf_moe_grouped_many_rows
     assert [many(rows * experts, experts, ff, k) for rows in (2, few, more, 4096)] == [0, 0, 1, 1]
+
+
+@pytest.mark.parametrize("q_lens,H,KV,pairs", [([33], 16, 1, False), ([256, 1], 16, 1, False), ([512], 32, 1, False),
+                                               ([513], 32, 1, True), ([200, 200, 200], 32, 8, True), ([64], 8, 8, False)])
+def test_items_of_wide_heads_go_in_pairs_where_they_are_more_than_the_compute_units(monkeypatch, q_lens, H, KV, pairs):
+    monkeypatch.setattr(attention, "compute_units", lambda device: 256)
+    seqs = [b for b, q in enumerate(q_lens) if q > 1]
+    step = SimpleNamespace(prefill_seqs=seqs, scratch={}, device=None, q_lens=q_lens, start_pos=[0] * len(q_lens),
+                           upload_ints=lambda ints: torch.tensor(ints, dtype=torch.int32))
+    part = SimpleNamespace(H=H, KV=KV, d=224)
+    work, per_item = attention.PagedAttention._prefill_work(part, step, torch.bfloat16, 16)
+    assert per_item == 64 and bool((work[:, 2] >= 0).any()) == pairs
+    items = sorted((b, i) for b, *both in work.tolist() for i in both if i >= 0)
+    assert items == [(b, i) for b in seqs for i in range(-(-q_lens[b] * (H // KV) // 64))]
