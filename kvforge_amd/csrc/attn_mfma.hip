@@ -107,11 +107,13 @@ struct DistTable {
   const float* mem;    // [H, n]
   int n;
 };
-__device__ __forceinline__ void stage_dist(const MArgs& a, int head0, int heads, float* lds) {
-  const int row = dist_row(a.n_dist);
-  for (int i = threadIdx.x; i < heads * row; i += blockDim.x) {
-    const int h = i / row, d = i - h * row - DIST_PAD;
-    lds[i] = d < 0 ? 0.f : a.dist[static_cast<size_t>(head0 + h) * a.n_dist + min(d, a.n_dist - 1)] * LOG2E;
+// The first `met` distances of the heads' rows, and what pads them: no more are read where queries and keys lie
+// among `met` positions (the whole table of 32 heads and 600 distances takes 64 queries longer than their keys).
+__device__ __forceinline__ void stage_dist(const MArgs& a, int head0, int heads, int met, float* lds) {
+  const int row = dist_row(a.n_dist), fill = min(row, DIST_PAD + max(met, 1));
+  for (int i = threadIdx.x; i < heads * fill; i += blockDim.x) {
+    const int h = i / fill, d = i - h * fill - DIST_PAD;
+    lds[h * row + d + DIST_PAD] = d < 0 ? 0.f : a.dist[static_cast<size_t>(head0 + h) * a.n_dist + min(d, a.n_dist - 1)] * LOG2E;
   }
 }
 // biases (log2 units) of the keys at distances n0, n0 - 1, .., n0 - 7; `off`: the head's row in the table
@@ -444,7 +446,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
                  j16, kg};
   float* dist_space = reinterpret_cast<float*>(frag_lds + 2 * N_FRAG * KVF_WAVE);
   if (SCORE == 4 && a.dist_lds) {
-    stage_dist(a, kvh * G, G, dist_space);
+    stage_dist(a, kvh * G, G, ctx, dist_space);
     __syncthreads();
   }
   const DistTable dist{SCORE == 4 && a.dist_lds ? dist_space : nullptr, a.dist, a.n_dist};
@@ -705,7 +707,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 6 || (DT > 8 && 
   bf16x8 qf[1][DC];
   int pos_min, pos_max;
   float* dist_space = lds + NW * DT * KVF_WAVE * 4 + NW * 16 * 2;
-  if (BIAS == 4 && a.dist_lds) stage_dist(a, kvh * G + tile * 16, min(16, G - tile * 16), dist_space);
+  if (BIAS == 4 && a.dist_lds) stage_dist(a, kvh * G + tile * 16, min(16, G - tile * 16), a.n_dist + DIST_PAD, dist_space);
   const DistTable dist{BIAS == 4 && a.dist_lds ? dist_space : nullptr, a.dist, a.n_dist};
   setup_rows<DT, 1>(q, a, q0, qlen, start, kvh, tile, j16, kg, seq_ok, rows, qf, pos_min, pos_max);
   if constexpr (BIAS == 4) {
@@ -1013,7 +1015,10 @@ unsigned chunk_magic_of(int window) {
 // 300 and 1,385.  What bounds it now: a fragment read from LDS for each matrix instruction (448 TFLOP/s and
 // 671 of them; two tiles a wave would halve the reads but leave one wave a SIMD: 182 and 782 us).
 constexpr int runs_max_rt(int dt) { return dt <= 8 ? 2 : 1; }
-constexpr size_t DIST_LDS_MOST = 64 * 1024;   // LDS a launch may ask for together with its table of biases
+// LDS a launch may ask for together with its table of biases.  Workgroups of two items have a compute unit to
+// themselves by their registers, and may fill it: 2,048 queries of 32 heads of 256 over one kv head, 300 distances 149 us
+// with the table in memory and 138 in LDS, 600 distances 192 and 154.
+constexpr size_t LDS_UNASKED = 64 * 1024, DIST_LDS_MOST = LDS_UNASKED, DIST_LDS_MOST_PAIR = 160 * 1024;
 
 template <int N> struct Count { static constexpr int value = N; };
 // calls go(tiles per wave, waves) for items of `row_tiles` times 64 rows
@@ -1042,7 +1047,13 @@ void launch_runs_rt(dim3 grid, hipStream_t s, const void* q, const void* k_pages
   else if (a.dist) {   // (never with any of the others)
     MArgs b = a;
     const size_t table = static_cast<size_t>(a.H / a.KV) * dist_row(a.n_dist) * sizeof(float);
-    b.dist_lds = lds + table <= DIST_LDS_MOST;
+    b.dist_lds = lds + table <= (runs_pair(DT) ? DIST_LDS_MOST_PAIR : DIST_LDS_MOST);
+    if (b.dist_lds && lds + table > LDS_UNASKED &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_runs_kernel<DT, RT, NW, 4, false>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds + table)) != hipSuccess) {
+      kvf_last_error();   // the table is read from memory then
+      b.dist_lds = 0;
+    }
     hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 4, false>), grid, dim3(NW * KVF_WAVE), b.dist_lds ? lds + table : lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
