@@ -841,6 +841,66 @@ def test_attn_prefill_of_wide_heads_takes_items_in_pairs(d, H, KV, window):
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("d", [144, 224, 256])
+@pytest.mark.parametrize("H,KV", [(16, 1), (6, 2)])
+@pytest.mark.parametrize("form", ["sinks", "slopes", "cap", "chunk", "far biases", "near biases", "many biases", "gate", "gate, sinks",
+                                  "kept", "kept, biases", "kept, gate"])
+def test_attn_prefill_of_wide_heads_in_pairs_with_all_that_is_done_to_scores(d, H, KV, form):
+    """Everything that query runs take beside plain scores, with both items of a work row present: rows as the
+    planner makes them and an early item with a late one, between whose windows (and kept first keys) keys
+    lie that neither sees, against plain attention and bit against bit with items alone.  ``biases``: tables
+    that end early, reach past every key, and, with a run's fragments, past the LDS that needs no asking for."""
+    seq_lens, q_lens, G = [300, 131, 33, 77], [211, 131, 33, 2], H // KV
+    window, keep = (20, 5) if "kept" in form else (0, 0)
+    g = torch.Generator().manual_seed(d + H)
+    dist = {"far biases": 40, "near biases": 301, "many biases": 700, "kept, biases": 300}.get(form)
+    with_scores = dict(
+        sinks=2 * torch.randn(H, generator=g) if "sinks" in form else None,
+        slopes=torch.linspace(-0.05, 0.08, H) if form == "slopes" else None, score_cap=2.0 if form == "cap" else None,
+        chunk=45 if form == "chunk" else 0, dist=torch.randn(H, dist, generator=g) if dist else None)
+    paged = Paged(seq_lens, KV, d, 16, torch.bfloat16, seed=d)
+    n, scale = sum(q_lens), 1 / math.sqrt(d)
+    buf = (1.5 * torch.randn(n, 2 * H * d, generator=g)).to(torch.bfloat16)
+    want, off = [], 0
+    for s, (m, ql) in enumerate(zip(seq_lens, q_lens)):
+        k, v = (t[s].float().repeat_interleave(G, dim=1) for t in (paged.keys, paged.values))
+        sc = torch.matmul(buf[off:off + ql, :H * d].float().view(ql, H, d).transpose(0, 1), k.permute(1, 2, 0)) * scale
+        i, j = torch.arange(m - ql, m)[:, None], torch.arange(m)[None, :]
+        if form == "cap":
+            sc = 2.0 * torch.tanh(sc / 2.0)
+        if form == "slopes":
+            sc = sc + with_scores["slopes"][:, None, None] * (j - i)
+        if dist:
+            sc = sc + with_scores["dist"][:, (i - j).clamp(0, dist - 1)]
+        seen = (j <= i) & ((i - j < window) | (j < keep)) if window else j <= i
+        if form == "chunk":
+            seen = seen & (i // 45 == j // 45)
+        sc = sc.masked_fill(~seen[None], float("-inf"))
+        if "sinks" in form:
+            sc = torch.cat([sc, with_scores["sinks"][:, None, None].expand(H, ql, 1)], -1)
+        want.append(torch.matmul(torch.softmax(sc, -1)[:, :, :m], v.transpose(0, 1)).transpose(0, 1).reshape(ql, H * d))
+        off += ql
+    want = torch.cat(want) * (torch.sigmoid(buf[:, H * d:].float()) if "gate" in form else 1.0)
+    cu = torch.tensor([0] + list(torch.tensor(q_lens).cumsum(0)), dtype=torch.int32).to(DEV)
+    ctx, dev = torch.tensor(seq_lens, dtype=torch.int32).to(DEV), buf.to(DEV)
+    per = ops().prefill_rows_per_item(torch.bfloat16, d, 16)
+    from kvforge_amd.parts.attention import prefill_work_rows
+    planned = prefill_work_rows(q_lens, range(4), G, per, [m - q for m, q in zip(seq_lens, q_lens)], pairs=True)
+    apart = prefill_work(q_lens, G, torch.bfloat16, d, 16).tolist()
+    alone = [(b, i, -1) for b, m in enumerate(q_lens) for i in range(-(-m * G // per))]
+    assert any(lo >= 0 for _, _, lo in planned) and any(hi > lo + 2 for _, lo, hi in apart)
+    kw = {name: v.to(DEV) if isinstance(v, torch.Tensor) else v for name, v in with_scores.items()}
+    got = []
+    for work in (planned, apart, alone):
+        out = torch.full((n, H * d), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops().attn_prefill(dev[:, :H * d], paged.k.to(DEV), paged.v.to(DEV), paged.table.to(DEV), cu, ctx,
+                           torch.tensor(work, dtype=torch.int32, device=DEV), out, H, KV, d, scale, window, rows_per_item=per,
+                           keep_first=keep, gate=dev[:, H * d:] if "gate" in form else None, **kw)
+        torch.testing.assert_close(out.float().cpu(), want, **tol(torch.bfloat16))
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
 def test_prefill_kernel_says_how_many_workgroups_a_compute_unit_holds():
     """What the planner of query runs weighs rows per item against: asked of the runtime for the
     kernel that would run, at least one, never more with two row tiles than with one; sizes the
