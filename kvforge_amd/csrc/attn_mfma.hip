@@ -536,7 +536,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
       lane_off[i] = static_cast<unsigned>(kvh) * a.bs * (D / 8) + key_fragment<DT>(c, kg);
     } else {
       key_off[i] = 8 * kg;
-      whole[i] = true;
+      whole[i] = wave + i * NW < N_FRAG;                 // (out of page 0, which the caches hold)
       lane_off[i] = (static_cast<unsigned>(kvh) * D + (f - N_K) * 16 + j16) * (a.bs / 8);
     }
   }
