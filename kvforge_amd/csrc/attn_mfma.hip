@@ -1,7 +1,7 @@
 // Paged causal attention for bf16 on the matrix cores, for query runs (prefill) and for single
 // tokens (decode).  Every operand fragment is loaded from the pages in the register layout the
-// instruction wants (no transposes); for query runs the four waves of a workgroup share the
-// fragments of a key block through LDS, each loading a quarter of them one block ahead.
+// instruction wants (no transposes); for query runs the waves of a workgroup (four, eight for heads wider
+// than 128) share the fragments of a key block through LDS, each loading its part of them a block or two ahead.
 //
 // Rows: row r of a (sequence, kv head) is (query token r / G, head r % G of the group), so the
 // G query heads that share a kv head share every K/V fragment.  A wave owns tiles of 16 rows;
@@ -40,11 +40,13 @@
 // Loads are never predicated: a lane without a valid page reads page 0 and its fragment is
 // cleared by a mask when it is consumed, so nothing waits on a load before its data is needed.
 //
-// Query runs: an item is 4 * RT consecutive row tiles of one (sequence, kv head), one tile set per
-//   wave; a workgroup takes the one or two items of a work row in turn (two: an early item with
-//   a late one, so that under the causal mask every workgroup walks about as many keys; one, the
-//   longest walks first in the grid, keeps more workgroups in flight and is what the engine's
-//   planner hands out).  The kv head is the grid's fastest index where the grid allows it:
+// Query runs: an item is 4 * RT consecutive row tiles of one (sequence, kv head), one tile set for each of
+//   four waves.  Up to 128 elements a workgroup is four waves and takes the one or two items of a
+//   work row in turn (two: an early item with a late one, so that under the causal mask every workgroup
+//   walks about as many keys; one, the longest walks first in the grid, keeps more workgroups in flight and
+//   is what the engine's planner hands out).  Wider heads have eight waves, four for each of a row's two
+//   items (or four idle but for staging), side by side over the keys that either item sees: the planner
+//   hands out neighbours, or single items where those are no more than the compute units.  The kv head is the grid's fastest index where the grid allows it:
 //   consecutive workgroups go to consecutive XCDs, so with eight kv heads an XCD walks the keys
 //   of one head only and finds them in its own L2.  Three or four stages are in
 //   flight: page lookups two or three blocks ahead, fragment loads one or two blocks ahead
@@ -408,7 +410,7 @@ __device__ __forceinline__ void setup_rows(const bf16_t* q, const MArgs& a, int 
 // ------------------------------------------------------------------------------------ query runs
 constexpr bool runs_pair(int dt) { return dt > 8; }
 // The waves stage the fragments of each key block in LDS for each other.
-// SINK: the softmax has a sink (a.sinks); a kernel without is the code it was before sinks came
+// SINK: the softmax has a sink (a.sinks)
 // NW: waves of the workgroup.  Eight stage half as much each as four do, and a key block is brought in for
 // twice the rows.  Heads wider than 128 have two items a work row, four waves each, side by side over the
 // keys that either sees; narrower ones one item of all the waves at a time.
@@ -503,7 +505,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
   }
 
   // fragment f of a block: K (tile f / DC, step f % DC) for f < N_K, then V^T element tiles;
-  // wave w stages fragments w, w + 4, ...
+  // wave w stages fragments w, w + NW, ...
   // What does not change from block to block is worked out once per fragment: the key a lane
   // reads relative to the block's start, and its offset inside a page apart from the key's slot
   // (in fragments of 16 bytes).
@@ -1159,7 +1161,7 @@ KVF_EXPORT void kvf_attn_mfma_set_split_waves(int waves) { g_split_waves = waves
 // Rows of a query run one workgroup takes with `row_tiles` (1 or 2) tiles per wave, where the
 // head size allows so many: 4 waves x tiles x 16 rows.
 KVF_EXPORT int kvf_attn_mfma_rows_per_item(int d, int row_tiles) {
-  const int most = d > 0 && d <= 128 ? 2 : 1;   // runs_max_rt(d / 16)
+  const int most = d > 0 ? runs_max_rt((d + 15) / 16) : 1;
   return WAVES * (row_tiles >= 2 ? most : 1) * 16;
 }
 

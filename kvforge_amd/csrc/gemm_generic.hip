@@ -178,11 +178,13 @@ template <> struct Quad<bf16_t> {
 // tile's walk along K otherwise.  The k-tile after the next is on its way into registers, two k-tiles lie
 // in LDS, and one barrier a k-tile is left: 0.66 us a k-tile of 64 x 64 alone, 0.98 with one k-tile ahead
 // and two barriers.  At 777 rows and a 16,384 / 3,072 / 2,048 x 2,048 and a 2,048 x 8,192 weight: 467, 110,
-// 81 and 302 us (112, 89, 81 and 86 TFLOP/s), 782, 224, 131 and 479 before.  Rows and columns past the end are read as the last and not stored, and what lies past K is
-// read inside the row and replaced by zero on its way into LDS: a load that stood against a zero under
-// a condition had become four loads of 4 bytes from a chosen address each, and half of the kernel's
-// time.  Consecutive workgroups go to the eight XCDs in turn; each XCD gets an unbroken eighth of the tiles,
-// the tiles that share columns of W side by side.
+// 81 and 302 us (112, 89, 81 and 86 TFLOP/s, 98 over the four), 782, 224, 131 and 479 before.
+// Rows and columns past the end are read as the last and not stored, and what lies past K (at least one
+// element: the caller checks) is read inside the row and replaced by zero on its way into LDS: a load that
+// stood against a zero under a condition had become four loads of 4 bytes from a chosen address each, and
+// half of the kernel's time.
+// Consecutive workgroups go to the eight XCDs in turn; each XCD gets an unbroken eighth of the tiles, the tiles
+// that share columns of W side by side.
 constexpr int XK = 32, XLD = XK + 4;   // LDS rows 144 bytes apart
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 

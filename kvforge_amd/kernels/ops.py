@@ -1277,8 +1277,8 @@ def prefill_rows_per_item(dtype: torch.dtype, head_dim: int, block_size: int, ro
 
 
 def prefill_takes_pairs(dtype: torch.dtype, head_dim: int, block_size: int) -> bool:
-    """Whether the kernel for query runs takes the two items of a work row side by side, so that rows are best made
-    of neighbouring items (heads wider than 128 on the matrix cores)."""
+    """Whether the kernel for query runs takes the two items of a work row side by side, so that rows of two are best
+    made of neighbouring items (heads wider than 128 on the matrix cores)."""
     return (attention_on_matrix_cores(dtype, block_size, head_dim)
             and bool(_fn("attn_mfma", "kvf_attn_mfma_prefill_pairs", [c_int])(int(head_dim))))
 
@@ -1311,7 +1311,7 @@ def attn_prefill(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
     (sequence row, item, item or -1) where a sequence has ``query_len * H/KV`` rows per kv head,
     an item covers ``rows_per_item`` of them (what ``prefill_rows_per_item`` gave when the rows
     were made; by default its answer for one row tile), and the items of one row are taken by
-    one workgroup in turn; rows start in the order given (the longest walks first).  ``v_pages`` are transposed:
+    one workgroup, in turn or side by side (``prefill_takes_pairs``); rows start in the order given (the longest walks first).  ``v_pages`` are transposed:
     ``[num_blocks, KV, head_dim, block_size]``.  ``slopes``: fp32 ``[H]``; the score of key ``j``
     for a query at position ``p`` of head ``h`` then is ``scale * q.k + slopes[h] * (j - p)``.
     ``keep_first``: with a window, the first so many keys of a sequence stay visible behind it.
