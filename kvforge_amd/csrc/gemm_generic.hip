@@ -4,8 +4,8 @@
 // activations are bf16).  No reduced-precision matrix instruction is used: operands stored in
 // bf16 are widened (exactly) before they are multiplied.
 //
-// Many rows (a portion of a prompt), rows of K that start on 16 bytes: tiles of 64 x 64 or 128 x 128
-// outputs on the matrix cores with v_mfma_f32_32x32x2_f32, which multiplies and adds in fp32
+// Many rows (a portion of a prompt), rows of K that start on 16 bytes: tiles of 16 to 128 rows x 64
+// outputs on the matrix cores with v_mfma_f32_16x16x4_f32, which multiplies and adds in fp32
 // (gemm_mfma32_kernel below).  Many rows otherwise, and kept for comparison: tiles of 64 x 64
 // outputs on the vector ALUs, every output summed
 // over k = 0..K-1 in that order by one thread.  Few rows (decode steps), where the product is
@@ -17,6 +17,8 @@
 // so results agree to rounding.
 //
 // Output modes: 0 = store as TO;  1 = add into a fp32 matrix (the residual stream).
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -153,142 +155,196 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const TA* __restrict__ A
 constexpr int SKC = 1024;    // elements of K per staged chunk of A
 constexpr int SQ = 4 * KVF_WAVE;  // elements of K a wave reads per step (16 bytes a lane)
 
+// four neighbouring elements: as they lie in memory, and as floats
 template <typename T> struct Quad;
 template <> struct Quad<float> {
-  static __device__ __forceinline__ float4 load(const float* p) { return *reinterpret_cast<const float4*>(p); }
+  typedef float4 Raw;
+  static __device__ __forceinline__ Raw raw(const float* p) { return *reinterpret_cast<const float4*>(p); }
+  static __device__ __forceinline__ float4 wide(const Raw& r) { return r; }
+  static __device__ __forceinline__ float4 load(const float* p) { return raw(p); }
+  static __device__ __forceinline__ void store(float* p, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+  }
 };
 template <> struct Quad<bf16_t> {
-  static __device__ __forceinline__ float4 load(const bf16_t* p) {
-    const uint2 r = *reinterpret_cast<const uint2*>(p);
+  typedef uint2 Raw;
+  static __device__ __forceinline__ Raw raw(const bf16_t* p) { return *reinterpret_cast<const uint2*>(p); }
+  static __device__ __forceinline__ float4 wide(const Raw& r) {
     return make_float4(__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u),
                        __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u));
+  }
+  static __device__ __forceinline__ float4 load(const bf16_t* p) { return wide(raw(p)); }
+  static __device__ __forceinline__ void store(bf16_t* p, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) =
+        make_uint2(static_cast<uint32_t>(f32_to_bf16(v[0])) | (static_cast<uint32_t>(f32_to_bf16(v[1])) << 16),
+                   static_cast<uint32_t>(f32_to_bf16(v[2])) | (static_cast<uint32_t>(f32_to_bf16(v[3])) << 16));
   }
 };
 
 // ---- many rows on the matrix cores, true fp32.
-// A workgroup of four waves owns XM x XN outputs; a wave owns a quarter of them, XM / 2 x XN / 2, as 32 x 32
-// tiles of v_mfma_f32_32x32x2_f32 (lane l supplies A[row l % 32][k = l / 32] and
-// W[column l % 32][k = l / 32], and holds 16 outputs of column l % 32).  K is walked in tiles of
-// 32.  Within a tile of 32 the two halves of the wave take k = 8u + e
-// and k = 8u + 4 + e in instruction (u, e), so that a lane reads its operands from LDS 16 bytes
-// at a time; the order of the sums is fixed by K alone, whatever the tile.  Rows of A and W start on 16
-// bytes (8 for bf16) and K is a multiple of 4: the caller checks.
+// A workgroup of four waves owns 16 RT rows x 64 columns of outputs; a wave owns 16 of the columns, as RT tiles of
+// v_mfma_f32_16x16x4_f32 with W as the first operand (lane 16 c + r supplies W[column r][k = c] and
+// A[row r][k = c], and holds columns 4 c .. 4 c + 3 of row r).  K is walked in tiles of 32.  A lane reads its operands
+// from LDS 16 bytes at a time, k = 16 u + 4 c .. + 3, so instruction (u, e) sums k = 16 u + e, + 4, + 8 and + 12: the
+// order of the sums is fixed by K alone, whatever the tile.  Rows of A and W start on 16 bytes (8 for bf16) and K is a
+// multiple of 4: the caller checks.
 //
-// What bounds it: the matrix cores (64 cycles an instruction) once several tiles share a compute unit, a
-// tile's walk along K otherwise.  The k-tile after the next is on its way into registers, two k-tiles lie
-// in LDS, and one barrier a k-tile is left: 0.66 us a k-tile of 64 x 64 alone, 0.98 with one k-tile ahead
-// and two barriers.  At 777 rows and a 16,384 / 3,072 / 2,048 x 2,048 and a 2,048 x 8,192 weight: 467, 110,
-// 81 and 302 us (112, 89, 81 and 86 TFLOP/s, 98 over the four), 782, 224, 131 and 479 before.
-// Rows and columns past the end are read as the last and not stored, and what lies past K (at least one
-// element: the caller checks) is read inside the row and replaced by zero on its way into LDS: a load that
-// stood against a zero under a condition had become four loads of 4 bytes from a chosen address each, and
-// half of the kernel's time.
-// Consecutive workgroups go to the eight XCDs in turn; each XCD gets an unbroken eighth of the tiles, the tiles
-// that share columns of W side by side.
-constexpr int XK = 32, XLD = XK + 4;   // LDS rows 144 bytes apart
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+// What bounds it: the matrix cores (32 cycles an instruction, 154 TFLOP/s when nothing else is done).  A k-tile's elements
+// are asked for three k-tiles ahead, two k-tiles lie in LDS, a wave holds the fragments of half a k-tile ahead, and what
+// is loaded, written and read is spread among the matrix instructions one by one: with the same work ahead of them
+// instead, 777 rows by 16,384 columns of 2,048 took 462 us, and now 386 (135 TFLOP/s; whole loads from 64-bit addresses
+// made anew for each and 32 x 32 tiles of v_mfma_f32_32x32x2_f32 on four separate waves 451).  The other products of such
+// a step: 3,072 and 2,048 x 2,048, 2,048 x 8,192: 82, 58 and 220 us, 108, 80 and 297 before.  2,048 rows: 997, 191, 127
+// and 492 us (135 to 140 TFLOP/s), 1,061, 224, 149 and 564 before.
+// Rows and columns past the end are read as the last and not stored.  Consecutive workgroups go to the eight XCDs in
+// turn; each XCD gets an unbroken eighth of the tiles, the tiles that share columns of W side by side.
+constexpr int XK = 32, XN = 64, XQ = XK / 4;   // elements of K and columns a tile, 16-byte pieces of a row
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <typename TA, typename TW, typename TO, int MODE, int XM, int XN>
-__global__ __launch_bounds__(256) void gemm_mfma32_kernel(const TA* __restrict__ A,
+// N times one matrix instruction and one of another kind, for the scheduler.
+template <int N, int MASK>
+__device__ __forceinline__ void spread() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(MASK, 1, 0);
+  }
+}
+
+template <typename TA, typename TW, typename TO, int MODE, int RT>
+__global__ __launch_bounds__(256, 2) void gemm_mfma32_kernel(const TA* __restrict__ A,
                                                           const TW* __restrict__ W,
                                                           TO* __restrict__ C, int M, int N, int K,
                                                           int lda, int ldc) {
-  constexpr int RT = XM / 64, CT = XN / 64;          // 32-row and 32-column tiles per wave
-  constexpr int AQ = XM / 32, WQ = XN / 32;          // float4 of A and W a thread stages per k-tile
-  __shared__ __align__(16) float As[2][XM][XLD];
-  __shared__ __align__(16) float Ws[2][XN][XLD];
+  constexpr int XM = 16 * RT;
+  constexpr int AQ = (XM + 31) / 32, WQ = XN / 32;   // 16-byte pieces of A and W a thread stages per k-tile
+  __shared__ float4 As[2][32 * AQ * XQ];
+  __shared__ float4 Ws[2][XN * XQ];
   const int down = (M + XM - 1) / XM, total = down * ((N + XN - 1) / XN), share = (total + 7) / 8;
   const int at = static_cast<int>(blockIdx.x / 8), item = static_cast<int>(blockIdx.x % 8) * share + at;
   if (at >= share || item >= total) return;
   const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE;
   const int m0 = item % down * XM, n0 = item / down * XN;
-  const int wm = (wave / 2) * (XM / 2), wn = (wave % 2) * (XN / 2);
-  const int r32 = lane % 32, half = lane / 32;
+  const int r16 = lane % 16, kg = lane / 16;
 
-  f32x16 acc[RT][CT];
+  f32x4 acc[RT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int j = 0; j < CT; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  for (int i = 0; i < RT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // what this thread stages: row srow + 32 i, elements skq .. skq + 3 of the k-tile
-  const int srow = tid / 8, skq = (tid % 8) * 4;
-  const TA* arow[AQ];
-  const TW* wrow[WQ];
+  // Piece q of row r lies at 8 r + (q ^ (r / 2 % 8)).  A 16-byte access serves lanes 0-3, 12-15 and 20-27 together,
+  // then 4-11, 16-19 and 28-31: either sixteen fall on all banks, written (row lane / 8, piece lane % 8) or read (row
+  // lane % 16, piece 4 u + lane / 16).
+  auto place = [](int row, int q) { return row * XQ + (q ^ (row / 2 % XQ)); };
+  const int srow = tid / XQ, sq = tid % XQ;        // staged: elements 4 sq .. + 3 of rows srow + 32 i
+  // a thread's pieces begin so many elements behind the tile's first row: 32 bits, the rest of an address is the same
+  // for all threads
+  uint32_t aoff[AQ], woff[WQ];
 #pragma unroll
-  for (int i = 0; i < AQ; ++i) arow[i] = A + static_cast<size_t>(min(m0 + srow + 32 * i, M - 1)) * lda;
+  for (int i = 0; i < AQ; ++i) aoff[i] = static_cast<uint32_t>(min(srow + 32 * i, M - 1 - m0)) * lda + 4 * sq;
 #pragma unroll
-  for (int i = 0; i < WQ; ++i) wrow[i] = W + static_cast<size_t>(min(n0 + srow + 32 * i, N - 1)) * K;
-  struct Staged { float4 a[AQ], w[WQ]; };
-  auto fetch = [&](int k0, Staged& f) {
-    const int k = min(k0 + skq, K - 4);
+  for (int i = 0; i < WQ; ++i) woff[i] = static_cast<uint32_t>(min(srow + 32 * i, N - 1 - n0)) * K + 4 * sq;
+  const TA* abase = A + static_cast<size_t>(m0) * lda;
+  const TW* wbase = W + static_cast<size_t>(n0) * K;
+  struct Staged { typename Quad<TA>::Raw a[AQ]; typename Quad<TW>::Raw w[WQ]; };
+  // WHOLE: the k-tile lies inside K.  Otherwise what lies past K is read inside the row and staged as zeros.
+  auto fetch = [&](auto whole, int k0, Staged& f) {
+    const int back = decltype(whole)::value ? 0 : max(k0 + 4 * sq - (K - 4), 0);
 #pragma unroll
-    for (int i = 0; i < AQ; ++i) f.a[i] = Quad<TA>::load(arow[i] + k);
+    for (int i = 0; i < AQ; ++i) f.a[i] = Quad<TA>::raw(abase + k0 + aoff[i] - back);
 #pragma unroll
-    for (int i = 0; i < WQ; ++i) f.w[i] = Quad<TW>::load(wrow[i] + k);
+    for (int i = 0; i < WQ; ++i) f.w[i] = Quad<TW>::raw(wbase + k0 + woff[i] - back);
   };
-  auto stage = [&](int k0, const Staged& f, int buf) {
-    const bool in = k0 + skq < K;
+  const int put_at = place(srow, sq);              // rows 32 apart are turned over alike
+  auto stage = [&](auto whole, int k0, const Staged& f, int buf) {
+    const bool in = decltype(whole)::value || k0 + 4 * sq < K;
     auto kept = [&](const float4& v) { return make_float4(in ? v.x : 0.f, in ? v.y : 0.f, in ? v.z : 0.f, in ? v.w : 0.f); };
 #pragma unroll
-    for (int i = 0; i < AQ; ++i) *reinterpret_cast<float4*>(&As[buf][srow + 32 * i][skq]) = kept(f.a[i]);
+    for (int i = 0; i < AQ; ++i) As[buf][put_at + 32 * XQ * i] = kept(Quad<TA>::wide(f.a[i]));
 #pragma unroll
-    for (int i = 0; i < WQ; ++i) *reinterpret_cast<float4*>(&Ws[buf][srow + 32 * i][skq]) = kept(f.w[i]);
+    for (int i = 0; i < WQ; ++i) Ws[buf][put_at + 32 * XQ * i] = kept(Quad<TW>::wide(f.w[i]));
   };
-  auto tile = [&](int k0, Staged& f, int buf) {
-    stage(k0, f, buf);       // its readers two tiles ago are past the barrier of the last one
-    fetch(k0 + 2 * XK, f);   // past the end: the row's last elements, not used
-    __syncthreads();
+  struct Frags { float4 a[RT], w; };
+  auto read = [&](int buf, int u, Frags& f) {
+    f.w = Ws[buf][place(16 * wave + r16, 4 * u + kg)];
 #pragma unroll
-    for (int u = 0; u < XK / 8; ++u) {
-      float4 a[RT], w[CT];
+    for (int i = 0; i < RT; ++i) f.a[i] = As[buf][place(r16, 4 * u + kg) + 16 * XQ * i];
+  };
+  auto product = [&](const Frags& f) {
 #pragma unroll
-      for (int i = 0; i < RT; ++i) a[i] = *reinterpret_cast<const float4*>(&As[buf][wm + 32 * i + r32][8 * u + 4 * half]);
+    for (int e = 0; e < 4; ++e) {
+      const float wv = e == 0 ? f.w.x : e == 1 ? f.w.y : e == 2 ? f.w.z : f.w.w;
 #pragma unroll
-      for (int j = 0; j < CT; ++j) w[j] = *reinterpret_cast<const float4*>(&Ws[buf][wn + 32 * j + r32][8 * u + 4 * half]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < RT; ++i)
-#pragma unroll
-          for (int j = 0; j < CT; ++j) {
-            const float av = e == 0 ? a[i].x : e == 1 ? a[i].y : e == 2 ? a[i].z : a[i].w;
-            const float wv = e == 0 ? w[j].x : e == 1 ? w[j].y : e == 2 ? w[j].z : w[j].w;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, wv, acc[i][j], 0, 0, 0);
-          }
+      for (int i = 0; i < RT; ++i) {
+        const float av = e == 0 ? f.a[i].x : e == 1 ? f.a[i].y : e == 2 ? f.a[i].z : f.a[i].w;
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, av, acc[i], 0, 0, 0);
+      }
     }
   };
 
-  Staged f0, f1;
-  fetch(0, f0);
-  fetch(XK, f1);
+  Frags f0, f1;
+  Staged s0, s1;
+  // One k-tile: its first fragments are in registers, the next k-tile's elements in `next` on their way.  What is read,
+  // written and asked for is spread among the matrix instructions, which are what takes the time.
+  auto tile = [&](auto whole, int k0, Staged& next, int buf) {
+    read(buf, 1, f1);
+    stage(whole, k0 + XK, next, buf ^ 1);   // its readers are past the last barrier
+    fetch(whole, k0 + 3 * XK, next);
+    product(f0);
+    spread<RT + 1, 0x100>();
+    spread<AQ + WQ, 0x200>();
+    spread<AQ + WQ, 0x020>();
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * RT, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    read(buf ^ 1, 0, f0);
+    product(f1);
+    spread<RT + 1, 0x100>();
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * RT, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr std::true_type WHOLE{};
+  constexpr std::false_type PART{};
+  fetch(PART, 0, s0);
+  fetch(PART, XK, s1);
+  stage(PART, 0, s0, 0);
+  fetch(PART, 2 * XK, s0);
+  __syncthreads();
+  read(0, 0, f0);
   int k0 = 0;
-  for (; k0 + XK < K; k0 += 2 * XK) {
-    tile(k0, f0, 0);
-    tile(k0 + XK, f1, 1);
+#pragma unroll 1
+  for (; k0 + 5 * XK <= K; k0 += 2 * XK) {
+    tile(WHOLE, k0, s1, 0);
+    tile(WHOLE, k0 + XK, s0, 1);
   }
-  if (k0 < K) tile(k0, f0, 0);
-  // output v of a lane: row 8 (v / 4) + 4 (lane / 32) + v % 4 of the tile, column lane % 32
+#pragma unroll 1
+  for (; k0 < K; k0 += 2 * XK) {
+    tile(PART, k0, s1, 0);
+    if (k0 + XK < K) tile(PART, k0 + XK, s0, 1);
+  }
+  const int n = n0 + 16 * wave + 4 * kg;
+  if (n >= N) return;
+  // four neighbouring columns at once where they exist and start on their size
+  const bool whole = n + 4 <= N && ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % (4 * sizeof(TO)) == 0;
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+  for (int i = 0; i < RT; ++i) {
+    const int m = m0 + 16 * i + r16;
+    if (m >= M) continue;
+    TO* c = C + static_cast<size_t>(m) * ldc + n;
+    float v[4] = {acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+    if (whole) {
+      if (MODE == 1) {
+        const float4 old = Quad<TO>::load(c);
+        v[0] += old.x; v[1] += old.y; v[2] += old.z; v[3] += old.w;
+      }
+      Quad<TO>::store(c, v);
+    } else {
 #pragma unroll
-    for (int j = 0; j < CT; ++j) {
-      const int n = n0 + wn + 32 * j + r32;
-      if (n >= N) continue;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm + 32 * i + 8 * (v / 4) + 4 * half + v % 4;
-        if (m >= M) continue;
-        TO* c = C + static_cast<size_t>(m) * ldc + n;
-        if (MODE == 1) {
-          Elem<TO>::store(c, Elem<TO>::load(c) + acc[i][j][v]);
-        } else {
-          Elem<TO>::store(c, acc[i][j][v]);
-        }
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) break;
+        Elem<TO>::store(c + e, MODE == 1 ? Elem<TO>::load(c + e) + v[e] : v[e]);
       }
     }
+  }
 }
 
 // MT rows per workgroup (1, 2, 4, 8 or 16); SN columns of W per wave, each read DEPTH steps
@@ -409,6 +465,26 @@ int compute_units() {
   return known[dev];
 }
 
+// Rows a tile holds of the fp32 product on the matrix cores, in sixteens: the fewest rounds of tiles over the compute
+// units, a tile's time being its rows' matrix instructions and about those of another sixteen rows for the walk along
+// K itself (one tile a compute unit, K 2,048: 20 us for 32 rows, 64 for 128).  Among equals the most rows, which read W
+// least often.  777 rows by 16,384 columns: 386 us with the 112 rows it chooses, 394 to 437 with 32 to 128; by 2,048:
+// 58, against 59 to 94.
+constexpr int MFMA32_MAX_ROW = 1 << 24;
+int mfma32_row_tiles(int M, int N) {
+  const long cus = compute_units(), across = (N + XN - 1) / XN;
+  int best = 8;
+  long least = -1;
+  for (int rt = 8; rt >= 1; --rt) {
+    const long cost = (across * ((M + 16 * rt - 1) / (16 * rt)) + cus - 1) / cus * (rt + 1);
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = rt;
+    }
+  }
+  return best;
+}
+
 template <typename TA, typename TW, typename TO, int MODE>
 int launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldc,
            hipStream_t s) {
@@ -433,23 +509,19 @@ int launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, 
                        N, K, lda, ldc);
     return kvf_last_error();
   }
-  if (quads && K > 0 && !g_vector_alus_only) {   // (its loads need an element of K to be clamped to)
-#define TILES(XM, XN)                                                                            \
-  do {                                                                                           \
-    const int total = ((N + XN - 1) / XN) * ((M + XM - 1) / XM);                                 \
-    hipLaunchKernelGGL((gemm_mfma32_kernel<TA, TW, TO, MODE, XM, XN>), dim3((total + 7) / 8 * 8), \
+  // (its loads need an element of K to be clamped to, and a tile's rows within 32 bits of each other)
+  if (quads && K > 0 && K < MFMA32_MAX_ROW && lda < MFMA32_MAX_ROW && !g_vector_alus_only) {
+#define TILES(RT)                                                                                \
+  case RT: {                                                                                     \
+    const int total = ((N + XN - 1) / XN) * ((M + 16 * RT - 1) / (16 * RT));                     \
+    hipLaunchKernelGGL((gemm_mfma32_kernel<TA, TW, TO, MODE, RT>), dim3((total + 7) / 8 * 8),    \
                        dim3(256), 0, s, static_cast<const TA*>(A), static_cast<const TW*>(W),    \
                        static_cast<TO*>(C), M, N, K, lda, ldc);                                  \
-  } while (0)
-    // Tiles of 64 x 64 unless tiles of 128 x 128 give every compute unit three or more to go through and
-    // leave the busiest one no more to do, by the 6% that they are faster once many are under way:
-    // 16,384 columns of 2,048 elements, 2,048 rows 1,123 against 1,198 us, 1,000 rows 534 against 563, but
-    // 777 rows 606 against 467 and 512 rows 294 against 287; 2,048 columns, 2,048 rows 163 against 148.
-    const long cus = compute_units();
-    auto tiles = [&](long side) { return ((N + side - 1) / side) * ((M + side - 1) / side); };
-    auto rounds = [&](long side) { return (tiles(side) + cus - 1) / cus; };
-    if (tiles(128) >= 3 * cus && 15 * 4 * rounds(128) <= 16 * rounds(64)) TILES(128, 128);
-    else TILES(64, 64);
+    break;                                                                                       \
+  }
+    switch (mfma32_row_tiles(M, N)) {
+      TILES(1) TILES(2) TILES(3) TILES(4) TILES(5) TILES(6) TILES(7) TILES(8)
+    }
 #undef TILES
     return kvf_last_error();
   }

@@ -607,7 +607,7 @@ def test_gemm_generic_few_rows_over_long_and_uneven_k(m, tw):
 @pytest.mark.parametrize("mnk", [(33, 130, 96), (200, 70, 260), (129, 257, 2052), (300, 1000, 64),
                                  (128, 128, 32), (260, 4100, 36)])
 def test_gemm_generic_many_rows_on_the_matrix_cores(ta, tw, mnk):
-    """More than 32 rows with rows of K that start on 16 bytes go to v_mfma_f32_32x32x2_f32:
+    """More than 32 rows with rows of K that start on 16 bytes go to v_mfma_f32_16x16x4_f32:
     32-bit multiply and add, so 32-bit operands that bfloat16 cannot hold give a 64-bit product's
     result to 32-bit rounding; tails in M, N and K, tiles of 128 and of 64 columns, both ways of
     storing and adding into the stream.  A row's result does not depend on the rows around it, and
@@ -673,6 +673,32 @@ def test_gemm_generic_tiles_of_both_sizes(tw, k):
     acc = torch.ones(1000, 12260, device=DEV)
     ops().gemm(a, w, acc, accumulate=True)
     assert torch.equal(acc, out + 1.0)
+
+
+@pytest.mark.parametrize("k", [4, 60, 160, 164, 228])
+@pytest.mark.parametrize("sixteens", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_gemm_generic_tiles_of_every_height(sixteens, k):
+    """2,046 columns make 32 tiles, so 256 compute units go through 128 x ``sixteens`` rows in one round of tiles of
+    so many sixteens.  K up to and past the whole tiles that the main loop asks for ahead, a part of one at its end;
+    rows and columns that end inside a tile, their last elements not finite: bit against bit with 40 of the rows (tiles
+    of sixteen), and against a 64-bit product."""
+    m, n = 128 * sixteens - 3, 2046
+    g = torch.Generator().manual_seed(m + k)
+    a = torch.randn(m, k, generator=g).to(DEV)
+    w = (torch.randn(n, k, generator=g) * 0.1).to(DEV)
+    a[5, k - 1], w[7, k - 1] = float("inf"), float("nan")
+    out = torch.full((m, n), 7.0, device=DEV)
+    ops().gemm(a, w, out)
+    assert bool(out[:, 7].isnan().all()) and not bool(out[5].isfinite().any())
+    rows = [r for r in range(m) if r != 5]
+    cols = [c for c in range(n) if c != 7]
+    x, y = a[rows].double(), w[cols].double()
+    # every sum adds k terms: k 2^-24 of the sum of their magnitudes at most
+    bound = k * 2.0 ** -24 * (x.abs() @ y.abs().T) + 1e-30
+    assert bool(((out[rows][:, cols].double() - x @ y.T).abs() <= bound).all())
+    part = torch.empty(40, n, device=DEV)
+    ops().gemm(a[m - 40:], w, part)
+    assert torch.equal(part[:, cols], out[m - 40:][:, cols])
 
 
 @pytest.mark.parametrize("tw", DTYPES)
