@@ -1,5 +1,7 @@
 // Routed experts: the router's choice per token, and the row-wise steps around the experts'
 // matrix products.  Router arithmetic is fp32 throughout.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -151,7 +153,8 @@ __global__ __launch_bounds__(256) void moe_identity_kernel(float* __restrict__ x
 //
 // moe_plan: the (token, choice) pairs are grouped by expert: where[pair] is the pair's place in
 // that order (-1 for a choice that names no expert), order[place] the pair; every expert's rows
-// are cut into tiles of up to 2^tile_shift: tiles[t] = (expert, first place, rows).  One workgroup; the order of
+// are cut into tiles of up to 2^tile_shift: tiles[t] = (expert | the tile's place among the expert's tiles << 9, first
+// place, rows | how many tiles the expert has << 8).  One workgroup; the order of
 // an expert's rows among themselves is whatever the atomics give, which no result depends on
 // (a row's products do not depend on its neighbours).  What bounds it is one workgroup's chain of trips: choices,
 // counters in LDS, sums over the experts, stores.  Up to 8,192 pairs the choices and their places stay in
@@ -159,9 +162,14 @@ __global__ __launch_bounds__(256) void moe_identity_kernel(float* __restrict__ x
 // and 24 pairs 19.4 us (20.3 with both passes over memory and sums over all 512 places).
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-constexpr int PLAN_MAX_EXPERTS = 512;
+constexpr int PLAN_EXPERT_BITS = 9, PLAN_MAX_EXPERTS = 1 << PLAN_EXPERT_BITS, PLAN_ROWS_BITS = 8;
 constexpr int PLAN_BATCH = 8;      // choices a thread of the plan has in flight
 constexpr int PREFETCH_SETS = 3;   // sets of operand registers in flight in the kernels of few rows
+
+__device__ __forceinline__ int tile_expert(const int* tiles, int t) { return tiles[3 * t] & (PLAN_MAX_EXPERTS - 1); }
+__device__ __forceinline__ int tile_in_expert(const int* tiles, int t) { return tiles[3 * t] >> PLAN_EXPERT_BITS; }
+__device__ __forceinline__ int tile_rows(const int* tiles, int t) { return tiles[3 * t + 2] & ((1 << PLAN_ROWS_BITS) - 1); }
+__device__ __forceinline__ int tiles_in_expert(const int* tiles, int t) { return tiles[3 * t + 2] >> PLAN_ROWS_BITS; }
 
 __device__ __forceinline__ uint2 pack4(const f32x4& a) {
   return make_uint2(static_cast<uint32_t>(f32_to_bf16(a[0])) | (static_cast<uint32_t>(f32_to_bf16(a[1])) << 16),
@@ -233,9 +241,9 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     if (nt > 1) each_has = ((c + nt - 1) / nt + 15) / 16 * 16;
     for (int i = 0; i < nt && first_tile[tid] + i < max_tiles; ++i) {
       int* t = tiles + 3 * (first_tile[tid] + i);
-      t[0] = tid;
+      t[0] = tid | i << PLAN_EXPERT_BITS;
       t[1] = off[tid] + i * each_has;
-      t[2] = min(each_has, c - i * each_has);
+      t[2] = min(each_has, c - i * each_has) | nt << PLAN_ROWS_BITS;
     }
   }
   for (int p0 = tid; p0 < pairs; p0 += PLAN_BATCH * step) {
@@ -295,7 +303,7 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* __restrict__ 
                                                      bf16_t* __restrict__ act) {
   const int tile = blockIdx.y;
   if (tile >= *num_tiles) return;
-  const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  const int e = tile_expert(tiles, tile), row0 = tiles[3 * tile + 1], rows = tile_rows(tiles, tile);
   const int lane = threadIdx.x % KVF_WAVE, wave = threadIdx.x / KVF_WAVE;
   const int j = lane % 16, c = lane / 16;
   const int groups = ff / 8, g = blockIdx.x * 4 + wave;   // groups of 16 interleaved rows per expert
@@ -325,7 +333,7 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const bf16_t* __restrict_
                                                        bf16_t* __restrict__ y, int hidden) {
   const int tile = blockIdx.y;
   if (tile >= *num_tiles) return;
-  const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  const int e = tile_expert(tiles, tile), row0 = tiles[3 * tile + 1], rows = tile_rows(tiles, tile);
   const int lane = threadIdx.x % KVF_WAVE, wave = threadIdx.x / KVF_WAVE;
   const int j = lane % 16, c = lane / 16;
   const int groups = (hidden + 15) / 16, g = blockIdx.x * 4 + wave;
@@ -350,28 +358,32 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const bf16_t* __restrict_
 //
 // What bounds it: the experts' matrices come from memory once (32 experts of 2,048 x 1,024: 403 MB, 80 us
 // at the 5 TB/s of a large copy), the other tiles of an expert find them in their XCD's L2 (see
-// wide_item).  A wave needs its own weight fragments only, so they go straight into registers; the rows,
-// which all four waves need, are gathered through LDS, 64 elements of K at a time in two buffers.  Both
-// are asked for one pass ahead, and three workgroups a compute unit cover what that leaves of the way to
-// memory.  Rows past an expert's last are read as its last and not stored; tiles of up to 96, 64 and 32
+// wide_item).  A wave needs its own weight fragments only, so they go straight into registers; the rows, which
+// all four waves need, are gathered through LDS, 64 elements of K at a time in two buffers.  Weights are asked for
+// two passes ahead, into the registers of those just used, rows three, and each of these loads stands between
+// two products.  Rows past an expert's last are read as its last and not stored; tiles of up to 96, 64 and 32
 // rows leave the other matrix instructions out.
 //
-// Up and down together with plan and sum, 2,048 tokens, 4 of 32 experts (ff 1,024 / 2,048): 200 / 358 us,
-// where tiles of 64 rows with every fragment straight from memory took 354 / 621.  On the way: 256
-// weight rows a workgroup, two of them a compute unit 215 / 364 (512 equal workgroups leave 40 for a
-// second round); 256 rows and 256 weight rows, eight waves 245 / 390; fragments read from LDS where they
-// are needed instead of two ahead 230 / 380.
+// Up and down together with plan and sum, 32 experts, 4 chosen, 2,048 wide.  2,047 tokens: 304 us at ff 2,048, 171 at
+// 1,024 (333 and 173 with an expert's tiles one behind the other, where both came from memory anew: 1.26 GB read
+// instead of 0.63; 307 and 170 with that mended alone).  180 tokens at 2,048: 148 (161), 5.4 TB/s.  On the way: 256 weight rows
+// a workgroup in 512 registers a lane 360 / 228; two workgroups a compute unit instead of three the same.
 constexpr int WIDE_SHIFT = 7, WIDE_ROWS = 1 << WIDE_SHIFT, WIDE_GW = 2;
 
 // What a workgroup takes: tile and block of columns.  Workgroups go to the eight XCDs in turn, and each
-// XCD gets an unbroken eighth of the (tile, block) pairs, the blocks of a tile side by side and the tiles of an
-// expert next to each other: an expert's rows and its matrices are then read into one XCD's L2 each.
-__device__ __forceinline__ bool wide_item(int num_tiles, int blocks, int& tile, int& block) {
+// XCD gets an unbroken eighth of the (expert, block, tile) triples: the tiles of an expert that read the same weight rows
+// start together and walk K side by side, so the L2 (4 MB, a fifth of an expert's matrices at ff 2,048) brings those in
+// once, and the expert's rows stay there over its blocks.
+__device__ __forceinline__ bool wide_item(const int* tiles, int num_tiles, int blocks, int& tile, int& block) {
   const int total = num_tiles * blocks, share = (total + 7) / 8, at = blockIdx.x / 8;
   const int item = static_cast<int>(blockIdx.x % 8) * share + at;
-  tile = item / blocks;
-  block = item % blocks;
-  return at < share && item < total;
+  if (at >= share || item >= total) return false;
+  const int some = item / blocks;                    // a tile of the item's expert
+  const int first = some - tile_in_expert(tiles, some), count = tiles_in_expert(tiles, some);
+  const int in = item - first * blocks;
+  block = in / count;
+  tile = first + in % count;
+  return true;
 }
 template <int N> struct Rows { static constexpr int value = N; };
 template <class F> __device__ __forceinline__ void wide_rows(int rows, const F& go) {
@@ -379,6 +391,17 @@ template <class F> __device__ __forceinline__ void wide_rows(int rows, const F& 
   else if (rows > 64) go(Rows<6>{});
   else if (rows > 32) go(Rows<4>{});
   else go(Rows<2>{});
+}
+
+// For the scheduler, N times: a row fragment's products, the read of another fragment, an instruction of a third kind.
+template <int N, int MASK>
+__device__ __forceinline__ void beside_products() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, WIDE_GW, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(MASK, 1, 0);
+  }
 }
 
 template <int RT> struct WideAcc { f32x4 v[RT][WIDE_GW]; };
@@ -401,74 +424,84 @@ __device__ __forceinline__ void wide_product(const RowOf& row_of, int K, const u
   const int put_at = ((sr / 16) * 2 + ch / 4) * KVF_WAVE + place(sr % 16, ch % 4);
   const int get_at = place(lane % 16, lane / 16);
   // No load stands under a condition: where paths with and without one meet, the compiler waits for the
-  // newest loads before the first product, and nothing is ahead of anything any more.
-  uint4 stage[PASSES];
-  auto fetch = [&](int it) {
-    const int k = min(64 * it, K - 8 - 8 * ch);      // K is a multiple of 8: past it a row's last 8, see put
+  // newest loads before the first product, and nothing is ahead of anything any more.  WHOLE: the pass lies inside K.
+  using Stage = uint4[PASSES];
+  auto fetch = [&](auto whole, int it, Stage& stage) {
+    const int k = decltype(whole)::value ? 64 * it : min(64 * it, K - 8 - 8 * ch);   // K is a multiple of 8: past it a row's last 8, see put
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) stage[p] = *reinterpret_cast<const uint4*>(src[p] + k);
   };
-  auto put = [&](int it) {
-    const bool in = 64 * it + 8 * ch < K;
+  auto put = [&](auto whole, int it, const Stage& stage) {
+    const bool in = decltype(whole)::value || 64 * it + 8 * ch < K;
     uint4* to = lds + (it & 1) * RT * 2 * KVF_WAVE + put_at;
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) to[p * 4 * KVF_WAVE] = in ? stage[p] : make_uint4(0u, 0u, 0u, 0u);
   };
   using Weights = uint4[2][WIDE_GW];
-  auto weights = [&](int it, Weights& w) {
+  auto weights = [&](int it, int h, Weights& w) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int g = 0; g < WIDE_GW; ++g) w[h][g] = (wbase + goff[g] + static_cast<size_t>(min(2 * it + h, S - 1)) * KVF_WAVE)[lane];
+    for (int g = 0; g < WIDE_GW; ++g) w[h][g] = (wbase + goff[g] + static_cast<size_t>(min(2 * it + h, S - 1)) * KVF_WAVE)[lane];
   };
-  // The products of a pass's first `halves` 32 elements.  Row fragments are read two ahead of the one in
-  // use; left alone the compiler reads each where it is needed, and every four products wait for LDS.
-  auto product = [&](int it, auto halves, const Weights& w) {
-    constexpr int N = RT * decltype(halves)::value;
+  auto product = [&](int it, int h, const Weights& w) {
     const uint4* frag = lds + (it & 1) * RT * 2 * KVF_WAVE + get_at;
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int h = i / RT, r = i % RT;
+    for (int r = 0; r < RT; ++r) {
       const bf16x8 x = __builtin_bit_cast(bf16x8, frag[(2 * r + h) * KVF_WAVE]);
 #pragma unroll
       for (int g = 0; g < WIDE_GW; ++g)
         acc.v[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[h][g]), x, acc.v[r][g], 0, 0, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-#pragma unroll
-    for (int i = 0; i < N - 2; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, WIDE_GW, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, 2 * WIDE_GW, 0);
   };
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int g = 0; g < WIDE_GW; ++g) acc.v[r][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Weights now, next;
-  fetch(0);
-  weights(0, now);
-  put(0);
-  fetch(1);
-  const int passes = S / 2;                          // whole ones; an odd step is left over
-#pragma unroll 1
-  for (int it = 0; it < passes; ++it) {
+  // A pass: rows of the next go from registers to LDS, those of the third from here are asked for, and so are the
+  // weights of the one after the next as soon as these have been used.
+  auto pass = [&](auto whole, int it, Weights& w, Stage& stage) {
     __syncthreads();                                 // this pass's rows are there, the other buffer is free
-    put(it + 1);
-    fetch(it + 2);
-    weights(it + 1, next);
-    __builtin_amdgcn_sched_barrier(0);               // all loads first, and no sums held elsewhere
-    product(it, Rows<2>{}, now);
+    put(whole, it + 1, stage);
+    fetch(whole, it + 3, stage);
+    product(it, 0, w);
+    weights(it + 2, 0, w);
+    product(it, 1, w);
+    weights(it + 2, 1, w);
+    // row fragments two ahead of the one in use, then everything else one by one between the products
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    beside_products<PASSES, 0x200>();
+    beside_products<RT - PASSES, 0x020>();
+    beside_products<RT - 2, 0x020>();
+    __builtin_amdgcn_sched_group_barrier(0x008, 2 * WIDE_GW, 0);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int g = 0; g < WIDE_GW; ++g) now[h][g] = next[h][g];
+  };
+  constexpr std::true_type WHOLE{};
+  constexpr std::false_type PART{};
+  Weights w0, w1;
+  Stage s0, s1;
+  fetch(PART, 0, s0);
+  fetch(PART, 1, s1);
+  weights(0, 0, w0);
+  weights(0, 1, w0);
+  weights(1, 0, w1);
+  weights(1, 1, w1);
+  put(PART, 0, s0);
+  fetch(PART, 2, s0);
+  const int passes = S / 2;                          // whole ones; an odd step is left over
+  int it = 0;
+#pragma unroll 1
+  for (; 64 * (it + 5) <= K; it += 2) {
+    pass(WHOLE, it, w0, s1);
+    pass(WHOLE, it + 1, w1, s0);
+  }
+#pragma unroll 1
+  for (; it < passes; it += 2) {
+    pass(PART, it, w0, s1);
+    if (it + 1 < passes) pass(PART, it + 1, w1, s0);
   }
   if (S % 2) {
     __syncthreads();
-    product(passes, Rows<1>{}, now);
+    if (passes % 2) product(passes, 0, w1);
+    else product(passes, 0, w0);
   }
 }
 
@@ -514,8 +547,8 @@ __global__ __launch_bounds__(256, 3) void moe_up_wide_kernel(const bf16_t* __res
                                                              bf16_t* __restrict__ act) {
   __shared__ uint4 lds[2 * WIDE_ROWS * 8];
   int tile, block;
-  if (!wide_item(*num_tiles, (ff / 8 + 4 * WIDE_GW - 1) / (4 * WIDE_GW), tile, block)) return;
-  const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  if (!wide_item(tiles, *num_tiles, (ff / 8 + 4 * WIDE_GW - 1) / (4 * WIDE_GW), tile, block)) return;
+  const int e = tile_expert(tiles, tile), row0 = tiles[3 * tile + 1], rows = tile_rows(tiles, tile);
   auto go = [&](auto rt) { wide_up_tile<decltype(rt)::value>(x, ldx, K, wt, S, order, e, row0, rows, block, top, ff, in_wgt, f, act, lds); };
   wide_rows(rows, go);
 }
@@ -555,8 +588,8 @@ __global__ __launch_bounds__(256, 3) void moe_down_wide_kernel(const bf16_t* __r
                                                                bf16_t* __restrict__ y, int hidden) {
   __shared__ uint4 lds[2 * WIDE_ROWS * 8];
   int tile, block;
-  if (!wide_item(*num_tiles, ((hidden + 15) / 16 + 4 * WIDE_GW - 1) / (4 * WIDE_GW), tile, block)) return;
-  const int e = tiles[3 * tile], row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  if (!wide_item(tiles, *num_tiles, ((hidden + 15) / 16 + 4 * WIDE_GW - 1) / (4 * WIDE_GW), tile, block)) return;
+  const int e = tile_expert(tiles, tile), row0 = tiles[3 * tile + 1], rows = tile_rows(tiles, tile);
   auto go = [&](auto rt) { wide_down_tile<decltype(rt)::value>(act, ff, wt, S_all, e, row0, rows, block, y, hidden, lds); };
   wide_rows(rows, go);
 }

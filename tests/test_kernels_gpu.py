@@ -1408,3 +1408,11 @@ def test_grouped_experts_at_the_edges_of_their_tiles(counts, K, ff, weigh_input)
         want += w[:, 1:].double() * x.double()
     err = (got.cpu().double() - want).abs()
     assert bool((err <= slack + 1e-5 * (1 + want.abs())).all()), float((err - slack).max())
+
+
+@pytest.mark.parametrize("K,ff", [(320, 320), (328, 352), (392, 384), (456, 416)])
+@pytest.mark.parametrize("weigh_input", [False, True])
+def test_grouped_experts_over_rows_of_many_passes(K, ff, weigh_input):
+    """Tiles of every height over rows of five to seven passes of 64 elements, where the loads of the last ones stand
+    ahead of the row's end, whole and part passes, odd steps; one expert of several tiles."""
+    test_grouped_experts_at_the_edges_of_their_tiles([20, 40, 290, 70, 128], K, ff, weigh_input)
