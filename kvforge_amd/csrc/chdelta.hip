@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256) void chdelta_scan_kernel(const float* __restri
 // A thread per (key channel, block of 16 tokens): it keeps the channel's q, k, decays and products over the
 // block in registers, and puts the level's scaled rows down in LDS for all waves.
 // chunks: rows (sequence, first token, tokens, 0).  T, A [chunks, H, CL, CL] (blocks above the diagonal are not
-// written), E [chunks, H, dk] = P(0, L), Kd, Kw, Qd [tokens, H, dk].
+// written), E [chunks, H, dk] = P(0, L), Kd, Qd [tokens, H, dk], Kw [chunks, H, dk, CL].
 template <int DKP, int CL> constexpr int solve_threads() { return DKP * (CL / 16); }
 template <int DKP, int CL> constexpr size_t solve_lds() {
   return 4 * (3 * CL * (DKP + 4) + 2 * CL * (CL + 4) + (CL / 16) * DKP + CL);
@@ -320,7 +320,14 @@ __global__ __launch_bounds__(DKP * (CL / 16)) void chdelta_solve_kernel(
       const float x = pre[j] * before;
       Kd[o] = k[j] * x;
       Qd[o] = q[j] * x;
-      Kw[o] = k[j] * (suf[j] * behind);
+    }
+    f32x4* kw = reinterpret_cast<f32x4*>(Kw + ((static_cast<size_t>(chunk) * a.H + head) * dk + ch) * CL + 16 * sub);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {   // zeros past the chunk's tokens, whose k are
+      f32x4 v;
+#pragma unroll
+      for (int y = 0; y < 4; ++y) v[y] = k[4 * j + y] * (suf[4 * j + y] * behind);
+      kw[j] = v;
     }
     if (sub == 0) E[(static_cast<size_t>(chunk) * a.H + head) * dk + ch] = pre[15] * behind;
   }
@@ -368,144 +375,220 @@ __global__ __launch_bounds__(DKP * (CL / 16)) void chdelta_solve_kernel(
   }
 }
 
-struct RowArgs {
-  int ld, dk;
-};
-
 // runs: rows (sequence, first chunk, chunks).  Workgroup (head, 16 value columns, run): the heads are the grid's
 // fastest index, so with eight heads or a multiple the slices of a head, which read the same Kd, Kw and T, lie on
-// one XCD and find them in its L2.  A chunk's Kd, Kw, T, V
-// and P(0, L) are asked for while the chunk before is worked on.  W [chunks, H, dk, dv] receives the state
-// before every chunk, U [tokens, H, dv] the chunks' u.
+// one XCD and find them in its L2.  W [chunks, H, dk, dv] receives the state before every chunk, U [tokens, H, dv] the
+// chunks' u.
+//
+// What bounds it: a chunk waits for the state of the one before, and a chunk is three products one after the other, each
+// a chain of up to 32 matrix instructions.  So nothing else may stand in the chain: a wave's left operands (16 rows of Kd
+// and T, the rows of Kw that belong to its part of the state, which chdelta_solve leaves turned round) go from memory
+// into registers as they are, those of the chunk after the next asked for as soon as a chunk's have been used; a wave's part of
+// the state stays in registers; LDS carries only what the waves exchange, S, R and U, one barrier each.  2,047 tokens, 16
+// heads of 128 x 128: 91 us (142 with Kd, Kw and T staged in LDS for all waves, five barriers a chunk); 66 of them are the chain,
+// the rest what 80 KB a chunk cost a compute unit.  (Pulling the operands into L2 five chunks ahead changed nothing.)
 constexpr int DCOLS = 16;
-template <int DKP, int CL> constexpr size_t delta_lds() {
-  return 4 * (DKP + 2 * CL * (DKP + 4) + CL * (CL + 4) + 3 * DCOLS * (CL + 4) + DCOLS * (DKP + 4));
-}
-template <int DKP, int CL, bool VEC>
+// VEC: as load_four has it.  WHOLE: heads of DKP channels and value columns in whole sixteens, so that only a run's last
+// chunk has anything to leave out.
+template <int DKP, int CL, bool VEC, bool WHOLE>
 __global__ __launch_bounds__(256) void chdelta_delta_kernel(
     const float* __restrict__ rows, const int* __restrict__ chunks, const int* __restrict__ runs,
     const int* __restrict__ positions, const int* __restrict__ slot_ids, float* __restrict__ state,
     const float* __restrict__ T, const float* __restrict__ E, const float* __restrict__ Kd, const float* __restrict__ Kw,
     float* __restrict__ W, float* __restrict__ U, ChArgs a) {
-  extern __shared__ __align__(16) float lds[];
-  constexpr int QLD = DKP + 4, TLD = CL + 4, RT = CL / 16;
-  float* el = lds;                               // [DKP] P(0, L)
-  float* Kds = el + DKP;                         // [CL][QLD]
-  float* Kws = Kds + CL * QLD;                   // [CL][QLD]
-  float* Tb = Kws + CL * QLD;                    // [CL][TLD]
-  float* Vt = Tb + CL * TLD;                     // [DCOLS][TLD]
-  float* Rt = Vt + DCOLS * TLD;                  // [DCOLS][TLD]
-  float* Ut = Rt + DCOLS * TLD;                  // [DCOLS][TLD]
-  float* St = Ut + DCOLS * TLD;                  // [DCOLS][QLD]
+  constexpr int QLD = DKP + 4, TLD = CL + 4, RT = CL / 16, KT = DKP / 16, MINE = (KT + 3) / 4;
+  __shared__ __align__(16) float Rt[DCOLS * TLD], Ut[DCOLS * TLD], St[DCOLS * QLD];
   const int head = blockIdx.x, col0 = blockIdx.y * DCOLS;
   const int seq = runs[3 * blockIdx.z], c0 = runs[3 * blockIdx.z + 1], nc = runs[3 * blockIdx.z + 2];
-  const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE, l16 = lane % 16, lq = lane / 16;
-  const int dk = a.dk, dv = a.dv;
+  const int tid = threadIdx.x, lane = tid % KVF_WAVE, l16 = lane % 16, lq = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / KVF_WAVE);
+  const int dk = WHOLE ? DKP : a.dk, dv = a.dv, c = col0 + l16;
+  const bool c_ok = WHOLE || c < dv;
   int slot = slot_ids[seq];
   if (slot < 0 || slot >= a.n_slots) slot = -1;
   float* S_slot = slot >= 0 ? state + static_cast<size_t>(slot) * a.slot_stride + static_cast<size_t>(head) * dk * dv
                             : nullptr;
   const bool resume = slot >= 0 && positions[chunks[4 * c0 + 1]] > 0;
-  for (int i = tid; i < DKP * DCOLS; i += 256) {
-    const int r = i / DCOLS, cl = i % DCOLS, c = col0 + cl;
-    St[cl * QLD + r] = (resume && r < dk && c < dv) ? S_slot[static_cast<size_t>(r) * dv + c] : 0.f;
-  }
-  const RowArgs ka{a.H * dk, dk};
-  const int k_off = head * dk, v_off = a.v_off + head * dv;
-  constexpr int NT = CL * CL / 4 / 256;
-  StagedRows<DKP, CL, 256, VEC> kd, kw;
-  StagedTurned<CL, DCOLS, 256, TLD> vs;
-  f32x4 treg[NT];
-  float ereg = 0.f;
-  auto ask = [&](int ch, int tb, int cnt) {
-    kd.ask(Kd, ka, k_off, tb, cnt);
-    kw.ask(Kw, ka, k_off, tb, cnt);
-    const float* Tg = T + (static_cast<size_t>(ch) * a.H + head) * CL * CL;
+  const bool has_rows = wave < RT;               // the chunk's rows 16 wave .. + 15
+  const int rw = has_rows ? wave : 0, t0 = 16 * rw + 4 * lq;
+
+  // tile x of the wave's state: rows row_of(x) .. + 3, column l16
+  auto row_of = [&](int x) { return 16 * (wave + 4 * x) + 4 * lq; };
+  f32x4 S[MINE];
 #pragma unroll
-    for (int x = 0; x < NT; ++x) treg[x] = *reinterpret_cast<const f32x4*>(Tg + 4 * (tid + 256 * x));
-    vs.ask(rows + static_cast<size_t>(tb) * a.ld + v_off + col0, a.ld, cnt, dv - col0);
-    ereg = E[(static_cast<size_t>(ch) * a.H + head) * dk + min(tid, dk - 1)];
-  };
-  int tb = chunks[4 * c0 + 1], cnt = chunks[4 * c0 + 2];
-  ask(c0, tb, cnt);
-  for (int j = 0; j < nc; ++j) {
-    const int ch = c0 + j;
-    // the next chunk's place, asked for early
-    const int tb_next = j + 1 < nc ? chunks[4 * (ch + 1) + 1] : 0, cnt_next = j + 1 < nc ? chunks[4 * (ch + 1) + 2] : 0;
-    __syncthreads();   // the chunk before is done with everything
-    kd.put(Kds, cnt, dk);
-    kw.put(Kws, cnt, dk);
+  for (int x = 0; x < MINE; ++x) {
 #pragma unroll
-    for (int x = 0; x < NT; ++x)
-      *reinterpret_cast<f32x4*>(Tb + (4 * tid / CL + x * (1024 / CL)) * TLD + 4 * tid % CL) = treg[x];
-    vs.put(Vt, cnt, dv - col0);
-    if (tid < DKP) el[tid] = ereg;
-    __syncthreads();
-    if (j + 1 < nc) ask(ch + 1, tb_next, cnt_next);
-    // R = V - Kd S
-    if (wave < RT) {
-      const f32x4 acc = mma_rows<DKP>(Kds + (16 * wave + l16) * QLD + 4 * lq, St + l16 * QLD + 4 * lq, zero4());
-      const int t = 16 * wave + 4 * lq;
-      *reinterpret_cast<f32x4*>(Rt + l16 * TLD + t) = *reinterpret_cast<const f32x4*>(Vt + l16 * TLD + t) - acc;
+    for (int v = 0; v < 4; ++v) {
+      const int r = row_of(x) + v;
+      S[x][v] = (resume && r < dk && c < dv) ? S_slot[static_cast<size_t>(r) * dv + c] : 0.f;
     }
+    if (wave + 4 * x < KT) *reinterpret_cast<f32x4*>(St + l16 * QLD + row_of(x)) = S[x];
+  }
+
+  // A chunk's operands; what lies past the chunk or the head is read inside and cleared where it is used.  The chunk's
+  // part of an address is the same for all lanes, a lane's part fits 32 bits.
+  struct Operands {
+    f32x4 kd[KT], tr[RT], kw[MINE][RT], el[MINE];
+    float vv[4];
+    int tb, cnt;
+  };
+  // where the chunk that is asked for next lies, read a chunk ahead of that
+  int tb_next = chunks[4 * c0 + 1], cnt_next = chunks[4 * c0 + 2];
+  auto place = [&](int j) {
+    const int ch = c0 + min(j, nc - 1);          // behind the last chunk: the last one again, not used
+    tb_next = chunks[4 * ch + 1];
+    cnt_next = chunks[4 * ch + 2];
+  };
+  auto ask_kd = [&](Operands& o) {
+    o.tb = tb_next;
+    o.cnt = cnt_next;
+    const float* p = Kd + (static_cast<size_t>(o.tb) * a.H + head) * dk + static_cast<uint32_t>(min(16 * rw + l16, o.cnt - 1) * a.H * dk);
+#pragma unroll
+    for (int u = 0; u < KT; ++u) o.kd[u] = WHOLE ? *reinterpret_cast<const f32x4*>(p + 16 * u + 4 * lq) : load_four<VEC>(p, p, 16 * u + 4 * lq, dk, true);
+  };
+  auto ask_v = [&](Operands& o) {
+    const float* p = rows + static_cast<size_t>(o.tb) * a.ld + a.v_off + head * dv;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o.vv[v] = p[static_cast<uint32_t>(min(t0 + v, o.cnt - 1) * a.ld + min(c, dv - 1))];
+  };
+  auto ask_t = [&](Operands& o, int ch) {
+    const float* p = T + (static_cast<size_t>(ch) * a.H + head) * CL * CL;
+#pragma unroll
+    for (int k = 0; k < RT; ++k) o.tr[k] = *reinterpret_cast<const f32x4*>(p + 16 * min(k, rw) + static_cast<uint32_t>((16 * rw + l16) * CL + 4 * lq));
+  };
+  auto ask_kw = [&](Operands& o, int ch) {
+    const float* p = Kw + (static_cast<size_t>(ch) * a.H + head) * dk * CL;
+    const float* pe = E + (static_cast<size_t>(ch) * a.H + head) * dk;
+#pragma unroll
+    for (int x = 0; x < MINE; ++x) {
+      const uint32_t at = min(16 * (wave + 4 * x) + l16, dk - 1) * CL + 4 * lq;
+#pragma unroll
+      for (int k = 0; k < RT; ++k) o.kw[x][k] = *reinterpret_cast<const f32x4*>(p + 16 * k + at);
+      if (VEC) {
+        o.el[x] = *reinterpret_cast<const f32x4*>(pe + static_cast<uint32_t>(min(row_of(x), dk - 4)));
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o.el[x][v] = pe[min(row_of(x) + v, dk - 1)];
+      }
+    }
+  };
+  Operands even, odd;
+  auto ask = [&](Operands& o, int ch) {
+    ask_kd(o);
+    ask_v(o);
+    ask_t(o, ch);
+    ask_kw(o, ch);
+  };
+  ask(even, c0);
+  place(1);
+  ask(odd, c0 + min(1, nc - 1));
+  place(2);
+  __syncthreads();
+  auto chunk = [&](Operands& o, int j) {
+    const int ch = c0 + j, next = c0 + min(j + 2, nc - 1), tb = o.tb, cnt = o.cnt;
+    // R = V - Kd S
+    f32x4 v4;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) v4[v] = t0 + v < cnt && c_ok ? o.vv[v] : 0.f;
+    if (!WHOLE || cnt < CL) {
+#pragma unroll
+      for (int u = 0; u < KT; ++u) o.kd[u] = clear_past(o.kd[u], 16 * u + 4 * lq, dk, 16 * rw + l16 < cnt);
+    }
+    {
+      f32x4 s4[KT], acc = zero4();
+#pragma unroll
+      for (int u = 0; u < KT; ++u) s4[u] = *reinterpret_cast<const f32x4*>(St + l16 * QLD + 16 * u + 4 * lq);
+      __builtin_amdgcn_sched_barrier(0);         // all of them on their way: left alone each waits for the one before
+#pragma unroll
+      for (int u = 0; u < KT; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kd[u][e], s4[u][e], acc, 0, 0, 0);
+      if (has_rows) *reinterpret_cast<f32x4*>(Rt + l16 * TLD + t0) = v4 - acc;
+    }
+    ask_kd(o);
+    ask_v(o);
     __syncthreads();
     // U = T R, over the blocks of T up to the diagonal
-    if (wave < RT) {
-      const int t = 16 * wave + 4 * lq, c = col0 + l16;
-      f32x4 a4[RT], b4[RT], u = zero4();
+    f32x4 u4 = zero4();
+    {
+      f32x4 b4[RT];
+#pragma unroll
+      for (int k = 0; k < RT; ++k) b4[k] = *reinterpret_cast<const f32x4*>(Rt + l16 * TLD + 16 * k + 4 * lq);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int k = 0; k < RT; ++k) {
-        a4[k] = *reinterpret_cast<const f32x4*>(Tb + (16 * wave + l16) * TLD + 16 * k + 4 * lq);
-        b4[k] = *reinterpret_cast<const f32x4*>(Rt + l16 * TLD + 16 * k + 4 * lq);
+        if (k > rw) break;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u4 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.tr[k][e], b4[k][e], u4, 0, 0, 0);
       }
-#pragma unroll
-      for (int k = 0; k < RT; ++k) {
-        if (k > wave) break;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) u = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[k][e], b4[k][e], u, 0, 0, 0);
-      }
-      *reinterpret_cast<f32x4*>(Ut + l16 * TLD + t) = u;
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (t + v < cnt && c < dv) U[(static_cast<size_t>(tb + t + v) * a.H + head) * dv + c] = u[v];
+      if (has_rows) *reinterpret_cast<f32x4*>(Ut + l16 * TLD + t0) = u4;
     }
+    ask_t(o, next);
     __syncthreads();
     // S <- P(0, L) S + Kw^T U; the state as it was goes to W
-    float* Wg = W + (static_cast<size_t>(ch) * a.H + head) * dk * dv;
-    f32x4 b4[RT];
+    f32x4 b4[RT], old[MINE];
 #pragma unroll
     for (int k = 0; k < RT; ++k) b4[k] = *reinterpret_cast<const f32x4*>(Ut + l16 * TLD + 16 * k + 4 * lq);
-    for (int kt = wave; kt < DKP / 16; kt += 4) {
-      f32x4* mine = reinterpret_cast<f32x4*>(St + l16 * QLD + 16 * kt + 4 * lq);
-      const float* kp = Kws + (4 * lq) * QLD + 16 * kt + l16;
-      float kv[RT][4];
+    place(j + 3);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < RT; ++k)
+    for (int x = 0; x < MINE; ++x) {
+      if (!WHOLE && 16 * (wave + 4 * x) + l16 >= dk) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) kv[k][e] = kp[(16 * k + e) * QLD];
-      const f32x4 old = *mine;
-      f32x4 acc = old * *reinterpret_cast<const f32x4*>(el + 16 * kt + 4 * lq);
+        for (int k = 0; k < RT; ++k) o.kw[x][k] = zero4();
+      }
+      old[x] = S[x];
+      S[x] = S[x] * o.el[x];
+    }
 #pragma unroll
-      for (int k = 0; k < RT; ++k)
+    for (int k = 0; k < RT; ++k)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[k][e], b4[k][e], acc, 0, 0, 0);
-      const int c = col0 + l16;
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < MINE; ++x) S[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kw[x][k][e], b4[k][e], S[x], 0, 0, 0);
+    {
+      float* Wg = W + (static_cast<size_t>(ch) * a.H + head) * dk * dv;
+      float* Ug = U + (static_cast<size_t>(tb) * a.H + head) * dv;
+      if (has_rows) {
+        if (WHOLE && cnt == CL) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) Ug[static_cast<uint32_t>((t0 + v) * a.H * dv + c)] = u4[v];
+        } else {
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            if (t0 + v < cnt && c_ok) Ug[static_cast<uint32_t>((t0 + v) * a.H * dv + c)] = u4[v];
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < MINE; ++x) {
+        if (wave + 4 * x >= KT) break;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (WHOLE || (row_of(x) + v < dk && c_ok)) Wg[static_cast<uint32_t>((row_of(x) + v) * dv + c)] = old[x][v];
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < MINE; ++x)
+      if (wave + 4 * x < KT) *reinterpret_cast<f32x4*>(St + l16 * QLD + row_of(x)) = S[x];
+    ask_kw(o, next);
+    __syncthreads();
+  };
+  // (whole pairs: a way round the second chunk and back to the first would have the first wait for the newest loads)
+  int j = 0;
+#pragma unroll 1
+  for (; j + 1 < nc; j += 2) {
+    chunk(even, j);
+    chunk(odd, j + 1);
+  }
+  if (j < nc) chunk(even, j);
+  if (S_slot != nullptr && c < dv) {
+#pragma unroll
+    for (int x = 0; x < MINE; ++x)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int r = 16 * kt + 4 * lq + v;
-        if (r < dk && c < dv) Wg[static_cast<size_t>(r) * dv + c] = old[v];
+        const int r = row_of(x) + v;
+        if (r < dk) S_slot[static_cast<size_t>(r) * dv + c] = S[x][v];
       }
-      *mine = acc;
-    }
-    tb = tb_next;
-    cnt = cnt_next;
-  }
-  __syncthreads();
-  if (S_slot != nullptr) {
-    for (int i = tid; i < DKP * DCOLS; i += 256) {
-      const int r = i / DCOLS, cl = i % DCOLS, c = col0 + cl;
-      if (r < dk && c < dv) S_slot[static_cast<size_t>(r) * dv + c] = St[cl * QLD + r];
-    }
   }
 }
 
@@ -583,19 +666,21 @@ struct ChunkPtrs {
 
 template <int DKP, int CL, bool VEC> int chunks_go(const ChunkPtrs& p, ChArgs a, hipStream_t s) {
   static bool allowed = false;
-  constexpr size_t lds_solve = solve_lds<DKP, CL>(), lds_delta = delta_lds<DKP, CL>(), lds_read = read_lds<DKP, CL>();
+  constexpr size_t lds_solve = solve_lds<DKP, CL>(), lds_read = read_lds<DKP, CL>();
   if (!allowed) {
     hipError_t e = allow_lds(&chdelta_solve_kernel<DKP, CL>, lds_solve);
-    if (e == hipSuccess) e = allow_lds(&chdelta_delta_kernel<DKP, CL, VEC>, lds_delta);
     if (e == hipSuccess) e = allow_lds(&chdelta_read_kernel<DKP, CL, VEC>, lds_read);
     if (e != hipSuccess) return static_cast<int>(e);
     allowed = true;
   }
   hipLaunchKernelGGL((chdelta_solve_kernel<DKP, CL>), dim3(a.H, p.n_chunks), dim3(solve_threads<DKP, CL>()), lds_solve, s,
                      p.rows, p.z, p.zb, p.neg_a, p.dt_bias, p.chunks, p.T, p.A, p.E, p.Kd, p.Kw, p.Qd, a);
-  hipLaunchKernelGGL((chdelta_delta_kernel<DKP, CL, VEC>), dim3(a.H, (a.dv + DCOLS - 1) / DCOLS, p.n_runs), dim3(256),
-                     lds_delta, s, p.rows, p.chunks, p.runs, p.positions, p.slot_ids, p.state, p.T, p.E, p.Kd, p.Kw, p.W,
-                     p.U, a);
+  auto delta = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(a.H, (a.dv + DCOLS - 1) / DCOLS, p.n_runs), dim3(256), 0, s, p.rows, p.chunks, p.runs,
+                       p.positions, p.slot_ids, p.state, p.T, p.E, p.Kd, p.Kw, p.W, p.U, a);
+  };
+  if (VEC && a.dk == DKP && a.dv % DCOLS == 0) delta(&chdelta_delta_kernel<DKP, CL, true, true>);
+  else delta(&chdelta_delta_kernel<DKP, CL, VEC, false>);
   hipLaunchKernelGGL((chdelta_read_kernel<DKP, CL, VEC>), dim3(a.H, (a.dv + VCOLS - 1) / VCOLS, p.n_chunks), dim3(512),
                      lds_read, s, p.chunks, p.Qd, p.A, p.W, p.U, p.out, a);
   return kvf_last_error();
@@ -636,7 +721,7 @@ KVF_EXPORT int kvf_chdelta_chunk_len(int dk) { return dk <= 128 ? 64 : 32; }
 
 // The runs named in `runs` (sequence, first chunk, chunks), cut into `chunks` (sequence, first token, tokens, 0; at
 // most kvf_chdelta_chunk_len(dk) tokens each, a run's chunks in order and one after another).  Scratch: T, A
-// [n_chunks, H, CL, CL], E [n_chunks, H, dk], Kd, Kw, Qd [tokens, H, dk], W [n_chunks, H, dk, dv], U [tokens, H, dv],
+// [n_chunks, H, CL, CL], E [n_chunks, H, dk], Kd, Qd [tokens, H, dk], Kw [n_chunks, H, dk, CL], W [n_chunks, H, dk, dv], U [tokens, H, dv],
 // all on 16 bytes.
 KVF_EXPORT int kvf_chdelta_chunks(CHDELTA_ARGS_DECL, const int* chunks, int n_chunks, const int* runs, int n_runs,
                                   float* T, float* A, float* E, float* Kd, float* Kw, float* Qd, float* W, float* U,

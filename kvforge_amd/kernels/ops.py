@@ -2236,8 +2236,8 @@ def chdelta_scratch(n_tokens: int, n_chunks: int, heads: int, key_dim: int, valu
     """(shape, dtype) of the scratch tensors the passes over the chunks (of ``ssm_plan``) need, by name."""
     H, dk, dv, cl = int(heads), int(key_dim), int(value_dim), ssm_chunk_len(key_dim)
     out = {name: ((n_chunks, H, cl, cl), F32) for name in ("T", "A")}
-    out.update({name: ((n_tokens, H, dk), F32) for name in ("Kd", "Kw", "Qd")})
-    out.update({"E": ((n_chunks, H, dk), F32), "W": ((n_chunks, H, dk, dv), F32), "U": ((n_tokens, H, dv), F32)})
+    out.update({name: ((n_tokens, H, dk), F32) for name in ("Kd", "Qd")})
+    out.update({"Kw": ((n_chunks, H, dk, cl), F32), "E": ((n_chunks, H, dk), F32), "W": ((n_chunks, H, dk, dv), F32), "U": ((n_tokens, H, dv), F32)})
     return out
 
 

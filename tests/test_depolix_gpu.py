@@ -275,6 +275,35 @@ def test_the_memory_over_runs_steps_and_slots(H, G, dk, dv):
     assert float((wide[:, :4] - 5.0).abs().max()) == 0.0 and float((wide[:, -3:] - 5.0).abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("H,G,dk,dv", [(3, 1, 32, 48), (2, 1, 64, 16), (2, 1, 64, 17), (8, 2, 128, 32)])
+def test_the_memory_over_heads_that_fill_the_kernels_tiles(H, G, dk, dv):
+    """Heads of exactly as many channels as the chunks' kernel holds, value columns in whole sixteens or not: its form
+    without anything to leave out, and the other."""
+    test_the_memory_over_runs_steps_and_slots(H, G, dk, dv)
+
+
+@pytest.mark.parametrize("n", [256, 257, 321, 500])
+def test_the_memory_over_many_chunks(n):
+    """Four to eight chunks of 64 in one run, whose operands are asked for two chunks ahead: bit by bit what the same
+    tokens give as runs of whole chunks, each from the slot that the one before left."""
+    H, G, dk, dv = 2, 1, 64, 32
+    g = torch.Generator().manual_seed(n)
+    q, k = plain.unit(torch.randn(n, G, dk, generator=g)).view(n, -1), plain.unit(torch.randn(n, G, dk, generator=g)).view(n, -1)
+    v, za, zb = torch.randn(n, H * dv, generator=g), torch.randn(n, H * dk, generator=g) - 2.0, torch.randn(n, H, generator=g)
+    neg_a, dt_bias = -torch.exp(torch.randn(H, generator=g)), torch.randn(H * dk, generator=g)
+
+    def go(lo, hi, state):
+        return run_memory(q[lo:hi], k[lo:hi], v[lo:hi], za[lo:hi], zb[lo:hi], neg_a, dt_bias, [hi - lo], state, [1],
+                          list(range(lo, hi)), H, G, dk, dv)
+
+    one, parts = torch.zeros(2, H * dk * dv, device=DEV), torch.zeros(2, H * dk * dv, device=DEV)
+    whole = go(0, n, one)
+    cuts = list(range(0, n - 64, 64)) + [n]      # (a short rest would go token by token: it stays with the last cut)
+    got = torch.cat([go(a, b, parts) for a, b in zip(cuts, cuts[1:])])
+    assert torch.equal(got, whole) and torch.equal(one, parts)
+
+
+
 def test_channels_that_are_kept_and_channels_that_are_dropped():
     """With beta near one, keys along single channels and no decay but on some channels, a query for a
     kept channel's key gets the last value written under it, across chunks, and one for a dropped
