@@ -12,6 +12,7 @@
 namespace {
 constexpr int TB = 8;          // tokens staged in LDS at a time
 constexpr int COLS = KVF_WAVE; // columns of S (elements of v) per workgroup: one per lane
+constexpr int TOKEN_MAX_KEY = 128;   // key sizes of the kernel for single tokens
 
 struct ScanArgs {
   int H, dk, dv, row_len;   // row_len: elements from one token's projected row to the next
@@ -150,6 +151,103 @@ __global__ __launch_bounds__(ROWS > KVF_WAVE ? 2 * KVF_WAVE : KVF_WAVE) void mls
     }
     if (threadIdx.x == 0) st[static_cast<size_t>(dk) * dv + dk] = m;
   }
+}
+
+// A step whose runs are single tokens (keys of up to 128): the same sums in the same order as above.  What bounds it is the
+// way of the state from and to memory, so it has to be on its way at once: workgroup (column block, head, sequence) of
+// four waves, a wave a quarter of the rows (R), every load of a lane asked for before the first is used and none under a
+// condition.  The new rows go to memory and through LDS to the first wave, which adds up o over all rows while the second
+// does n . q.  Eight sequences, 8 heads of 128 x 256: 11.3 us, 26.4 in the kernel above, a wave for 64 columns of a head.
+template <typename T, int R>
+__global__ __launch_bounds__(4 * KVF_WAVE) void mlstm_token_kernel(const T* __restrict__ qkv, const float* __restrict__ zif,
+                                                                   const float* __restrict__ bias_if,
+                                                                   const int* __restrict__ cu_q,
+                                                                   const int* __restrict__ positions,
+                                                                   const int* __restrict__ slot_ids,
+                                                                   float* __restrict__ state, float* __restrict__ out,
+                                                                   ScanArgs a) {
+  constexpr int ROWS = 4 * R, NJ = ROWS > KVF_WAVE ? ROWS / KVF_WAVE : 1;
+  __shared__ __align__(16) float ks[ROWS], qs[ROWS];
+  __shared__ float Ss[ROWS][COLS];
+  __shared__ float nq_all;
+  const int seq = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * COLS;
+  const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / KVF_WAVE);
+  const int dk = a.dk, dv = a.dv, slot = slot_ids[seq], t = cu_q[seq], c = col0 + lane;
+  if (cu_q[seq + 1] <= t) return;
+  const bool col_ok = c < dv;
+  float* o_at = out + static_cast<size_t>(t) * a.H * dv + head * dv + c;
+  if (slot < 0 || slot >= a.n_slots) {   // as in the kernel above
+    if (wave == 0 && col_ok) *o_at = 0.f;
+    return;
+  }
+  const bool fresh = positions[t] == 0;
+  const int r0 = wave * R;
+  float* st = state + (static_cast<size_t>(slot) * a.H + head) * (static_cast<size_t>(dk) * dv + dk + 1);
+  const T* row = qkv + static_cast<size_t>(t) * a.row_len;
+  const float* z = zif + static_cast<size_t>(t) * a.gate_stride;
+  float S[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) S[r] = st[static_cast<size_t>(min(r0 + r, dk - 1)) * dv + min(c, dv - 1)];
+  float nv[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) nv[j] = st[static_cast<size_t>(dk) * dv + min(lane + KVF_WAVE * j, dk - 1)];
+  const float m_old = st[static_cast<size_t>(dk) * dv + dk];
+  const float v = Elem<T>::load(row + a.v_off + head * dv + min(c, dv - 1));
+  const float zi = z[head] + bias_if[head], zf = z[a.H + head] + bias_if[a.H + head];
+  for (int i = tid; i < 2 * ROWS; i += 4 * KVF_WAVE) {     // k, then q: a half of the threads each
+    const int e = i % ROWS;
+    const float x = Elem<T>::load(row + (i < ROWS ? a.k_off : a.q_off) + head * dk + min(e, dk - 1));
+    if (i < ROWS) ks[e] = e < dk ? x : 0.f;
+    else qs[e] = e < dk ? x * a.q_scale : 0.f;
+  }
+  // (as numbers of their own: the last product of one must not become part of the sum that it goes into below)
+  auto apart = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
+  const float li = apart(capped(zi, a.cap)), lf = apart(log_sigmoid(capped(zf, a.cap)));
+  const float m = fresh ? 0.f : m_old;
+  const float al = lf + m;
+  const float m_new = fmaxf(al, li);
+  const float keep = expf(al - m_new), take = expf(li - m_new);
+  const float tv = take * (col_ok ? v : 0.f);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    S[r] = fmaf(keep, fresh ? 0.f : S[r], ks[r0 + r] * tv);
+    Ss[r0 + r][lane] = S[r];
+  }
+  __syncthreads();
+  float o = 0.f;
+  if (wave == 0) {
+    constexpr int AHEAD = ROWS < 32 ? ROWS : 32;
+#pragma unroll
+    for (int r1 = 0; r1 < ROWS; r1 += AHEAD) {
+      float s[AHEAD];
+#pragma unroll
+      for (int r = 0; r < AHEAD; ++r) s[r] = Ss[r1 + r][lane];
+#pragma unroll
+      for (int r = 0; r < AHEAD; ++r)
+        if (r1 + r < dk) o = fmaf(s[r], qs[r1 + r], o);
+    }
+  }
+  if (wave == 1) {
+    float nq = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int r = lane + KVF_WAVE * j;
+      if (r < dk) {
+        nv[j] = fmaf(keep, fresh ? 0.f : nv[j], take * ks[r]);
+        nq = fmaf(nv[j], qs[r], nq);
+        if (blockIdx.x == 0) st[static_cast<size_t>(dk) * dv + r] = nv[j];
+      }
+    }
+    nq = wave_sum(nq);
+    if (lane == 0) nq_all = nq;
+    if (lane == 0 && blockIdx.x == 0) st[static_cast<size_t>(dk) * dv + dk] = m_new;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (col_ok && r0 + r < dk) st[static_cast<size_t>(r0 + r) * dv + c] = S[r];
+  __syncthreads();
+  if (wave == 0 && col_ok) *o_at = o / (fmaxf(fabsf(nq_all), expf(-m_new)) + 1e-6f);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -831,8 +929,18 @@ int multi_launch(const void* qkv, const float* zif, const float* bias_if, const 
 
 template <typename T>
 int scan_launch(const void* qkv, const float* zif, const float* bias_if, const int* cu_q, const int* positions,
-                const int* slot_ids, float* state, float* out, int num_seqs, ScanArgs a, hipStream_t s) {
+                const int* slot_ids, float* state, float* out, int num_seqs, bool single, ScanArgs a, hipStream_t s) {
   if (num_seqs <= 0) return 0;
+  if (single && a.dk <= TOKEN_MAX_KEY) {
+#define GO(R)                                                                                           \
+  hipLaunchKernelGGL((mlstm_token_kernel<T, R>), dim3((a.dv + COLS - 1) / COLS, a.H, num_seqs), dim3(4 * KVF_WAVE), 0, s, \
+                     static_cast<const T*>(qkv), zif, bias_if, cu_q, positions, slot_ids, state, out, a)
+    if (a.dk <= 32) GO(8);
+    else if (a.dk <= 64) GO(16);
+    else GO(32);
+#undef GO
+    return kvf_last_error();
+  }
   const int rows = a.dk <= 32 ? 32 : (a.dk <= 64 ? 64 : 128);
   const int rg = (a.dk + rows - 1) / rows;
   const dim3 grid((a.dv + COLS - 1) / COLS, a.H, num_seqs), block(rg * KVF_WAVE);
@@ -881,7 +989,7 @@ int out_launch(const float* o, const void* g, int g_stride, const float* w, floa
 // out [tokens, H dv] fp32.  Sequence s owns tokens cu_q[s] .. cu_q[s+1]-1 and slot slot_ids[s]
 // (negative: skipped); it starts from zeros when its first token's position is 0.
 // Runs of fewer than chunk_from tokens are walked token by token (`short_runs`: launch that
-// kernel), runs of chunk_from to multi_from - 1 tokens chunk by chunk in one kernel (`long_runs`),
+// kernel; 2: every run of the step is one token or none), runs of chunk_from to multi_from - 1 tokens chunk by chunk in one kernel (`long_runs`),
 // runs of at least multi_from tokens by the four passes over all chunks at once (n_chunks > 0:
 // `chunks` [n_chunks, 4] and `runs` [n_runs, 3] name them, the other pointers are their scratch);
 // each kernel leaves the others' sequences alone.
@@ -900,8 +1008,8 @@ KVF_EXPORT int kvf_mlstm_scan(int dtype, const void* qkv, const float* zif, cons
                    multi_from};
   int code = 0;
   if (short_runs)
-    code = dtype == 0 ? scan_launch<float>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, a, s)
-                      : scan_launch<bf16_t>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, a, s);
+    code = dtype == 0 ? scan_launch<float>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, short_runs == 2, a, s)
+                      : scan_launch<bf16_t>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, short_runs == 2, a, s);
   if (code == 0 && long_runs)
     code = dtype == 0 ? chunk_launch<float>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, a, s)
                       : chunk_launch<bf16_t>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, a, s);

@@ -1489,7 +1489,7 @@ def mlstm_scan(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor,
                num_seqs: int, heads: int, key_dim: int, value_dim: int, q_off: int, k_off: int,
                v_off: int, cap: float, q_scale: float, chunk_from: int = MLSTM_CHUNK_FROM,
                short_runs: bool = True, long_runs: bool = True, multi_from: int | None = None,
-               multi: dict | None = None) -> None:
+               multi: dict | None = None, single: bool = False) -> None:
     """The matrix-memory recurrence over every sequence's tokens of this step, from and into the
     sequences' state slots.  ``rows [N, >= ...]``: projected rows holding q (``heads * key_dim``
     elements from column ``q_off``), k (from ``k_off``) and v (``heads * value_dim`` from
@@ -1506,7 +1506,8 @@ def mlstm_scan(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor,
     are then taken all at once by four passes (gates, every chunk's own contribution, the
     carry over a run's chunks, the outputs): ``chunks`` ``[n, 4]`` and ``runs`` ``[r, 3]`` (int32,
     from ``mlstm_multi_plan``) and the scratch tensors of ``mlstm_multi_scratch``; without it no
-    run is that long for the kernels (``multi_from`` is then ignored)."""
+    run is that long for the kernels (``multi_from`` is then ignored).  ``single``: no run of the step holds more than one
+    token (a decode step), which keys of up to 128 have a kernel for; the same bits."""
     n = rows.shape[0]
     H, dk, dv = int(heads), int(key_dim), int(value_dim)
     _check(rows, "rows", None, (n, None), contiguous=False)
@@ -1548,7 +1549,7 @@ def mlstm_scan(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor,
     _ok(f(_tcode(rows.dtype), rows.data_ptr(), gates.data_ptr(), gate_bias.data_ptr(), cu_q.data_ptr(),
           positions.data_ptr(), slot_ids.data_ptr(), state.data_ptr(), out.data_ptr(), int(num_seqs),
           H, dk, dv, rows.stride(0) if n > 1 else rows.shape[1], int(q_off), int(k_off), int(v_off),
-          state.shape[0], gates.shape[1], float(cap), float(q_scale), int(chunk_from), 1 if short_runs else 0,
+          state.shape[0], gates.shape[1], float(cap), float(q_scale), int(chunk_from), (2 if single and chunk_from > 1 else 1) if short_runs else 0,
           1 if long_runs else 0, multi_from if multi is not None else big, n_chunks, n_runs, *extra,
           _stream()), "mlstm_scan")
 

@@ -124,14 +124,14 @@ class MatrixLSTM(Mixer):
         gates = ws.buf("mlstm_gates", (n, self.G_pad), torch.float32)
         ops.gemm(x, self.w_gates, gates)
         raw = ws.buf("mlstm_raw", (n, H * dv), torch.float32)
-        # which of the two kernels have work is known from the runs' lengths (all ones in a
+        # which of the kernels have work is known from the runs' lengths (all ones in a
         # captured step of single tokens, so a replay launches what the capture launched)
         long_runs = any(ops.MLSTM_CHUNK_FROM <= q < ops.MLSTM_MULTI_FROM for q in step.q_lens)
         short_runs = any(q < ops.MLSTM_CHUNK_FROM for q in step.q_lens)
         ops.mlstm_scan(rows, gates, self.gate_bias, step.cu_q, step.positions, step.slot_ids,
                        layer.state, raw, step.n_seqs, H, dk, dv, 0, H * dk, 2 * H * dk,
                        self.gate_cap, float(dk) ** -0.5, short_runs=short_runs, long_runs=long_runs,
-                       multi=self._longest_runs(step, n))
+                       multi=self._longest_runs(step, n), single=max(step.q_lens, default=0) <= 1)
         heads = ws.buf("mlstm_heads", (n, H * dv), act)
         g0 = 2 * H * dk + H * dv
         ops.mlstm_out(raw, rows[:, g0:g0 + H * dv], self.head_weight, self.norm_eps, heads, H, dv)

@@ -177,6 +177,34 @@ def scan_reference(q, k, v, zi, zf, bias, cap, H, dk, dv):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,dk,dv", [(2, 8, 16), (3, 32, 64), (1, 33, 65), (2, 64, 24), (2, 100, 130), (8, 128, 256), (1, 129, 8)])
+def test_matrix_memory_of_single_tokens(dtype, H, dk, dv):
+    """A step of single tokens has a kernel of its own for keys of up to 128: outputs and slots are the bits of the kernel
+    that walks runs token by token, over several steps.  A sequence at position 0 in a slot full of NaN, one without a slot,
+    one without a token, slots that no sequence has; keys and columns that end inside a wave's rows and block."""
+    n, cap = 6, 6.0
+    cu, slots = i32([0, 1, 2, 2, 3, 4, 5]), i32([4, -1, 5, 0, 7, 2])
+    bias = rand(2 * H, seed=9, scale=2.0).to(DEV)
+    states = []
+    for single in (False, True):
+        state = rand(8, ops().mlstm_state_floats(H, dk, dv), seed=3).to(DEV)
+        state[2] = float("nan")
+        outs = []
+        for step in range(3):
+            rows = rand(5, 2 * H * dk + H * dv + 3, seed=20 + step).to(dtype).to(DEV)
+            z = rand(5, 2 * H + 1, seed=40 + step, scale=5.0).to(DEV)
+            pos = i32([7 + step, 3, 1 + step, 900 + step, step])
+            out = torch.full((5, H * dv), 7.0, device=DEV)
+            ops().mlstm_scan(rows, z, bias, cu, pos, slots, state, out, n, H, dk, dv, 0, H * dk, 2 * H * dk, cap, dk ** -0.5,
+                             long_runs=False, single=single)
+            outs.append(out)
+        states.append((state, *outs))
+    for a, b in zip(*states):
+        assert torch.equal(a.nan_to_num(1e9), b.nan_to_num(1e9)), float((a - b).nan_to_num(0.0).abs().max())
+    assert bool(torch.stack(states[1][1:]).isfinite().all()) and bool((states[1][1][1] == 0.0).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,dk,dv", [(2, 8, 16), (6, 32, 64), (1, 40, 100), (3, 64, 24), (2, 100, 130),
                                      (2, 128, 64), (1, 200, 70), (1, 256, 8)])
 @pytest.mark.parametrize("chunk_from", [1, 8, 1000])
