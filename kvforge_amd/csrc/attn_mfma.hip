@@ -59,6 +59,8 @@
 //   split order.
 // block_size must be a multiple of 8 (a lane's eight keys lie in one page), d a multiple of 16;
 // kernels are instantiated for each d / 16 so that no loop bound is left to run time.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -181,6 +183,16 @@ __device__ __forceinline__ uint4 keep_first(const uint4& r, int live) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) w[e] &= first_mask(e, live);
   return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// The same in the registers that hold it.
+__device__ __forceinline__ void clear_behind(uint4& r, int live) {
+  if (__any(live < 8)) {
+    r.x &= first_mask(0, live);
+    r.y &= first_mask(1, live);
+    r.z &= first_mask(2, live);
+    r.w &= first_mask(3, live);
+  }
 }
 
 // max / sum over the four lanes of a row (lanes j, j+16, j+32, j+48)
@@ -414,7 +426,13 @@ constexpr bool runs_pair(int dt) { return dt > 8; }
 // NW: waves of the workgroup.  Eight stage half as much each as four do, and a key block is brought in for
 // twice the rows.  Heads wider than 128 have two items a work row, four waves each, side by side over the
 // keys that either sees; narrower ones one item of all the waves at a time.
-template <int DT, int RT, int NW, int BIAS, bool SINK>
+// EVEN: pages of 16 keys.  A key block then has two pages, the same for all lanes: one lookup a wave instead of one a
+// fragment, the pages' places worked out in scalar registers, and a lane's part of an address the same for every block.
+// A block was 104 vector instructions beside its 8 products, half of them for addresses, and is 90: 32 heads over 8 kv heads of
+// 64, 2,048 queries 49.1 -> 46.5 us, through a window of 1,024 42.5 -> 33.7 (blocks that every row sees whole need no mask
+// there either), three ragged runs behind up to 3,072 keys 88.5 -> 80.8; of 128, 2,048 queries 76.1 -> 70.4; 32 heads of 224
+// over one 110.3 -> 106.5.
+template <int DT, int RT, int NW, int BIAS, bool SINK, bool EVEN>
 __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) void attn_mfma_runs_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
     const bf16_t* __restrict__ vt_pages, const int* __restrict__ block_table,
@@ -493,6 +511,13 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
   if (hi_g < 0) lo_g = 0;
   const float scale2 = a.scale * LOG2E;
   const int keep_w = a.window > 0 ? a.keep : 0;
+  // With a window or chunks, the first key that the wave's last row sees through it: blocks from there on need no mask for it.
+  // (None where the wave has rows past the run's last, whose scores a mask has to keep at nothing.)
+  int seen_by_all = 0;
+  if (a.window != 0) {
+    const bool filled = ((max(item, 0) * IW + wave % IW) * RT + RT) * 16 <= qlen * G;
+    seen_by_all = !filled ? 0x7fffffff : CHUNK ? chunk_first(a, max(pos_max, 0)) : pos_max - a.window + 1;
+  }
 
   float m_ref[RT], l_run[RT];
   f32x4 acc[RT][DT];
@@ -521,11 +546,12 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
     int live[FPW];
   };
   struct Lookup {
-    PageRef page[FPW];
+    PageRef page[EVEN ? 1 : FPW];
   };
   int key_off[FPW];
   unsigned lane_off[FPW];
-  bool is_k[FPW], whole[FPW];
+  bool is_k[FPW], whole[FPW], second[FPW];   // second: EVEN, the lane's key lies in the block's second page
+  const int ctx_even = min(ctx, a.table_stride * 16);
   const unsigned page_stride = static_cast<unsigned>(a.KV) * a.bs * (D / 8);
 #pragma unroll
   for (int i = 0; i < FPW; ++i) {
@@ -541,6 +567,8 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
       whole[i] = wave + i * NW < N_FRAG;                 // (out of page 0, which the caches hold)
       lane_off[i] = (static_cast<unsigned>(kvh) * D + (f - N_K) * 16 + j16) * (a.bs / 8);
     }
+    second[i] = key_off[i] >= 16;
+    if (EVEN) lane_off[i] += is_k[i] ? (key_off[i] % 16) * (D / 8) : key_off[i] % 16 / 8;
   }
   // Every load below reads a valid address whatever the block (a key past the context reads
   // the table's last entry and page 0, and counts for nothing), so none of them sits in a
@@ -548,13 +576,32 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
   const Walk wk = walk_of(a, lo_g, hi_g);
   auto locate = [&](int kb, Lookup& l) {
     kb = wk.at(kb);
+    if constexpr (EVEN) {   // even lanes the block's first page, odd ones its second
+      l.page[0].page = pg.table[min((kb >> 4) + (lane & 1), a.table_stride - 1)];
+      return;
+    }
 #pragma unroll
-    for (int i = 0; i < FPW; ++i) l.page[i] = page_of_key(pg, a, kb + key_off[i]);
+    for (int i = 0; i < (EVEN ? 1 : FPW); ++i) l.page[i] = page_of_key(pg, a, kb + key_off[i]);
   };
   auto fetch = [&](int kb, const Lookup& l, Stage& st) {
     kb = wk.at(kb);
+    if constexpr (EVEN) {
+      const unsigned p0 = __builtin_amdgcn_readlane(l.page[0].page, 0), p1 = __builtin_amdgcn_readlane(l.page[0].page, 1);
+      const unsigned nb = a.nb;
+      const bool ok0 = p0 < nb, ok1 = p1 < nb;
+      const unsigned at0 = __builtin_amdgcn_readfirstlane((ok0 ? p0 : 0) * page_stride);
+      const unsigned at1 = __builtin_amdgcn_readfirstlane((ok1 ? p1 : 0) * page_stride);
+      const int left = ctx_even - kb;
 #pragma unroll
-    for (int i = 0; i < FPW; ++i) {
+      for (int i = 0; i < FPW; ++i) {
+        const bool ok = (second[i] ? ok1 : ok0) && key_off[i] < left && whole[i];
+        st.live[i] = !ok ? 0 : is_k[i] ? 8 : min(left - key_off[i], 8);
+        st.frag[i] = ld16((is_k[i] ? k_pages : vt_pages) + static_cast<size_t>((second[i] ? at1 : at0) + lane_off[i]) * 8);
+      }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < (EVEN ? 1 : FPW); ++i) {
       const int key = kb + key_off[i];
       const unsigned slot = static_cast<unsigned>(key - block_of(a, key) * a.bs);
       const bool ok = l.page[i].ok(a.nb) && whole[i];
@@ -564,11 +611,13 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
       st.frag[i] = ld16((is_k[i] ? k_pages : vt_pages) + static_cast<size_t>(off) * 8);
     }
   };
-  auto put = [&](int buf, const Stage& st) {
+  auto put = [&](int buf, Stage& st) {
 #pragma unroll
     for (int i = 0; i < FPW; ++i) {
       const int f = wave + i * NW;
-      if (f < N_FRAG) frag_lds[(buf * N_FRAG + f) * KVF_WAVE + lane] = keep_first(st.frag[i], st.live[i]);
+      if (f >= N_FRAG) continue;
+      clear_behind(st.frag[i], st.live[i]);
+      frag_lds[(buf * N_FRAG + f) * KVF_WAVE + lane] = st.frag[i];
     }
   };
   auto work_on = [&](int kb, int buf) {
@@ -581,7 +630,7 @@ __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) vo
         for (int c = 0; c < DC; ++c)
           kf[t][c] = as_frag(frag_lds[(buf * N_FRAG + t * DC + c) * KVF_WAVE + lane]);
       const uint4* values = frag_lds + (buf * N_FRAG + N_K) * KVF_WAVE + lane;
-      const bool edge = kb + 31 > pos_min || kb + 32 > ctx || a.window > 0 || CHUNK;
+      const bool edge = kb + 31 > pos_min || kb + 32 > ctx || kb < seen_by_all;
       if constexpr (DT <= 14) {
         bf16x8 vf[DT];
 #pragma unroll
@@ -1032,19 +1081,19 @@ template <int DT, class Go> void runs_shape(int row_tiles, const Go& go) {
   else go(Count<2>{}, Count<4>{});
 }
 
-template <int DT, int RT, int NW>
+template <int DT, int RT, int NW, bool EVEN>
 void launch_runs_rt(dim3 grid, hipStream_t s, const void* q, const void* k_pages, const void* vt_pages,
                     const int* block_table, const int* work, const int* cu_q, const int* ctx_lens, void* out,
                     const MArgs& a) {
   constexpr int N_FRAG = 2 * ((DT + 1) / 2) + DT;
   const size_t lds = static_cast<size_t>(2) * N_FRAG * KVF_WAVE * sizeof(uint4);
   if (a.window < 0)   // (never with a cap, sinks or slopes: the exported entry refuses the pairs)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 3, false>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 3, false, EVEN>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
   else if (a.cap > 0.f)   // (never with sinks or slopes: the exported entry refuses the pairs)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 2, false>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 2, false, EVEN>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
@@ -1053,27 +1102,27 @@ void launch_runs_rt(dim3 grid, hipStream_t s, const void* q, const void* k_pages
     const size_t table = static_cast<size_t>(a.H / a.KV) * dist_row(a.n_dist) * sizeof(float);
     b.dist_lds = lds + table <= (runs_pair(DT) ? DIST_LDS_MOST_PAIR : DIST_LDS_MOST);
     if (b.dist_lds && lds + table > LDS_UNASKED &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_runs_kernel<DT, RT, NW, 4, false>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_runs_kernel<DT, RT, NW, 4, false, EVEN>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds + table)) != hipSuccess) {
       kvf_last_error();   // the table is read from memory then
       b.dist_lds = 0;
     }
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 4, false>), grid, dim3(NW * KVF_WAVE), b.dist_lds ? lds + table : lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 4, false, EVEN>), grid, dim3(NW * KVF_WAVE), b.dist_lds ? lds + table : lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), b);
   } else if (a.sinks)   // (never with slopes: the exported entry refuses the pair)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 0, true>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 0, true, EVEN>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
   else if (a.slopes)
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 1, false>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 1, false, EVEN>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
   else
-    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 0, false>), grid, dim3(NW * KVF_WAVE), lds, s,
+    hipLaunchKernelGGL((attn_mfma_runs_kernel<DT, RT, NW, 0, false, EVEN>), grid, dim3(NW * KVF_WAVE), lds, s,
                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages),
                        static_cast<const bf16_t*>(vt_pages), block_table, work, cu_q, ctx_lens,
                        static_cast<bf16_t*>(out), a);
@@ -1084,8 +1133,12 @@ void launch_runs(int row_tiles, dim3 grid, hipStream_t s, const void* q, const v
                  const void* vt_pages, const int* block_table, const int* work, const int* cu_q,
                  const int* ctx_lens, void* out, const MArgs& a) {
   auto go = [&](auto rt, auto nw) {
-    launch_runs_rt<DT, decltype(rt)::value, decltype(nw)::value>(grid, s, q, k_pages, vt_pages, block_table, work, cu_q,
-                                                                 ctx_lens, out, a);
+    auto with = [&](auto even) {
+      launch_runs_rt<DT, decltype(rt)::value, decltype(nw)::value, decltype(even)::value>(grid, s, q, k_pages, vt_pages, block_table,
+                                                                                          work, cu_q, ctx_lens, out, a);
+    };
+    if (a.bs == 16) with(std::true_type{});
+    else with(std::false_type{});
   };
   runs_shape<DT>(row_tiles, go);
 }
@@ -1193,7 +1246,7 @@ KVF_EXPORT int kvf_attn_mfma_prefill_blocks_per_cu(int d, int row_tiles) {
       constexpr int NW = decltype(nw)::value;                                                        \
       const size_t lds = static_cast<size_t>(2) * (2 * ((DT + 1) / 2) + DT) * KVF_WAVE * sizeof(uint4); \
       if (hipOccupancyMaxActiveBlocksPerMultiprocessor(                                              \
-              &n, attn_mfma_runs_kernel<DT, decltype(rt)::value, NW, 0, false>, NW * KVF_WAVE, lds) != hipSuccess) \
+              &n, attn_mfma_runs_kernel<DT, decltype(rt)::value, NW, 0, false, true>, NW * KVF_WAVE, lds) != hipSuccess) \
         n = 0;                                                                                       \
     });                                                                                              \
     break;

@@ -7,6 +7,7 @@ import math
 import random
 
 import pytest
+import numpy as np
 import torch
 
 from tests.plain import llama as plain
@@ -1416,3 +1417,60 @@ def test_grouped_experts_over_rows_of_many_passes(K, ff, weigh_input):
     """Tiles of every height over rows of five to seven passes of 64 elements, where the loads of the last ones stand
     ahead of the row's end, whole and part passes, odd steps; one expert of several tiles."""
     test_grouped_experts_at_the_edges_of_their_tiles([20, 40, 290, 70, 128], K, ff, weigh_input)
+
+
+@pytest.mark.parametrize("d", [16, 48, 64, 128, 208])
+@pytest.mark.parametrize("form", ["plain", "window", "kept", "chunk", "slopes", "cap", "sinks", "dist"])
+def test_query_runs_over_pages_of_sixteen_keys(d, form):
+    """Pages of 16 keys have a form of the query-run kernel that looks a block's two pages up once for the wave; pages of 8
+    keys go fragment by fragment.  The same keys in either give the same bits: runs from position 0 and behind a context,
+    ends inside a page, a block and a tile of rows, pages that a window has given back, and entries that name no page."""
+    H, KV = 6, 2
+    q_lens, starts = [70, 33, 150, 5], [0, 201, 64, 1000]
+    g = torch.Generator().manual_seed(d)
+    ctxs = [a + b for a, b in zip(q_lens, starts)]
+    keys = [torch.randn(c, KV, d, generator=g).to(torch.bfloat16) for c in ctxs]
+    vals = [torch.randn(c, KV, d, generator=g).to(torch.bfloat16) for c in ctxs]
+    q = (2.0 * torch.randn(sum(q_lens), H * d, generator=g)).to(torch.bfloat16).to(DEV)
+    kw = {"window": dict(window=40), "kept": dict(window=48, keep_first=21), "chunk": dict(chunk=50), "cap": dict(score_cap=5.0),
+          "slopes": dict(slopes=torch.rand(H, generator=g).to(DEV) * 0.1), "sinks": dict(sinks=torch.randn(H, generator=g).to(DEV)),
+          "dist": dict(dist=torch.randn(H, 37, generator=g).to(DEV))}.get(form, {})
+    window, keep = kw.pop("window", None), kw.get("keep_first", 0)
+    outs = []
+    for bs in (8, 16):
+        nb = sum(-(-c // bs) for c in ctxs) + 5
+        ids = torch.randperm(nb, generator=torch.Generator().manual_seed(bs)).tolist()
+        k, v = torch.full((nb, KV, bs, d), 3.0).to(torch.bfloat16), torch.full((nb, KV, d, bs), 3.0).to(torch.bfloat16)
+        table = torch.full((len(ctxs), -(-max(ctxs) // 16) * 16 // bs), -1, dtype=torch.int32)
+        for s, c in enumerate(ctxs):
+            for b in range(-(-c // bs)):
+                # 16 keys at a time, so that either size has lost the same ones: behind the window, or lost altogether
+                first = b * bs // 16 * 16
+                if window is not None and first + 16 <= starts[s] - window + 1 and first >= keep:
+                    continue
+                if s == 2 and first in (32, 160):
+                    table[s, b] = nb + 7 if first == 32 else -5
+                    continue
+                page = ids.pop()
+                table[s, b] = page
+                n = min(bs, c - b * bs)
+                k[page, :, :n] = keys[s][b * bs:b * bs + n].transpose(0, 1)
+                v[page, :, :, :n] = vals[s][b * bs:b * bs + n].permute(1, 2, 0)
+        for tiles in ((1, 2) if d <= 128 else (1,)):
+            per = ops().prefill_rows_per_item(torch.bfloat16, d, bs, tiles)
+            rows = attention_rows(q_lens, H // KV, per, starts, ops().prefill_takes_pairs(torch.bfloat16, d, bs))
+            out = torch.full_like(q, 7.0)
+            ops().attn_prefill(q, k.to(DEV), v.to(DEV), table.to(DEV),
+                               torch.tensor([0] + list(np.cumsum(q_lens)), dtype=torch.int32, device=DEV),
+                               torch.tensor(ctxs, dtype=torch.int32, device=DEV), rows, out, H, KV, d, 0.3, window or 0,
+                               rows_per_item=per, **kw)
+            outs.append(out)
+    half = len(outs) // 2
+    for a, b in zip(outs[:half], outs[half:]):
+        assert torch.equal(a.nan_to_num(9.0), b.nan_to_num(9.0))
+
+
+def attention_rows(q_lens, G, per, starts, pairs):
+    from kvforge_amd.parts.attention import prefill_work_rows
+    rows = prefill_work_rows(q_lens, list(range(len(q_lens))), G, per, starts, pairs)
+    return torch.tensor([x for r in rows for x in r], dtype=torch.int32, device=DEV).view(-1, 3)
