@@ -625,6 +625,142 @@ __global__ __launch_bounds__(max_waves(MT, NT, AT) * KVF_WAVE) void gemm_skinny_
   }
 }
 
+// 17 to 64 rows of bf16 over tiled weights (EPI 0, 1 and 3).
+//
+// What bounded gemm_skinny_kernel here: every wave read its own fragments of A through the L1, 16
+// rows of 64 bytes each, as many bytes as of W at 64 rows, and a pass over its few k-steps ended in a
+// wait for all of them (2,048 x 16,384 with the gate: 23.6 us at 41 rows, 2.8 TB/s).  Here A goes
+// through LDS once for the workgroup, 128 columns a stage (whole cache lines), and W straight into
+// registers, both MID_AHEAD stages before they are used, so that the memory always has 64 to 96 KB of
+// a workgroup's requests; two workgroups fit a compute unit (128 registers a lane) and cover each
+// other's barriers.  Four or six stages ahead were no faster (17.6 / 18.4 us) and cost registers.
+// Eight waves: NG groups of 16 columns, the k-steps of a stage shared by 8 / NG waves whose sums are
+// added in LDS.  41 rows: 17.5 us; 20 and 61 rows 21.2 -> 16.1, 25.0 -> 18.3; a head of
+// 128,256 columns at 41 rows 131 -> 109 us, where the library took 128.
+//
+// `parts`: K is cut over gridDim.y and every cut stores its sums in fp32 as a plane of [M][N] of its
+// own, which the reader adds (rmsnorm_parts_kernel): a narrow C has too few workgroups otherwise.
+// 8,192 x 2,048 in 8 cuts at 41 / 61 rows: 10.5 / 11.0 us (the library 14.4 / 15.7 with a result
+// rounded to bf16), 2,048 x 2,048 in 4: 4.9 / 5.2 us (8.4).
+constexpr int MID_WAVES = 8;     // waves of a workgroup
+constexpr int MID_STEPS = 4;     // k-steps of 32 in a stage
+constexpr int MID_AHEAD = 3;     // stages whose loads are on their way
+template <int MT, int NG, int EPI>
+__global__ __launch_bounds__(MID_WAVES * KVF_WAVE, 4) void gemm_mid_kernel(
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ Cv, int M, int N, int K,
+    int lda, int ldc, RopeEpi rp, float* __restrict__ parts, int stages_each) {
+  constexpr int D = MID_AHEAD;
+  constexpr int KW = MID_WAVES / NG;            // waves that share a group of columns, by k-steps
+  constexpr int FR = MID_STEPS / KW;            // k-steps of a stage that one wave takes
+  constexpr int XROWS = MT * 16;
+  constexpr int XL = (XROWS * 16 + MID_WAVES * KVF_WAVE - 1) / (MID_WAVES * KVF_WAVE);   // 16-byte pieces a thread
+  static_assert(NG >= 2 && NG <= 8, "a wave takes whole k-steps of one group");
+  static_assert(2 * XROWS * 256 == MID_WAVES * MT * 1024, "the sums of the waves take the place of both stages of A");
+  __shared__ __attribute__((aligned(16))) char lds[2 * XROWS * 256];
+  const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE;
+  const int r16 = lane % 16, kg = lane / 16;
+  const int ksteps = (K + 31) / 32;
+  const int groups = (N + 15) / 16;
+  const int grp = blockIdx.x * NG + wave % NG;
+  const int stages = (ksteps + MID_STEPS - 1) / MID_STEPS;
+  const int s_lo = blockIdx.y * stages_each, s_hi = min(stages, s_lo + stages_each);
+  const int kw = wave / NG;
+  const bf16_t* wp = W + (static_cast<size_t>(min(grp, groups - 1)) * ksteps * KVF_WAVE + lane) * 8;
+  // A thread's pieces of a stage of A: rows tid / 16 (+ 32), 8 columns at tid % 16.  In LDS a row's
+  // pieces are turned by the row, so that neither the rows of a fragment nor a row's pieces share a bank.
+  const int xc = tid % 16;
+  const bf16_t* xp[XL];
+  int xo[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int row = tid / 16 + i * 32;
+    xp[i] = A + static_cast<size_t>(min(row, M - 1)) * lda + xc * 8;
+    xo[i] = row * 256 + ((xc ^ (row & 15)) * 16);
+  }
+  uint4 wr[D][FR], xr[D][XL];
+  auto load_w = [&](int slot, int s) {
+#pragma unroll
+    for (int f = 0; f < FR; ++f) {
+      const int ks = min(s * MID_STEPS + kw * FR + f, ksteps - 1);
+      wr[slot][f] = *reinterpret_cast<const uint4*>(wp + static_cast<size_t>(ks) * (KVF_WAVE * 8));
+    }
+  };
+  auto load_x = [&](int slot, int s) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      if (XROWS % 32 != 0 && i == XL - 1 && wave >= 4) continue;
+      const int k = s * (MID_STEPS * 32);
+      const bool in = k + xc * 8 + 8 <= K;
+      const uint4 v = *reinterpret_cast<const uint4*>(xp[i] + (in ? k : -xc * 8));
+      xr[slot][i] = in ? v : make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  auto put_x = [&](int slot, int buf) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      if (XROWS % 32 != 0 && i == XL - 1 && wave >= 4) continue;
+      *reinterpret_cast<uint4*>(lds + buf * (XROWS * 256) + xo[i]) = xr[slot][i];
+    }
+  };
+  f32x4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Loads past the last stage repeat it (no load stands under a condition) and are never used.
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    load_x(d, min(s_lo + d, s_hi - 1));
+    load_w(d, min(s_lo + d, s_hi - 1));
+  }
+  put_x(0, 0);
+  load_x(0, min(s_lo + D, s_hi - 1));
+  __syncthreads();
+  for (int s0 = s_lo; s0 < s_hi; s0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int s = s0 + d;
+      if (s < s_hi) {
+        const char* buf = lds + ((s - s_lo) & 1) * (XROWS * 256);
+#pragma unroll
+        for (int f = 0; f < FR; ++f) {
+          const int kl = kw * FR + f;
+          if (s * MID_STEPS + kl < ksteps) {   // the same for all lanes
+            const bf16x8 wf = __builtin_bit_cast(bf16x8, wr[d][f]);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+              const uint4 xv = *reinterpret_cast<const uint4*>(buf + (t * 16 + r16) * 256 + (((kl * 4 + kg) ^ r16) * 16));
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, xv), acc[t], 0, 0, 0);
+            }
+          }
+        }
+        load_w(d, min(s + D, s_hi - 1));
+        put_x((d + 1) % D, (s + 1 - s_lo) & 1);
+        load_x((d + 1) % D, min(s + 1 + D, s_hi - 1));
+        __syncthreads();
+      }
+    }
+  }
+  float* red = reinterpret_cast<float*>(lds);   // behind the last stage's barrier
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+    *reinterpret_cast<f32x4*>(red + ((wave * MT + t) * KVF_WAVE + lane) * 4) = acc[t];
+  __syncthreads();
+  for (int item = tid; item < NG * MT * KVF_WAVE; item += MID_WAVES * KVF_WAVE) {
+    const int l = item % KVF_WAVE, t = item / KVF_WAVE % MT, g = item / KVF_WAVE / MT;
+    f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < KW; ++q)
+      sum += *reinterpret_cast<const f32x4*>(red + (((q * NG + g) * MT + t) * KVF_WAVE + l) * 4);
+    const int m = t * 16 + l % 16, n = (blockIdx.x * NG + g) * 16 + 4 * (l / 16);
+    if (m >= M || n >= N) continue;
+    EpiOperands fresh;
+    fresh.have = false;
+    if (EPI == 0 && parts)
+      store_tile<0>(sum, m, n, N, N, parts + static_cast<size_t>(blockIdx.y) * M * N, nullptr, rp, fresh);
+    else
+      store_tile<EPI>(sum, m, n, N, ldc, Cv, nullptr, rp, fresh);
+  }
+}
+
 int g_waves_override = 0;
 int g_rows_override = 0;
 
@@ -677,6 +813,66 @@ int compute_units() {
   return known[dev];
 }
 
+// How 17 to 64 rows are cut: groups of columns a workgroup and cuts of K.  The rule takes the least
+// bytes through a compute unit's L1, over the rounds of workgroups: rows and columns over the cut's K,
+// and 16 bytes for every sum that is stored in fp32, added to the stream and read back (measured: 2,048 x
+// 2,048 at 61 rows 5.2 us as 2 x 4, 5.9 as 4 x 8; 8,192 x 2,048 11.0 as 4 x 8, 12.9 as 2 x 8; without
+// cuts 2,048 x 8,192 at 48 rows 12.7 with 2 groups, 14.2 with 4, and x 16,384 18.1 and 17.4).
+struct MidCut {
+  int groups, splits;
+};
+MidCut mid_cut(int M, int N, int K, bool may_split) {
+  const int tiles = (N + 15) / 16, stages = ((K + 31) / 32 + MID_STEPS - 1) / MID_STEPS, cus = compute_units();
+  MidCut best{4, 1};
+  long least = -1;
+  for (int ng = 2; ng <= 4; ng *= 2) {
+    for (int sp = may_split ? 2 : 1; sp <= (may_split ? 8 : 1); sp *= 2) {
+      if (sp > stages) break;
+      const int each = (stages + sp - 1) / sp;
+      if ((stages + each - 1) / each != sp) continue;    // a cut would be empty
+      const long wgs = static_cast<long>((tiles + ng - 1) / ng) * sp;
+      const long bytes = (wgs + cus - 1) / cus * (2l * MID_STEPS * 32 * each * (M + 16 * ng) + (may_split ? 16l * M * 16 * ng : 0));
+      if (least < 0 || bytes < least) {
+        least = bytes;
+        best = MidCut{ng, sp};
+      }
+    }
+  }
+  return best;
+}
+
+// Whether 17 to 64 rows without cuts of K take gemm_mid_kernel instead of gemm_skinny_kernel, which takes
+// fewer columns a workgroup and so reaches more of the chip where there are few: up to 32 rows from three
+// groups of 16 columns for each compute unit on (12,288 columns x 2,048: 16.5 -> 14.0 us; 8,192: 11.1
+// and 11.1; 4,096: 7.5 and 9.6), above, where it also re-reads more rows, from one and a half on (6,144 x
+// 2,048: 13.8 -> 12.2; 4,096: 9.8 and 11.2).
+bool mid_pays(int M, int N, int epi, int w_tiled) {
+  if (M <= 16 || M > 64 || !w_tiled || (epi != 0 && epi != 1 && epi != 3)) return false;
+  const long tiles = (N + 15) / 16, cus = compute_units();
+  return M <= 32 ? tiles >= 3 * cus : 2 * tiles >= 3 * cus;
+}
+
+template <int MT, int EPI>
+int launch_mid_mt(const bf16_t* A, const bf16_t* W, void* C, int M, int N, int K, int lda, int ldc, const RopeEpi& rp,
+                  float* parts, const MidCut& cut, hipStream_t s) {
+  const int stages = ((K + 31) / 32 + MID_STEPS - 1) / MID_STEPS, each = (stages + cut.splits - 1) / cut.splits;
+  const dim3 grid(((N + 15) / 16 + cut.groups - 1) / cut.groups, cut.splits), block(MID_WAVES * KVF_WAVE);
+  if (cut.groups == 2)
+    hipLaunchKernelGGL((gemm_mid_kernel<MT, 2, EPI>), grid, block, 0, s, A, W, C, M, N, K, lda, ldc, rp, parts, each);
+  else
+    hipLaunchKernelGGL((gemm_mid_kernel<MT, 4, EPI>), grid, block, 0, s, A, W, C, M, N, K, lda, ldc, rp, parts, each);
+  return kvf_last_error();
+}
+
+template <int EPI>
+int launch_mid(const void* A, const bf16_t* W, void* C, int M, int N, int K, int lda, int ldc, const RopeEpi& rp,
+               float* parts, const MidCut& cut, hipStream_t s) {
+  const bf16_t* a = static_cast<const bf16_t*>(A);
+  if (M <= 32) return launch_mid_mt<2, EPI>(a, W, C, M, N, K, lda, ldc, rp, parts, cut, s);
+  if (M <= 48) return launch_mid_mt<3, EPI>(a, W, C, M, N, K, lda, ldc, rp, parts, cut, s);
+  return launch_mid_mt<4, EPI>(a, W, C, M, N, K, lda, ldc, rp, parts, cut, s);
+}
+
 // How many 16-row groups of W a wave takes when A has several row tiles.  With 17 to 64 rows the
 // product is bound by what every compute unit has to bring in through its L1, which keeps only
 // some fifty lines in flight: all rows of A for each of its workgroups, and their columns of W.
@@ -718,6 +914,10 @@ int launch_nt(const void* A, const bf16_t* W, void* C, int M, int N, int K, int 
 template <int AT, int EPI>
 int launch_rows(const void* A, const bf16_t* W, void* C, int M, int N, int K, int lda, int ldc,
                 float eps, int w_tiled, const Riders& rd, const RopeEpi& rp, hipStream_t s) {
+  if constexpr (AT == 0 && (EPI == 0 || EPI == 1 || EPI == 3)) {
+    if (mid_pays(M, N, EPI, w_tiled))
+      return launch_mid<EPI>(A, W, C, M, N, K, lda, ldc, rp, nullptr, mid_cut(M, N, K, false), s);
+  }
   int err = 0;
   for (int m_base = 0; m_base < M && !err; m_base += 128) {
     const int rows = M - m_base < 128 ? M - m_base : 128;
@@ -769,6 +969,25 @@ KVF_EXPORT int kvf_gemm_bf16(const void* A, int a_type, const void* W, int w_til
   if (a_type == 0) return launch_epi<0>(A, w, C, epi, M, N, K, lda, ldc, eps, w_tiled, rd, none, s);
   if (a_type == 1) return launch_epi<1>(A, w, C, epi, M, N, K, lda, ldc, eps, w_tiled, rd, none, s);
   return static_cast<int>(hipErrorInvalidValue);
+}
+
+// A product of 17 to 64 bf16 rows cut over K, see gemm_mid_kernel.  How many parts M rows over W [N, K]
+// are stored in, or 0 where they had better be one product: wide outputs fill the chip by themselves, and
+// up to 32 rows over a matrix with fewer rows than columns gemm_skinny_kernel is as fast (4,096 x 2,048 at
+// 17 rows: 6.1 us both).
+KVF_EXPORT int kvf_gemm_bf16_parts_count(int M, int N, int K) {
+  if (M <= 16 || M > 64 || N <= 0 || N % 16 != 0 || N > 4096 || K < 1024 || K % 8 != 0 || (M <= 32 && K < N)) return 0;
+  return mid_cut(M, N, K, true).splits;
+}
+
+// parts: fp32 [kvf_gemm_bf16_parts_count(M, N, K)][M][N], whose sum is A * W^T; W in tiles.
+KVF_EXPORT int kvf_gemm_bf16_parts(const void* A, const void* W, float* parts, int count, int M, int N, int K,
+                                   int lda, hipStream_t s) {
+  if (count <= 0 || count != kvf_gemm_bf16_parts_count(M, N, K) || lda % 8 != 0 || reinterpret_cast<uintptr_t>(parts) % 16 != 0)
+    return static_cast<int>(hipErrorInvalidValue);
+  RopeEpi none{};
+  none.act_scale = 1.f;
+  return launch_mid<0>(A, static_cast<const bf16_t*>(W), nullptr, M, N, K, lda, N, none, parts, mid_cut(M, N, K, true), s);
 }
 
 // The gated pair epilogue (epi 3) with its activation chosen and biases: out[m, j] =

@@ -253,12 +253,13 @@ class Step:
             ops.add_bias(*self.owed_bias)
             self.owed_bias = None
 
-    def take_owed(self, residual: torch.Tensor) -> torch.Tensor | None:
-        """The product owed to ``residual``, for a norm kernel that adds it itself."""
+    def take_owed(self, residual: torch.Tensor, parts: bool = False) -> torch.Tensor | None:
+        """The product owed to ``residual``, for a norm kernel that adds it itself.  ``parts``: whether
+        the kernel takes a product in parts (``ops.gemm_parts``); one that does not finds it added."""
         self._settle_bias()
         if self.owed is None:
             return None
-        if self.owed[0] is not residual or len(self.owed) != 2:
+        if self.owed[0] is not residual or len(self.owed) != 2 or (self.owed[1].dim() == 3 and not parts):
             self.settle()
             return None
         product = self.owed[1]

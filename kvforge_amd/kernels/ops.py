@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 from ctypes import c_float, c_int, c_long, c_void_p
+from functools import lru_cache
 
 import torch
 
@@ -138,7 +139,8 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor | None, eps: float, out: torch
     (``weight=None``: no weight, for a norm whose weight is folded into the next matrix).
     ``add`` (``[rows of x, h]``, dtype of ``out`` or fp32) is a sum still owed to ``x``: the norm
     is taken of ``x + add``, and without ``rows`` the sum is written back to ``x`` as well.  ``bias``
-    (fp32 ``[h]``): a vector still owed to every row of ``x``, likewise."""
+    (fp32 ``[h]``): a vector still owed to every row of ``x``, likewise.  An ``add`` of three dimensions
+    is a product in parts (``gemm_parts``), fp32 ``[parts, rows of x, h]``, for a bf16 ``out``."""
     _check(x, "x", F32, (None, None))
     xr, h = x.shape
     m = out.shape[0]
@@ -151,12 +153,24 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor | None, eps: float, out: torch
         _check(rows, "rows", I32, (m,))
     elif m > xr:
         raise KernelError("rmsnorm: more output rows than input rows")
+    if bias is not None:
+        _check(bias, "bias", F32, (h,))
+    if add is not None and add.dim() == 3:
+        _check(add, "add", F32, (None, xr, h))
+        if out.dtype != BF16:
+            raise KernelError("rmsnorm: a product in parts goes with a bf16 output")
+        f = _fn("elementwise", "kvf_rmsnorm_parts",
+                [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_float, c_void_p, c_int, c_int,
+                 c_int, c_void_p])
+        _ok(f(x.data_ptr(), rows.data_ptr() if rows is not None else None, add.data_ptr(), add.shape[0],
+              bias.data_ptr() if bias is not None else None, weight.data_ptr() if weight is not None else None,
+              1 if weight is not None and weight.dtype == F32 else 0, float(eps), out.data_ptr(), m, h, xr,
+              _stream()), "rmsnorm_parts")
+        return
     if add is not None:
         _check(add, "add", None, (xr, h))
         if add.dtype not in (F32, out.dtype):
             raise KernelError(f"rmsnorm: add must be float32 or {out.dtype}, got {add.dtype}")
-    if bias is not None:
-        _check(bias, "bias", F32, (h,))
     f = _fn("elementwise", f"kvf_rmsnorm_{_suffix(out.dtype)}",
             [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_float, c_void_p, c_int, c_int,
              c_int, c_void_p])
@@ -192,8 +206,14 @@ def rmsnorm_pair(x: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, 
 
 
 def add_rows(x: torch.Tensor, delta: torch.Tensor) -> None:
-    """``x += delta`` for the fp32 residual stream ``x`` and a product ``delta`` of equal shape."""
+    """``x += delta`` for the fp32 residual stream ``x`` and a product ``delta`` of equal shape, or in
+    parts (``gemm_parts``)."""
     _check(x, "x", F32, (None, None))
+    if delta.dim() == 3:
+        _check(delta, "delta", F32, (None,) + tuple(x.shape))
+        f = _fn("elementwise", "kvf_add_parts", [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p])
+        _ok(f(x.data_ptr(), delta.data_ptr(), delta.shape[0], x.shape[0], x.shape[1], _stream()), "add_parts")
+        return
     _check(delta, "delta", None, tuple(x.shape))
     f = _fn("elementwise", f"kvf_add_rows_{_suffix(delta.dtype)}", [c_void_p, c_void_p, c_int, c_int, c_void_p])
     _ok(f(x.data_ptr(), delta.data_ptr(), x.shape[0], x.shape[1], _stream()), "add_rows")
@@ -726,6 +746,7 @@ def gated_act_rowgate(gate_up: torch.Tensor, row_gate: torch.Tensor, out: torch.
 SKINNY_MAX_M = 32
 FUSED_NORM_MAX_M = 16
 FUSED_EPILOGUE_MAX_M = 64
+MID_MAX_M = 64              # rows of the kernel that takes A through LDS, and of products in parts
 _GEMM_BF16_ARGS = ([c_void_p, c_int, c_void_p, c_int, c_void_p] + [c_int] * 6
                    + [c_float, c_void_p, c_void_p, c_void_p])
 # A product that is added to a narrow fp32 stream (few output columns, long K) has too few
@@ -844,14 +865,52 @@ def bf16_kernel_takes(a: torch.Tensor, w: torch.Tensor, rms: bool = False,
 
 def is_library_product(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm(a, w, ...)`` hands the product to the library: bf16 with more rows than the
-    weight-streaming kernel takes; or more than one tile of rows over a deep and narrow weight
-    (K >= 2 N), where that kernel has few workgroups and each re-reads every row of ``a`` along
-    a long K (measured at [2048, 8192] and 32 rows: 19 us against the library's 15)."""
+    weight-streaming kernels take; or more than one tile of rows over a deep and narrow weight
+    (K >= 2 N), where those kernels have few workgroups and each re-reads every row of ``a`` along
+    a long K (measured at [2048, 8192] and 32 rows: 19 us against the library's 15).  Over tiled weights
+    that alone bring a workgroup of 64 columns to every compute unit the streaming kernel stays ahead up
+    to 64 rows ([128256, 2048] at 41 rows 110 us against 128, [16384, 2048] 17.4 and 17.9; [12288, 4096]
+    at 48 rows 26.5 and 24.8, [32768, 1024] at 64 rows 18.2 and 16.5)."""
     m, k = a.shape
     n = w.shape[0]
     lda = a.stride(0) if m > 1 else k
-    return (a.dtype == BF16 and w.dtype == BF16 and _rows_aligned(a, k, lda)
-            and (m > SKINNY_MAX_M or (m > 16 and k >= 2 * n)))
+    if not (a.dtype == BF16 and w.dtype == BF16 and _rows_aligned(a, k, lda)):
+        return False
+    if m > SKINNY_MAX_M:
+        return not (m <= MID_MAX_M and k >= 2048 and isinstance(w, StreamedWeight)
+                    and n >= 64 * compute_units(a.device))
+    return m > 16 and k >= 2 * n
+
+
+@lru_cache(maxsize=None)
+def _parts_count(m: int, n: int, k: int, device: int) -> int:
+    with torch.cuda.device(device):
+        return int(_fn("gemm_bf16", "kvf_gemm_bf16_parts_count", [c_int] * 3)(m, n, k))
+
+
+def parts_count(a: torch.Tensor, w) -> int:
+    """In how many parts ``gemm_parts(a, w, ...)`` stores the product, 0 where it does not pay (or
+    fit): 17 to 64 bf16 rows over a tiled weight with few columns."""
+    m, k = a.shape
+    if not (16 < m <= MID_MAX_M and isinstance(w, StreamedWeight) and a.dtype == BF16 and a.stride(1) == 1
+            and _rows_aligned(a, k, a.stride(0))):
+        return 0
+    return _parts_count(m, w.shape[0], k, a.get_device())
+
+
+def gemm_parts(a: torch.Tensor, w, parts: torch.Tensor) -> None:
+    """``a @ w.T`` cut over K: ``parts``, fp32 ``[parts_count(a, w), M, N]``, receives the sums of every
+    cut, which the reader adds (``rmsnorm``, ``add_rows``).  More workgroups pull on a weight with few
+    columns than without cuts."""
+    m, k = a.shape
+    n = w.shape[0]
+    _check(a, "a", BF16, (m, w.shape[1]), contiguous=False)
+    count = parts_count(a, w)
+    if not count:
+        raise KernelError("gemm_parts: only where parts_count(a, w)")
+    _check(parts, "parts", F32, (count, m, n))
+    f = _fn("gemm_bf16", "kvf_gemm_bf16_parts", [c_void_p] * 3 + [c_int] * 5 + [c_void_p])
+    _ok(f(a.data_ptr(), w.tiles.data_ptr(), parts.data_ptr(), count, m, n, k, a.stride(0), _stream()), "gemm_parts")
 
 
 def k_halves_pay(a: torch.Tensor, w) -> bool:

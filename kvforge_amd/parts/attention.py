@@ -490,7 +490,7 @@ class PagedAttention(Mixer):
             # too many rows for the norm to ride in the projection: a norm kernel of its own,
             # which also adds what the layer before still owes the stream
             normed = ws.buf("normed", (n, self.hidden), act)
-            ops.rmsnorm(x, None, rms, normed, add=step.take_owed(residual))
+            ops.rmsnorm(x, None, rms, normed, add=step.take_owed(residual, parts=True))
             x, rms = normed, None
         fused = (not self._hooked() and self.qk_norm is None and self.row_norm is None and self.conv is None
                  and ops.bf16_kernel_takes(x, self.w_qkv, rms is not None, True)

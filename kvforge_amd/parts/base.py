@@ -172,6 +172,8 @@ class Part:
 class Norm(Part):
     # whether ``forward`` takes ``bias=``, a vector still owed to every row of ``x`` (``Step.owe_bias``)
     adds_bias = False
+    # whether ``add`` may be a product in parts (``ops.gemm_parts``: fp32 ``[parts, rows, width]``)
+    takes_parts = False
 
     def forward(self, x: torch.Tensor, out: torch.Tensor, rows: torch.Tensor | None = None,
                 add: torch.Tensor | None = None) -> None:
@@ -318,7 +320,8 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
     product is left owed to the stream (``step.owe``) so that the next norm adds it on its way
     instead of an add kernel of its own.  One tile of rows over a deep weight with few columns
     is cut into two halves of K so that every compute unit pulls on the weight: the first half
-    is added here, the second is left owed (rounded to bf16, as a stored product is).
+    is added here, the second is left owed (rounded to bf16, as a stored product is).  17 to 64 rows
+    over such a weight are cut further, and all parts are left owed in fp32 (``ops.gemm_parts``).
     ``owed``: a sum the caller took from the step (``step.take_owed``) and has not added yet;
     it is added here, in the same kernel where that is possible.
     A ``residual`` that the step holds as *fresh* (``step.fresh``: a sublayer's own output rows,
@@ -332,7 +335,14 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
         if owed is not None:
             ops.add_rows(residual, owed)
         return
-    if ops.is_library_product(a, w):
+    count = ops.parts_count(a, w) if residual.is_contiguous() and residual.data_ptr() % 16 == 0 else 0
+    if count:
+        if owed is not None:
+            ops.add_rows(residual, owed)
+        parts = step.ws.buf("owed_parts", (count, a.shape[0], w.shape[0]), torch.float32)
+        ops.gemm_parts(a, w, parts)
+        step.owe(residual, parts)
+    elif ops.is_library_product(a, w):
         if owed is not None:
             ops.add_rows(residual, owed)
         product = step.ws.buf("owed_product", (a.shape[0], w.shape[0]), a.dtype)

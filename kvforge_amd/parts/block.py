@@ -16,9 +16,9 @@ def norm_rows(norm: Norm, stream: torch.Tensor, out: torch.Tensor, step, rows: t
     """``out = norm(stream)`` (of the rows ``rows``), with what the step still owes the stream added on the way."""
     if norm.adds_bias and step.owed_bias is not None:
         bias = step.take_owed_bias(stream)
-        norm.forward(stream, out, rows, add=step.take_owed(stream), bias=bias)
+        norm.forward(stream, out, rows, add=step.take_owed(stream, norm.takes_parts), bias=bias)
     else:
-        norm.forward(stream, out, rows, add=step.take_owed(stream))
+        norm.forward(stream, out, rows, add=step.take_owed(stream, norm.takes_parts))
 
 
 @register_block("pre_norm")

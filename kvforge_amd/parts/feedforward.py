@@ -72,7 +72,7 @@ class SwiGLU(FeedForward):
             # too many rows for the norm to ride in the projection: a norm kernel of its own,
             # which also adds what the mixer still owes the stream
             normed = ws.buf("normed", (n, self.hidden), dt)
-            ops.rmsnorm(x, None, rms, normed, add=step.take_owed(residual))
+            ops.rmsnorm(x, None, rms, normed, add=step.take_owed(residual, parts=True))
             x, rms = normed, None
         else:
             step.settle()

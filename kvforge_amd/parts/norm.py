@@ -39,6 +39,10 @@ class RMSNorm(Norm):
                 add: torch.Tensor | None = None, bias: torch.Tensor | None = None) -> None:
         ops.rmsnorm(x, self.weight, self.eps, out, rows, add, bias)
 
+    @property
+    def takes_parts(self) -> bool:
+        return type(self).forward is RMSNorm.forward
+
     def add_to(self, stream: torch.Tensor, y: torch.Tensor) -> None:
         if self.weight.dtype != torch.float32:
             self.weight = self.weight.float()    # the kernel multiplies by an fp32 vector

@@ -195,6 +195,102 @@ def test_gemm_bf16_rows_in_two_to_four_tiles_over_many_columns(m, n, k, monkeypa
                                    atol=1e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(12292, 8), (16404, 136), (12288, 1000), (33000, 40)])
+def test_gemm_bf16_rows_through_lds(m, n, k):
+    """17 to 64 rows over tiles of weights with many columns: edges of the row tiles, columns that end
+    inside a group, K that ends inside a piece, a k-step or a stage; infinities stay in their columns and rows."""
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    plain_w = (torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16)
+    plain_w[5, k - 1] = plain_w[n - 1, 0] = math.inf
+    a[m - 1, k - 1] = -math.inf
+    want = a.double() @ plain_w.double().T
+    wide = torch.full((m, k + 8), math.nan, dtype=torch.bfloat16, device=DEV)   # behind the rows: never part of a sum
+    wide[:, :k] = a.to(DEV)
+    av, w = wide[:, :k], ops().StreamedWeight(plain_w.to(DEV))
+    outb = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    gate = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_fused(av, w, gate, silu_pairs=True)
+    if m <= ops().SKINNY_MAX_M:               # above, the library takes what has no epilogue over so few columns of A
+        out = torch.empty(m, n, device=DEV)
+        ops().gemm_fused(av, w, out)
+        ops().gemm_fused(av, w, outb)
+        # fp32 sums of up to 1000 products below 4 in magnitude, K 2^-24 of them
+        torch.testing.assert_close(out.double().cpu(), want, atol=1e-4, rtol=1e-4, equal_nan=True)
+        torch.testing.assert_close(outb.double().cpu(), want, atol=1e-4, rtol=2.0 ** -8, equal_nan=True)
+    gw = torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2]
+    torch.testing.assert_close(gate.double().cpu(), gw, atol=1e-3, rtol=2.0 ** -7, equal_nan=True)
+
+
+@pytest.mark.parametrize("m", [33, 64])
+def test_gemm_bf16_rows_through_lds_in_place_of_the_library(m):
+    n, k = 64 * ops().compute_units(DEV) + 16, 2056
+    g = torch.Generator().manual_seed(m)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops().StreamedWeight((torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV))
+    assert not ops().is_library_product(a, w) and ops().is_library_product(a, w.plain)
+    out = torch.empty(m, n, device=DEV)
+    ops().gemm(a, w, out)
+    torch.testing.assert_close(out.double(), a.double() @ w.plain.double().T, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 48, 64])
+@pytest.mark.parametrize("n,k", [(16, 1024), (2048, 2048), (2048, 8200), (1040, 1128), (4096, 4096), (512, 16384)])
+@pytest.mark.parametrize("weighted", [None, torch.float32, torch.bfloat16])
+def test_gemm_in_parts_and_the_norm_that_adds_them(m, n, k, weighted):
+    """The parts' sum is the product; the norm adds it to the stream (in place, or for some rows alone)
+    and ``add_rows`` does without a norm."""
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops().StreamedWeight((torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV))
+    count = ops().parts_count(a, w)
+    assert count in (2, 4, 8) and not ops().parts_count(a, w.plain)
+    parts = torch.full((count, m, n), math.nan, device=DEV)
+    ops().gemm_parts(a, w, parts)
+    product = a.double() @ w.plain.double().T
+    torch.testing.assert_close(parts.double().sum(0), product, atol=1e-4, rtol=1e-4)
+    again = torch.empty_like(parts)
+    ops().gemm_parts(a, w, again)
+    assert torch.equal(parts, again)
+    x = torch.randn(m, n, generator=g).to(DEV)
+    # a weight off its 16 bytes is read element by element
+    weight = None if weighted is None else torch.randn(n + 1, generator=g).to(weighted).to(DEV)[1:]
+    bias = None if weighted is None else torch.randn(n, generator=g).to(DEV)
+    want = x.double() + product + (0 if bias is None else bias.double())
+    normed = want * torch.rsqrt(want.pow(2).mean(-1, keepdim=True) + 1e-5) * (1 if weight is None else weight.double())
+    rows = torch.tensor([m - 1, 0, -1], dtype=torch.int32, device=DEV)
+    some, kept = torch.empty(3, n, dtype=torch.bfloat16, device=DEV), x.clone()
+    ops().rmsnorm(x, weight, 1e-5, some, rows, parts, bias)
+    assert torch.equal(x, kept)
+    torch.testing.assert_close(some[:2].double(), normed[[m - 1, 0]], atol=1e-3, rtol=2.0 ** -8)
+    assert not some[2].any()
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops().rmsnorm(x, weight, 1e-5, out, add=parts, bias=bias)
+    torch.testing.assert_close(out.double(), normed, atol=1e-3, rtol=2.0 ** -8)
+    torch.testing.assert_close(x.double(), want, atol=1e-4, rtol=1e-4)
+    ops().add_rows(kept, parts)
+    torch.testing.assert_close(kept.double(), want - (0 if bias is None else bias.double()), atol=1e-4, rtol=1e-4)
+
+
+def test_gemm_in_parts_refuses_what_does_not_fit():
+    w = ops().StreamedWeight(torch.zeros(2048, 2048, dtype=torch.bfloat16, device=DEV))
+    for m in (1, 16, 65, 128):
+        a = torch.zeros(m, 2048, dtype=torch.bfloat16, device=DEV)
+        assert not ops().parts_count(a, w)
+        with pytest.raises(ops().KernelError):
+            ops().gemm_parts(a, w, torch.zeros(4, m, 2048, device=DEV))
+    a = torch.zeros(40, 2048, dtype=torch.bfloat16, device=DEV)
+    for shape in ((ops().parts_count(a, w) + 1, 40, 2048), (40, 2048)):
+        with pytest.raises(ops().KernelError):
+            ops().gemm_parts(a, w, torch.zeros(shape, device=DEV))
+    parts = torch.zeros(ops().parts_count(a, w), 40, 2048, device=DEV)
+    with pytest.raises(ops().KernelError):               # a stream of another height
+        ops().rmsnorm(torch.zeros(41, 2048, device=DEV), None, 1e-5, torch.zeros(41, 2048, dtype=torch.bfloat16, device=DEV), add=parts)
+    with pytest.raises(ops().KernelError):               # parts go with bf16 rows
+        ops().rmsnorm(torch.zeros(40, 2048, device=DEV), None, 1e-5, torch.zeros(40, 2048, device=DEV), add=parts)
+
+
 @pytest.mark.parametrize("m", [33, 64, 100, 257])
 @pytest.mark.parametrize("n,k", [(37, 96), (384, 176), (2048, 2048), (200, 8192), (3072, 64)])
 def test_gemm_of_many_rows_through_the_library_entry_point(m, n, k):
