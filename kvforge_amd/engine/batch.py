@@ -179,6 +179,9 @@ class Step:
         self.token_ids = self.positions = self.seq_of_token = None
         self.cu_q = self.ctx_lens = self.slot_ids = self.logits_rows = None
         self.decode_seq_ids: torch.Tensor | None = None
+        # of a step of single tokens alone: all its sequences, longest context first (as they stood when
+        # the step was filled; steps that the device advances to by itself keep the order)
+        self.decode_order: torch.Tensor | None = None
         self.block_tables: list[torch.Tensor] = []
         # host copies
         self.request_ids: list[str] = []
@@ -413,7 +416,9 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     R = len(rows)
     host[off["logits_rows"]:off["logits_rows"] + R] = rows
 
-    decode = [b for b in range(Bp) if lens[b] == 1]
+    # longest context first, so that kernels which take them in this order start what lasts longest first
+    singles = np.flatnonzero(lens == 1)
+    decode = singles[np.argsort(-ctx[singles], kind="stable")].tolist()
     prefill = [b for b in range(B) if lens[b] > 1]
     host[off["decode_seq_ids"]:off["decode_seq_ids"] + len(decode)] = decode
 
@@ -436,6 +441,7 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     step.slot_ids = meta.view("slot_ids", Bp)
     step.logits_rows = meta.view("logits_rows", max(R, 1))[:R]
     step.decode_seq_ids = None if len(decode) == Bp else meta.view("decode_seq_ids", len(decode))
+    step.decode_order = meta.view("decode_seq_ids", Bp) if len(decode) == Bp else None
     step.block_tables = [meta.table_view(g)[:Bp] for g in range(len(meta.table_widths))]
     step.request_ids = [e.request_id for e in entries]
     step.q_lens = [int(x) for x in lens]

@@ -1436,7 +1436,8 @@ def attn_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                 token_is_seq: bool = False, slopes: torch.Tensor | None = None,
                 keep_first: int = 0, gate: torch.Tensor | None = None,
                 sinks: torch.Tensor | None = None, score_cap: float | None = None,
-                chunk: int = 0, dist: torch.Tensor | None = None) -> None:
+                chunk: int = 0, dist: torch.Tensor | None = None,
+                order: torch.Tensor | None = None) -> None:
     """Attention of one-token queries: sequence rows ``seq_ids[:num_seqs]`` (or ``0..num_seqs-1``)
     each attend from their token ``cu_q[seq]`` over ``ctx_lens[seq]`` cached keys.  The key
     range may be cut into ``splits`` runs; ``workspace`` then holds fp32 partial accumulators
@@ -1446,10 +1447,15 @@ def attn_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
     ``attn_prefill``; ``keep_first`` and ``gate`` likewise (the matrix-core kernels only: the
     32-bit path is given no gate, its caller gates the rows afterwards); ``sinks`` likewise (all
     kernels; with cuts the term joins the sum where the cuts are merged); ``score_cap``,
-    ``chunk`` and ``dist`` likewise."""
+    ``chunk`` and ``dist`` likewise.  ``order`` (with ``token_is_seq``): all sequences once, in the order in
+    which their workgroups are to start; results do not depend on it."""
     H, KV, d = num_heads, num_kv_heads, head_dim
     window = _mask_arg(window, chunk)
     n_seqs = _attn_common(q, k_pages, v_pages, block_table, cu_q, ctx_lens, out, H, KV, d)
+    if order is not None:
+        if not token_is_seq or seq_ids is not None:
+            raise KernelError("attn_decode: an order goes with token_is_seq")
+        _check(order, "order", I32, (num_seqs,))
     cap = _score_cap(score_cap, sinks, slopes, attention_on_matrix_cores(q.dtype, k_pages.shape[2], d))
     sl = _slopes_ptr(slopes, H, q)
     sk = _sinks_ptr(sinks, H, q)
@@ -1463,6 +1469,7 @@ def attn_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
             raise KernelError("attn_decode: seq_ids shorter than num_seqs")
     elif num_seqs > n_seqs:
         raise KernelError("attn_decode: more sequences than block-table rows")
+    first = order if order is not None else seq_ids
     nb, _, bs, _ = k_pages.shape
     if not 1 <= splits <= 64:
         raise KernelError(f"attn_decode: 1 to 64 cuts of the key range, got {splits}")
@@ -1483,7 +1490,7 @@ def attn_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
         f = _fn("attn_generic", "kvf_attn_generic_decode",
                 [c_int] + [c_void_p] * 10 + [c_int] * 13 + [c_float, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p])
         _ok(f(_tcode(q.dtype), q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(),
-              block_table.data_ptr(), seq_ids.data_ptr() if seq_ids is not None else None,
+              block_table.data_ptr(), first.data_ptr() if first is not None else None,
               None if token_is_seq else cu_q.data_ptr(), ctx_lens.data_ptr(), out.data_ptr(),
               pa.data_ptr() if pa is not None else None, pm.data_ptr() if pm is not None else None,
               num_seqs, H, KV, d, bs, nb, block_table.shape[1], q.stride(0), out.stride(0),
@@ -1493,7 +1500,7 @@ def attn_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
             [c_void_p] * 10 + [c_int] * 13
             + [c_float, c_void_p, c_void_p, c_int, c_void_p, c_float, c_void_p, c_int, c_void_p])
     _ok(f(q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), block_table.data_ptr(),
-          seq_ids.data_ptr() if seq_ids is not None else None,
+          first.data_ptr() if first is not None else None,
           None if token_is_seq else cu_q.data_ptr(),
           ctx_lens.data_ptr(), out.data_ptr(), pa.data_ptr() if pa is not None else None,
           pm.data_ptr() if pm is not None else None, num_seqs, H, KV, d, bs, nb,

@@ -567,6 +567,12 @@ class PagedAttention(Mixer):
                              score_cap=self.score_cap, chunk=chunk, dist=self.dist)
         if step.n_decode:
             splits = self._decode_cuts(step, ops.attention_on_matrix_cores(act, bs, d))
+            token_is_seq = step.decode_seq_ids is None and work is None
+            # With more workgroups than compute units the longest walks have to start first: two on one unit set
+            # the kernel's time (41 contexts of 60 to 2,900, 8 kv heads of 64: 36.5 us as the requests came, 30.9 longest
+            # first; 41 of 1,500: 31.2 and 31.4).  Up to one a unit the order's own load would be all it changes.
+            order = step.decode_order if (token_is_seq and not (window or chunk) and splits * step.n_decode * KV
+                                          > compute_units(step.device)) else None
             workspace = None
             if splits > 1:
                 workspace = (ws.buf("decode_part_acc", (step.n_decode * H * splits * d,), torch.float32),
@@ -574,9 +580,9 @@ class PagedAttention(Mixer):
             ops.attn_decode(qkv, layer.k_pages, layer.v_pages, table, step.decode_seq_ids,
                             step.n_decode, step.cu_q, step.ctx_lens, out, H, KV, d, self.scale,
                             window, splits, workspace,
-                            token_is_seq=step.decode_seq_ids is None and work is None,
-                            slopes=self.slopes, keep_first=self.keep_first, gate=gate_in_kernel,
-                            sinks=self.sinks, score_cap=self.score_cap, chunk=chunk, dist=self.dist)
+                            token_is_seq=token_is_seq, slopes=self.slopes, keep_first=self.keep_first,
+                            gate=gate_in_kernel, sinks=self.sinks, score_cap=self.score_cap, chunk=chunk,
+                            dist=self.dist, order=order)
         if gate is not None and gate_in_kernel is None:
             ops.sigmoid_gate(out, gate)
         if head_gates is not None or self.out_scale != 1.0:

@@ -69,6 +69,17 @@ def test_wanted_places_and_modes():
         StepEntry("a", [1], 0, "some").wanted()
 
 
+def test_single_tokens_are_listed_longest_context_first():
+    cache, meta, step = setup()
+    for r, n in (("a", 3), ("b", 8), ("c", 5), ("d", 8)):
+        cache.allocate(r, n)
+    entries = [StepEntry("a", [3], 2), StepEntry("b", [4], 7), StepEntry("c", [5], 4), StepEntry("d", [6], 7)]
+    fill_step(step, meta, entries, cache.block_table, lambda r: -1, 4)
+    assert step.decode_seq_ids is None and step.decode_order.tolist() == [1, 3, 2, 0]
+    fill_step(step, meta, [StepEntry("a", [3, 4], 0)] + entries[1:3], cache.block_table, lambda r: -1, 4)
+    assert step.decode_order is None and step.decode_seq_ids.tolist() == [1, 2]
+
+
 def test_pure_decode_padding_is_inert():
     cache, meta, step = setup()
     for r in "ab":
@@ -78,6 +89,7 @@ def test_pure_decode_padding_is_inert():
     assert step.n_seqs == 4 and step.n_tokens == 4 and step.n_decode == 4
     assert step.decode_seq_ids is None
     assert step.ctx_lens.tolist() == [5, 5, 0, 0]
+    assert step.decode_order.tolist() == [0, 1, 2, 3]
     assert (step.block_tables[0][2:] == -1).all()
     # a padded batch has a fixed shape: one logits row per sequence, padding included
     assert step.decode_shape == DecodeShape(n=2, max_ctx=5, sum_ctx=10) and step.n_logits == 4

@@ -1068,6 +1068,12 @@ def test_attn_decode(dtype, H, KV, d, bs, splits, window):
                       cu.to(DEV), ctx.to(DEV), same, H, KV, d, scale, window, splits, ws,
                       token_is_seq=True)
     assert torch.equal(same, out)
+    # and have them started in another order
+    ordered = torch.zeros_like(out)
+    ops().attn_decode(buf.to(DEV), paged.k.to(DEV), paged.v.to(DEV), paged.table.to(DEV), None, n,
+                      cu.to(DEV), ctx.to(DEV), ordered, H, KV, d, scale, window, splits, ws, token_is_seq=True,
+                      order=torch.tensor([4, 5, 3, 1, 0, 2], dtype=torch.int32, device=DEV))
+    assert torch.equal(ordered, out)
     # a subset of the sequences, named by seq_ids; the others stay untouched
     ids = torch.tensor([4, 1], dtype=torch.int32)
     out2 = torch.full((n, H * d), 5.0, dtype=dtype, device=DEV)
