@@ -417,9 +417,11 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     host[off["logits_rows"]:off["logits_rows"] + R] = rows
 
     # longest context first, so that kernels which take them in this order start what lasts longest first
-    singles = np.flatnonzero(lens == 1)
-    decode = singles[np.argsort(-ctx[singles], kind="stable")].tolist()
-    prefill = [b for b in range(B) if lens[b] > 1]
+    lengths = ctx.tolist()
+    decode = [b for b, n in enumerate(q_lens) if n == 1] + list(range(B, Bp))
+    if len(decode) > 1:
+        decode.sort(key=lengths.__getitem__, reverse=True)
+    prefill = [b for b, n in enumerate(q_lens) if n > 1]
     host[off["decode_seq_ids"]:off["decode_seq_ids"] + len(decode)] = decode
 
     end = off["logits_rows"] + max(R, 1)

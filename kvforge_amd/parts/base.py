@@ -335,7 +335,9 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
         if owed is not None:
             ops.add_rows(residual, owed)
         return
-    count = ops.parts_count(a, w) if residual.is_contiguous() and residual.data_ptr() % 16 == 0 else 0
+    count = 0
+    if 16 < a.shape[0] <= ops.MID_MAX_M and residual.is_contiguous() and residual.data_ptr() % 16 == 0:
+        count = ops.parts_count(a, w)
     if count:
         if owed is not None:
             ops.add_rows(residual, owed)

@@ -930,6 +930,43 @@ def test_attn_prefill(dtype, seq_lens, q_lens, H, KV, d, bs, window):
         torch.testing.assert_close(out.float().cpu(), want, **tol(dtype))
 
 
+@pytest.mark.parametrize("d,bs", [(16, 16), (64, 16), (64, 6), (128, 32), (144, 16), (256, 4), (272, 16), (640, 16)])
+@pytest.mark.parametrize("window", [0, 70, 130])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_attn_prefill_of_the_32_bit_kernel_at_the_edges_of_its_tiles(dtype, d, bs, window):
+    """Runs that end at, before and behind a tile of 64, 32 or 16 keys, windows that begin inside one and hold whole
+    ones, items alone and as second of a row; whatever lies in free pages and behind a sequence's last key is NaN."""
+    if dtype == torch.bfloat16 and ops().attention_on_matrix_cores(dtype, bs, d):
+        pytest.skip("16-bit pages of this kind go to another kernel")
+    seq_lens, q_lens, H, KV = [63, 64, 193, 257, 330], [63, 64, 65, 257, 10], 4, 2
+    paged = Paged(seq_lens, KV, d, bs, dtype, seed=d + bs)
+    free = torch.ones(paged.nb, dtype=torch.bool)
+    free[paged.table[paged.table >= 0].long()] = False
+    paged.k[free], paged.v[free] = math.nan, math.nan
+    for s, m in enumerate(seq_lens):
+        if m % bs:
+            last = paged.table[s, m // bs]
+            paged.k[last, :, m % bs:], paged.v[last, :, :, m % bs:] = math.nan, math.nan
+    g = torch.Generator().manual_seed(d)
+    n = sum(q_lens)
+    q = torch.randn(n, H * d, generator=g).to(dtype)
+    want = attn_reference(paged, q.view(n, H, d), seq_lens, q_lens, 1 / math.sqrt(d), window or None).reshape(n, H * d)
+    cu = torch.tensor([0] + list(torch.tensor(q_lens).cumsum(0)), dtype=torch.int32).to(DEV)
+    items = [(s, i) for s, m in enumerate(q_lens) for i in range(-(-m * H // KV // 64))]
+    alone = [(s, i, -1) for s, i in items]
+    paired = [(s, i, i + 1 if (s, i + 1) in items else -1) for s, i in items if i % 2 == 0]
+    got = []
+    for work in (alone, paired):
+        out = torch.full((n, H * d), 7.0, dtype=dtype, device=DEV)
+        ops().attn_prefill(q.to(DEV), paged.k.to(DEV), paged.v.to(DEV), paged.table.to(DEV), cu,
+                           torch.tensor(seq_lens, dtype=torch.int32, device=DEV),
+                           torch.tensor(work, dtype=torch.int32, device=DEV), out, H, KV, d, 1 / math.sqrt(d), window,
+                           rows_per_item=ops().prefill_rows_per_item(dtype, d, bs))
+        torch.testing.assert_close(out.float().cpu(), want, **tol(dtype))
+        got.append(out)
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("d", [144, 208, 224, 240, 256])
 @pytest.mark.parametrize("H,KV", [(32, 1), (3, 1), (6, 2)])
 @pytest.mark.parametrize("window", [0, 11])
