@@ -33,12 +33,24 @@ __device__ __forceinline__ float log_sigmoid(float x) { return fminf(x, 0.f) - l
 // v, the two log gates) goes through LDS; within a stage nothing waits for memory.  With one
 // wave there is no barrier per token; with several, the waves' shares of o and of n . q are
 // added through LDS in wave order.
+// The workgroups of a head's column blocks all read its n and m and one of them writes both: whichever has read
+// them last, for a workgroup may start when another has finished.  One thread asks, behind a barrier before
+// which every wave has used what it read; `ticket` is zero before and after.
+__device__ __forceinline__ bool last_reader(int* ticket) {
+  if (gridDim.x == 1) return true;
+  if (__hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != static_cast<int>(gridDim.x) - 1)
+    return false;
+  __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
 template <typename T, int ROWS>
 __global__ __launch_bounds__(ROWS > KVF_WAVE ? 2 * KVF_WAVE : KVF_WAVE) void mlstm_scan_kernel(const T* __restrict__ qkv, const float* __restrict__ zif,
                                   const float* __restrict__ bias_if, const int* __restrict__ cu_q,
                                   const int* __restrict__ positions, const int* __restrict__ slot_ids,
-                                  float* __restrict__ state, float* __restrict__ out, ScanArgs a) {
+                                  float* __restrict__ state, float* __restrict__ out, int* __restrict__ tickets, ScanArgs a) {
   extern __shared__ __align__(16) float lds[];
+  __shared__ int last;
   const int seq = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * COLS;
   const int lane = threadIdx.x % KVF_WAVE, wave = threadIdx.x / KVF_WAVE, RG = blockDim.x / KVF_WAVE;
   const int slot = slot_ids[seq];
@@ -143,7 +155,10 @@ __global__ __launch_bounds__(ROWS > KVF_WAVE ? 2 * KVF_WAVE : KVF_WAVE) void mls
 #pragma unroll
   for (int r = 0; r < ROWS; ++r)
     if (col_ok && r0 + r < dk) st[static_cast<size_t>(r0 + r) * dv + c] = S[r];
-  if (blockIdx.x == 0) {
+  __syncthreads();
+  if (threadIdx.x == 0) last = last_reader(tickets + seq * a.H + head);
+  __syncthreads();
+  if (last) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int r = lane + KVF_WAVE * j;
@@ -165,7 +180,7 @@ __global__ __launch_bounds__(4 * KVF_WAVE) void mlstm_token_kernel(const T* __re
                                                                    const int* __restrict__ positions,
                                                                    const int* __restrict__ slot_ids,
                                                                    float* __restrict__ state, float* __restrict__ out,
-                                                                   ScanArgs a) {
+                                                                   int* __restrict__ tickets, ScanArgs a) {
   constexpr int ROWS = 4 * R, NJ = ROWS > KVF_WAVE ? ROWS / KVF_WAVE : 1;
   __shared__ __align__(16) float ks[ROWS], qs[ROWS];
   __shared__ float Ss[ROWS][COLS];
@@ -230,18 +245,20 @@ __global__ __launch_bounds__(4 * KVF_WAVE) void mlstm_token_kernel(const T* __re
   }
   if (wave == 1) {
     float nq = 0.f;
+    int last = lane == 0 ? last_reader(tickets + seq * a.H + head) : 0;
+    last = __builtin_amdgcn_readfirstlane(last);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int r = lane + KVF_WAVE * j;
       if (r < dk) {
         nv[j] = fmaf(keep, fresh ? 0.f : nv[j], take * ks[r]);
         nq = fmaf(nv[j], qs[r], nq);
-        if (blockIdx.x == 0) st[static_cast<size_t>(dk) * dv + r] = nv[j];
+        if (last) st[static_cast<size_t>(dk) * dv + r] = nv[j];
       }
     }
     nq = wave_sum(nq);
     if (lane == 0) nq_all = nq;
-    if (lane == 0 && blockIdx.x == 0) st[static_cast<size_t>(dk) * dv + dk] = m_new;
+    if (lane == 0 && last) st[static_cast<size_t>(dk) * dv + dk] = m_new;
   }
 #pragma unroll
   for (int r = 0; r < R; ++r)
@@ -277,7 +294,8 @@ __global__ __launch_bounds__(256) void mlstm_chunk_kernel(const T* __restrict__ 
                                                           const int* __restrict__ positions,
                                                           const int* __restrict__ slot_ids,
                                                           float* __restrict__ state, float* __restrict__ out,
-                                                          ScanArgs a) {
+                                                          int* __restrict__ tickets, ScanArgs a) {
+  __shared__ int last;
   extern __shared__ __align__(16) float lds[];
   constexpr int QLD = DKP + 4, ALD = CL + 4, VLD = CL + 4, SLD = DKP + 4;
   // the running sum of the log forget gates is kept in 64 bits: its differences b_t - b_s are
@@ -494,11 +512,13 @@ __global__ __launch_bounds__(256) void mlstm_chunk_kernel(const T* __restrict__ 
     if (tid == 0) m_c = mt[last];
   }
   __syncthreads();
+  if (tid == 0) last = last_reader(tickets + blockIdx.z * a.H + blockIdx.y);
   for (int i = tid; i < DKP * CCOLS; i += blockDim.x) {
     const int r = i / CCOLS, cl = i % CCOLS, c = col0 + cl;
     if (r < dk && c < dv) st[static_cast<size_t>(r) * dv + c] = St[cl * SLD + r];
   }
-  if (blockIdx.x == 0) {
+  __syncthreads();
+  if (last) {
     for (int r = tid; r < dk; r += blockDim.x) st[static_cast<size_t>(dk) * dv + r] = ns[r];
     if (tid == 0) st[static_cast<size_t>(dk) * dv + dk] = m_c;
   }
@@ -511,7 +531,7 @@ template <int DKP, int CL> constexpr size_t chunk_lds() {
 
 template <typename T, int DKP, int CL>
 int chunk_go(const void* qkv, const float* zif, const float* bias_if, const int* cu_q, const int* positions,
-             const int* slot_ids, float* state, float* out, int num_seqs, ScanArgs a, hipStream_t s) {
+             const int* slot_ids, float* state, float* out, int num_seqs, int* tickets, ScanArgs a, hipStream_t s) {
   constexpr size_t lds = chunk_lds<DKP, CL>();
   static bool allowed = false;   // more LDS than a kernel gets unasked: asked for once per kernel
   if (!allowed) {
@@ -522,15 +542,15 @@ int chunk_go(const void* qkv, const float* zif, const float* bias_if, const int*
   }
   const dim3 grid((a.dv + CCOLS - 1) / CCOLS, a.H, num_seqs);
   hipLaunchKernelGGL((mlstm_chunk_kernel<T, DKP, CL>), grid, dim3(256), lds, s, static_cast<const T*>(qkv), zif,
-                     bias_if, cu_q, positions, slot_ids, state, out, a);
+                     bias_if, cu_q, positions, slot_ids, state, out, tickets, a);
   return kvf_last_error();
 }
 
 template <typename T>
 int chunk_launch(const void* qkv, const float* zif, const float* bias_if, const int* cu_q, const int* positions,
-                 const int* slot_ids, float* state, float* out, int num_seqs, ScanArgs a, hipStream_t s) {
+                 const int* slot_ids, float* state, float* out, int num_seqs, int* tickets, ScanArgs a, hipStream_t s) {
   if (num_seqs <= 0) return 0;
-#define GO(DKP, CL) return chunk_go<T, DKP, CL>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, a, s)
+#define GO(DKP, CL) return chunk_go<T, DKP, CL>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, tickets, a, s)
   if (a.dk <= 32) GO(32, 64);
   if (a.dk <= 64) GO(64, 64);
   if (a.dk <= 128) GO(128, 64);
@@ -929,12 +949,12 @@ int multi_launch(const void* qkv, const float* zif, const float* bias_if, const 
 
 template <typename T>
 int scan_launch(const void* qkv, const float* zif, const float* bias_if, const int* cu_q, const int* positions,
-                const int* slot_ids, float* state, float* out, int num_seqs, bool single, ScanArgs a, hipStream_t s) {
+                const int* slot_ids, float* state, float* out, int num_seqs, bool single, int* tickets, ScanArgs a, hipStream_t s) {
   if (num_seqs <= 0) return 0;
   if (single && a.dk <= TOKEN_MAX_KEY) {
 #define GO(R)                                                                                           \
   hipLaunchKernelGGL((mlstm_token_kernel<T, R>), dim3((a.dv + COLS - 1) / COLS, a.H, num_seqs), dim3(4 * KVF_WAVE), 0, s, \
-                     static_cast<const T*>(qkv), zif, bias_if, cu_q, positions, slot_ids, state, out, a)
+                     static_cast<const T*>(qkv), zif, bias_if, cu_q, positions, slot_ids, state, out, tickets, a)
     if (a.dk <= 32) GO(8);
     else if (a.dk <= 64) GO(16);
     else GO(32);
@@ -947,7 +967,7 @@ int scan_launch(const void* qkv, const float* zif, const float* bias_if, const i
   const size_t lds = sizeof(float) * (static_cast<size_t>(TB) * (2 * a.dk + COLS + 2) + rg * (COLS + 1));
 #define GO(ROWS)                                                                                  \
   hipLaunchKernelGGL((mlstm_scan_kernel<T, ROWS>), grid, block, lds, s, static_cast<const T*>(qkv), zif, \
-                     bias_if, cu_q, positions, slot_ids, state, out, a)
+                     bias_if, cu_q, positions, slot_ids, state, out, tickets, a)
   if (rows == 32) GO(32);
   else if (rows == 64) GO(64);
   else GO(128);
@@ -993,13 +1013,15 @@ int out_launch(const float* o, const void* g, int g_stride, const float* w, floa
 // runs of at least multi_from tokens by the four passes over all chunks at once (n_chunks > 0:
 // `chunks` [n_chunks, 4] and `runs` [n_runs, 3] name them, the other pointers are their scratch);
 // each kernel leaves the others' sequences alone.
+// tickets: int [num_seqs][H], zero before and after (see last_reader); calls that share them must not overlap.
 KVF_EXPORT int kvf_mlstm_scan(int dtype, const void* qkv, const float* zif, const float* bias_if,
                               const int* cu_q, const int* positions, const int* slot_ids, float* state,
                               float* out, int num_seqs, int H, int dk, int dv, int row_len, int q_off,
                               int k_off, int v_off, int n_slots, int gate_stride, float cap, float q_scale, int chunk_from,
                               int short_runs, int long_runs, int multi_from, int n_chunks, int n_runs,
                               const int* chunks, const int* runs, float* w_li, float* w_mt, double* w_bc,
-                              float* w_mc, float* w_gl, float* w_W, float* w_un, hipStream_t s) {
+                              float* w_mc, float* w_gl, float* w_W, float* w_un, int* tickets, hipStream_t s) {
+  if ((short_runs || long_runs) && !tickets) return static_cast<int>(hipErrorInvalidValue);
   if (H <= 0 || dk <= 0 || dk > 256 || dv <= 0 || !(cap > 0.f) || num_seqs > 65535 || H > 65535 || chunk_from < 1 ||
       gate_stride < 2 * H || multi_from < chunk_from)
     return static_cast<int>(hipErrorInvalidValue);
@@ -1008,11 +1030,11 @@ KVF_EXPORT int kvf_mlstm_scan(int dtype, const void* qkv, const float* zif, cons
                    multi_from};
   int code = 0;
   if (short_runs)
-    code = dtype == 0 ? scan_launch<float>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, short_runs == 2, a, s)
-                      : scan_launch<bf16_t>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, short_runs == 2, a, s);
+    code = dtype == 0 ? scan_launch<float>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, short_runs == 2, tickets, a, s)
+                      : scan_launch<bf16_t>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, short_runs == 2, tickets, a, s);
   if (code == 0 && long_runs)
-    code = dtype == 0 ? chunk_launch<float>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, a, s)
-                      : chunk_launch<bf16_t>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, a, s);
+    code = dtype == 0 ? chunk_launch<float>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, tickets, a, s)
+                      : chunk_launch<bf16_t>(qkv, zif, bias_if, cu_q, positions, slot_ids, state, out, num_seqs, tickets, a, s);
   if (code == 0 && n_chunks > 0) {
     if (!chunks || !runs || !w_li || !w_mt || !w_bc || !w_mc || !w_gl || !w_W || !w_un)
       return static_cast<int>(hipErrorInvalidValue);

@@ -1555,7 +1555,7 @@ def mlstm_scan(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor,
                num_seqs: int, heads: int, key_dim: int, value_dim: int, q_off: int, k_off: int,
                v_off: int, cap: float, q_scale: float, chunk_from: int = MLSTM_CHUNK_FROM,
                short_runs: bool = True, long_runs: bool = True, multi_from: int | None = None,
-               multi: dict | None = None, single: bool = False) -> None:
+               multi: dict | None = None, single: bool = False, tickets: torch.Tensor | None = None) -> None:
     """The matrix-memory recurrence over every sequence's tokens of this step, from and into the
     sequences' state slots.  ``rows [N, >= ...]``: projected rows holding q (``heads * key_dim``
     elements from column ``q_off``), k (from ``k_off``) and v (``heads * value_dim`` from
@@ -1597,6 +1597,11 @@ def mlstm_scan(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor,
     _check(out, "out", F32, (n, H * dv))
     if chunk_from < 1:
         raise KernelError(f"mlstm_scan: chunk_from must be positive, got {chunk_from}")
+    if tickets is None:
+        tickets = torch.zeros(max(1, int(num_seqs) * H), dtype=I32, device=rows.device)
+    _check(tickets, "tickets", I32, (None,))
+    if tickets.shape[0] < num_seqs * H:
+        raise KernelError("mlstm_scan: fewer tickets than sequences times heads")
     n_chunks = n_runs = 0
     extra = [None] * 9
     big = 2**31 - 1
@@ -1611,13 +1616,13 @@ def mlstm_scan(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor,
             _check(multi[name], name, dtype, shape)
         extra = [multi[k].data_ptr() for k in ("chunks", "runs", "li", "mt", "bc", "mc", "gl", "W", "un")]
     f = _fn("mlstm", "kvf_mlstm_scan", [c_int] + [c_void_p] * 8 + [c_int] * 10 + [c_float, c_float] + [c_int] * 6
-            + [c_void_p] * 9 + [c_void_p])
+            + [c_void_p] * 10 + [c_void_p])
     _ok(f(_tcode(rows.dtype), rows.data_ptr(), gates.data_ptr(), gate_bias.data_ptr(), cu_q.data_ptr(),
           positions.data_ptr(), slot_ids.data_ptr(), state.data_ptr(), out.data_ptr(), int(num_seqs),
           H, dk, dv, rows.stride(0) if n > 1 else rows.shape[1], int(q_off), int(k_off), int(v_off),
           state.shape[0], gates.shape[1], float(cap), float(q_scale), int(chunk_from), (2 if single and chunk_from > 1 else 1) if short_runs else 0,
           1 if long_runs else 0, multi_from if multi is not None else big, n_chunks, n_runs, *extra,
-          _stream()), "mlstm_scan")
+          tickets.data_ptr(), _stream()), "mlstm_scan")
 
 
 def mlstm_out(heads_raw: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, eps: float,

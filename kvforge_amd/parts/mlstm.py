@@ -131,7 +131,8 @@ class MatrixLSTM(Mixer):
         ops.mlstm_scan(rows, gates, self.gate_bias, step.cu_q, step.positions, step.slot_ids,
                        layer.state, raw, step.n_seqs, H, dk, dv, 0, H * dk, 2 * H * dk,
                        self.gate_cap, float(dk) ** -0.5, short_runs=short_runs, long_runs=long_runs,
-                       multi=self._longest_runs(step, n), single=max(step.q_lens, default=0) <= 1)
+                       multi=self._longest_runs(step, n), single=max(step.q_lens, default=0) <= 1,
+                       tickets=ws.zeros("mlstm_tickets", (max(1, step.n_seqs * H),), torch.int32))
         heads = ws.buf("mlstm_heads", (n, H * dv), act)
         g0 = 2 * H * dk + H * dv
         ops.mlstm_out(raw, rows[:, g0:g0 + H * dv], self.head_weight, self.norm_eps, heads, H, dv)

@@ -385,6 +385,47 @@ def test_heads_normed_weighted_and_gated(dtype):
     torch.testing.assert_close(out.float().cpu(), want, **tol(dtype))
 
 
+@pytest.mark.parametrize("T", [1, 5, 40])
+@pytest.mark.parametrize("dk,dv,n", [(24, 130, 3), (128, 256, 70), (200, 700, 9)])
+def test_column_blocks_of_a_head_read_its_sums_before_one_of_them_writes(T, dk, dv, n):
+    """The state's key sum and maximum belong to all workgroups of a head, more of them than run at a time: every
+    column's output and state in 64 bits from the state as it was, by all three kernels (single tokens, runs
+    token by token, runs in chunks); the tickets are zero again."""
+    H, cap = 5, 15.0
+    g = torch.Generator().manual_seed(dk + T)
+    rows = torch.randn(n * T, 2 * H * dk + H * dv, generator=g)
+    z, bias = torch.randn(n * T, 2 * H, generator=g), torch.randn(2 * H, generator=g)
+    old = torch.randn(n, H, dk * dv + dk + 1, generator=g) * 0.5
+    state, out = old.clone().view(n, -1).to(DEV), torch.empty(n * T, H * dv, device=DEV)
+    tickets = torch.zeros(n * H, dtype=torch.int32, device=DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    ops().mlstm_scan(rows.to(DEV), z.to(DEV), bias.to(DEV), i32([T * j for j in range(n + 1)]),
+                     i32([3 + t for _ in range(n) for t in range(T)]), i32(list(range(n))), state, out, n, H, dk, dv,
+                     0, H * dk, 2 * H * dk, cap, dk ** -0.5, single=T == 1, tickets=tickets)
+    q, k, v = (t.reshape(n, T, H, -1).double() for t in rows.split([H * dk, H * dk, H * dv], 1))
+    li, lf = (cap * torch.tanh((z + bias).view(n, T, 2, H).double() / cap)).unbind(2)
+    lf = torch.nn.functional.logsigmoid(lf)
+    S, s, m = (t.double() for t in (old[..., :dk * dv].reshape(n, H, dk, dv), old[..., dk * dv:-1], old[..., -1]))
+    want = []
+    for t in range(T):
+        new = torch.maximum(lf[:, t] + m, li[:, t])
+        keep, take = torch.exp(lf[:, t] + m - new), torch.exp(li[:, t] - new)
+        m, kt = new, take[..., None] * k[:, t]
+        S = keep[..., None, None] * S + kt[..., None] * v[:, t, :, None]
+        s = keep[..., None] * s + kt
+        qt = q[:, t] * dk ** -0.5
+        den = torch.maximum((s * qt).sum(-1).abs(), torch.exp(-m)) + 1e-6
+        want.append((S * qt[..., None]).sum(2) / den[..., None])
+    want = torch.stack(want, 1).reshape(n * T, H * dv)
+    got = state.view(n, H, -1).double().cpu()
+    # fp32 sums of up to 200 products and 40 tokens: some hundred roundings of 2^-24
+    for a, b in ((got[..., :dk * dv], S.flatten(2)), (got[..., dk * dv:-1], s), (got[..., -1], m)):
+        torch.testing.assert_close(a, b, atol=1e-4, rtol=1e-4)
+    # a denominator near zero magnifies the numerator's rounding
+    assert float((out.double().cpu() - want).norm() / want.norm()) < 1e-3
+    assert not tickets.any()
+
+
 @pytest.mark.parametrize("R,top", [(5, 1), (20, 3), (64, 8), (130, 4), (512, 16), (3, 3)])
 def test_router_chooses_by_corrected_probability_and_weighs_by_probability(R, top):
     n = 50
