@@ -15,83 +15,99 @@ constexpr int MAX_TOP = 16;
 // largest z are chosen, and weighted by the softmax over the chosen z.  The weights are then
 // multiplied by `scale`.  sel [N, top], wgt [N, top].
 enum { SCORE_SOFTMAX = 0, SCORE_SIGMOID = 1, SCORE_CHOSEN = 2 };
-__global__ __launch_bounds__(KVF_WAVE) void moe_topk_kernel(const float* __restrict__ z, int z_stride,
-                                                            const float* __restrict__ bias,
-                                                            const float* __restrict__ correction,
-                                                            int* __restrict__ sel, float* __restrict__ wgt,
-                                                            int R, int top, int score, int renorm, float scale) {
-  const int n = blockIdx.x, lane = threadIdx.x;
-  const float* zr = z + static_cast<size_t>(n) * z_stride;
-  float s[MAX_PER_LANE], c[MAX_PER_LANE];
+// PER: router outputs a lane holds.  What bounds a token is the chain of sums and maxima over the lanes: a choice
+// takes one maximum, its index (one output a lane: from the lanes that hold the maximum) and its score are read
+// off the lane.  8 tokens of 34 outputs, 4 choices: 6.7 us with eight outputs a lane and three chains a choice; now
+// 5.8 with the plan behind them (moe_choose_plan_kernel).
+template <int PER>
+__device__ __forceinline__ void choose(const float* __restrict__ zr, const float* __restrict__ bias,
+                                       const float* __restrict__ correction, int R, int top, int score, int renorm,
+                                       float scale, int& picked, float& weight) {
+  const int lane = threadIdx.x % KVF_WAVE;
+  float s[PER], c[PER];
   float mx = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < MAX_PER_LANE; ++j) {
+  for (int j = 0; j < PER; ++j) {
     const int e = lane + KVF_WAVE * j;
+    c[j] = correction && e < R ? correction[e] : 0.f;
     s[j] = e < R ? zr[e] + (bias ? bias[e] : 0.f) : -INFINITY;
     mx = fmaxf(mx, s[j]);
   }
   if (score == SCORE_SIGMOID) {
 #pragma unroll
-    for (int j = 0; j < MAX_PER_LANE; ++j) s[j] = 1.f / (1.f + expf(-s[j]));
+    for (int j = 0; j < PER; ++j) s[j] = 1.f / (1.f + expf(-s[j]));
   } else if (score == SCORE_SOFTMAX) {
     mx = wave_max(mx);
     float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < MAX_PER_LANE; ++j) {
+    for (int j = 0; j < PER; ++j) {
       const int e = lane + KVF_WAVE * j;
       s[j] = e < R ? expf(s[j] - mx) : 0.f;
       sum += s[j];
     }
     sum = wave_sum(sum);
 #pragma unroll
-    for (int j = 0; j < MAX_PER_LANE; ++j) s[j] = s[j] / sum;
+    for (int j = 0; j < PER; ++j) s[j] = s[j] / sum;
   }
 #pragma unroll
-  for (int j = 0; j < MAX_PER_LANE; ++j) {
+  for (int j = 0; j < PER; ++j) {
     const int e = lane + KVF_WAVE * j;
-    c[j] = e < R ? s[j] + (correction ? correction[e] : 0.f) : -INFINITY;
+    c[j] = e < R ? s[j] + c[j] : -INFINITY;
   }
+  constexpr int NONE = 0x7fffffff;
   float picked_s = 0.f, total = 0.f;   // lane k keeps the k-th choice
-  int picked_e = -1;
+  picked = -1;
   for (int k = 0; k < top; ++k) {
-    float best = -INFINITY;
-    int at = 0x7fffffff;
+    float best = -INFINITY, mine = 0.f;
+    int at = NONE;
 #pragma unroll
-    for (int j = 0; j < MAX_PER_LANE; ++j) {
-      const int e = lane + KVF_WAVE * j;
+    for (int j = 0; j < PER; ++j) {
       if (c[j] > best) {   // a lane's own candidates come in rising index: '>' keeps the lowest
         best = c[j];
-        at = e;
+        mine = s[j];
+        at = lane + KVF_WAVE * j;
       }
     }
     const float wbest = wave_max(best);
-    int cand = best == wbest ? at : 0x7fffffff;
+    int cand = best == wbest ? at : NONE;
+    if (PER == 1) {
+      const unsigned long long who = __ballot(cand != NONE);
+      cand = who ? __builtin_ctzll(who) : NONE;
+    } else {
 #pragma unroll
-    for (int o = KVF_WAVE / 2; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, KVF_WAVE));
-    // the owner hands over its probability and retires the choice
-    float sv = 0.f;
-#pragma unroll
-    for (int j = 0; j < MAX_PER_LANE; ++j) {
-      if (lane + KVF_WAVE * j == cand) {
-        sv = s[j];
-        c[j] = -INFINITY;
-      }
+      for (int o = KVF_WAVE / 2; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, KVF_WAVE));
     }
-    sv = wave_sum(sv);   // one lane holds it, the others zero
+    // the owner hands over its score and retires the choice
+    const float sv = cand == NONE ? 0.f : __shfl(mine, cand % KVF_WAVE, KVF_WAVE);
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (lane + KVF_WAVE * j == cand) c[j] = -INFINITY;
     total += sv;
     if (lane == k) {
       picked_s = sv;
-      picked_e = cand;
+      picked = cand;
     }
   }
   if (score == SCORE_CHOSEN) {   // the first choice has the largest z
     picked_s = lane < top ? expf(picked_s - __shfl(picked_s, 0, KVF_WAVE)) : 0.f;
     total = wave_sum(picked_s);
   }
+  weight = (score == SCORE_CHOSEN ? picked_s / total : renorm ? picked_s / (total + 1e-20f) : picked_s) * scale;
+}
+
+template <int PER>
+__global__ __launch_bounds__(KVF_WAVE) void moe_topk_kernel(const float* __restrict__ z, int z_stride,
+                                                            const float* __restrict__ bias,
+                                                            const float* __restrict__ correction,
+                                                            int* __restrict__ sel, float* __restrict__ wgt,
+                                                            int R, int top, int score, int renorm, float scale) {
+  const int n = blockIdx.x, lane = threadIdx.x;
+  int picked;
+  float weight;
+  choose<PER>(z + static_cast<size_t>(n) * z_stride, bias, correction, R, top, score, renorm, scale, picked, weight);
   if (lane < top) {
-    sel[static_cast<size_t>(n) * top + lane] = picked_e;
-    wgt[static_cast<size_t>(n) * top + lane] =
-        (score == SCORE_CHOSEN ? picked_s / total : renorm ? picked_s / (total + 1e-20f) : picked_s) * scale;
+    sel[static_cast<size_t>(n) * top + lane] = picked;
+    wgt[static_cast<size_t>(n) * top + lane] = weight;
   }
 }
 
@@ -176,10 +192,9 @@ __device__ __forceinline__ uint2 pack4(const f32x4& a) {
                     static_cast<uint32_t>(f32_to_bf16(a[2])) | (static_cast<uint32_t>(f32_to_bf16(a[3])) << 16));
 }
 
-__global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ sel, int pairs, int E,
-                                                        int* __restrict__ where, int* __restrict__ order,
-                                                        int* __restrict__ tiles, int* __restrict__ num_tiles,
-                                                        int max_tiles, int tile_shift) {
+// All threads of the one workgroup; sel in LDS or memory.
+__device__ __forceinline__ void plan(const int* sel, int pairs, int E, int* __restrict__ where, int* __restrict__ order,
+                                     int* __restrict__ tiles, int* __restrict__ num_tiles, int max_tiles, int tile_shift) {
   __shared__ int cnt[PLAN_MAX_EXPERTS], off[PLAN_MAX_EXPERTS], first_tile[PLAN_MAX_EXPERTS];
   const int tid = threadIdx.x, step = static_cast<int>(blockDim.x);
   const int per = (E + KVF_WAVE - 1) / KVF_WAVE;   // experts a lane of the first wave adds up
@@ -258,6 +273,39 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
       if (named || once) where[p] = named ? off[expert] + place : -1;
     });
   }
+}
+
+__global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ sel, int pairs, int E,
+                                                        int* __restrict__ where, int* __restrict__ order,
+                                                        int* __restrict__ tiles, int* __restrict__ num_tiles,
+                                                        int max_tiles, int tile_shift) {
+  plan(sel, pairs, E, where, order, tiles, num_tiles, max_tiles, tile_shift);
+}
+
+// The choices of a few tokens, a wave each, and their plan in one kernel: up to CHOOSE_TOKENS tokens a launch
+// and a trip of the choices through memory cost more than the waves of one workgroup do (8 tokens of 34 outputs:
+// 5.8 us, two kernels of 6.7 and 3.9 before).
+constexpr int CHOOSE_TOKENS = 16;
+template <int PER>
+__global__ __launch_bounds__(CHOOSE_TOKENS * KVF_WAVE) void moe_choose_plan_kernel(
+    const float* __restrict__ z, int z_stride, const float* __restrict__ bias, const float* __restrict__ correction,
+    int* __restrict__ sel, float* __restrict__ wgt, int n, int R, int top, int score, int renorm, float scale, int E,
+    int* __restrict__ where, int* __restrict__ order, int* __restrict__ tiles, int* __restrict__ num_tiles, int max_tiles,
+    int tile_shift) {
+  __shared__ int chosen[CHOOSE_TOKENS * MAX_TOP];
+  const int lane = threadIdx.x % KVF_WAVE, token = threadIdx.x / KVF_WAVE;
+  if (token < n) {
+    int picked;
+    float weight;
+    choose<PER>(z + static_cast<size_t>(token) * z_stride, bias, correction, R, top, score, renorm, scale, picked, weight);
+    if (lane < top) {
+      chosen[token * top + lane] = picked;
+      sel[token * top + lane] = picked;
+      wgt[token * top + lane] = weight;
+    }
+  }
+  __syncthreads();
+  plan(chosen, n * top, E, where, order, tiles, num_tiles, max_tiles, tile_shift);
 }
 
 // v_mfma_f32_16x16x32_bf16 computes D[i][j] += sum_k A[i][k] B[j][k]; lane 16 c + r gives row r,
@@ -657,8 +705,13 @@ KVF_EXPORT int kvf_moe_topk(const float* z, int z_stride, const float* bias, con
   if (score < SCORE_SOFTMAX || score > SCORE_CHOSEN || (score == SCORE_CHOSEN && correction) ||
       R <= 0 || R > MAX_PER_LANE * KVF_WAVE || top <= 0 || top > MAX_TOP || top > R)
     return static_cast<int>(hipErrorInvalidValue);
-  hipLaunchKernelGGL(moe_topk_kernel, dim3(n), dim3(KVF_WAVE), 0, s, z, z_stride, bias, correction, sel, wgt, R,
-                     top, score, renorm, scale);
+#define GO(PER)                                                                                                    \
+  hipLaunchKernelGGL(moe_topk_kernel<PER>, dim3(n), dim3(KVF_WAVE), 0, s, z, z_stride, bias, correction, sel, wgt, R, \
+                     top, score, renorm, scale)
+  if (R <= KVF_WAVE) GO(1);
+  else if (R <= 2 * KVF_WAVE) GO(2);
+  else GO(MAX_PER_LANE);
+#undef GO
   return kvf_last_error();
 }
 
@@ -720,18 +773,45 @@ KVF_EXPORT int kvf_moe_grouped_many_rows(int pairs, int E, int ff, int K) {
   return pairs >= 6ll * E && (pairs + 8ll * E) * ff * K >= 248000ll * (ff + K);
 }
 
+// kvf_moe_topk of up to CHOOSE_TOKENS tokens together with the plan of kvf_moe_grouped, which is then called with
+// `planned`; arguments as there.
+KVF_EXPORT int kvf_moe_choose_tokens() { return CHOOSE_TOKENS; }
+KVF_EXPORT int kvf_moe_topk_plan(const float* z, int z_stride, const float* bias, const float* correction, int* sel,
+                                 float* wgt, int n, int R, int top, int score, int renorm, float scale, int E, int ff, int K,
+                                 int* where, int* order, int* tiles, int* num_tiles, int max_tiles, int many_rows,
+                                 hipStream_t s) {
+  if (n <= 0) return 0;
+  const int pairs = n * top;
+  if (n > CHOOSE_TOKENS || score < SCORE_SOFTMAX || score > SCORE_CHOSEN || (score == SCORE_CHOSEN && correction) ||
+      R <= 0 || R > MAX_PER_LANE * KVF_WAVE || top <= 0 || top > MAX_TOP || top > R || E <= 0 || E > PLAN_MAX_EXPERTS ||
+      max_tiles < (pairs + 15) / 16 + E)
+    return static_cast<int>(hipErrorInvalidValue);
+  const bool many = many_rows < 0 ? kvf_moe_grouped_many_rows(pairs, E, ff, K) != 0 : many_rows != 0;
+  // the plan has a thread for every expert
+  const int threads = n * KVF_WAVE > E ? n * KVF_WAVE : (E + KVF_WAVE - 1) / KVF_WAVE * KVF_WAVE;
+#define GO(PER)                                                                                                      \
+  hipLaunchKernelGGL(moe_choose_plan_kernel<PER>, dim3(1), dim3(threads), 0, s, z, z_stride, bias, correction, sel, wgt, n, \
+                     R, top, score, renorm, scale, E, where, order, tiles, num_tiles, max_tiles, many ? WIDE_SHIFT : 4)
+  if (R <= KVF_WAVE) GO(1);
+  else if (R <= 2 * KVF_WAVE) GO(2);
+  else GO(MAX_PER_LANE);
+#undef GO
+  return kvf_last_error();
+}
+
 // The routed experts of a bf16 step without the rows that did not choose them.  x [n, K] (row
 // stride ldx), w_gate_up / w_down: the tiled forms of [E 2 ff, K] (gate and up rows interleaved)
 // and [K, E ff]; sel / wgt [n, top]; scratch: where, order [n top], tiles [3 max_tiles],
 // num_tiles [1], act [n top, ff], y [n top, K].  Needs K % 8 == 0 and ff % 32 == 0.  weigh_input: the
 // weights go into the experts' inputs instead of the sum over their outputs.  fresh: residual is
 // written, not added to.  form, limit: how an expert's pairs are joined (GateForm's act 0 or 2).  many_rows: below
-// 0, or which kernels are taken whatever the sizes (0: those of few rows, else those of more).
+// 0, or which kernels are taken whatever the sizes (0: those of few rows, else those of more).  planned: where,
+// order, tiles and num_tiles hold the plan already (kvf_moe_topk_plan).
 KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int K, int E, int ff, int top,
                                const void* w_gate_up, const void* w_down, const int* sel, const float* wgt,
                                int* where, int* order, int* tiles, int* num_tiles, int max_tiles, void* act,
                                void* y, float* residual, int weigh_input, int fresh, int form, float limit,
-                               int many_rows, hipStream_t s) {
+                               int many_rows, int planned, hipStream_t s) {
   if (n <= 0) return 0;
   const int pairs = n * top;
   const bool many = many_rows < 0 ? kvf_moe_grouped_many_rows(pairs, E, ff, K) != 0 : many_rows != 0;
@@ -739,8 +819,9 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int
   if (!form_ok(form, limit) || E <= 0 || E > PLAN_MAX_EXPERTS || K % 8 != 0 || ff % 32 != 0 || ldx % 8 != 0 || max_tiles > 65535 ||
       max_tiles < (pairs + 15) / 16 + E)
     return static_cast<int>(hipErrorInvalidValue);
-  hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel, pairs, E, where, order, tiles, num_tiles,
-                     max_tiles, many ? WIDE_SHIFT : 4);
+  if (!planned)
+    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel, pairs, E, where, order, tiles, num_tiles,
+                       max_tiles, many ? WIDE_SHIFT : 4);
   const int S = (K + 31) / 32, up_groups = ff / 8, down_groups = (K + 15) / 16;
   const bf16_t* xb = static_cast<const bf16_t*>(x);
   const uint4 *up = static_cast<const uint4*>(w_gate_up), *down = static_cast<const uint4*>(w_down);

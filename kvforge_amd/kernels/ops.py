@@ -1573,7 +1573,8 @@ def mlstm_scan(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor,
     carry over a run's chunks, the outputs): ``chunks`` ``[n, 4]`` and ``runs`` ``[r, 3]`` (int32,
     from ``mlstm_multi_plan``) and the scratch tensors of ``mlstm_multi_scratch``; without it no
     run is that long for the kernels (``multi_from`` is then ignored).  ``single``: no run of the step holds more than one
-    token (a decode step), which keys of up to 128 have a kernel for; the same bits."""
+    token (a decode step), which keys of up to 128 have a kernel for; the same bits.  ``tickets``: at least
+    ``num_seqs * heads`` ints that are zero and left so (made anew if not given; calls that share them must not overlap)."""
     n = rows.shape[0]
     H, dk, dv = int(heads), int(key_dim), int(value_dim)
     _check(rows, "rows", None, (n, None), contiguous=False)
@@ -1879,16 +1880,29 @@ def _moe_form(form: str, limit: float | None, who: str) -> tuple[int, float]:
     return _gate_form(form, limit, who)
 
 
+MOE_PLAN_TOKENS = 16        # CHOOSE_TOKENS of moe.hip
+
+
+def _check_moe_plan(scratch: dict, n: int, top: int, experts: int) -> int:
+    """The scratch that holds the plan of ``moe_grouped``; returns how many tiles it has room for."""
+    pairs, max_tiles = n * top, moe_grouped_tiles(n, top, experts)
+    for name, shape in (("where", (pairs,)), ("order", (pairs,)), ("tiles", (3 * max_tiles,)), ("num_tiles", (1,))):
+        _check(scratch[name], name, I32, shape)
+    return max_tiles
+
+
 def moe_topk(logits: torch.Tensor, correction: torch.Tensor | None, chosen: torch.Tensor,
              weights: torch.Tensor, scores: str = "softmax", renormalize: bool = True,
-             bias: torch.Tensor | None = None, scale: float = 1.0) -> None:
+             bias: torch.Tensor | None = None, scale: float = 1.0, plan: tuple | None = None) -> None:
     """The router's choice per token from its fp32 ``logits [N, R]``: ``s = softmax(logits)`` or, with
     ``scores="sigmoid"``, ``s = sigmoid(logits)`` of every output by itself; the ``top`` outputs with
     the largest ``s + correction`` (``None``: ``s`` alone; the lowest index among equals) go to
     ``chosen [N, top]`` (int32) and their ``s``, with ``renormalize`` divided by the sum of the chosen
     ``s`` (+ 1e-20), to ``weights [N, top]`` (fp32).  ``scores="chosen"``: the outputs with the largest
     logits are chosen and weighted by the softmax over the chosen logits alone (no correction).
-    ``bias`` (fp32 ``[R]``) is added to the logits first; the weights are multiplied by ``scale`` last."""
+    ``bias`` (fp32 ``[R]``) is added to the logits first; the weights are multiplied by ``scale`` last.
+    ``plan``: ``(w_gate_up, w_down, experts, ff, scratch)`` as ``moe_grouped`` takes them: for up to
+    ``MOE_PLAN_TOKENS`` tokens the same kernel leaves its plan in ``scratch``, and it is called with ``planned``."""
     if scores not in MOE_SCORES:
         raise KernelError(f"moe_topk: unknown scores {scores!r}; known: {sorted(MOE_SCORES)}")
     n, R = logits.shape
@@ -1906,6 +1920,22 @@ def moe_topk(logits: torch.Tensor, correction: torch.Tensor | None, chosen: torc
     _check(weights, "weights", F32, (n, top))
     if R > MOE_MAX_ROUTER_OUTPUTS or not 0 < top <= min(MOE_MAX_TOP, R):
         raise KernelError(f"moe_topk: up to {MOE_MAX_ROUTER_OUTPUTS} router outputs and {MOE_MAX_TOP} choices, got {R} / {top}")
+    if plan is not None:
+        w_gate_up, w_down, experts, ff, scratch = plan
+        k = w_down.shape[0]
+        if not 0 < n <= MOE_PLAN_TOKENS:
+            raise KernelError(f"moe_topk: a plan is made beside the choices of 1 to {MOE_PLAN_TOKENS} tokens, got {n}")
+        if tuple(w_gate_up.shape) != (experts * 2 * ff, k) or tuple(w_down.shape) != (k, experts * ff):
+            raise KernelError("moe_topk: the plan's weights do not fit its experts")
+        max_tiles = _check_moe_plan(scratch, n, top, experts)
+        f = _fn("moe", "kvf_moe_topk_plan", [c_void_p, c_int] + [c_void_p] * 4 + [c_int] * 5 + [c_float] + [c_int] * 3
+                + [c_void_p] * 4 + [c_int, c_int, c_void_p])
+        _ok(f(logits.data_ptr(), logits.stride(0) if n > 1 else R, bias.data_ptr() if bias is not None else None,
+              correction.data_ptr() if correction is not None else None, chosen.data_ptr(), weights.data_ptr(), n, R,
+              top, MOE_SCORES[scores], 1 if renormalize else 0, float(scale), int(experts), int(ff), k,
+              scratch["where"].data_ptr(), scratch["order"].data_ptr(), scratch["tiles"].data_ptr(),
+              scratch["num_tiles"].data_ptr(), max_tiles, -1, _stream()), "moe_topk_plan")
+        return
     f = _fn("moe", "kvf_moe_topk", [c_void_p, c_int] + [c_void_p] * 4 + [c_int] * 5 + [c_float, c_void_p])
     _ok(f(logits.data_ptr(), logits.stride(0) if n > 1 else R, bias.data_ptr() if bias is not None else None,
           correction.data_ptr() if correction is not None else None, chosen.data_ptr(), weights.data_ptr(), n, R, top,
@@ -1963,7 +1993,8 @@ def moe_grouped_tiles(rows: int, top: int, experts: int) -> int:
 def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedWeight", chosen: torch.Tensor,
                 weights: torch.Tensor, residual: torch.Tensor, experts: int, ff: int,
                 scratch: dict[str, torch.Tensor], weigh_input: bool = False, fresh: bool = False,
-                form: str = "silu", limit: float | None = None, many_rows: bool | None = None) -> None:
+                form: str = "silu", limit: float | None = None, many_rows: bool | None = None,
+                planned: bool = False) -> None:
     """``residual[n] += sum_k weights[n, k] * expert_{chosen[n, k]}(x[n])`` (a choice ``>= experts``
     stands for ``x[n]`` itself) with every expert's products taken over only the rows that chose
     it: the pairs are grouped by expert on the device, tiles of up to 16 or up to 128 rows go through the
@@ -1975,7 +2006,10 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
     weight times the row, ``expert(weights[n, k] * x[n])``, and the outputs are summed as they are.
     ``fresh``: ``residual`` is written instead of added to.  ``form``, ``limit``: how an expert joins its
     pairs (``MOE_FORMS``).  ``many_rows``: for tests, which of the two tile sizes is taken; the sizes
-    decide otherwise (``kvf_moe_grouped_many_rows`` in ``moe.hip``).  The results are the same bits."""
+    decide otherwise (``kvf_moe_grouped_many_rows`` in ``moe.hip``).  The results are the same bits.
+    ``planned``: ``moe_topk(..., plan=...)`` has left the plan in ``scratch``."""
+    if planned and many_rows is not None:
+        raise KernelError("moe_grouped: a plan that is there decides about the tiles")
     code, lim = _moe_form(form, limit, "moe_grouped")
     n, k = x.shape
     top = chosen.shape[1]
@@ -1987,18 +2021,17 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
     _check(chosen, "chosen", I32, (n, top))
     _check(weights, "weights", F32, (n, top))
     _check(residual, "residual", F32, (n, k))
-    pairs, max_tiles = n * top, moe_grouped_tiles(n, top, experts)
-    for name, dtype, shape in (("where", I32, (pairs,)), ("order", I32, (pairs,)), ("tiles", I32, (3 * max_tiles,)),
-                               ("num_tiles", I32, (1,)), ("act", BF16, (pairs, ff)), ("y", BF16, (pairs, k))):
+    pairs, max_tiles = n * top, _check_moe_plan(scratch, n, top, experts)
+    for name, dtype, shape in (("act", BF16, (pairs, ff)), ("y", BF16, (pairs, k))):
         _check(scratch[name], name, dtype, shape)
     f = _fn("moe", "kvf_moe_grouped", [c_void_p, c_int, c_void_p] + [c_int] * 5 + [c_void_p] * 8 + [c_int]
-            + [c_void_p] * 3 + [c_int, c_int, c_int, c_float, c_int, c_void_p])
+            + [c_void_p] * 3 + [c_int, c_int, c_int, c_float, c_int, c_int, c_void_p])
     _ok(f(x.data_ptr(), x.stride(0) if n > 1 else k, x.data_ptr(), n, k, int(experts), int(ff), top,
           w_gate_up.tiles.data_ptr(), w_down.tiles.data_ptr(), chosen.data_ptr(), weights.data_ptr(),
           scratch["where"].data_ptr(), scratch["order"].data_ptr(), scratch["tiles"].data_ptr(),
           scratch["num_tiles"].data_ptr(), max_tiles, scratch["act"].data_ptr(), scratch["y"].data_ptr(),
           residual.data_ptr(), 1 if weigh_input else 0, 1 if fresh else 0, code, lim,
-          -1 if many_rows is None else int(many_rows), _stream()), "moe_grouped")
+          -1 if many_rows is None else int(many_rows), 1 if planned else 0, _stream()), "moe_grouped")
 
 
 

@@ -191,15 +191,8 @@ class RoutedExperts(FeedForward):
         step.settle()
         chosen = ws.buf("moe_chosen", (n, self.top), torch.int32)
         weights = ws.buf("moe_weights", (n, self.top), torch.float32)
-        if self.table is not None:
-            ops.moe_table(step.token_ids, self.table, chosen, weights, self.E)
-        else:
-            logits = ws.buf("moe_logits", (n, self.R_pad), torch.float32)[:, :self.R]
-            ops.gemm(x, self.w_router, ws.buf("moe_logits", (n, self.R_pad), torch.float32))   # 32-bit sums, stored so
-            ops.moe_topk(logits, self.correction, chosen, weights, self.scores, self.renormalize, bias=self.r_bias,
-                         scale=self.out_scale)
-        if ops.moe_grouped_takes(x, self.w_gate_up, self.w_down, self.E, self.ff) and x.is_contiguous():
-            # bf16: every expert over only the rows that chose it, grouped on the device
+        grouped = ops.moe_grouped_takes(x, self.w_gate_up, self.w_down, self.E, self.ff) and x.is_contiguous()
+        if grouped:
             pairs, tiles = n * self.top, ops.moe_grouped_tiles(n, self.top, self.E)
             scratch = {"where": ws.buf("moe_where", (pairs,), torch.int32),
                        "order": ws.buf("moe_order", (pairs,), torch.int32),
@@ -207,11 +200,23 @@ class RoutedExperts(FeedForward):
                        "num_tiles": ws.buf("moe_num_tiles", (1,), torch.int32),
                        "act": ws.buf("moe_act_rows", (pairs, self.ff), dt),
                        "y": ws.buf("moe_y_rows", (pairs, self.hidden), dt)}
+        planned = grouped and self.table is None and n <= ops.MOE_PLAN_TOKENS
+        if self.table is not None:
+            ops.moe_table(step.token_ids, self.table, chosen, weights, self.E)
+        else:
+            logits = ws.buf("moe_logits", (n, self.R_pad), torch.float32)[:, :self.R]
+            ops.gemm(x, self.w_router, ws.buf("moe_logits", (n, self.R_pad), torch.float32))   # 32-bit sums, stored so
+            ops.moe_topk(logits, self.correction, chosen, weights, self.scores, self.renormalize, bias=self.r_bias,
+                         scale=self.out_scale,
+                         plan=(self.w_gate_up, self.w_down, self.E, self.ff, scratch) if planned else None)
+        if grouped:
+            # bf16: every expert over only the rows that chose it, grouped on the device
             fresh = step.fresh is residual
             if fresh:
                 step.fresh = None      # written here instead of added to
             ops.moe_grouped(x, self.w_gate_up, self.w_down, chosen, weights, residual, self.E, self.ff, scratch,
-                            weigh_input=self.weigh_input, fresh=fresh, form=self.form, limit=self.limit)
+                            weigh_input=self.weigh_input, fresh=fresh, form=self.form, limit=self.limit,
+                            planned=planned)
             self._shared_forward(x, step, residual)
             return
         # otherwise (32-bit, or sizes the grouped kernels do not take): every expert over every

@@ -89,6 +89,22 @@ def test_two_norms_of_one_stream_in_one_pass(dtype, h, owed):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("h", [4, 512, 516, 1020, 1024, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("off", [0, 1])
+def test_two_norms_of_one_stream_at_the_edges_of_what_stays_in_registers(dtype, h, off):
+    """Widths at which a row just fits a workgroup's registers or does not, and weights off their 16 bytes."""
+    x, w1, w2 = rand(3, h, seed=h, scale=3.0), rand(h + off, seed=1, scale=0.3)[off:], rand(h + off, seed=2, scale=0.3)[off:]
+    add, dev = rand(3, h, seed=3).to(dtype), x.clone().to(DEV)
+    o1, o2 = torch.empty(3, h, dtype=dtype, device=DEV), torch.empty(3, h, dtype=dtype, device=DEV)
+    d1, d2 = (torch.empty(h + off, device=DEV)[off:].copy_(1.0 + w) for w in (w1, w2))
+    ops().rmsnorm_pair(dev, d1, d2, 1e-5, o1, o2, add=add.to(DEV))
+    total = x + add.float()
+    torch.testing.assert_close(dev.cpu(), total, atol=1e-6, rtol=1e-6)
+    torch.testing.assert_close(o1.float().cpu(), plain.one_plus_norm(total, w1, 1e-5), **tol(dtype))
+    torch.testing.assert_close(o2.float().cpu(), plain.one_plus_norm(total, w2, 1e-5), **tol(dtype))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,KV,dk,d,rot", [(4, 2, 16, 16, 16), (3, 1, 24, 32, 10), (8, 1, 64, 64, 64),
                                            (2, 2, 100, 112, 64), (5, 5, 7, 16, 6), (2, 1, 256, 256, 128)])
 def test_head_norm_rotation_and_cache_write_in_one_kernel(dtype, H, KV, dk, d, rot):
@@ -383,6 +399,38 @@ def test_heads_normed_weighted_and_gated(dtype):
     ops().mlstm_out(raw.to(DEV), wide.to(DEV)[:, H * dv:2 * H * dv], w.to(DEV), eps, out, H, dv)
     want = plain.rms(raw.view(n, H, dv), eps).reshape(n, H * dv) * w * torch.sigmoid(wide[:, H * dv:2 * H * dv].float())
     torch.testing.assert_close(out.float().cpu(), want, **tol(dtype))
+
+
+@pytest.mark.parametrize("n", [1, 7, 16])
+@pytest.mark.parametrize("R,E,top", [(4, 4, 1), (34, 32, 4), (64, 64, 16), (65, 65, 2), (129, 120, 3), (512, 512, 16)])
+@pytest.mark.parametrize("scores", ["softmax", "sigmoid", "chosen"])
+def test_choices_and_their_plan_in_one_kernel(n, R, E, top, scores):
+    """The same choices, weights and results as with the plan in a kernel of its own: ties, infinities and rows of
+    NaN among the router's outputs, outputs that name no expert."""
+    K, ff = 64, 32
+    g = torch.Generator().manual_seed(n + R)
+    z = rand(n, R, seed=R, scale=3.0).to(DEV)
+    z[0] = 1.5                                    # nothing but ties
+    if n > 1:
+        z[1, 2], z[2], z[3, 0] = -math.inf, math.nan, math.inf
+    corr = None if scores == "chosen" else rand(R, seed=1, scale=0.3).to(DEV)
+    up = ops().streamed(torch.randn(E * 2 * ff, K, generator=g).to(torch.bfloat16).to(DEV))
+    down = ops().streamed(torch.randn(K, E * ff, generator=g).to(torch.bfloat16).to(DEV))
+    x = torch.randn(n, K, generator=g).to(torch.bfloat16).to(DEV)
+    tiles, outs = ops().moe_grouped_tiles(n, top, E), []
+    for together in (False, True):
+        scratch = {k: torch.full((m,), -7, dtype=torch.int32, device=DEV)
+                   for k, m in (("where", n * top), ("order", n * top), ("tiles", 3 * tiles), ("num_tiles", 1))}
+        scratch |= {"act": torch.empty(n * top, ff, dtype=torch.bfloat16, device=DEV),
+                    "y": torch.empty(n * top, K, dtype=torch.bfloat16, device=DEV)}
+        chosen, weights = torch.empty(n, top, dtype=torch.int32, device=DEV), torch.empty(n, top, device=DEV)
+        ops().moe_topk(z, corr, chosen, weights, scores, plan=(up, down, E, ff, scratch) if together else None)
+        res = torch.zeros(n, K, device=DEV)
+        ops().moe_grouped(x, up, down, chosen, weights, res, E, ff, scratch, planned=together)
+        outs.append((chosen, weights.view(torch.int32), res.view(torch.int32), scratch["num_tiles"], scratch["tiles"][:3 * int(scratch["num_tiles"])]))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    with pytest.raises(ops().KernelError):
+        ops().moe_topk(z.repeat(17, 1), corr, chosen.repeat(17, 1), weights.repeat(17, 1), scores, plan=(up, down, E, ff, scratch))
 
 
 @pytest.mark.parametrize("T", [1, 5, 40])
