@@ -974,9 +974,10 @@ KVF_EXPORT int kvf_gemm_bf16(const void* A, int a_type, const void* W, int w_til
 // A product of 17 to 64 bf16 rows cut over K, see gemm_mid_kernel.  How many parts M rows over W [N, K]
 // are stored in, or 0 where they had better be one product: wide outputs fill the chip by themselves, and
 // up to 32 rows over a matrix with fewer rows than columns gemm_skinny_kernel is as fast (4,096 x 2,048 at
-// 17 rows: 6.1 us both).
+// 17 rows: 6.1 us both).  A shorter K gains a microsecond a product (1,024 x 2,048 at 33 rows 5.5 and 4.2), which the
+// models that have it do not show: their steps are bound by the host's launches (0.56 and 0.58 ms for 50 tokens).
 KVF_EXPORT int kvf_gemm_bf16_parts_count(int M, int N, int K) {
-  if (M <= 16 || M > 64 || N <= 0 || N % 16 != 0 || N > 4096 || K < 1024 || K % 8 != 0 || (M <= 32 && K < N)) return 0;
+  if (M <= 16 || M > 64 || N <= 0 || N % 16 != 0 || N > 4096 || K < 2048 || K % 8 != 0 || (M <= 32 && K < N)) return 0;
   return mid_cut(M, N, K, true).splits;
 }
 
