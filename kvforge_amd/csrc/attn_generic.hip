@@ -113,8 +113,11 @@ __global__ __launch_bounds__(256) void attn_mfma32_kernel(
   constexpr int KLD = DMAX + 4, VLD = BK + 4;  // LDS rows 16 bytes apart in the banks
   constexpr int NK = BK * DMAX / 8 / 256;      // pieces of 8 elements of a tile's keys that a thread brings in
   constexpr int NV = BK * DMAX / 4 / 256;      // and of four keys of an element of its values
-  __shared__ __align__(16) float Ks[BK * KLD];    // the tile's keys [BK][KLD]
-  __shared__ __align__(16) float Vs[DMAX * VLD];  // and its values [d][VLD]
+  constexpr bool AHEAD = DMAX <= 128, APART = DMAX <= 256;
+  constexpr int K_LDS = BK * KLD, V_LDS = DMAX * VLD;
+  __shared__ __align__(16) float KVs[APART ? K_LDS + V_LDS : K_LDS > V_LDS ? K_LDS : V_LDS];
+  float* Ks = KVs;                           // the tile's keys [BK][KLD]
+  float* Vs = APART ? KVs + K_LDS : KVs;     // its values [d][VLD], apart from the keys or in their place
 
   // Rows (sequence, item, item or -1): a workgroup for each kv head and item.  The kv heads are the fastest index
   // (a head's keys and values stay in one XCD's L2), and all second items, which are often none, come behind all
@@ -191,11 +194,17 @@ __global__ __launch_bounds__(256) void attn_mfma32_kernel(
     }
     tc_first = 0;
   }
-  // A thread's pieces of a tile, the same ones in every tile.  Where the registers suffice (heads of up to 128)
-  // they are asked for while the tile before is worked on, and the pages they lie in a tile earlier still, so that
-  // the walk waits for no memory; heads of up to 256 ask for keys and values together, wider ones for one after the
-  // other.  A piece past the tile or without a page is read from page 0 and counts as zeros.
-  constexpr bool AHEAD = DMAX <= 128, TOGETHER = DMAX <= 256;
+  auto staged = [&](int j) { return (j >= lo || j < keep) && j <= hi; };   // other keys of a tile count as zeros
+  // A thread's pieces of a tile, the same ones in every tile.
+  // Heads of up to 128: they are asked for while the tile before is worked on, and the pages they lie in a tile
+  // earlier still, so that the walk waits for no memory.  A piece past the tile or without a page is read from page 0 and
+  // counts as zeros.  (32 heads of 128 over 8, fp32: 777 queries 115 us and 2,048 580; 154 and 523 with two workgroups a
+  // compute unit, which then wait; 302 and 1,382 when every second workgroup was an empty one.)
+  // Heads of up to 256: keys and values together (16 of 256 over 4: 208 and 574 us; 224 and 609 asked for ahead, 290 and
+  // 820 one after the other).
+  // Wider ones: the queries and the sums take most of the registers, so a piece at a time, and the values take the keys'
+  // place in LDS (16 of 576 over one: 33 queries 37 us, 777 615; with all pieces of a tile in registers, most of them
+  // spilled, 48 and 648).
   int kc[NK], k8[NK];
   bool k_in[NK];
 #pragma unroll
@@ -251,55 +260,73 @@ __global__ __launch_bounds__(256) void attn_mfma32_kernel(
   }
   for (int tc = tc_first; tc <= tc_last; tc += BK) {
     const int t0 = tile_at(tc);
-    if (!AHEAD) {
-      locate(tc);
-      fetch_keys();
-      if (TOGETHER) fetch_values();
-    }
-    __syncthreads();   // the tile before has been used
-#pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      if (!k_in[i]) continue;
-      const int j = t0 + kc[i];
-      const bool ok = k_ok[i] && (j >= lo || j < keep) && j <= hi;
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = ok ? kraw[i].at(e) : 0.f;
-      *reinterpret_cast<float4*>(&Ks[kc[i] * KLD + k8[i]]) = make_float4(v[0], v[1], v[2], v[3]);
-      *reinterpret_cast<float4*>(&Ks[kc[i] * KLD + k8[i] + 4]) = make_float4(v[4], v[5], v[6], v[7]);
-    }
-    if (!TOGETHER) fetch_values();
-    if (quads) {
-      // four neighbouring keys of one element lie side by side in a page
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        if (ve + i * VE >= D) continue;
-        f32x4 v;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int j = t0 + vc + x;
-          v[x] = v_ok && (j >= lo || j < keep) && j <= hi ? vraw[i].at(x) : 0.f;
-        }
-        *reinterpret_cast<f32x4*>(&Vs[(ve + i * VE) * VLD + vc]) = v;
-      }
-    } else {
+    // values whose pages do not hold four neighbouring keys side by side
+    auto put_values_singly = [&]() {
       for (int idx = tid; idx < BK * D; idx += 256) {
         const int e = idx / BK, c = idx - e * BK;
-        const int j = t0 + c;
         float v = 0.f;
-        if ((j >= lo || j < keep) && j <= hi) {
-          const PageAt at = page_at(j);
+        if (staged(t0 + c)) {
+          const PageAt at = page_at(t0 + c);
           if (at.page >= 0 && at.page < a.num_blocks)
             v = Elem<T>::load(v_pages + ((static_cast<size_t>(at.page) * a.KV + kvh) * D + e) * a.block_size + at.slot);
         }
         Vs[e * VLD + c] = v;
       }
-    }
-    __syncthreads();
-    if (AHEAD) {
-      fetch_keys();           // of the next tile
-      fetch_values();
-      locate(tc + 2 * BK);
+    };
+    auto put_key = [&](int c, int e, const float (&v)[8]) {
+      *reinterpret_cast<float4*>(&Ks[c * KLD + e]) = make_float4(v[0], v[1], v[2], v[3]);
+      *reinterpret_cast<float4*>(&Ks[c * KLD + e + 4]) = make_float4(v[4], v[5], v[6], v[7]);
+    };
+    if constexpr (APART) {
+      if (!AHEAD) {
+        locate(tc);
+        fetch_keys();
+        fetch_values();
+      }
+      __syncthreads();   // the tile before has been used
+#pragma unroll
+      for (int i = 0; i < NK; ++i) {
+        if (!k_in[i]) continue;
+        const bool ok = k_ok[i] && staged(t0 + kc[i]);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = ok ? kraw[i].at(e) : 0.f;
+        put_key(kc[i], k8[i], v);
+      }
+      if (quads) {
+        // four neighbouring keys of one element lie side by side in a page
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          if (ve + i * VE >= D) continue;
+          f32x4 v;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) v[x] = v_ok && staged(t0 + vc + x) ? vraw[i].at(x) : 0.f;
+          *reinterpret_cast<f32x4*>(&Vs[(ve + i * VE) * VLD + vc]) = v;
+        }
+      } else {
+        put_values_singly();
+      }
+      __syncthreads();
+      if (AHEAD && tc + BK <= tc_last) {
+        fetch_keys();           // of the next tile
+        fetch_values();
+        locate(tc + 2 * BK);
+      }
+    } else {
+      __syncthreads();   // the values of the tile before have been used
+#pragma unroll 1
+      for (int i = 0; i < NK; ++i) {
+        const int ch = tid + i * 256, c = ch / chunks, e = (ch - c * chunks) * 8;
+        if (c >= BK) break;
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (staged(t0 + c)) {
+          const PageAt at = page_at(t0 + c);
+          if (at.page >= 0 && at.page < a.num_blocks)
+            load8(k_pages + ((static_cast<size_t>(at.page) * a.KV + kvh) * a.block_size + at.slot) * D + e, v);
+        }
+        put_key(c, e, v);
+      }
+      __syncthreads();
     }
     const bool mine = t0 <= hi_w && (t0 + BK > lo_w || t0 < keep);   // the same in all lanes of the wave
     f32x4 p[ST];
@@ -364,6 +391,25 @@ __global__ __launch_bounds__(256) void attn_mfma32_kernel(
       psum += __shfl_xor(psum, 32, KVF_WAVE);
       l_run = l_run * corr + psum;
       m_run = m_new;
+    }
+    if constexpr (!APART) {
+      __syncthreads();   // every wave has finished with the keys
+      if (quads) {
+        const PageAt at = page_at(min(t0 + vc, hi / 4 * 4));
+        const bool ok = at.page >= 0 && at.page < a.num_blocks;
+        const T* v = v_pages + (static_cast<size_t>(ok ? at.page : 0) * a.KV + kvh) * D * a.block_size + at.slot;
+#pragma unroll 1
+        for (int e = ve; e < D; e += VE) {
+          f32x4 w = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (ok) w = load4(v + static_cast<size_t>(e) * a.block_size);
+#pragma unroll
+          for (int x = 0; x < 4; ++x) w[x] = staged(t0 + vc + x) ? w[x] : 0.f;
+          *reinterpret_cast<f32x4*>(&Vs[e * VLD + vc]) = w;
+        }
+      } else {
+        put_values_singly();
+      }
+      __syncthreads();
     }
     if (mine) {
 #pragma unroll

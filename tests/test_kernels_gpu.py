@@ -930,7 +930,7 @@ def test_attn_prefill(dtype, seq_lens, q_lens, H, KV, d, bs, window):
         torch.testing.assert_close(out.float().cpu(), want, **tol(dtype))
 
 
-@pytest.mark.parametrize("d,bs", [(16, 16), (64, 16), (64, 6), (128, 32), (144, 16), (256, 4), (272, 16), (640, 16)])
+@pytest.mark.parametrize("d,bs", [(16, 16), (64, 16), (64, 6), (128, 32), (144, 16), (256, 4), (272, 16), (320, 6), (576, 8), (640, 16)])
 @pytest.mark.parametrize("window", [0, 70, 130])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attn_prefill_of_the_32_bit_kernel_at_the_edges_of_its_tiles(dtype, d, bs, window):
