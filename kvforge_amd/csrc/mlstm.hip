@@ -27,15 +27,10 @@ struct ScanArgs {
 __device__ __forceinline__ float capped(float z, float cap) { return cap * tanhf(z / cap); }
 __device__ __forceinline__ float log_sigmoid(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
 
-// Workgroup (column block, head, sequence) of RG waves; wave w holds rows w*ROWS .. w*ROWS+ROWS-1
-// of the block's 64 columns of S, a lane one column (ROWS registers), and lanes 0..ROWS-1 the
-// wave's rows of n (row lane + 64 j).  A stage of TB tokens (k, q scaled, the block's elements of
-// v, the two log gates) goes through LDS; within a stage nothing waits for memory.  With one
-// wave there is no barrier per token; with several, the waves' shares of o and of n . q are
-// added through LDS in wave order.
 // The workgroups of a head's column blocks all read its n and m and one of them writes both: whichever has read
-// them last, for a workgroup may start when another has finished.  One thread asks, behind a barrier before
-// which every wave has used what it read; `ticket` is zero before and after.
+// them last, for a workgroup may start when another has finished.  One thread asks when all that the workgroup
+// read of them has arrived: behind a barrier before which every wave has used what it read, or a wait of its own for what
+// it uses later; `ticket` is zero before and after.
 __device__ __forceinline__ bool last_reader(int* ticket) {
   if (gridDim.x == 1) return true;
   if (__hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != static_cast<int>(gridDim.x) - 1)
@@ -44,6 +39,12 @@ __device__ __forceinline__ bool last_reader(int* ticket) {
   return true;
 }
 
+// Workgroup (column block, head, sequence) of RG waves; wave w holds rows w*ROWS .. w*ROWS+ROWS-1
+// of the block's 64 columns of S, a lane one column (ROWS registers), and lanes 0..ROWS-1 the
+// wave's rows of n (row lane + 64 j).  A stage of TB tokens (k, q scaled, the block's elements of
+// v, the two log gates) goes through LDS; within a stage nothing waits for memory.  With one
+// wave there is no barrier per token; with several, the waves' shares of o and of n . q are
+// added through LDS in wave order.
 template <typename T, int ROWS>
 __global__ __launch_bounds__(ROWS > KVF_WAVE ? 2 * KVF_WAVE : KVF_WAVE) void mlstm_scan_kernel(const T* __restrict__ qkv, const float* __restrict__ zif,
                                   const float* __restrict__ bias_if, const int* __restrict__ cu_q,
@@ -245,6 +246,9 @@ __global__ __launch_bounds__(4 * KVF_WAVE) void mlstm_token_kernel(const T* __re
   }
   if (wave == 1) {
     float nq = 0.f;
+    // Only this wave uses n, and not before the ticket: its loads have to be back.  (Loads asked for behind them have been
+    // used, so this takes no time: 128 x 256, 8 sequences 9.8 us with and without; n . q ahead of the barrier 10.0.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     int last = lane == 0 ? last_reader(tickets + seq * a.H + head) : 0;
     last = __builtin_amdgcn_readfirstlane(last);
 #pragma unroll

@@ -434,7 +434,7 @@ def test_choices_and_their_plan_in_one_kernel(n, R, E, top, scores):
 
 
 @pytest.mark.parametrize("T", [1, 5, 40])
-@pytest.mark.parametrize("dk,dv,n", [(24, 130, 3), (128, 256, 70), (200, 700, 9)])
+@pytest.mark.parametrize("dk,dv,n", [(24, 130, 3), (128, 256, 70), (128, 960, 41), (200, 700, 9)])
 def test_column_blocks_of_a_head_read_its_sums_before_one_of_them_writes(T, dk, dv, n):
     """The state's key sum and maximum belong to all workgroups of a head, more of them than run at a time: every
     column's output and state in 64 bits from the state as it was, by all three kernels (single tokens, runs
