@@ -867,19 +867,34 @@ def is_library_product(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm(a, w, ...)`` hands the product to the library: bf16 with more rows than the
     weight-streaming kernels take; or more than one tile of rows over a deep and narrow weight
     (K >= 2 N), where those kernels have few workgroups and each re-reads every row of ``a`` along
-    a long K (measured at [2048, 8192] and 32 rows: 19 us against the library's 15).  Over tiled weights
-    that alone bring a workgroup of 64 columns to every compute unit the streaming kernel stays ahead up
-    to 64 rows ([128256, 2048] at 41 rows 110 us against 128, [16384, 2048] 17.4 and 17.9; [12288, 4096]
-    at 48 rows 26.5 and 24.8, [32768, 1024] at 64 rows 18.2 and 16.5)."""
+    a long K (measured at [2048, 8192] and 32 rows: 19 us against the library's 15).  ``accumulate=True``
+    hands it the products of ``streams_in_place_of_library`` as well."""
     m, k = a.shape
     n = w.shape[0]
     lda = a.stride(0) if m > 1 else k
     if not (a.dtype == BF16 and w.dtype == BF16 and _rows_aligned(a, k, lda)):
         return False
     if m > SKINNY_MAX_M:
-        return not (m <= MID_MAX_M and k >= 2048 and isinstance(w, StreamedWeight)
-                    and n >= 64 * compute_units(a.device))
+        return not streams_in_place_of_library(a, w)
     return m > 16 and k >= 2 * n
+
+
+def streams_in_place_of_library(a: torch.Tensor, w) -> bool:
+    """Whether a product of more than ``SKINNY_MAX_M`` rows that is stored (not added) stays with the
+    weight-streaming kernels all the same: tiled weights that alone bring a workgroup of 64 columns to every
+    compute unit, and a K that the library does badly: 2,048, up to 56 rows (more over 256 columns a unit and
+    up), or one that its k-tiles of 64 do not divide.  Weights from memory, the library against this at 33 / 48 /
+    64 rows: [128256, 2048] 118 / 122 / 119 and 106 / 112 / 117 us, [65536, 2048] 69 / 70 / 68 and 56 / 57 / 60,
+    [24576, 2048] 26.7 / 26.8 / 26.7 and 25.8 / 26.3 / 28.1; [24576, 2056] 34 / 35 / 33 and 27 / 29 / 31, [128256,
+    2056] 153 / 157 / 136 and 106 / 109 / 126.  Other K: [128256, 2112] 103 / 106 / 109 and 105 / 110 / 119, [24576,
+    2304] 26.0 / 26.3 / 25.9 and 28.3 / 29.5 / 31.9, [24576, 4096] 44 / 45 / 44 and 46 / 48 / 52, [32768, 1024] at 64
+    rows 16.5 and 18.2.  With ``accumulate`` gemm_skinny_kernel would take it, slower throughout ([16384, 2048] 19
+    against 24)."""
+    m, k = a.shape
+    if not (SKINNY_MAX_M < m <= MID_MAX_M and k >= 2048 and (k < 2112 or k % 64) and isinstance(w, StreamedWeight)):
+        return False
+    columns = w.shape[0] // compute_units(a.device)
+    return columns >= (64 if m <= 56 or k % 64 else 256)
 
 
 @lru_cache(maxsize=None)
@@ -999,7 +1014,7 @@ def gemm(a: torch.Tensor, w, out: torch.Tensor, accumulate: bool = False,
     if not accumulate:
         _tcode(out.dtype)
     if a.dtype == BF16 and w.dtype == BF16 and _rows_aligned(a, k, lda):
-        if not is_library_product(a, w):
+        if not is_library_product(a, w) and not (accumulate and streams_in_place_of_library(a, w)):
             f = _fn("gemm_bf16", "kvf_gemm_bf16", _GEMM_BF16_ARGS)
             wp, tiled = _w_args(w)
             _ok(f(a.data_ptr(), 0, wp, tiled, out.data_ptr(), out_kind, m, n, k, lda, ldc, 0.0,

@@ -10,7 +10,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 
-from kvforge_amd.kernels import library
+from kvforge_amd.kernels import library, ops
 from kvforge_amd.parts import attention
 
 
@@ -54,3 +54,28 @@ def test_items_of_wide_heads_go_in_pairs_where_they_are_more_than_the_compute_un
     assert per_item == 64 and bool((work[:, 2] >= 0).any()) == pairs
     items = sorted((b, i) for b, *both in work.tolist() for i in both if i >= 0)
     assert items == [(b, i) for b in seqs for i in range(-(-q_lens[b] * (H // KV) // 64))]
+
+
+@pytest.mark.parametrize("m,n,k,own", [
+    (33, 16384, 2048, True), (56, 24576, 2048, True), (57, 24576, 2048, False), (64, 65536, 2048, True), (64, 128256, 2048, True),
+    (33, 16368, 2048, False), (65, 128256, 2048, False), (33, 32768, 1024, False), (33, 24576, 2304, False),
+    (48, 128256, 2112, False), (33, 16384, 4096, False), (64, 24576, 2056, True), (64, 128256, 4104, True)])
+def test_products_that_stream_in_place_of_the_library(monkeypatch, m, n, k, own):
+    """33 to 64 rows over tiled weights, either side of every line of the rule; over plain weights, and where the product
+    is added to what is there, the library takes them all."""
+    monkeypatch.setattr(ops, "compute_units", lambda device: 256)
+    w = object.__new__(ops.StreamedWeight)
+    w.shape, w.dtype, w.plain = (n, k), torch.bfloat16, SimpleNamespace(shape=(n, k), dtype=torch.bfloat16)
+    a = torch.empty(m, k, dtype=torch.bfloat16)
+    assert ops.streams_in_place_of_library(a, w) == own and ops.is_library_product(a, w) == (not own)
+    assert ops.is_library_product(a, w.plain)
+    routes = []
+    monkeypatch.setattr(ops, "_gemm_operands", lambda a, w, out, n_out: (m, n, k, k, n))
+    monkeypatch.setattr(ops, "_w_args", lambda w: (0, 1))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_fn", lambda module, name, types: lambda *args: routes.append(module) or 0)
+    monkeypatch.setattr(ops, "_library_product", lambda *args: routes.append("library"))
+    out = SimpleNamespace(dtype=torch.float32, data_ptr=lambda: 0)
+    ops.gemm(a, w, out)
+    ops.gemm(a, w, out, accumulate=True)
+    assert routes == ["gemm_bf16" if own else "library", "library"]

@@ -233,6 +233,9 @@ def test_gemm_bf16_rows_through_lds_in_place_of_the_library(m):
     out = torch.empty(m, n, device=DEV)
     ops().gemm(a, w, out)
     torch.testing.assert_close(out.double(), a.double() @ w.plain.double().T, atol=1e-4, rtol=1e-4)
+    # added to what is there the library takes it, whose product is rounded to bf16 ahead of the sum
+    ops().gemm(a, w, out, accumulate=True)
+    torch.testing.assert_close(out.double(), 2.0 * (a.double() @ w.plain.double().T), atol=2e-2, rtol=2e-2)
 
 
 @pytest.mark.parametrize("m", [17, 32, 33, 48, 64])
