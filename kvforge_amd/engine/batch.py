@@ -207,6 +207,9 @@ class Step:
         # nothing yet: the sublayer's last product is written there instead of added
         # (``parts.base.add_product``), which then forgets the mark.
         self.fresh: torch.Tensor | None = None
+        # Whether the sublayer that runs adds to a stream whose next reader does not take a product in
+        # parts (``take_owed``), so that an add kernel of its own has to follow one.
+        self.settled_next = False
         # the staging memory this step was filled from (``fill_step``), for ``upload_ints``
         self._meta: "MetaBuffers | None" = None
         self._turn = 0

@@ -321,7 +321,11 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
     instead of an add kernel of its own.  One tile of rows over a deep weight with few columns
     is cut into two halves of K so that every compute unit pulls on the weight: the first half
     is added here, the second is left owed (rounded to bf16, as a stored product is).  17 to 64 rows
-    over such a weight are cut further, and all parts are left owed in fp32 (``ops.gemm_parts``).
+    over such a weight are cut further, and all parts are left owed in fp32 (``ops.gemm_parts``); but
+    not fewer than 24 over a matrix with K < 2 N where the next reader takes no parts (``Step.settled_next``):
+    there the kernel that adds in its epilogue is faster than parts and an add kernel (17 rows, weights from
+    memory, with the norm behind: [2048, 2048] 10.2 against 11.0 us, [3072, 3072] 13.2 and 14.9; 24 rows 10.8 and
+    11.0, 13.9 and 13.5; with a norm that takes the parts 8.2 and 11.9 at 17 rows).
     ``owed``: a sum the caller took from the step (``step.take_owed``) and has not added yet;
     it is added here, in the same kernel where that is possible.
     A ``residual`` that the step holds as *fresh* (``step.fresh``: a sublayer's own output rows,
@@ -336,7 +340,9 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
             ops.add_rows(residual, owed)
         return
     count = 0
-    if 16 < a.shape[0] <= ops.MID_MAX_M and residual.is_contiguous() and residual.data_ptr() % 16 == 0:
+    rows = a.shape[0]
+    if (16 < rows <= ops.MID_MAX_M and residual.is_contiguous() and residual.data_ptr() % 16 == 0
+            and not (rows < 24 and getattr(step, "settled_next", False) and w.shape[1] < 2 * w.shape[0])):
         count = ops.parts_count(a, w)
     if count:
         if owed is not None:

@@ -135,12 +135,13 @@ class ParallelBlock(Block):
     def forward(self, residual, step, layer: LayerState) -> None:
         shape = tuple(residual.shape)
         h = step.ws.buf("parallel_normed", shape, step.act_dtype)
+        pair = self.mu is None and self._norms_pair()
         if self.mu is not None:
             step.settle()
             hs = step.ws.buf("parallel_shifted", shape, step.act_dtype)
             ops.norm_shift(residual, self.norm.weight, self.mu, layer.state, step.slot_ids,
                            step.seq_of_token, step.cu_q, step.positions, self.norm.eps, h, hs)
-        elif self._norms_pair():
+        elif pair:
             # two RMS norms of the same stream: one pass over it, two weights
             hs = h
             h = step.ws.buf("parallel_normed_ffn", shape, step.act_dtype)
@@ -149,11 +150,16 @@ class ParallelBlock(Block):
         else:
             norm_rows(self.norm, residual, h, step)
             hs = h
-        if self.ffn_norm is not None and not (self.mu is None and self._norms_pair()):
+        if self.ffn_norm is not None and not pair:
             # of the same stream as the mixer's norm: taken before the mixer adds to it
             h = step.ws.buf("parallel_normed_ffn", shape, step.act_dtype)
             self.ffn_norm.forward(residual, h)
+        # who reads the stream next: the feed-forward settles what the mixer owes; what is owed behind both goes to
+        # `after` or to the next block's norms, of which only a single one takes parts
+        behind = pair or self.mu is not None or self.after is not None
+        step.settled_next = self.ffn is not None or behind
         self.mixer.forward(hs, step, layer, residual)
+        step.settled_next = behind
         bias = None
         if self.ffn is not None:
             if not self.ffn.settles_residual:
@@ -161,6 +167,7 @@ class ParallelBlock(Block):
             self.ffn.forward(h, step, residual)
             if getattr(self.ffn, "defer_down_bias", False):
                 bias = self.ffn.down_bias
+        step.settled_next = False
         if self.after is not None:
             self.after.forward(residual, step, bias=bias)
 

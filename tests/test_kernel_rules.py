@@ -1,6 +1,6 @@
 """What the compiled modules say of themselves without a GPU, and what is planned from it: where the matrix-core
-attention kernels read a key's row, how items of wide heads are put together, and which kernels the routed experts'
-sizes choose."""
+attention kernels read a key's row, how items of wide heads are put together, which kernels the routed experts'
+sizes choose, and which route products of some rows take."""
 
 from __future__ import annotations
 
@@ -10,8 +10,10 @@ from types import SimpleNamespace
 import pytest
 import torch
 
+from kvforge_amd.engine.batch import Step, Workspace
 from kvforge_amd.kernels import library, ops
-from kvforge_amd.parts import attention
+from kvforge_amd.parts import attention, block
+from kvforge_amd.parts.base import add_product
 
 
 @pytest.mark.parametrize("d", range(16, 257, 16))
@@ -79,3 +81,43 @@ def test_products_that_stream_in_place_of_the_library(monkeypatch, m, n, k, own)
     ops.gemm(a, w, out)
     ops.gemm(a, w, out, accumulate=True)
     assert routes == ["gemm_bf16" if own else "library", "library"]
+
+
+@pytest.mark.parametrize("rows,n,k,settled,route", [
+    (17, 2048, 2048, True, "added"), (23, 3072, 3072, True, "added"), (24, 3072, 3072, True, "parts"),
+    (17, 2048, 2048, False, "parts"), (17, 2048, 4096, True, "parts"), (33, 2048, 2048, True, "parts"),
+    (16, 2048, 2048, False, "added"), (65, 2048, 2048, False, "owed")])
+def test_products_go_in_parts_where_what_reads_them_next_pays_for_it(monkeypatch, rows, n, k, settled, route):
+    """Parts that the next reader cannot take cost an add kernel: few rows are then added by the product's own kernel."""
+    took = []
+    monkeypatch.setattr(ops, "parts_count", lambda a, w: 4 if 16 < a.shape[0] <= 64 else 0)
+    monkeypatch.setattr(ops, "gemm_parts", lambda a, w, parts: took.append("parts"))
+    monkeypatch.setattr(ops, "k_halves_pay", lambda a, w: False)
+    monkeypatch.setattr(ops, "gemm", lambda a, w, out, accumulate=False, owed=None: took.append("added" if accumulate else "owed"))
+    step = Step()
+    step.ws, step.settled_next = Workspace("cpu"), settled
+    monkeypatch.setattr(step, "owe", lambda stream, product: None)
+    add_product(step, torch.empty(rows, k, dtype=torch.bfloat16), torch.empty(n, k, dtype=torch.bfloat16), torch.empty(rows, n))
+    assert took == [route]
+
+
+@pytest.mark.parametrize("feed_forward,pair,after,wanted", [
+    (True, True, False, [True, True]), (True, False, False, [True, False]), (True, False, True, [True, True]),
+    (False, False, False, [False]), (False, False, True, [True])])
+def test_a_parallel_block_says_who_settles_what_its_sublayers_owe(monkeypatch, feed_forward, pair, after, wanted):
+    said = []
+    sub = SimpleNamespace(settles_residual=False, state_spec=None, forward=lambda *args: said.append(args[1].settled_next))
+    ffn = SimpleNamespace(settles_residual=False, forward=lambda x, step, residual: said.append(step.settled_next))
+    norm = SimpleNamespace(adds_bias=False, takes_parts=True, forward=lambda *args, **kw: None)
+    then = SimpleNamespace(forward=lambda residual, step, bias=None: said.append(("after", step.settled_next)))
+    part = block.ParallelBlock(norm, sub, ffn if feed_forward else None, 8, after=then if after else None,
+                               ffn_norm=norm if pair else None)
+    monkeypatch.setattr(part, "_norms_pair", lambda: pair)
+    monkeypatch.setattr(ops, "rmsnorm_pair", lambda *args, **kw: None)
+    part.norm = part.ffn_norm = SimpleNamespace(weight=None, eps=0.0, adds_bias=False, takes_parts=True, forward=norm.forward)
+    if not pair:
+        part.ffn_norm = None
+    step = Step()
+    step.ws = Workspace("cpu")
+    part.forward(torch.zeros(3, 8), step, None)
+    assert said == wanted + ([("after", False)] if after else []) and not step.settled_next
