@@ -28,6 +28,8 @@
 // divided.  A level of the tree is one 16 x 16 product per block of 16 tokens, of which the level's own
 // pairs are kept; blocks of 16 against each other take the blocks' products up to t and behind r, and
 // those of the blocks between.
+#include <type_traits>
+
 #include "memory_chunks.h"
 
 namespace {
@@ -161,7 +163,10 @@ __global__ __launch_bounds__(256) void chdelta_scan_kernel(const float* __restri
 // A thread per (key channel, block of 16 tokens): it keeps the channel's q, k, decays and products over the
 // block in registers, and puts the level's scaled rows down in LDS for all waves.
 // chunks: rows (sequence, first token, tokens, 0).  T, A [chunks, H, CL, CL] (blocks above the diagonal are not
-// written), E [chunks, H, dk] = P(0, L), Kd, Qd [tokens, H, dk], Kw [chunks, H, dk, CL].
+// written), E [chunks, H, dkp] = P(0, L), Kd, Qd [tokens, H, dkp], Kw [chunks, H, dkp, CL]; dkp is dk rounded up to
+// PAD channels, those past dk hold zeros.
+constexpr int PAD = 32;
+__host__ __device__ __forceinline__ int padded(int dk) { return (dk + PAD - 1) / PAD * PAD; }
 template <int DKP, int CL> constexpr int solve_threads() { return DKP * (CL / 16); }
 template <int DKP, int CL> constexpr size_t solve_lds() {
   return 4 * (3 * CL * (DKP + 4) + 2 * CL * (CL + 4) + (CL / 16) * DKP + CL);
@@ -209,7 +214,7 @@ __global__ __launch_bounds__(DKP * (CL / 16)) void chdelta_solve_kernel(
       const bool in = 16 * sub + j < cnt;
       q[j] = in && ch_ok ? q[j] : 0.f;
       k[j] = in && ch_ok ? k[j] : 0.f;
-      pre[j] = in ? decay_of(pre[j] + db, na) : 1.f;
+      pre[j] = in && ch_ok ? decay_of(pre[j] + db, na) : 1.f;
       suf[j] = 1.f;
     }
   }
@@ -305,15 +310,16 @@ __global__ __launch_bounds__(DKP * (CL / 16)) void chdelta_solve_kernel(
       else Ls[t * TLD + r] = sw[t] * acc[v];
     }
   }
-  if (ch_ok) {
+  const int dkp = DKP <= 2 * PAD ? DKP : padded(dk);
+  if (ch < dkp) {
     float before = 1.f, behind = 1.f;
 #pragma unroll
     for (int m = 0; m < RT; ++m) {
       before *= m < sub ? tot[m * DKP + ch] : 1.f;
       behind *= m > sub ? tot[m * DKP + ch] : 1.f;
     }
-    const size_t step = static_cast<size_t>(a.H) * dk;
-    size_t o = static_cast<size_t>(tb + 16 * sub) * step + head * dk + ch;
+    const size_t step = static_cast<size_t>(a.H) * dkp;
+    size_t o = static_cast<size_t>(tb + 16 * sub) * step + head * dkp + ch;
 #pragma unroll
     for (int j = 0; j < 16; ++j, o += step) {
       if (16 * sub + j >= cnt) continue;
@@ -321,7 +327,7 @@ __global__ __launch_bounds__(DKP * (CL / 16)) void chdelta_solve_kernel(
       Kd[o] = k[j] * x;
       Qd[o] = q[j] * x;
     }
-    f32x4* kw = reinterpret_cast<f32x4*>(Kw + ((static_cast<size_t>(chunk) * a.H + head) * dk + ch) * CL + 16 * sub);
+    f32x4* kw = reinterpret_cast<f32x4*>(Kw + ((static_cast<size_t>(chunk) * a.H + head) * dkp + ch) * CL + 16 * sub);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {   // zeros past the chunk's tokens, whose k are
       f32x4 v;
@@ -329,7 +335,7 @@ __global__ __launch_bounds__(DKP * (CL / 16)) void chdelta_solve_kernel(
       for (int y = 0; y < 4; ++y) v[y] = k[4 * j + y] * (suf[4 * j + y] * behind);
       kw[j] = v;
     }
-    if (sub == 0) E[(static_cast<size_t>(chunk) * a.H + head) * dk + ch] = pre[15] * behind;
+    if (sub == 0) E[(static_cast<size_t>(chunk) * a.H + head) * dkp + ch] = ch_ok ? pre[15] * behind : 0.f;
   }
   __syncthreads();
   // the diagonal blocks' inverses: lane c column c (forward substitution)
@@ -381,16 +387,19 @@ __global__ __launch_bounds__(DKP * (CL / 16)) void chdelta_solve_kernel(
 // chunks' u.
 //
 // What bounds it: a chunk waits for the state of the one before, and a chunk is three products one after the other, each
-// a chain of up to 32 matrix instructions.  So nothing else may stand in the chain: a wave's left operands (16 rows of Kd
+// a chain of up to 32 matrix instructions (64 for 256 channels).  So nothing else may stand in the chain: a wave's left operands (16 rows of Kd
 // and T, the rows of Kw that belong to its part of the state, which chdelta_solve leaves turned round) go from memory
 // into registers as they are, those of the chunk after the next asked for as soon as a chunk's have been used; a wave's part of
 // the state stays in registers; LDS carries only what the waves exchange, S, R and U, one barrier each.  2,047 tokens, 16
 // heads of 128 x 128: 91 us (142 with Kd, Kw and T staged in LDS for all waves, five barriers a chunk); 66 of them are the chain,
 // the rest what 80 KB a chunk cost a compute unit.  (Pulling the operands into L2 five chunks ahead changed nothing.)
+// Heads of any size have whole operands, DKP channels of them (see PAD), so that only a run's last chunk has something to leave
+// out: 4 heads of 192 x 192 over 2,047 tokens 267 us with the passes before and behind, of 250 x 256 332; read and cleared element
+// by element where the head ends 400 and 765, staged in LDS 335 and 538.  (Sixteen runs of 40 tokens, 256 x 256: 97 us, in LDS 91:
+// so many registers leave a compute unit one workgroup.)
 constexpr int DCOLS = 16;
-// VEC: as load_four has it.  WHOLE: heads of DKP channels and value columns in whole sixteens, so that only a run's last
-// chunk has anything to leave out.
-template <int DKP, int CL, bool VEC, bool WHOLE>
+// WHOLE: heads of DKP channels and value columns in whole sixteens.
+template <int DKP, int CL, bool WHOLE>
 __global__ __launch_bounds__(256) void chdelta_delta_kernel(
     const float* __restrict__ rows, const int* __restrict__ chunks, const int* __restrict__ runs,
     const int* __restrict__ positions, const int* __restrict__ slot_ids, float* __restrict__ state,
@@ -403,7 +412,7 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
   const int tid = threadIdx.x, lane = tid % KVF_WAVE, l16 = lane % 16, lq = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / KVF_WAVE);
   const int dk = WHOLE ? DKP : a.dk, dv = a.dv, c = col0 + l16;
-  const bool c_ok = WHOLE || c < dv;
+  const bool c_ok = WHOLE || c < dv, columns = WHOLE || col0 + DCOLS <= dv;
   int slot = slot_ids[seq];
   if (slot < 0 || slot >= a.n_slots) slot = -1;
   float* S_slot = slot >= 0 ? state + static_cast<size_t>(slot) * a.slot_stride + static_cast<size_t>(head) * dk * dv
@@ -425,7 +434,7 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
     if (wave + 4 * x < KT) *reinterpret_cast<f32x4*>(St + l16 * QLD + row_of(x)) = S[x];
   }
 
-  // A chunk's operands; what lies past the chunk or the head is read inside and cleared where it is used.  The chunk's
+  // A chunk's operands; rows past the chunk are read inside and cleared where they are used.  The chunk's
   // part of an address is the same for all lanes, a lane's part fits 32 bits.
   struct Operands {
     f32x4 kd[KT], tr[RT], kw[MINE][RT], el[MINE];
@@ -442,9 +451,9 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
   auto ask_kd = [&](Operands& o) {
     o.tb = tb_next;
     o.cnt = cnt_next;
-    const float* p = Kd + (static_cast<size_t>(o.tb) * a.H + head) * dk + static_cast<uint32_t>(min(16 * rw + l16, o.cnt - 1) * a.H * dk);
+    const float* p = Kd + (static_cast<size_t>(o.tb) * a.H + head) * DKP + static_cast<uint32_t>(min(16 * rw + l16, o.cnt - 1) * a.H * DKP);
 #pragma unroll
-    for (int u = 0; u < KT; ++u) o.kd[u] = WHOLE ? *reinterpret_cast<const f32x4*>(p + 16 * u + 4 * lq) : load_four<VEC>(p, p, 16 * u + 4 * lq, dk, true);
+    for (int u = 0; u < KT; ++u) o.kd[u] = *reinterpret_cast<const f32x4*>(p + 16 * u + 4 * lq);
   };
   auto ask_v = [&](Operands& o) {
     const float* p = rows + static_cast<size_t>(o.tb) * a.ld + a.v_off + head * dv;
@@ -457,19 +466,14 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
     for (int k = 0; k < RT; ++k) o.tr[k] = *reinterpret_cast<const f32x4*>(p + 16 * min(k, rw) + static_cast<uint32_t>((16 * rw + l16) * CL + 4 * lq));
   };
   auto ask_kw = [&](Operands& o, int ch) {
-    const float* p = Kw + (static_cast<size_t>(ch) * a.H + head) * dk * CL;
-    const float* pe = E + (static_cast<size_t>(ch) * a.H + head) * dk;
+    const float* p = Kw + (static_cast<size_t>(ch) * a.H + head) * DKP * CL;
+    const float* pe = E + (static_cast<size_t>(ch) * a.H + head) * DKP;
 #pragma unroll
     for (int x = 0; x < MINE; ++x) {
-      const uint32_t at = min(16 * (wave + 4 * x) + l16, dk - 1) * CL + 4 * lq;
+      const uint32_t at = min(16 * (wave + 4 * x) + l16, DKP - 1) * CL + 4 * lq;   // (past the tiles the last row, not used)
 #pragma unroll
       for (int k = 0; k < RT; ++k) o.kw[x][k] = *reinterpret_cast<const f32x4*>(p + 16 * k + at);
-      if (VEC) {
-        o.el[x] = *reinterpret_cast<const f32x4*>(pe + static_cast<uint32_t>(min(row_of(x), dk - 4)));
-      } else {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) o.el[x][v] = pe[min(row_of(x) + v, dk - 1)];
-      }
+      o.el[x] = *reinterpret_cast<const f32x4*>(pe + static_cast<uint32_t>(min(row_of(x), DKP - 4)));
     }
   };
   Operands even, odd;
@@ -490,9 +494,10 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
     f32x4 v4;
 #pragma unroll
     for (int v = 0; v < 4; ++v) v4[v] = t0 + v < cnt && c_ok ? o.vv[v] : 0.f;
-    if (!WHOLE || cnt < CL) {
+    if (cnt < CL) {
+      const bool in = 16 * rw + l16 < cnt;
 #pragma unroll
-      for (int u = 0; u < KT; ++u) o.kd[u] = clear_past(o.kd[u], 16 * u + 4 * lq, dk, 16 * rw + l16 < cnt);
+      for (int u = 0; u < KT; ++u) o.kd[u] = in ? o.kd[u] : zero4();
     }
     {
       f32x4 s4[KT], acc = zero4();
@@ -533,10 +538,6 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int x = 0; x < MINE; ++x) {
-      if (!WHOLE && 16 * (wave + 4 * x) + l16 >= dk) {
-#pragma unroll
-        for (int k = 0; k < RT; ++k) o.kw[x][k] = zero4();
-      }
       old[x] = S[x];
       S[x] = S[x] * o.el[x];
     }
@@ -550,7 +551,7 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
       float* Wg = W + (static_cast<size_t>(ch) * a.H + head) * dk * dv;
       float* Ug = U + (static_cast<size_t>(tb) * a.H + head) * dv;
       if (has_rows) {
-        if (WHOLE && cnt == CL) {
+        if (columns && cnt == CL) {
 #pragma unroll
           for (int v = 0; v < 4; ++v) Ug[static_cast<uint32_t>((t0 + v) * a.H * dv + c)] = u4[v];
         } else {
@@ -562,9 +563,14 @@ __global__ __launch_bounds__(256) void chdelta_delta_kernel(
 #pragma unroll
       for (int x = 0; x < MINE; ++x) {
         if (wave + 4 * x >= KT) break;
+        if (columns && 16 * (wave + 4 * x) + 16 <= dk) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-          if (WHOLE || (row_of(x) + v < dk && c_ok)) Wg[static_cast<uint32_t>((row_of(x) + v) * dv + c)] = old[x][v];
+          for (int v = 0; v < 4; ++v) Wg[static_cast<uint32_t>((row_of(x) + v) * dv + c)] = old[x][v];
+        } else {
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            if (row_of(x) + v < dk && c_ok) Wg[static_cast<uint32_t>((row_of(x) + v) * dv + c)] = old[x][v];
+        }
       }
     }
 #pragma unroll
@@ -598,7 +604,7 @@ constexpr int VCOLS = 64;
 template <int DKP, int CL> constexpr size_t read_lds() {
   return 4 * (VCOLS * (DKP + 4) + CL * (CL + 4) + VCOLS * (CL + 4));
 }
-template <int DKP, int CL, bool VEC>
+template <int DKP, int CL>
 __global__ __launch_bounds__(512, DKP <= 128 ? 4 : 2) void chdelta_read_kernel(
     const int* __restrict__ chunks, const float* __restrict__ Qd, const float* __restrict__ A,
     const float* __restrict__ W, const float* __restrict__ U, float* __restrict__ out, ChArgs a) {
@@ -610,7 +616,7 @@ __global__ __launch_bounds__(512, DKP <= 128 ? 4 : 2) void chdelta_read_kernel(
   const int chunk = blockIdx.z, head = blockIdx.x, col0 = blockIdx.y * VCOLS;
   const int tb = chunks[4 * chunk + 1], cnt = chunks[4 * chunk + 2];
   const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE, l16 = lane % 16, lq = lane / 16;
-  const int dk = a.dk, dv = a.dv, rt = wave % RT, share = wave / RT;
+  const int dk = a.dk, dkp = DKP <= 2 * PAD ? DKP : padded(dk), dv = a.dv, rt = wave % RT, share = wave / RT;
   StagedTurned<CL, VCOLS, 512, TLD> us;
   StagedTurned<DKP, VCOLS, 512, QLD> ws;
   us.ask(U + (static_cast<size_t>(tb) * a.H + head) * dv + col0, static_cast<size_t>(a.H) * dv, cnt, dv - col0);
@@ -625,9 +631,9 @@ __global__ __launch_bounds__(512, DKP <= 128 ? 4 : 2) void chdelta_read_kernel(
   f32x4 q4[DKP / 16];
   const bool q_ok = 16 * rt + l16 < cnt;
   {
-    const float* p = Qd + (static_cast<size_t>(tb + 16 * rt + l16) * a.H + head) * dk;
+    const float* p = Qd + (static_cast<size_t>(tb + 16 * rt + l16) * a.H + head) * dkp;
 #pragma unroll
-    for (int u = 0; u < DKP / 16; ++u) q4[u] = load_four<VEC>(Qd, p, 16 * u + 4 * lq, dk, q_ok);
+    for (int u = 0; u < DKP / 16; ++u) q4[u] = load_four<true>(Qd, p, 16 * u + 4 * lq, dkp, q_ok);
   }
   us.put(Ut, cnt, dv - col0);
   ws.put(Sc, dk, dv - col0);
@@ -637,7 +643,7 @@ __global__ __launch_bounds__(512, DKP <= 128 ? 4 : 2) void chdelta_read_kernel(
     if (i < CL * CL) *reinterpret_cast<f32x4*>(As + (i / CL) * TLD + i % CL) = areg[x];
   }
 #pragma unroll
-  for (int u = 0; u < DKP / 16; ++u) q4[u] = clear_past(q4[u], 16 * u + 4 * lq, dk, q_ok);
+  for (int u = 0; u < DKP / 16; ++u) q4[u] = clear_past(q4[u], 16 * u + 4 * lq, dkp, q_ok);
   __syncthreads();
   const int col_tiles = min(VCOLS / 16, (dv - col0 + 15) / 16), t4 = 16 * rt + 4 * lq;
   for (int ct = share; ct < col_tiles; ct += SHARES) {
@@ -664,12 +670,12 @@ struct ChunkPtrs {
   int n_chunks, n_runs;
 };
 
-template <int DKP, int CL, bool VEC> int chunks_go(const ChunkPtrs& p, ChArgs a, hipStream_t s) {
+template <int DKP, int CL> int chunks_go(const ChunkPtrs& p, ChArgs a, hipStream_t s) {
   static bool allowed = false;
   constexpr size_t lds_solve = solve_lds<DKP, CL>(), lds_read = read_lds<DKP, CL>();
   if (!allowed) {
     hipError_t e = allow_lds(&chdelta_solve_kernel<DKP, CL>, lds_solve);
-    if (e == hipSuccess) e = allow_lds(&chdelta_read_kernel<DKP, CL, VEC>, lds_read);
+    if (e == hipSuccess) e = allow_lds(&chdelta_read_kernel<DKP, CL>, lds_read);
     if (e != hipSuccess) return static_cast<int>(e);
     allowed = true;
   }
@@ -679,9 +685,20 @@ template <int DKP, int CL, bool VEC> int chunks_go(const ChunkPtrs& p, ChArgs a,
     hipLaunchKernelGGL(kernel, dim3(a.H, (a.dv + DCOLS - 1) / DCOLS, p.n_runs), dim3(256), 0, s, p.rows, p.chunks, p.runs,
                        p.positions, p.slot_ids, p.state, p.T, p.E, p.Kd, p.Kw, p.W, p.U, a);
   };
-  if (VEC && a.dk == DKP && a.dv % DCOLS == 0) delta(&chdelta_delta_kernel<DKP, CL, true, true>);
-  else delta(&chdelta_delta_kernel<DKP, CL, VEC, false>);
-  hipLaunchKernelGGL((chdelta_read_kernel<DKP, CL, VEC>), dim3(a.H, (a.dv + VCOLS - 1) / VCOLS, p.n_chunks), dim3(512),
+  auto fit = [&](auto channels) {
+    constexpr int N = decltype(channels)::value;
+    if (padded(a.dk) != N) return;
+    if (a.dk == N && a.dv % DCOLS == 0) delta(&chdelta_delta_kernel<N, CL, true>);
+    else delta(&chdelta_delta_kernel<N, CL, false>);
+  };
+  fit(std::integral_constant<int, DKP>{});   // dk is above DKP / 2
+  if constexpr (DKP == 128) fit(std::integral_constant<int, 96>{});
+  if constexpr (DKP == 256) {
+    fit(std::integral_constant<int, 160>{});
+    fit(std::integral_constant<int, 192>{});
+    fit(std::integral_constant<int, 224>{});
+  }
+  hipLaunchKernelGGL((chdelta_read_kernel<DKP, CL>), dim3(a.H, (a.dv + VCOLS - 1) / VCOLS, p.n_chunks), dim3(512),
                      lds_read, s, p.chunks, p.Qd, p.A, p.W, p.U, p.out, a);
   return kvf_last_error();
 }
@@ -721,8 +738,9 @@ KVF_EXPORT int kvf_chdelta_chunk_len(int dk) { return dk <= 128 ? 64 : 32; }
 
 // The runs named in `runs` (sequence, first chunk, chunks), cut into `chunks` (sequence, first token, tokens, 0; at
 // most kvf_chdelta_chunk_len(dk) tokens each, a run's chunks in order and one after another).  Scratch: T, A
-// [n_chunks, H, CL, CL], E [n_chunks, H, dk], Kd, Qd [tokens, H, dk], Kw [n_chunks, H, dk, CL], W [n_chunks, H, dk, dv], U [tokens, H, dv],
-// all on 16 bytes.
+// [n_chunks, H, CL, CL], E [n_chunks, H, dkp], Kd, Qd [tokens, H, dkp], Kw [n_chunks, H, dkp, CL],
+// W [n_chunks, H, dk, dv], U [tokens, H, dv], all on 16 bytes; dkp is kvf_chdelta_padded(dk).
+KVF_EXPORT int kvf_chdelta_padded(int dk) { return padded(dk); }
 KVF_EXPORT int kvf_chdelta_chunks(CHDELTA_ARGS_DECL, const int* chunks, int n_chunks, const int* runs, int n_runs,
                                   float* T, float* A, float* E, float* Kd, float* Kw, float* Qd, float* W, float* U,
                                   hipStream_t s) {
@@ -732,8 +750,7 @@ KVF_EXPORT int kvf_chdelta_chunks(CHDELTA_ARGS_DECL, const int* chunks, int n_ch
     return static_cast<int>(hipErrorInvalidValue);
   const ChunkPtrs p{rows, z, zb, neg_a, dt_bias, positions, slot_ids, chunks, runs, state, out, T, A, E, Kd, Kw, Qd, W, U,
                     n_chunks, n_runs};
-  const bool vec = dk % 4 == 0;
-#define GO(DKP, CL) return vec ? chunks_go<DKP, CL, true>(p, a, s) : chunks_go<DKP, CL, false>(p, a, s)
+#define GO(DKP, CL) return chunks_go<DKP, CL>(p, a, s)
   if (dk <= 32) GO(32, 64);
   if (dk <= 64) GO(64, 64);
   if (dk <= 128) GO(128, 64);

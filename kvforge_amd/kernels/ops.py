@@ -2350,14 +2350,16 @@ def ssm_scan(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, gates: torc
 
 # ------------------------------------------------------------------------------ delta rule, a decay per key channel
 CHDELTA_CHUNK_FROM = 24
+CHDELTA_PAD = 32            # PAD of chdelta.hip: some scratch tensors hold heads of whole so many channels
 
 
 def chdelta_scratch(n_tokens: int, n_chunks: int, heads: int, key_dim: int, value_dim: int) -> dict[str, tuple]:
     """(shape, dtype) of the scratch tensors the passes over the chunks (of ``ssm_plan``) need, by name."""
     H, dk, dv, cl = int(heads), int(key_dim), int(value_dim), ssm_chunk_len(key_dim)
+    dkp = -(-dk // CHDELTA_PAD) * CHDELTA_PAD
     out = {name: ((n_chunks, H, cl, cl), F32) for name in ("T", "A")}
-    out.update({name: ((n_tokens, H, dk), F32) for name in ("Kd", "Qd")})
-    out.update({"Kw": ((n_chunks, H, dk, cl), F32), "E": ((n_chunks, H, dk), F32), "W": ((n_chunks, H, dk, dv), F32), "U": ((n_tokens, H, dv), F32)})
+    out.update({"Kd": ((n_tokens, H, dkp), F32), "Qd": ((n_tokens, H, dkp), F32), "Kw": ((n_chunks, H, dkp, cl), F32),
+                "E": ((n_chunks, H, dkp), F32), "W": ((n_chunks, H, dk, dv), F32), "U": ((n_tokens, H, dv), F32)})
     return out
 
 

@@ -275,10 +275,12 @@ def test_the_memory_over_runs_steps_and_slots(H, G, dk, dv):
     assert float((wide[:, :4] - 5.0).abs().max()) == 0.0 and float((wide[:, -3:] - 5.0).abs().max()) == 0.0
 
 
-@pytest.mark.parametrize("H,G,dk,dv", [(3, 1, 32, 48), (2, 1, 64, 16), (2, 1, 64, 17), (8, 2, 128, 32)])
+@pytest.mark.parametrize("H,G,dk,dv", [(3, 1, 32, 48), (2, 1, 64, 16), (2, 1, 64, 17), (2, 1, 65, 32), (1, 1, 96, 40), (2, 2, 97, 16),
+                                       (8, 2, 128, 32), (2, 1, 129, 32), (1, 1, 160, 16), (2, 1, 161, 20), (1, 1, 192, 32),
+                                       (1, 1, 223, 16), (1, 1, 224, 48), (1, 1, 225, 16), (1, 1, 256, 33)])
 def test_the_memory_over_heads_that_fill_the_kernels_tiles(H, G, dk, dv):
-    """Heads of exactly as many channels as the chunks' kernel holds, value columns in whole sixteens or not: its form
-    without anything to leave out, and the other."""
+    """Heads of exactly as many channels as a form of the chunks' kernel holds, of one more and one fewer, value columns in
+    whole sixteens or not: the form without anything to leave out, and the other."""
     test_the_memory_over_runs_steps_and_slots(H, G, dk, dv)
 
 

@@ -58,6 +58,16 @@ def test_items_of_wide_heads_go_in_pairs_where_they_are_more_than_the_compute_un
     assert items == [(b, i) for b in seqs for i in range(-(-q_lens[b] * (H // KV) // 64))]
 
 
+@pytest.mark.parametrize("dk", [1, 31, 32, 33, 96, 97, 128, 129, 192, 250, 256])
+def test_the_scratch_of_channel_decays_holds_whole_heads(dk):
+    """What the kernels write is as wide as what is given to them."""
+    padded = ctypes.CDLL(library.build_module("chdelta")).kvf_chdelta_padded(dk)
+    shapes = ops.chdelta_scratch(5, 2, 3, dk, 16)
+    assert padded % 32 == 0 and padded - 32 < dk <= padded
+    assert shapes["Kd"][0] == shapes["Qd"][0] == (5, 3, padded) and shapes["E"][0] == (2, 3, padded)
+    assert shapes["Kw"][0] == (2, 3, padded, ops.ssm_chunk_len(dk))
+
+
 @pytest.mark.parametrize("m,n,k,own", [
     (33, 16384, 2048, True), (56, 24576, 2048, True), (57, 24576, 2048, False), (64, 65536, 2048, True), (64, 128256, 2048, True),
     (33, 16368, 2048, False), (65, 128256, 2048, False), (33, 32768, 1024, False), (33, 24576, 2304, False),
