@@ -249,15 +249,15 @@ KVF_EXPORT int kvf_add_parts(float* x, const float* delta, int parts, int rows, 
   return kvf_last_error();
 }
 
-constexpr int PAIR_KEEP = 8;  // elements of a row, and of each weight, that a thread keeps in registers
-
 // Two norms of the same row in one pass: y1 = v r w1 and y2 = v r w2 with v = x (+ delta, which is
 // then written back to x) and r = rsqrt(mean(v^2) + eps): for a block whose two sublayers each
 // have a norm of their own over the same stream.  Weights are fp32.  With few rows the trips to memory bound it: a
-// row and both weights are asked for together and stay in registers (2,048 wide: 8 rows 5.0 us, 2,042 rows
-// 11.9; element by element with a second read of the row 7.8 and 15.2).  A thread's elements are those that it
-// has in the loop for wider rows, so the sums are the same.
-template <typename T, typename D>
+// row and both weights are asked for together and stay in registers, KEEP elements of each a thread (2,048 wide: 8
+// rows 5.0 us, 2,042 rows 11.9; element by element with a second read of the row 7.8 and 15.2).  KEEP 0: rows too wide
+// for that.  What a thread asks for past the row costs too: 64 wide, 8 rows with a sum to add 2.1 us with KEEP 1, 2.7
+// with 8 (2.3 without registers), 1,024 wide, 2,048 rows 6.4 with 4, 7.8 with 8 (7.2).  A thread's elements are the same
+// in every form, so the sums are.
+template <typename T, typename D, int KEEP>
 __global__ void rmsnorm_pair_kernel(float* __restrict__ x, const D* __restrict__ delta,
                                     const float* __restrict__ w1, const float* __restrict__ w2, float eps,
                                     T* __restrict__ out1, T* __restrict__ out2, int h) {
@@ -266,10 +266,10 @@ __global__ void rmsnorm_pair_kernel(float* __restrict__ x, const D* __restrict__
   float* xr = x + m * h;
   const D* dr = delta ? delta + m * h : nullptr;
   float ss = 0.f;
-  if (h <= static_cast<int>(blockDim.x) * PAIR_KEEP) {
-    float v[PAIR_KEEP], d[PAIR_KEEP], g1[PAIR_KEEP], g2[PAIR_KEEP];
+  if constexpr (KEEP > 0) {
+    float v[KEEP], d[KEEP], g1[KEEP], g2[KEEP];
 #pragma unroll
-    for (int k = 0; k < PAIR_KEEP; ++k) {   // past the row: its last element, not used
+    for (int k = 0; k < KEEP; ++k) {   // past the row: its last element, not used
       const int i = min(static_cast<int>(k * blockDim.x + threadIdx.x), h - 1);
       v[k] = xr[i];
       d[k] = dr ? Elem<D>::load(dr + i) : 0.f;
@@ -277,7 +277,7 @@ __global__ void rmsnorm_pair_kernel(float* __restrict__ x, const D* __restrict__
       g2[k] = w2[i];
     }
 #pragma unroll
-    for (int k = 0; k < PAIR_KEEP; ++k) {
+    for (int k = 0; k < KEEP; ++k) {
       const int i = k * blockDim.x + threadIdx.x;
       if (i < h) {
         if (dr) {
@@ -290,7 +290,7 @@ __global__ void rmsnorm_pair_kernel(float* __restrict__ x, const D* __restrict__
     ss = block_sum(ss, scratch);
     const float r = rsqrtf(ss / static_cast<float>(h) + eps);
 #pragma unroll
-    for (int k = 0; k < PAIR_KEEP; ++k) {
+    for (int k = 0; k < KEEP; ++k) {
       const int i = k * blockDim.x + threadIdx.x;
       if (i < h) {
         const float y = v[k] * r;
@@ -320,9 +320,15 @@ template <typename T, typename D>
 static int rmsnorm_pair_launch(float* x, const void* delta, const float* w1, const float* w2, float eps, void* o1,
                                void* o2, int m, int h, hipStream_t s) {
   if (m <= 0) return 0;
-  const int threads = h >= 1024 ? 256 : (h >= 256 ? 128 : 64);
-  hipLaunchKernelGGL((rmsnorm_pair_kernel<T, D>), dim3(m), dim3(threads), 0, s, x, static_cast<const D*>(delta), w1, w2,
-                     eps, static_cast<T*>(o1), static_cast<T*>(o2), h);
+  const int threads = h >= 1024 ? 256 : (h >= 256 ? 128 : 64), each = (h + threads - 1) / threads;
+#define KVF_PAIR(KEEP)                                                                                                \
+  hipLaunchKernelGGL((rmsnorm_pair_kernel<T, D, KEEP>), dim3(m), dim3(threads), 0, s, x, static_cast<const D*>(delta), \
+                     w1, w2, eps, static_cast<T*>(o1), static_cast<T*>(o2), h)
+  if (each <= 1) KVF_PAIR(1);
+  else if (each <= 4) KVF_PAIR(4);
+  else if (each <= 8) KVF_PAIR(8);
+  else KVF_PAIR(0);
+#undef KVF_PAIR
   return kvf_last_error();
 }
 KVF_EXPORT int kvf_rmsnorm_pair_f32(float* x, const void* delta, int delta_f32, const float* w1, const float* w2,

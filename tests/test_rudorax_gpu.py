@@ -89,7 +89,7 @@ def test_two_norms_of_one_stream_in_one_pass(dtype, h, owed):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("h", [4, 512, 516, 1020, 1024, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("h", [4, 64, 65, 255, 256, 512, 516, 1020, 1023, 1024, 1028, 2048, 2052, 4096, 4100])
 @pytest.mark.parametrize("off", [0, 1])
 def test_two_norms_of_one_stream_at_the_edges_of_what_stays_in_registers(dtype, h, off):
     """Widths at which a row just fits a workgroup's registers or does not, and weights off their 16 bytes."""
