@@ -176,18 +176,9 @@ __device__ __forceinline__ bf16x8 as_frag(const uint4& r) { return __builtin_bit
 __device__ __forceinline__ uint32_t first_mask(int e, int live) {
   return 2 * e + 1 < live ? 0xffffffffu : (2 * e < live ? 0xffffu : 0u);
 }
-// Keeps the first `live` (0..8) bf16 of a fragment, clears the rest.
-__device__ __forceinline__ uint4 keep_first(const uint4& r, int live) {
-  if (!__any(live < 8)) return r;  // nearly every fragment is whole in every lane
-  uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-  for (int e = 0; e < 4; ++e) w[e] &= first_mask(e, live);
-  return make_uint4(w[0], w[1], w[2], w[3]);
-}
-
-// The same in the registers that hold it.
+// Keeps the first `live` (0..8) bf16 of a fragment, clears the rest, in the registers that hold it.
 __device__ __forceinline__ void clear_behind(uint4& r, int live) {
-  if (__any(live < 8)) {
+  if (__any(live < 8)) {  // nearly every fragment is whole in every lane
     r.x &= first_mask(0, live);
     r.y &= first_mask(1, live);
     r.z &= first_mask(2, live);

@@ -211,16 +211,16 @@ static int rmsnorm_parts_launch(float* x, const int* rows, const float* delta, i
   if (parts == P)                                                                                                 \
     hipLaunchKernelGGL((rmsnorm_parts_kernel<bf16_t, W, P>), grid, block, 0, s, x, rows, delta, bias,             \
                        static_cast<const W*>(w), eps, static_cast<bf16_t*>(out), h, x_rows, vec);
-  KVF_PARTS(1) KVF_PARTS(2) KVF_PARTS(4) KVF_PARTS(8)
+  KVF_PARTS(2) KVF_PARTS(4) KVF_PARTS(8)
 #undef KVF_PARTS
   return kvf_last_error();
 }
-// delta: fp32 [parts][xr][h], parts 1, 2, 4 or 8; h a multiple of 4 up to 4096; x and delta on 16 bytes, out on 8.
+// delta: fp32 [parts][xr][h], parts 2, 4 or 8 (what a product is cut into); h a multiple of 4 up to 4096; x and delta on 16 bytes, out on 8.
 KVF_EXPORT int kvf_rmsnorm_parts(float* x, const int* rows, const float* delta, int parts, const float* bias, const void* w,
                                  int wf, float eps, void* out, int m, int h, int xr, hipStream_t s) {
   if (m <= 0) return 0;
   auto at = [](const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; };
-  if (h <= 0 || h % 4 != 0 || h > 4096 || (parts != 1 && parts != 2 && parts != 4 && parts != 8) || !at(x, 16) ||
+  if (h <= 0 || h % 4 != 0 || h > 4096 || (parts != 2 && parts != 4 && parts != 8) || !at(x, 16) ||
       !at(out, 8) || !at(delta, 16))
     return static_cast<int>(hipErrorInvalidValue);
   const int vec = at(bias, 16) && at(w, wf ? 16 : 8);

@@ -775,18 +775,16 @@ KVF_EXPORT int kvf_moe_grouped_many_rows(int pairs, int E, int ff, int K) {
 
 // kvf_moe_topk of up to CHOOSE_TOKENS tokens together with the plan of kvf_moe_grouped, which is then called with
 // `planned`; arguments as there.
-KVF_EXPORT int kvf_moe_choose_tokens() { return CHOOSE_TOKENS; }
 KVF_EXPORT int kvf_moe_topk_plan(const float* z, int z_stride, const float* bias, const float* correction, int* sel,
                                  float* wgt, int n, int R, int top, int score, int renorm, float scale, int E, int ff, int K,
-                                 int* where, int* order, int* tiles, int* num_tiles, int max_tiles, int many_rows,
-                                 hipStream_t s) {
+                                 int* where, int* order, int* tiles, int* num_tiles, int max_tiles, hipStream_t s) {
   if (n <= 0) return 0;
   const int pairs = n * top;
   if (n > CHOOSE_TOKENS || score < SCORE_SOFTMAX || score > SCORE_CHOSEN || (score == SCORE_CHOSEN && correction) ||
       R <= 0 || R > MAX_PER_LANE * KVF_WAVE || top <= 0 || top > MAX_TOP || top > R || E <= 0 || E > PLAN_MAX_EXPERTS ||
       max_tiles < (pairs + 15) / 16 + E)
     return static_cast<int>(hipErrorInvalidValue);
-  const bool many = many_rows < 0 ? kvf_moe_grouped_many_rows(pairs, E, ff, K) != 0 : many_rows != 0;
+  const bool many = kvf_moe_grouped_many_rows(pairs, E, ff, K) != 0;
   // the plan has a thread for every expert
   const int threads = n * KVF_WAVE > E ? n * KVF_WAVE : (E + KVF_WAVE - 1) / KVF_WAVE * KVF_WAVE;
 #define GO(PER)                                                                                                      \

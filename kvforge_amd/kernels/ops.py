@@ -1895,7 +1895,7 @@ def _moe_form(form: str, limit: float | None, who: str) -> tuple[int, float]:
     return _gate_form(form, limit, who)
 
 
-MOE_PLAN_TOKENS = 16        # CHOOSE_TOKENS of moe.hip
+MOE_PLAN_TOKENS = 16        # CHOOSE_TOKENS of moe.hip, which refuses more
 
 
 def _check_moe_plan(scratch: dict, n: int, top: int, experts: int) -> int:
@@ -1944,12 +1944,12 @@ def moe_topk(logits: torch.Tensor, correction: torch.Tensor | None, chosen: torc
             raise KernelError("moe_topk: the plan's weights do not fit its experts")
         max_tiles = _check_moe_plan(scratch, n, top, experts)
         f = _fn("moe", "kvf_moe_topk_plan", [c_void_p, c_int] + [c_void_p] * 4 + [c_int] * 5 + [c_float] + [c_int] * 3
-                + [c_void_p] * 4 + [c_int, c_int, c_void_p])
+                + [c_void_p] * 4 + [c_int, c_void_p])
         _ok(f(logits.data_ptr(), logits.stride(0) if n > 1 else R, bias.data_ptr() if bias is not None else None,
               correction.data_ptr() if correction is not None else None, chosen.data_ptr(), weights.data_ptr(), n, R,
               top, MOE_SCORES[scores], 1 if renormalize else 0, float(scale), int(experts), int(ff), k,
               scratch["where"].data_ptr(), scratch["order"].data_ptr(), scratch["tiles"].data_ptr(),
-              scratch["num_tiles"].data_ptr(), max_tiles, -1, _stream()), "moe_topk_plan")
+              scratch["num_tiles"].data_ptr(), max_tiles, _stream()), "moe_topk_plan")
         return
     f = _fn("moe", "kvf_moe_topk", [c_void_p, c_int] + [c_void_p] * 4 + [c_int] * 5 + [c_float, c_void_p])
     _ok(f(logits.data_ptr(), logits.stride(0) if n > 1 else R, bias.data_ptr() if bias is not None else None,

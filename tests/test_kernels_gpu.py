@@ -292,6 +292,8 @@ def test_gemm_in_parts_refuses_what_does_not_fit():
         ops().rmsnorm(torch.zeros(41, 2048, device=DEV), None, 1e-5, torch.zeros(41, 2048, dtype=torch.bfloat16, device=DEV), add=parts)
     with pytest.raises(ops().KernelError):               # parts go with bf16 rows
         ops().rmsnorm(torch.zeros(40, 2048, device=DEV), None, 1e-5, torch.zeros(40, 2048, device=DEV), add=parts)
+    with pytest.raises(ops().KernelError):               # a product is cut in two at least
+        ops().rmsnorm(torch.zeros(40, 2048, device=DEV), None, 1e-5, torch.zeros(40, 2048, dtype=torch.bfloat16, device=DEV), add=parts[:1])
 
 
 @pytest.mark.parametrize("m", [33, 64, 100, 257])
