@@ -939,8 +939,8 @@ def test_wide_layers_through_graphs_and_queued_runs(tmp_path):
 @pytest.mark.parametrize("count,bucket", [(24, 32), (40, 64)])
 def test_graph_replay_with_many_requests(model_a, count, bucket):
     """Many requests decode together.  A padded batch of 32 is two row tiles of the hand-written
-    matrix product; one of 64 is past what it takes, so the captured graph holds the library's
-    products.  Replays must give the tokens of eager launches either way."""
+    matrix product; one of 64 is past what it takes over layers as small as these, so the captured graph
+    holds the library's products.  Replays must give the tokens of eager launches either way."""
     folder, oracle = model_a
     prompts = prompts_for(256, count, 12, 4, 20)
     params = SamplingParams(max_tokens=14, temperature=0.0)
@@ -957,6 +957,57 @@ def test_graph_replay_with_many_requests(model_a, count, bucket):
     assert graphed == eager
     for p, out in zip(prompts, graphed):
         oracle.of("bfloat16").check_choices(p, out, 3e-2)
+
+
+@pytest.mark.parametrize("count,bucket", [(24, 32), (40, 64)])
+def test_graph_replay_with_many_requests_of_wide_layers(tmp_path, monkeypatch, count, bucket):
+    """Batches of 32 and 64 over layers as deep as a served model's: the products that are added to the stream are cut over
+    K into parts, which the captured steps' norms add, and single tokens start longest context first (more of them than compute
+    units).  Every captured step picks what the same padded step picks launched eagerly, and the tokens are the
+    plain model's choice within bf16 rounding."""
+    from kvforge_amd.engine.batch import StepEntry
+    from kvforge_amd.kernels import ops
+    from tests.replay_util import WIDE, sharpen
+    folder = str(tmp_path / "deep")
+    kvforge_amd.write_random_model(folder, dict(WIDE, vocab_size=500, num_hidden_layers=2, num_attention_heads=32,
+                                                num_key_value_heads=16, intermediate_size=2048), seed=6)
+    sharpen(folder, 4.0)
+    oracle = Oracle(folder)
+    engine = engine_for(folder, "bfloat16", block_size=16, max_num_seqs=64, num_blocks=1024, max_num_batched_tokens=512)
+    runner = engine.runner
+    used = {"parts": 0, "order": 0}
+    parts, decode = ops.gemm_parts, ops.attn_decode
+
+    def count_parts(*args):
+        used["parts"] += 1
+        parts(*args)
+
+    def count_order(*args, **kw):
+        used["order"] += kw.get("order") is not None
+        decode(*args, **kw)
+
+    monkeypatch.setattr(ops, "gemm_parts", count_parts)
+    monkeypatch.setattr(ops, "attn_decode", count_order)
+    prompts = prompts_for(500, count, 12, 4, 150)
+    for i, p in enumerate(prompts):
+        engine.cache.allocate(f"r{i}", len(p) + 12)
+        runner.step([StepEntry(f"r{i}", p[:-1], 0, "none")])
+    params = [SamplingParams(max_tokens=12, temperature=0.0)] * count
+    got = [list(p) for p in prompts]
+    for step in range(10):
+        entries = [StepEntry(f"r{i}", ids[-1:], len(ids) - 1, "last") for i, ids in enumerate(got)]
+        used.update(parts=0, order=0)
+        if step % 3 != 2:           # replays follow each other, and eager steps stand between them
+            eager = runner.model.forward(runner.build_step(entries, pad_to=bucket)[0])[:count].argmax(-1).tolist()
+            assert used == {"parts": 4, "order": 2}
+        picked = runner.decode_run(entries, 0, params, list(range(count)), [step] * count, 1)[0]
+        if step % 3 != 2:
+            assert picked == eager
+        for ids, token in zip(got, picked):
+            ids.append(token)
+    assert any(b == bucket for b, *_ in runner.graphs) and runner.num_graph_replays >= 8
+    for p, ids in zip(prompts, got):
+        oracle.of("bfloat16").check_choices(p, ids[len(p):], 3e-2)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -1614,6 +1614,61 @@ def test_query_runs_over_pages_of_sixteen_keys(d, form):
         assert torch.equal(a.nan_to_num(9.0), b.nan_to_num(9.0))
 
 
+@pytest.mark.parametrize("d", [64, 128, 208])
+@pytest.mark.parametrize("bs", [8, 16])
+@pytest.mark.parametrize("window,keep,chunk", [(70, 0, 0), (70, 21, 0), (130, 0, 0), (200, 40, 0), (0, 0, 96), (0, 0, 128)])
+def test_query_runs_through_windows_that_hold_whole_blocks(d, bs, window, keep, chunk):
+    """Blocks of 32 keys that every row of a wave sees whole go without a mask, also inside a window or a chunk: runs that end
+    one key before, at and behind a block, with a last tile of rows that is not full, pages behind the window given back and a
+    page lost on the way (its keys and values count as zeros), against attention in 64 bits.  Scores are so far apart that a
+    key too many or too few takes or leaves most of a row's weight."""
+    H, KV, scale = 6, 2, 0.3
+    q_lens, starts = [70, 33, 39, 40, 41, 5, 193], [0, 201, 216, 216, 216, 1000, 320]
+    g = torch.Generator().manual_seed(d + window + chunk)
+    ctxs = [a + b for a, b in zip(q_lens, starts)]
+    keys = [torch.randn(c, KV, d, generator=g).to(torch.bfloat16) for c in ctxs]
+    vals = [torch.randn(c, KV, d, generator=g).to(torch.bfloat16) for c in ctxs]
+    q = (2.0 * torch.randn(sum(q_lens), H, d, generator=g)).to(torch.bfloat16)
+    nb = sum(-(-c // bs) for c in ctxs) + 5
+    ids = torch.randperm(nb, generator=g).tolist()
+    k, v = torch.full((nb, KV, bs, d), 3.0).to(torch.bfloat16), torch.full((nb, KV, d, bs), 3.0).to(torch.bfloat16)
+    table = torch.full((len(ctxs), -(-max(ctxs) // bs)), -1, dtype=torch.int32)
+    want, at = [], 0
+    for s, (n, lo, c) in enumerate(zip(q_lens, starts, ctxs)):
+        kk, vv = keys[s].double(), vals[s].double()
+        for b in range(-(-c // bs)):
+            span = slice(b * bs, min(c, (b + 1) * bs))
+            if window and span.start >= keep and span.stop <= lo - window + 1:
+                continue
+            if s == 4 and 190 in range(span.start, span.stop):
+                kk[span], vv[span] = 0.0, 0.0
+                continue
+            page = ids.pop()
+            table[s, b] = page
+            k[page, :, :span.stop - span.start] = keys[s][span].transpose(0, 1)
+            v[page, :, :, :span.stop - span.start] = vals[s][span].permute(1, 2, 0)
+        pos, j = torch.arange(lo, c)[:, None], torch.arange(c)
+        seen = j <= pos
+        if window:
+            seen &= (j > pos - window) | (j < keep)
+        if chunk:
+            seen &= j // chunk == pos // chunk
+        x = torch.einsum("qhd,jhd->hqj", q[at:at + n].double(), kk.repeat_interleave(H // KV, 1)) * scale
+        p = torch.softmax(x.masked_fill(~seen, -math.inf), -1)
+        want.append(torch.einsum("hqj,jhd->qhd", p, vv.repeat_interleave(H // KV, 1)))
+        at += n
+    want, qd = torch.cat(want).reshape(at, H * d), q.reshape(at, H * d).to(DEV)
+    for tiles in ((1, 2) if d <= 128 else (1,)):
+        per = ops().prefill_rows_per_item(torch.bfloat16, d, bs, tiles)
+        rows = attention_rows(q_lens, H // KV, per, starts, ops().prefill_takes_pairs(torch.bfloat16, d, bs))
+        out = torch.full_like(qd, 7.0)
+        ops().attn_prefill(qd, k.to(DEV), v.to(DEV), table.to(DEV), torch.tensor([0] + list(np.cumsum(q_lens)), dtype=torch.int32, device=DEV),
+                           torch.tensor(ctxs, dtype=torch.int32, device=DEV), rows, out, H, KV, d, scale, window,
+                           rows_per_item=per, keep_first=keep, chunk=chunk)
+        # probabilities and results are rounded to bf16, the largest values are about 4
+        torch.testing.assert_close(out.double().cpu(), want, atol=3e-2, rtol=2.0 ** -7)
+
+
 def attention_rows(q_lens, G, per, starts, pairs):
     from kvforge_amd.parts.attention import prefill_work_rows
     rows = prefill_work_rows(q_lens, list(range(len(q_lens))), G, per, starts, pairs)
