@@ -78,6 +78,8 @@ def test_single_tokens_are_listed_longest_context_first():
     assert step.decode_seq_ids is None and step.decode_order.tolist() == [1, 3, 2, 0]
     fill_step(step, meta, [StepEntry("a", [3, 4], 0)] + entries[1:3], cache.block_table, lambda r: -1, 4)
     assert step.decode_order is None and step.decode_seq_ids.tolist() == [1, 2]
+    fill_step(step, meta, entries[:1], cache.block_table, lambda r: -1, 4)
+    assert step.decode_order is None and step.decode_seq_ids is None      # a single one has no order
 
 
 def test_pure_decode_padding_is_inert():

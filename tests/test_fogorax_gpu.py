@@ -526,8 +526,9 @@ def plain_logits(cfg, w, toks, dtype):
     key = (id(w), tuple(toks), dtype)
     if key not in _WANT:
         _WANT[key] = (plain.forward(cfg, w, toks),
-                      plain.forward(cfg, w, toks, store=torch.bfloat16) if dtype == torch.bfloat16 else None)
-    return _WANT[key]
+                      plain.forward(cfg, w, toks, store=torch.bfloat16) if dtype == torch.bfloat16 else None,
+                      w)                  # with the weights, whose id is theirs as long as they are held
+    return _WANT[key][:2]
 
 
 def check(got, cfg, w, toks, dtype, what=""):
