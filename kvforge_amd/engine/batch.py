@@ -104,6 +104,9 @@ class Workspace:
 
     def zeros(self, name: str, shape: tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
         """Like ``buf`` for memory whose users leave it zero: cleared once, when it is made."""
+        view = self._views.get((name, dtype, shape))
+        if view is not None:
+            return view
         n = 1
         for s in shape:
             n *= int(s)
@@ -116,7 +119,10 @@ class Workspace:
             self._bufs[key] = flat
             for k in [k for k in self._views if k[0] == name and k[1] == dtype]:
                 del self._views[k]
-        return flat[:n].view(shape)
+        view = flat[:n].view(shape)
+        if len(self._views) < 4096:
+            self._views[(name, dtype, shape)] = view
+        return view
 
     def snapshot(self) -> list[torch.Tensor]:
         return list(self._bufs.values())
@@ -179,7 +185,7 @@ class Step:
         self.token_ids = self.positions = self.seq_of_token = None
         self.cu_q = self.ctx_lens = self.slot_ids = self.logits_rows = None
         self.decode_seq_ids: torch.Tensor | None = None
-        # of a step of single tokens alone: all its sequences, longest context first (as they stood when
+        # of a step of several single tokens alone: all its sequences, longest context first (as they stood when
         # the step was filled; steps that the device advances to by itself keep the order)
         self.decode_order: torch.Tensor | None = None
         self.block_tables: list[torch.Tensor] = []
@@ -420,10 +426,9 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     host[off["logits_rows"]:off["logits_rows"] + R] = rows
 
     # longest context first, so that kernels which take them in this order start what lasts longest first
-    lengths = ctx.tolist()
     decode = [b for b, n in enumerate(q_lens) if n == 1] + list(range(B, Bp))
     if len(decode) > 1:
-        decode.sort(key=lengths.__getitem__, reverse=True)
+        decode.sort(key=ctx.tolist().__getitem__, reverse=True)
     prefill = [b for b, n in enumerate(q_lens) if n > 1]
     host[off["decode_seq_ids"]:off["decode_seq_ids"] + len(decode)] = decode
 
@@ -446,7 +451,7 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     step.slot_ids = meta.view("slot_ids", Bp)
     step.logits_rows = meta.view("logits_rows", max(R, 1))[:R]
     step.decode_seq_ids = None if len(decode) == Bp else meta.view("decode_seq_ids", len(decode))
-    step.decode_order = meta.view("decode_seq_ids", Bp) if len(decode) == Bp else None
+    step.decode_order = meta.view("decode_seq_ids", Bp) if len(decode) == Bp > 1 else None
     step.block_tables = [meta.table_view(g)[:Bp] for g in range(len(meta.table_widths))]
     step.request_ids = [e.request_id for e in entries]
     step.q_lens = [int(x) for x in lens]

@@ -54,9 +54,11 @@ def _check(t: torch.Tensor, name: str, dtype=None, shape=None, contiguous=True) 
         raise KernelError(f"{name} must be {dtype}, got {t.dtype}")
     if shape is not None:
         have = t.shape
-        bad = len(have) != len(shape)
-        if not bad:
-            for want, got in zip(shape, have):   # a plain loop: this runs for every operand of every launch
+        # this runs for every operand of every launch: most shapes name every size, the others take a plain loop
+        bad = have != shape
+        if bad and len(have) == len(shape):
+            bad = False
+            for want, got in zip(shape, have):
                 if want is not None and want != got:
                     bad = True
                     break
@@ -755,17 +757,20 @@ _GEMM_BF16_ARGS = ([c_void_p, c_int, c_void_p, c_int, c_void_p] + [c_int] * 6
 # (``k_halves_pay``).  The half that is left owed costs its consumers a second fp32 operand, so
 # wider streams lose more there than the product gains (measured at 3072 columns: 7% of the step).
 K_HALVES_MIN_K = 4096
-_compute_units: dict[int, int] = {}
+_compute_units: dict[int | torch.device, int] = {}   # by index, and by devices that name one
 
 
 def compute_units(device) -> int:
     """Compute units of the device, asked of the device once."""
-    index = torch.device(device).index
-    if index is None:
-        index = torch.cuda.current_device()
-    if index not in _compute_units:
-        _compute_units[index] = int(torch.cuda.get_device_properties(index).multi_processor_count)
-    return _compute_units[index]
+    units = _compute_units.get(device)
+    if units is None:
+        index = torch.device(device).index
+        if index is None:
+            device = index = torch.cuda.current_device()
+        if index not in _compute_units:
+            _compute_units[index] = int(torch.cuda.get_device_properties(index).multi_processor_count)
+        units = _compute_units[device] = _compute_units[index]
+    return units
 
 
 class StreamedWeight:
@@ -875,7 +880,7 @@ def is_library_product(a: torch.Tensor, w: torch.Tensor) -> bool:
     if not (a.dtype == BF16 and w.dtype == BF16 and _rows_aligned(a, k, lda)):
         return False
     if m > SKINNY_MAX_M:
-        return not streams_in_place_of_library(a, w)
+        return m > MID_MAX_M or not streams_in_place_of_library(a, w)
     return m > 16 and k >= 2 * n
 
 
@@ -907,10 +912,10 @@ def parts_count(a: torch.Tensor, w) -> int:
     """In how many parts ``gemm_parts(a, w, ...)`` stores the product, 0 where it does not pay (or
     fit): 17 to 64 bf16 rows over a tiled weight with few columns."""
     m, k = a.shape
-    if not (16 < m <= MID_MAX_M and isinstance(w, StreamedWeight) and a.dtype == BF16 and a.stride(1) == 1
-            and _rows_aligned(a, k, a.stride(0))):
+    count = _parts_count(m, w.shape[0], k, a.get_device()) if 16 < m <= MID_MAX_M and isinstance(w, StreamedWeight) else 0
+    if count and not (a.dtype == BF16 and a.stride(1) == 1 and _rows_aligned(a, k, a.stride(0))):
         return 0
-    return _parts_count(m, w.shape[0], k, a.get_device())
+    return count
 
 
 def gemm_parts(a: torch.Tensor, w, parts: torch.Tensor) -> None:
@@ -1014,7 +1019,7 @@ def gemm(a: torch.Tensor, w, out: torch.Tensor, accumulate: bool = False,
     if not accumulate:
         _tcode(out.dtype)
     if a.dtype == BF16 and w.dtype == BF16 and _rows_aligned(a, k, lda):
-        if not is_library_product(a, w) and not (accumulate and streams_in_place_of_library(a, w)):
+        if not is_library_product(a, w) and not (accumulate and SKINNY_MAX_M < m <= MID_MAX_M and streams_in_place_of_library(a, w)):
             f = _fn("gemm_bf16", "kvf_gemm_bf16", _GEMM_BF16_ARGS)
             wp, tiled = _w_args(w)
             _ok(f(a.data_ptr(), 0, wp, tiled, out.data_ptr(), out_kind, m, n, k, lda, ldc, 0.0,

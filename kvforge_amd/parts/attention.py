@@ -571,8 +571,10 @@ class PagedAttention(Mixer):
             # With more workgroups than compute units the longest walks have to start first: two on one unit set
             # the kernel's time (41 contexts of 60 to 2,900, 8 kv heads of 64: 36.5 us as the requests came, 30.9 longest
             # first; 41 of 1,500: 31.2 and 31.4).  Up to one a unit the order's own load would be all it changes.
-            order = step.decode_order if (token_is_seq and not (window or chunk) and splits * step.n_decode * KV
-                                          > compute_units(step.device)) else None
+            order = step.decode_order
+            if order is not None and (not token_is_seq or window or chunk
+                                      or splits * step.n_decode * KV <= compute_units(qkv.device)):
+                order = None
             workspace = None
             if splits > 1:
                 workspace = (ws.buf("decode_part_acc", (step.n_decode * H * splits * d,), torch.float32),
