@@ -749,6 +749,8 @@ SKINNY_MAX_M = 32
 FUSED_NORM_MAX_M = 16
 FUSED_EPILOGUE_MAX_M = 64
 MID_MAX_M = 64              # rows of the kernel that takes A through LDS, and of products in parts
+PARTS_MIN_K = 2048          # kvf_gemm_bf16_parts_count has no parts below
+STREAMED_MIN_K = 2048       # and the rule of streams_in_place_of_library leaves every smaller K to the library
 _GEMM_BF16_ARGS = ([c_void_p, c_int, c_void_p, c_int, c_void_p] + [c_int] * 6
                    + [c_float, c_void_p, c_void_p, c_void_p])
 # A product that is added to a narrow fp32 stream (few output columns, long K) has too few
@@ -880,7 +882,7 @@ def is_library_product(a: torch.Tensor, w: torch.Tensor) -> bool:
     if not (a.dtype == BF16 and w.dtype == BF16 and _rows_aligned(a, k, lda)):
         return False
     if m > SKINNY_MAX_M:
-        return m > MID_MAX_M or not streams_in_place_of_library(a, w)
+        return m > MID_MAX_M or k < STREAMED_MIN_K or not streams_in_place_of_library(a, w)
     return m > 16 and k >= 2 * n
 
 
@@ -896,7 +898,7 @@ def streams_in_place_of_library(a: torch.Tensor, w) -> bool:
     rows 16.5 and 18.2.  With ``accumulate`` gemm_skinny_kernel would take it, slower throughout ([16384, 2048] 19
     against 24)."""
     m, k = a.shape
-    if not (SKINNY_MAX_M < m <= MID_MAX_M and k >= 2048 and (k < 2112 or k % 64) and isinstance(w, StreamedWeight)):
+    if not (SKINNY_MAX_M < m <= MID_MAX_M and k >= STREAMED_MIN_K and (k < 2112 or k % 64) and isinstance(w, StreamedWeight)):
         return False
     columns = w.shape[0] // compute_units(a.device)
     return columns >= (64 if m <= 56 or k % 64 else 256)

@@ -433,6 +433,21 @@ class PagedAttention(Mixer):
         cuts = max(1, min(room // workgroups, finest, MAX_CUTS))
         return max(cuts, min(skew, max(1, cell)))
 
+    def _decode_plan(self, step, on_matrix_cores: bool) -> tuple[int, bool]:
+        """(cuts of the key range, whether the workgroups start in the step's order) for the single tokens.  With
+        more workgroups than compute units the longest walks have to start first: two on one unit set the kernel's
+        time (41 contexts of 60 to 2,900, 8 kv heads of 64: 36.5 us as the requests came, 30.9 longest first; 41 of
+        1,500: 31.2 and 31.4).  Up to one a unit the order's own load would be all it changes.  Layers that agree on all that
+        this depends on share it through the step's scratch: worked out in every layer it was host time that steps of narrow
+        models wait for (6 layers, 8 requests, kernels left out: 580 us a step on one host core, 548 with this)."""
+        key = ("attention.decode_plan", type(self), self.H, self.KV, self.window, self.chunk, self.keep_first, on_matrix_cores)
+        plan = step.scratch.get(key)
+        if plan is None:
+            cuts = self._decode_cuts(step, on_matrix_cores)
+            in_order = not (self.window or self.chunk) and cuts * step.n_decode * self.KV > compute_units(step.device)
+            plan = step.scratch[key] = cuts, in_order
+        return plan
+
     def _prefill_work(self, step, act: torch.dtype, block_size: int):
         """(work rows on the device, rows per item) of the step's query runs, or ``(None, 0)``.
         Items of 128 rows halve what a key block costs per row (its page lookups,
@@ -566,15 +581,9 @@ class PagedAttention(Mixer):
                              keep_first=self.keep_first, gate=gate_in_kernel, sinks=self.sinks,
                              score_cap=self.score_cap, chunk=chunk, dist=self.dist)
         if step.n_decode:
-            splits = self._decode_cuts(step, ops.attention_on_matrix_cores(act, bs, d))
+            splits, in_order = self._decode_plan(step, ops.attention_on_matrix_cores(act, bs, d))
             token_is_seq = step.decode_seq_ids is None and work is None
-            # With more workgroups than compute units the longest walks have to start first: two on one unit set
-            # the kernel's time (41 contexts of 60 to 2,900, 8 kv heads of 64: 36.5 us as the requests came, 30.9 longest
-            # first; 41 of 1,500: 31.2 and 31.4).  Up to one a unit the order's own load would be all it changes.
-            order = step.decode_order
-            if order is not None and (not token_is_seq or window or chunk
-                                      or splits * step.n_decode * KV <= compute_units(qkv.device)):
-                order = None
+            order = step.decode_order if in_order and token_is_seq else None
             workspace = None
             if splits > 1:
                 workspace = (ws.buf("decode_part_acc", (step.n_decode * H * splits * d,), torch.float32),

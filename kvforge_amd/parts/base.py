@@ -341,7 +341,7 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
         return
     count = 0
     rows = a.shape[0]
-    if (16 < rows <= ops.MID_MAX_M
+    if (16 < rows <= ops.MID_MAX_M and w.shape[1] >= ops.PARTS_MIN_K
             and not (rows < 24 and getattr(step, "settled_next", False) and w.shape[1] < 2 * w.shape[0])):
         count = ops.parts_count(a, w)
         if count and not (residual.is_contiguous() and residual.data_ptr() % 16 == 0):

@@ -131,3 +131,38 @@ def test_a_parallel_block_says_who_settles_what_its_sublayers_owe(monkeypatch, f
     step.ws = Workspace("cpu")
     part.forward(torch.zeros(3, 8), step, None)
     assert said == wanted + ([("after", False)] if after else []) and not step.settled_next
+
+
+@pytest.mark.parametrize("n", [1, 16, 4096])
+@pytest.mark.parametrize("m", [17, 64])
+def test_no_product_goes_in_parts_below_the_least_k(m, n):
+    """What the host leaves unasked is what the kernel's rule refuses."""
+    count = ctypes.CDLL(library.build_module("gemm_bf16")).kvf_gemm_bf16_parts_count
+    assert not any(count(m, n, k) for k in range(8, ops.PARTS_MIN_K, 8))
+
+
+@pytest.mark.parametrize("n,KV,window,chunk,in_order", [
+    (41, 8, None, None, True), (32, 8, None, None, False), (33, 8, None, None, True), (41, 8, 512, None, False),
+    (41, 8, None, 512, False), (257, 1, None, None, True), (256, 1, None, None, False)])
+def test_layers_alike_share_the_plan_of_single_tokens(monkeypatch, n, KV, window, chunk, in_order):
+    """The step's order is taken where the workgroups outnumber the compute units and every layer sees whole contexts; it is
+    worked out once a step for layers alike, and again for ones that are not and for a step filled anew."""
+    monkeypatch.setattr(attention, "compute_units", lambda device: 256)
+    asked = []
+
+    def layer(**other):
+        part = object.__new__(attention.PagedAttention)
+        part.__dict__.update(dict(H=32, KV=KV, window=window, chunk=chunk, keep_first=0), **other)
+        part._decode_cuts = lambda step, on_matrix_cores: asked.append(part) or 1
+        return part
+
+    step = Step()
+    step.device, step.n_decode = None, n
+    parts = [layer(), layer(), layer(window=64), layer(H=64)]
+    plans = [p._decode_plan(step, True) for p in parts * 2]
+    assert plans == [(1, in_order), (1, in_order), (1, False), (1, in_order)] * 2
+    assert asked == [parts[0], parts[2], parts[3]]
+    assert parts[1]._decode_plan(step, False) == (1, in_order) and asked[3:] == [parts[1]]
+    step.scratch = {}
+    parts[1]._decode_plan(step, True)
+    assert asked[4:] == [parts[1]]
