@@ -422,7 +422,9 @@ constexpr bool runs_pair(int dt) { return dt > 8; }
 // A block was 104 vector instructions beside its 8 products, half of them for addresses, and is 90: 32 heads over 8 kv heads of
 // 64, 2,048 queries 49.1 -> 46.5 us, through a window of 1,024 42.5 -> 33.7 (blocks that every row sees whole need no mask
 // there either), three ragged runs behind up to 3,072 keys 88.5 -> 80.8; of 128, 2,048 queries 76.1 -> 70.4; 32 heads of 224
-// over one 110.3 -> 106.5.
+// over one 110.3 -> 106.5.  Every form gains, so each has both (32 heads of 128, 2,048 queries): slopes 81.7 -> 74.4, sinks 71.3 ->
+// 64.4, a cap 90.8 -> 85.7, chunks of 512 35.1 -> 30.8, biases by distance 86.0 -> 70.0 and through a window of 1,024 83.9 -> 59.0.
+// Runs of 61 queries are as fast either way.
 template <int DT, int RT, int NW, int BIAS, bool SINK, bool EVEN>
 __global__ __launch_bounds__(NW * KVF_WAVE) KVF_VGPR_FORM(DT <= 8 || RT == 1) void attn_mfma_runs_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,

@@ -631,8 +631,8 @@ __global__ __launch_bounds__(max_waves(MT, NT, AT) * KVF_WAVE) void gemm_skinny_
 // rows of 64 bytes each, as many bytes as of W at 64 rows, and a pass over its few k-steps ended in a
 // wait for all of them (2,048 x 16,384 with the gate: 23.6 us at 41 rows, 2.8 TB/s).  Here A goes
 // through LDS once for the workgroup, 128 columns a stage (whole cache lines), and W straight into
-// registers, both MID_AHEAD stages before they are used, so that the memory always has 64 to 96 KB of
-// a workgroup's requests; two workgroups fit a compute unit (128 registers a lane) and cover each
+// registers, both MID_AHEAD stages before they are used, so that the memory always has 48 to 96 KB of
+// a workgroup's requests (by rows and groups); two workgroups fit a compute unit (128 registers a lane) and cover each
 // other's barriers.  Four or six stages ahead were no faster (17.6 / 18.4 us) and cost registers.
 // Eight waves: NG groups of 16 columns, the k-steps of a stage shared by 8 / NG waves whose sums are
 // added in LDS.  41 rows: 17.5 us; 20 and 61 rows 21.2 -> 16.1, 25.0 -> 18.3; a head of
@@ -974,8 +974,9 @@ KVF_EXPORT int kvf_gemm_bf16(const void* A, int a_type, const void* W, int w_til
 // A product of 17 to 64 bf16 rows cut over K, see gemm_mid_kernel.  How many parts M rows over W [N, K]
 // are stored in, or 0 where they had better be one product: wide outputs fill the chip by themselves, and
 // up to 32 rows over a matrix with fewer rows than columns gemm_skinny_kernel is as fast (4,096 x 2,048 at
-// 17 rows: 6.1 us both).  A shorter K gains a microsecond a product (1,024 x 2,048 at 33 rows 5.5 and 4.2), which the
-// models that have it do not show: their steps are bound by the host's launches (0.56 and 0.58 ms for 50 tokens).
+// 17 rows: 6.1 us both).  A shorter K would gain a microsecond a product (1,024 x 2,048 at 33 rows 5.5 and 4.2).  It is left
+// out because cuts sum in another order: models of such layers, whose steps are mostly bound by the host's launches (0.56 ms
+// and 0.58 with cuts for 50 tokens of layers 512 wide), would give other tokens near ties for next to nothing.
 KVF_EXPORT int kvf_gemm_bf16_parts_count(int M, int N, int K) {
   if (M <= 16 || M > 64 || N <= 0 || N % 16 != 0 || N > 4096 || K < 2048 || K % 8 != 0 || (M <= 32 && K < N)) return 0;
   return mid_cut(M, N, K, true).splits;
