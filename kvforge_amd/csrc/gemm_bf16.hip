@@ -50,29 +50,9 @@
 // rows 16g..16g+15, columns 32s..32s+31 in the order the instruction wants them (lane
 // 16*c + r holds row r, columns 8c..8c+7), zero-padded.  A fragment is then 1 KB of consecutive
 // bytes.  Both layouts give the same bits.
-#include "common.h"
+#include "gemm_common.h"
 
 namespace {
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
-struct RopeEpi {
-  const int* positions;
-  const int* seq_of_token;
-  const float* cos_t;
-  const float* sin_t;
-  const int* block_table;
-  bf16_t* k_pages;
-  bf16_t* v_pages;
-  int H, KV, d, rot, table_len, block_size, table_stride, num_blocks, write_kv, n_seqs;
-  // EPI 3: how a pair is joined (GateForm's act and limit), what it is multiplied by, and fp32 biases
-  // of the gate and up columns (by pair, may be null)
-  int act;
-  float act_limit, act_scale;
-  const float* gate_bias;
-  const float* up_bias;
-};
-
 // Sums that ride along, all bf16 (a workgroup of the fused projection reads every row of A and
 // of a_add: with the addend in fp32 that was as many bytes again as A, 1.8 us of a 8.6 us kernel
 // at eight rows).  `a_add` (kernels built with ADD): the left operand is A + a_add, A in fp32,
@@ -798,19 +778,6 @@ int launch_one(const void* A, const bf16_t* W, void* C, int M, int N, int K, int
                        lda, ldc, m_base, eps, w_tiled, rd, rp, pk);
   }
   return kvf_last_error();
-}
-
-// Compute units of the current device, asked once per device.
-int compute_units() {
-  static int known[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (known[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    known[dev] = n;
-  }
-  return known[dev];
 }
 
 // How 17 to 64 rows are cut: groups of columns a workgroup and cuts of K.  The rule takes the least

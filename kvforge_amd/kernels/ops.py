@@ -1108,35 +1108,31 @@ def gemm_fused(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rms_eps: flo
           float(rms_eps or 0.0), None, None, _stream()), "gemm_bf16")
 
 
-def gemm_qkv_rope(a: torch.Tensor, w: torch.Tensor, q_out: torch.Tensor, positions: torch.Tensor,
-                  seq_of_token: torch.Tensor, cos: torch.Tensor | None, sin: torch.Tensor | None,
-                  block_table: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
-                  num_heads: int, num_kv_heads: int, head_dim: int, write_kv: bool = True,
-                  rms_eps: float | None = None, a_owed: torch.Tensor | None = None,
-                  extra_cols: int = 0) -> None:
-    """Fused q/k/v projection: ``a @ w.T`` with rotary applied to q and k (neighbouring columns
-    are pairs), rotated q stored to ``q_out [M, H*d]`` and rotated k and v written into the
-    pages; without tables (``None``) nothing is rotated.  ``rms_eps`` as in ``gemm_fused``.  ``a_owed`` (with ``rms_eps``; bf16, shape and
-    strides, counted in elements, of ``a``): a sum still owed to ``a``; the projection is taken of ``a + a_owed``, and
-    ``a`` itself is left as it is.  ``extra_cols``: so many further rows of ``w`` behind q, k and v
-    (an output gate, say), whose columns of the product are stored behind q, ``q_out [M, H*d +
-    extra_cols]``; ``num_kv_heads`` may then be 0 for a projection without keys and values."""
-    H, KV, d = num_heads, num_kv_heads, head_dim
-    extra = int(extra_cols)
+@lru_cache(maxsize=4096)
+def _qkv_tiles_take(m: int, n: int, k: int, rot: int, device: int) -> bool:
+    with torch.cuda.device(device):
+        return bool(_fn("gemm_tile", "kvf_gemm_tile_qkv_takes", [c_int] * 4)(m, n, k, rot))
+
+
+def qkv_tiles_take(a: torch.Tensor, w, rot: int) -> bool:
+    """Whether ``gemm_qkv_rope_tiles`` is to take ``a @ w.T``: more rows
+    than the weight-streaming kernel's epilogue pays for, tiled bf16 weights, K in whole steps of 64, a rotary width ``rot``
+    in whole 8s up to 128, and a size at which it is
+    no slower than a product of its own and ``rope_kvwrite``.  Both give the same bits."""
+    m, k = a.shape
+    return (m > FUSED_EPILOGUE_MAX_M and isinstance(w, StreamedWeight) and a.dtype == BF16 and a.is_cuda
+            and k % 64 == 0 and a.stride(1) == 1 and _rows_aligned(a, k, a.stride(0))
+            and _qkv_tiles_take(m, w.shape[0], k, rot, a.device.index or 0))
+
+
+def _qkv_rope_args(a, w, q_out, positions, seq_of_token, cos, sin, block_table, k_pages, v_pages, H: int, KV: int, d: int,
+                   write_kv: bool, extra: int) -> tuple:
+    """Checks what both forms of the fused projection take; their arguments behind the product's."""
+    m, k = a.shape
     if extra < 0 or extra % 4:
         raise KernelError(f"gemm_qkv_rope: extra_cols must be a non-negative multiple of 4, got {extra}")
-    rms = rms_eps is not None
-    m, k = a.shape
     _check(a, "a", None, (m, k), contiguous=False)
     _check(plain_of(w), "w", BF16, ((H + 2 * KV) * d + extra, k))
-    if not bf16_kernel_takes(a, w, rms, True) or a.stride(1) != 1:
-        raise KernelError("gemm_qkv_rope: operands do not fit the MFMA kernel")
-    if a_owed is not None:
-        if not rms or m > FUSED_NORM_MAX_M:
-            raise KernelError("gemm_qkv_rope: a_owed goes with rms_eps (fp32 rows, one tile of them)")
-        _check(a_owed, "a_owed", BF16, (m, k), contiguous=False)
-        if a_owed.stride() != a.stride():
-            raise KernelError("gemm_qkv_rope: a_owed must have the strides of a")
     _check(q_out, "q_out", BF16, (m, H * d + extra))
     _check(positions, "positions", I32, (None,))
     _check(seq_of_token, "seq_of_token", I32, (None,))
@@ -1151,6 +1147,37 @@ def gemm_qkv_rope(a: torch.Tensor, w: torch.Tensor, q_out: torch.Tensor, positio
     _check(k_pages, "k_pages", BF16, (None, KV if KV else None, None, d))
     nb, _, bs, _ = k_pages.shape
     _check(v_pages, "v_pages", BF16, (nb, k_pages.shape[1], d, bs))
+    return (positions.data_ptr(), seq_of_token.data_ptr(), cos_p, sin_p, block_table.data_ptr(), k_pages.data_ptr(),
+            v_pages.data_ptr(), H, KV, d, rot, table_len, bs, block_table.shape[1], nb, 1 if write_kv else 0,
+            block_table.shape[0], extra)
+
+
+def gemm_qkv_rope(a: torch.Tensor, w: torch.Tensor, q_out: torch.Tensor, positions: torch.Tensor,
+                  seq_of_token: torch.Tensor, cos: torch.Tensor | None, sin: torch.Tensor | None,
+                  block_table: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
+                  num_heads: int, num_kv_heads: int, head_dim: int, write_kv: bool = True,
+                  rms_eps: float | None = None, a_owed: torch.Tensor | None = None,
+                  extra_cols: int = 0) -> None:
+    """Fused q/k/v projection (few rows): ``a @ w.T`` with rotary applied to q and k (neighbouring columns
+    are pairs), rotated q stored to ``q_out [M, H*d]`` and rotated k and v written into the
+    pages; without tables (``None``) nothing is rotated.  ``rms_eps`` as in ``gemm_fused``.  ``a_owed`` (with ``rms_eps``; bf16, shape and
+    strides, counted in elements, of ``a``): a sum still owed to ``a``; the projection is taken of ``a + a_owed``, and
+    ``a`` itself is left as it is.  ``extra_cols``: so many further rows of ``w`` behind q, k and v
+    (an output gate, say), whose columns of the product are stored behind q, ``q_out [M, H*d +
+    extra_cols]``; ``num_kv_heads`` may then be 0 for a projection without keys and values."""
+    H, KV, d = num_heads, num_kv_heads, head_dim
+    rms = rms_eps is not None
+    m, k = a.shape
+    rest = _qkv_rope_args(a, w, q_out, positions, seq_of_token, cos, sin, block_table, k_pages, v_pages, H, KV, d, write_kv,
+                          int(extra_cols))
+    if not bf16_kernel_takes(a, w, rms, True) or a.stride(1) != 1:
+        raise KernelError("gemm_qkv_rope: operands do not fit the MFMA kernel")
+    if a_owed is not None:
+        if not rms or m > FUSED_NORM_MAX_M:
+            raise KernelError("gemm_qkv_rope: a_owed goes with rms_eps (fp32 rows, one tile of them)")
+        _check(a_owed, "a_owed", BF16, (m, k), contiguous=False)
+        if a_owed.stride() != a.stride():
+            raise KernelError("gemm_qkv_rope: a_owed must have the strides of a")
     if m == 0:
         return
     f = _fn("gemm_bf16", "kvf_gemm_bf16_qkv_rope",
@@ -1158,11 +1185,33 @@ def gemm_qkv_rope(a: torch.Tensor, w: torch.Tensor, q_out: torch.Tensor, positio
             + [c_void_p] * 8 + [c_int] * 11 + [c_void_p])
     wp, tiled = _w_args(w)
     _ok(f(a.data_ptr(), 1 if rms else 0, wp, tiled, q_out.data_ptr(), m, k,
-          a.stride(0) if m > 1 else k, q_out.stride(0) if m > 1 else H * d + extra, float(rms_eps or 0.0),
-          a_owed.data_ptr() if a_owed is not None else None, positions.data_ptr(), seq_of_token.data_ptr(), cos_p, sin_p,
-          block_table.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), H, KV, d, rot,
-          table_len, bs, block_table.shape[1], nb, 1 if write_kv else 0, block_table.shape[0],
-          extra, _stream()), "gemm_qkv_rope")
+          a.stride(0) if m > 1 else k, q_out.stride(0) if m > 1 else q_out.shape[1], float(rms_eps or 0.0),
+          a_owed.data_ptr() if a_owed is not None else None, *rest, _stream()), "gemm_qkv_rope")
+
+
+QKV_TILES = 6    # tiles of gemm_qkv_rope_tiles
+
+
+def gemm_qkv_rope_tiles(a: torch.Tensor, w: "StreamedWeight", q_out: torch.Tensor, positions: torch.Tensor,
+                        seq_of_token: torch.Tensor, cos: torch.Tensor | None, sin: torch.Tensor | None,
+                        block_table: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
+                        num_heads: int, num_kv_heads: int, head_dim: int, write_kv: bool = True,
+                        extra_cols: int = 0, tile: int = -1) -> None:
+    """``gemm_qkv_rope`` for many rows of bf16 over tiled weights, with the product rounded to bf16 before it is rotated:
+    the bits of ``gemm`` and ``rope_kvwrite``.  K in whole steps of 64, a
+    rotary width in whole 8s up to 128.  ``tile``: which of its ``QKV_TILES`` tiles of rows and columns
+    is taken (-1: by size)."""
+    m, k = a.shape
+    rest = _qkv_rope_args(a, w, q_out, positions, seq_of_token, cos, sin, block_table, k_pages, v_pages, num_heads,
+                          num_kv_heads, head_dim, write_kv, int(extra_cols))
+    if not (isinstance(w, StreamedWeight) and a.dtype == BF16 and k % 64 == 0 and a.stride(1) == 1
+            and _rows_aligned(a, k, a.stride(0) if m > 1 else k) and -1 <= tile < QKV_TILES):
+        raise KernelError("gemm_qkv_rope_tiles: operands do not fit the kernel")
+    if m == 0:
+        return
+    f = _fn("gemm_tile", "kvf_gemm_tile_qkv_rope", [c_void_p] * 3 + [c_int] * 4 + [c_void_p] * 7 + [c_int] * 12 + [c_void_p])
+    _ok(f(a.data_ptr(), w.tiles.data_ptr(), q_out.data_ptr(), m, k, a.stride(0) if m > 1 else k,
+          q_out.stride(0) if m > 1 else q_out.shape[1], *rest, tile, _stream()), "gemm_qkv_rope_tiles")
 
 
 def pick_workspace(rows: int, n: int, device) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:

@@ -387,7 +387,7 @@ class PagedAttention(Mixer):
         if self.conv is not None:
             mods.add("convkv")
         if dtype == torch.bfloat16:
-            mods |= {"gemm_bf16", "attn_mfma"}
+            mods |= {"gemm_bf16", "gemm_tile", "attn_mfma"}
         return mods
 
     def num_bytes(self) -> int:
@@ -507,9 +507,11 @@ class PagedAttention(Mixer):
             normed = ws.buf("normed", (n, self.hidden), act)
             ops.rmsnorm(x, None, rms, normed, add=step.take_owed(residual, parts=True))
             x, rms = normed, None
-        fused = (not self._hooked() and self.qk_norm is None and self.row_norm is None and self.conv is None
-                 and ops.bf16_kernel_takes(x, self.w_qkv, rms is not None, True)
-                 and layer.k_pages.dtype == torch.bfloat16)
+        plain_qkv = (not self._hooked() and self.qk_norm is None and self.row_norm is None and self.conv is None
+                     and layer.k_pages.dtype == torch.bfloat16)
+        fused = plain_qkv and ops.bf16_kernel_takes(x, self.w_qkv, rms is not None, True)
+        in_tiles = (plain_qkv and not fused and rms is None
+                    and ops.qkv_tiles_take(x, self.w_qkv, 2 * cos.shape[1] if cos is not None else 0))
         if fused and rms is not None:
             # what the layer before owes the stream rides in this projection's loads and is
             # added to the stream by the output projection
@@ -520,14 +522,16 @@ class PagedAttention(Mixer):
         else:
             step.settle()
         g0 = H * d     # where the gate's columns begin in a row of qkv
-        if fused:
+        if fused or in_tiles:
             # one kernel: (norm,) projection, rotary, cache write; a gate's columns land behind q
             extra = H * d if self.gated else 0
             qkv = ws.buf("q_rot", (n, H * d + extra), act)
-            ops.gemm_qkv_rope(x, self.w_qkv, qkv, step.positions, step.seq_of_token, cos, sin, table,
-                              layer.k_pages, layer.v_pages, H, KV if self.own_kv else 0, d,
-                              write_kv=layer.owns_cache and self.own_kv, rms_eps=rms, a_owed=owed,
-                              extra_cols=extra)
+            args = (x, self.w_qkv, qkv, step.positions, step.seq_of_token, cos, sin, table, layer.k_pages, layer.v_pages, H,
+                    KV if self.own_kv else 0, d, layer.owns_cache and self.own_kv)
+            if in_tiles:
+                ops.gemm_qkv_rope_tiles(*args, extra_cols=extra)
+            else:
+                ops.gemm_qkv_rope(*args, rms_eps=rms, a_owed=owed, extra_cols=extra)
         elif self.conv is not None:
             if layer.state is None and self.conv[0] > 1:
                 raise RuntimeError("attention behind a convolution needs a state slot per request")

@@ -586,6 +586,58 @@ def test_gemm_qkv_rope_equals_the_three_steps(m, H, KV, d, rot, bs, rms):
         assert all(torch.equal(x1, x2) for x1, x2 in zip(*got))
 
 
+@pytest.mark.parametrize("tile", range(6))
+@pytest.mark.parametrize("m,k,H,KV,d,rot,bs,extra", [
+    (65, 64, 4, 2, 16, 16, 8, 0),          # one stage of K; fewer columns than a tile
+    (129, 128, 3, 1, 40, 32, 4, 24),       # heads across the 16s, columns behind q, k and v, a row past a tile
+    (193, 192, 5, 0, 48, 0, 16, 16),       # neither keys nor rotation
+    (320, 448, 32, 8, 64, 64, 16, 0),      # whole tiles
+    (257, 1088, 12, 4, 64, 32, 16, 8)])
+def test_gemm_qkv_rope_tiles_has_the_bits_of_the_three_steps(tile, m, k, H, KV, d, rot, bs, extra):
+    """The fused projection of many rows against a product summed along K in order (the streaming kernel on one wave)
+    and ``rope_kvwrite``: the same bits, for every tile, with rows of ``a`` further apart than K, positions off the tables
+    and pages that were given back."""
+    g = torch.Generator().manual_seed(m + d)
+    wide = torch.randn(m, k + 8, generator=g)
+    wide[3, 5], wide[m - 1, 0] = float("inf"), float("nan")      # they stay in their rows
+    a = wide.to(torch.bfloat16).to(DEV)[:, :k]
+    n = (H + 2 * KV) * d + extra
+    w = ops().StreamedWeight((torch.randn(n, k, generator=g) / 6).to(torch.bfloat16).to(DEV))
+    nb, cap = 3 * 60, 60
+    at = torch.randperm(3 * (cap * bs - 4), generator=g)[:m]     # no two tokens at one place
+    seq_of, positions = (at % 3).to(torch.int32).to(DEV), (at // 3).to(torch.int32).to(DEV)
+    positions[1], positions[2] = -1, 100000
+    seq_of[5] = -1
+    table = torch.randperm(nb, generator=g).reshape(3, cap).to(torch.int32)
+    table[1, 2], table[2, 3] = -1, nb + 7
+    table = table.to(DEV)
+    cos = sin = None
+    if rot:
+        cos_full, sin_full = plain.rope_cos_sin(torch.arange(cap * bs - 9), plain.rope_inv_freq(rot, 10000.0))
+        cos, sin = (t[:, :rot // 2].contiguous().to(DEV) for t in (cos_full, sin_full))
+    rows = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    f = ops()._fn("gemm_bf16", "kvf_gemm_bf16", ops()._GEMM_BF16_ARGS)
+    ops().set_gemm_waves(1)
+    try:
+        assert f(a.data_ptr(), 0, w.tiles.data_ptr(), 1, rows.data_ptr(), 1, m, n, k, a.stride(0), n, 0.0, None, None,
+                 ops()._stream()) == 0
+    finally:
+        ops().set_gemm_waves(0)
+    heads = max(KV, 1)
+    pages = [torch.zeros(nb, heads, *s, dtype=torch.bfloat16, device=DEV) for s in 2 * ((bs, d), (d, bs))]
+    q = torch.empty(m, H * d + extra, dtype=torch.bfloat16, device=DEV)
+    args = (positions, seq_of, cos, sin, table)
+    ops().gemm_qkv_rope_tiles(a, w, q, *args, pages[0], pages[1], H, KV, d, write_kv=KV > 0, extra_cols=extra, tile=tile)
+    if KV:
+        ops().rope_kvwrite(rows, *args, pages[2], pages[3], H, KV, d)
+    want = torch.cat([rows[:, :H * d], rows[:, (H + 2 * KV) * d:]], 1)
+
+    def same(x, y):
+        return torch.equal(torch.nan_to_num(x, nan=123.0), torch.nan_to_num(y, nan=123.0))
+    assert same(q, want) and same(pages[0], pages[2]) and same(pages[1], pages[3])
+    assert not KV or pages[0].count_nonzero() > 0
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,KV,d,bs", [(4, 2, 16, 4), (3, 1, 40, 8), (32, 8, 64, 16)])
 @pytest.mark.parametrize("m", [1, 7, 48])
