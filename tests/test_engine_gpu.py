@@ -1066,3 +1066,49 @@ def test_float32_steps_on_both_sides_of_the_streaming_kernels_row_limit(model_a)
     assert [len(o.output_token_ids) for o in outs] == [p.max_tokens for p in params]
     for i in range(0, 40, 3):
         oracle.check_choices(prompts[i], outs[i].output_token_ids, 1e-4)
+
+
+@pytest.mark.parametrize("kept", [1, 16])
+@pytest.mark.parametrize("kind", ["float32", "bfloat16", "state"])
+def test_steps_of_single_tokens_give_the_bits_of_eager_ones(kind, kept, monkeypatch):
+    """``ModelRunner.step`` replays steps of single tokens that come again from a graph: the logits are those of a runner
+    that launches every step, bit for bit, over batches that change, contexts that grow into other pages, longer steps
+    between them that make the workspace grow, and graphs that are dropped for others."""
+    from kvforge_amd import ModelRunner, StepEntry, Transformer
+    from kvforge_amd.config.presets import rudorax_stack
+    from kvforge_amd.engine import runner as runner_module
+    monkeypatch.setattr(runner_module, "STEP_GRAPHS", kept)
+    if kind == "state":
+        cfg = rudorax_stack(vocab=300, width=128, pairs=1, heads=4, kv_heads=2, dim=32, window=24, lstm_heads=2, lstm_dim=32,
+                            lstm_vdim=32, ff=64, experts=4, top=2, identity=1, shared_ff=64, max_positions=512)
+        vocab, dtype = 300, torch.bfloat16
+    else:
+        cfg = kvforge_amd.preset_dict("tiny-b")
+        vocab, dtype = cfg["vocab_size"], getattr(torch, kind)
+    runners = [ModelRunner(Transformer.from_random(cfg, 3, dtype, "cuda"), 8, 128, max_num_seqs=8, max_num_batched_tokens=96,
+                           max_model_len=128, use_graphs=graphs) for graphs in (True, False)]
+    g = random.Random(kept)
+    lens = [g.randint(3, 30) for _ in range(5)]
+    at = list(lens)
+    for i, n in enumerate(lens):
+        ids = [g.randrange(1, vocab) for _ in range(n)]
+        for r in runners:
+            r.cache.allocate(f"r{i}", n + 60)
+            r.step([StepEntry(f"r{i}", ids, 0, "none")])
+    for turn in range(24):
+        batch = [range(5), range(3), [4]][turn // 2 % 3]
+        entries = [StepEntry(f"r{i}", [g.randrange(1, vocab)], at[i], "last") for i in batch]
+        for i in batch:
+            at[i] += 1
+        got, want = (r.step(entries).clone() for r in runners)
+        assert torch.equal(got, want), turn
+        if turn % 7 == 3:          # eager work between replays, longer every time
+            ids = [g.randrange(1, vocab) for _ in range(10 + 3 * turn)]
+            for r in runners:
+                r.cache.allocate("long", len(ids))
+            got, want = (r.step([StepEntry("long", ids, 0, "last")]).clone() for r in runners)
+            assert torch.equal(got, want)
+            for r in runners:
+                r.cache.free("long")
+    assert runners[0].num_graph_replays >= 6 and len(runners[0].step_graphs) <= kept
+    assert runners[1].num_graph_replays == 0 and not runners[1].step_graphs
