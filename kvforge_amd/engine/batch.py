@@ -136,7 +136,8 @@ class MetaBuffers:
         self.max_tokens, self.max_seqs, self.table_widths = max_tokens, max_seqs, list(table_widths)
         off = 0
         self.off: dict[str, int] = {}
-        for name, size in (("cu_q", max_seqs + 1), ("ctx_lens", max_seqs), ("slot_ids", max_seqs),
+        # ("run_counter" is zero in the staging memory: every batch that is sent begins a run's count anew)
+        for name, size in (("run_counter", 1), ("cu_q", max_seqs + 1), ("ctx_lens", max_seqs), ("slot_ids", max_seqs),
                            ("decode_seq_ids", max_seqs), ("token_ids", max_tokens),
                            ("positions", max_tokens), ("seq_of_token", max_tokens),
                            ("logits_rows", max_tokens)):
@@ -161,15 +162,25 @@ class MetaBuffers:
         # step before (a request that keeps its row only appends pages)
         self.table_host = [np.full((max_seqs, w), -1, dtype=np.int32) for w in self.table_widths]
         self.row_owner: list[list[tuple | None]] = [[None] * max_seqs for _ in self.table_widths]
-        self.row_filled = [np.zeros(max_seqs, dtype=np.int64) for _ in self.table_widths]
+        self.row_filled = [[0] * max_seqs for _ in self.table_widths]
+        self.counting = np.arange(max(max_tokens, max_seqs + 1), dtype=np.int32)
+        self._views: dict[tuple, torch.Tensor] = {}   # of the one buffer, by name and length
 
     def view(self, name: str, n: int) -> torch.Tensor:
-        o = self.off[name]
-        return self.device_buf[o:o + n]
+        v = self._views.get((name, n))
+        if v is None:
+            o = self.off[name]
+            v = self.device_buf[o:o + n]
+            if len(self._views) < 4096:
+                self._views[name, n] = v
+        return v
 
-    def table_view(self, g: int) -> torch.Tensor:
-        o, w = self.table_off[g], self.table_widths[g]
-        return self.device_buf[o:o + self.max_seqs * w].view(self.max_seqs, w)
+    def table_view(self, g: int, rows: int) -> torch.Tensor:
+        v = self._views.get((g, rows))
+        if v is None:
+            o, w = self.table_off[g], self.table_widths[g]
+            v = self._views[g, rows] = self.device_buf[o:o + rows * w].view(rows, w)
+        return v
 
 
 class Step:
@@ -319,7 +330,7 @@ def _fill_tables(meta: "MetaBuffers", host: np.ndarray, entries: Sequence[StepEn
             if need > w or need > len(t):
                 raise ValueError(f"request {e.request_id} needs {need} pages in group {g}; "
                                  f"table holds {len(t)}, width {w}")
-            have = int(filled[b])
+            have = filled[b]
             tag = (e.request_id, serial_of(e.request_id)) if serial_of is not None else None
             if tag is not None and owner[b] == tag and have <= need and not windowed:
                 if have < need:
@@ -331,7 +342,7 @@ def _fill_tables(meta: "MetaBuffers", host: np.ndarray, entries: Sequence[StepEn
             filled[b] = need
         for b in range(B, Bp):
             if filled[b]:
-                mirror[b, :int(filled[b])] = -1
+                mirror[b, :filled[b]] = -1
             owner[b], filled[b] = None, 0
         host[to:to + Bp * w].reshape(Bp, w)[:] = mirror[:Bp]
         end = to + Bp * w
@@ -391,10 +402,19 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     host = meta.staging_np[turn]
     off = meta.off
 
-    lens = np.asarray(q_lens + [1] * (Bp - B), dtype=np.int32)
-    starts = np.asarray([e.start_pos for e in entries] + [0] * (Bp - B), dtype=np.int32)
-    cu = np.zeros(Bp + 1, dtype=np.int32)
-    np.cumsum(lens, out=cu[1:])
+    singles = max(q_lens) == 1      # one token each, padding too: token b belongs to sequence b
+    count = meta.counting
+    if singles:
+        lens_of = [1] * Bp
+        lens, cu = 1, count[:Bp + 1]
+        starts = np.array([e.start_pos for e in entries] + [0] * (Bp - B), dtype=np.int32)
+        starts_of = starts.tolist()
+    else:
+        lens = np.asarray(q_lens + [1] * (Bp - B), dtype=np.int32)
+        starts = np.asarray([e.start_pos for e in entries] + [0] * (Bp - B), dtype=np.int32)
+        lens_of, starts_of = lens.tolist(), starts.tolist()
+        cu = np.zeros(Bp + 1, dtype=np.int32)
+        np.cumsum(lens, out=cu[1:])
     host[off["cu_q"]:off["cu_q"] + Bp + 1] = cu
     ctx = starts + lens
     ctx[B:] = 0  # padding sequences hold nothing
@@ -403,20 +423,31 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     host[off["slot_ids"]:off["slot_ids"] + Bp] = slots
     tok = host[off["token_ids"]:off["token_ids"] + N]
     pos = host[off["positions"]:off["positions"] + N]
-    p = 0
-    for e, n, s in zip(entries, q_lens, starts[:B]):
-        tok[p:p + n] = e.token_ids
-        pos[p:p + n] = np.arange(s, s + n, dtype=np.int32)
-        p += n
-    tok[p:] = 0
-    pos[p:] = 0
-    host[off["seq_of_token"]:off["seq_of_token"] + N] = np.repeat(np.arange(Bp, dtype=np.int32), lens)
+    if singles:
+        tok[:B] = [e.token_ids[0] for e in entries]
+        tok[B:] = 0
+        pos[:] = starts
+        host[off["seq_of_token"]:off["seq_of_token"] + N] = count[:Bp]
+    else:
+        p = 0
+        for e, n, s in zip(entries, q_lens, starts_of):
+            tok[p:p + n] = e.token_ids
+            pos[p:p + n] = np.arange(s, s + n, dtype=np.int32)
+            p += n
+        tok[p:] = 0
+        pos[p:] = 0
+        host[off["seq_of_token"]:off["seq_of_token"] + N] = np.repeat(count[:Bp], lens)
 
     counts, rows = [], []
     for b, e in enumerate(entries):
+        if singles and e.want == "last":
+            counts.append(1)
+            rows.append(b)
+            continue
         w = e.wanted()
         counts.append(len(w))
-        rows.extend(int(cu[b]) + i for i in w)
+        first = int(cu[b])
+        rows.extend(first + i for i in w)
     if pad_to is not None:
         # a padded batch has a fixed shape: one wanted row per sequence, padding included
         if any(c != 1 for c in counts) or any(n != 1 for n in q_lens):
@@ -426,14 +457,15 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     host[off["logits_rows"]:off["logits_rows"] + R] = rows
 
     # longest context first, so that kernels which take them in this order start what lasts longest first
-    decode = [b for b, n in enumerate(q_lens) if n == 1] + list(range(B, Bp))
+    ctx_of = ctx.tolist()
+    decode = list(range(Bp)) if singles else [b for b, n in enumerate(q_lens) if n == 1] + list(range(B, Bp))
     if len(decode) > 1:
-        decode.sort(key=ctx.tolist().__getitem__, reverse=True)
-    prefill = [b for b, n in enumerate(q_lens) if n > 1]
+        decode.sort(key=ctx_of.__getitem__, reverse=True)
+    prefill = [] if singles else [b for b, n in enumerate(q_lens) if n > 1]
     host[off["decode_seq_ids"]:off["decode_seq_ids"] + len(decode)] = decode
 
     end = off["logits_rows"] + max(R, 1)
-    need_tokens = [int(ctx[b]) + lookahead for b in range(B)]
+    need_tokens = [c + lookahead for c in ctx_of[:B]]
     end = max(end, _fill_tables(meta, host, entries, Bp, need_tokens, tables_of, block_size,
                                 windowed_groups, serial_of))
     meta.device_buf[:end].copy_(meta.staging[turn][:end], non_blocking=True)
@@ -452,16 +484,16 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
     step.logits_rows = meta.view("logits_rows", max(R, 1))[:R]
     step.decode_seq_ids = None if len(decode) == Bp else meta.view("decode_seq_ids", len(decode))
     step.decode_order = meta.view("decode_seq_ids", Bp) if len(decode) == Bp > 1 else None
-    step.block_tables = [meta.table_view(g)[:Bp] for g in range(len(meta.table_widths))]
+    step.block_tables = [meta.table_view(g, Bp) for g in range(len(meta.table_widths))]
     step.request_ids = [e.request_id for e in entries]
-    step.q_lens = [int(x) for x in lens]
-    step.start_pos = [int(x) for x in starts]
+    step.q_lens = lens_of
+    step.start_pos = starts_of
     step.host_slot_ids = slots
     step.host_token_ids = tok.copy()
     step.prefill_seqs = prefill
-    live = [int(ctx[b]) for b in decode if ctx[b] > 0]
+    live = [ctx_of[b] for b in decode if ctx_of[b] > 0]
     step.decode_shape = DecodeShape(len(live), max(live, default=0), sum(live))
-    step.max_position = int(ctx.max()) if Bp else 0
+    step.max_position = max(ctx_of)
     step.scratch = {}
     step._meta, step._turn, step._extra_used = meta, turn, 0
     return counts

@@ -19,7 +19,7 @@ from kvforge_amd.cache.storage import PagedStorage, StateStorage, bytes_per_bloc
 from kvforge_amd.engine.batch import (DecodeShape, DecodeTail, MetaBuffers, Step, StepEntry,
                                       Workspace, extend_tables, fill_step)
 from kvforge_amd.kernels import ops
-from kvforge_amd.sampling.rng import uniform
+from kvforge_amd.sampling.rng import uniforms
 from kvforge_amd.kernels import library
 from kvforge_amd.models.transformer import Transformer
 
@@ -71,7 +71,7 @@ class ModelRunner:
         nf = (2 + MAX_DECODE_RUN) * cap
         self._sample_f = torch.zeros(nf, dtype=torch.float32, device=self.device)
         self._sample_i = torch.zeros(2 * cap, dtype=torch.int32, device=self.device)
-        self._run_counter = torch.zeros(1, dtype=torch.int32, device=self.device)
+        self._run_counter = self.meta.view("run_counter", 1)     # zero behind every batch that is sent
         # tickets and chunk results of greedy rows read by several workgroups (zero between launches)
         self._sample_work = torch.zeros(ops.sample_work_size(cap), dtype=torch.int32, device=self.device)
         self._run_ring = torch.zeros(MAX_DECODE_RUN, cap, dtype=torch.int32, device=self.device)
@@ -289,12 +289,9 @@ class ModelRunner:
             dirty = True
         else:
             dirty = bool(self._sample_drawn)
-        for i in self._sample_drawn:
-            for j in range(k):
-                fh[(2 + j) * cap + i] = uniform(seed, streams[i], counters[i] + j)
+        self._put_uniforms(seed, streams, counters, k, 2)
         if dirty:
             self._sample_f.copy_(self._sample_f_host, non_blocking=True)
-        self._run_counter.zero_()
         greedy = self._tail is not None and not self._sample_drawn and self.model.can_pick(bucket)
         key = (bucket, launch_key, greedy)
         graph = self.graphs.get(key)
@@ -310,6 +307,15 @@ class ModelRunner:
         for _ in range(replays):
             graph.graph.replay()
         return self._queue_read(ids, [e.start_pos for e in entries], k, 0, bucket, replays, greedy)
+
+    def _put_uniforms(self, seed, streams, counters, k: int, row: int) -> None:
+        """The numbers that the drawn rows of ``k`` steps take, into the host's rows ``row ..``."""
+        drawn, cap = self._sample_drawn, self.meta.max_seqs
+        if not drawn:
+            return
+        s, c = [streams[i] for i in drawn], [counters[i] for i in drawn]
+        for j in range(k):
+            self._sample_f_np[(row + j) * cap:(row + j + 1) * cap][drawn] = uniforms(seed, s, [x + j for x in c])
 
     def _queue_read(self, ids, begins, k: int, base: int, bucket: int, replays: int,
                     greedy: bool = False) -> "_QueuedRun":
@@ -341,11 +347,8 @@ class ModelRunner:
         extend_tables(self.meta, entries, run.bucket, [s + k for s in starts], self.cache.block_table,
                       self.block_size, self._windowed, self.cache.serial)
         if self._sample_drawn:
-            fh = self._sample_f_np
             lo = (2 + base) * cap
-            for i in self._sample_drawn:
-                for j in range(k):
-                    fh[lo + j * cap + i] = uniform(seed, streams[i], counters[i] + k + j)
+            self._put_uniforms(seed, streams, [c + k for c in counters], k, 2 + base)
             self._sample_f[lo:lo + k * cap].copy_(self._sample_f_host[lo:lo + k * cap], non_blocking=True)
         if base == 0:
             self._run_counter.zero_()

@@ -3,6 +3,9 @@ tests/test_continuous_batching.py:27-39, padding, and what is refused."""
 
 from __future__ import annotations
 
+import random
+
+import numpy as np
 import pytest
 import torch
 
@@ -235,3 +238,46 @@ def test_prefill_work_rows_hold_every_item_once_longest_walk_first():
         assert sorted((b, i) for b, i, _ in rows) == want
         ends = [start[b] + min(q_lens[b], -(-(i + 1) * per_item // group)) for b, i, _ in rows]
         assert ends == sorted(ends, reverse=True)
+
+
+@pytest.mark.parametrize("count,padded,lookahead", [(1, None, 0), (1, 4, 2), (5, None, 0), (5, 8, 3), (7, 7, 0)])
+def test_batches_of_single_tokens_hold_what_any_batch_does(count, padded, lookahead):
+    """A batch of one token each is filled without going through its entries' lengths: every field against
+    its meaning, sent twice (the second time the requests have moved on, one of them into its next page)."""
+    block, width = 4, 12
+    tables = {f"r{i}": [100 * i + p for p in range(width)] for i in range(count)}
+    meta = MetaBuffers(32, 8, [width], "cpu")
+    for turn in range(2):
+        at = [(3 * i) % 11 + turn for i in range(count)]
+        entries = [StepEntry(f"r{i}", [50 + i], at[i], "last" if i % 2 else [0]) for i in range(count)]
+        step = Step()
+        counts = fill_step(step, meta, entries, lambda r, g: tables[r], lambda r: int(r[1:]) + 1, block, padded, [False],
+                           lambda r: 0, lookahead)
+        n = padded or count
+        ctx = [a + 1 for a in at] + [0] * (n - count)
+        assert counts == [1] * count and (step.n_tokens, step.n_seqs, step.n_logits, step.n_decode) == (n, n, n, n)
+        assert step.token_ids.tolist() == [50 + i for i in range(count)] + [0] * (n - count)
+        assert step.positions.tolist() == at + [0] * (n - count) and step.start_pos == at + [0] * (n - count)
+        assert step.seq_of_token.tolist() == step.logits_rows.tolist() == list(range(n)) and step.q_lens == [1] * n
+        assert step.cu_q.tolist() == list(range(n + 1)) and step.ctx_lens.tolist() == ctx
+        assert step.slot_ids.tolist() == step.host_slot_ids == [i + 1 for i in range(count)] + [-1] * (n - count)
+        order = sorted(range(n), key=lambda b: -ctx[b])
+        assert step.decode_order is None if n == 1 else step.decode_order.tolist() == order
+        assert step.decode_seq_ids is None and step.prefill_seqs == [] and step.max_position == max(ctx)
+        assert (step.decode_shape.n, step.decode_shape.max_ctx, step.decode_shape.sum_ctx) == (count, max(ctx), sum(ctx))
+        for b in range(n):
+            need = -(-(ctx[b] + lookahead) // block) if b < count else 0
+            assert step.block_tables[0][b].tolist() == (tables[f"r{b}"][:need] if b < count else []) + [-1] * (width - need)
+        assert meta.view("run_counter", 1).tolist() == [0]
+        meta.view("run_counter", 1).fill_(9)          # a run has counted: the next batch begins anew
+
+
+@pytest.mark.parametrize("count", [0, 1, 15, 16, 41])
+def test_uniform_numbers_of_a_batch_are_those_of_its_rows(count):
+    from kvforge_amd.sampling.rng import uniform, uniforms
+    g = random.Random(count)
+    for seed in (0, -5, 2 ** 64 - 1, 2 ** 70 + 3):
+        streams = [g.choice([0, -1, 2 ** 63, 2 ** 64 - 1, g.randrange(2 ** 64)]) for _ in range(count)]
+        counters = [g.choice([0, 1, 2 ** 40, g.randrange(1000)]) for _ in range(count)]
+        got = uniforms(seed, streams, counters)
+        assert got.dtype == np.float32 and got.tolist() == [uniform(seed, s, c) for s, c in zip(streams, counters)]
