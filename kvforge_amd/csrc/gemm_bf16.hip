@@ -741,6 +741,67 @@ __global__ __launch_bounds__(MID_WAVES * KVF_WAVE, 4) void gemm_mid_kernel(
   }
 }
 
+// Several products of at most 16 bf16 rows over tiled weights in one launch (EPI 0, 1 or 3 each, inputs of their own):
+// the projections that a step's parts begin with.  In a decode step each is a kernel of 4 to 7 us whose time is its
+// launch and two trips to memory; together those come once.  Eight rows of 2,048, a recurrence's rows, its gates, a router
+// and a gated pair of 4,096 columns: 7.0 + 4.6 + 4.6 + 6.0 us apart, 9.7 together.  A workgroup takes 16 columns of one product as gemm_skinny_kernel<1, 1, 0,
+// EPI> on eight waves does, with the same sums in the same order, so that the results are the same to the bit.
+struct GroupItem {
+  const bf16_t* A;
+  const bf16_t* W;
+  void* C;
+  int N, K, lda, ldc, epi, first;   // first: its first workgroup
+};
+constexpr int GROUP_MAX = 8, GROUP_WAVES = 8;
+struct Group {
+  GroupItem item[GROUP_MAX];
+  int count;
+};
+
+__global__ __launch_bounds__(GROUP_WAVES * KVF_WAVE) void gemm_group_kernel(Group group, int M, RopeEpi rp) {
+  __shared__ __attribute__((aligned(16))) float red[GROUP_WAVES * KVF_WAVE * 4];
+  int which = 0;
+  for (int i = 1; i < group.count; ++i)
+    if (static_cast<int>(blockIdx.x) >= group.item[i].first) which = i;   // the same for the whole workgroup
+  const GroupItem it = group.item[which];
+  const int lane = threadIdx.x % KVF_WAVE, wave = threadIdx.x / KVF_WAVE, r16 = lane % 16, kg = lane / 16;
+  const int grp = blockIdx.x - it.first, n0 = grp * 16, ksteps = (it.K + 31) / 32;
+  const bf16_t* wp = it.W + (static_cast<size_t>(grp) * ksteps * KVF_WAVE + lane) * 8;
+  const bool live = r16 < M;
+  const bf16_t* ap = it.A + static_cast<size_t>(live ? r16 : 0) * it.lda + kg * 8;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  constexpr int U = depth(1, 1, 0), nw = GROUP_WAVES;
+  int ks = wave;
+  for (; ks + (U - 1) * nw < ksteps; ks += U * nw) {
+    bf16x8 wf[U], af[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = (ks + u * nw) * 32;
+      wf[u] = load_frag(wp + static_cast<size_t>(ks + u * nw) * (KVF_WAVE * 8), true);
+      af[u] = load_frag(ap + k, live && k + kg * 8 + 8 <= it.K);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], af[u], acc, 0, 0, 0);
+  }
+  for (; ks < ksteps; ks += nw) {
+    const bf16x8 wf = load_frag(wp + static_cast<size_t>(ks) * (KVF_WAVE * 8), true);
+    const bf16x8 af = load_frag(ap + ks * 32, live && ks * 32 + kg * 8 + 8 <= it.K);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
+  }
+  *reinterpret_cast<f32x4*>(red + (wave * KVF_WAVE + lane) * 4) = acc;
+  __syncthreads();
+  const int n = n0 + 4 * kg;
+  if (wave != 0 || !live || n >= it.N) return;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < nw; ++w) s += *reinterpret_cast<const f32x4*>(red + (w * KVF_WAVE + lane) * 4);
+  EpiOperands none;
+  none.have = false;
+  if (it.epi == 0) store_tile<0>(s, r16, n, it.N, it.ldc, it.C, nullptr, rp, none);
+  else if (it.epi == 1) store_tile<1>(s, r16, n, it.N, it.ldc, it.C, nullptr, rp, none);
+  else store_tile<3>(s, r16, n, it.N, it.ldc, it.C, nullptr, rp, none);
+}
+
 int g_waves_override = 0;
 int g_rows_override = 0;
 
@@ -936,6 +997,31 @@ KVF_EXPORT int kvf_gemm_bf16(const void* A, int a_type, const void* W, int w_til
   if (a_type == 0) return launch_epi<0>(A, w, C, epi, M, N, K, lda, ldc, eps, w_tiled, rd, none, s);
   if (a_type == 1) return launch_epi<1>(A, w, C, epi, M, N, K, lda, ldc, eps, w_tiled, rd, none, s);
   return static_cast<int>(hipErrorInvalidValue);
+}
+
+// Several products of M <= 16 rows in one launch (see gemm_group_kernel).  items: for each A, W, C (addresses), N, K, lda, ldc
+// and epi (0 store fp32, 1 store bf16, 3 SwiGLU pairs -> bf16 [M, N/2]); W in tiles, K beyond 224 (a k-step for every wave).
+KVF_EXPORT int kvf_gemm_bf16_group(const long long* items, int count, int M, hipStream_t s) {
+  if (M <= 0 || count <= 0) return 0;
+  if (M > 16 || count > GROUP_MAX) return static_cast<int>(hipErrorInvalidValue);
+  Group g{};
+  int blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    const long long* v = items + 8 * i;
+    GroupItem& it = g.item[i];
+    it = GroupItem{reinterpret_cast<const bf16_t*>(v[0]), reinterpret_cast<const bf16_t*>(v[1]), reinterpret_cast<void*>(v[2]),
+                   static_cast<int>(v[3]), static_cast<int>(v[4]), static_cast<int>(v[5]), static_cast<int>(v[6]),
+                   static_cast<int>(v[7]), blocks};
+    if (!it.A || !it.W || !it.C || it.N <= 0 || it.K <= 224 || it.K % 8 != 0 || it.lda % 8 != 0 || v[0] % 16 != 0 || v[1] % 16 != 0 ||
+        !(it.epi == 0 || it.epi == 1 || (it.epi == 3 && it.N % 4 == 0)))
+      return static_cast<int>(hipErrorInvalidValue);
+    blocks += (it.N + 15) / 16;
+  }
+  g.count = count;
+  RopeEpi rp{};
+  rp.act_scale = 1.f;
+  hipLaunchKernelGGL(gemm_group_kernel, dim3(blocks), dim3(GROUP_WAVES * KVF_WAVE), 0, s, g, M, rp);
+  return kvf_last_error();
 }
 
 // A product of 17 to 64 bf16 rows cut over K, see gemm_mid_kernel.  How many parts M rows over W [N, K]

@@ -227,6 +227,8 @@ class Step:
         # Whether the sublayer that runs adds to a stream whose next reader does not take a product in
         # parts (``take_owed``), so that an add kernel of its own has to follow one.
         self.settled_next = False
+        # products that a block has had made together with others, ahead of the parts they belong to
+        self.made: set = set()
         # the staging memory this step was filled from (``fill_step``), for ``upload_ints``
         self._meta: "MetaBuffers | None" = None
         self._turn = 0
@@ -249,6 +251,33 @@ class Step:
         dst.copy_(meta.staging[self._turn][lo:lo + n], non_blocking=True)
         meta.events[self._turn].record()     # the staging memory is free again after this copy
         return dst
+
+    def make(self, products: list) -> None:
+        """Make a part's products ``(key, a, w, out, pairs)`` (see ``Mixer.input_products``) that have not been made
+        yet: with few rows several of them in one launch."""
+        rest = [p for p in products if p[0] not in self.made]
+        self.made.difference_update(p[0] for p in products)
+        done = self._make_together(rest)
+        from kvforge_amd.kernels import ops
+        for key, a, w, out, pairs in rest:
+            if key not in done:
+                (ops.gemm_gated if pairs else ops.gemm)(a, w, out)
+
+    def make_early(self, products: list) -> None:
+        """Products that several parts are going to begin with and whose inputs are there: those that
+        go into one launch are made now, and the parts find them made."""
+        self.made |= self._make_together(products)
+
+    @staticmethod
+    def _make_together(products: list) -> set:
+        from kvforge_amd.kernels import ops
+        if len(products) < 2 or products[0][1].shape[0] > ops.FUSED_NORM_MAX_M:
+            return set()
+        some = [p for p in products if ops.gemm_group_takes(p[1], p[2], p[3])][:ops.GROUP_MAX]
+        if len(some) < 2:
+            return set()
+        ops.gemm_group([p[1:] for p in some])
+        return {p[0] for p in some}
 
     def owe(self, residual: torch.Tensor, product: torch.Tensor) -> None:
         self.settle()

@@ -11,7 +11,7 @@ here.
 from __future__ import annotations
 
 import ctypes
-from ctypes import c_float, c_int, c_long, c_void_p
+from ctypes import c_float, c_int, c_long, c_longlong, c_void_p
 from functools import lru_cache
 
 import torch
@@ -1075,6 +1075,35 @@ def gemm_gated(a: torch.Tensor, w, out: torch.Tensor, activation: str = "silu",
     _ok(f(a.data_ptr(), 1 if rms else 0, wp, tiled, out.data_ptr(), m, n, k, lda, ldc, float(rms_eps or 0.0),
           act, lim, float(scale), gate_bias.data_ptr() if gate_bias is not None else None,
           up_bias.data_ptr() if up_bias is not None else None, _stream()), "gemm_gated")
+
+
+GROUP_MAX = 8            # products of one launch
+GROUP_MAX_TILES = 512    # groups of 16 columns from which a product alone has other workgroups
+
+
+def gemm_group_takes(a: torch.Tensor, w, out: torch.Tensor) -> bool:
+    """Whether ``a @ w.T`` may be one of the products of ``gemm_group``: at most 16 rows of bf16 over tiled weights, K beyond
+    224, not so many columns that it fills the chip by itself."""
+    m, k = a.shape
+    return (isinstance(w, StreamedWeight) and a.dtype == BF16 and a.is_cuda and 0 < m <= FUSED_NORM_MAX_M and k > 224
+            and a.stride(1) == 1 and _rows_aligned(a, k, a.stride(0) if m > 1 else k) and w.shape[0] <= 16 * (GROUP_MAX_TILES - 1)
+            and out.dtype in (F32, BF16))
+
+
+def gemm_group(products) -> None:
+    """Several products ``out = a @ w.T`` of equally many rows in one launch: ``(a, w, out, pairs)`` each, ``out`` fp32 or bf16;
+    with ``pairs`` neighbouring columns are (gate, up) and ``out = silu(gate) * up`` (``gemm_gated`` without
+    biases).  For products that ``gemm_group_takes``; the bits of ``gemm`` and ``gemm_gated``."""
+    if not 0 < len(products) <= GROUP_MAX:
+        raise KernelError(f"gemm_group: 1 to {GROUP_MAX} products, got {len(products)}")
+    rows, items = products[0][0].shape[0], []
+    for a, w, out, pairs in products:
+        m, n, k, lda, ldc = _gemm_operands(a, w, out, (lambda n: n // 2) if pairs else (lambda n: n))
+        if m != rows or not gemm_group_takes(a, w, out) or (pairs and (n % 4 or out.dtype != BF16)):
+            raise KernelError("gemm_group: operands do not fit the kernel")
+        items += [a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), n, k, lda, ldc, 3 if pairs else 0 if out.dtype == F32 else 1]
+    f = _fn("gemm_bf16", "kvf_gemm_bf16_group", [c_void_p, c_int, c_int, c_void_p])
+    _ok(f((c_longlong * len(items))(*items), len(products), rows, _stream()), "gemm_group")
 
 
 def gemm_fused(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rms_eps: float | None = None,

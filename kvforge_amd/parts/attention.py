@@ -491,6 +491,18 @@ class PagedAttention(Mixer):
             step.scratch[key] = found
         return found
 
+    def input_products(self, x, step) -> list:
+        """(A projection that rotates and writes the cache itself, or takes the norm along, is none of these.)"""
+        n, ws = x.shape[0], step.ws
+        out = []
+        if self.norm_eps is None and self.row_norm is None and (self.conv is not None or self.qk_norm is not None or self._hooked()):
+            rows = ws.buf("conv_rows" if self.conv is not None else "qkv", (n, self.w_qkv.shape[0]), step.act_dtype)
+            out.append(((self.prefix, "qkv"), x, self.w_qkv, rows, False))
+        if self.norm_eps is None and self.w_head_gate is not None:
+            gates = ws.buf("attn_head_gates", (n, self.w_head_gate.shape[0]), torch.float32)
+            out.append(((self.prefix, "head_gates"), x, self.w_head_gate, gates, False))
+        return out
+
     def forward(self, x, step, layer: LayerState, residual) -> None:
         """``x``: normalised activations, or (after ``absorb_norm``) the fp32 residual stream."""
         n = x.shape[0]
@@ -536,7 +548,7 @@ class PagedAttention(Mixer):
             if layer.state is None and self.conv[0] > 1:
                 raise RuntimeError("attention behind a convolution needs a state slot per request")
             rows = ws.buf("conv_rows", (n, self.w_qkv.shape[0]), act)
-            ops.gemm(x, self.w_qkv, rows)
+            step.make([((self.prefix, "qkv"), x, self.w_qkv, rows, False)])
             qkv = ws.buf("conv_q", (n, H * d), act)
             ops.conv_norm_kvwrite(rows, self.conv_w, step.cu_q, step.positions, step.slot_ids, layer.state, table, qkv,
                                   layer.k_pages, layer.v_pages, H, KV, d, step.n_seqs, max(step.q_lens),
@@ -557,7 +569,7 @@ class PagedAttention(Mixer):
         else:
             g0 = (H + (2 * KV if self.own_kv else 0)) * d
             qkv = ws.buf("qkv", (n, self.w_qkv.shape[0]), act)
-            ops.gemm(x, self.w_qkv, qkv)
+            step.make([((self.prefix, "qkv"), x, self.w_qkv, qkv, False)])
             self.after_projection(qkv, step)
             if self.qk_norm is not None:
                 ops.qknorm_rope_kvwrite(qkv, step.positions, step.seq_of_token, cos, sin, table,
@@ -571,7 +583,7 @@ class PagedAttention(Mixer):
         head_gates = None
         if self.w_head_gate is not None:
             head_gates = ws.buf("attn_head_gates", (n, self.w_head_gate.shape[0]), torch.float32)
-            ops.gemm(x, self.w_head_gate, head_gates)
+            step.make([((self.prefix, "head_gates"), x, self.w_head_gate, head_gates, False)])
         out = ws.buf("attn_out", (n, H * d), act)
         window, chunk = self.window or 0, self.chunk or 0
         bs = layer.k_pages.shape[2]

@@ -213,6 +213,13 @@ class Mixer(Part):
     # whether ``LayerState.state`` may be a block of columns of wider slots (``[slots, floats]``, dense rows)
     shares_slot = False
 
+    def input_products(self, x: torch.Tensor, step: "Step") -> list:
+        """The products over ``x`` alone that ``forward`` begins with, as ``(key, a, w, out, pairs)``: ``out = a @ w.T``, with
+        ``pairs`` of (gate, up) columns ``silu(gate) * up``; ``key`` names the product within the model.  ``forward`` hands the same list
+        to ``step.make``, which leaves out what a block has had made already (``Step.make_early``), side by side with
+        other parts' products.  Only for an ``x`` of the step's activation type."""
+        return []
+
     def forward(self, x: torch.Tensor, step: "Step", layer: LayerState,
                 residual: torch.Tensor) -> None:
         """Add the mixer's output for activations ``x [N, hidden]`` into ``residual`` (fp32)."""
@@ -221,6 +228,10 @@ class Mixer(Part):
 
 class FeedForward(Part):
     settles_residual = False
+
+    def input_products(self, x: torch.Tensor, step: "Step") -> list:
+        """As ``Mixer.input_products``."""
+        return []
 
     def forward(self, x: torch.Tensor, step: "Step", residual: torch.Tensor) -> None:
         """Add the feed-forward output for ``x [N, hidden]`` into ``residual`` (fp32)."""
@@ -311,6 +322,17 @@ class Block(Part):
     @property
     def replayable(self) -> bool:
         return all(p.replayable for p in self.parts())
+
+
+def products_of(part: Part, x: torch.Tensor, step: "Step") -> list:
+    """``part.input_products(x, step)``, unless a subclass has given the part another ``forward``, of which the list that
+    it inherits says nothing."""
+    for cls in type(part).__mro__:
+        if "input_products" in vars(cls):
+            return part.input_products(x, step)
+        if "forward" in vars(cls):
+            return []
+    return []
 
 
 def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,

@@ -8,7 +8,7 @@ import torch
 
 from kvforge_amd.kernels import ops
 from kvforge_amd.parts.base import (Block, FeedForward, LayerState, Mixer, Norm, Part, StateSpec,
-                                    WeightSpec)
+                                    WeightSpec, products_of)
 from kvforge_amd.registry import register_block
 
 
@@ -158,6 +158,8 @@ class ParallelBlock(Block):
         # `after` or to the next block's norms, of which only a single one takes parts
         behind = pair or self.mu is not None or self.after is not None
         step.settled_next = self.ffn is not None or behind
+        # both sublayers' inputs are there: what they begin with is made together
+        step.make_early(products_of(self.mixer, hs, step) + (products_of(self.ffn, h, step) if self.ffn is not None else []))
         self.mixer.forward(hs, step, layer, residual)
         step.settled_next = behind
         bias = None
@@ -168,6 +170,8 @@ class ParallelBlock(Block):
             if getattr(self.ffn, "defer_down_bias", False):
                 bias = self.ffn.down_bias
         step.settled_next = False
+        if step.made:
+            raise RuntimeError(f"products that were made ahead of their parts and not used: {sorted(step.made)}")
         if self.after is not None:
             self.after.forward(residual, step, bias=bias)
 

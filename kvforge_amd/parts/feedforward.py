@@ -151,13 +151,24 @@ class GatedFeedForward(SwiGLU):
         return super().held_tensors() + [b for b in (self.gate_bias, self.up_bias, self.down_bias)
                                          if b is not None]
 
+    def input_products(self, x, step) -> list:
+        """Gate and up where ``step.make`` has a kernel for the whole of them (silu, no biases, few rows)."""
+        if (self.activation != "silu" or self.gate_bias is not None or self.out_scale != 1.0 or self.inter % 2
+                or not ops.bf16_kernel_takes(x, self.w_gate_up, False, True)):
+            return []
+        act = step.ws.buf("ffn_act", (x.shape[0], self.inter), step.act_dtype)
+        return [((self.prefix, "act"), x, self.w_gate_up, act, True)]
+
     def forward(self, x, step, residual) -> None:
         """``x``: normalised activations."""
         n = x.shape[0]
         ws, dt = step.ws, step.act_dtype
         step.settle()
         act = ws.buf("ffn_act", (n, self.inter), dt)
-        if ops.bf16_kernel_takes(x, self.w_gate_up, False, True) and self.inter % 2 == 0:
+        first = self.input_products(x, step)
+        if first:
+            step.make(first)
+        elif ops.bf16_kernel_takes(x, self.w_gate_up, False, True) and self.inter % 2 == 0:
             # one kernel: gate/up projection, biases, activation, gate
             ops.gemm_gated(x, self.w_gate_up, act, self.activation, self.gate_bias, self.up_bias, limit=self.limit,
                            scale=self.out_scale)

@@ -111,6 +111,12 @@ class MatrixLSTM(Mixer):
             out[name] = step.ws.buf("mlstm_multi_" + name, shape, dtype)
         return out
 
+    def input_products(self, x, step) -> list:
+        n, ws = x.shape[0], step.ws
+        rows = ws.buf("mlstm_rows", (n, 2 * self.H * (self.dk + self.dv)), step.act_dtype)
+        gates = ws.buf("mlstm_gates", (n, self.G_pad), torch.float32)
+        return [((self.prefix, "rows"), x, self.w_rows, rows, False), ((self.prefix, "gates"), x, self.w_gates, gates, False)]
+
     def forward(self, x, step, layer: LayerState, residual) -> None:
         """``x``: normalised activations."""
         if layer.state is None:
@@ -119,10 +125,9 @@ class MatrixLSTM(Mixer):
         H, dk, dv = self.H, self.dk, self.dv
         ws, act = step.ws, step.act_dtype
         step.settle()
-        rows = ws.buf("mlstm_rows", (n, 2 * H * dk + 2 * H * dv), act)
-        ops.gemm(x, self.w_rows, rows)
-        gates = ws.buf("mlstm_gates", (n, self.G_pad), torch.float32)
-        ops.gemm(x, self.w_gates, gates)
+        products = self.input_products(x, step)
+        step.make(products)
+        rows, gates = (p[3] for p in products)
         raw = ws.buf("mlstm_raw", (n, H * dv), torch.float32)
         # which of the kernels have work is known from the runs' lengths (all ones in a
         # captured step of single tokens, so a replay launches what the capture launched)

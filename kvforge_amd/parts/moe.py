@@ -184,11 +184,22 @@ class RoutedExperts(FeedForward):
                 + [t for t in (self.correction, self.r_bias, self.table) if t is not None]
                 + (self.shared.held_tensors() if self.shared is not None else []))
 
+    def input_products(self, x, step) -> list:
+        """The router, and gate and up of the shared expert."""
+        out = []
+        if self.table is None:
+            logits = step.ws.buf("moe_logits", (x.shape[0], self.R_pad), torch.float32)     # 32-bit sums, stored so
+            out.append(((self.prefix, "router"), x, self.w_router, logits, False))
+        if self.shared is not None and self.w_shared_gate is None:
+            out += self.shared.input_products(x, step)
+        return out
+
     def forward(self, x, step, residual) -> None:
         """``x``: normalised activations."""
         n = x.shape[0]
         ws, dt = step.ws, step.act_dtype
         step.settle()
+        step.make_early([p for p in self.input_products(x, step) if p[0] not in step.made])
         chosen = ws.buf("moe_chosen", (n, self.top), torch.int32)
         weights = ws.buf("moe_weights", (n, self.top), torch.float32)
         grouped = ops.moe_grouped_takes(x, self.w_gate_up, self.w_down, self.E, self.ff) and x.is_contiguous()
@@ -204,8 +215,9 @@ class RoutedExperts(FeedForward):
         if self.table is not None:
             ops.moe_table(step.token_ids, self.table, chosen, weights, self.E)
         else:
-            logits = ws.buf("moe_logits", (n, self.R_pad), torch.float32)[:, :self.R]
-            ops.gemm(x, self.w_router, ws.buf("moe_logits", (n, self.R_pad), torch.float32))   # 32-bit sums, stored so
+            logits = ws.buf("moe_logits", (n, self.R_pad), torch.float32)
+            step.make([((self.prefix, "router"), x, self.w_router, logits, False)])
+            logits = logits[:, :self.R]
             ops.moe_topk(logits, self.correction, chosen, weights, self.scores, self.renormalize, bias=self.r_bias,
                          scale=self.out_scale,
                          plan=(self.w_gate_up, self.w_down, self.E, self.ff, scratch) if planned else None)

@@ -7,7 +7,7 @@ from __future__ import annotations
 import torch
 
 from kvforge_amd.kernels import ops
-from kvforge_amd.parts.base import CacheSpec, LayerState, Mixer, Norm, Part, StateSpec, WeightSpec
+from kvforge_amd.parts.base import CacheSpec, LayerState, Mixer, Norm, Part, StateSpec, WeightSpec, products_of
 from kvforge_amd.registry import register_mixer
 
 
@@ -97,10 +97,14 @@ class MixerPair(Mixer):
         halves = (layer.state[:, :n], layer.state[:, self.right_off:self.right_off + _floats(self.right.state_spec)])
         return tuple(LayerState(layer.group, layer.pages, layer.owns_cache, s) for s in halves)
 
+    def input_products(self, x, step) -> list:
+        return products_of(self.left, x, step) + products_of(self.right, x, step)
+
     def forward(self, x, step, layer: LayerState, residual) -> None:
         """``x``: normalised activations.  Without norms, what the first leaves owed to the stream the
         second settles (or takes along) as any part does; with norms, each writes rows of its own."""
         ll, rl = self._layers(layer)
+        step.make_early([p for p in self.input_products(x, step) if p[0] not in step.made])
         if self.norms is None:
             self.left.forward(x, step, ll, residual)
             self.right.forward(x, step, rl, residual)

@@ -111,6 +111,12 @@ class ConvMemory(Mixer):
     def _chunk_scratch(self, n_tokens: int, n_chunks: int) -> dict[str, tuple]:
         return ops.ssm_scratch(n_tokens, n_chunks, self.H, self.dk, self.dv, self.b_off is not None)
 
+    def input_products(self, x, step) -> list:
+        n, ws = x.shape[0], step.ws
+        rows = ws.buf("ssm_rows", (n, self.w_rows.shape[0]), step.act_dtype)
+        gates = ws.buf("ssm_gates", (n, self.w_gates.shape[0]), torch.float32)     # 32-bit sums, stored so
+        return [((self.prefix, "rows"), x, self.w_rows, rows, False), ((self.prefix, "gates"), x, self.w_gates, gates, False)]
+
     def forward(self, x, step, layer: LayerState, residual) -> None:
         """``x``: the mixer's input rows in the step's activation type."""
         if layer.state is None:
@@ -118,10 +124,9 @@ class ConvMemory(Mixer):
         n = x.shape[0]
         ws, act = step.ws, step.act_dtype
         step.settle()
-        rows = ws.buf("ssm_rows", (n, self.w_rows.shape[0]), act)
-        ops.gemm(x, self.w_rows, rows)
-        gates = ws.buf("ssm_gates", (n, self.w_gates.shape[0]), torch.float32)
-        ops.gemm(x, self.w_gates, gates)            # 32-bit sums, stored so
+        products = self.input_products(x, step)
+        step.make(products)
+        rows, gates = (p[3] for p in products)
         mixed = ws.buf("ssm_mixed", (n, self.channels), torch.float32)
         ops.ssm_conv(rows, self.conv_col, self.conv_w, self.conv_b, step.cu_q, step.positions, step.slot_ids,
                      layer.state, self.state_off, mixed, step.n_seqs, max(step.q_lens), unit=self.unit,

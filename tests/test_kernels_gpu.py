@@ -586,6 +586,36 @@ def test_gemm_qkv_rope_equals_the_three_steps(m, H, KV, d, rot, bs, rms):
         assert all(torch.equal(x1, x2) for x1, x2 in zip(*got))
 
 
+@pytest.mark.parametrize("m", [1, 3, 8, 16])
+@pytest.mark.parametrize("shapes", [
+    [(48, 2048, "f32"), (3072, 2048, "bf16"), (4096, 2048, "pairs")],
+    [(16, 232, "f32"), (20, 256, "bf16"), (36, 2056, "pairs"), (8176, 264, "bf16"), (4, 1000, "f32"), (33, 480, "f32"),
+     (17, 768, "bf16"), (16, 512, "pairs")]])
+def test_gemm_group_has_the_bits_of_the_single_products(m, shapes):
+    """Products of one launch, each with rows, width, K and result of its own, against the kernels they stand for."""
+    g = torch.Generator().manual_seed(m)
+    products, want = [], []
+    for n, k, kind in shapes:
+        a = torch.randn(m, k + 16, generator=g).to(torch.bfloat16).to(DEV)[:, :k]
+        w = ops().StreamedWeight((torch.randn(n, k, generator=g) / 20).to(torch.bfloat16).to(DEV))
+        cols, dtype = (n // 2 if kind == "pairs" else n), (torch.float32 if kind == "f32" else torch.bfloat16)
+        wide = torch.full((2, m, cols + 8), 7.0, dtype=dtype, device=DEV)    # rows of results further apart than they are wide
+        if kind == "pairs":
+            ops().gemm_gated(a, w, wide[0][:, :cols])
+        else:
+            ops().gemm(a, w, wide[0][:, :cols])
+        assert ops().gemm_group_takes(a, w, wide[1][:, :cols])
+        products.append((a, w, wide[1][:, :cols], kind == "pairs"))
+        want.append(wide)
+    ops().gemm_group(products)
+    for wide in want:
+        assert torch.equal(wide[0], wide[1]) and wide[0][:, :-8].ne(7.0).any()
+    a, w, out, _ = products[0]
+    assert not ops().gemm_group_takes(a, w.plain, out) and not ops().gemm_group_takes(a.float(), w, out)
+    with pytest.raises(ops().KernelError):
+        ops().gemm_group(products * 3)
+
+
 @pytest.mark.parametrize("tile", range(6))
 @pytest.mark.parametrize("m,k,H,KV,d,rot,bs,extra", [
     (65, 64, 4, 2, 16, 16, 8, 0),          # one stage of K; fewer columns than a tile
