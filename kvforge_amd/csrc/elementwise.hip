@@ -342,6 +342,189 @@ KVF_EXPORT int kvf_rmsnorm_pair_bf16(float* x, const void* delta, int delta_f32,
   return rmsnorm_pair_launch<bf16_t, bf16_t>(x, delta, w1, w2, eps, o1, o2, m, h, s);
 }
 
+// ----------------------------------------------------------------------------- experts' sum and the next norm
+// What a routed layer leaves owed to the stream, and the norm or the two norms of one eps that read it next, in one pass over
+// the rows: x += pre; x += sum over the token's choices (as moe_combine_kernel); x += post; out1 (and out2) = norm(x).
+// pre, post (may be null): a product owed before the experts and one behind them, bf16 or fp32.
+//
+// What bounds it is memory, and with few rows the trips to it: 8 rows of 2,048 with two norms 4.7 + 4.8 us as two kernels,
+// and 2,042 rows 9.3 + 14.9 + 11.8 with the product ahead of the experts; 5.5 and 20.5 together.  The sums are
+// those of the kernels that stand for the steps, element by element and in the order of their threads: the
+// row goes through LDS between the two.  TWO: the two norms of rmsnorm_pair_kernel, else rmsnorm_kernel's.
+// A chain of loads is what a row of its own would wait for: the choices are read by the lanes side by side and handed round, the rows they
+// lead to and the norms' weights are all asked for before the first is used (one choice after the other: 9.6 us).
+constexpr int COMBINE_KEEP = 16, COMBINE_AHEAD = 4;    // elements of the row a thread has at most; choices whose rows are asked for together
+struct CombineArgs {
+  const void *pre, *post;
+  int pre_f32, post_f32;
+  const bf16_t *y, *in;
+  const int *sel, *where;
+  const float* wgt;
+  int top, E;
+};
+// eight numbers of either type as they lie, and widened
+struct Raw8 {
+  uint4 lo, hi;
+};
+__device__ __forceinline__ Raw8 raw8(const void* p, int f32, size_t at) {
+  Raw8 r;
+  const char* b = static_cast<const char*>(p) + at * (f32 ? 4 : 2);
+  r.lo = *reinterpret_cast<const uint4*>(b);
+  r.hi = f32 ? *reinterpret_cast<const uint4*>(b + 16) : make_uint4(0u, 0u, 0u, 0u);
+  return r;
+}
+__device__ __forceinline__ void wide8(const Raw8& r, int f32, float (&v)[8]) {
+  const uint32_t lo[4] = {r.lo.x, r.lo.y, r.lo.z, r.lo.w}, hi[4] = {r.hi.x, r.hi.y, r.hi.z, r.hi.w};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    v[2 * u] = __uint_as_float(lo[u] << 16);
+    v[2 * u + 1] = __uint_as_float(lo[u] & 0xffff0000u);
+  }
+  if (f32) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      v[u] = __uint_as_float(lo[u]);
+      v[4 + u] = __uint_as_float(hi[u]);
+    }
+  }
+}
+
+template <bool TWO, int KEEP>
+__global__ __launch_bounds__(256) void combine_norm_kernel(float* x, CombineArgs c, const float* __restrict__ w1,
+                                                           const float* __restrict__ w2, float eps, bf16_t* out1, bf16_t* out2, int h) {
+  extern __shared__ __align__(16) float combined[];   // [h]
+  __shared__ float scratch[16];
+  const int n = blockIdx.x, tid = threadIdx.x, lane = tid % KVF_WAVE;
+  const size_t row = static_cast<size_t>(n) * h;
+  int my_e = -1, my_at = 0;
+  float my_w = 1.f;
+  if (lane < c.top) {
+    const int p = n * c.top + lane;
+    my_e = c.sel[p];
+    my_at = c.where[p];
+    if (c.wgt) my_w = c.wgt[p];
+  }
+  float g1[KEEP], g2[KEEP];
+#pragma unroll
+  for (int k = 0; k < KEEP; ++k) {                     // as the thread needs them behind the sums; past the row its last
+    const int i = TWO ? k * static_cast<int>(blockDim.x) + tid : (k / 4 * static_cast<int>(blockDim.x) + tid) * 4 + k % 4;
+    g1[k] = w1[min(i, h - 1)];
+    if (TWO) g2[k] = w2[min(i, h - 1)];
+  }
+  for (int i = 8 * tid; i < h; i += 8 * blockDim.x) {
+    float a[8], sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    load8(x + row + i, a);
+    Raw8 pre = {}, post = {};
+    if (c.pre) pre = raw8(c.pre, c.pre_f32, row + i);
+    if (c.post) post = raw8(c.post, c.post_f32, row + i);
+    for (int k0 = 0; k0 < c.top; k0 += COMBINE_AHEAD) {
+      uint4 v[COMBINE_AHEAD];
+#pragma unroll
+      for (int k = 0; k < COMBINE_AHEAD; ++k) {        // a choice past the last, or one that names nothing: the row itself, not used
+        const int at = min(k0 + k, c.top - 1), e = __builtin_amdgcn_readlane(my_e, at), to = __builtin_amdgcn_readlane(my_at, at);
+        const bf16_t* from = e >= 0 && e < c.E ? c.y + static_cast<size_t>(to) * h : c.in + row;
+        v[k] = *reinterpret_cast<const uint4*>(from + i);
+      }
+#pragma unroll
+      for (int k = 0; k < COMBINE_AHEAD; ++k) {
+        if (k0 + k >= c.top || __builtin_amdgcn_readlane(my_e, k0 + k) < 0) continue;
+        const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_w), k0 + k));
+        float t[8];
+        wide8(Raw8{v[k], make_uint4(0u, 0u, 0u, 0u)}, 0, t);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum[u] = fmaf(w, t[u], sum[u]);
+      }
+    }
+    float t[8];
+    if (c.pre) {
+      wide8(pre, c.pre_f32, t);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] += t[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] += sum[u];
+    if (c.post) {
+      wide8(post, c.post_f32, t);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] += t[u];
+    }
+    const float4 lo = make_float4(a[0], a[1], a[2], a[3]), hi = make_float4(a[4], a[5], a[6], a[7]);
+    store4(x + row + i, lo);
+    store4(x + row + i + 4, hi);
+    store4(combined + i, lo);
+    store4(combined + i + 4, hi);
+  }
+  __syncthreads();                                     // (and the rows that `in` may share with an output have been read)
+  float ss = 0.f;
+  if (TWO) {
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k) {
+      const int i = k * blockDim.x + tid;
+      if (i < h) {
+        const float v = combined[i];
+        ss += v * v;
+      }
+    }
+    ss = block_sum(ss, scratch);
+    const float r = rsqrtf(ss / static_cast<float>(h) + eps);
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k) {
+      const int i = k * blockDim.x + tid;
+      if (i < h) {
+        const float y = combined[i] * r;
+        Elem<bf16_t>::store(out1 + row + i, y * g1[k]);
+        Elem<bf16_t>::store(out2 + row + i, y * g2[k]);
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < KEEP / 4; ++k) {
+    const int i = (k * blockDim.x + tid) * 4;
+    if (i < h) {
+      const float4 v = load4(combined + i);
+      ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+    }
+  }
+  ss = block_sum(ss, scratch);
+  const float r = rsqrtf(ss / static_cast<float>(h) + eps);
+#pragma unroll
+  for (int k = 0; k < KEEP / 4; ++k) {
+    const int i = (k * blockDim.x + tid) * 4;
+    if (i < h) {
+      const float4 v = load4(combined + i);
+      float4 y = make_float4(v.x * r, v.y * r, v.z * r, v.w * r);
+      y.x *= g1[4 * k]; y.y *= g1[4 * k + 1]; y.z *= g1[4 * k + 2]; y.w *= g1[4 * k + 3];
+      store4(out1 + row + i, y);
+    }
+  }
+}
+// x, y, in, pre, post, the weights and the outputs on 16 bytes; h a multiple of 8 up to COMBINE_KEEP a thread.
+KVF_EXPORT int kvf_combine_norm(float* x, const void* pre, int pre_f32, const void* y, const void* in, const int* sel, const float* wgt,
+                                const int* where, int top, int E, const void* post, int post_f32, const float* w1, const float* w2,
+                                float eps, void* out1, void* out2, int n, int h, hipStream_t s) {
+  if (n <= 0) return 0;
+  const int threads = h >= 1024 ? 256 : (h >= 256 ? 128 : 64);   // as the norms'
+  auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (h <= 0 || h % 8 != 0 || h > COMBINE_KEEP * threads || top <= 0 || top > KVF_WAVE || E <= 0 || !w1 || (w2 == nullptr) != (out2 == nullptr) || !at16(x) ||
+      !at16(pre) || !at16(y) || !at16(in) || !at16(post) || !at16(w1) || !at16(w2) || !at16(out1) || !at16(out2))
+    return static_cast<int>(hipErrorInvalidValue);
+  const CombineArgs c{pre, post, pre_f32, post_f32, static_cast<const bf16_t*>(y), static_cast<const bf16_t*>(in), sel, where, wgt, top, E};
+  const size_t lds = static_cast<size_t>(h) * sizeof(float);
+#define KVF_COMBINE(TWO, KEEP)                                                                                                 \
+  hipLaunchKernelGGL((combine_norm_kernel<TWO, KEEP>), dim3(n), dim3(threads), lds, s, x, c, w1, w2, eps, static_cast<bf16_t*>(out1), \
+                     static_cast<bf16_t*>(out2), h)
+  if (h <= 8 * threads) {
+    if (w2) KVF_COMBINE(true, 8);
+    else KVF_COMBINE(false, 8);
+  } else {
+    if (w2) KVF_COMBINE(true, 16);
+    else KVF_COMBINE(false, 16);
+  }
+#undef KVF_COMBINE
+  return kvf_last_error();
+}
+
 // ----------------------------------------------------------------------------- residual sum
 // x[m] += delta[m] in fp32 (x is the residual stream, delta a product in T).
 template <typename T>

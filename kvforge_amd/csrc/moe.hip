@@ -800,15 +800,14 @@ KVF_EXPORT int kvf_moe_topk_plan(const float* z, int z_stride, const float* bias
 // The routed experts of a bf16 step without the rows that did not choose them.  x [n, K] (row
 // stride ldx), w_gate_up / w_down: the tiled forms of [E 2 ff, K] (gate and up rows interleaved)
 // and [K, E ff]; sel / wgt [n, top]; scratch: where, order [n top], tiles [3 max_tiles],
-// num_tiles [1], act [n top, ff], y [n top, K].  Needs K % 8 == 0 and ff % 32 == 0.  weigh_input: the
-// weights go into the experts' inputs instead of the sum over their outputs.  fresh: residual is
-// written, not added to.  form, limit: how an expert's pairs are joined (GateForm's act 0 or 2).  many_rows: below
+// num_tiles [1], act [n top, ff], y [n top, K].  Needs K % 8 == 0 and ff % 32 == 0.  The outputs' rows stay in y, which
+// kvf_moe_combine adds up.  weigh_input: the weights go into the experts' inputs instead of the sum over their outputs.  form, limit: how an expert's pairs are joined (GateForm's act 0 or 2).  many_rows: below
 // 0, or which kernels are taken whatever the sizes (0: those of few rows, else those of more).  planned: where,
 // order, tiles and num_tiles hold the plan already (kvf_moe_topk_plan).
-KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int K, int E, int ff, int top,
+KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, int n, int K, int E, int ff, int top,
                                const void* w_gate_up, const void* w_down, const int* sel, const float* wgt,
                                int* where, int* order, int* tiles, int* num_tiles, int max_tiles, void* act,
-                               void* y, float* residual, int weigh_input, int fresh, int form, float limit,
+                               void* y, int weigh_input, int form, float limit,
                                int many_rows, int planned, hipStream_t s) {
   if (n <= 0) return 0;
   const int pairs = n * top;
@@ -839,7 +838,16 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, const void* h, int n, int
     hipLaunchKernelGGL(moe_down_kernel, dim3(down_blocks, max_tiles), dim3(256), 0, s, a, ff, down, E * (ff / 32), tiles,
                        num_tiles, out, K);
   }
-  hipLaunchKernelGGL(moe_combine_kernel<bf16_t>, dim3(n), dim3(256), 0, s, residual, static_cast<const bf16_t*>(y),
-                     static_cast<const bf16_t*>(h), sel, weigh_input ? nullptr : wgt, where, K, top, E, fresh);
+  return kvf_last_error();
+}
+
+// The sum over the choices behind kvf_moe_grouped, arguments as there: x [n, K] is the residual stream; wgt null: the weights went
+// into the experts' inputs.
+KVF_EXPORT int kvf_moe_combine(float* x, const void* y, const void* h, const int* sel, const float* wgt, const int* where, int n,
+                               int K, int top, int E, int fresh, hipStream_t s) {
+  if (n <= 0) return 0;
+  if (K <= 0 || K % 8 != 0 || top <= 0 || top > MAX_TOP || E <= 0) return static_cast<int>(hipErrorInvalidValue);
+  hipLaunchKernelGGL(moe_combine_kernel<bf16_t>, dim3(n), dim3(256), 0, s, x, static_cast<const bf16_t*>(y),
+                     static_cast<const bf16_t*>(h), sel, wgt, where, K, top, E, fresh);
   return kvf_last_error();
 }

@@ -208,6 +208,7 @@ class Step:
         self.host_token_ids: np.ndarray | None = None
         self.prefill_seqs: list[int] = []
         self.decode_shape = DecodeShape(0, 0, 0)
+        self.all_rows = False        # every token wants its logits, in order
         self.max_position = 0
         # What parts keep for the length of the step (work lists, launch plans, tables), under
         # keys of their own choosing: the step knows nothing of any part's tiling.
@@ -220,6 +221,9 @@ class Step:
         # A vector still owed to every row of the stream: (stream, fp32 vector), the bias of a
         # feed-forward's last product; a norm that adds biases takes it (``take_owed_bias``).
         self.owed_bias: tuple[torch.Tensor, torch.Tensor] | None = None
+        # The sum over a routed layer's experts: (stream, what is owed ahead of it or None, arguments of ``ops.moe_combine`` behind the
+        # stream, what is owed behind it or None).  Nothing else is owed beside it.
+        self.owed_experts: tuple | None = None
         # Rows that a block has handed to a sublayer in place of the stream and that hold
         # nothing yet: the sublayer's last product is written there instead of added
         # (``parts.base.add_product``), which then forgets the mark.
@@ -283,13 +287,39 @@ class Step:
         self.settle()
         self.owed = (residual, product)
 
+    def owe_experts(self, residual: torch.Tensor, pre: torch.Tensor | None, combine: tuple, post: torch.Tensor | None) -> None:
+        """Leave ``residual += pre``, ``ops.moe_combine(residual, *combine)`` and ``residual += post`` to whoever reads the stream
+        next: a norm takes it along (``take_owed_experts``), for anything else it is done by itself."""
+        self.settle()
+        self.owed_experts = (residual, pre, combine, post)
+
+    def take_owed_experts(self, residual: torch.Tensor) -> tuple | None:
+        """``(pre, combine, post)`` if experts are owed to ``residual``, for a kernel that adds them itself."""
+        if self.owed_experts is None or self.owed_experts[0] is not residual:
+            return None
+        owed, self.owed_experts = self.owed_experts[1:], None
+        return owed
+
+    def _settle_experts(self) -> None:
+        if self.owed_experts is not None:
+            from kvforge_amd.kernels import ops
+            residual, pre, combine, post = self.owed_experts
+            self.owed_experts = None
+            if pre is not None:
+                ops.add_rows(residual, pre)
+            ops.moe_combine(residual, *combine)
+            if post is not None:
+                ops.add_rows(residual, post)
+
     def owe_bias(self, residual: torch.Tensor, bias: torch.Tensor) -> None:
+        self._settle_experts()
         self._settle_bias()
         self.owed_bias = (residual, bias)
 
     def take_owed_bias(self, residual: torch.Tensor) -> torch.Tensor | None:
         """The vector owed to every row of ``residual``, for a norm kernel that adds it itself (to be
         asked for before ``take_owed``, which otherwise brings the stream up to date)."""
+        self._settle_experts()
         if self.owed_bias is None:
             return None
         if self.owed_bias[0] is not residual:
@@ -308,6 +338,7 @@ class Step:
     def take_owed(self, residual: torch.Tensor, parts: bool = False) -> torch.Tensor | None:
         """The product owed to ``residual``, for a norm kernel that adds it itself.  ``parts``: whether
         the kernel takes a product in parts (``ops.gemm_parts``); one that does not finds it added."""
+        self._settle_experts()
         self._settle_bias()
         if self.owed is None:
             return None
@@ -322,6 +353,7 @@ class Step:
         """``(rows, weight, eps)`` if what is owed to ``residual`` is the RMS norm of fp32 rows (a
         sublayer's output that joins the stream through a norm of its own), for a kernel that
         adds it itself; ``None`` otherwise (whatever else is owed stays owed)."""
+        self._settle_experts()
         self._settle_bias()
         if self.owed is None or self.owed[0] is not residual or len(self.owed) != 4:
             return None
@@ -331,7 +363,8 @@ class Step:
 
     def settle(self) -> None:
         """Add what is owed to the residual stream now: ``(stream, rows)``, or ``(stream, rows,
-        weight, eps)`` for rows that join through their RMS norm; and a bias owed to every row."""
+        weight, eps)`` for rows that join through their RMS norm; a bias owed to every row; and experts."""
+        self._settle_experts()
         self._settle_bias()
         if self.owed is not None:
             from kvforge_amd.kernels import ops
@@ -483,6 +516,7 @@ def fill_step(step: Step, meta: MetaBuffers, entries: Sequence[StepEntry], table
             raise ValueError("padding is for batches of single tokens that each want their logits")
         rows = list(range(Bp))
     R = len(rows)
+    step.all_rows = singles and R == N and rows == list(range(N))
     host[off["logits_rows"]:off["logits_rows"] + R] = rows
 
     # longest context first, so that kernels which take them in this order start what lasts longest first

@@ -2094,7 +2094,7 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
                 weights: torch.Tensor, residual: torch.Tensor, experts: int, ff: int,
                 scratch: dict[str, torch.Tensor], weigh_input: bool = False, fresh: bool = False,
                 form: str = "silu", limit: float | None = None, many_rows: bool | None = None,
-                planned: bool = False) -> None:
+                planned: bool = False, combine: bool = True) -> None:
     """``residual[n] += sum_k weights[n, k] * expert_{chosen[n, k]}(x[n])`` (a choice ``>= experts``
     stands for ``x[n]`` itself) with every expert's products taken over only the rows that chose
     it: the pairs are grouped by expert on the device, tiles of up to 16 or up to 128 rows go through the
@@ -2107,7 +2107,8 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
     ``fresh``: ``residual`` is written instead of added to.  ``form``, ``limit``: how an expert joins its
     pairs (``MOE_FORMS``).  ``many_rows``: for tests, which of the two tile sizes is taken; the sizes
     decide otherwise (``kvf_moe_grouped_many_rows`` in ``moe.hip``).  The results are the same bits.
-    ``planned``: ``moe_topk(..., plan=...)`` has left the plan in ``scratch``."""
+    ``planned``: ``moe_topk(..., plan=...)`` has left the plan in ``scratch``.  Without ``combine`` the experts' output
+    rows stay in ``scratch`` and ``residual`` as it is, for ``moe_combine`` or ``moe_combine_norm``."""
     if planned and many_rows is not None:
         raise KernelError("moe_grouped: a plan that is there decides about the tiles")
     code, lim = _moe_form(form, limit, "moe_grouped")
@@ -2124,14 +2125,76 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
     pairs, max_tiles = n * top, _check_moe_plan(scratch, n, top, experts)
     for name, dtype, shape in (("act", BF16, (pairs, ff)), ("y", BF16, (pairs, k))):
         _check(scratch[name], name, dtype, shape)
-    f = _fn("moe", "kvf_moe_grouped", [c_void_p, c_int, c_void_p] + [c_int] * 5 + [c_void_p] * 8 + [c_int]
-            + [c_void_p] * 3 + [c_int, c_int, c_int, c_float, c_int, c_int, c_void_p])
-    _ok(f(x.data_ptr(), x.stride(0) if n > 1 else k, x.data_ptr(), n, k, int(experts), int(ff), top,
+    f = _fn("moe", "kvf_moe_grouped", [c_void_p] + [c_int] * 6 + [c_void_p] * 8 + [c_int]
+            + [c_void_p] * 2 + [c_int, c_int, c_float, c_int, c_int, c_void_p])
+    _ok(f(x.data_ptr(), x.stride(0) if n > 1 else k, n, k, int(experts), int(ff), top,
           w_gate_up.tiles.data_ptr(), w_down.tiles.data_ptr(), chosen.data_ptr(), weights.data_ptr(),
           scratch["where"].data_ptr(), scratch["order"].data_ptr(), scratch["tiles"].data_ptr(),
           scratch["num_tiles"].data_ptr(), max_tiles, scratch["act"].data_ptr(), scratch["y"].data_ptr(),
-          residual.data_ptr(), 1 if weigh_input else 0, 1 if fresh else 0, code, lim,
-          -1 if many_rows is None else int(many_rows), 1 if planned else 0, _stream()), "moe_grouped")
+          1 if weigh_input else 0, code, lim, -1 if many_rows is None else int(many_rows), 1 if planned else 0,
+          _stream()), "moe_grouped")
+    if combine:
+        moe_combine(residual, scratch["y"], x, chosen, None if weigh_input else weights, scratch["where"], experts, fresh)
+
+
+def _combine_args(residual, y, x, chosen, weights, where, who: str) -> tuple[int, int, int]:
+    n, k = residual.shape
+    top = chosen.shape[1]
+    _check(residual, "residual", F32, (n, k))
+    _check(y, "y", BF16, (n * top, k))
+    _check(x, "x", BF16, (n, k))
+    _check(chosen, "chosen", I32, (n, top))
+    if weights is not None:
+        _check(weights, "weights", F32, (n, top))
+    _check(where, "where", I32, (n * top,))
+    if k % 8:
+        raise KernelError(f"{who}: rows of {k} elements are not whole eights")
+    return n, k, top
+
+
+def moe_combine(residual: torch.Tensor, y: torch.Tensor, x: torch.Tensor, chosen: torch.Tensor, weights: torch.Tensor | None,
+                where: torch.Tensor, experts: int, fresh: bool = False) -> None:
+    """The last step of ``moe_grouped``: ``residual[n] += sum_k weights[n, k] * y[where[n, k]]`` over the token's choices (``x[n]``
+    for a choice ``>= experts``), in their order.  ``weights`` ``None``: ones.  ``fresh``: written, not added to."""
+    n, k, top = _combine_args(residual, y, x, chosen, weights, where, "moe_combine")
+    f = _fn("moe", "kvf_moe_combine", [c_void_p] * 6 + [c_int] * 5 + [c_void_p])
+    _ok(f(residual.data_ptr(), y.data_ptr(), x.data_ptr(), chosen.data_ptr(), weights.data_ptr() if weights is not None else None,
+          where.data_ptr(), n, k, top, int(experts), 1 if fresh else 0, _stream()), "moe_combine")
+
+
+def moe_combine_norm_takes(residual: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor | None, out: torch.Tensor) -> bool:
+    """Whether ``moe_combine_norm`` takes these: fp32 weights, bf16 outputs, contiguous rows of whole eights, at most
+    16 elements a thread of the norm."""
+    n, h = residual.shape
+    return (out.dtype == BF16 and w1.dtype == F32 and (w2 is None or w2.dtype == F32) and h % 8 == 0
+            and h <= 16 * (256 if h >= 1024 else 128 if h >= 256 else 64)
+            and all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (residual, w1, w2, out)))
+
+
+def moe_combine_norm(residual: torch.Tensor, pre: torch.Tensor | None, y: torch.Tensor, x: torch.Tensor, chosen: torch.Tensor,
+                     weights: torch.Tensor | None, where: torch.Tensor, experts: int, post: torch.Tensor | None,
+                     w1: torch.Tensor, w2: torch.Tensor | None, eps: float, out1: torch.Tensor, out2: torch.Tensor | None) -> None:
+    """``residual += pre``, ``moe_combine``, ``residual += post`` and the norm that reads the rows next, ``rmsnorm`` into ``out1`` or
+    with ``w2`` ``rmsnorm_pair`` into both, in one pass with the same bits.  ``pre``, ``post``: bf16 or fp32, may be ``None``.
+    ``x`` may be one of the outputs.  Callers ask ``moe_combine_norm_takes`` first."""
+    n, h, top = _combine_args(residual, y, x, chosen, weights, where, "moe_combine_norm")
+    for t, name in ((pre, "pre"), (post, "post")):
+        if t is not None:
+            _check(t, name, None, (n, h))
+            _tcode(t.dtype)
+    for w, out, name in ((w1, out1, "1"), (w2, out2, "2")):
+        if w is not None or out is not None:
+            _check(w, "w" + name, F32, (h,))
+            _check(out, "out" + name, BF16, (n, h))
+    if not moe_combine_norm_takes(residual, w1, w2, out1):
+        raise KernelError("moe_combine_norm: operands it does not take (see moe_combine_norm_takes)")
+    ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
+    f = _fn("elementwise", "kvf_combine_norm", [c_void_p, c_void_p, c_int] + [c_void_p] * 5 + [c_int, c_int, c_void_p, c_int]
+            + [c_void_p] * 2 + [c_float] + [c_void_p] * 2 + [c_int, c_int, c_void_p])
+    _ok(f(residual.data_ptr(), ptr(pre), 1 if pre is not None and pre.dtype == F32 else 0, y.data_ptr(), x.data_ptr(),
+          chosen.data_ptr(), ptr(weights), where.data_ptr(), top, int(experts), ptr(post),
+          1 if post is not None and post.dtype == F32 else 0, w1.data_ptr(), ptr(w2), float(eps), out1.data_ptr(), ptr(out2),
+          n, h, _stream()), "moe_combine_norm")
 
 
 

@@ -187,11 +187,11 @@ class Transformer:
             raise ValueError("the greedy tail is for steps of single tokens that all want their "
                              "logits, on a model that can_pick")
         if r == 0:
-            step.owed = step.owed_bias = None
+            step.owed = step.owed_bias = step.owed_experts = None
             return torch.empty((0, cfg.vocab_size), dtype=torch.float32, device=residual.device)
         x = step.ws.buf("final_normed", (r, hidden), step.act_dtype)
         # only the wanted rows matter now: what is still owed to the stream is added to them alone
-        norm_rows(spec.final_norm, residual, x, step, step.logits_rows)
+        norm_rows(spec.final_norm, residual, x, step, None if step.all_rows else step.logits_rows)
         if tail is not None:
             spec.head.pick(x, residual, step, tail)
             return None

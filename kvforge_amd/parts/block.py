@@ -12,8 +12,24 @@ from kvforge_amd.parts.base import (Block, FeedForward, LayerState, Mixer, Norm,
 from kvforge_amd.registry import register_block
 
 
+def norm_experts(stream: torch.Tensor, step, w1: torch.Tensor, w2: torch.Tensor | None, eps: float, out1: torch.Tensor,
+                 out2: torch.Tensor | None) -> bool:
+    """Whether experts were owed to ``stream`` and have been added by the kernel that also took its norm (or both norms)."""
+    if step.owed_experts is None or not ops.moe_combine_norm_takes(stream, w1, w2, out1):
+        return False
+    owed = step.take_owed_experts(stream)
+    if owed is None:
+        return False
+    pre, combine, post = owed
+    ops.moe_combine_norm(stream, pre, *combine, post, w1, w2, eps, out1, out2)
+    return True
+
+
 def norm_rows(norm: Norm, stream: torch.Tensor, out: torch.Tensor, step, rows: torch.Tensor | None = None) -> None:
     """``out = norm(stream)`` (of the rows ``rows``), with what the step still owes the stream added on the way."""
+    weight = norm.fp32_weight() if rows is None and step.owed_experts is not None and hasattr(norm, "fp32_weight") else None
+    if weight is not None and norm_experts(stream, step, weight, None, norm.eps, out, None):
+        return
     if norm.adds_bias and step.owed_bias is not None:
         bias = step.take_owed_bias(stream)
         norm.forward(stream, out, rows, add=step.take_owed(stream, norm.takes_parts), bias=bias)
@@ -145,8 +161,9 @@ class ParallelBlock(Block):
             # two RMS norms of the same stream: one pass over it, two weights
             hs = h
             h = step.ws.buf("parallel_normed_ffn", shape, step.act_dtype)
-            ops.rmsnorm_pair(residual, self.norm.weight, self.ffn_norm.weight, self.norm.eps, hs, h,
-                             add=step.take_owed(residual))
+            if not norm_experts(residual, step, self.norm.weight, self.ffn_norm.weight, self.norm.eps, hs, h):
+                ops.rmsnorm_pair(residual, self.norm.weight, self.ffn_norm.weight, self.norm.eps, hs, h,
+                                 add=step.take_owed(residual))
         else:
             norm_rows(self.norm, residual, h, step)
             hs = h

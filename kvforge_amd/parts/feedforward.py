@@ -159,11 +159,10 @@ class GatedFeedForward(SwiGLU):
         act = step.ws.buf("ffn_act", (x.shape[0], self.inter), step.act_dtype)
         return [((self.prefix, "act"), x, self.w_gate_up, act, True)]
 
-    def forward(self, x, step, residual) -> None:
-        """``x``: normalised activations."""
+    def activations(self, x, step) -> torch.Tensor:
+        """What the down projection reads."""
         n = x.shape[0]
         ws, dt = step.ws, step.act_dtype
-        step.settle()
         act = ws.buf("ffn_act", (n, self.inter), dt)
         first = self.input_products(x, step)
         if first:
@@ -177,6 +176,12 @@ class GatedFeedForward(SwiGLU):
             ops.gemm(x, self.w_gate_up, gu)
             ops.gated_act(gu, act, self.activation, paired=True, gate_bias=self.gate_bias,
                           up_bias=self.up_bias, limit=self.limit, scale=self.out_scale)
+        return act
+
+    def forward(self, x, step, residual) -> None:
+        """``x``: normalised activations."""
+        step.settle()
+        act = self.activations(x, step)
         add_product(step, act, self.w_down, residual)
         if self.down_bias is not None and not self.defer_down_bias:
             step.owe_bias(residual, self.down_bias)

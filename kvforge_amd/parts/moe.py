@@ -51,6 +51,7 @@ class RoutedExperts(FeedForward):
              "router_bias": "router.b"}
 
     replayable = True
+    settles_residual = True      # what is owed goes along with the experts' sum, or is added first
 
     def __init__(self, prefix: str, hidden: int, ff: int, experts: int, top: int, identity: int = 0,
                  shared_ff: int = 0, names: dict[str, str] | None = None, table_vocab: int | None = None,
@@ -198,11 +199,16 @@ class RoutedExperts(FeedForward):
         """``x``: normalised activations."""
         n = x.shape[0]
         ws, dt = step.ws, step.act_dtype
+        grouped = ops.moe_grouped_takes(x, self.w_gate_up, self.w_down, self.E, self.ff) and x.is_contiguous()
+        # the sum over the experts may wait for the norm that reads the stream next, and what is owed now with it
+        later = (grouped and step.fresh is not residual and residual.is_contiguous() and self.hidden % 8 == 0
+                 and residual.data_ptr() % 16 == 0
+                 and (self.shared is None or self._shared_type(x, step) is not None))
+        pre = step.take_owed(residual) if later else None
         step.settle()
         step.make_early([p for p in self.input_products(x, step) if p[0] not in step.made])
         chosen = ws.buf("moe_chosen", (n, self.top), torch.int32)
         weights = ws.buf("moe_weights", (n, self.top), torch.float32)
-        grouped = ops.moe_grouped_takes(x, self.w_gate_up, self.w_down, self.E, self.ff) and x.is_contiguous()
         if grouped:
             pairs, tiles = n * self.top, ops.moe_grouped_tiles(n, self.top, self.E)
             scratch = {"where": ws.buf("moe_where", (pairs,), torch.int32),
@@ -228,8 +234,12 @@ class RoutedExperts(FeedForward):
                 step.fresh = None      # written here instead of added to
             ops.moe_grouped(x, self.w_gate_up, self.w_down, chosen, weights, residual, self.E, self.ff, scratch,
                             weigh_input=self.weigh_input, fresh=fresh, form=self.form, limit=self.limit,
-                            planned=planned)
-            self._shared_forward(x, step, residual)
+                            planned=planned, combine=not later)
+            if later:
+                step.owe_experts(residual, pre, (scratch["y"], x, chosen, None if self.weigh_input else weights, scratch["where"],
+                                                 self.E), self._shared_rows(x, step))
+            else:
+                self._shared_forward(x, step, residual)
             return
         # otherwise (32-bit, or sizes the grouped kernels do not take): every expert over every
         # row in one product, the rows that did not choose it multiplied by an exact zero
@@ -244,6 +254,25 @@ class RoutedExperts(FeedForward):
         if self.identity and not first:     # fresh rows are written by the product before they are added to
             ops.moe_identity(residual, x, chosen, weights, self.E)
         self._shared_forward(x, step, residual)
+
+    def _shared_type(self, x, step) -> torch.dtype | None:
+        """The type of the shared expert's output where it is made as rows of its own, which join the stream behind the experts with
+        the bits that ``parts.base.add_product`` gives them: fp32 sums of the kernel of few rows, many rows as the library
+        stores them.  ``None`` where ``add_product`` has another form, or a gate joins in."""
+        sh, n = self.shared, x.shape[0]
+        act = step.ws.buf("ffn_act", (n, sh.inter), step.act_dtype)
+        if self.w_shared_gate is not None or sh.down_bias is not None or act.dtype != torch.bfloat16 or not ops.bf16_kernel_takes(act[:1], sh.w_down):
+            return None
+        if n <= ops.FUSED_NORM_MAX_M:
+            return None if ops.k_halves_pay(act, sh.w_down) else torch.float32
+        return act.dtype if n > ops.MID_MAX_M and ops.is_library_product(act, sh.w_down) else None
+
+    def _shared_rows(self, x, step) -> torch.Tensor | None:
+        if self.shared is None:
+            return None
+        rows = step.ws.buf("moe_shared_rows", (x.shape[0], self.hidden), self._shared_type(x, step))
+        ops.gemm(self.shared.activations(x, step), self.shared.w_down, rows)
+        return rows
 
     def _shared_forward(self, x, step, residual) -> None:
         if self.shared is None:

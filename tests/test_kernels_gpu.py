@@ -616,6 +616,39 @@ def test_gemm_group_has_the_bits_of_the_single_products(m, shapes):
         ops().gemm_group(products * 3)
 
 
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("n,h,top,E,pre,post", [(1, 8, 1, 2, None, None), (3, 248, 2, 3, "f32", "bf16"), (8, 1024, 4, 6, None, "f32"),
+                                                 (5, 2048, 4, 6, "bf16", "bf16"), (300, 2040, 3, 5, "bf16", None), (2, 4096, 16, 9, None, "f32")])
+def test_experts_sum_and_the_next_norm_have_the_bits_of_their_steps(n, h, top, E, pre, post, two):
+    """What is owed before the experts, their sum (choices that name an expert, the row itself, or nothing), what is owed
+    behind, and one or two norms, against the kernels of the single steps: the stream and the outputs, with the
+    experts' input in the memory of an output."""
+    g = torch.Generator().manual_seed(n + h)
+    x = torch.randn(n, h, generator=g).to(DEV)
+    types = {"f32": torch.float32, "bf16": torch.bfloat16}
+    before, behind = (torch.randn(n, h, generator=g).to(types[t]).to(DEV) if t else None for t in (pre, post))
+    y = torch.randn(n * top, h, generator=g).to(torch.bfloat16).to(DEV)
+    rows = torch.randn(n, h, generator=g).to(torch.bfloat16).to(DEV)
+    chosen = torch.randint(-1, E + 2, (n, top), generator=g, dtype=torch.int32).to(DEV)
+    weights = torch.rand(n, top, generator=g).to(DEV)
+    where = torch.randperm(n * top, generator=g).to(torch.int32).to(DEV)
+    w1, w2 = (torch.randn(h, generator=g).to(DEV) for _ in range(2))
+    for wgt in (weights, None):
+        want_x, want = x.clone(), [torch.empty_like(rows) for _ in range(2)]
+        if before is not None:
+            ops().add_rows(want_x, before)
+        ops().moe_combine(want_x, y, rows, chosen, wgt, where, E)
+        if two:
+            ops().rmsnorm_pair(want_x, w1, w2, 1e-6, *want, add=behind)
+        else:
+            ops().rmsnorm(want_x, w1, 1e-6, want[0], add=behind)
+        got_x, own = x.clone(), rows.clone()
+        out1, out2 = (torch.empty_like(rows), own) if two else (own, None)
+        assert ops().moe_combine_norm_takes(got_x, w1, w2 if two else None, out1)
+        ops().moe_combine_norm(got_x, before, y, own, chosen, wgt, where, E, behind, w1, w2 if two else None, 1e-6, out1, out2)
+        assert torch.equal(got_x, want_x) and torch.equal(out1, want[0]) and (not two or torch.equal(out2, want[1]))
+
+
 @pytest.mark.parametrize("tile", range(6))
 @pytest.mark.parametrize("m,k,H,KV,d,rot,bs,extra", [
     (65, 64, 4, 2, 16, 16, 8, 0),          # one stage of K; fewer columns than a tile
