@@ -741,7 +741,7 @@ __global__ __launch_bounds__(MID_WAVES * KVF_WAVE, 4) void gemm_mid_kernel(
   }
 }
 
-// Several products of at most 16 bf16 rows over tiled weights in one launch (EPI 0, 1 or 3 each, inputs of their own):
+// Several products of at most 16 bf16 rows over tiled weights in one launch (EPI 0 to 3 each, inputs of their own):
 // the projections that a step's parts begin with.  In a decode step each is a kernel of 4 to 7 us whose time is its
 // launch and two trips to memory; together those come once.  Eight rows of 2,048, a recurrence's rows, its gates, a router
 // and a gated pair of 4,096 columns: 7.0 + 4.6 + 4.6 + 6.0 us apart, 9.7 together.  A workgroup takes 16 columns of one product as gemm_skinny_kernel<1, 1, 0,
@@ -770,6 +770,10 @@ __global__ __launch_bounds__(GROUP_WAVES * KVF_WAVE) void gemm_group_kernel(Grou
   const bool live = r16 < M;
   const bf16_t* ap = it.A + static_cast<size_t>(live ? r16 : 0) * it.lda + kg * 8;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  EpiOperands pre;                     // what the product is added to, asked for now (see EpiOperands)
+  pre.have = false;
+  if (it.epi == 2 && wave == 0 && live && n0 + 4 * kg < it.N)
+    epi_prefetch_a<2>(pre, r16, n0 + 4 * kg, it.N, it.ldc, it.C, nullptr, rp);
   constexpr int U = depth(1, 1, 0), nw = GROUP_WAVES;
   int ks = wave;
   for (; ks + (U - 1) * nw < ksteps; ks += U * nw) {
@@ -799,6 +803,7 @@ __global__ __launch_bounds__(GROUP_WAVES * KVF_WAVE) void gemm_group_kernel(Grou
   none.have = false;
   if (it.epi == 0) store_tile<0>(s, r16, n, it.N, it.ldc, it.C, nullptr, rp, none);
   else if (it.epi == 1) store_tile<1>(s, r16, n, it.N, it.ldc, it.C, nullptr, rp, none);
+  else if (it.epi == 2) store_tile<2>(s, r16, n, it.N, it.ldc, it.C, nullptr, rp, pre);
   else store_tile<3>(s, r16, n, it.N, it.ldc, it.C, nullptr, rp, none);
 }
 
@@ -1000,7 +1005,7 @@ KVF_EXPORT int kvf_gemm_bf16(const void* A, int a_type, const void* W, int w_til
 }
 
 // Several products of M <= 16 rows in one launch (see gemm_group_kernel).  items: for each A, W, C (addresses), N, K, lda, ldc
-// and epi (0 store fp32, 1 store bf16, 3 SwiGLU pairs -> bf16 [M, N/2]); W in tiles, K beyond 224 (a k-step for every wave).
+// and epi (0 store fp32, 1 store bf16, 2 add into fp32, 3 SwiGLU pairs -> bf16 [M, N/2]); W in tiles, K beyond 224 (a k-step for every wave).
 KVF_EXPORT int kvf_gemm_bf16_group(const long long* items, int count, int M, hipStream_t s) {
   if (M <= 0 || count <= 0) return 0;
   if (M > 16 || count > GROUP_MAX) return static_cast<int>(hipErrorInvalidValue);
@@ -1013,7 +1018,7 @@ KVF_EXPORT int kvf_gemm_bf16_group(const long long* items, int count, int M, hip
                    static_cast<int>(v[3]), static_cast<int>(v[4]), static_cast<int>(v[5]), static_cast<int>(v[6]),
                    static_cast<int>(v[7]), blocks};
     if (!it.A || !it.W || !it.C || it.N <= 0 || it.K <= 224 || it.K % 8 != 0 || it.lda % 8 != 0 || v[0] % 16 != 0 || v[1] % 16 != 0 ||
-        !(it.epi == 0 || it.epi == 1 || (it.epi == 3 && it.N % 4 == 0)))
+        !(it.epi >= 0 && (it.epi <= 2 || (it.epi == 3 && it.N % 4 == 0))))
       return static_cast<int>(hipErrorInvalidValue);
     blocks += (it.N + 15) / 16;
   }

@@ -233,6 +233,10 @@ class Step:
         self.settled_next = False
         # products that a block has had made together with others, ahead of the parts they belong to
         self.made: set = set()
+        # products that are ready and ride with the next one that a mixer ends in; whether a mixer's last product waits for
+        # another's instead of being made (rows of its own only)
+        self.riders: list = []
+        self.wait = False
         # the staging memory this step was filled from (``fill_step``), for ``upload_ints``
         self._meta: "MetaBuffers | None" = None
         self._turn = 0
@@ -257,15 +261,28 @@ class Step:
         return dst
 
     def make(self, products: list) -> None:
-        """Make a part's products ``(key, a, w, out, pairs)`` (see ``Mixer.input_products``) that have not been made
+        """Make a part's products ``(key, a, w, out, how)`` (see ``Mixer.input_products``) that have not been made
         yet: with few rows several of them in one launch."""
-        rest = [p for p in products if p[0] not in self.made]
-        self.made.difference_update(p[0] for p in products)
-        done = self._make_together(rest)
         from kvforge_amd.kernels import ops
-        for key, a, w, out, pairs in rest:
+        rest, done = products, ()
+        if products[0][1].shape[0] <= ops.FUSED_NORM_MAX_M:
+            rest = [p for p in products if p[0] not in self.made]
+            self.made.difference_update(p[0] for p in products)
+            done = self._make_together(rest)
+        for key, a, w, out, how in rest:
             if key not in done:
-                (ops.gemm_gated if pairs else ops.gemm)(a, w, out)
+                (ops.gemm_gated if how == "pairs" else ops.gemm)(a, w, out)
+
+    def ride(self, product: tuple) -> bool:
+        """Make ``product`` and, in the same launch, those that wait for such a one (``riders``).  ``False`` where none
+        does, or the product is not one that takes others along: the caller makes it by itself."""
+        from kvforge_amd.kernels import ops
+        if not self.riders or not ops.gemm_group_takes(*product[1:4]):
+            return False
+        along, self.riders = self.riders[:ops.GROUP_MAX - 1], self.riders[ops.GROUP_MAX - 1:]
+        ops.gemm_group([p[1:] for p in (product, *along)])
+        self.made.update(p[0] for p in along)
+        return True
 
     def make_early(self, products: list) -> None:
         """Products that several parts are going to begin with and whose inputs are there: those that

@@ -1091,17 +1091,20 @@ def gemm_group_takes(a: torch.Tensor, w, out: torch.Tensor) -> bool:
 
 
 def gemm_group(products) -> None:
-    """Several products ``out = a @ w.T`` of equally many rows in one launch: ``(a, w, out, pairs)`` each, ``out`` fp32 or bf16;
-    with ``pairs`` neighbouring columns are (gate, up) and ``out = silu(gate) * up`` (``gemm_gated`` without
-    biases).  For products that ``gemm_group_takes``; the bits of ``gemm`` and ``gemm_gated``."""
+    """Several products ``out = a @ w.T`` of equally many rows in one launch: ``(a, w, out, how)`` each, ``out`` fp32 or bf16, ``how``
+    ``"store"``, ``"add"`` (``out += a @ w.T``, fp32) or ``"pairs"``: neighbouring columns are (gate, up) and ``out = silu(gate) * up``
+    (``gemm_gated`` without biases).  For products that ``gemm_group_takes``; the bits of ``gemm`` and ``gemm_gated``.  No product
+    reads what another writes."""
     if not 0 < len(products) <= GROUP_MAX:
         raise KernelError(f"gemm_group: 1 to {GROUP_MAX} products, got {len(products)}")
     rows, items = products[0][0].shape[0], []
-    for a, w, out, pairs in products:
-        m, n, k, lda, ldc = _gemm_operands(a, w, out, (lambda n: n // 2) if pairs else (lambda n: n))
-        if m != rows or not gemm_group_takes(a, w, out) or (pairs and (n % 4 or out.dtype != BF16)):
+    for a, w, out, how in products:
+        m, n, k, lda, ldc = _gemm_operands(a, w, out, (lambda n: n // 2) if how == "pairs" else (lambda n: n))
+        epi = {"store": 0 if out.dtype == F32 else 1, "add": 2, "pairs": 3}.get(how)
+        if (m != rows or epi is None or not gemm_group_takes(a, w, out) or (epi == 3 and (n % 4 or out.dtype != BF16))
+                or (epi == 2 and out.dtype != F32)):
             raise KernelError("gemm_group: operands do not fit the kernel")
-        items += [a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), n, k, lda, ldc, 3 if pairs else 0 if out.dtype == F32 else 1]
+        items += [a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), n, k, lda, ldc, epi]
     f = _fn("gemm_bf16", "kvf_gemm_bf16_group", [c_void_p, c_int, c_int, c_void_p])
     _ok(f((c_longlong * len(items))(*items), len(products), rows, _stream()), "gemm_group")
 

@@ -162,6 +162,7 @@ class PagedAttention(Mixer):
              "g": "g_proj.weight"}
 
     replayable = True
+    buffers = "attn"
     shares_slot = True
     settles_residual = True  # its norm kernel adds what is owed to the stream
 
@@ -497,10 +498,10 @@ class PagedAttention(Mixer):
         out = []
         if self.norm_eps is None and self.row_norm is None and (self.conv is not None or self.qk_norm is not None or self._hooked()):
             rows = ws.buf("conv_rows" if self.conv is not None else "qkv", (n, self.w_qkv.shape[0]), step.act_dtype)
-            out.append(((self.prefix, "qkv"), x, self.w_qkv, rows, False))
+            out.append(((self.prefix, "qkv"), x, self.w_qkv, rows, "store"))
         if self.norm_eps is None and self.w_head_gate is not None:
             gates = ws.buf("attn_head_gates", (n, self.w_head_gate.shape[0]), torch.float32)
-            out.append(((self.prefix, "head_gates"), x, self.w_head_gate, gates, False))
+            out.append(((self.prefix, "head_gates"), x, self.w_head_gate, gates, "store"))
         return out
 
     def forward(self, x, step, layer: LayerState, residual) -> None:
@@ -548,7 +549,7 @@ class PagedAttention(Mixer):
             if layer.state is None and self.conv[0] > 1:
                 raise RuntimeError("attention behind a convolution needs a state slot per request")
             rows = ws.buf("conv_rows", (n, self.w_qkv.shape[0]), act)
-            step.make([((self.prefix, "qkv"), x, self.w_qkv, rows, False)])
+            step.make([((self.prefix, "qkv"), x, self.w_qkv, rows, "store")])
             qkv = ws.buf("conv_q", (n, H * d), act)
             ops.conv_norm_kvwrite(rows, self.conv_w, step.cu_q, step.positions, step.slot_ids, layer.state, table, qkv,
                                   layer.k_pages, layer.v_pages, H, KV, d, step.n_seqs, max(step.q_lens),
@@ -569,7 +570,7 @@ class PagedAttention(Mixer):
         else:
             g0 = (H + (2 * KV if self.own_kv else 0)) * d
             qkv = ws.buf("qkv", (n, self.w_qkv.shape[0]), act)
-            step.make([((self.prefix, "qkv"), x, self.w_qkv, qkv, False)])
+            step.make([((self.prefix, "qkv"), x, self.w_qkv, qkv, "store")])
             self.after_projection(qkv, step)
             if self.qk_norm is not None:
                 ops.qknorm_rope_kvwrite(qkv, step.positions, step.seq_of_token, cos, sin, table,
@@ -583,7 +584,7 @@ class PagedAttention(Mixer):
         head_gates = None
         if self.w_head_gate is not None:
             head_gates = ws.buf("attn_head_gates", (n, self.w_head_gate.shape[0]), torch.float32)
-            step.make([((self.prefix, "head_gates"), x, self.w_head_gate, head_gates, False)])
+            step.make([((self.prefix, "head_gates"), x, self.w_head_gate, head_gates, "store")])
         out = ws.buf("attn_out", (n, H * d), act)
         window, chunk = self.window or 0, self.chunk or 0
         bs = layer.k_pages.shape[2]

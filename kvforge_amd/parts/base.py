@@ -208,14 +208,18 @@ class Mixer(Part):
 
     settles_residual = False
 
+    # Names the workspace buffers that this make of mixer keeps its rows in, which no other make touches: the last products of two
+    # mixers of different makes may then be made together, behind both.  ``None``: not known.
+    buffers: str | None = None
+
     cache_spec: CacheSpec | None = None
     state_spec: StateSpec | None = None
     # whether ``LayerState.state`` may be a block of columns of wider slots (``[slots, floats]``, dense rows)
     shares_slot = False
 
     def input_products(self, x: torch.Tensor, step: "Step") -> list:
-        """The products over ``x`` alone that ``forward`` begins with, as ``(key, a, w, out, pairs)``: ``out = a @ w.T``, with
-        ``pairs`` of (gate, up) columns ``silu(gate) * up``; ``key`` names the product within the model.  ``forward`` hands the same list
+        """The products over ``x`` alone that ``forward`` begins with, as ``(key, a, w, out, how)``: ``how`` is ``"store"``
+        (``out = a @ w.T``) or ``"pairs"`` (of (gate, up) columns ``silu(gate) * up``); ``key`` names the product within the model.  ``forward`` hands the same list
         to ``step.make``, which leaves out what a block has had made already (``Step.make_early``), side by side with
         other parts' products.  Only for an ``x`` of the step's activation type."""
         return []
@@ -231,6 +235,11 @@ class FeedForward(Part):
 
     def input_products(self, x: torch.Tensor, step: "Step") -> list:
         """As ``Mixer.input_products``."""
+        return []
+
+    def ready_products(self, x: torch.Tensor, step: "Step") -> list:
+        """Further products of ``forward`` whose inputs are there once those of ``input_products`` have been made
+        (``step.made``): they may ride with a product of the mixer beside it (``Step.riders``)."""
         return []
 
     def forward(self, x: torch.Tensor, step: "Step", residual: torch.Tensor) -> None:
@@ -324,12 +333,12 @@ class Block(Part):
         return all(p.replayable for p in self.parts())
 
 
-def products_of(part: Part, x: torch.Tensor, step: "Step") -> list:
-    """``part.input_products(x, step)``, unless a subclass has given the part another ``forward``, of which the list that
-    it inherits says nothing."""
+def products_of(part: Part, x: torch.Tensor, step: "Step", which: str = "input_products") -> list:
+    """``part.input_products(x, step)`` (or ``which``), unless a subclass has given the part another ``forward``, of which
+    the list that it inherits says nothing."""
     for cls in type(part).__mro__:
-        if "input_products" in vars(cls):
-            return part.input_products(x, step)
+        if which in vars(cls):
+            return getattr(part, which)(x, step)
         if "forward" in vars(cls):
             return []
     return []
@@ -357,7 +366,11 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
 
     if getattr(step, "fresh", None) is residual:
         step.fresh = None
-        ops.gemm(a, w, residual)
+        if getattr(step, "wait", False) and owed is None and ops.gemm_group_takes(a, w, residual):
+            step.riders.append((("rider", len(step.riders)), a, w, residual, "store"))     # the block has it made
+            return
+        if not step.ride((None, a, w, residual, "store")):
+            ops.gemm(a, w, residual)
         if owed is not None:
             ops.add_rows(residual, owed)
         return
@@ -389,7 +402,7 @@ def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.
             half = step.ws.buf("owed_half_other", tuple(residual.shape), torch.bfloat16)
         ops.gemm(a, w, residual, accumulate=True, owed=owed, half_out=half)
         step.owe(residual, half)
-    else:
+    elif owed is not None or not step.ride((None, a, w, residual, "add")):
         ops.gemm(a, w, residual, accumulate=True, owed=owed)
 
 

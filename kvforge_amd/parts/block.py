@@ -175,9 +175,12 @@ class ParallelBlock(Block):
         # `after` or to the next block's norms, of which only a single one takes parts
         behind = pair or self.mu is not None or self.after is not None
         step.settled_next = self.ffn is not None or behind
-        # both sublayers' inputs are there: what they begin with is made together
-        step.make_early(products_of(self.mixer, hs, step) + (products_of(self.ffn, h, step) if self.ffn is not None else []))
+        if shape[0] <= ops.FUSED_NORM_MAX_M and self.ffn is not None:
+            # both sublayers' inputs are there: what they begin with is made together
+            step.make_early(products_of(self.mixer, hs, step) + products_of(self.ffn, h, step))
+            step.riders = [p for p in products_of(self.ffn, h, step, "ready_products") if ops.gemm_group_takes(*p[1:4])]
         self.mixer.forward(hs, step, layer, residual)
+        step.riders = []             # what has not been taken along is made by the feed-forward
         step.settled_next = behind
         bias = None
         if self.ffn is not None:

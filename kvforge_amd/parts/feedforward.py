@@ -157,7 +157,7 @@ class GatedFeedForward(SwiGLU):
                 or not ops.bf16_kernel_takes(x, self.w_gate_up, False, True)):
             return []
         act = step.ws.buf("ffn_act", (x.shape[0], self.inter), step.act_dtype)
-        return [((self.prefix, "act"), x, self.w_gate_up, act, True)]
+        return [((self.prefix, "act"), x, self.w_gate_up, act, "pairs")]
 
     def activations(self, x, step) -> torch.Tensor:
         """What the down projection reads."""

@@ -33,6 +33,7 @@ class MatrixLSTM(Mixer):
     NAMES = {"q": "q", "k": "k", "v": "v", "g": "g", "o": "o", "norm": "norm", "i": "i", "f": "f"}
 
     replayable = True
+    buffers = "mlstm"
     cache_spec = None
 
     def __init__(self, prefix: str, hidden: int, heads: int, key_dim: int, value_dim: int,
@@ -115,7 +116,7 @@ class MatrixLSTM(Mixer):
         n, ws = x.shape[0], step.ws
         rows = ws.buf("mlstm_rows", (n, 2 * self.H * (self.dk + self.dv)), step.act_dtype)
         gates = ws.buf("mlstm_gates", (n, self.G_pad), torch.float32)
-        return [((self.prefix, "rows"), x, self.w_rows, rows, False), ((self.prefix, "gates"), x, self.w_gates, gates, False)]
+        return [((self.prefix, "rows"), x, self.w_rows, rows, "store"), ((self.prefix, "gates"), x, self.w_gates, gates, "store")]
 
     def forward(self, x, step, layer: LayerState, residual) -> None:
         """``x``: normalised activations."""

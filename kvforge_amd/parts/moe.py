@@ -190,7 +190,7 @@ class RoutedExperts(FeedForward):
         out = []
         if self.table is None:
             logits = step.ws.buf("moe_logits", (x.shape[0], self.R_pad), torch.float32)     # 32-bit sums, stored so
-            out.append(((self.prefix, "router"), x, self.w_router, logits, False))
+            out.append(((self.prefix, "router"), x, self.w_router, logits, "store"))
         if self.shared is not None and self.w_shared_gate is None:
             out += self.shared.input_products(x, step)
         return out
@@ -201,12 +201,13 @@ class RoutedExperts(FeedForward):
         ws, dt = step.ws, step.act_dtype
         grouped = ops.moe_grouped_takes(x, self.w_gate_up, self.w_down, self.E, self.ff) and x.is_contiguous()
         # the sum over the experts may wait for the norm that reads the stream next, and what is owed now with it
-        later = (grouped and step.fresh is not residual and residual.is_contiguous() and self.hidden % 8 == 0
-                 and residual.data_ptr() % 16 == 0
-                 and (self.shared is None or self._shared_type(x, step) is not None))
+        later = grouped and step.fresh is not residual and self.hidden % 8 == 0
+        shared_type = self._shared_type(x, step) if later and self.shared is not None else None
+        later = later and (self.shared is None or shared_type is not None)
         pre = step.take_owed(residual) if later else None
         step.settle()
-        step.make_early([p for p in self.input_products(x, step) if p[0] not in step.made])
+        if n <= ops.FUSED_NORM_MAX_M:
+            step.make_early([p for p in self.input_products(x, step) if p[0] not in step.made])
         chosen = ws.buf("moe_chosen", (n, self.top), torch.int32)
         weights = ws.buf("moe_weights", (n, self.top), torch.float32)
         if grouped:
@@ -222,7 +223,7 @@ class RoutedExperts(FeedForward):
             ops.moe_table(step.token_ids, self.table, chosen, weights, self.E)
         else:
             logits = ws.buf("moe_logits", (n, self.R_pad), torch.float32)
-            step.make([((self.prefix, "router"), x, self.w_router, logits, False)])
+            step.make([((self.prefix, "router"), x, self.w_router, logits, "store")])
             logits = logits[:, :self.R]
             ops.moe_topk(logits, self.correction, chosen, weights, self.scores, self.renormalize, bias=self.r_bias,
                          scale=self.out_scale,
@@ -237,7 +238,7 @@ class RoutedExperts(FeedForward):
                             planned=planned, combine=not later)
             if later:
                 step.owe_experts(residual, pre, (scratch["y"], x, chosen, None if self.weigh_input else weights, scratch["where"],
-                                                 self.E), self._shared_rows(x, step))
+                                                 self.E), self._shared_rows(x, step, shared_type))
             else:
                 self._shared_forward(x, step, residual)
             return
@@ -267,12 +268,26 @@ class RoutedExperts(FeedForward):
             return None if ops.k_halves_pay(act, sh.w_down) else torch.float32
         return act.dtype if n > ops.MID_MAX_M and ops.is_library_product(act, sh.w_down) else None
 
-    def _shared_rows(self, x, step) -> torch.Tensor | None:
+    def _shared_rows(self, x, step, dtype: torch.dtype | None) -> torch.Tensor | None:
         if self.shared is None:
             return None
-        rows = step.ws.buf("moe_shared_rows", (x.shape[0], self.hidden), self._shared_type(x, step))
-        ops.gemm(self.shared.activations(x, step), self.shared.w_down, rows)
-        return rows
+        product = self._shared_product(x, self.shared.activations(x, step), step, dtype)
+        step.make([product])
+        return product[3]
+
+    def _shared_product(self, x, act, step, dtype: torch.dtype) -> tuple:
+        rows = step.ws.buf("moe_shared_rows", (x.shape[0], self.hidden), dtype)
+        return (self.prefix, "shared_rows"), act, self.shared.w_down, rows, "store"
+
+    def ready_products(self, x, step) -> list:
+        """The shared expert's last product, once its pair has been made, where its output is rows of its own."""
+        if (self.shared is None or (self.shared.prefix, "act") not in step.made
+                or not ops.moe_grouped_takes(x, self.w_gate_up, self.w_down, self.E, self.ff)):
+            return []
+        dtype = self._shared_type(x, step)
+        if dtype is None:
+            return []
+        return [self._shared_product(x, step.ws.buf("ffn_act", (x.shape[0], self.shared.inter), step.act_dtype), step, dtype)]
 
     def _shared_forward(self, x, step, residual) -> None:
         if self.shared is None:

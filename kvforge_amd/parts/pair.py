@@ -104,19 +104,30 @@ class MixerPair(Mixer):
         """``x``: normalised activations.  Without norms, what the first leaves owed to the stream the
         second settles (or takes along) as any part does; with norms, each writes rows of its own."""
         ll, rl = self._layers(layer)
-        step.make_early([p for p in self.input_products(x, step) if p[0] not in step.made])
+        few = x.shape[0] <= ops.FUSED_NORM_MAX_M
+        if few:
+            step.make_early([p for p in self.input_products(x, step) if p[0] not in step.made])
         if self.norms is None:
             self.left.forward(x, step, ll, residual)
             self.right.forward(x, step, rl, residual)
             return
         step.settle()
         rows = []
+        # the first one's last product waits for the second one's, which takes it along, where the second leaves its rows alone
+        waits = few and None not in (self.left.buffers, self.right.buffers) and self.left.buffers != self.right.buffers
+        riders, step.riders = step.riders, []
         for m, state, name in ((self.left, ll, "pair_left_out"), (self.right, rl, "pair_right_out")):
             out = step.ws.buf(name, tuple(residual.shape), torch.float32)
             step.fresh = out
+            step.wait = waits and m is self.left
             m.forward(x, step, state, out)
+            step.wait = False
             if step.fresh is out:
                 raise RuntimeError("a mixer whose output passes a norm must write its fresh rows (end in "
                                    "parts.base.add_product)")
             rows.append(out)
+        for _, a, w, out, _how in step.riders:      # (not taken along)
+            ops.gemm(a, w, out)
+        step.made -= {key for key in step.made if key[0] == "rider"}
+        step.riders = riders
         ops.rms_add_two(residual, rows[0], self.weights[0], rows[1], self.weights[1], self.norms[0].eps)

@@ -42,6 +42,7 @@ class ConvMemory(Mixer):
     the gates' columns (``a_off``, ``b_off``) and what becomes of the read-out (``finish``)."""
 
     replayable = True
+    buffers = "ssm"
     shares_slot = True
     cache_spec = None
 
@@ -115,7 +116,7 @@ class ConvMemory(Mixer):
         n, ws = x.shape[0], step.ws
         rows = ws.buf("ssm_rows", (n, self.w_rows.shape[0]), step.act_dtype)
         gates = ws.buf("ssm_gates", (n, self.w_gates.shape[0]), torch.float32)     # 32-bit sums, stored so
-        return [((self.prefix, "rows"), x, self.w_rows, rows, False), ((self.prefix, "gates"), x, self.w_gates, gates, False)]
+        return [((self.prefix, "rows"), x, self.w_rows, rows, "store"), ((self.prefix, "gates"), x, self.w_gates, gates, "store")]
 
     def forward(self, x, step, layer: LayerState, residual) -> None:
         """``x``: the mixer's input rows in the step's activation type."""

@@ -588,7 +588,7 @@ def test_gemm_qkv_rope_equals_the_three_steps(m, H, KV, d, rot, bs, rms):
 
 @pytest.mark.parametrize("m", [1, 3, 8, 16])
 @pytest.mark.parametrize("shapes", [
-    [(48, 2048, "f32"), (3072, 2048, "bf16"), (4096, 2048, "pairs")],
+    [(48, 2048, "f32"), (3072, 2048, "bf16"), (4096, 2048, "pairs"), (2048, 2048, "add"), (18, 776, "add")],
     [(16, 232, "f32"), (20, 256, "bf16"), (36, 2056, "pairs"), (8176, 264, "bf16"), (4, 1000, "f32"), (33, 480, "f32"),
      (17, 768, "bf16"), (16, 512, "pairs")]])
 def test_gemm_group_has_the_bits_of_the_single_products(m, shapes):
@@ -598,14 +598,14 @@ def test_gemm_group_has_the_bits_of_the_single_products(m, shapes):
     for n, k, kind in shapes:
         a = torch.randn(m, k + 16, generator=g).to(torch.bfloat16).to(DEV)[:, :k]
         w = ops().StreamedWeight((torch.randn(n, k, generator=g) / 20).to(torch.bfloat16).to(DEV))
-        cols, dtype = (n // 2 if kind == "pairs" else n), (torch.float32 if kind == "f32" else torch.bfloat16)
+        cols, dtype = (n // 2 if kind == "pairs" else n), (torch.float32 if kind in ("f32", "add") else torch.bfloat16)
         wide = torch.full((2, m, cols + 8), 7.0, dtype=dtype, device=DEV)    # rows of results further apart than they are wide
         if kind == "pairs":
             ops().gemm_gated(a, w, wide[0][:, :cols])
         else:
-            ops().gemm(a, w, wide[0][:, :cols])
+            ops().gemm(a, w, wide[0][:, :cols], accumulate=kind == "add")
         assert ops().gemm_group_takes(a, w, wide[1][:, :cols])
-        products.append((a, w, wide[1][:, :cols], kind == "pairs"))
+        products.append((a, w, wide[1][:, :cols], kind if kind in ("pairs", "add") else "store"))
         want.append(wide)
     ops().gemm_group(products)
     for wide in want:
@@ -614,6 +614,8 @@ def test_gemm_group_has_the_bits_of_the_single_products(m, shapes):
     assert not ops().gemm_group_takes(a, w.plain, out) and not ops().gemm_group_takes(a.float(), w, out)
     with pytest.raises(ops().KernelError):
         ops().gemm_group(products * 3)
+    with pytest.raises(ops().KernelError):
+        ops().gemm_group([(a, w, out, "other")])
 
 
 @pytest.mark.parametrize("two", [False, True])
