@@ -35,6 +35,8 @@ MODULE_FLAGS: dict[str, list[str]] = {"attn_mfma": ["-fno-honor-nans"]}
 # Libraries a module is linked against (after its sources on the command line).
 ROCM_LIB = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib")
 MODULE_LINK: dict[str, list[str]] = {"gemm_library": [f"-L{ROCM_LIB}", f"-Wl,-rpath,{ROCM_LIB}", "-lhipblaslt"]}
+# Modules of host code alone: CPython modules over torch's C++ types (``load_host``), compiled by the host's compiler.
+HOST_MODULES = ("hostcheck",)
 HEADERS = ["common.h", "gemm_common.h", "sampling_static.h", "memory_chunks.h"]
 MODULES: dict[str, list[str]] = {
     "elementwise": ["elementwise.hip"],
@@ -53,6 +55,7 @@ MODULES: dict[str, list[str]] = {
     "ssm": ["ssm.hip"],
     "convkv": ["convkv.hip"],
     "chdelta": ["chdelta.hip"],
+    "hostcheck": ["hostcheck.cpp"],
 }
 
 
@@ -61,6 +64,7 @@ class KernelBuildError(RuntimeError):
 
 
 _loaded: dict[str, ctypes.CDLL] = {}
+_loaded_host: dict[str, object] = {}
 _lock = threading.Lock()
 
 
@@ -87,10 +91,23 @@ def _build_dir() -> str:
     raise KernelBuildError(f"no writable folder for kernel libraries among {candidates}")
 
 
+def _host_command() -> list[str]:
+    """The compiler and what all host modules are compiled with (the versions they are compiled for among it)."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    libs = os.path.join(root, "lib")
+    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f"-DKVF_TORCH={torch.__version__}", f"-I{os.path.join(root, 'include')}",
+            f"-I{os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include')}", f"-I{sysconfig.get_paths()['include']}",
+            f"-L{libs}", f"-Wl,-rpath,{libs}"]
+
+
 def _source_hash(name: str) -> str:
     h = hashlib.sha256()
-    h.update(" ".join(FLAGS + MODULE_FLAGS.get(name, [])).encode())
-    for f in MODULES[name] + HEADERS:
+    h.update(" ".join(_host_command() if name in HOST_MODULES else FLAGS + MODULE_FLAGS.get(name, [])).encode())
+    for f in MODULES[name] + ([] if name in HOST_MODULES else HEADERS):
         with open(os.path.join(CSRC, f), "rb") as fh:
             h.update(fh.read())
     return h.hexdigest()
@@ -129,18 +146,22 @@ def build_module(name: str, force: bool = False, verbose: bool = True) -> str:
         found = _find_built(name, want)
         if found:
             return found
+    host = name in HOST_MODULES
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    if not os.path.isfile(hipcc):
+    if not host and not os.path.isfile(hipcc):
         raise KernelBuildError(
             f"kernel module {name!r} is not built and hipcc was not found; "
             "run `python -c 'import __graft_entry__ as g; g.build()'` where ROCm is installed")
     out_dir = _build_dir()
     so, stamp = os.path.join(out_dir, f"{name}.so"), os.path.join(out_dir, f"{name}.stamp")
     tmp = os.path.join(out_dir, f".{name}.{os.getpid()}.{threading.get_ident()}.so")
-    cmd = [hipcc, *FLAGS, *MODULE_FLAGS.get(name, []), f"-I{CSRC}", *[os.path.join(CSRC, s) for s in MODULES[name]], *MODULE_LINK.get(name, []), "-o", tmp]
+    if host:
+        cmd = [*_host_command(), *[os.path.join(CSRC, s) for s in MODULES[name]], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-o", tmp]
+    else:
+        cmd = [hipcc, *FLAGS, *MODULE_FLAGS.get(name, []), f"-I{CSRC}", *[os.path.join(CSRC, s) for s in MODULES[name]], *MODULE_LINK.get(name, []), "-o", tmp]
     t0 = time.time()
     if verbose:
-        _log(f"compiling kernel module {name} for {ARCH} ...")
+        _log(f"compiling {'host' if host else 'kernel'} module {name} for {'Python' if host else ARCH} ...")
     env = dict(os.environ)
     env.setdefault("HOME", tempfile.gettempdir())
     proc = subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
@@ -162,7 +183,7 @@ def build_module(name: str, force: bool = False, verbose: bool = True) -> str:
         except OSError:
             pass
         lines = [ln for ln in output.splitlines() if "packed-fp32-ops" not in ln]
-        raise KernelBuildError(f"hipcc failed for module {name!r}:\n" + "\n".join(lines[-60:]))
+        raise KernelBuildError(f"{os.path.basename(cmd[0])} failed for module {name!r}:\n" + "\n".join(lines[-60:]))
     os.replace(tmp, so)
     with open(stamp + ".tmp", "w") as f:
         f.write(want)
@@ -197,6 +218,24 @@ def load(name: str) -> ctypes.CDLL:
                 raise KernelBuildError(f"cannot load kernel module {name!r} from {path}: {e}") from e
             _loaded[name] = lib
     return lib
+
+
+def load_host(name: str):
+    """The loaded host module, built first when it has to be."""
+    with _lock:
+        module = _loaded_host.get(name)
+        if module is None:
+            import importlib.machinery
+            import importlib.util
+            path = build_module(name)
+            try:
+                loader = importlib.machinery.ExtensionFileLoader(name, path)
+                module = importlib.util.module_from_spec(importlib.util.spec_from_loader(name, loader))
+                loader.exec_module(module)
+            except ImportError as e:
+                raise KernelBuildError(f"cannot load host module {name!r} from {path}: {e}") from e
+            _loaded_host[name] = module
+    return module
 
 
 def ensure(names: list[str]) -> None:

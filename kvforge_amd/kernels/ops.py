@@ -68,6 +68,19 @@ def _check(t: torch.Tensor, name: str, dtype=None, shape=None, contiguous=True) 
         raise KernelError(f"{name} must be contiguous")
 
 
+_check_in_python = _check
+_operands = None     # hostcheck's, once it is loaded
+
+
+def _check_natively() -> None:
+    """From the first launch on operands are checked by native code; what it does not pass goes to ``_check_in_python``,
+    which says why."""
+    global _check, _operands
+    native = library.load_host("hostcheck")
+    native.set_slow(_check_in_python)
+    _check, _operands = native.check, native.operands
+
+
 def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether the memory spanned by two tensors' storage views intersects."""
     def span(t):
@@ -107,6 +120,8 @@ def _fn(module: str, name: str, argtypes: list):
         f.argtypes = argtypes
         f.restype = c_int
         _fn_cache[key] = f
+        if _operands is None and torch.cuda.is_available():
+            _check_natively()
     return f
 
 
@@ -831,7 +846,20 @@ def _w_args(w) -> tuple[int, int]:
     return w.data_ptr(), 0
 
 
+def _whole(n: int) -> int:
+    return n
+
+
+def _halves(n: int) -> int:
+    return n // 2
+
+
 def _gemm_operands(a, w, out, n_out):
+    """(m, n, k, lda, ldc) of ``out = a @ w.T``, of ``n_out(n)`` columns (``_whole`` or ``_halves``)."""
+    if _operands is not None:
+        found = _operands(a, plain_of(w), out, n_out is _halves)
+        if found is not None:
+            return found
     if a.dim() != 2 or w.dim() != 2 or out.dim() != 2:
         raise KernelError("gemm takes 2-D tensors")
     m, k = a.shape
@@ -997,7 +1025,7 @@ def gemm(a: torch.Tensor, w, out: torch.Tensor, accumulate: bool = False,
     ``out`` and is added on the way; ``half_out`` (bf16, likewise, only where ``k_halves_pay``)
     receives the product over the second half of K *instead of* ``out``, which the caller then
     owes to ``out``: twice the workgroups pull on ``w``."""
-    m, n, k, lda, ldc = _gemm_operands(a, w, out, lambda n: n)
+    m, n, k, lda, ldc = _gemm_operands(a, w, out, _whole)
     if accumulate and out.dtype != F32:
         raise KernelError("gemm: accumulation needs an fp32 output")
     for t, name in ((owed, "owed"), (half_out, "half_out")):
@@ -1057,7 +1085,7 @@ def gemm_gated(a: torch.Tensor, w, out: torch.Tensor, activation: str = "silu",
     ``out: [M, N/2]`` bf16.  ``activation``, ``limit``: as in ``gated_act``; biases fp32 ``[N/2]`` or
     ``None``; ``rms_eps`` as in ``gemm_fused``.  Callers check ``bf16_kernel_takes`` first."""
     rms = rms_eps is not None
-    m, n, k, lda, ldc = _gemm_operands(a, w, out, lambda n: n // 2)
+    m, n, k, lda, ldc = _gemm_operands(a, w, out, _halves)
     if not bf16_kernel_takes(a, w, rms, True):
         raise KernelError("gemm_gated: operands do not fit the MFMA kernel")
     if n % 4 or out.dtype != BF16:
@@ -1099,7 +1127,7 @@ def gemm_group(products) -> None:
         raise KernelError(f"gemm_group: 1 to {GROUP_MAX} products, got {len(products)}")
     rows, items = products[0][0].shape[0], []
     for a, w, out, how in products:
-        m, n, k, lda, ldc = _gemm_operands(a, w, out, (lambda n: n // 2) if how == "pairs" else (lambda n: n))
+        m, n, k, lda, ldc = _gemm_operands(a, w, out, _halves if how == "pairs" else _whole)
         epi = {"store": 0 if out.dtype == F32 else 1, "add": 2, "pairs": 3}.get(how)
         if (m != rows or epi is None or not gemm_group_takes(a, w, out) or (epi == 3 and (n % 4 or out.dtype != BF16))
                 or (epi == 2 and out.dtype != F32)):
@@ -1118,7 +1146,7 @@ def gemm_fused(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rms_eps: flo
     ``silu_pairs``: columns are (gate, up) pairs and ``out[:, j] = silu(c[2j]) * c[2j+1]``,
     ``out: [M, N/2]`` bf16.  Callers check ``bf16_kernel_takes`` first."""
     rms = rms_eps is not None
-    m, n, k, lda, ldc = _gemm_operands(a, w, out, (lambda n: n // 2) if silu_pairs else (lambda n: n))
+    m, n, k, lda, ldc = _gemm_operands(a, w, out, _halves if silu_pairs else _whole)
     if not bf16_kernel_takes(a, w, rms, silu_pairs):
         raise KernelError("gemm_fused: operands do not fit the MFMA kernel")
     if silu_pairs:
