@@ -684,11 +684,23 @@ __global__ void rope_kvwrite_kernel(T* __restrict__ qkv, const int* __restrict__
 }
 
 // The same work for a tile of 16 tokens per workgroup with 8 elements per lane and access
-// (d and the rotary width multiples of 8).  V is stored transposed, so a token's elements lie
-// block_size apart; where the tile's 16 tokens fill consecutive places of one page (a prompt
-// read from a page boundary) the tile is turned in LDS and each (head, element) row of 16
-// tokens is stored in one piece.  Other tiles store V element by element.
+// (d and the rotary width multiples of 8), also with the norm per head that is described at
+// qknorm_rope_kvwrite_kernel in front (NORM: P lanes, a power of two, share a head of at most 128).
+// V is stored transposed, so a token's elements lie block_size apart; where the tile's 16 tokens
+// fill consecutive places of one page (a prompt read from a page boundary) each (head, element)
+// row of 16 tokens is stored in one piece.  Other tiles store V element by element.
+//
+// The bytes are few (25 MB for 2,042 tokens of 48 heads of 64: 4 us), so what bounds a workgroup
+// is the chain position -> table row -> page in front of its stores.  All that does not hang on
+// it is under way before: the first ROPE_AHEAD vectors of every lane, the V columns (into LDS, from
+// where both ways of storing them read) and, once the positions are there, the tile's angles (into
+// LDS, since every head of a token asks for the same ones).  Behind the products of a pass: 2,042 tokens with a norm
+// 28.2 us (a workgroup a token, two bytes an access) -> 16.1, without one 18.8 (the loads behind the look-up) -> 16.4,
+// five tokens without one 7.9 -> 6.5.
 constexpr int ROPE_TILE = 16;
+constexpr int ROPE_AHEAD = 4;
+constexpr int ROPE_ANGLES = 64;   // angles of a token that are staged in LDS (a rotary width of 128)
+constexpr int ROPE_NORM_MAX = 128;  // elements of a head with a norm: two weight vectors are a workgroup's 256 threads
 
 __device__ __forceinline__ void store8(float* p, const float (&v)[8]) {
   *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
@@ -702,112 +714,217 @@ __device__ __forceinline__ void store8(bf16_t* p, const float (&v)[8]) {
   *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-template <typename T>
+struct HeadNorm {
+  const float *qw, *kw;   // [dk]
+  int dk, P;
+  float eps, qt_coef;
+  int qt_every;
+};
+
+template <typename T, bool NORM>
 __global__ __launch_bounds__(256) void rope_kvwrite_tile_kernel(
     T* __restrict__ qkv, const int* __restrict__ positions, const int* __restrict__ seq_of_token,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     const int* __restrict__ block_table, T* __restrict__ k_pages, T* __restrict__ v_pages, int n,
-    int turn_v, RopeArgs a) {
+    int turn_v, HeadNorm h, RopeArgs a) {
   extern __shared__ __align__(16) unsigned char tile_raw[];  // [ROPE_TILE][V columns of this share] of T, if turn_v
+  __shared__ __align__(16) float s_cos[ROPE_TILE * ROPE_ANGLES], s_sin[ROPE_TILE * ROPE_ANGLES];
   __shared__ int s_pos[ROPE_TILE], s_page[ROPE_TILE], s_off[ROPE_TILE], s_run;
+  __shared__ float s_temp[ROPE_TILE];
+  __shared__ __align__(16) float s_w[NORM ? 2 * ROPE_NORM_MAX : 4];  // the norm's weights of q and of k, zeros past dk
+  constexpr int Q = sizeof(T) * 8 / 16;  // 16-byte pieces of eight elements
   const int n0 = blockIdx.x * ROPE_TILE;
   const int cnt = min(ROPE_TILE, n - n0);
   const int half = a.rot / 2;
-  if (threadIdx.x < ROPE_TILE) {
-    const int t = threadIdx.x;
-    int p = -1, page = -1, off = 0;
-    if (t < cnt) {
-      p = positions[n0 + t];
-      if (p < 0 || p >= a.table_len) p = -1;
-      if (p >= 0 && a.write_kv) {
-        const int seq = seq_of_token[n0 + t];
-        const int blk = p / a.block_size;
-        if (seq >= 0 && seq < a.n_seqs && blk < a.table_stride) {
-          page = block_table[static_cast<size_t>(seq) * a.table_stride + blk];
-          if (page >= a.num_blocks) page = -1;
-          off = p - blk * a.block_size;
-        }
-      }
-    }
-    s_pos[t] = p;
-    s_page[t] = page;
-    s_off[t] = off;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    bool run = turn_v && cnt == ROPE_TILE && s_page[0] >= 0 && s_off[0] % 8 == 0 &&
-               a.block_size % 8 == 0 && s_off[0] + ROPE_TILE <= a.block_size;
-    for (int t = 1; t < ROPE_TILE; ++t) run = run && s_page[t] == s_page[0] && s_off[t] == s_off[0] + t;
-    s_run = run;
-  }
-  __syncthreads();
-  // blockIdx.y names a share of the row: of its q and k vectors, and of its V columns
   const int row_len = a.row_len;
-  const int qk_vecs = (a.H + a.KV) * a.d / 8;
-  const int qk_share = (qk_vecs + gridDim.y - 1) / gridDim.y;
+  // blockIdx.y names a share of the row: of its q and k vectors (whole heads with a norm, P lanes each), and of its
+  // V columns
+  const int heads = a.H + (a.write_kv ? a.KV : 0);
+  const int head_vecs = NORM ? h.P : a.d / 8;
+  const int qk_vecs = heads * head_vecs;
+  const int qk_share = NORM ? (heads + gridDim.y - 1) / gridDim.y * h.P : (qk_vecs + gridDim.y - 1) / gridDim.y;
   const int qk_begin = blockIdx.y * qk_share;
   const int qk_mine = max(0, min(qk_share, qk_vecs - qk_begin));
-  for (int item = threadIdx.x; item < cnt * qk_mine; item += blockDim.x) {
-    const int t = item / qk_mine, e = (qk_begin + item - t * qk_mine) * 8;
-    const int head = e / a.d, i0 = e - head * a.d;
-    const bool is_k = head >= a.H;
-    const int p = s_pos[t], page = s_page[t];
-    // a query that is not rotated stays as it is; a key without a page is not stored
-    if (is_k ? page < 0 : (p < 0 || i0 >= a.rot)) continue;
-    T* src = qkv + static_cast<size_t>(n0 + t) * row_len + e;
-    float x[8];
-    load8(src, x);
-    if (p >= 0 && i0 < a.rot) {
-      const float4 c = *reinterpret_cast<const float4*>(cos_t + static_cast<size_t>(p) * half + i0 / 2);
-      const float4 sn = *reinterpret_cast<const float4*>(sin_t + static_cast<size_t>(p) * half + i0 / 2);
-      const float cs[4] = {c.x, c.y, c.z, c.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+  const int items = cnt * qk_mine;
+  // the item's token, head and first element; items past the end are the first one again, lanes past d read element 0
+  auto place = [&](int item, int& t, int& head, int& i0) {
+    t = item / max(qk_mine, 1);
+    const int v = qk_begin + item - t * qk_mine;
+    head = v / head_vecs;
+    i0 = (v - head * head_vecs) * 8;
+  };
+  uint4 raw[ROPE_AHEAD][Q];
+  auto fetch = [&](int first) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float x1 = x[2 * i], x2 = x[2 * i + 1];
-        x[2 * i] = x1 * cs[i] - x2 * ss[i];
-        x[2 * i + 1] = x2 * cs[i] + x1 * ss[i];
-      }
+    for (int u = 0; u < ROPE_AHEAD; ++u) {
+      const int item = first + u * 256;
+      int t, head, i0;
+      place(item < items ? item : 0, t, head, i0);
+      const T* src = qkv + static_cast<size_t>(n0 + t) * row_len + head * a.d + (i0 < a.d ? i0 : 0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) raw[u][q] = reinterpret_cast<const uint4*>(src)[q];
     }
-    T* dst = is_k ? k_pages + ((static_cast<size_t>(page) * a.KV + (head - a.H)) * a.block_size + s_off[t]) * a.d + i0
-                  : src;
-    store8(dst, x);
+  };
+  // the first wave looks up the pages, a token a lane; the angles are the last waves' to begin with, the V columns the
+  // first waves', so that no wave waits for one of the three behind another
+  // (no load up to the first vectors is predicated: a wait for one of them would be a wait for all)
+  const int mine = min(static_cast<int>(threadIdx.x), cnt - 1), w_at = threadIdx.x % ROPE_NORM_MAX;
+  const int pos = positions[n0 + mine], seq = seq_of_token[n0 + mine];
+  int page = -1, off = 0;
+  float norm_w = 0.f;
+  if constexpr (NORM) norm_w = (threadIdx.x < ROPE_NORM_MAX || !a.write_kv ? h.qw : h.kw)[min(w_at, h.dk - 1)];
+  const int angle_vecs = half <= ROPE_ANGLES && cos_t ? half / 4 : 0;
+  if (items > 0) fetch(threadIdx.x);
+  const int p = static_cast<int>(threadIdx.x) < cnt && pos >= 0 && pos < a.table_len ? pos : -1;
+  if (p >= 0 && a.write_kv) {
+    const int blk = p / a.block_size;
+    if (seq >= 0 && seq < a.n_seqs && blk < a.table_stride) {
+      page = block_table[static_cast<size_t>(seq) * a.table_stride + blk];
+      off = p - blk * a.block_size;
+    }
   }
-  if (!a.write_kv) return;
   const int v0 = (a.H + a.KV) * a.d, v_len = a.KV * a.d;
   const int v_share = (v_len / 8 + gridDim.y - 1) / gridDim.y * 8;  // columns, whole vectors
   const int v_begin = blockIdx.y * v_share;
-  const int v_mine = max(0, min(v_share, v_len - v_begin));
-  if (s_run) {
-    T* tile = reinterpret_cast<T*>(tile_raw);  // [ROPE_TILE][v_share]
+  const int v_mine = a.write_kv ? max(0, min(v_share, v_len - v_begin)) : 0;
+  T* tile = reinterpret_cast<T*>(tile_raw);  // [ROPE_TILE][v_share]
+  if (turn_v) {
     const int v_vecs = v_mine / 8;
-    for (int item = threadIdx.x; item < ROPE_TILE * v_vecs; item += blockDim.x) {
+    for (int item = threadIdx.x; item < cnt * v_vecs; item += 256) {
       const int t = item / v_vecs, e = (item - t * v_vecs) * 8;
       const T* src = qkv + static_cast<size_t>(n0 + t) * row_len + v0 + v_begin + e;
-      constexpr int Q = sizeof(T) * 8 / 16;  // 16-byte pieces of eight elements
 #pragma unroll
       for (int q = 0; q < Q; ++q)
         reinterpret_cast<uint4*>(tile + t * v_share + e)[q] = reinterpret_cast<const uint4*>(src)[q];
     }
-    __syncthreads();
-    const int page = s_page[0], off0 = s_off[0];
-    for (int c = threadIdx.x; c < v_mine; c += blockDim.x) {  // v_begin + c = head * d + element
+  }
+  for (int item = 255 - threadIdx.x; item < cnt * angle_vecs; item += 256) {
+    const int t = item / angle_vecs, i = (item - t * angle_vecs) * 4;
+    int at = positions[n0 + t];
+    if (at < 0 || at >= a.table_len) at = 0;   // (not used)
+    *reinterpret_cast<float4*>(s_cos + t * ROPE_ANGLES + i) =
+        *reinterpret_cast<const float4*>(cos_t + static_cast<size_t>(at) * half + i);
+    *reinterpret_cast<float4*>(s_sin + t * ROPE_ANGLES + i) =
+        *reinterpret_cast<const float4*>(sin_t + static_cast<size_t>(at) * half + i);
+  }
+  if constexpr (NORM) s_w[threadIdx.x] = w_at < h.dk ? norm_w : 0.f;
+  if (threadIdx.x < KVF_WAVE) {
+    const int t = threadIdx.x;
+    if (page >= a.num_blocks) page = -1;
+    if (t < ROPE_TILE) {
+      // query temperature: q heads are stretched by 1 + coef * ln(floor((p + 1) / every) + 1)
+      if (NORM)
+        s_temp[t] = h.qt_every > 0 && pos >= 0
+                        ? 1.f + h.qt_coef * logf(static_cast<float>((pos + 1) / h.qt_every) + 1.f)
+                        : 1.f;
+      s_pos[t] = p;
+      s_page[t] = page;
+      s_off[t] = off;
+    }
+    const int page0 = __shfl(page, 0, KVF_WAVE), off0 = __shfl(off, 0, KVF_WAVE);
+    const bool follows = t >= ROPE_TILE || (page == page0 && off == off0 + t);
+    const bool run = turn_v && cnt == ROPE_TILE && page0 >= 0 && off0 % 8 == 0 && a.block_size % 8 == 0 &&
+                     off0 + ROPE_TILE <= a.block_size && __all(follows);
+    if (t == 0) s_run = run;
+  }
+  __syncthreads();
+  for (int first = threadIdx.x; first - static_cast<int>(threadIdx.x) < items; first += ROPE_AHEAD * 256) {
+    if (first != static_cast<int>(threadIdx.x)) fetch(first);
+#pragma unroll
+    for (int u = 0; u < ROPE_AHEAD; ++u) {
+      const int item = first + u * 256;
+      if (item >= items) break;   // (P lanes of a head at once: items are whole heads)
+      int t, head, i0;
+      place(item, t, head, i0);
+      const bool is_k = head >= a.H;
+      const int at = s_pos[t], to = s_page[t];
+      float x[8];
+      load8(reinterpret_cast<const T*>(&raw[u][0]), x);
+      bool keep;   // a key without a page is not stored
+      if constexpr (NORM) {
+        // the squares are added up in the order of a wave that holds a pair a lane
+        float s[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (i0 + 2 * i >= h.dk) x[2 * i] = 0.f;
+          if (i0 + 2 * i + 1 >= h.dk) x[2 * i + 1] = 0.f;
+          s[i] = fmaf(x[2 * i], x[2 * i], fmaf(x[2 * i + 1], x[2 * i + 1], 0.f));
+        }
+        for (int o = h.P / 2; o > 0; o >>= 1) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[i] += __shfl_xor(s[i], o, KVF_WAVE);
+        }
+        const float sum = (s[0] + s[2]) + (s[1] + s[3]);
+        const float r = (is_k ? 1.f : s_temp[t]) / sqrtf(sum / static_cast<float>(h.dk) + h.eps);
+        float w[8];
+        load8(s_w + (is_k ? ROPE_NORM_MAX : 0) + (i0 < a.d ? i0 : 0), w);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = i0 + i < h.dk ? x[i] * r * w[i] : 0.f;
+        keep = i0 < a.d && (!is_k || to >= 0);
+      } else {
+        keep = is_k ? to >= 0 : at >= 0 && i0 < a.rot;   // a query that is not rotated stays as it is
+      }
+      if (!keep) continue;
+      if (at >= 0 && i0 < a.rot) {
+        float4 c, sn;
+        if (angle_vecs > 0) {
+          c = *reinterpret_cast<const float4*>(s_cos + t * ROPE_ANGLES + i0 / 2);
+          sn = *reinterpret_cast<const float4*>(s_sin + t * ROPE_ANGLES + i0 / 2);
+        } else {
+          c = *reinterpret_cast<const float4*>(cos_t + static_cast<size_t>(at) * half + i0 / 2);
+          sn = *reinterpret_cast<const float4*>(sin_t + static_cast<size_t>(at) * half + i0 / 2);
+        }
+        const float cs[4] = {c.x, c.y, c.z, c.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float x1 = x[2 * i], x2 = x[2 * i + 1];
+          x[2 * i] = fmaf(x1, cs[i], -(x2 * ss[i]));
+          // (which product is rounded first is what the kernels without tiles have)
+          x[2 * i + 1] = NORM ? fmaf(x2, cs[i], x1 * ss[i]) : fmaf(x1, ss[i], x2 * cs[i]);
+        }
+      }
+      T* dst = is_k ? k_pages + ((static_cast<size_t>(to) * a.KV + (head - a.H)) * a.block_size + s_off[t]) * a.d + i0
+                    : qkv + static_cast<size_t>(n0 + t) * row_len + head * a.d + i0;
+      store8(dst, x);
+    }
+  }
+  if (s_run) {
+    const int to = s_page[0], off0 = s_off[0];
+    for (int c = threadIdx.x; c < v_mine; c += 256) {  // v_begin + c = head * d + element
       __align__(16) T vals[ROPE_TILE];
 #pragma unroll
       for (int t = 0; t < ROPE_TILE; ++t) vals[t] = tile[t * v_share + c];
-      T* dst = v_pages + (static_cast<size_t>(page) * v_len + v_begin + c) * a.block_size + off0;
-      constexpr int Q = sizeof(T) * ROPE_TILE / 16;
+      T* dst = v_pages + (static_cast<size_t>(to) * v_len + v_begin + c) * a.block_size + off0;
+      constexpr int R = sizeof(T) * ROPE_TILE / 16;
 #pragma unroll
-      for (int q = 0; q < Q; ++q) reinterpret_cast<uint4*>(dst)[q] = reinterpret_cast<const uint4*>(vals)[q];
+      for (int q = 0; q < R; ++q) reinterpret_cast<uint4*>(dst)[q] = reinterpret_cast<const uint4*>(vals)[q];
     }
   } else {
-    for (int item = threadIdx.x; item < cnt * v_mine; item += blockDim.x) {
-      const int t = item / v_mine, c = v_begin + item - t * v_mine;
-      const int page = s_page[t];
-      if (page < 0) continue;
-      v_pages[(static_cast<size_t>(page) * v_len + c) * a.block_size + s_off[t]] =
-          qkv[static_cast<size_t>(n0 + t) * row_len + v0 + c];
+    for (int item = threadIdx.x; item < cnt * v_mine; item += 256) {
+      const int t = item / v_mine, c = item - t * v_mine;
+      const int to = s_page[t];
+      if (to < 0) continue;
+      v_pages[(static_cast<size_t>(to) * v_len + v_begin + c) * a.block_size + s_off[t]] =
+          turn_v ? tile[t * v_share + c] : qkv[static_cast<size_t>(n0 + t) * row_len + v0 + v_begin + c];
     }
   }
+}
+
+template <typename T, bool NORM>
+static int rope_tile_launch(T* qkv, const int* positions, const int* seq_of_token, const float* cos_t,
+                            const float* sin_t, const int* block_table, T* k_pages, T* v_pages, int n,
+                            const HeadNorm& h, const RopeArgs& a, hipStream_t s) {
+  // few tiles: several workgroups share a tile's row, so that the chip has work
+  const int tiles = (n + ROPE_TILE - 1) / ROPE_TILE;
+  int shares = tiles >= 512 ? 1 : (512 + tiles - 1) / tiles;
+  if (shares > 8) shares = 8;
+  const int v_share = (a.KV * a.d / 8 + shares - 1) / shares * 8;
+  // the tile of V rows turned in LDS; without room for it V goes element by element
+  const size_t lds = static_cast<size_t>(ROPE_TILE) * v_share * sizeof(T);
+  const int turn_v = lds <= 48 * 1024;
+  hipLaunchKernelGGL((rope_kvwrite_tile_kernel<T, NORM>), dim3(tiles, shares), dim3(256), turn_v ? lds : 0, s, qkv,
+                     positions, seq_of_token, cos_t, sin_t, block_table, k_pages, v_pages, n, turn_v, h, a);
+  return kvf_last_error();
 }
 
 template <typename T>
@@ -816,18 +933,8 @@ static int rope_launch(void* qkv, const int* positions, const int* seq_of_token,
                        int n, RopeArgs a, hipStream_t s) {
   if (n <= 0) return 0;
   if (a.d % 8 == 0 && a.rot % 8 == 0 && a.row_len % 8 == 0) {
-    // few tiles: several workgroups share a tile's row, so that the chip has work
-    const int tiles = (n + ROPE_TILE - 1) / ROPE_TILE;
-    int shares = tiles >= 512 ? 1 : (512 + tiles - 1) / tiles;
-    if (shares > 8) shares = 8;
-    const int v_share = (a.KV * a.d / 8 + shares - 1) / shares * 8;
-    // the tile of V rows turned in LDS; without room for it V goes element by element
-    const size_t lds = static_cast<size_t>(ROPE_TILE) * v_share * sizeof(T);
-    const int turn_v = lds <= 48 * 1024;
-    hipLaunchKernelGGL(rope_kvwrite_tile_kernel<T>, dim3(tiles, shares), dim3(256), turn_v ? lds : 0, s,
-                       static_cast<T*>(qkv), positions, seq_of_token, cos_t, sin_t, block_table,
-                       static_cast<T*>(k_pages), static_cast<T*>(v_pages), n, turn_v, a);
-    return kvf_last_error();
+    return rope_tile_launch<T, false>(static_cast<T*>(qkv), positions, seq_of_token, cos_t, sin_t, block_table,
+                                      static_cast<T*>(k_pages), static_cast<T*>(v_pages), n, HeadNorm{}, a, s);
   }
   hipLaunchKernelGGL(rope_kvwrite_kernel<T>, dim3(n), dim3(128), 0, s, static_cast<T*>(qkv),
                      positions, seq_of_token, cos_t, sin_t, block_table, static_cast<T*>(k_pages),
@@ -934,6 +1041,19 @@ static int qknorm_rope_launch(void* qkv, const int* positions, const int* seq_of
   if (n <= 0) return 0;
   if (a.d > 4 * KVF_WAVE || dk > a.d || dk <= 0 || a.rot > dk || a.rot % 2 || !qw || (a.write_kv && !kw))
     return static_cast<int>(hipErrorInvalidValue);
+  const bool vectors = a.d % 8 == 0 && a.rot % 8 == 0 && a.row_len % 8 == 0 &&
+                       reinterpret_cast<uintptr_t>(qkv) % 16 == 0 &&
+                       (!a.write_kv || (reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) % 16 == 0) &&
+                       (reinterpret_cast<uintptr_t>(cos_t) | reinterpret_cast<uintptr_t>(sin_t)) % 16 == 0;
+  // Tiles from 256 tokens on (32 + 2 * 8 heads of 64, bf16, this kernel and in tiles: 17 tokens 3.4 and 5.9 us, 64 tokens
+  // 3.7 and 6.0, 300 tokens 7.2 and 6.3, 2,042 tokens 25.4 and 11.3): for few tokens a wave a head is the shorter chain.
+  if (vectors && a.d <= ROPE_NORM_MAX && n >= 256) {
+    int P = 1;
+    while (8 * P < a.d) P *= 2;
+    return rope_tile_launch<T, true>(static_cast<T*>(qkv), positions, seq_of_token, cos_t, sin_t, block_table,
+                                     static_cast<T*>(k_pages), static_cast<T*>(v_pages), n,
+                                     HeadNorm{qw, kw, dk, P, eps, qt_coef, qt_every}, a, s);
+  }
   // a wave a head where the tokens alone do not fill the chip; four heads a wave for many tokens
   const int heads = a.H + (a.write_kv ? a.KV : 0);
   int shares = n >= 1024 ? 1 : (heads + 3) / 4;

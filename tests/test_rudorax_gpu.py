@@ -139,6 +139,65 @@ def test_head_norm_rotation_and_cache_write_in_one_kernel(dtype, H, KV, dk, d, r
         torch.testing.assert_close(vp[page, :, :, off].float().cpu(), x[t, H + KV:], **tol(dtype))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,KV,dk,d,rot,bs", [(4, 2, 64, 64, 64, 16), (3, 1, 8, 8, 8, 24), (5, 3, 37, 40, 24, 12), (1, 1, 128, 128, 128, 32),
+                                              (9, 4, 90, 96, 0, 16)])
+@pytest.mark.parametrize("n", [255, 256, 271])
+def test_head_norm_and_cache_write_in_tiles_have_the_bits_of_single_tokens(dtype, H, KV, dk, d, rot, bs, n):
+    """Many tokens whose rows are whole vectors go in tiles; rows a few elements further apart do not.  Runs from and off
+    page boundaries, padding, positions off the tables, pages that were given back, no cache write."""
+    table_len, width = 200, -(-260 // bs)
+    pos = torch.arange(n, dtype=torch.int32)
+    pos[100:140] = torch.arange(40, dtype=torch.int32) + 3
+    pos[:9] = torch.tensor([-1, 5, 199, 200, 259, 7, 0, 100000, 64])
+    seq = torch.zeros(n, dtype=torch.int32)
+    seq[100:140], seq[150:160], seq[20], seq[[2, 3, 4, 8]] = 1, -1, 2, 1   # (no two tokens at one place)
+    table = torch.randperm(2 * width, generator=torch.Generator().manual_seed(n)).view(2, width).to(torch.int32)
+    table[0, 2], table[1, 0] = -1, 2 * width
+    angle = rand(table_len, max(rot // 2, 1), seed=7, scale=3.0)
+    tabs = (angle.cos().to(DEV), angle.sin().to(DEV)) if rot else (None, None)
+    rows = rand(n, (H + 2 * KV) * d, seed=dk, scale=2.0).view(n, H + 2 * KV, d).clone()
+    rows[:, :H + KV, dk:] = 0.0
+    rows = rows.view(n, -1).to(dtype)
+    qw, kw = (1.0 + rand(dk, seed=sd, scale=0.2).to(DEV) for sd in (1, 2))
+    where = (pos.to(DEV), seq.to(DEV), *tabs, table.to(DEV))
+    for write_kv, q_temp in ((True, None), (True, (0.3, 8)), (False, None)):
+        got = []
+        for more in (0, 3):
+            qkv = torch.nn.functional.pad(rows, (0, more), value=5.0).to(DEV)
+            kp = torch.full((2 * width, KV, bs, d), 9.0, dtype=dtype, device=DEV)
+            vp = torch.full((2 * width, KV, d, bs), 9.0, dtype=dtype, device=DEV)
+            ops().qknorm_rope_kvwrite(qkv, *where, kp, vp, H, KV, d, qw, kw, dk, 1e-4, write_kv=write_kv, q_temp=q_temp)
+            got.append((qkv[:, :rows.shape[1]].contiguous(), kp, vp))
+        assert not torch.equal(got[0][0].cpu(), rows)
+        for a, b in zip(*got):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [5, 16, 33])
+def test_rotation_wider_than_the_staged_angles_has_the_same_bits(dtype, n):
+    """Of 80 angles a token the first 64 rotate as they do where only they are given; the others as the formula says."""
+    H, KV, d, bs = 3, 1, 176, 16
+    rows, pos = rand(n, (H + 2 * KV) * d, seed=n).to(dtype), torch.arange(n, dtype=torch.int32)
+    angle, table = rand(64, 80, seed=7, scale=3.0), torch.arange(4, dtype=torch.int32).view(1, 4)
+    got = []
+    for half in (80, 64):
+        dev, kp = rows.clone().to(DEV), torch.zeros(4, KV, bs, d, dtype=dtype, device=DEV)
+        vp = torch.zeros(4, KV, d, bs, dtype=dtype, device=DEV)
+        ops().rope_kvwrite(dev, pos.to(DEV), torch.zeros(n, dtype=torch.int32, device=DEV),
+                           angle[:, :half].cos().contiguous().to(DEV), angle[:, :half].sin().contiguous().to(DEV),
+                           table.to(DEV), kp, vp, H, KV, d)
+        got.append((dev.cpu().view(n, -1, d), kp.cpu(), vp.cpu()))
+    (q, k, v), (q64, k64, v64) = got
+    assert torch.equal(q[..., :128], q64[..., :128]) and torch.equal(k[..., :128], k64[..., :128]) and torch.equal(v, v64)
+    x = rows.float().view(n, -1, d)[:, :H, 128:160]
+    c, s = (f(angle[:n, 64:])[:, None] for f in (torch.cos, torch.sin))
+    want = torch.stack([x[..., 0::2] * c - x[..., 1::2] * s, x[..., 1::2] * c + x[..., 0::2] * s], -1).flatten(-2)
+    torch.testing.assert_close(q[:, :H, 128:160].float(), want, **tol(dtype))
+    assert torch.equal(q[:, :H, 160:], rows.view(n, -1, d)[:, :H, 160:])
+
+
 def sink_reference(paged, q, seq_lens, q_lens, scale, window, sink):
     outs, off = [], 0
     for s, (n, ql) in enumerate(zip(seq_lens, q_lens)):
