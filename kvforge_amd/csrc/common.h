@@ -66,6 +66,17 @@ template <int G> __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// 16 bytes that are read once a launch (STREAMED: marked so, that they push nothing out of the caches and wait for
+// no room there) or that others read too.
+template <bool STREAMED> __device__ __forceinline__ uint4 load_16(const void* p) {
+  if constexpr (STREAMED) {
+    typedef uint32_t words __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(uint4, __builtin_nontemporal_load(static_cast<const words*>(p)));
+  } else {
+    return *static_cast<const uint4*>(p);
+  }
+}
+template <bool B> struct Flag { static constexpr bool value = B; };
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = KVF_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, KVF_WAVE);

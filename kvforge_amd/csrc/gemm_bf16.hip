@@ -208,6 +208,21 @@ __device__ __forceinline__ bf16x8 load_frag(const bf16_t* p, bool ok) {
   return __builtin_bit_cast(bf16x8, r);
 }
 
+template <bool STREAMED> __device__ __forceinline__ bf16x8 load_weight(const bf16_t* p, bool ok) {
+  uint4 r = make_uint4(0u, 0u, 0u, 0u);
+  if (ok) r = load_16<STREAMED>(p);
+  return __builtin_bit_cast(bf16x8, r);
+}
+
+// Whether a matrix in tiles goes past the caches: one launch of few rows reads each of its bytes once, in whole lines, so
+// nothing is lost where it cannot lie there from the last step, and what can (activations, keys and values) stays.
+// Eight rows (us, cached and streamed): output head of 525 MB 89.5 and 76.6, gated pair of 67 MB 15.3 and 14.6, q/k/v
+// of 12.6 MB 8.4 and 7.8 and the attention behind them 8.8 and 7.7; 41 rows over 12.6 MB 11.3 and 10.3.  The line is at what
+// an XCD's L2 holds: the matrices of a decoder 512 wide (0.5 to 2.9 MB), which do lie in the caches, took 0.2 to 0.6 us longer
+// streamed, one of 8 MB the same.  (gemm_mid_kernel, whose workgroups share lines: 15.7 and 16.9, so it does not.)
+constexpr long STREAM_BYTES = 4l << 20;
+__host__ __device__ inline bool streams(int N, int K) { return 2l * N * K >= STREAM_BYTES; }
+
 // 8 fp32 (with ADD plus 8 of `q`) -> 8 bf16 (round to nearest even); adds their squares to ss.
 // Nothing inside the branches uses what they load, so no branch ends in a wait and the loads of
 // a whole pass stay in flight together.
@@ -401,7 +416,8 @@ constexpr int depth(int mt, int nt, int at) {
   return at ? (mt == 1 ? 4 : mt <= 4 ? 2 : 1) : (mt * nt == 1 ? 8 : mt * nt <= 4 ? 4 : 2);
 }
 
-template <int MT, int NT, int AT, int EPI, bool ADD>
+// ST: W is streamed past the caches (see streams); a kernel of its own, so that either has the other's arithmetic.
+template <int MT, int NT, int AT, int EPI, bool ADD, bool ST>
 __global__ __launch_bounds__(max_waves(MT, NT, AT) * KVF_WAVE) void gemm_skinny_kernel(
     const void* __restrict__ Av, const bf16_t* __restrict__ W, void* __restrict__ Cv, int M, int N,
     int K, int lda, int ldc, int m_base, float eps, int w_tiled, Riders rd, RopeEpi rp, PickEpi pk) {
@@ -478,7 +494,7 @@ __global__ __launch_bounds__(max_waves(MT, NT, AT) * KVF_WAVE) void gemm_skinny_
       const int k = (ks + u * nw) * 32;
       const bool ok = k + kg * 8 + 8 <= K;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) wf[u][j] = load_frag(wp[j] + (ks + u * nw) * w_step, ok || w_tiled);
+      for (int j = 0; j < NT; ++j) wf[u][j] = load_weight<ST>(wp[j] + (ks + u * nw) * w_step, ok || w_tiled);
 #pragma unroll
       for (int t = 0; t < MT; ++t)
         af[u][t] = AT ? load_frag_f32<ADD>(Af + aoff[t] + k, a_add + aoff[t] + k, ok && a_live[t], ss[t])
@@ -515,7 +531,7 @@ __global__ __launch_bounds__(max_waves(MT, NT, AT) * KVF_WAVE) void gemm_skinny_
                  : load_frag(Ab + aoff[t] + k, ok && a_live[t]);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      const bf16x8 wf = load_frag(wp[j] + ks * w_step, ok || w_tiled);
+      const bf16x8 wf = load_weight<ST>(wp[j] + ks * w_step, ok || w_tiled);
 #pragma unroll
       for (int t = 0; t < MT; ++t)
         acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af[t], acc[j][t], 0, 0, 0);
@@ -775,23 +791,28 @@ __global__ __launch_bounds__(GROUP_WAVES * KVF_WAVE) void gemm_group_kernel(Grou
   if (it.epi == 2 && wave == 0 && live && n0 + 4 * kg < it.N)
     epi_prefetch_a<2>(pre, r16, n0 + 4 * kg, it.N, it.ldc, it.C, nullptr, rp);
   constexpr int U = depth(1, 1, 0), nw = GROUP_WAVES;
-  int ks = wave;
-  for (; ks + (U - 1) * nw < ksteps; ks += U * nw) {
-    bf16x8 wf[U], af[U];
+  auto walk = [&](auto streamed) {
+    constexpr bool S = decltype(streamed)::value;
+    int ks = wave;
+    for (; ks + (U - 1) * nw < ksteps; ks += U * nw) {
+      bf16x8 wf[U], af[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = (ks + u * nw) * 32;
-      wf[u] = load_frag(wp + static_cast<size_t>(ks + u * nw) * (KVF_WAVE * 8), true);
-      af[u] = load_frag(ap + k, live && k + kg * 8 + 8 <= it.K);
+      for (int u = 0; u < U; ++u) {
+        const int k = (ks + u * nw) * 32;
+        wf[u] = load_weight<S>(wp + static_cast<size_t>(ks + u * nw) * (KVF_WAVE * 8), true);
+        af[u] = load_frag(ap + k, live && k + kg * 8 + 8 <= it.K);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], af[u], acc, 0, 0, 0);
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], af[u], acc, 0, 0, 0);
-  }
-  for (; ks < ksteps; ks += nw) {
-    const bf16x8 wf = load_frag(wp + static_cast<size_t>(ks) * (KVF_WAVE * 8), true);
-    const bf16x8 af = load_frag(ap + ks * 32, live && ks * 32 + kg * 8 + 8 <= it.K);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
-  }
+    for (; ks < ksteps; ks += nw) {
+      const bf16x8 wf = load_weight<S>(wp + static_cast<size_t>(ks) * (KVF_WAVE * 8), true);
+      const bf16x8 af = load_frag(ap + ks * 32, live && ks * 32 + kg * 8 + 8 <= it.K);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
+    }
+  };
+  if (streams(it.N, it.K)) walk(Flag<true>{});
+  else walk(Flag<false>{});
   *reinterpret_cast<f32x4*>(red + (wave * KVF_WAVE + lane) * 4) = acc;
   __syncthreads();
   const int n = n0 + 4 * kg;
@@ -821,6 +842,19 @@ int pick_waves(int K) {
   return nw;
 }
 
+template <int MT, int NT, int AT, int EPI, bool ADD>
+int launch_as(dim3 grid, dim3 block, size_t lds, const void* A, const bf16_t* W, void* C, int M, int N, int K, int lda,
+              int ldc, int m_base, float eps, int w_tiled, const Riders& rd, const RopeEpi& rp, const PickEpi& pk,
+              hipStream_t s) {
+  if (w_tiled && streams(N, K))
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NT, AT, EPI, ADD, true>), grid, block, lds, s, A, W, C, M, N, K, lda,
+                       ldc, m_base, eps, w_tiled, rd, rp, pk);
+  else
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NT, AT, EPI, ADD, false>), grid, block, lds, s, A, W, C, M, N, K, lda,
+                       ldc, m_base, eps, w_tiled, rd, rp, pk);
+  return kvf_last_error();
+}
+
 template <int MT, int NT, int AT, int EPI>
 int launch_one(const void* A, const bf16_t* W, void* C, int M, int N, int K, int lda, int ldc,
                int m_base, float eps, int w_tiled, const Riders& rd, const RopeEpi& rp, hipStream_t s,
@@ -835,15 +869,12 @@ int launch_one(const void* A, const bf16_t* W, void* C, int M, int N, int K, int
     // the sum that rides in the left operand's loads: only the fused q/k/v projection of one
     // tile of rows is built with it
     if constexpr (MT == 1 && AT == 1 && EPI == 4)
-      hipLaunchKernelGGL((gemm_skinny_kernel<MT, NT, AT, EPI, true>), grid, block, lds, s, A, W, C, M, N, K,
-                         lda, ldc, m_base, eps, w_tiled, rd, rp, pk);
-    else
-      return static_cast<int>(hipErrorInvalidValue);
-  } else {
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NT, AT, EPI, false>), grid, block, lds, s, A, W, C, M, N, K,
-                       lda, ldc, m_base, eps, w_tiled, rd, rp, pk);
+      return launch_as<MT, NT, AT, EPI, true>(grid, block, lds, A, W, C, M, N, K, lda, ldc, m_base, eps, w_tiled, rd, rp,
+                                              pk, s);
+    return static_cast<int>(hipErrorInvalidValue);
   }
-  return kvf_last_error();
+  return launch_as<MT, NT, AT, EPI, false>(grid, block, lds, A, W, C, M, N, K, lda, ldc, m_base, eps, w_tiled, rd, rp,
+                                           pk, s);
 }
 
 // How 17 to 64 rows are cut: groups of columns a workgroup and cuts of K.  The rule takes the least

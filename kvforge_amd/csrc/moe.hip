@@ -181,6 +181,9 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int PLAN_EXPERT_BITS = 9, PLAN_MAX_EXPERTS = 1 << PLAN_EXPERT_BITS, PLAN_ROWS_BITS = 8;
 constexpr int PLAN_BATCH = 8;      // choices a thread of the plan has in flight
 constexpr int PREFETCH_SETS = 3;   // sets of operand registers in flight in the kernels of few rows
+constexpr int DEEP_SETS = 8;       // the same where there can be no more workgroups than
+constexpr int DEEP_BLOCKS = 384;
+constexpr long EXPERTS_STREAM_BYTES = 32l << 20;   // the eight L2s
 
 __device__ __forceinline__ int tile_expert(const int* tiles, int t) { return tiles[3 * t] & (PLAN_MAX_EXPERTS - 1); }
 __device__ __forceinline__ int tile_in_expert(const int* tiles, int t) { return tiles[3 * t] >> PLAN_EXPERT_BITS; }
@@ -314,9 +317,16 @@ __global__ __launch_bounds__(CHOOSE_TOKENS * KVF_WAVE) void moe_choose_plan_kern
 // rows: a lane ends with four neighbouring output columns of one row.
 //
 // The kernels of few rows (a decode step): a wave takes 16 rows of one expert and 16 weight rows, so that
-// the experts' matrices, which bound it, come in through as many workgroups as there are.  A step's two
-// fragments are asked for two steps ahead of the matrix instruction that uses them: PREFETCH_SETS sets
-// of registers take turns.
+// the experts' matrices, which bound it, come in through as many workgroups as there are.  Two ways:
+// narrow_product, where there can be more workgroups than DEEP_BLOCKS: a step's two fragments are asked for two steps
+// ahead of the matrix instruction that uses them (PREFETCH_SETS sets of registers take turns), and lanes without a
+// row ask for none.  deep_product, where there are no more: a wave's own chain of trips is then what takes the time, so eight
+// steps are on their way, and no load is predicated (lanes without a row read the last one).
+// STREAMED (see load_16): up to 16 tokens, of whose experts each is read by one tile alone, over layers whose experts take
+// more than the L2s.  Four kernels and no branch in one: that was 3 to 10 us slower than either way by itself.
+// Plan, up and down (us; tokens, experts, 4 chosen, ff, K; matrices from memory): before, streamed, streamed and deep:
+//   1, 32, 1,024, 2,048: 32.8, 31.1, 18.4      8: 51.3, 46.4, 49.7      13: 70.3, 63.3, 62.2
+//   5, 32, 2,048, 2,048: 74.8, 67.8, 65.3      16, 16, 512, 1,024: 22.2, 20.4, 16.0      3: 18.9, 19.4, 14.2
 template <class Load>
 __device__ __forceinline__ f32x4 narrow_product(int S, const Load& load) {
   constexpr int NB = PREFETCH_SETS;
@@ -336,12 +346,40 @@ __device__ __forceinline__ f32x4 narrow_product(int S, const Load& load) {
   }
   return acc;
 }
+template <class Load>
+__device__ __forceinline__ f32x4 deep_product(int S, const Load& load) {
+  constexpr int NB = DEEP_SETS;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  bf16x8 x[NB], w[NB];
+  if (S < NB) return narrow_product(S, load);
+#pragma unroll
+  for (int i = 0; i < NB; ++i) load(i, x[i], w[i]);
+  int s = 0;
+  for (; s + 2 * NB <= S; s += NB) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], x[i], acc, 0, 0, 0);
+      load(s + NB + i, x[i], w[i]);
+    }
+  }
+  const int left = S - s - NB;   // steps not asked for yet, fewer than NB
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], x[i], acc, 0, 0, 0);
+    if (i < left) load(s + NB + i, x[i], w[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i)
+    if (i < left) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], x[i], acc, 0, 0, 0);
+  return acc;
+}
 
 // moe_up: act[place, :] = silu(gate) * up for the tile's rows with their expert's matrices; the
 // weight holds every expert's gate and up rows interleaved (gate_j, up_j neighbours), so a lane's
 // four columns are two whole pairs.  Grid (column blocks, tiles).  in_wgt (or null): the choice's weight
 // belongs to the expert's input; gate and up are linear in it, so it is multiplied into both sums ahead
 // of the activation.
+template <bool DEEP, bool STREAMED>
 __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* __restrict__ x, int ldx, int K,
                                                      const uint4* __restrict__ wt, int S,
                                                      const int* __restrict__ order,
@@ -356,15 +394,27 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* __restrict__ 
   const int j = lane % 16, c = lane / 16;
   const int groups = ff / 8, g = blockIdx.x * 4 + wave;   // groups of 16 interleaved rows per expert
   if (g >= groups) return;
-  const bf16_t* xr = j < rows ? x + static_cast<size_t>(order[row0 + j] / top) * ldx + 8 * c : nullptr;
   const uint4* wbase = wt + (static_cast<size_t>(e) * groups + g) * S * KVF_WAVE + lane;
   const int s_full = K / 32;   // steps whose 32 elements all lie inside a row
-  const f32x4 acc = narrow_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
-    uint4 xf = make_uint4(0u, 0u, 0u, 0u);
-    if (xr && (s < s_full || 32 * s + 8 * c + 8 <= K)) xf = *reinterpret_cast<const uint4*>(xr + 32 * s);
-    xs = __builtin_bit_cast(bf16x8, xf);
-    ws = __builtin_bit_cast(bf16x8, wbase[static_cast<size_t>(s) * KVF_WAVE]);
-  });
+  f32x4 acc;
+  if constexpr (DEEP) {
+    const bf16_t* own = x + static_cast<size_t>(order[row0 + min(j, rows - 1)] / top) * ldx;
+    acc = deep_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
+      const bool in = s < s_full || 32 * s + 8 * c + 8 <= K;
+      uint4 xf = *reinterpret_cast<const uint4*>(own + (in ? 32 * s + 8 * c : 0));
+      if (!in) xf = make_uint4(0u, 0u, 0u, 0u);
+      xs = __builtin_bit_cast(bf16x8, xf);
+      ws = __builtin_bit_cast(bf16x8, load_16<STREAMED>(wbase + static_cast<size_t>(s) * KVF_WAVE));
+    });
+  } else {
+    const bf16_t* xr = j < rows ? x + static_cast<size_t>(order[row0 + j] / top) * ldx + 8 * c : nullptr;
+    acc = narrow_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
+      uint4 xf = make_uint4(0u, 0u, 0u, 0u);
+      if (xr && (s < s_full || 32 * s + 8 * c + 8 <= K)) xf = *reinterpret_cast<const uint4*>(xr + 32 * s);
+      xs = __builtin_bit_cast(bf16x8, xf);
+      ws = __builtin_bit_cast(bf16x8, load_16<STREAMED>(wbase + static_cast<size_t>(s) * KVF_WAVE));
+    });
+  }
   if (j >= rows) return;
   const float w = in_wgt ? in_wgt[order[row0 + j]] : 1.f;
   const float y0 = joined(f, w * acc[0], w * acc[1]), y1 = joined(f, w * acc[2], w * acc[3]);
@@ -374,6 +424,7 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* __restrict__ 
 
 // moe_down: y[place, :] = act[place, :] W_down[expert]^T (bf16, not yet weighted).  The weight
 // holds the experts' down matrices side by side along K: expert e owns the steps e ff/32 ...
+template <bool DEEP, bool STREAMED>
 __global__ __launch_bounds__(256) void moe_down_kernel(const bf16_t* __restrict__ act, int ff,
                                                        const uint4* __restrict__ wt, int S_all,
                                                        const int* __restrict__ tiles,
@@ -386,15 +437,24 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const bf16_t* __restrict_
   const int j = lane % 16, c = lane / 16;
   const int groups = (hidden + 15) / 16, g = blockIdx.x * 4 + wave;
   if (g >= groups) return;
-  const bf16_t* ar = j < rows ? act + static_cast<size_t>(row0 + j) * ff + 8 * c : nullptr;
   const int S = ff / 32;
   const uint4* wbase = wt + (static_cast<size_t>(g) * S_all + static_cast<size_t>(e) * S) * KVF_WAVE + lane;
-  const f32x4 acc = narrow_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
-    uint4 af = make_uint4(0u, 0u, 0u, 0u);
-    if (ar) af = *reinterpret_cast<const uint4*>(ar + 32 * s);
-    xs = __builtin_bit_cast(bf16x8, af);
-    ws = __builtin_bit_cast(bf16x8, wbase[static_cast<size_t>(s) * KVF_WAVE]);
-  });
+  f32x4 acc;
+  if constexpr (DEEP) {
+    const bf16_t* own = act + static_cast<size_t>(row0 + min(j, rows - 1)) * ff + 8 * c;
+    acc = deep_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
+      xs = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(own + 32 * s));
+      ws = __builtin_bit_cast(bf16x8, load_16<STREAMED>(wbase + static_cast<size_t>(s) * KVF_WAVE));
+    });
+  } else {
+    const bf16_t* ar = j < rows ? act + static_cast<size_t>(row0 + j) * ff + 8 * c : nullptr;
+    acc = narrow_product(S, [&](int s, bf16x8& xs, bf16x8& ws) {
+      uint4 af = make_uint4(0u, 0u, 0u, 0u);
+      if (ar) af = *reinterpret_cast<const uint4*>(ar + 32 * s);
+      xs = __builtin_bit_cast(bf16x8, af);
+      ws = __builtin_bit_cast(bf16x8, load_16<STREAMED>(wbase + static_cast<size_t>(s) * KVF_WAVE));
+    });
+  }
   const int col = g * 16 + 4 * c;
   if (j >= rows || col >= hidden) return;   // hidden is a multiple of 8
   *reinterpret_cast<uint2*>(y + static_cast<size_t>(row0 + j) * hidden + col) = pack4(acc);
@@ -833,10 +893,22 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, int n, int K, int E, int 
     hipLaunchKernelGGL(moe_down_wide_kernel, dim3((down_blocks * most + 7) / 8 * 8), dim3(256), 0, s, a, ff, down,
                        E * (ff / 32), tiles, num_tiles, out, K);
   } else {
-    hipLaunchKernelGGL(moe_up_kernel, dim3(up_blocks, max_tiles), dim3(256), 0, s, xb, ldx, K, up, S, order, tiles,
-                       num_tiles, top, ff, in_wgt, f, a);
-    hipLaunchKernelGGL(moe_down_kernel, dim3(down_blocks, max_tiles), dim3(256), 0, s, a, ff, down, E * (ff / 32), tiles,
-                       num_tiles, out, K);
+    const bool streamed = n <= 16 && 6l * E * ff * K >= EXPERTS_STREAM_BYTES;
+    const int most = pairs < pairs / 16 + E ? pairs : pairs / 16 + E;    // tiles there can be
+    const auto both = [&](auto deep, auto st) {
+      hipLaunchKernelGGL((moe_up_kernel<decltype(deep)::value, decltype(st)::value>), dim3(up_blocks, max_tiles), dim3(256), 0, s,
+                         xb, ldx, K, up, S, order, tiles, num_tiles, top, ff, in_wgt, f, a);
+      hipLaunchKernelGGL((moe_down_kernel<decltype(deep)::value, decltype(st)::value>), dim3(down_blocks, max_tiles), dim3(256),
+                         0, s, a, ff, down, E * (ff / 32), tiles, num_tiles, out, K);
+    };
+    const auto deep_or_not = [&](auto st) {
+      if (most * static_cast<int>(up_blocks > down_blocks ? up_blocks : down_blocks) <= DEEP_BLOCKS)
+        both(Flag<true>{}, st);
+      else
+        both(Flag<false>{}, st);
+    };
+    if (streamed) deep_or_not(Flag<true>{});
+    else deep_or_not(Flag<false>{});
   }
   return kvf_last_error();
 }

@@ -390,6 +390,24 @@ def test_gemm_pick_takes_the_lowest_of_equal_columns():
     assert tokens.tolist() == want
 
 
+@pytest.mark.parametrize("m", [1, 8, 16])
+@pytest.mark.parametrize("n,k", [(2048, 1024), (2044, 1024), (1036, 2056), (8192, 2048)])
+def test_streamed_weights_give_the_bits_of_cached_ones(m, n, k):
+    """Matrices in tiles of 4 MB and more go past the caches, smaller and row-major ones do not."""
+    g = torch.Generator().manual_seed(m + n)
+    a, x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV), torch.randn(m, k, generator=g).to(DEV)
+    w = (torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV)
+    res, outs = torch.randn(m, n, generator=g).to(DEV), []
+    for form in (w, ops().StreamedWeight(w)):
+        c, half, pairs = res.clone(), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+        ops().gemm(a, form, c, accumulate=True)
+        ops().gemm(a, form, half)
+        ops().gemm_fused(x, form, pairs, rms_eps=1e-5, silu_pairs=True)
+        outs.append((c, half, pairs))
+    for one, other in zip(*outs):
+        assert torch.equal(one.view(torch.uint8), other.view(torch.uint8))
+
+
 @pytest.mark.parametrize("m", [1, 5, 16])
 @pytest.mark.parametrize("n,k", [(352, 96), (40, 2048), (100, 40), (2048, 136), (16, 32)])
 def test_gemm_over_tiled_weights_gives_the_same_bits(m, n, k):
@@ -1678,6 +1696,31 @@ def test_grouped_experts_over_rows_of_many_passes(K, ff, weigh_input):
     """Tiles of every height over rows of five to seven passes of 64 elements, where the loads of the last ones stand
     ahead of the row's end, whole and part passes, odd steps; one expert of several tiles."""
     test_grouped_experts_at_the_edges_of_their_tiles([20, 40, 290, 70, 128], K, ff, weigh_input)
+
+
+@pytest.mark.parametrize("E,ff,K", [(32, 512, 1024), (6, 512, 1024), (24, 96, 2312), (48, 224, 1032)])
+def test_a_token_s_experts_give_the_same_bits_in_every_batch(E, ff, K):
+    """One token (few workgroups), 16 (each expert's rows in one tile) and 17 (no longer so) over layers whose experts
+    are more and less than the caches hold take different kernels: a token's row is the same in all of them."""
+    g = torch.Generator().manual_seed(E)
+    top, o = 3, ops()
+    x = torch.randn(17, K, generator=g).to(torch.bfloat16).to(DEV)
+    up = o.streamed((torch.randn(E * 2 * ff, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV))
+    down = o.streamed((torch.randn(K, E * ff, generator=g) * ff ** -0.5).to(torch.bfloat16).to(DEV))
+    chosen = torch.stack([torch.randperm(E + 1, generator=g)[:top] for _ in range(17)]).to(torch.int32).to(DEV)
+    w, res = torch.rand(17, top, generator=g).to(DEV), torch.randn(17, K, generator=g).to(DEV)
+
+    def run(first, n):
+        tiles, got = o.moe_grouped_tiles(n, top, E), res[first:first + n].clone()
+        scratch = {k: torch.empty(m, dtype=torch.int32, device=DEV) for k, m in (("where", n * top), ("order", n * top),
+                                                                                 ("tiles", 3 * tiles), ("num_tiles", 1))}
+        scratch |= {k: torch.full((n * top, m), math.nan, dtype=torch.bfloat16, device=DEV) for k, m in (("act", ff), ("y", K))}
+        o.moe_grouped(x[first:first + n], up, down, chosen[first:first + n], w[first:first + n], got, E, ff, scratch,
+                      many_rows=False)
+        return got.view(torch.int32)
+
+    alone = torch.cat([run(i, 1) for i in range(17)])
+    assert torch.equal(run(0, 17), alone) and torch.equal(run(1, 16), alone[1:]) and torch.equal(run(0, 5), alone[:5])
 
 
 @pytest.mark.parametrize("d", [16, 48, 64, 128, 208])
