@@ -325,7 +325,7 @@ __global__ __launch_bounds__(CHOOSE_TOKENS * KVF_WAVE) void moe_choose_plan_kern
 // STREAMED (see load_16): up to 16 tokens, of whose experts each is read by one tile alone, over layers whose experts take
 // more than the L2s.  Four kernels and no branch in one: that was 3 to 10 us slower than either way by itself.
 // Plan, up and down (us; tokens, experts, 4 chosen, ff, K; matrices from memory): before, streamed, streamed and deep:
-//   1, 32, 1,024, 2,048: 32.8, 31.1, 18.4      8: 51.3, 46.4, 49.7      13: 70.3, 63.3, 62.2
+//   1, 32, 1,024, 2,048: 32.8, 31.1, 18.3      8: 51.3, 46.4, 49.7      13: 70.3, 63.3, 62.2
 //   5, 32, 2,048, 2,048: 74.8, 67.8, 65.3      16, 16, 512, 1,024: 22.2, 20.4, 16.0      3: 18.9, 19.4, 14.2
 template <class Load>
 __device__ __forceinline__ f32x4 narrow_product(int S, const Load& load) {
