@@ -208,8 +208,8 @@ class Mixer(Part):
 
     settles_residual = False
 
-    # Names the workspace buffers that this make of mixer keeps its rows in, which no other make touches: the last products of two
-    # mixers of different makes may then be made together, behind both.  ``None``: not known.
+    # Names the workspace buffers that this make of mixer keeps its rows in, which no other make touches: the first products of two
+    # mixers of different makes may then be made together, ahead of both, and the last ones behind both.  ``None``: not known.
     buffers: str | None = None
 
     cache_spec: CacheSpec | None = None

@@ -97,8 +97,15 @@ class MixerPair(Mixer):
         halves = (layer.state[:, :n], layer.state[:, self.right_off:self.right_off + _floats(self.right.state_spec)])
         return tuple(LayerState(layer.group, layer.pages, layer.owns_cache, s) for s in halves)
 
+    @property
+    def _apart(self) -> bool:
+        """Whether neither of the two writes into a buffer in which the other keeps its rows."""
+        return None not in (self.left.buffers, self.right.buffers) and self.left.buffers != self.right.buffers
+
     def input_products(self, x, step) -> list:
-        return products_of(self.left, x, step) + products_of(self.right, x, step)
+        """Those of both; the first one's alone where its ``forward`` may use the second one's buffers."""
+        first = products_of(self.left, x, step)
+        return first + products_of(self.right, x, step) if self._apart else first
 
     def forward(self, x, step, layer: LayerState, residual) -> None:
         """``x``: normalised activations.  Without norms, what the first leaves owed to the stream the
@@ -114,7 +121,7 @@ class MixerPair(Mixer):
         step.settle()
         rows = []
         # the first one's last product waits for the second one's, which takes it along, where the second leaves its rows alone
-        waits = few and None not in (self.left.buffers, self.right.buffers) and self.left.buffers != self.right.buffers
+        waits = few and self._apart
         riders, step.riders = step.riders, []
         for m, state, name in ((self.left, ll, "pair_left_out"), (self.right, rl, "pair_right_out")):
             out = step.ws.buf(name, tuple(residual.shape), torch.float32)
@@ -128,6 +135,6 @@ class MixerPair(Mixer):
             rows.append(out)
         for _, a, w, out, _how in step.riders:      # (not taken along)
             ops.gemm(a, w, out)
-        step.made -= {key for key in step.made if key[0] == "rider"}
+        step.made = {key: out for key, out in step.made.items() if key[0] != "rider"}
         step.riders = riders
         ops.rms_add_two(residual, rows[0], self.weights[0], rows[1], self.weights[1], self.norms[0].eps)

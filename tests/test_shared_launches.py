@@ -1,0 +1,195 @@
+"""Products that parts have made together, ahead of them or behind: mixers side by side give what they give one by one, also where
+both keep their rows in the same workspace buffers."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import kvforge_amd
+from kvforge_amd.config.model import ModelConfig
+from kvforge_amd.engine.batch import Step, StepEntry, Workspace
+from kvforge_amd.engine.runner import ModelRunner
+from kvforge_amd.kernels import ops
+from kvforge_amd.models.transformer import Transformer
+from kvforge_amd.parts import (ChannelDelta, GatedDelta, LMHead, Mamba2, Mixer, MixerPair, ModelSpec, NamedRMSNorm, ParallelBlock,
+                               PlainFeedForward, RMSNorm, TokenEmbedding)
+from kvforge_amd.parts.base import LayerState, add_product
+
+
+# ------------------------------------------------------------------------------------- on the CPU, products by torch
+class Toy(Mixer):
+    """``residual += (x @ w.T)^2 @ w_o.T + sin(x @ w_g.T)`` over rows in buffers of the names ``name`` (``lists``: the first products
+    are announced)."""
+
+    def __init__(self, key: str, name: str, buffers: str | None, width: int, lists: bool = True) -> None:
+        g = torch.Generator().manual_seed(width + ord(key))
+        self.prefix, self.name, self.buffers, self.lists = key, name, buffers, lists
+        self.w, self.w_g, self.w_o = (torch.randn(*s, generator=g) for s in ((width, 24), (24, 24), (24, width)))
+
+    def plainly(self, x):
+        return (x @ self.w.T) ** 2 @ self.w_o.T + torch.sin(x @ self.w_g.T)
+
+    def _products(self, x, step):
+        return [((self.prefix, k), x, w, step.ws.buf(self.name + k, (x.shape[0], w.shape[0]), torch.float32), "store")
+                for k, w in (("rows", self.w), ("gates", self.w_g))]
+
+    def input_products(self, x, step):
+        return self._products(x, step) if self.lists else []
+
+    def forward(self, x, step, layer, residual):
+        step.settle()
+        products = self._products(x, step)
+        if self.lists:
+            step.make(products)
+        else:
+            for _, a, w, out, _how in products:
+                ops.gemm(a, w, out)
+        rows, gates = (p[3] for p in products)
+        residual += torch.sin(gates)
+        add_product(step, rows ** 2, self.w_o, residual)
+
+
+@pytest.fixture
+def by_torch(monkeypatch):
+    """Products as torch makes them, and how many went into each launch of several."""
+    sizes = []
+
+    def gemm(a, w, out, accumulate=False, **_):
+        out.copy_(out + a @ w.T if accumulate else a @ w.T)
+
+    def group(products):
+        sizes.append(len(products))
+        for a, w, out, how in reversed(products):     # (in any order: they run at the same time)
+            gemm(a, w, out, how == "add")
+    for name, f in (("gemm", gemm), ("gemm_group", group), ("gemm_group_takes", lambda a, w, out: a.shape[0] <= 16),
+                    ("is_library_product", lambda a, w: False), ("k_halves_pay", lambda a, w: False)):
+        monkeypatch.setattr(ops, name, f)
+    monkeypatch.setattr(ops, "parts_count", lambda a, w: 0)
+    return sizes
+
+
+def _step():
+    step = Step()
+    step.ws, step.act_dtype = Workspace("cpu"), torch.float32
+    return step
+
+
+@pytest.mark.parametrize("early", [False, True])     # whether a block has asked for the products before the pair does
+@pytest.mark.parametrize("left,right,launches", [
+    (("a", "", "toy", 40), ("b", "", "toy", 40), [2, 2]),             # one make: the same memory
+    (("a", "", "toy", 24), ("b", "", "toy", 56), [2, 2]),             # ... and the wider one makes it move
+    (("a", "", "toy", 56), ("b", "", "toy", 24), [2, 2]),
+    (("a", "", "toy", 40, False), ("b", "", "toy", 40), [2]),         # the first says nothing of its products
+    (("a", "", None, 40), ("b", "", None, 40), [2, 2]),               # makes that do not say what they use
+    (("a", "", "one", 40), ("b", "", "two", 40), [2, 2]),             # makes that say so wrongly
+    (("a", "", "one", 24), ("b", "", "two", 56), [3, 2]),
+    (("a", "left_", "one", 40), ("b", "right_", "two", 56), [4])])
+def test_mixers_side_by_side_as_one_by_one(by_torch, left, right, launches, early):
+    for rows in (1, 7, 16, 17):
+        by_torch.clear()
+        x = torch.randn(rows, 24, generator=torch.Generator().manual_seed(rows))
+        pair, got, step = MixerPair(Toy(*left), Toy(*right)), torch.zeros(rows, 24), _step()
+        want = pair.left.plainly(x) + pair.right.plainly(x)
+        if early and rows <= 16:
+            step.make_early(pair.input_products(x, step))
+        pair.forward(x, step, LayerState(), got)
+        step.settle()
+        torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-3)
+        assert not step.made and by_torch == (launches if rows <= 16 else [])
+
+
+def test_a_launch_of_several_products_refuses_memory_that_two_of_them_use():
+    a, wide = torch.zeros(3, 64), torch.zeros(3, 48)
+    w = torch.zeros(16, 64)
+    for products in ([(a, w, wide[:, :16], "store"), (a, w, wide[:, 8:24], "store")],
+                     [(a, w, wide.view(-1)[:48].view(3, 16), "store"), (a, w, wide.view(-1)[40:88].view(3, 16), "store")],
+                     [(a, w, wide[:, 16:32], "store"), (a, w, wide.view(-1)[:48].view(3, 16), "store")]):
+        with pytest.raises(ops.KernelError, match="write the same memory"):
+            ops.gemm_group(products)
+    with pytest.raises(ops.KernelError, match="reads what another writes"):
+        ops.gemm_group([(a, w, wide[:, :16], "store"), (wide[:, 16:32], w, a[:, :16], "store")])
+    ops._check_column_blocks([wide[:, :16], wide[:, 16:32], wide[:, 40:], a])
+
+
+# ------------------------------------------------------------------------------------- on the GPU, whole models
+class OneByOne(MixerPair):
+    """The two mixers one after the other, each with launches of its own."""
+
+    def input_products(self, x, step):
+        return []
+
+    def forward(self, x, step, layer, residual):
+        outs = []
+        for m, state, name in zip((self.left, self.right), self._layers(layer), ("one_left", "one_right")):
+            if self.norms is None:
+                m.forward(x, step, state, residual)
+                continue
+            step.settle()
+            step.fresh = step.ws.buf(name, tuple(residual.shape), torch.float32)
+            outs.append(step.fresh)
+            m.forward(x, step, state, step.fresh)
+        if self.norms is not None:
+            ops.rms_add_two(residual, outs[0], self.weights[0], outs[1], self.weights[1], self.norms[0].eps)
+
+
+class PairConfig(ModelConfig):
+    def __init__(self, d):
+        super().__init__(architecture="ToyPairForCausalLM", vocab_size=96, max_position_embeddings=256)
+        self.d = d
+
+    @classmethod
+    def from_dict(cls, d):
+        return cls(d)
+
+    def to_dict(self):
+        return self.d
+
+
+def _memory(kind, name, h):
+    cls, heads, dim = kind
+    more = dict(norm_parts=2) if cls is Mamba2 else dict(a_rank=16, g_rank=32) if cls is ChannelDelta else {}
+    return cls(name, h, heads, 2, dim, 32, 4, norm_eps=1e-5, **more)
+
+
+def _build(cfg):
+    d, h = cfg.d, 256
+    pair_cls = OneByOne if d["one_by_one"] else MixerPair
+    blocks = []
+    for i in range(2):
+        norms = tuple(NamedRMSNorm(f"l.{i}.out_{s}", h, 1e-5) for s in "lr") if d["normed"] else None
+        pair = pair_cls(*(_memory(k, f"l.{i}.{s}", h) for k, s in zip(d["kinds"], "lr")), norms=norms)
+        blocks.append(ParallelBlock(RMSNorm(f"l.{i}.n", h, 1e-5), pair, PlainFeedForward(f"l.{i}.ff", h, 256), h))
+    return ModelSpec(config=cfg, embedding=TokenEmbedding("embed", 96, h), blocks=blocks, final_norm=RMSNorm("norm", h, 1e-5),
+                     head=LMHead("head", 96, h), positions=[])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("normed", [False, True])
+@pytest.mark.parametrize("kinds", [((Mamba2, 8, 16), (GatedDelta, 8, 16)), ((GatedDelta, 4, 16), (Mamba2, 8, 32)),
+                                   ((ChannelDelta, 4, 32), (ChannelDelta, 4, 32))])
+def test_memories_of_one_make_side_by_side_as_one_by_one(kinds, normed):
+    """Prompts of 1, 8 and 16 tokens and steps of 1, 8 and 16 requests behind longer ones: the same bits as from two mixers with
+    launches of their own."""
+    kvforge_amd.register_architecture("ToyPairForCausalLM", PairConfig, _build)
+    logits = []
+    for one_by_one in (True, False):
+        cfg = PairConfig({"kinds": kinds, "normed": normed, "one_by_one": one_by_one})
+        model = Transformer.from_random(cfg, 3, torch.bfloat16, "cuda")
+        runner = ModelRunner(model, 16, 64, max_num_seqs=16, max_num_batched_tokens=256, max_model_len=64)
+        g, out = torch.Generator().manual_seed(1), []
+        ids = lambda n: torch.randint(0, 96, (n,), generator=g).tolist()  # noqa: E731
+        for n in (1, 8, 16):
+            runner.cache.allocate(f"p{n}", n)
+            out.append(runner.step([StepEntry(f"p{n}", ids(n), 0, "all")]).clone())
+            runner.cache.free(f"p{n}")
+        for r in range(16):
+            runner.cache.allocate(f"r{r}", 20)
+        out.append(runner.step([StepEntry(f"r{r}", ids(9 + r % 3), 0) for r in range(16)]).clone())
+        at = [9 + r % 3 for r in range(16)]
+        for rows in (16, 8, 1, 8):
+            out.append(runner.step([StepEntry(f"r{r}", ids(1), at[r]) for r in range(rows)]).clone())
+            at = [p + (r < rows) for r, p in enumerate(at)]
+        logits.append(torch.cat(out).cpu())
+    assert bool(logits[0].isfinite().all()) and float(logits[0].std()) > 0
+    assert torch.equal(*logits)
