@@ -411,7 +411,11 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(float* x, CombineArgs
     g1[k] = w1[min(i, h - 1)];
     if (TWO) g2[k] = w2[min(i, h - 1)];
   }
-  for (int i = 8 * tid; i < h; i += 8 * blockDim.x) {
+  // (every lane takes every turn, those past the row with its last elements: a choice is read from the lane that holds it, which
+  // has to be active there)
+  for (int i0 = 0; i0 < h; i0 += 8 * blockDim.x) {
+    const bool live = i0 + 8 * tid < h;
+    const int i = live ? i0 + 8 * tid : h - 8;
     float a[8], sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     load8(x + row + i, a);
     Raw8 pre = {}, post = {};
@@ -449,10 +453,12 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(float* x, CombineArgs
       for (int u = 0; u < 8; ++u) a[u] += t[u];
     }
     const float4 lo = make_float4(a[0], a[1], a[2], a[3]), hi = make_float4(a[4], a[5], a[6], a[7]);
-    store4(x + row + i, lo);
-    store4(x + row + i + 4, hi);
-    store4(combined + i, lo);
-    store4(combined + i + 4, hi);
+    if (live) {
+      store4(x + row + i, lo);
+      store4(x + row + i + 4, hi);
+      store4(combined + i, lo);
+      store4(combined + i + 4, hi);
+    }
   }
   __syncthreads();                                     // (and the rows that `in` may share with an output have been read)
   float ss = 0.f;

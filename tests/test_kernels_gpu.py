@@ -638,7 +638,8 @@ def test_gemm_group_has_the_bits_of_the_single_products(m, shapes):
 
 @pytest.mark.parametrize("two", [False, True])
 @pytest.mark.parametrize("n,h,top,E,pre,post", [(1, 8, 1, 2, None, None), (3, 248, 2, 3, "f32", "bf16"), (8, 1024, 4, 6, None, "f32"),
-                                                 (5, 2048, 4, 6, "bf16", "bf16"), (300, 2040, 3, 5, "bf16", None), (2, 4096, 16, 9, None, "f32")])
+                                                 (5, 2048, 4, 6, "bf16", "bf16"), (4, 1032, 4, 6, "bf16", "f32"),
+                                                 (2, 16, 4, 3, None, "bf16"), (300, 2040, 3, 5, "bf16", None), (2, 4096, 16, 9, None, "f32")])
 def test_experts_sum_and_the_next_norm_have_the_bits_of_their_steps(n, h, top, E, pre, post, two):
     """What is owed before the experts, their sum (choices that name an expert, the row itself, or nothing), what is owed
     behind, and one or two norms, against the kernels of the single steps: the stream and the outputs, with the
