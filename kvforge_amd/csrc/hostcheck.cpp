@@ -45,13 +45,13 @@ PyObject* check(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* kw
   for (Py_ssize_t i = 0; good && i < nargs; ++i) v[i] = args[i];
   for (Py_ssize_t k = 0; good && k < more; ++k) {
     good = false;
-    for (int i = 0; i < 5 && !good; ++i)
+    for (Py_ssize_t i = nargs; i < 5 && !good; ++i)      // (one given by place already is not one more)
       if (PyUnicode_CompareWithASCIIString(PyTuple_GET_ITEM(kwnames, k), names[i]) == 0) {
         v[i] = args[nargs + k];
         good = true;
       }
   }
-  if (good && v[0] && (v[4] == Py_True || v[4] == Py_False)) {
+  if (good && v[0] && v[1] && (v[4] == Py_True || v[4] == Py_False)) {
     try {
       if (passes(v[0], v[2], v[3], v[4] == Py_True)) Py_RETURN_NONE;
     } catch (...) {   // (nothing here is known to throw; the Python function says what is wrong)

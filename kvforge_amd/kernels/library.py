@@ -4,7 +4,8 @@ A module is compiled with ``hipcc --offload-arch=gfx950`` the first time somethi
 and the source has changed since the library on disk was built (a stamp file holds the hash of
 the sources and flags).  Libraries live in ``kvforge_amd/csrc/_build``; when that folder cannot
 be written (a read-only checkout) they go to a per-user folder under the temporary directory.
-There is no fallback path: a module that cannot be built or loaded raises ``KernelBuildError``.
+There is no fallback path: a module that cannot be built or loaded raises ``KernelBuildError``.  Modules of host code alone
+are the exception (``load_host``): they do faster what Python does too.
 """
 
 from __future__ import annotations
@@ -64,8 +65,8 @@ class KernelBuildError(RuntimeError):
 
 
 _loaded: dict[str, ctypes.CDLL] = {}
-_loaded_host: dict[str, object] = {}
-_lock = threading.Lock()
+_loaded_host: dict[str, object] = {}     # None: there is none
+_lock, _host_lock = threading.Lock(), threading.Lock()
 
 
 def available_modules() -> list[str]:
@@ -91,22 +92,31 @@ def _build_dir() -> str:
     raise KernelBuildError(f"no writable folder for kernel libraries among {candidates}")
 
 
+def _host_flags() -> list[str]:
+    """What decides whether a built host module fits this process: how it is compiled, and the torch and Python it is
+    compiled for.  (Not where the compiler and the headers lie: a built module does not need them.)"""
+    import sysconfig
+
+    import torch
+    return ["-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f"-DKVF_TORCH={torch.__version__}", f"-DKVF_PYTHON={sysconfig.get_config_var('SOABI')}"]
+
+
 def _host_command() -> list[str]:
-    """The compiler and what all host modules are compiled with (the versions they are compiled for among it)."""
+    """The compiler with its flags and where it finds torch and Python."""
     import sysconfig
 
     import torch
     root = os.path.dirname(torch.__file__)
     libs = os.path.join(root, "lib")
-    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-            f"-DKVF_TORCH={torch.__version__}", f"-I{os.path.join(root, 'include')}",
+    return [shutil.which("g++") or "g++", *_host_flags(), f"-I{os.path.join(root, 'include')}",
             f"-I{os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include')}", f"-I{sysconfig.get_paths()['include']}",
             f"-L{libs}", f"-Wl,-rpath,{libs}"]
 
 
 def _source_hash(name: str) -> str:
     h = hashlib.sha256()
-    h.update(" ".join(_host_command() if name in HOST_MODULES else FLAGS + MODULE_FLAGS.get(name, [])).encode())
+    h.update(" ".join(_host_flags() if name in HOST_MODULES else FLAGS + MODULE_FLAGS.get(name, [])).encode())
     for f in MODULES[name] + ([] if name in HOST_MODULES else HEADERS):
         with open(os.path.join(CSRC, f), "rb") as fh:
             h.update(fh.read())
@@ -164,8 +174,11 @@ def build_module(name: str, force: bool = False, verbose: bool = True) -> str:
         _log(f"compiling {'host' if host else 'kernel'} module {name} for {'Python' if host else ARCH} ...")
     env = dict(os.environ)
     env.setdefault("HOME", tempfile.gettempdir())
-    proc = subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
-                            env=env, cwd=out_dir)
+    try:
+        proc = subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                                env=env, cwd=out_dir)
+    except OSError as e:
+        raise KernelBuildError(f"module {name!r} is not built and {cmd[0]} cannot be run: {e}") from e
     done = threading.Event()
 
     def heartbeat() -> None:
@@ -221,27 +234,37 @@ def load(name: str) -> ctypes.CDLL:
 
 
 def load_host(name: str):
-    """The loaded host module, built first when it has to be."""
-    with _lock:
-        module = _loaded_host.get(name)
-        if module is None:
+    """The loaded host module, built first when it has to be; ``None``, said once, where there is none for this process
+    and none can be built: what it does has a form in Python."""
+    if name in _loaded_host:
+        return _loaded_host[name]
+    with _host_lock:
+        if name not in _loaded_host:
             import importlib.machinery
             import importlib.util
-            path = build_module(name)
+            module = None
             try:
-                loader = importlib.machinery.ExtensionFileLoader(name, path)
+                loader = importlib.machinery.ExtensionFileLoader(name, build_module(name))
                 module = importlib.util.module_from_spec(importlib.util.spec_from_loader(name, loader))
                 loader.exec_module(module)
-            except ImportError as e:
-                raise KernelBuildError(f"cannot load host module {name!r} from {path}: {e}") from e
+            except (KernelBuildError, ImportError) as e:
+                module = None
+                _log(f"host module {name} is done without, in Python: {e}")
             _loaded_host[name] = module
-    return module
+    return _loaded_host[name]
 
 
 def ensure(names: list[str]) -> None:
-    """Build (side by side) and load the named modules."""
+    """Build (side by side) and load the named modules, and the host modules beside them."""
     missing = [n for n in names if n not in _loaded]
-    if missing:
-        build_modules(missing)
-        for n in missing:
-            load(n)
+    hosts = [threading.Thread(target=load_host, args=(h,)) for h in HOST_MODULES if h not in _loaded_host]
+    for t in hosts:
+        t.start()
+    try:
+        if missing:
+            build_modules(missing)
+            for n in missing:
+                load(n)
+    finally:
+        for t in hosts:
+            t.join()

@@ -73,12 +73,13 @@ _operands = None     # hostcheck's, once it is loaded
 
 
 def _check_natively() -> None:
-    """From the first launch on operands are checked by native code; what it does not pass goes to ``_check_in_python``,
-    which says why."""
+    """From the first launch on operands are checked by native code, where there is any (``library.load_host``); what it does not
+    pass goes to ``_check_in_python``, which says why."""
     global _check, _operands
     native = library.load_host("hostcheck")
-    native.set_slow(_check_in_python)
-    _check, _operands = native.check, native.operands
+    if native is not None:
+        native.set_slow(_check_in_python)
+        _check, _operands = native.check, native.operands
 
 
 def span_of(t: torch.Tensor) -> tuple[int, int]:
@@ -119,6 +120,8 @@ def _fn(module: str, name: str, argtypes: list):
     key = (module, name)
     f = _fn_cache.get(key)
     if f is None:
+        if _operands is None and torch.cuda.is_available():
+            _check_natively()
         lib = library.load(module)
         try:
             f = getattr(lib, name)
@@ -127,8 +130,6 @@ def _fn(module: str, name: str, argtypes: list):
         f.argtypes = argtypes
         f.restype = c_int
         _fn_cache[key] = f
-        if _operands is None and torch.cuda.is_available():
-            _check_natively()
     return f
 
 
