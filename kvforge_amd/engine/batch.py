@@ -80,6 +80,7 @@ class Workspace:
         # views handed out before, by (name, dtype, shape): a step asks for the same ones again
         self._views: dict[tuple, torch.Tensor] = {}
         self.frozen = False
+        self.moves = 0          # how often a buffer has been let go for a larger one
 
     def buf(self, name: str, shape: tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
         view = self._views.get((name, dtype, shape))
@@ -93,6 +94,7 @@ class Workspace:
         if flat is None or flat.numel() < n:
             if self.frozen:
                 raise RuntimeError(f"workspace buffer {name} would grow during graph capture")
+            self.moves += flat is not None
             flat = torch.empty(max(n, 1), dtype=dtype, device=self.device)
             self._bufs[key] = flat
             for k in [k for k in self._views if k[0] == name and k[1] == dtype]:
@@ -115,6 +117,7 @@ class Workspace:
         if flat is None or flat.numel() < n:
             if self.frozen:
                 raise RuntimeError(f"workspace buffer {name} would grow during graph capture")
+            self.moves += flat is not None
             flat = torch.zeros(max(n, 1), dtype=dtype, device=self.device)
             self._bufs[key] = flat
             for k in [k for k in self._views if k[0] == name and k[1] == dtype]:

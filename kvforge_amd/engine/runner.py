@@ -62,8 +62,11 @@ class ModelRunner:
         # only if every part's launches may be replayed for another batch
         self.use_graphs = bool(use_graphs) and all(p.replayable for p in model.spec.all_parts())
         self.graphs: dict[tuple[int, tuple], _DecodeGraph] = {}
-        # steps of single tokens without sampling: (batch, launch keys) -> graph, None once seen, last used last
-        self.step_graphs: dict[tuple[int, tuple], _DecodeGraph | None] = {}
+        # steps of single tokens without sampling, by (batch, launch keys): graphs, last used last, and how often a kind that
+        # has none has come and has to come before it gets one
+        self.step_graphs: dict[tuple[int, tuple], _DecodeGraph] = {}
+        self.step_seen: dict[tuple[int, tuple], tuple[int, int]] = {}
+        self._step_moves = 0
         self.num_graph_replays = 0
         cap = self.meta.max_seqs
         # floats: temperatures, top-p, then MAX_DECODE_RUN rows of uniform numbers; ints: top-k,
@@ -138,30 +141,40 @@ class ModelRunner:
     def _singles_step(self, entries: Sequence[StepEntry]) -> torch.Tensor:
         """A step of single tokens without sampling, for a caller that picks tokens by itself.  Such steps come
         again and again with the same launches, which the host makes more slowly than the device runs them (12 to 15
-        us each; batch 1 of a small model 0.50 ms of host for 0.15 on the device, batch 8 at the 1B shape 1.36 and
-        0.86, a routed model of 130 launches 2.0 and 1.0).  The second step of a kind is captured, as it is, without
-        padding (so that it gives the bits of the first), and it and those after it are replayed.  The graphs of
-        the ``STEP_GRAPHS`` kinds used last are kept."""
+        us each; batch 1 of a small model 0.36 ms a step and 0.16 from a graph, batch 8 at the 1B shape 1.03 and 0.81,
+        a routed model of 130 launches 1.11 and 0.74).  A kind of step that is not known is launched as ever; once it has come
+        ``STEP_SIGHTINGS`` times it is captured, as it is, without padding (so that it gives the bits of the others), and
+        replayed from then on.  A capture costs 0.2 to 0.9 ms beyond the step, which four replays make up for: kinds that come
+        less often never pay it, and one whose graph gave way to another's before it had paid is captured later the
+        next time.  The graphs of the ``STEP_GRAPHS`` kinds used last are kept, none beyond the workspace it was made with."""
         step, _ = self.build_step(entries, pad_to=len(entries))
         key = (len(entries), self.model.launch_key(step.decode_shape))
-        known = self.step_graphs.pop(key, False)
-        if known is False:
-            self.step_graphs[key] = None      # seen once
-            logits = self.model.forward(step)
-        else:
-            if known is None:
-                # (other threads may go on allocating and launching meanwhile)
-                known = self._capture_launches(lambda: self.model.forward(step), capture_error_mode="thread_local")
-            self.step_graphs[key] = known
-            known.graph.replay()
-            self.num_graph_replays += 1
-            logits = known.logits
-        if len(self.step_graphs) > STEP_GRAPHS:
-            oldest = next(iter(self.step_graphs))
-            if self.step_graphs[oldest] is not None:
-                torch.cuda.synchronize()      # it may still run
-            del self.step_graphs[oldest]
-        return logits
+        if self._step_moves != self.ws.moves:
+            if self.step_graphs:
+                torch.cuda.synchronize()      # (one may still run)
+                self.step_graphs.clear()      # they hold memory that the workspace has let go
+            self._step_moves = self.ws.moves
+        known = self.step_graphs.pop(key, None)
+        if known is None:
+            seen, due = self.step_seen.pop(key, (0, STEP_SIGHTINGS))
+            self.step_seen[key] = (seen + 1, due)
+            if len(self.step_seen) > 8 * STEP_GRAPHS:
+                del self.step_seen[next(iter(self.step_seen))]
+            if seen + 1 < due:
+                return self.model.forward(step)
+            torch.cuda.synchronize()
+            while len(self.step_graphs) >= STEP_GRAPHS:
+                oldest = next(iter(self.step_graphs))
+                paid = self.step_graphs.pop(oldest).replays > STEP_SIGHTINGS
+                due = self.step_seen.get(oldest, (0, STEP_SIGHTINGS))[1]
+                self.step_seen[oldest] = (0, due if paid else min(2 * due, 1024))
+            # (other threads may go on allocating and launching meanwhile)
+            known = self._capture_launches(lambda: self.model.forward(step), capture_error_mode="thread_local")
+        self.step_graphs[key] = known
+        known.graph.replay()
+        known.replays += 1
+        self.num_graph_replays += 1
+        return known.logits
 
     def takes_runs(self, num_requests: int) -> bool:
         """Whether runs of decode steps on the device are possible for so many requests."""
@@ -391,6 +404,7 @@ class ModelRunner:
 
 GRAPH_MAX_BATCH = 128  # beyond this the matrix products leave the weight-streaming kernel
 STEP_GRAPHS = 16       # kinds of steps of single tokens (batch size and launch keys) whose launches are kept
+STEP_SIGHTINGS = 4     # steps of a kind after which they are
 MAX_DECODE_RUN = 16    # decode steps the device can take by itself before the host looks
 
 
@@ -406,4 +420,4 @@ class _QueuedRun:
 
 class _DecodeGraph:
     def __init__(self, graph, logits, keep) -> None:
-        self.graph, self.logits, self.keep = graph, logits, keep
+        self.graph, self.logits, self.keep, self.replays = graph, logits, keep, 0

@@ -1112,3 +1112,41 @@ def test_steps_of_single_tokens_give_the_bits_of_eager_ones(kind, kept, monkeypa
                 r.cache.free("long")
     assert runners[0].num_graph_replays >= 6 and len(runners[0].step_graphs) <= kept
     assert runners[1].num_graph_replays == 0 and not runners[1].step_graphs
+
+
+def test_steps_of_single_tokens_are_captured_when_they_have_come_often_enough(monkeypatch):
+    """Kinds that come a few times are launched as ever and push out no graph; a graph that gives way before its replays have made up
+    for it is made later the next time; none holds memory that the workspace has let go."""
+    from kvforge_amd import ModelRunner, StepEntry, Transformer
+    from kvforge_amd.engine import runner as runner_module
+    monkeypatch.setattr(runner_module, "STEP_GRAPHS", 2)
+    cfg = kvforge_amd.preset_dict("tiny-b")
+    r = ModelRunner(Transformer.from_random(cfg, 3, torch.bfloat16, "cuda"), 8, 256, max_num_seqs=12, max_num_batched_tokens=256,
+                    max_model_len=256)
+    for i in range(12):
+        r.cache.allocate(f"r{i}", 40)
+        r.step([StepEntry(f"r{i}", [3, 4, 5], 0, "none")])
+
+    def steps(batch, times=1):
+        before = r.num_graph_replays
+        for _ in range(times):
+            r.step([StepEntry(f"r{i}", [7], 3, "last") for i in range(batch)])
+        return r.num_graph_replays - before
+
+    def batches():
+        return [key[0] for key in r.step_graphs]
+    few = runner_module.STEP_SIGHTINGS
+    steps(12)        # (the workspace has room for every batch)
+    assert steps(1, few - 1) == 0 and not r.step_graphs
+    assert steps(1) == 1 and steps(1, 6) == 6 and batches() == [1]
+    assert sum(steps(b, few - 1) for b in range(3, 12)) == 0 and batches() == [1]     # not often enough, each
+    assert steps(2, few) == 1 and batches() == [1, 2]
+    assert steps(1) == 1 and batches() == [2, 1]
+    assert steps(3) == 1 and batches() == [1, 3]          # 2 gives way, used once
+    assert steps(2, 2 * few - 1) == 0 and steps(2) == 1 and batches() == [3, 2]
+    assert steps(1, few - 1) == 0 and steps(1) == 1 and batches() == [2, 1]          # 1 had been used often
+    r.cache.allocate("long", 200)
+    r.step([StepEntry("long", [5] * 200, 0, "last")])      # the workspace grows
+    assert steps(1) == 1 and batches() == [1]
+    held = {t.data_ptr() for t in r.ws.snapshot()}
+    assert all(t.data_ptr() in held for g in r.step_graphs.values() for t in g.keep)
