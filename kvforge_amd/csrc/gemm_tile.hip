@@ -27,9 +27,10 @@ typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
 // 64 lanes x 16 bytes from memory straight into LDS: base + off (per lane) -> lds + 16 * lane.  Written by hand because
 // the compiler, which cannot tell the stages of a buffer apart, waits for every such load before any read of
-// LDS.  The loads have no output register; whoever reads the bytes waits for vmcnt and the barrier first.
+// LDS.  The loads have no output register; whoever reads the bytes waits for vmcnt and the barrier first, in loads_left, which
+// says to the compiler that memory has changed: here it would order every read of LDS beside the load behind it.
 __device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0");
 }
 // At most N of the wave's own loads are still on their way, and the other waves have come as far.
 template <int N> __device__ __forceinline__ void loads_left() { asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory"); }

@@ -675,6 +675,7 @@ def test_experts_sum_and_the_next_norm_have_the_bits_of_their_steps(n, h, top, E
     (65, 64, 4, 2, 16, 16, 8, 0),          # one stage of K; fewer columns than a tile
     (129, 128, 3, 1, 40, 32, 4, 24),       # heads across the 16s, columns behind q, k and v, a row past a tile
     (193, 192, 5, 0, 48, 0, 16, 16),       # neither keys nor rotation
+    (130, 320, 4, 2, 32, 0, 8, 8),         # keys and values without rotation
     (320, 448, 32, 8, 64, 64, 16, 0),      # whole tiles
     (257, 1088, 12, 4, 64, 32, 16, 8)])
 def test_gemm_qkv_rope_tiles_has_the_bits_of_the_three_steps(tile, m, k, H, KV, d, rot, bs, extra):
@@ -720,6 +721,11 @@ def test_gemm_qkv_rope_tiles_has_the_bits_of_the_three_steps(tile, m, k, H, KV, 
         return torch.equal(torch.nan_to_num(x, nan=123.0), torch.nan_to_num(y, nan=123.0))
     assert same(q, want) and same(pages[0], pages[2]) and same(pages[1], pages[3])
     assert not KV or pages[0].count_nonzero() > 0
+    for p in pages[:2]:        # a layer that reads another's cache: q alone
+        p.fill_(5.0)
+    q.zero_()
+    ops().gemm_qkv_rope_tiles(a, w, q, *args, pages[0], pages[1], H, KV, d, write_kv=False, extra_cols=extra, tile=tile)
+    assert same(q, want) and all(bool((p == 5.0).all()) for p in pages[:2])
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
