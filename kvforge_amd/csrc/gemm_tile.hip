@@ -1,9 +1,10 @@
 // The fused q/k/v projection of many rows: C = A * W^T for bf16 rows and bf16 weights in tiles (see the head of
 // gemm_bf16.hip), fp32 sums, with rotary and the cache write in its epilogue (RopeEpi).
 //
-// Sums run along K in steps of 32 on one accumulator, as the library's product does at these shapes, and
-// are rounded to bf16 before they are rotated, as a stored product is: the results are the same to the bit as
-// those of the library's product and rope_kvwrite behind it.
+// Sums run along K in steps of 32 on one accumulator and are rounded to bf16 before they are rotated, as a stored product is.
+// The library's product, which stood here with rope_kvwrite behind it, does the same at most sizes, to the bit; it cuts K at 14 of
+// 306 that were compared (65 to 77 rows over 3,072 and 3,136 columns, 128 rows over 1,024 and 2,048), where 3 in 100,000 of the
+// result turn a rounding.
 //
 // A workgroup takes a tile of BM rows x BN columns, 64 of K a stage.  Rows and weights go from memory straight
 // into LDS, NB stages side by side, without passing through registers, and are asked for NB - 1.5 stages ahead.  A

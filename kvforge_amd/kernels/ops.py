@@ -1203,8 +1203,8 @@ def _qkv_tiles_take(m: int, n: int, k: int, rot: int, device: int) -> bool:
 def qkv_tiles_take(a: torch.Tensor, w, rot: int) -> bool:
     """Whether ``gemm_qkv_rope_tiles`` is to take ``a @ w.T``: more rows
     than the weight-streaming kernel's epilogue pays for, tiled bf16 weights, K in whole steps of 64, a rotary width ``rot``
-    in whole 8s up to 128, and a size at which it is
-    no slower than a product of its own and ``rope_kvwrite``.  Both give the same bits."""
+    in whole 8s up to 128, and a size at which it is no slower than a product of its own and ``rope_kvwrite``.  Where the library
+    does not cut K, which is most sizes, both give the same bits."""
     m, k = a.shape
     return (m > FUSED_EPILOGUE_MAX_M and isinstance(w, StreamedWeight) and a.dtype == BF16 and a.is_cuda
             and k % 64 == 0 and a.stride(1) == 1 and _rows_aligned(a, k, a.stride(0))
@@ -1283,8 +1283,8 @@ def gemm_qkv_rope_tiles(a: torch.Tensor, w: "StreamedWeight", q_out: torch.Tenso
                         block_table: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                         num_heads: int, num_kv_heads: int, head_dim: int, write_kv: bool = True,
                         extra_cols: int = 0, tile: int = -1) -> None:
-    """``gemm_qkv_rope`` for many rows of bf16 over tiled weights, with the product rounded to bf16 before it is rotated:
-    the bits of ``gemm`` and ``rope_kvwrite``.  K in whole steps of 64, a
+    """``gemm_qkv_rope`` for many rows of bf16 over tiled weights, with the product summed along K in order and rounded to bf16
+    before it is rotated: the bits of such a product stored and of ``rope_kvwrite``.  K in whole steps of 64, a
     rotary width in whole 8s up to 128.  ``tile``: which of its ``QKV_TILES`` tiles of rows and columns
     is taken (-1: by size)."""
     m, k = a.shape
