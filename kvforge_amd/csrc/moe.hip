@@ -1,5 +1,6 @@
 // Routed experts: the router's choice per token, and the row-wise steps around the experts'
 // matrix products.  Router arithmetic is fp32 throughout.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -181,8 +182,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int PLAN_EXPERT_BITS = 9, PLAN_MAX_EXPERTS = 1 << PLAN_EXPERT_BITS, PLAN_ROWS_BITS = 8;
 constexpr int PLAN_BATCH = 8;      // choices a thread of the plan has in flight
 constexpr int PREFETCH_SETS = 3;   // sets of operand registers in flight in the kernels of few rows
-constexpr int DEEP_SETS = 8;       // the same where there can be no more workgroups than
-constexpr int DEEP_BLOCKS = 384;
+constexpr int DEEP_SETS = 8;       // the same in deep_product
 constexpr long EXPERTS_STREAM_BYTES = 32l << 20;   // the eight L2s
 
 __device__ __forceinline__ int tile_expert(const int* tiles, int t) { return tiles[3 * t] & (PLAN_MAX_EXPERTS - 1); }
@@ -318,15 +318,14 @@ __global__ __launch_bounds__(CHOOSE_TOKENS * KVF_WAVE) void moe_choose_plan_kern
 //
 // The kernels of few rows (a decode step): a wave takes 16 rows of one expert and 16 weight rows, so that
 // the experts' matrices, which bound it, come in through as many workgroups as there are.  Two ways:
-// narrow_product, where there can be more workgroups than DEEP_BLOCKS: a step's two fragments are asked for two steps
-// ahead of the matrix instruction that uses them (PREFETCH_SETS sets of registers take turns), and lanes without a
-// row ask for none.  deep_product, where there are no more: a wave's own chain of trips is then what takes the time, so eight
-// steps are on their way, and no load is predicated (lanes without a row read the last one).
+// narrow_product: a step's two fragments are asked for two steps ahead of the matrix instruction that uses them
+// (PREFETCH_SETS sets of registers take turns), and lanes without a row ask for none.  deep_product: a wave's own chain
+// of trips is what takes the time where there are few workgroups, so eight steps are on their way, and no load is predicated
+// (lanes without a row read the last one).  See goes_deep for which is taken.
 // STREAMED (see load_16): up to 16 tokens, of whose experts each is read by one tile alone, over layers whose experts take
 // more than the L2s.  Four kernels and no branch in one: that was 3 to 10 us slower than either way by itself.
-// Plan, up and down (us; tokens, experts, 4 chosen, ff, K; matrices from memory): before, streamed, streamed and deep:
-//   1, 32, 1,024, 2,048: 32.8, 31.1, 18.3      8: 51.3, 46.4, 49.7      13: 70.3, 63.3, 62.2
-//   5, 32, 2,048, 2,048: 74.8, 67.8, 65.3      16, 16, 512, 1,024: 22.2, 20.4, 16.0      3: 18.9, 19.4, 14.2
+// Plan, up and down (us; tokens, experts, 4 chosen, ff, K; matrices from memory), cached and streamed, both narrow:
+//   8, 32, 1,024, 2,048: 51.3, 46.4      13: 70.3, 63.3      5, 32, 2,048, 2,048: 74.8, 67.8      16, 16, 512, 1,024: 22.2, 20.4
 template <class Load>
 __device__ __forceinline__ f32x4 narrow_product(int S, const Load& load) {
   constexpr int NB = PREFETCH_SETS;
@@ -857,6 +856,16 @@ KVF_EXPORT int kvf_moe_topk_plan(const float* z, int z_stride, const float* bias
   return kvf_last_error();
 }
 
+// Whether one of the kernels of few rows that can have so many workgroups takes deep_product.  What was measured over 13 layers
+// (8 to 128 experts, ff 256 to 3,584, K 1,024 to 4,096) and 1 to 41 tokens, each kernel by itself, narrow less deep in us:
+// up to two workgroups a compute unit (256 of them) faster or the same (0 to 18: up of 32 experts of 1,024 x 2,048, one token 8.3, four
+// 3.0; down of 8 of 3,584 x 2,048, ten tokens 11.7); from there to four either way, as few of the compute units have a third
+// one to wait for (5 tokens of the first -3.5, 8 of them 0.8; 4 of the second's up -2.7, 10 of them 3.0); beyond that faster
+// again or the same (down of the first at 13 tokens 0.8, up of 128 of 768 x 2,048, 13 tokens 3.6; worst -1.8 of 95).
+// Whole layers, deep up to 384 workgroups of the larger kernel / this: 4 tokens, 32 of 1,024 x 2,048 39.9 / 35.3; 5 tokens, 32 of
+// 2,048 x 2,048 64.7 / 63.3; 8 tokens, 8 of 3,584 x 2,048 76.6 / 66.0; of 168 none slower by more than runs differ (1.4%).
+static bool goes_deep(long blocks) { return blocks <= 512 || blocks > 1024; }
+
 // The routed experts of a bf16 step without the rows that did not choose them.  x [n, K] (row
 // stride ldx), w_gate_up / w_down: the tiled forms of [E 2 ff, K] (gate and up rows interleaved)
 // and [K, E ff]; sel / wgt [n, top]; scratch: where, order [n top], tiles [3 max_tiles],
@@ -894,21 +903,25 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, int n, int K, int E, int 
                        E * (ff / 32), tiles, num_tiles, out, K);
   } else {
     const bool streamed = n <= 16 && 6l * E * ff * K >= EXPERTS_STREAM_BYTES;
-    const int most = pairs < pairs / 16 + E ? pairs : pairs / 16 + E;    // tiles there can be
-    const auto both = [&](auto deep, auto st) {
-      hipLaunchKernelGGL((moe_up_kernel<decltype(deep)::value, decltype(st)::value>), dim3(up_blocks, max_tiles), dim3(256), 0, s,
-                         xb, ldx, K, up, S, order, tiles, num_tiles, top, ff, in_wgt, f, a);
-      hipLaunchKernelGGL((moe_down_kernel<decltype(deep)::value, decltype(st)::value>), dim3(down_blocks, max_tiles), dim3(256),
-                         0, s, a, ff, down, E * (ff / 32), tiles, num_tiles, out, K);
+    // (up to 16 tokens make one tile of every expert they choose)
+    const long most = std::min(pairs, n <= 16 ? E : pairs / 16 + E);
+    const auto go = [&](auto st) {
+      constexpr bool ST = decltype(st)::value;
+      const auto up_as = [&](auto deep) {
+        hipLaunchKernelGGL((moe_up_kernel<decltype(deep)::value, ST>), dim3(up_blocks, max_tiles), dim3(256), 0, s, xb, ldx, K, up, S,
+                           order, tiles, num_tiles, top, ff, in_wgt, f, a);
+      };
+      const auto down_as = [&](auto deep) {
+        hipLaunchKernelGGL((moe_down_kernel<decltype(deep)::value, ST>), dim3(down_blocks, max_tiles), dim3(256), 0, s, a, ff, down,
+                           E * (ff / 32), tiles, num_tiles, out, K);
+      };
+      if (goes_deep(most * up_blocks)) up_as(Flag<true>{});
+      else up_as(Flag<false>{});
+      if (goes_deep(most * down_blocks)) down_as(Flag<true>{});
+      else down_as(Flag<false>{});
     };
-    const auto deep_or_not = [&](auto st) {
-      if (most * static_cast<int>(up_blocks > down_blocks ? up_blocks : down_blocks) <= DEEP_BLOCKS)
-        both(Flag<true>{}, st);
-      else
-        both(Flag<false>{}, st);
-    };
-    if (streamed) deep_or_not(Flag<true>{});
-    else deep_or_not(Flag<false>{});
+    if (streamed) go(Flag<true>{});
+    else go(Flag<false>{});
   }
   return kvf_last_error();
 }

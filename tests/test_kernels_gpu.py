@@ -1729,7 +1729,7 @@ def test_grouped_experts_over_rows_of_many_passes(K, ff, weigh_input):
     test_grouped_experts_at_the_edges_of_their_tiles([20, 40, 290, 70, 128], K, ff, weigh_input)
 
 
-@pytest.mark.parametrize("E,ff,K", [(32, 512, 1024), (6, 512, 1024), (24, 96, 2312), (48, 224, 1032)])
+@pytest.mark.parametrize("E,ff,K", [(32, 512, 1024), (6, 512, 1024), (24, 96, 2312), (48, 224, 1032), (32, 1024, 1024), (20, 2080, 1032)])
 def test_a_token_s_experts_give_the_same_bits_in_every_batch(E, ff, K):
     """One token (few workgroups), 16 (each expert's rows in one tile) and 17 (no longer so) over layers whose experts
     are more and less than the caches hold take different kernels: a token's row is the same in all of them."""
