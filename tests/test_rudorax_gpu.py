@@ -619,7 +619,18 @@ def shape_c():
                        loop=(0, 2, 2), embedding_scale=11.3, logit_softcap=30.0, eps=1e-6, max_positions=512)
 
 
+def shape_wide():
+    """Wide enough (K beyond 224) for products of several parts to share launches: attention with head norms, a recurrence, routed
+    experts beside a shared one in every layer."""
+    att = dict(heads=8, kv_heads=2, dim=32, vdim=32, window=24, rot_dims=32, scale=32 ** -0.5, scaling=None)
+    rec = dict(heads=4, dim=64, vdim=64, gate_cap=15.0)
+    moe = dict(ff=64, experts=6, top=2, identity=1, shared_ff=288)
+    return make_config(vocab=300, width=256, layers=[("attention", att, moe), ("mlstm", rec, moe), ("attention", att, moe)],
+                       loop=None, embedding_scale=3.0, logit_softcap=30.0, eps=1e-6, max_positions=512)
+
+
 SHAPE = {"a": shape_a, "b": shape_b, "c": shape_c}
+WIDE = {"wide": shape_wide}
 
 
 def liven(folder: str) -> None:
@@ -653,7 +664,7 @@ def model_folder(tmp_path_factory, name: str, dtype):
     key = (name, dtype)
     if key not in _MODELS:
         folder = str(tmp_path_factory.mktemp(f"rudorax_{name}_{NAME[dtype]}"))
-        cfg = SHAPE[name]()
+        cfg = (SHAPE | WIDE)[name]()
         kvforge_amd.write_random_model(folder, cfg, seed=len(name) + 23, dtype=NAME[dtype])
         liven(folder)
         _MODELS[key] = (folder, cfg, load_file(os.path.join(folder, "model.safetensors")))
@@ -782,6 +793,38 @@ def test_prompts_in_portions(tmp_path_factory, name, dtype, sizes):
     seqs = prompts_for(cfg, [101], 4)
     got = replay(runner, seqs, in_portions("r0", 101, sizes))
     check(got["r0"], cfg, w, seqs["r0"], dtype, f"{name} {sizes}")
+
+
+@pytest.mark.parametrize("sizes", [(1, 8, 16, 2, 5), (16, 17, 15)])
+def test_products_that_ride_with_others_give_the_bits_of_launches_of_their_own(tmp_path_factory, monkeypatch, sizes):
+    """Steps of 1 to 16 rows have what mixer and experts begin with made in one launch, and the shared expert's last product in that
+    of the mixer's; 17 rows have not.  Against the same model with every product in a launch of its own, and against the plain one."""
+    from kvforge_amd.engine.batch import Step
+    folder, cfg, w = model_folder(tmp_path_factory, "wide", torch.bfloat16)
+    seqs = prompts_for(cfg, [101], 4)
+    plan = in_portions("r0", 101, sizes)
+    together, ride, rides, groups = Step._make_together, Step.ride, [], []
+
+    def counted(self, product):
+        rides.append((product[1].shape[0], sum(p[0][-1] == "shared_rows" for p in self.riders), ride(self, product)))
+        return rides[-1][-1]
+
+    def grouped(products, *taken):
+        made = together(products, *taken)
+        groups.append({key[-1] for key in made})
+        return made
+    monkeypatch.setattr(Step, "ride", counted)
+    monkeypatch.setattr(Step, "_make_together", staticmethod(grouped))
+    shared = replay(make_runner(folder, torch.bfloat16), seqs, plan)["r0"]
+    few = sum(b - a <= 16 for step in plan for _, a, b in step)
+    assert sum(rode and n == 1 for rows, n, rode in rides) == 3 * few and all(rows <= 16 for rows, n, rode in rides if rode)
+    assert sum({"act", "router", "qkv"} <= keys for keys in groups) == 2 * few
+    assert sum({"act", "router", "rows", "gates"} <= keys for keys in groups) == few
+    monkeypatch.setattr(Step, "ride", lambda self, product: False)
+    monkeypatch.setattr(Step, "_make_together", staticmethod(lambda *_: {}))
+    apart = replay(make_runner(folder, torch.bfloat16), seqs, plan)["r0"]
+    assert torch.equal(shared, apart)
+    check(shared, cfg, w, seqs["r0"], torch.bfloat16, str(sizes))
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -12,8 +12,8 @@ from kvforge_amd.engine.batch import Step, StepEntry, Workspace
 from kvforge_amd.engine.runner import ModelRunner
 from kvforge_amd.kernels import ops
 from kvforge_amd.models.transformer import Transformer
-from kvforge_amd.parts import (ChannelDelta, GatedDelta, LMHead, Mamba2, Mixer, MixerPair, ModelSpec, NamedRMSNorm, ParallelBlock,
-                               PlainFeedForward, RMSNorm, TokenEmbedding)
+from kvforge_amd.parts import (ChannelDelta, FeedForward, GatedDelta, LMHead, Mamba2, Mixer, MixerPair, ModelSpec, NamedRMSNorm, Norm,
+                               ParallelBlock, PlainFeedForward, RMSNorm, TokenEmbedding)
 from kvforge_amd.parts.base import LayerState, add_product
 
 
@@ -97,6 +97,58 @@ def test_mixers_side_by_side_as_one_by_one(by_torch, left, right, launches, earl
         step.settle()
         torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-3)
         assert not step.made and by_torch == (launches if rows <= 16 else [])
+
+
+class ToyNorm(Norm):
+    def __init__(self) -> None:
+        self.prefix = "n"
+
+    def forward(self, x, out, rows=None, add=None):
+        if add is not None:
+            x += add
+        out.copy_(x)
+
+
+class ToyFeedForward(FeedForward):
+    """``sin(x @ w.T) @ w_o.T`` for the stream, and the rows ``x @ w_r.T`` for ``seen``, which may ride with a product of the mixer's;
+    ``uses``: whether it looks for the products that it has announced."""
+
+    settles_residual = True
+
+    def __init__(self, uses: bool = True) -> None:
+        g = torch.Generator().manual_seed(5)
+        self.prefix, self.uses, self.seen = "f", uses, []
+        self.w, self.w_o, self.w_r = (torch.randn(*s, generator=g) for s in ((32, 24), (24, 32), (16, 24)))
+
+    def input_products(self, x, step):
+        return [(("f", "first"), x, self.w, step.ws.buf("f_first", (x.shape[0], 32), torch.float32), "store")]
+
+    def ready_products(self, x, step):
+        return [(("f", "ready"), x, self.w_r, step.ws.buf("f_ready", (x.shape[0], 16), torch.float32), "store")]
+
+    def forward(self, x, step, residual):
+        step.settle()
+        if self.uses:
+            step.make(self.input_products(x, step))
+            step.make(self.ready_products(x, step))
+            self.seen.append(step.ws.buf("f_ready", (x.shape[0], 16), torch.float32).clone())
+        add_product(step, torch.sin(x @ self.w.T), self.w_o, residual)
+
+
+def test_products_ride_with_the_mixers_last_one_and_none_may_be_left_over(by_torch):
+    for rows in (1, 16, 17):
+        by_torch.clear()
+        x, step, ffn = torch.randn(rows, 24, generator=torch.Generator().manual_seed(rows)), _step(), ToyFeedForward()
+        mixer = Toy("a", "", "toy", 40)
+        got = x.clone()
+        ParallelBlock(ToyNorm(), mixer, ffn, 24).forward(got, step, LayerState())
+        step.settle()
+        torch.testing.assert_close(got, x + mixer.plainly(x) + torch.sin(x @ ffn.w.T) @ ffn.w_o.T, rtol=1e-5, atol=1e-3)
+        torch.testing.assert_close(ffn.seen[0], x @ ffn.w_r.T, rtol=1e-5, atol=1e-4)
+        assert by_torch == ([3, 2] if rows <= 16 else []) and not step.riders     # first products; last one and rider
+    with pytest.raises(RuntimeError, match="not used.*first"):
+        ParallelBlock(ToyNorm(), Toy("a", "", "toy", 40), ToyFeedForward(uses=False), 24).forward(
+            torch.randn(4, 24), _step(), LayerState())
 
 
 def test_a_launch_of_several_products_refuses_memory_that_two_of_them_use():
