@@ -1035,11 +1035,33 @@ KVF_EXPORT int kvf_gemm_bf16(const void* A, int a_type, const void* W, int w_til
   return static_cast<int>(hipErrorInvalidValue);
 }
 
+// Whether no product of a launch of several (items and M as kvf_gemm_bf16_group) reads or writes what another one writes, since they run
+// at the same time.  Results that are blocks of columns of rows of one length are apart.
+KVF_EXPORT int kvf_gemm_bf16_group_apart(const long long* items, int count, int M) {
+  struct Rows { long long at, pitch, width, end; };
+  const auto rows = [M](long long at, long long pitch, long long width) { return Rows{at, pitch, width, at + (M - 1) * pitch + width}; };
+  const auto meet = [](const Rows& a, const Rows& b) { return a.at < b.end && b.at < a.end; };
+  for (int i = 0; i < count; ++i) {
+    const long long *v = items + 8 * i, size = v[7] == 0 || v[7] == 2 ? 4 : 2;
+    const Rows out = rows(v[2], v[6] * size, (v[7] == 3 ? v[3] / 2 : v[3]) * size);
+    for (int j = 0; j < count; ++j) {
+      const long long *u = items + 8 * j, other = u[7] == 0 || u[7] == 2 ? 4 : 2;
+      if (meet(out, rows(u[0], 2 * u[5], 2 * u[4]))) return 0;
+      const Rows to = rows(u[2], u[6] * other, (u[7] == 3 ? u[3] / 2 : u[3]) * other);
+      if (j >= i || !meet(out, to)) continue;
+      if (out.pitch != to.pitch || out.pitch <= 0) return 0;
+      const long long away = ((to.at - out.at) % out.pitch + out.pitch) % out.pitch;
+      if (away < out.width || away + to.width > out.pitch) return 0;
+    }
+  }
+  return 1;
+}
+
 // Several products of M <= 16 rows in one launch (see gemm_group_kernel).  items: for each A, W, C (addresses), N, K, lda, ldc
 // and epi (0 store fp32, 1 store bf16, 2 add into fp32, 3 SwiGLU pairs -> bf16 [M, N/2]); W in tiles, K beyond 224 (a k-step for every wave).
 KVF_EXPORT int kvf_gemm_bf16_group(const long long* items, int count, int M, hipStream_t s) {
   if (M <= 0 || count <= 0) return 0;
-  if (M > 16 || count > GROUP_MAX) return static_cast<int>(hipErrorInvalidValue);
+  if (M > 16 || count > GROUP_MAX || !kvf_gemm_bf16_group_apart(items, count, M)) return static_cast<int>(hipErrorInvalidValue);
   Group g{};
   int blocks = 0;
   for (int i = 0; i < count; ++i) {

@@ -234,8 +234,8 @@ class Step:
         # Whether the sublayer that runs adds to a stream whose next reader does not take a product in
         # parts (``take_owed``), so that an add kernel of its own has to follow one.
         self.settled_next = False
-        # products that a block has had made together with others, ahead of the parts they belong to: key -> rows
-        self.made: dict[tuple, torch.Tensor] = {}
+        # products that a block has had made together with others, ahead of the parts they belong to: key -> address of the rows
+        self.made: dict[tuple, int] = {}
         # products that are ready and ride with the next one that a mixer ends in; whether a mixer's last product waits for
         # another's instead of being made (rows of its own only)
         self.riders: list = []
@@ -269,13 +269,14 @@ class Step:
         from kvforge_amd.kernels import ops
         rest, done = products, ()
         if products[0][1].shape[0] <= ops.FUSED_NORM_MAX_M:
-            # (a product counts as made where its part looks for it: a buffer may have moved since)
-            rest = [p for p in products if p[0] not in self.made or self.made[p[0]].data_ptr() != p[3].data_ptr()]
-            for p in products:
-                self.made.pop(p[0], None)
-            if self.made and rest:       # rows of others that are written over now are theirs to make again
-                written = [ops.span_of(p[3]) for p in rest]
-                self.made = {k: out for k, out in self.made.items() if not ops.meets(ops.span_of(out), written)}
+            made = self.made
+            if made:
+                # (a product counts as made where its part looks for it: a buffer may have moved since)
+                rest = [p for p in products if made.pop(p[0], None) != p[3].data_ptr()]
+                if made and rest:       # rows of others that are written over now are theirs to make again
+                    written = [(p[3].data_ptr(), p[3].data_ptr() + p[3].nbytes) for p in rest]
+                    for key in [k for k, at in made.items() if any(lo <= at < hi for lo, hi in written)]:
+                        del made[key]
             done = self._make_together(rest)
         for key, a, w, out, how in rest:
             if key not in done:
@@ -289,31 +290,33 @@ class Step:
             return False
         along, self.riders = self.riders[:ops.GROUP_MAX - 1], self.riders[ops.GROUP_MAX - 1:]
         ops.gemm_group([p[1:] for p in (product, *along)])
-        self.made.update((p[0], p[3]) for p in along)
+        self.made.update((p[0], p[3].data_ptr()) for p in along)
         return True
 
     def make_early(self, products: list) -> None:
         """Products that several parts are going to begin with and whose inputs are there: those that go into one launch are
-        made now, and the parts find them made.  Rows that lie where another part's do, which is ahead of it here and
-        has not read them yet, are not: such a product is left to its part."""
-        from kvforge_amd.kernels import ops
-        self.made.update(self._make_together(products, [ops.span_of(out) for out in self.made.values()]))
+        made now, and the parts find them made.  Rows that begin where another part's do, which is ahead of it here and
+        has not read them yet (one buffer of the workspace), are not: such a product is left to its part."""
+        self.made.update(self._make_together(products, self.made.values()))
 
     @staticmethod
-    def _make_together(products: list, taken: Sequence[tuple[int, int]] = ()) -> dict:
+    def _make_together(products: list, taken=()) -> dict:
+        """What was made, key -> address.  ``taken``: addresses that are not to be written to."""
         from kvforge_amd.kernels import ops
         if len(products) < 2 or products[0][1].shape[0] > ops.FUSED_NORM_MAX_M:
             return {}
-        some, spans = [], list(taken)
+        some, made, taken = [], {}, set(taken)
         for p in products:
-            span = ops.span_of(p[3])
-            if len(some) < ops.GROUP_MAX and ops.gemm_group_takes(p[1], p[2], p[3]) and not ops.meets(span, spans):
-                some.append(p)
-            spans.append(span)
+            at = p[3].data_ptr()
+            if at not in taken:
+                taken.add(at)
+                if len(some) < ops.GROUP_MAX and ops.gemm_group_takes(p[1], p[2], p[3]):
+                    some.append(p[1:])
+                    made[p[0]] = at
         if len(some) < 2:
             return {}
-        ops.gemm_group([p[1:] for p in some])
-        return {p[0]: p[3] for p in some}
+        ops.gemm_group(some)
+        return made
 
     def owe(self, residual: torch.Tensor, product: torch.Tensor) -> None:
         self.settle()

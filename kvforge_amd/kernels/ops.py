@@ -82,22 +82,15 @@ def _check_natively() -> None:
         _check, _operands = native.check, native.operands
 
 
-def span_of(t: torch.Tensor) -> tuple[int, int]:
-    """Where the memory that a tensor's storage view spans begins and ends."""
-    begin, n = t.data_ptr(), t.numel()
-    if n and not t.is_contiguous():
-        n = 1 + sum((size - 1) * stride for size, stride in zip(t.shape, t.stride()))
-    return begin, begin + n * t.element_size()
-
-
-def meets(span: tuple[int, int], others) -> bool:
-    """Whether a span and any of the others intersect."""
-    return any(span[0] < end and begin < span[1] for begin, end in others)
-
-
 def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether the memory spanned by two tensors' storage views intersects."""
-    return meets(span_of(a), [span_of(b)])
+    def span(t):
+        if t.numel() == 0:
+            return t.data_ptr(), t.data_ptr()
+        last = sum((n - 1) * st for n, st in zip(t.shape, t.stride()))
+        return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
+    (a0, a1), (b0, b1) = span(a), span(b)
+    return a0 < b1 and b0 < a1
 
 
 def _ok(code: int, what: str) -> None:
@@ -1126,32 +1119,14 @@ def gemm_group_takes(a: torch.Tensor, w, out: torch.Tensor) -> bool:
             and out.dtype in (F32, BF16))
 
 
-def _check_column_blocks(outs) -> None:
-    """Outputs whose spans intersect: each pair of them are blocks of columns, apart, of rows of one length."""
-    for i, a in enumerate(outs):
-        for b in outs[:i]:
-            if not _overlap(a, b):
-                continue
-            pitch, width, other = (a.stride(0) * a.element_size(), a.shape[1] * a.element_size(), b.shape[1] * b.element_size())
-            away = (b.data_ptr() - a.data_ptr()) % pitch if pitch else 0
-            if pitch != b.stride(0) * b.element_size() or away < width or away + other > pitch:
-                raise KernelError("gemm_group: products write the same memory")
-
-
 def gemm_group(products) -> None:
     """Several products ``out = a @ w.T`` of equally many rows in one launch: ``(a, w, out, how)`` each, ``out`` fp32 or bf16, ``how``
     ``"store"``, ``"add"`` (``out += a @ w.T``, fp32) or ``"pairs"``: neighbouring columns are (gate, up) and ``out = silu(gate) * up``
     (``gemm_gated`` without biases).  For products that ``gemm_group_takes``; the bits of ``gemm`` and ``gemm_gated``.  They run at
-    the same time: none reads or writes what another writes (column blocks of the same rows are apart)."""
+    the same time: none reads or writes what another writes (column blocks of rows of one length are apart)."""
     if not 0 < len(products) <= GROUP_MAX:
         raise KernelError(f"gemm_group: 1 to {GROUP_MAX} products, got {len(products)}")
     rows, items = products[0][0].shape[0], []
-    reads = {span_of(p[0]) for p in products}
-    writes = sorted(span_of(p[2]) for p in products)
-    if any(meets(w, reads) for w in writes):
-        raise KernelError("gemm_group: a product reads what another writes")
-    if any(second[0] < first[1] for first, second in zip(writes, writes[1:])):
-        _check_column_blocks([p[2] for p in products])
     for a, w, out, how in products:
         m, n, k, lda, ldc = _gemm_operands(a, w, out, _halves if how == "pairs" else _whole)
         epi = {"store": 0 if out.dtype == F32 else 1, "add": 2, "pairs": 3}.get(how)
@@ -1160,7 +1135,11 @@ def gemm_group(products) -> None:
             raise KernelError("gemm_group: operands do not fit the kernel")
         items += [a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), n, k, lda, ldc, epi]
     f = _fn("gemm_bf16", "kvf_gemm_bf16_group", [c_void_p, c_int, c_int, c_void_p])
-    _ok(f((c_longlong * len(items))(*items), len(products), rows, _stream()), "gemm_group")
+    items = (c_longlong * len(items))(*items)
+    code = f(items, len(products), rows, _stream())
+    if code != 0 and not _fn("gemm_bf16", "kvf_gemm_bf16_group_apart", [c_void_p, c_int, c_int])(items, len(products), rows):
+        raise KernelError("gemm_group: a product reads or writes what another one writes")
+    _ok(code, "gemm_group")
 
 
 def gemm_fused(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rms_eps: float | None = None,

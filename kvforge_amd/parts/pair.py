@@ -135,6 +135,7 @@ class MixerPair(Mixer):
             rows.append(out)
         for _, a, w, out, _how in step.riders:      # (not taken along)
             ops.gemm(a, w, out)
-        step.made = {key: out for key, out in step.made.items() if key[0] != "rider"}
+        for key in [k for k in step.made if k[0] == "rider"]:
+            del step.made[key]
         step.riders = riders
         ops.rms_add_two(residual, rows[0], self.weights[0], rows[1], self.weights[1], self.norms[0].eps)

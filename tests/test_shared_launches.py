@@ -3,6 +3,9 @@ both keep their rows in the same workspace buffers."""
 
 from __future__ import annotations
 
+import ctypes
+import random
+
 import pytest
 import torch
 
@@ -10,7 +13,7 @@ import kvforge_amd
 from kvforge_amd.config.model import ModelConfig
 from kvforge_amd.engine.batch import Step, StepEntry, Workspace
 from kvforge_amd.engine.runner import ModelRunner
-from kvforge_amd.kernels import ops
+from kvforge_amd.kernels import library, ops
 from kvforge_amd.models.transformer import Transformer
 from kvforge_amd.parts import (ChannelDelta, FeedForward, GatedDelta, LMHead, Mamba2, Mixer, MixerPair, ModelSpec, NamedRMSNorm, Norm,
                                ParallelBlock, PlainFeedForward, RMSNorm, TokenEmbedding)
@@ -151,17 +154,49 @@ def test_products_ride_with_the_mixers_last_one_and_none_may_be_left_over(by_tor
             torch.randn(4, 24), _step(), LayerState())
 
 
+STORE_F32, STORE_BF16, ADD, PAIRS = range(4)      # what becomes of a product
+
+
+@pytest.mark.parametrize("rows", [1, 3, 16])
+def test_products_of_one_launch_lie_apart(rows):
+    """Results of a launch against memory written out: a product is refused where it writes what another writes or reads."""
+    apart = ctypes.CDLL(library.build_module("gemm_bf16")).kvf_gemm_bf16_group_apart
+    rng = random.Random(rows)
+    seen = set()
+    for _ in range(3000):
+        items, writes, reads = [], [], []
+        for _ in range(rng.randint(1, 4)):
+            n, k, epi = rng.choice([4, 8, 16]), rng.choice([8, 16]), rng.choice([STORE_F32, STORE_BF16, ADD, PAIRS])
+            size, cols = 4 if epi in (STORE_F32, ADD) else 2, n // 2 if epi == PAIRS else n
+            ldc, lda = (cols if rows == 1 else rng.choice([cols, 16, 24])), (k if rows == 1 else rng.choice([k, 24]))
+            ldc = max(ldc, cols)
+            a, c = 4096 + 16 * rng.randint(0, 100), 4096 + 4 * rng.randint(0, 400) + rng.choice([0, 1 << 16])
+            items += [a, 64, c, n, k, lda, ldc, epi]
+            reads.append({a + 2 * (r * lda + i) + b for r in range(rows) for i in range(k) for b in range(2)})
+            writes.append({c + size * (r * ldc + i) + b for r in range(rows) for i in range(cols) for b in range(size)})
+        clash = any(x & y for i, x in enumerate(writes) for y in writes[:i]) or any(x & y for x in writes for y in reads)
+        said = apart((ctypes.c_longlong * len(items))(*items), len(items) // 8, rows)
+        assert not (said and clash), items
+        seen.add((bool(said), clash))
+    assert seen >= {(True, False), (False, True)}
+    column = lambda at, first: [4096, 64, at + 4 * first, 16, 64, 64, 48, STORE_F32]  # noqa: E731
+    if rows > 1:
+        for firsts, want in (((0, 16, 32), 1), ((32, 0, 16), 1), ((0, 8), 0), ((0, 40), 0), ((0, 0), 0), ((0, 48), 0)):
+            items = sum((column(1 << 20, f) for f in firsts), [])
+            assert apart((ctypes.c_longlong * len(items))(*items), len(firsts), rows) == want, firsts
+
+
+@pytest.mark.gpu
 def test_a_launch_of_several_products_refuses_memory_that_two_of_them_use():
-    a, wide = torch.zeros(3, 64), torch.zeros(3, 48)
-    w = torch.zeros(16, 64)
-    for products in ([(a, w, wide[:, :16], "store"), (a, w, wide[:, 8:24], "store")],
-                     [(a, w, wide.view(-1)[:48].view(3, 16), "store"), (a, w, wide.view(-1)[40:88].view(3, 16), "store")],
-                     [(a, w, wide[:, 16:32], "store"), (a, w, wide.view(-1)[:48].view(3, 16), "store")]):
-        with pytest.raises(ops.KernelError, match="write the same memory"):
+    a, wide = torch.ones(3, 512, dtype=torch.bfloat16, device="cuda"), torch.zeros(3, 48, device="cuda")
+    w = ops.StreamedWeight(torch.ones(16, 256, dtype=torch.bfloat16, device="cuda"))
+    for products in ([(a[:, :256], w, wide[:, :16], "store"), (a[:, :256], w, wide[:, 8:24], "add")],
+                     [(a[:, :256], w, a[:, 400:416], "store"), (a[:, :256], w, wide[:, :16], "store")]):
+        with pytest.raises(ops.KernelError, match="what another one writes"):
             ops.gemm_group(products)
-    with pytest.raises(ops.KernelError, match="reads what another writes"):
-        ops.gemm_group([(a, w, wide[:, :16], "store"), (wide[:, 16:32], w, a[:, :16], "store")])
-    ops._check_column_blocks([wide[:, :16], wide[:, 16:32], wide[:, 40:], a])
+    assert bool((wide == 0).all()) and bool((a == 1).all())
+    ops.gemm_group([(a[:, :256], w, wide[:, f:f + 16], "store") for f in (0, 32, 16)])
+    assert bool((wide == 256).all())
 
 
 # ------------------------------------------------------------------------------------- on the GPU, whole models
