@@ -219,8 +219,12 @@ template <bool STREAMED> __device__ __forceinline__ bf16x8 load_weight(const bf1
 // Eight rows (us, cached and streamed): output head of 525 MB 89.5 and 76.6, gated pair of 67 MB 15.3 and 14.6, q/k/v
 // of 12.6 MB 8.4 and 7.8 and the attention behind them 8.8 and 7.7; 41 rows over 12.6 MB 11.3 and 10.3.  The line is at what
 // an XCD's L2 holds: the matrices of a decoder 512 wide (0.5 to 2.9 MB), which do lie in the caches, took 0.2 to 0.6 us longer
-// streamed, one of 8 MB the same.  (gemm_mid_kernel, whose workgroups share lines: 15.7 and 16.9, so it does not.)
+// streamed, one of 8 MB the same.  (gemm_mid_kernel, whose workgroups share lines: 15.7 and 16.9, so it does not.)  A matrix of
+// a model that lies in the last-level cache as a whole does come from there the next step: the caller says so (CACHED), see
+// StreamedWeight.
 constexpr long STREAM_BYTES = 4l << 20;
+constexpr int CACHED = 2;          // w_tiled: in tiles, and through the caches whatever its size
+constexpr int GROUP_CACHED = 8;    // the same in an item of a launch of several
 __host__ __device__ inline bool streams(int N, int K) { return 2l * N * K >= STREAM_BYTES; }
 
 // 8 fp32 (with ADD plus 8 of `q`) -> 8 bf16 (round to nearest even); adds their squares to ss.
@@ -767,6 +771,7 @@ struct GroupItem {
   const bf16_t* W;
   void* C;
   int N, K, lda, ldc, epi, first;   // first: its first workgroup
+  bool streamed;
 };
 constexpr int GROUP_MAX = 8, GROUP_WAVES = 8;
 struct Group {
@@ -811,7 +816,7 @@ __global__ __launch_bounds__(GROUP_WAVES * KVF_WAVE) void gemm_group_kernel(Grou
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
     }
   };
-  if (streams(it.N, it.K)) walk(Flag<true>{});
+  if (it.streamed) walk(Flag<true>{});
   else walk(Flag<false>{});
   *reinterpret_cast<f32x4*>(red + (wave * KVF_WAVE + lane) * 4) = acc;
   __syncthreads();
@@ -846,7 +851,7 @@ template <int MT, int NT, int AT, int EPI, bool ADD>
 int launch_as(dim3 grid, dim3 block, size_t lds, const void* A, const bf16_t* W, void* C, int M, int N, int K, int lda,
               int ldc, int m_base, float eps, int w_tiled, const Riders& rd, const RopeEpi& rp, const PickEpi& pk,
               hipStream_t s) {
-  if (w_tiled && streams(N, K))
+  if (w_tiled && w_tiled != CACHED && streams(N, K))
     hipLaunchKernelGGL((gemm_skinny_kernel<MT, NT, AT, EPI, ADD, true>), grid, block, lds, s, A, W, C, M, N, K, lda,
                        ldc, m_base, eps, w_tiled, rd, rp, pk);
   else
@@ -1014,7 +1019,7 @@ KVF_EXPORT void kvf_gemm_bf16_set_rows(int rows) { g_rows_override = rows; }
 
 // a_type: 0 = bf16 rows, 1 = fp32 rows normalised by rsqrt(mean(x^2) + eps) in the kernel.
 // epi: 0 store fp32, 1 store bf16, 2 add into fp32, 3 SwiGLU pairs -> bf16 [M, N/2].
-// w_tiled: W is [N, K] row-major (0) or in tiles of 16 x 32 (1, see the head of this file).
+// w_tiled: W is [N, K] row-major (0) or in tiles of 16 x 32 (1, see the head of this file; CACHED: and not to go past the caches).
 // c_add (epi 2 only, may be null): bf16 [M, ldc], added to C together with the product.
 // half_out (epi 2 with bf16 rows only, may be null): bf16 [M, ldc]; the product over the second
 //   half of K is stored there instead of being added to C, by a second layer of workgroups.
@@ -1042,12 +1047,12 @@ KVF_EXPORT int kvf_gemm_bf16_group_apart(const long long* items, int count, int 
   const auto rows = [M](long long at, long long pitch, long long width) { return Rows{at, pitch, width, at + (M - 1) * pitch + width}; };
   const auto meet = [](const Rows& a, const Rows& b) { return a.at < b.end && b.at < a.end; };
   for (int i = 0; i < count; ++i) {
-    const long long *v = items + 8 * i, size = v[7] == 0 || v[7] == 2 ? 4 : 2;
-    const Rows out = rows(v[2], v[6] * size, (v[7] == 3 ? v[3] / 2 : v[3]) * size);
+    const long long *v = items + 8 * i, epi = v[7] & ~GROUP_CACHED, size = epi == 0 || epi == 2 ? 4 : 2;
+    const Rows out = rows(v[2], v[6] * size, (epi == 3 ? v[3] / 2 : v[3]) * size);
     for (int j = 0; j < count; ++j) {
-      const long long *u = items + 8 * j, other = u[7] == 0 || u[7] == 2 ? 4 : 2;
+      const long long *u = items + 8 * j, its = u[7] & ~GROUP_CACHED, other = its == 0 || its == 2 ? 4 : 2;
       if (meet(out, rows(u[0], 2 * u[5], 2 * u[4]))) return 0;
-      const Rows to = rows(u[2], u[6] * other, (u[7] == 3 ? u[3] / 2 : u[3]) * other);
+      const Rows to = rows(u[2], u[6] * other, (its == 3 ? u[3] / 2 : u[3]) * other);
       if (j >= i || !meet(out, to)) continue;
       if (out.pitch != to.pitch || out.pitch <= 0) return 0;
       const long long away = ((to.at - out.at) % out.pitch + out.pitch) % out.pitch;
@@ -1058,7 +1063,8 @@ KVF_EXPORT int kvf_gemm_bf16_group_apart(const long long* items, int count, int 
 }
 
 // Several products of M <= 16 rows in one launch (see gemm_group_kernel).  items: for each A, W, C (addresses), N, K, lda, ldc
-// and epi (0 store fp32, 1 store bf16, 2 add into fp32, 3 SwiGLU pairs -> bf16 [M, N/2]); W in tiles, K beyond 224 (a k-step for every wave).
+// and epi (0 store fp32, 1 store bf16, 2 add into fp32, 3 SwiGLU pairs -> bf16 [M, N/2]; with GROUP_CACHED: W not past the caches); W in
+// tiles, K beyond 224 (a k-step for every wave).
 KVF_EXPORT int kvf_gemm_bf16_group(const long long* items, int count, int M, hipStream_t s) {
   if (M <= 0 || count <= 0) return 0;
   if (M > 16 || count > GROUP_MAX || !kvf_gemm_bf16_group_apart(items, count, M)) return static_cast<int>(hipErrorInvalidValue);
@@ -1069,7 +1075,8 @@ KVF_EXPORT int kvf_gemm_bf16_group(const long long* items, int count, int M, hip
     GroupItem& it = g.item[i];
     it = GroupItem{reinterpret_cast<const bf16_t*>(v[0]), reinterpret_cast<const bf16_t*>(v[1]), reinterpret_cast<void*>(v[2]),
                    static_cast<int>(v[3]), static_cast<int>(v[4]), static_cast<int>(v[5]), static_cast<int>(v[6]),
-                   static_cast<int>(v[7]), blocks};
+                   static_cast<int>(v[7] & ~GROUP_CACHED), blocks, false};
+    it.streamed = !(v[7] & GROUP_CACHED) && streams(it.N, it.K);
     if (!it.A || !it.W || !it.C || it.N <= 0 || it.K <= 224 || it.K % 8 != 0 || it.lda % 8 != 0 || v[0] % 16 != 0 || v[1] % 16 != 0 ||
         !(it.epi >= 0 && (it.epi <= 2 || (it.epi == 3 && it.N % 4 == 0))))
       return static_cast<int>(hipErrorInvalidValue);

@@ -872,12 +872,13 @@ static bool goes_deep(long blocks) { return blocks <= 512 || blocks > 1024; }
 // num_tiles [1], act [n top, ff], y [n top, K].  Needs K % 8 == 0 and ff % 32 == 0.  The outputs' rows stay in y, which
 // kvf_moe_combine adds up.  weigh_input: the weights go into the experts' inputs instead of the sum over their outputs.  form, limit: how an expert's pairs are joined (GateForm's act 0 or 2).  many_rows: below
 // 0, or which kernels are taken whatever the sizes (0: those of few rows, else those of more).  planned: where,
-// order, tiles and num_tiles hold the plan already (kvf_moe_topk_plan).
+// order, tiles and num_tiles hold the plan already (kvf_moe_topk_plan).  cached: the matrices are not to go past the caches, whatever
+// their size.
 KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, int n, int K, int E, int ff, int top,
                                const void* w_gate_up, const void* w_down, const int* sel, const float* wgt,
                                int* where, int* order, int* tiles, int* num_tiles, int max_tiles, void* act,
                                void* y, int weigh_input, int form, float limit,
-                               int many_rows, int planned, hipStream_t s) {
+                               int many_rows, int planned, int cached, hipStream_t s) {
   if (n <= 0) return 0;
   const int pairs = n * top;
   const bool many = many_rows < 0 ? kvf_moe_grouped_many_rows(pairs, E, ff, K) != 0 : many_rows != 0;
@@ -902,7 +903,7 @@ KVF_EXPORT int kvf_moe_grouped(const void* x, int ldx, int n, int K, int E, int 
     hipLaunchKernelGGL(moe_down_wide_kernel, dim3((down_blocks * most + 7) / 8 * 8), dim3(256), 0, s, a, ff, down,
                        E * (ff / 32), tiles, num_tiles, out, K);
   } else {
-    const bool streamed = n <= 16 && 6l * E * ff * K >= EXPERTS_STREAM_BYTES;
+    const bool streamed = n <= 16 && !cached && 6l * E * ff * K >= EXPERTS_STREAM_BYTES;
     // (up to 16 tokens make one tile of every expert they choose)
     const long most = std::min(pairs, n <= 16 ? E : pairs / 16 + E);
     const auto go = [&](auto st) {

@@ -798,9 +798,13 @@ class StreamedWeight:
     matrix-core instruction takes them (position ``16*c + r`` holds row ``r``, columns
     ``8c..8c+7``), zero-padded.  The weight-streaming kernel then loads 1 KB of consecutive bytes
     per operand fragment instead of 64 bytes from each of 16 rows, which is what lets it reach
-    the memory's bandwidth.  Costs the matrix's size in memory a second time."""
+    the memory's bandwidth.  Costs the matrix's size in memory a second time.
 
-    def __init__(self, plain: torch.Tensor) -> None:
+    ``cached``: kernels of few rows do not ask for it past the caches, as they do for large matrices otherwise.  A model sets it
+    where all its matrices lie in the last-level cache from one step to the next (``LAST_LEVEL_BYTES``); what they are worth
+    together no kernel can know."""
+
+    def __init__(self, plain: torch.Tensor, cached: bool = False) -> None:
         if plain.dim() != 2 or plain.dtype != BF16 or not plain.is_contiguous():
             raise KernelError("a streamed weight is a contiguous bf16 matrix")
         n, k = plain.shape
@@ -813,12 +817,19 @@ class StreamedWeight:
         self.tiles = (padded.view(n_pad // 16, 16, k_pad // 32, 4, 8).permute(0, 2, 3, 1, 4)
                       .contiguous().view(n_pad // 16, k_pad // 32, 64, 8))
         self.shape, self.dtype, self.device = plain.shape, plain.dtype, plain.device
+        self.cached = bool(cached)
 
     def dim(self) -> int:
         return 2
 
 
 TILE_WEIGHTS = True  # parts keep the matrices they stream for few rows in tiles as well
+
+
+# What the last-level cache holds.  Decode steps of one request and of 16, us, matrices of 4 MB and more past the caches / through
+# them: models of 139 MB 122.9 / 117.5, 148.2 / 142.1; 200 MB 169.6 / 164.2, 208.0 / 198.8; 214 MB 96.3 / 91.2, 121.7 / 114.2; 277 MB
+# 103.2 / 107.7, 126.0 / 130.9; 383 MB 316.6 / 351.5, 387.5 / 419.5.
+LAST_LEVEL_BYTES = 256 << 20
 
 
 def streamed(w: torch.Tensor):
@@ -843,7 +854,7 @@ def copies_of(w) -> list[torch.Tensor]:
 def _w_args(w) -> tuple[int, int]:
     """(pointer, tiled flag) of a weight for the weight-streaming kernel."""
     if isinstance(w, StreamedWeight):
-        return w.tiles.data_ptr(), 1
+        return w.tiles.data_ptr(), 2 if w.cached else 1
     return w.data_ptr(), 0
 
 
@@ -1133,7 +1144,7 @@ def gemm_group(products) -> None:
         if (m != rows or epi is None or not gemm_group_takes(a, w, out) or (epi == 3 and (n % 4 or out.dtype != BF16))
                 or (epi == 2 and out.dtype != F32)):
             raise KernelError("gemm_group: operands do not fit the kernel")
-        items += [a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), n, k, lda, ldc, epi]
+        items += [a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), n, k, lda, ldc, epi | 8 if w.cached else epi]
     f = _fn("gemm_bf16", "kvf_gemm_bf16_group", [c_void_p, c_int, c_int, c_void_p])
     items = (c_longlong * len(items))(*items)
     code = f(items, len(products), rows, _stream())
@@ -2162,13 +2173,13 @@ def moe_grouped(x: torch.Tensor, w_gate_up: "StreamedWeight", w_down: "StreamedW
     for name, dtype, shape in (("act", BF16, (pairs, ff)), ("y", BF16, (pairs, k))):
         _check(scratch[name], name, dtype, shape)
     f = _fn("moe", "kvf_moe_grouped", [c_void_p] + [c_int] * 6 + [c_void_p] * 8 + [c_int]
-            + [c_void_p] * 2 + [c_int, c_int, c_float, c_int, c_int, c_void_p])
+            + [c_void_p] * 2 + [c_int, c_int, c_float, c_int, c_int, c_int, c_void_p])
     _ok(f(x.data_ptr(), x.stride(0) if n > 1 else k, n, k, int(experts), int(ff), top,
           w_gate_up.tiles.data_ptr(), w_down.tiles.data_ptr(), chosen.data_ptr(), weights.data_ptr(),
           scratch["where"].data_ptr(), scratch["order"].data_ptr(), scratch["tiles"].data_ptr(),
           scratch["num_tiles"].data_ptr(), max_tiles, scratch["act"].data_ptr(), scratch["y"].data_ptr(),
           1 if weigh_input else 0, code, lim, -1 if many_rows is None else int(many_rows), 1 if planned else 0,
-          _stream()), "moe_grouped")
+          1 if w_gate_up.cached and w_down.cached else 0, _stream()), "moe_grouped")
     if combine:
         moe_combine(residual, scratch["y"], x, chosen, None if weigh_input else weights, scratch["where"], experts, fresh)
 

@@ -8,7 +8,7 @@ import torch
 
 from kvforge_amd import registry
 from kvforge_amd.cache.manager import CacheGroup
-from kvforge_amd.kernels import library
+from kvforge_amd.kernels import library, ops
 from kvforge_amd.parts.block import norm_rows
 from kvforge_amd.parts.base import Block, CacheSpec, LayerState, ModelSpec, StateSpec
 from kvforge_amd.weights.loader import load_model_weights
@@ -87,6 +87,12 @@ class Transformer:
     def _seal(self) -> None:
         for p in self.spec.all_parts():
             p.seal()
+        # a model that the last-level cache holds from one step to the next is read through it
+        weights = {w.tiles.data_ptr(): w for p in self.spec.all_parts() for w in p.streamed_weights()}
+        cached = sum(w.tiles.nbytes for w in weights.values()) <= ops.LAST_LEVEL_BYTES
+        for p in self.spec.all_parts():
+            for w in p.streamed_weights():
+                w.cached = cached
         self._loaded = True
 
     def kernel_modules(self) -> list[str]:

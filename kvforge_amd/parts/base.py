@@ -148,6 +148,25 @@ class Part:
         (what the weights occupy, as opposed to what a step reads)."""
         return []
 
+    def streamed_weights(self) -> list:
+        """The matrices in tiles (``ops.StreamedWeight``) that this part and the parts it is made of hold, each once."""
+        from kvforge_amd.kernels.ops import StreamedWeight
+        found, seen, todo = [], set(), [self]
+        while todo:
+            v = todo.pop()
+            if id(v) in seen:
+                continue
+            seen.add(id(v))
+            if isinstance(v, StreamedWeight):
+                found.append(v)
+            elif isinstance(v, Part):
+                todo += vars(v).values()
+            elif isinstance(v, (list, tuple)):
+                todo += v
+            elif isinstance(v, dict):
+                todo += v.values()
+        return found
+
     def launch_key(self, shape):
         """What this part's launches for a step of single tokens depend on besides the padded
         batch size, worked out from ``shape`` (``n`` sequences with a context, ``max_ctx``,

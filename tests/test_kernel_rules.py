@@ -166,3 +166,36 @@ def test_layers_alike_share_the_plan_of_single_tokens(monkeypatch, n, KV, window
     step.scratch = {}
     parts[1]._decode_plan(step, True)
     assert asked[4:] == [parts[1]]
+
+
+@pytest.mark.parametrize("config", ["llama", "rudorax", "depolix"])
+def test_a_model_that_the_last_level_cache_holds_is_read_through_it(monkeypatch, config):
+    """Every matrix in tiles that the parts of a model hold is found, and all are marked, or none, by what they are worth together."""
+    import kvforge_amd
+    from kvforge_amd.config import presets
+    from kvforge_amd.models.transformer import Transformer
+    cfg = {"llama": lambda: kvforge_amd.preset_dict("tiny-b"),
+           "rudorax": lambda: presets.rudorax_stack(vocab=300, width=64, pairs=1, heads=4, kv_heads=2, dim=16, window=24, lstm_heads=2,
+                                                    lstm_dim=32, lstm_vdim=32, ff=32, experts=4, top=2, identity=1, shared_ff=32,
+                                                    max_positions=512),
+           "depolix": lambda: presets.depolix_stack(vocab=300, width=64, groups=1, heads=4, latent_dim=16, rot_dim=16, q_rank=32,
+                                                    kv_rank=32, att_heads=4, att_kv_heads=2, att_dim=16, window=24, mem_heads=4,
+                                                    mem_kv_heads=2, mem_dim=16, mem_vdim=16, gate_rank=16, ff=64, moe_ff=32,
+                                                    experts=4, top=2, max_positions=512)}[config]()
+    made = []
+
+    def streamed(w):
+        if w is None or w.dtype != torch.bfloat16 or w.dim() != 2:
+            return w
+        made.append(ops.StreamedWeight(w.contiguous()))
+        return made[-1]
+    monkeypatch.setattr(ops, "streamed", streamed)
+    model = Transformer.from_random(cfg, 3, torch.bfloat16, "cpu")
+    held = {t.data_ptr() for p in model.spec.all_parts() for t in p.held_tensors()}
+    assert made and {w.tiles.data_ptr() for w in made} <= held and {w.cached for w in made} == {True}
+    total = sum(w.tiles.nbytes for w in made)
+    for limit, cached in ((total - 1, False), (total, True)):
+        monkeypatch.setattr(ops, "LAST_LEVEL_BYTES", limit)
+        del made[:]
+        model = Transformer.from_random(cfg, 3, torch.bfloat16, "cpu")
+        assert sum(w.tiles.nbytes for w in made) == total and {w.cached for w in made} == {cached}

@@ -393,19 +393,24 @@ def test_gemm_pick_takes_the_lowest_of_equal_columns():
 @pytest.mark.parametrize("m", [1, 8, 16])
 @pytest.mark.parametrize("n,k", [(2048, 1024), (2044, 1024), (1036, 2056), (8192, 2048)])
 def test_streamed_weights_give_the_bits_of_cached_ones(m, n, k):
-    """Matrices in tiles of 4 MB and more go past the caches, smaller and row-major ones do not."""
+    """Matrices in tiles of 4 MB and more go past the caches, smaller and row-major ones do not, and none of a model that lies there
+    as a whole."""
     g = torch.Generator().manual_seed(m + n)
     a, x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV), torch.randn(m, k, generator=g).to(DEV)
     w = (torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV)
     res, outs = torch.randn(m, n, generator=g).to(DEV), []
-    for form in (w, ops().StreamedWeight(w)):
+    for form in (w, ops().StreamedWeight(w), ops().StreamedWeight(w, cached=True)):
         c, half, pairs = res.clone(), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
         ops().gemm(a, form, c, accumulate=True)
         ops().gemm(a, form, half)
         ops().gemm_fused(x, form, pairs, rms_eps=1e-5, silu_pairs=True)
         outs.append((c, half, pairs))
-    for one, other in zip(*outs):
-        assert torch.equal(one.view(torch.uint8), other.view(torch.uint8))
+        if ops().gemm_group_takes(a, form, half):
+            c, half = torch.empty(m, n, device=DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+            ops().gemm_group([(a, form, c, "store"), (a, form, half, "store")])
+            assert torch.equal(half, outs[0][1])
+    for one, *others in zip(*outs):
+        assert all(torch.equal(one.view(torch.uint8), other.view(torch.uint8)) for other in others)
 
 
 @pytest.mark.parametrize("m", [1, 5, 16])
@@ -1752,6 +1757,8 @@ def test_a_token_s_experts_give_the_same_bits_in_every_batch(E, ff, K):
 
     alone = torch.cat([run(i, 1) for i in range(17)])
     assert torch.equal(run(0, 17), alone) and torch.equal(run(1, 16), alone[1:]) and torch.equal(run(0, 5), alone[:5])
+    up.cached = down.cached = True          # (a model that the last-level cache holds)
+    assert torch.equal(run(0, 1), alone[:1]) and torch.equal(run(1, 16), alone[1:])
 
 
 @pytest.mark.parametrize("d", [16, 48, 64, 128, 208])
