@@ -120,10 +120,8 @@ class ParallelBlock(Block):
         """Whether the two norms are RMS norms with fp32 weight vectors and one eps, which one
         kernel then takes together."""
         a, b = self.norm, self.ffn_norm
-        return (b is not None and type(a).forward is type(b).forward
-                and all(isinstance(getattr(n, "weight", None), torch.Tensor) and n.weight.dtype == torch.float32
-                        for n in (a, b))
-                and getattr(a, "eps", None) == getattr(b, "eps", 0.0))
+        return (all(hasattr(n, "fp32_weight") and n.fp32_weight() is not None for n in (a, b))
+                and a.eps == b.eps)
 
     def weight_specs(self) -> dict[str, WeightSpec]:
         out = super().weight_specs()

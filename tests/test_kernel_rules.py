@@ -13,7 +13,8 @@ import torch
 from kvforge_amd.engine.batch import Step, Workspace
 from kvforge_amd.kernels import library, ops
 from kvforge_amd.parts import attention, block
-from kvforge_amd.parts.base import add_product
+from kvforge_amd.parts.base import Norm, add_product
+from kvforge_amd.parts.norm import NamedRMSNorm, RMSNorm
 
 
 @pytest.mark.parametrize("d", range(16, 257, 16))
@@ -199,3 +200,44 @@ def test_a_model_that_the_last_level_cache_holds_is_read_through_it(monkeypatch,
         del made[:]
         model = Transformer.from_random(cfg, 3, torch.bfloat16, "cpu")
         assert sum(w.tiles.nbytes for w in made) == total and {w.cached for w in made} == {cached}
+
+
+class Centred(Norm):
+    """No RMS norm, though it has a weight vector and an eps."""
+
+    def __init__(self, weight):
+        self.weight, self.eps = weight, 1e-5
+
+    def forward(self, x, out, rows=None, add=None):
+        out.copy_(torch.nn.functional.layer_norm(x, x.shape[1:], self.weight, None, self.eps))
+
+
+class Doubled(RMSNorm):
+    def forward(self, x, out, rows=None, add=None, bias=None):
+        out.copy_(2.0 * x)
+
+
+def test_two_norms_of_one_stream_are_one_kernel_only_if_they_are_rms_norms():
+    """Norms of other kinds, two of one kind among them, are each asked for their rows."""
+    g = torch.Generator().manual_seed(1)
+    x, weights = torch.randn(17, 8, generator=g), [torch.randn(8, generator=g) for _ in range(2)]
+    got = []
+    sub = SimpleNamespace(settles_residual=False, state_spec=None, forward=lambda rows, *args: got.append(rows.clone()))
+    ffn = SimpleNamespace(settles_residual=False, forward=lambda rows, *args: got.append(rows.clone()))
+    step = Step()
+    step.ws, step.act_dtype = Workspace("cpu"), torch.float32
+    block.ParallelBlock(Centred(weights[0]), sub, ffn, 8, ffn_norm=Centred(weights[1])).forward(x, step, None)
+    for rows, w in zip(got, weights):
+        assert torch.equal(rows, torch.nn.functional.layer_norm(x, (8,), w, None, 1e-5))
+
+    def rms(cls, eps=1e-5, dtype=torch.float32):
+        norm = cls("n", 8, eps)
+        norm.weight = torch.ones(8, dtype=dtype)
+        return norm
+
+    def together(a, b):
+        return block.ParallelBlock(a, sub, ffn, 8, ffn_norm=b)._norms_pair()
+    assert together(rms(RMSNorm), rms(NamedRMSNorm))
+    for other in (rms(RMSNorm, 1e-6), rms(RMSNorm, dtype=torch.bfloat16), rms(Doubled), Centred(weights[0]), None):
+        assert not together(rms(RMSNorm), other)
+    assert not together(rms(Doubled), rms(Doubled))
