@@ -1,110 +1,213 @@
-// The fused q/k/v projection of many rows: C = A * W^T for bf16 rows and bf16 weights in tiles (see the head of
-// gemm_bf16.hip), fp32 sums, with rotary and the cache write in its epilogue (RopeEpi).
+// Products of many rows: C = A * W^T for bf16 rows and bf16 weights in tiles (see the head of gemm_bf16.hip), fp32 sums.
+// Two kernels over the walk of tile_walk.h: plain and gated products (gemm_tile_kernel), and the fused q/k/v projection with
+// rotary and the cache write in its epilogue (qkv_tile_kernel, RopeEpi).
 //
-// Sums run along K in steps of 32 on one accumulator and are rounded to bf16 before they are rotated, as a stored product is.
-// The library's product, which stood here with rope_kvwrite behind it, does the same at most sizes, to the bit; it cuts K at 14 of
-// 306 that were compared (65 to 77 rows over 3,072 and 3,136 columns, 128 rows over 1,024 and 2,048), where 3 in 100,000 of the
-// result turn a rounding.
-//
-// A workgroup takes a tile of BM rows x BN columns, 64 of K a stage.  Rows and weights go from memory straight
-// into LDS, NB stages side by side, without passing through registers, and are asked for NB - 1.5 stages ahead.  A
-// stage has one barrier, in its middle: before it come the products of the stage's first half, beside which the
-// second half's operands are read from LDS and the last loads of an earlier stage are asked for; behind it
-// those of the second half, beside which the next stage's operands are read (they have arrived by
-// then) and the first loads of the stage that takes the place of the one before are asked for.  Loads stand one by one between products:
-// asked for in one go behind the barrier they block the waves for as long as a product of the
-// stage takes (2,048 x 2,048 x 2,048: 28.5 us on four waves, 19.9 spread out).
-//
-// What bounds it: a stage of 128 x 128 takes 0.5 us where its matrix instructions take 0.21, its loads from L2 0.32 and its
-// reads of LDS 0.16; they overlap in part, and weights from memory add 0.08.  Without
-// the epilogue it is as fast as the library's product, 28.5 us for 2,048 rows of 3,072 x 2,048 (0.9 PFLOP/s); with it 33, where
-// product and rope_kvwrite took 42.
+// Sums run along K in steps of 32 on one accumulator, and are rounded to bf16 before they are rotated or joined, as a stored product
+// is.  The library's product does the same at most sizes, to the bit; it cuts K at some (14 of 306 that were compared, of 65 to 128 rows), where 3 in
+// 100,000 of the result turn a rounding.
 #include <type_traits>
 
-#include "gemm_common.h"
+#include "tile_walk.h"
 
 namespace {
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-
-// 64 lanes x 16 bytes from memory straight into LDS: base + off (per lane) -> lds + 16 * lane.  Written by hand because
-// the compiler, which cannot tell the stages of a buffer apart, waits for every such load before any read of
-// LDS.  The loads have no output register; whoever reads the bytes waits for vmcnt and the barrier first, in loads_left, which
-// says to the compiler that memory has changed: here it would order every read of LDS beside the load behind it.
-__device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0");
-}
-// At most N of the wave's own loads are still on their way, and the other waves have come as far.
-template <int N> __device__ __forceinline__ void loads_left() { asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory"); }
-
 constexpr int MAX_ROT = 128;
 
-template <int WM, int WN, int RT, int CT, int NB>
-__global__ __launch_bounds__(WM * WN * KVF_WAVE, 2) void gemm_tile_kernel(
-    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, bf16_t* __restrict__ q_out, int M, int N, int K, int lda,
-    int ldq, int tm, int tn, RopeEpi rp) {
-  constexpr int WAVES = WM * WN, BM = 16 * RT * WM, BN = 16 * CT * WN;
-  constexpr int AC = BM / 8, WC = BN / 8;             // KB of a stage
-  constexpr int AL = AC / WAVES, WL = WC / WAVES, LOADS = AL + WL;
-  static_assert(AC % WAVES == 0 && WC % WAVES == 0 && NB >= 3, "a wave asks for whole KB of rows and of weights");
-  constexpr uint32_t STAGE = (AC + WC) * 1024;
-  static_assert(NB * STAGE >= BM * (MAX_ROT * 4 + 16), "the angles take the place of the stages");
-  __shared__ __attribute__((aligned(1024))) char lds[NB * STAGE];
-  const int lane = threadIdx.x % KVF_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVF_WAVE);
-  const int r16 = lane % 16, kg = lane / 16;
-  const int total = tm * tn, share = (total + 7) / 8;
-  const int item = static_cast<int>(blockIdx.x % 8) * share + static_cast<int>(blockIdx.x / 8);
-  if (static_cast<int>(blockIdx.x / 8) >= share || item >= total) return;
-  constexpr int GM = 4;
-  const int band = item / (GM * tn), in = item - band * GM * tn, gm = min(GM, tm - band * GM);
-  const int m0 = (band * GM + in % gm) * BM, n0 = in / gm * BN;
-  const int S = K / 64, ksteps = K / 32, groups = (N + 15) / 16;
-  uint32_t aoff[AL], woff[WL];
-  const char* abase = reinterpret_cast<const char*>(A + static_cast<size_t>(m0) * lda);
-  const char* wbase = reinterpret_cast<const char*>(W) + static_cast<size_t>(n0 / 16) * ksteps * 1024;
-  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u32*)lds));
-#pragma unroll
-  for (int i = 0; i < AL; ++i)
-    aoff[i] = static_cast<uint32_t>(min((wave * AL + i) * 8 + lane / 8, M - 1 - m0)) * lda * 2 + ((lane % 8) ^ (lane / 8)) * 16;
-#pragma unroll
-  for (int i = 0; i < WL; ++i) {
-    const int w = wave * WL + i;
-    woff[i] = (static_cast<uint32_t>(min(w / 2, groups - 1 - n0 / 16)) * ksteps + w % 2) * 1024 + lane * 16;
+// How far the tiles of one band of rows go before the next column: tiles that run at the same time share rows and weights in L2.
+constexpr int BAND = 4;
+__device__ __forceinline__ void place_of(int item, int tm, int tn, int& row_tile, int& col_tile) {
+  const int band = item / (BAND * tn), in = item - band * BAND * tn, rows = min(BAND, tm - band * BAND);
+  row_tile = band * BAND + in % rows;
+  col_tile = in / rows;
+}
+
+// What a product's tiles are read from: rows and weights of the tile `item`, then of the one `step` behind it, up to `last`.
+struct Product {
+  const bf16_t* A;
+  const bf16_t* W;
+  int M, N, K, lda, tm, tn, last, step, row_item, weight_item;
+  template <class W_> __device__ __forceinline__ void rows(W_& walk) {
+    int row_tile, col_tile;
+    place_of(row_item, tm, tn, row_tile, col_tile);
+    const int m0 = row_tile * W_::BM;
+    walk.aim_rows(reinterpret_cast<const char*>(A + static_cast<size_t>(m0) * lda),
+                  [&](int r) { return static_cast<uint32_t>(min(r, M - 1 - m0)) * lda * 2; }, K / 32);
+    if (row_item + step < last) row_item += step;
   }
-  auto issue1 = [&](int i, uint32_t buf, int s) {
-    if (i < AL) load_to_lds(abase + static_cast<size_t>(s) * 128, aoff[i < AL ? i : 0], lds0 + buf + (wave * AL + i) * 1024);
-    else load_to_lds(wbase + static_cast<size_t>(s) * 2048, woff[i >= AL ? i - AL : 0], lds0 + buf + (AC + wave * WL + i - AL) * 1024);
+  template <class W_> __device__ __forceinline__ void weights(W_& walk) {
+    int row_tile, col_tile;
+    place_of(weight_item, tm, tn, row_tile, col_tile);
+    const int g0 = col_tile * W_::WC, S = K / 32, groups = (N + 15) / 16;
+    walk.aim_weights(reinterpret_cast<const char*>(W) + static_cast<size_t>(g0) * S * 1024,
+                     [&](int g) { return static_cast<uint32_t>(min(g, groups - 1 - g0)) * S * 1024; }, S);
+    if (weight_item + step < last) weight_item += step;
+  }
+};
+
+// An unbroken eighth of `total` tiles for every XCD (workgroups go to the eight of them in turn): the workgroup's first and
+// the end of its XCD's.
+__device__ __forceinline__ bool share_of(int total, int& first, int& last) {
+  const int share = (total + 7) / 8, begin = static_cast<int>(blockIdx.x % 8) * share;
+  first = begin + static_cast<int>(blockIdx.x / 8);
+  last = min(total, begin + share);
+  return first < last;
+}
+
+// What becomes of a sum: stored as bf16 or fp32, or neighbouring columns are (gate, up) pairs (GateForm, with fp32 biases by
+// pair or null) and their join is stored as bf16; SILU_PAIRS: joined by silu, without biases and scale.
+enum Kind { STORE_BF16 = 0, STORE_F32 = 1, PAIRS = 2, SILU_PAIRS = 3 };
+struct TileEpi {
+  void* out;
+  int ldc;
+  GateForm form;
+  const float* gate_bias;
+  const float* up_bias;
+};
+
+// x / y but for the last bit, seldom: a third of the instructions of a division that also scales its operands against
+// quotients outside the range of fp32.
+__device__ __forceinline__ float ratio(float x, float y) {
+  const float r = __builtin_amdgcn_rcpf(y), q = x * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, y, x), r, q), y, x);
+}
+// a (gate, up) pair joined, without the scale
+template <int ACT> __device__ __forceinline__ float join(const GateForm& f, float g, float u) {
+  if constexpr (ACT == GATE_LIMITED) {
+    g = fminf(g, f.limit);
+    u = fminf(fmaxf(u, -f.limit), f.limit);
+    return ratio(g, 1.f + __expf(-LIMITED_SLOPE * g)) * (u + 1.f);
+  } else if constexpr (ACT == 1) {   // tanh(t) = 1 - 2 / (1 + exp(2 t)); exp overflows to +inf for large t, which gives 1
+    const float t = 0.7978845608028654f * (g + 0.044715f * g * g * g);
+    return 0.5f * g * (2.f - ratio(2.f, 1.f + __expf(2.f * t))) * u;
+  } else {
+    return ratio(g, 1.f + __expf(-g)) * u;
+  }
+}
+// as a stored product is read again
+__device__ __forceinline__ float stored(float v) { return bf16_to_f32(f32_to_bf16(v)); }
+
+// bf16 results leave through the wave's own rows in LDS, as whole pieces of 16 bytes: N, ldc in whole 8s of them.
+template <class T, int KIND> constexpr int own_bytes() {
+  return KIND == STORE_F32 ? 0 : OwnRows<KIND == STORE_BF16 ? 2 * T::CT : T::CT>::BYTES;
+}
+
+// between a wave's writes of its own rows in LDS and its reads of them: a wave's accesses go in order, the compiler's must too
+__device__ __forceinline__ void wave_rows() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Whole rows of bf16: value(r, c, where the lane's four columns go).
+template <class T, int PIECES, class Value>
+__device__ __forceinline__ void store_rows(const T& w, void* out, int ldc, char* own, int m0, int M, int col0, int cols, const Value& value) {
+  using Own = OwnRows<PIECES>;
+#pragma unroll
+  for (int r = 0; r < T::RT; ++r) {
+#pragma unroll
+    for (int c = 0; c < T::CT; ++c) value(r, c);
+    wave_rows();
+    Own::each(own, w.lane, [&](int row, int piece, const uint4& v) {
+      const int m = m0 + (w.wm * T::RT + r) * 16 + row, n = col0 + piece * 8;
+      if (m < M && n < cols) *reinterpret_cast<uint4*>(static_cast<bf16_t*>(out) + static_cast<size_t>(m) * ldc + n) = v;
+    });
+    wave_rows();
+  }
+}
+
+// (a form at a time: with the forms told apart pair by pair the code outgrows the instruction cache)
+template <class T, int ACT, bool BIASED>
+__device__ __forceinline__ void store_pairs(const T& w, const TileEpi& e, char* own, int m0, int n0, int M, int N) {
+  using Own = OwnRows<T::CT>;
+  const int r16 = w.lane % 16, kg = w.lane / 16, cols = N / 2, col0 = (n0 + w.wn * T::CT * 16) / 2;
+  float gb[T::CT][2], ub[T::CT][2];
+  if constexpr (BIASED) {
+#pragma unroll
+    for (int c = 0; c < T::CT; ++c)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int at = min(col0 + c * 8 + 2 * kg + i, cols - 1);
+        gb[c][i] = e.gate_bias ? e.gate_bias[at] : 0.f;
+        ub[c][i] = e.up_bias ? e.up_bias[at] : 0.f;
+      }
+  }
+  store_rows<T, T::CT>(w, e.out, e.ldc, own, m0, M, col0, cols, [&](int r, int c) {
+    const f32x4 a = w.acc[r][c];
+    float y[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      y[i] = BIASED ? join<ACT>(e.form, stored(a[2 * i]) + gb[c][i], stored(a[2 * i + 1]) + ub[c][i]) * e.form.scale
+                    : join<ACT>(e.form, stored(a[2 * i]), stored(a[2 * i + 1]));
+    *reinterpret_cast<uint32_t*>(own + Own::place(r16, c) + kg * 4) = f32_to_bf16(y[0]) | static_cast<uint32_t>(f32_to_bf16(y[1])) << 16;
+  });
+}
+
+template <class T, int KIND>
+__device__ __forceinline__ void store_tile(const T& w, const TileEpi& e, char* own, int m0, int n0, int M, int N) {
+  const int r16 = w.lane % 16, kg = w.lane / 16;
+  if constexpr (KIND == STORE_F32) {
+#pragma unroll
+    for (int r = 0; r < T::RT; ++r)
+#pragma unroll
+      for (int c = 0; c < T::CT; ++c) {
+        const int m = m0 + (w.wm * T::RT + r) * 16 + r16, n = n0 + (w.wn * T::CT + c) * 16 + kg * 4;
+        if (m >= M || n >= N) continue;
+        *reinterpret_cast<f32x4*>(static_cast<float*>(e.out) + static_cast<size_t>(m) * e.ldc + n) = w.acc[r][c];
+      }
+  } else if constexpr (KIND == SILU_PAIRS) {
+    store_pairs<T, 0, false>(w, e, own, m0, n0, M, N);
+  } else if constexpr (KIND == PAIRS) {
+    if (e.form.act == GATE_LIMITED) store_pairs<T, GATE_LIMITED, true>(w, e, own, m0, n0, M, N);
+    else if (e.form.act == 1) store_pairs<T, 1, true>(w, e, own, m0, n0, M, N);
+    else store_pairs<T, 0, true>(w, e, own, m0, n0, M, N);
+  } else {
+    using Own = OwnRows<2 * T::CT>;
+    const int col0 = n0 + w.wn * T::CT * 16;
+    store_rows<T, 2 * T::CT>(w, e.out, e.ldc, own, m0, M, col0, N, [&](int r, int c) {
+      const f32x4 a = w.acc[r][c];
+      *reinterpret_cast<uint2*>(own + Own::place(r16, 2 * c + kg / 2) + (kg % 2) * 8) =
+          make_uint2(f32_to_bf16(a[0]) | static_cast<uint32_t>(f32_to_bf16(a[1])) << 16,
+                     f32_to_bf16(a[2]) | static_cast<uint32_t>(f32_to_bf16(a[3])) << 16);
+    });
+  }
+}
+
+template <class T, int KIND>
+__global__ __launch_bounds__(T::THREADS, 2) void gemm_tile_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int M, int N,
+                                                                  int K, int lda, int tm, int tn, int step, TileEpi e) {
+  constexpr int OWN = own_bytes<T, KIND>();
+  __shared__ __attribute__((aligned(1024))) char lds[T::BYTES + T::WAVES * OWN];
+  int item, last;
+  if (!share_of(tm * tn, item, last)) return;
+  Product src{A, W, M, N, K, lda, tm, tn, last, step, item, item};
+  T walk;
+  walk.template start<false>(lds, K / 32, src);
+  char* own = lds + T::BYTES + walk.wave * OWN;
+  const auto tile = [&](auto is_last, bool first) {
+    walk.template run<T::RT, decltype(is_last)::value>(K / 32, first, src);
+    int row_tile, col_tile;
+    place_of(item, tm, tn, row_tile, col_tile);
+    store_tile<T, KIND>(walk, e, own, row_tile * T::BM, col_tile * T::BN, M, N);
   };
-  const int wm = wave % WM, wn = wave / WM;
-  const int a_at = wm * RT * 2048 + (r16 / 8) * 1024 + (r16 % 8) * 128, x0 = (kg ^ (r16 % 8)) * 16;
-  const int w_at = AC * 1024 + wn * CT * 2048 + lane * 16;
-  f32x4 acc[RT][CT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  struct Frags { bf16x8 a[RT], w[CT]; } f0, f1;
-  constexpr int PR = RT * CT, RD = RT + CT;
-  auto read1 = [&](Frags& f, int i, uint32_t buf, int h) {
-    if (i < CT) f.w[i < CT ? i : 0] = *reinterpret_cast<const bf16x8*>(lds + buf + w_at + i * 2048 + h * 1024);
-    else f.a[i >= CT ? i - CT : 0] = *reinterpret_cast<const bf16x8*>(lds + buf + (a_at + (x0 ^ (h * 64))) + (i - CT) * 2048);
-  };
-  auto half = [&](const Frags& f, Frags& g, uint32_t gbuf, int gh, auto lo, auto hi, uint32_t to, int ts) {
-    constexpr int LO = decltype(lo)::value, HI = decltype(hi)::value;
-    __builtin_amdgcn_sched_barrier(0);
-    int rd = 0, ld = LO;
-#pragma unroll
-    for (int p = 0; p < PR; ++p) {
-#pragma unroll
-      for (; rd < RD && rd < (p + 1) * RD * 2 / PR; ++rd) read1(g, rd, gbuf, gh);
-      __builtin_amdgcn_sched_barrier(0);
-      acc[p / CT][p % CT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[p % CT], f.a[p / CT], acc[p / CT][p % CT], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (; ld < HI && ld - LO < (p + 1) * (HI - LO) / PR; ++ld)
-        if (ts < S) issue1(ld, to, ts);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
+  bool first = true;
+  for (; item + step < last; item += step, first = false) tile(std::false_type{}, first);
+  tile(std::true_type{}, first);
+}
+
+// One tile a workgroup (FEW: see Walk::start).
+template <class T, bool FEW>
+__global__ __launch_bounds__(T::THREADS, 2) void qkv_tile_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                 bf16_t* __restrict__ q_out, int M, int N, int K, int lda, int ldq,
+                                                                 int tm, int tn, RopeEpi rp) {
+  constexpr int BM = T::BM, BN = T::BN, RT = T::RT, CT = T::CT, WM = T::WM, WAVES = T::WAVES;
+  constexpr int ANGLES = BM * (MAX_ROT * 4 + 16);
+  __shared__ __attribute__((aligned(1024))) char lds[T::BYTES > ANGLES ? T::BYTES : ANGLES];
+  int item, last;
+  if (!share_of(tm * tn, item, last)) return;
+  int row_tile, col_tile;
+  place_of(item, tm, tn, row_tile, col_tile);
+  const int m0 = row_tile * BM, n0 = col_tile * BN;
+  T walk;
+  const int lane = threadIdx.x % KVF_WAVE, r16 = lane % 16, kg = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVF_WAVE), wm = wave % WM, wn = wave / WM;
   // What the epilogue needs of a lane's tokens is asked for ahead of the walk over K: position and sequence before the first
   // stages, the page they lead to behind those.
   int pos[RT], page[RT];
@@ -114,38 +217,17 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, 2) void gemm_tile_kernel(
     pos[r] = rp.positions[m];
     page[r] = rp.write_kv ? rp.seq_of_token[m] : -1;   // the sequence for now
   }
-  using Int0 = std::integral_constant<int, 0>;
-  using IntH = std::integral_constant<int, LOADS / 2>;
-  using IntL = std::integral_constant<int, LOADS>;
-#pragma unroll
-  for (int i = 0; i < NB - 2; ++i)
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j)
-      if (i < S) issue1(j, i * STAGE, i);
-#pragma unroll
-  for (int j = 0; j < LOADS / 2; ++j)
-    if (NB - 2 < S) issue1(j, (NB - 2) * STAGE, NB - 2);
+  Product src{A, W, M, N, K, lda, tm, tn, item + 1, 1, item, item};
+  walk.template start<FEW>(lds, K / 32, src);
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     const int blk = pos[r] / rp.block_size;
     const bool has = pos[r] >= 0 && pos[r] < rp.table_len && page[r] >= 0 && page[r] < rp.n_seqs && blk < rp.table_stride;
     page[r] = has ? rp.block_table[static_cast<size_t>(page[r]) * rp.table_stride + blk] : -1;
   }
-  if (NB - 2 < S) loads_left<LOADS * (NB - 3) + LOADS / 2>();
-  else loads_left<0>();
-#pragma unroll
-  for (int i = 0; i < RD; ++i) read1(f0, i, 0, 0);
-  uint32_t cur = 0, last = (NB - 1) * STAGE, fill = (NB - 2) * STAGE;
-#pragma unroll 1
-  for (int s = 0; s < S; ++s) {
-    half(f0, f1, cur, 1, IntH{}, IntL{}, fill, s + NB - 2);
-    if (s + NB - 2 < S) loads_left<LOADS * (NB - 3)>();
-    else loads_left<0>();
-    fill = last;
-    last = cur;
-    cur = cur == (NB - 1) * STAGE ? 0 : cur + STAGE;
-    half(f1, f0, cur, 0, Int0{}, IntH{}, fill, s + NB - 1);
-  }
+  if constexpr (FEW) walk.template run_few<RT>(K / 32);
+  else walk.template run<RT, true>(K / 32, true, src);
+  const auto& acc = walk.acc;
   // The angles of the tile's tokens go through LDS, a cosine and a sine side by side: a lane would read them 4 bytes at
   // a time from 16 rows of the tables otherwise, for every head anew (10 of 42 us at 2,048 x 3,072).
   const int rot8 = rp.rot / 8, pitch = rp.rot * 4 + 16;   // 16 more bytes a row: 16 rows lie on all banks
@@ -201,26 +283,30 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, 2) void gemm_tile_kernel(
   }
 }
 
-// Tiles that are tried, and what one round of them over the chip takes at K = 2,048, and how much of that does not grow with K (us,
-// weights from memory, with rotation and cache write; two of 64 x 64 fit beside each other on a compute unit).  3,072
-// columns: 2,048 rows as 128 x 192 33.9, 1,876 as 192 x 128 30.2, 1,024 as 128 x 128 23.5 and as 64 x 192 24.6, 512 as 64 x 128 18.2
-// and as 64 x 64 19.8, 100 as 64 x 64 16.3.  6,144 columns at K = 4,096: 1,024 rows as 128 x 192 56.9, 512 as 128 x 128 42.0,
-// 200 as 64 x 128 28.7.  The rule takes the least over the rounds that M x N has of each.
+// Tiles that are tried and what they take, in us: once a launch, once a round of them over the chip (weights from memory), and with
+// K, a round at K = 2,048.  Those of plain and gated products were fitted to 244 sizes of 66 to 2,048 rows, 1,024 to
+// 28,672 columns and K of 512 to 14,336: within 8% (64 x 64: 12%) in the mean.
 struct Tile {
   int bm, bn, per_cu;
-  float us, start;
+  float once, round, k2048;
 };
-constexpr Tile TILES[] = {{128, 192, 1, 33.f, 9.f}, {192, 128, 1, 31.f, 5.f}, {128, 128, 1, 24.f, 5.f},
-                          {64, 192, 1, 24.f, 4.f}, {64, 128, 1, 18.5f, 7.f}, {64, 64, 2, 20.f, 4.f}};
+constexpr Tile TILES[] = {{256, 256, 1, -7.1f, 13.3f, 37.3f}, {192, 256, 1, -2.4f, 7.5f, 29.6f}, {128, 256, 1, -1.0f, 5.1f, 23.7f},
+                          {128, 128, 1, 0.9f, 2.6f, 17.1f},   {64, 128, 1, 1.4f, 1.6f, 12.0f},   {192, 128, 1, 0.4f, 3.5f, 20.2f},
+                          {256, 128, 1, -0.8f, 5.0f, 24.4f},  {64, 64, 2, 2.4f, 0.7f, 12.7f}};
+constexpr Tile PLAIN_TILES[] = {{192, 256, 1, -3.6f, 8.7f, 29.0f}, {128, 256, 1, -2.2f, 6.3f, 23.3f}, {128, 128, 1, 0.1f, 3.3f, 16.6f},
+                                {64, 128, 1, 1.2f, 1.9f, 11.9f},   {192, 128, 1, -0.4f, 4.2f, 19.8f}, {256, 128, 1, -1.9f, 6.1f, 23.9f},
+                                {64, 64, 2, 2.4f, 0.8f, 12.6f}};
+constexpr Tile QKV_TILES[] = {{128, 192, 1, 0.f, 9.f, 24.f}, {192, 128, 1, 0.f, 5.f, 26.f},   {128, 128, 1, 0.f, 5.f, 19.f},
+                              {64, 192, 1, 0.f, 4.f, 20.f},  {64, 128, 1, 0.f, 7.f, 11.5f}, {64, 64, 2, 0.f, 4.f, 16.f}};
 
-int best_tile(int M, int N, int K, int cus, float& us) {
+template <int COUNT> int best_tile(const Tile (&tiles)[COUNT], int M, int N, int K, int cus, float& us) {
   int best = 0;
   us = 0.f;
-  for (int i = 0; i < static_cast<int>(sizeof(TILES) / sizeof(TILES[0])); ++i) {
-    const Tile& t = TILES[i];
-    const long tiles = static_cast<long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    const long rounds = (tiles + static_cast<long>(cus) * t.per_cu - 1) / (static_cast<long>(cus) * t.per_cu);
-    const float cost = rounds * (t.start + (t.us - t.start) * K / 2048.f) * (t.per_cu == 2 && tiles <= cus ? 0.82f : 1.f);
+  for (int i = 0; i < COUNT; ++i) {
+    const Tile& t = tiles[i];
+    const long of = static_cast<long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const long at_once = static_cast<long>(cus) * t.per_cu, rounds = (of + at_once - 1) / at_once;
+    const float cost = (t.once + rounds * (t.round + t.k2048 * K / 2048.f)) * (t.per_cu == 2 && of <= cus ? 0.82f : 1.f);
     if (i == 0 || cost < us) {
       best = i;
       us = cost;
@@ -228,26 +314,64 @@ int best_tile(int M, int N, int K, int cus, float& us) {
   }
   return best;
 }
+template <int N> constexpr int count_of(const Tile (&)[N]) { return N; }
 
-template <int WM, int WN, int RT, int CT, int NB>
-int launch(const bf16_t* A, const bf16_t* W, bf16_t* q_out, int M, int N, int K, int lda, int ldq, const RopeEpi& rp, hipStream_t s) {
-  constexpr int BM = 16 * RT * WM, BN = 16 * CT * WN;
-  const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-  hipLaunchKernelGGL((gemm_tile_kernel<WM, WN, RT, CT, NB>), dim3((tm * tn + 7) / 8 * 8), dim3(WM * WN * KVF_WAVE), 0, s, A, W, q_out, M, N, K,
-                     lda, ldq, tm, tn, rp);
-  return kvf_last_error();
+template <class T>
+int launch_qkv(const bf16_t* A, const bf16_t* W, bf16_t* q_out, int M, int N, int K, int lda, int ldq, const RopeEpi& rp, hipStream_t s) {
+  const int tm = (M + T::BM - 1) / T::BM, tn = (N + T::BN - 1) / T::BN;
+  const auto go = [&](auto few) {
+    hipLaunchKernelGGL((qkv_tile_kernel<T, decltype(few)::value>), dim3((tm * tn + 7) / 8 * 8), dim3(T::THREADS), 0, s, A, W, q_out, M, N, K,
+                       lda, ldq, tm, tn, rp);
+    return kvf_last_error();
+  };
+  return K / 32 < T::NW + 2 ? go(std::true_type{}) : go(std::false_type{});
 }
 
-int launch_tile(int tile, const bf16_t* A, const bf16_t* W, bf16_t* q_out, int M, int N, int K, int lda, int ldq, const RopeEpi& rp, hipStream_t s) {
+int launch_qkv_tile(int tile, const bf16_t* A, const bf16_t* W, bf16_t* q_out, int M, int N, int K, int lda, int ldq, const RopeEpi& rp, hipStream_t s) {
   switch (tile) {
-    case 0: return launch<2, 4, 4, 3, 4>(A, W, q_out, M, N, K, lda, ldq, rp, s);
-    case 1: return launch<4, 2, 3, 4, 4>(A, W, q_out, M, N, K, lda, ldq, rp, s);
-    case 2: return launch<2, 4, 4, 2, 4>(A, W, q_out, M, N, K, lda, ldq, rp, s);
-    case 3: return launch<2, 4, 2, 3, 5>(A, W, q_out, M, N, K, lda, ldq, rp, s);
-    case 4: return launch<2, 4, 2, 2, 6>(A, W, q_out, M, N, K, lda, ldq, rp, s);
-    case 5: return launch<2, 2, 2, 2, 4>(A, W, q_out, M, N, K, lda, ldq, rp, s);
+    case 0: return launch_qkv<Walk<2, 4, 4, 3, 4>>(A, W, q_out, M, N, K, lda, ldq, rp, s);
+    case 1: return launch_qkv<Walk<4, 2, 3, 4, 3>>(A, W, q_out, M, N, K, lda, ldq, rp, s);
+    case 2: return launch_qkv<Walk<2, 4, 4, 2, 4>>(A, W, q_out, M, N, K, lda, ldq, rp, s);
+    case 3: return launch_qkv<Walk<2, 4, 2, 3, 4>>(A, W, q_out, M, N, K, lda, ldq, rp, s);
+    case 4: return launch_qkv<Walk<2, 4, 2, 2, 4>>(A, W, q_out, M, N, K, lda, ldq, rp, s);
+    case 5: return launch_qkv<Walk<2, 2, 2, 2, 4>>(A, W, q_out, M, N, K, lda, ldq, rp, s);
   }
   return static_cast<int>(hipErrorInvalidValue);
+}
+
+template <class T, int... KINDS>
+int launch_tiles(int kind, int per_cu, const bf16_t* A, const bf16_t* W, int M, int N, int K, int lda, const TileEpi& e, hipStream_t s) {
+  const int tm = (M + T::BM - 1) / T::BM, tn = (N + T::BN - 1) / T::BN;
+  const int share = (tm * tn + 7) / 8, room = compute_units() / 8 * per_cu, step = share < room ? share : room;
+  int code = static_cast<int>(hipErrorInvalidValue);
+  const auto go = [&](auto k) {
+    if (kind != decltype(k)::value) return;
+    hipLaunchKernelGGL((gemm_tile_kernel<T, decltype(k)::value>), dim3(8 * step), dim3(T::THREADS), 0, s, A, W, M, N, K, lda, tm, tn, step, e);
+    code = kvf_last_error();
+  };
+  (go(std::integral_constant<int, KINDS>{}), ...);
+  return code;
+}
+template <class T>
+int launch_pairs(int kind, int per_cu, const bf16_t* A, const bf16_t* W, int M, int N, int K, int lda, const TileEpi& e, hipStream_t s) {
+  return launch_tiles<T, PAIRS, SILU_PAIRS>(kind, per_cu, A, W, M, N, K, lda, e, s);
+}
+template <class T>
+int launch_plain(int kind, int per_cu, const bf16_t* A, const bf16_t* W, int M, int N, int K, int lda, const TileEpi& e, hipStream_t s) {
+  return launch_tiles<T, STORE_BF16, STORE_F32>(kind, per_cu, A, W, M, N, K, lda, e, s);
+}
+
+int launch_tile(int tile, int kind, const bf16_t* A, const bf16_t* W, int M, int N, int K, int lda, const TileEpi& e, hipStream_t s) {
+  using Launch = int (*)(int, int, const bf16_t*, const bf16_t*, int, int, int, int, const TileEpi&, hipStream_t);
+  static constexpr Launch pairs[] = {launch_pairs<Walk<4, 2, 4, 8, 2>>, launch_pairs<Walk<4, 2, 3, 8, 2>>, launch_pairs<Walk<2, 4, 4, 4, 3>>,
+                                     launch_pairs<Walk<2, 4, 4, 2, 4>>, launch_pairs<Walk<2, 4, 2, 2, 4>>, launch_pairs<Walk<4, 2, 3, 4, 3>>,
+                                     launch_pairs<Walk<4, 2, 4, 4, 3>>, launch_pairs<Walk<2, 2, 2, 2, 4>>};
+  static constexpr Launch plain[] = {launch_plain<Walk<4, 2, 3, 8, 2>>, launch_plain<Walk<2, 4, 4, 4, 3>>, launch_plain<Walk<2, 4, 4, 2, 4>>,
+                                     launch_plain<Walk<2, 4, 2, 2, 4>>, launch_plain<Walk<4, 2, 3, 4, 3>>, launch_plain<Walk<4, 2, 4, 4, 3>>,
+                                     launch_plain<Walk<2, 2, 2, 2, 4>>};
+  static_assert(sizeof(pairs) / sizeof(pairs[0]) == count_of(TILES) && sizeof(plain) / sizeof(plain[0]) == count_of(PLAIN_TILES), "one for each tile");
+  return kind == PAIRS || kind == SILU_PAIRS ? pairs[tile](kind, TILES[tile].per_cu, A, W, M, N, K, lda, e, s)
+                                             : plain[tile](kind, PLAIN_TILES[tile].per_cu, A, W, M, N, K, lda, e, s);
 }
 }  // namespace
 
@@ -261,7 +385,7 @@ KVF_EXPORT int kvf_gemm_tile_qkv_takes(int M, int N, int K, int rot) {
   if (rot < 0 || rot % 8 != 0 || rot > MAX_ROT) return 0;
   if (M <= 0 || N <= 0 || N % 4 != 0 || K <= 0 || K % 64 != 0) return 0;
   float us;
-  best_tile(M, N, K, compute_units(), us);
+  best_tile(QKV_TILES, M, N, K, compute_units(), us);
   const double two = 9.0 + K / 285.0 + 2.0 * N * K / 5.3e6 + 2.0 * M * N * K / 1.5e9 + 4.0 * M * N / 3.5e6;
   return us <= 0.97 * two;
 }
@@ -284,6 +408,44 @@ KVF_EXPORT int kvf_gemm_tile_qkv_rope(const void* A, const void* W, void* q_out,
   const int N = (H + 2 * KV) * d + extra_cols;
   if (N <= 0) return 0;
   float us;
-  if (tile < 0) tile = best_tile(M, N, K, compute_units(), us);
-  return launch_tile(tile, static_cast<const bf16_t*>(A), static_cast<const bf16_t*>(W), static_cast<bf16_t*>(q_out), M, N, K, lda, ldq, rp, s);
+  if (tile < 0) tile = best_tile(QKV_TILES, M, N, K, compute_units(), us);
+  return launch_qkv_tile(tile, static_cast<const bf16_t*>(A), static_cast<const bf16_t*>(W), static_cast<bf16_t*>(q_out), M, N, K, lda, ldq, rp, s);
+}
+
+constexpr int MIN_K = 320;   // ten stages: eight on their way and one pair more
+
+// Whether kvf_gemm_tile takes M rows of [N, K]: where it is expected to be faster than the library's product, and, with `pairs`, a pass over
+// it that joins the pairs.  What those take was fitted to the same 244 sizes (11% in the mean): 5.5 us, 1.34 with 1,000 of
+// K, 8 TB/s over the weights, 1.57 PFLOP/s, 5 TB/s over what is stored; the pass 1 us and 5 TB/s.  Over those sizes gated products take
+// 0.73 of the time of the two (0.71 with the better of both chosen each time; none is slower), plain ones, of which about a half are
+// taken, 0.92 of the library's (0.90).  Both measured, library / this in us.  Gated: 2,048 rows of 16,384 x 2,048 120 / 107, 512
+// 41 / 34, 66 21 / 17; of 4,096 x 2,048 40 / 32; 2,048 of 28,672 x 4,096 378 / 376.  Plain: 2,048 rows of 3,072 x 2,048 30.0 / 29.1, 320 13.1 /
+// 11.6, of 2,048 x 1,024 13.3 / 12.8, of 1,024 x 512 8.8 / 6.8, 66 6.1 / 4.4; of 2,048 x 8,192 73 / 78 and of 6,144 x 4,096 80 / 93: the library's.
+// (Tiles of 256 x 256 are not for plain products: of 22 sizes at which they would be the best, the library is faster at 17.)
+KVF_EXPORT int kvf_gemm_tile_takes(int M, int N, int K, int pairs) {
+  if (M <= 0 || N <= 0 || N % (pairs ? 16 : 8) != 0 || K < MIN_K || K % 64 != 0) return 0;
+  float us;
+  if (pairs) best_tile(TILES, M, N, K, compute_units(), us);
+  else best_tile(PLAIN_TILES, M, N, K, compute_units(), us);
+  const double mn = 1e-6 * M * N, library = 5.5 + 1.34e-3 * K + 0.25e-6 * N * K + 1.28e-3 * mn * K + 0.4 * mn;
+  return us <= 0.95 * (library + (pairs ? 1.0 + 0.6 * mn : 0.0));
+}
+
+// The product of many rows: arguments as kvf_gemm_bf16 with bf16 rows and tiled weights.  kind: what becomes of it (Kind), `form`, limit, scale
+// and the biases (null: none) with PAIRS.  K in whole 64s from MIN_K; N and ldc in whole 8s (PAIRS: N in 16s, ldc counted in pairs),
+// out at 16 bytes.  tile: which of TILES (PAIRS) or PLAIN_TILES, or -1 for the one that the rule takes.
+KVF_EXPORT int kvf_gemm_tile(const void* A, const void* W, void* out, int kind, int M, int N, int K, int lda, int ldc, int form, float limit,
+                             float scale, const float* gate_bias, const float* up_bias, int tile, hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  const bool pairs = kind == PAIRS;
+  if (K < MIN_K || K % 64 != 0 || lda % 8 != 0 || lda < K || lda > (1 << 23) || reinterpret_cast<uintptr_t>(A) % 16 != 0 ||
+      reinterpret_cast<uintptr_t>(W) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0 || kind < STORE_BF16 || kind > PAIRS ||
+      N % (pairs ? 16 : 8) != 0 || ldc % 8 != 0 || ldc < (pairs ? N / 2 : N) || form < 0 || form > GATE_LIMITED ||
+      (form == GATE_LIMITED && !(limit > 0.f)) || tile < -1 || tile >= (pairs ? count_of(TILES) : count_of(PLAIN_TILES)))
+    return static_cast<int>(hipErrorInvalidValue);
+  const TileEpi e{out, ldc, GateForm{form, limit, scale}, gate_bias, up_bias};
+  float us;
+  if (tile < 0) tile = pairs ? best_tile(TILES, M, N, K, compute_units(), us) : best_tile(PLAIN_TILES, M, N, K, compute_units(), us);
+  const bool silu = pairs && form == 0 && scale == 1.f && !gate_bias && !up_bias;
+  return launch_tile(tile, silu ? static_cast<int>(SILU_PAIRS) : kind, static_cast<const bf16_t*>(A), static_cast<const bf16_t*>(W), M, N, K, lda, e, s);
 }

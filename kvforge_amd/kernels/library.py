@@ -38,7 +38,7 @@ ROCM_LIB = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib")
 MODULE_LINK: dict[str, list[str]] = {"gemm_library": [f"-L{ROCM_LIB}", f"-Wl,-rpath,{ROCM_LIB}", "-lhipblaslt"]}
 # Modules of host code alone: CPython modules over torch's C++ types (``load_host``), compiled by the host's compiler.
 HOST_MODULES = ("hostcheck",)
-HEADERS = ["common.h", "gemm_common.h", "sampling_static.h", "memory_chunks.h"]
+HEADERS = ["common.h", "gemm_common.h", "tile_walk.h", "sampling_static.h", "memory_chunks.h"]
 MODULES: dict[str, list[str]] = {
     "elementwise": ["elementwise.hip"],
     "gemm_generic": ["gemm_generic.hip"],

@@ -911,7 +911,7 @@ def bf16_kernel_takes(a: torch.Tensor, w: torch.Tensor, rms: bool = False,
 
 
 def is_library_product(a: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``gemm(a, w, ...)`` hands the product to the library: bf16 with more rows than the
+    """Whether ``gemm(a, w, ...)`` hands the product to the library, or makes it in tiles (``tiles_take``): bf16 with more rows than the
     weight-streaming kernels take; or more than one tile of rows over a deep and narrow weight
     (K >= 2 N), where those kernels have few workgroups and each re-reads every row of ``a`` along
     a long K (measured at [2048, 8192] and 32 rows: 19 us against the library's 15).  ``accumulate=True``
@@ -1070,6 +1070,9 @@ def gemm(a: torch.Tensor, w, out: torch.Tensor, accumulate: bool = False,
             return
         if owed is not None:
             add_rows(out, owed)
+        if not accumulate and tiles_take(a, w, out):
+            gemm_tiles(a, w, out)
+            return
         _library_product(a, plain_of(w), out, accumulate, m, n, k, lda, ldc)
         return
     if owed is not None:
@@ -1115,6 +1118,60 @@ def gemm_gated(a: torch.Tensor, w, out: torch.Tensor, activation: str = "silu",
     _ok(f(a.data_ptr(), 1 if rms else 0, wp, tiled, out.data_ptr(), m, n, k, lda, ldc, float(rms_eps or 0.0),
           act, lim, float(scale), gate_bias.data_ptr() if gate_bias is not None else None,
           up_bias.data_ptr() if up_bias is not None else None, _stream()), "gemm_gated")
+
+
+@lru_cache(maxsize=8192)
+def _tiles_take(m: int, n: int, k: int, pairs: bool, device: int) -> bool:
+    with torch.cuda.device(device):
+        return bool(_fn("gemm_tile", "kvf_gemm_tile_takes", [c_int] * 4)(m, n, k, int(pairs)))
+
+
+def tiles_take(a: torch.Tensor, w, out: torch.Tensor, pairs: bool = False) -> bool:
+    """Whether ``gemm`` (``pairs``: ``gemm_gated_tiles``) is to make ``a @ w.T`` in tiles: more rows than the weight-streaming kernels take,
+    tiled bf16 weights, K in whole steps of 64, whole 16-byte pieces of ``out``'s rows, and a size at which that is faster than the library's product
+    (and the pass behind it that joins the pairs)."""
+    m, k = a.shape
+    return (m > MID_MAX_M and isinstance(w, StreamedWeight) and a.dtype == BF16 and a.is_cuda and k % 64 == 0 and out.dtype in (F32, BF16)
+            and a.stride(1) == 1 and _rows_aligned(a, k, a.stride(0)) and out.stride(1) == 1 and out.stride(0) % 8 == 0
+            and out.data_ptr() % 16 == 0 and a.stride(0) <= 1 << 23 and _tiles_take(m, w.shape[0], k, pairs, a.get_device()))
+
+
+_TILE_ARGS = [c_void_p] * 3 + [c_int] * 7 + [c_float, c_float] + [c_void_p] * 2 + [c_int, c_void_p]
+TILES_PLAIN, TILES_PAIRS = 7, 8          # tiles of rows and columns that there are
+
+
+def gemm_tiles(a: torch.Tensor, w: "StreamedWeight", out: torch.Tensor, tile: int = -1) -> None:
+    """``out = a @ w.T`` for many rows of bf16 over tiled weights, summed along K in order; K in whole 64s from 320.  ``tile``: which of its ``TILES_PLAIN``
+    tiles of rows and columns is taken (-1: by size)."""
+    m, n, k, lda, ldc = _gemm_operands(a, w, out, _whole)
+    if not isinstance(w, StreamedWeight) or a.dtype != BF16 or out.dtype not in (F32, BF16):
+        raise KernelError("gemm_tiles: operands do not fit the kernel")
+    if m == 0:
+        return
+    _ok(_fn("gemm_tile", "kvf_gemm_tile", _TILE_ARGS)(
+        a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), 0 if out.dtype == BF16 else 1, m, n, k, lda, ldc, 0, 0.0, 1.0, None, None, tile,
+        _stream()), "gemm_tiles")
+
+
+def gemm_gated_tiles(a: torch.Tensor, w: "StreamedWeight", out: torch.Tensor, activation: str = "silu",
+                     gate_bias: torch.Tensor | None = None, up_bias: torch.Tensor | None = None, limit: float | None = None,
+                     scale: float = 1.0, tile: int = -1) -> None:
+    """``gemm_gated`` for many rows (callers ask ``tiles_take`` with ``pairs``): the product is rounded to bf16 before it is joined, so this is
+    ``gemm_tiles`` and ``gated_act``, but for the last bit of a few quotients.  K in whole 64s from 320.  ``tile``: which of its ``TILES_PAIRS``
+    tiles."""
+    m, n, k, lda, ldc = _gemm_operands(a, w, out, _halves)
+    if not isinstance(w, StreamedWeight) or a.dtype != BF16 or out.dtype != BF16 or n % 16:
+        raise KernelError("gemm_gated_tiles: operands do not fit the kernel")
+    act, lim = _gate_form(activation, limit, "gemm_gated_tiles")
+    for b, name in ((gate_bias, "gate_bias"), (up_bias, "up_bias")):
+        if b is not None:
+            _check(b, name, F32, (n // 2,))
+    if m == 0:
+        return
+    _ok(_fn("gemm_tile", "kvf_gemm_tile", _TILE_ARGS)(
+        a.data_ptr(), w.tiles.data_ptr(), out.data_ptr(), 2, m, n, k, lda, ldc, act, lim, float(scale),
+        gate_bias.data_ptr() if gate_bias is not None else None, up_bias.data_ptr() if up_bias is not None else None, tile, _stream()),
+        "gemm_gated_tiles")
 
 
 GROUP_MAX = 8            # products of one launch

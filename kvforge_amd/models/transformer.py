@@ -99,6 +99,8 @@ class Transformer:
         mods: set[str] = {"elementwise", "sampling"}
         for p in self.spec.all_parts():
             mods |= p.kernel_modules(self.dtype)
+        if "gemm_bf16" in mods:
+            mods.add("gemm_tile")     # its products of many rows
         return sorted(m for m in mods if m in library.available_modules())
 
     def prepare(self, max_positions: int) -> None:

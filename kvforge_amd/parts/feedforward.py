@@ -79,6 +79,8 @@ class SwiGLU(FeedForward):
         if ops.bf16_kernel_takes(x, self.w_gate_up, rms is not None, True) and self.inter % 2 == 0:
             # one kernel: (norm,) gate/up projection, SwiGLU gate
             ops.gemm_fused(x, self.w_gate_up, act, rms_eps=rms, silu_pairs=True)
+        elif ops.tiles_take(x, self.w_gate_up, act, pairs=True):
+            ops.gemm_gated_tiles(x, self.w_gate_up, act)
         else:
             gu = ws.buf("gate_up", (n, 2 * self.inter), dt)
             ops.gemm(x, self.w_gate_up, gu)
@@ -171,6 +173,9 @@ class GatedFeedForward(SwiGLU):
             # one kernel: gate/up projection, biases, activation, gate
             ops.gemm_gated(x, self.w_gate_up, act, self.activation, self.gate_bias, self.up_bias, limit=self.limit,
                            scale=self.out_scale)
+        elif ops.tiles_take(x, self.w_gate_up, act, pairs=True):
+            ops.gemm_gated_tiles(x, self.w_gate_up, act, self.activation, self.gate_bias, self.up_bias, limit=self.limit,
+                                 scale=self.out_scale)
         else:
             gu = ws.buf("gate_up", (n, 2 * self.inter), dt)
             ops.gemm(x, self.w_gate_up, gu)

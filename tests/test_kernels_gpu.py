@@ -733,6 +733,78 @@ def test_gemm_qkv_rope_tiles_has_the_bits_of_the_three_steps(tile, m, k, H, KV, 
     assert same(q, want) and all(bool((p == 5.0).all()) for p in pages[:2])
 
 
+def _tile_case(m, n, k, seed):
+    """Rows that lie further apart than K, with values that stay in theirs, and a weight, with 64-bit products and the slack of their sums."""
+    g = torch.Generator().manual_seed(seed)
+    wide = torch.randn(m, k + 8, generator=g)
+    wide[3, 5], wide[m - 1, 0] = float("inf"), float("nan")
+    a = wide.to(torch.bfloat16).to(DEV)[:, :k]
+    w = ops().StreamedWeight((torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV))
+    rows = [i for i in range(m) if i not in (3, m - 1)]
+    exact = a[rows].double() @ w.plain.double().T
+    # a sum of k products, each step rounded: k 2^-24 of what the terms have in magnitude
+    slack = k * 2.0 ** -24 * (a[rows].double().abs() @ w.plain.double().abs().T)
+    return a, w, rows, exact, slack
+
+
+# the smallest K that is taken and the next (ten and twelve stages), rows and columns on either side of a tile's end, and several tiles a
+# workgroup (a launch has at most as many workgroups as there are compute units, in eighths)
+TILE_SIZES = [(65, 64, 320), (129, 200, 384), (257, 328, 512), (66, 16 * 1030, 320), (700, 8 * 1200, 448), (2048, 4112, 320)]
+
+
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("m,n,k", TILE_SIZES)
+def test_gemm_tiles(m, n, k, tile):
+    a, w, rows, exact, slack = _tile_case(m, n, k, m + n + k)
+    for dtype, unit in ((torch.float32, 2.0 ** -23), (torch.bfloat16, 2.0 ** -8)):
+        wide = torch.full((m + 1, n + 8), 7.0, dtype=dtype, device=DEV)
+        ops().gemm_tiles(a, w, wide[:m, :n], tile)
+        got = wide[rows][:, :n].double()
+        assert bool(((got - exact).abs() <= unit * exact.abs() + slack).all())
+        assert bool((wide[:, n:] == 7.0).all()) and bool((wide[m] == 7.0).all())
+        assert bool(wide[m - 1, :n].isnan().all()) and not bool(wide[3, :n].isfinite().any())
+
+
+@pytest.mark.parametrize("tile", range(8))
+@pytest.mark.parametrize("form", ["silu", "silu biased", "gelu_tanh", "limited"])
+@pytest.mark.parametrize("m,n,k", [s for s in TILE_SIZES if s[1] % 16 == 0])
+def test_gemm_gated_tiles(m, n, k, form, tile):
+    """Against the product and the pass that joins its pairs: the same but for quotients that differ in their last bit of 24, which turn
+    a rounding to bf16 in some 2^-15 of all cases, to the neighbouring number."""
+    a, w, rows, _, _ = _tile_case(m, n, k, m + n + k + 1)
+    g = torch.Generator().manual_seed(n)
+    activation, limit, scale = form.split()[0], 1.5 if form == "limited" else None, 1.0 if form == "silu" else 0.75
+    gb, ub = (None, None) if form in ("silu", "gelu_tanh") else (torch.randn(n // 2, generator=g).to(DEV) for _ in range(2))
+    product, want = torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_tiles(a, w, product)
+    ops().gated_act(product, want, activation, paired=True, gate_bias=gb, up_bias=ub, limit=limit, scale=scale)
+    wide = torch.full((m + 1, n // 2 + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_gated_tiles(a, w, wide[:m, :n // 2], activation, gb, ub, limit, scale, tile)
+    got = wide[:m, :n // 2].contiguous()
+    assert bool((wide[:, n // 2:] == 7.0).all()) and bool((wide[m] == 7.0).all())
+    assert torch.equal(got.isnan(), want.isnan())
+    off = (got.view(torch.int16).int() - want.view(torch.int16).int()).abs()[~want.isnan()]
+    assert int(off.max()) <= 1 and float((off > 0).double().mean()) < 2.0 ** -12
+
+
+def test_products_of_many_rows_go_in_tiles_where_they_fit():
+    """What the rule takes is made in tiles and what does not fit them is refused there and made by the library."""
+    w = ops().StreamedWeight(torch.zeros(1024, 512, dtype=torch.bfloat16, device=DEV))
+    a, out = torch.zeros(128, 512, dtype=torch.bfloat16, device=DEV), torch.empty(128, 1024, dtype=torch.bfloat16, device=DEV)
+    assert ops().tiles_take(a, w, out) and ops().tiles_take(a, w, out[:, :512], pairs=True)
+    assert not ops().tiles_take(a, w.plain, out) and not ops().tiles_take(a[:64], w, out[:64])
+    wide = torch.empty(128, 1032, dtype=torch.bfloat16, device=DEV)
+    assert not ops().tiles_take(a, w, wide[:, 4:1028]) and ops().tiles_take(a, w, wide[:, 8:])
+    for n, k in ((1020, 512), (1024, 256), (1024, 544)):
+        other = ops().StreamedWeight(torch.zeros(n, k, dtype=torch.bfloat16, device=DEV))
+        rows, into = torch.zeros(128, k, dtype=torch.bfloat16, device=DEV), torch.empty(128, n, dtype=torch.bfloat16, device=DEV)
+        assert not ops().tiles_take(rows, other, into)
+        with pytest.raises(ops().KernelError):
+            ops().gemm_tiles(rows, other, into)
+        ops().gemm(rows, other, into)
+        assert not into.any()
+
+
 @pytest.mark.parametrize("n,k", [(3072, 2048), (6144, 4096), (1024, 512), (2048, 2048)])
 def test_gemm_qkv_rope_tiles_beside_the_library(n, k):
     """Served sizes, rows on both sides of the rule that chooses between them: the library adds most of them up in the same order and
