@@ -1,10 +1,11 @@
 // C[M, N] = A[M, K] * W[N, K]^T with fp32 multiply and fp32 accumulate.
 // This is the matrix product of the true 32-bit path and the fallback for operand types the
 // bf16 MFMA kernels do not take (for instance a weight that the checkpoint stores in fp32 while
-// activations are bf16).  No reduced-precision matrix instruction is used: operands stored in
-// bf16 are widened (exactly) before they are multiplied.
+// activations are bf16).  Operands stored in bf16 are widened (exactly) before they are multiplied.
 //
-// Many rows (a portion of a prompt), rows of K that start on 16 bytes: tiles of 16 to 128 rows x 64
+// Many rows of fp32 by fp32 where there are enough of them: the bf16 matrix cores over operands split without loss
+// (gemm_split_kernel below), whose sums are nearer to 64 bits than those of fp32 instructions.
+// Many rows (a portion of a prompt) otherwise, rows of K that start on 16 bytes: tiles of 16 to 128 rows x 64
 // outputs on the matrix cores with v_mfma_f32_16x16x4_f32, which multiplies and adds in fp32
 // (gemm_mfma32_kernel below).  Many rows otherwise, and kept for comparison: tiles of 64 x 64
 // outputs on the vector ALUs, every output summed
@@ -350,6 +351,166 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma32_kernel(const TA* __restric
   }
 }
 
+// Many rows, both operands fp32: every element is the sum of three bf16 numbers (x = h + m + l, each the rest of the one before rounded to nearest: 24
+// bits but for |x| below 2^-110, whose last bits lie under the least number of the type), and the product is six products of such parts on the
+// bf16 matrix cores, exact each, with fp32 sums: h h in one accumulator, h m, m h, m m, h l and l h in another.  What is
+// left out (m l, l m, l l) is below 2^-25 of a product of two elements, less than the rounding of one fp32 product.
+//
+// Against 64 bits (2-norm; this / the fp32 instruction it takes the place of): normal rows and weights, K 512 1.3e-7 / 2.9e-7, 2,048 2.7e-7 / 5.8e-7,
+// 8,192 5.7e-7 / 1.1e-6, 28,672 1.1e-6 / 2.2e-6; all positive 0.7 of it; rows as they leave a gate, 0.5.
+// A result that is not finite (an element that is none, or more than bf16 can round, makes its row or column NaN here), or so small that its
+// elements' last parts may have been lost, is summed anew in fp32 by its lane.
+//
+// What bounds it: 777 rows of 16,384 x 2,048 take 310 us (fp32 instruction 414), 168 TFLOP/s; the matrix instructions of a stage of 128 x 128 are
+// 1,536 cycles a SIMD, what splits its elements 700, reads and writes of LDS 1,500 at 128 bytes a cycle, in 2,600.  Tried: three buffers
+// and the first operands read a stage ahead 328 us; four waves of 64 x 64 379; 128 x 256 a workgroup 609 (registers spilled); conversions one by one in place of pairs 370.
+//
+// A workgroup of eight waves takes BM = 16 RT WM rows by BN = 16 CT WN columns, 32 of K a stage.  Elements come through registers, two stages
+// ahead, where they are split, into three planes of LDS, double-buffered, with one barrier a stage; splitting, reads, writes and loads stand
+// between the matrix instructions.
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+constexpr int SPLIT_K = 32;
+
+// For the scheduler: PRODUCTS matrix instructions with READS reads of LDS behind the first ones, WRITES writes and LOADS loads behind the last, and
+// the vector instructions that split elements between all of them.
+template <int PRODUCTS, int READS, int WRITES, int LOADS>
+__device__ __forceinline__ void spread_with() {
+#pragma unroll
+  for (int i = 0; i < PRODUCTS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if (i < READS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+    if (i >= PRODUCTS - WRITES - LOADS && i < PRODUCTS - LOADS) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+    if (i >= PRODUCTS - LOADS) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+  }
+}
+// (not inlined: seldom needed, by lanes one by one.  Eight sums side by side round no more than the fp32 instruction's.)
+__device__ __attribute__((noinline)) float plain_dot(const float* a, const float* w, int K) {
+  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < K; k += 8)                     // K is a multiple of 32
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum[i] = fmaf(a[k + i], w[k + i], sum[i]);
+  return ((sum[0] + sum[1]) + (sum[2] + sum[3])) + ((sum[4] + sum[5]) + (sum[6] + sum[7]));
+}
+
+template <int WM, int WN, int RT, int CT, int MODE>
+__global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                                                            int M, int N, int K, int lda, int ldc) {
+  constexpr int TM_ = 16 * RT * WM, TN_ = 16 * CT * WN, ROWS = TM_ + TN_, PLANE = ROWS * 64, BUF = 3 * PLANE;
+  constexpr int PASS = WM * WN * 8;                  // rows that are staged at a time
+  constexpr int Q = ROWS / PASS, AQ = TM_ / PASS;    // 16-byte pieces a thread stages, and how many of them are of A
+  static_assert(TM_ % PASS == 0 && TN_ % PASS == 0, "whole passes");
+  __shared__ __attribute__((aligned(1024))) char lds[2 * BUF];
+  const int down = (M + TM_ - 1) / TM_, total = down * ((N + TN_ - 1) / TN_), share = (total + 7) / 8;
+  const int at = blockIdx.x / 8, item = static_cast<int>(blockIdx.x % 8) * share + at;   // an unbroken eighth for every XCD
+  if (at >= share || item >= total) return;
+  const int tid = threadIdx.x, lane = tid % KVF_WAVE, wave = tid / KVF_WAVE, wm = wave % WM, wn = wave / WM;
+  const int r16 = lane % 16, kg = lane / 16;
+  const int m0 = item % down * TM_, n0 = item / down * TN_;
+  // Piece c (8 elements) of row j of sixteen lies at 4 j + c, c turned over for rows 8..15: no bank conflicts, read or written.
+  auto place = [](int row, int c) { return row / 16 * 1024 + (4 * (row % 16) + (c ^ (row % 16 >= 8 ? 3 : 0))) * 16; };
+  const int srow = tid / 8, sq = tid % 8;            // staged: elements 4 sq .. + 3 of rows srow + PASS i
+  const int put_at = place(srow, sq / 2) + sq % 2 * 8;
+  const float* src[Q];
+#pragma unroll
+  for (int i = 0; i < Q; ++i)
+    src[i] = i < AQ ? A + static_cast<size_t>(min(m0 + srow + PASS * i, M - 1)) * lda + 4 * sq
+                    : W + static_cast<size_t>(min(n0 + srow + PASS * (i - AQ), N - 1)) * K + 4 * sq;
+  struct Staged { float4 v[Q]; };
+  const int stages = K / SPLIT_K;
+  auto fetch = [&](int s, Staged& f) {
+    const int k = min(s, stages - 1) * SPLIT_K;      // past the end the last once more, for nobody
+#pragma unroll
+    for (int i = 0; i < Q; ++i) f.v[i] = *reinterpret_cast<const float4*>(src[i] + k);
+  };
+  auto put = [&](const Staged& f, uint32_t buf) {
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+      f32x2 x[2] = {{f.v[i].x, f.v[i].y}, {f.v[i].z, f.v[i].w}};
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+        uint32_t b[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          b[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x[p], bf16x2));
+          if (part < 2) {
+            x[p][0] -= __uint_as_float(b[p] << 16);
+            x[p][1] -= __uint_as_float(b[p] & 0xffff0000u);
+          }
+        }
+        *reinterpret_cast<uint2*>(lds + buf + part * PLANE + put_at + i * PASS * 64) = make_uint2(b[0], b[1]);
+      }
+    }
+  };
+  const int a_at = place(16 * wm * RT + r16, kg), w_at = place(TM_ + 16 * wn * CT + r16, kg);
+  f32x4 big[RT][CT], small[RT][CT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) big[r][c] = small[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  struct Frags { bf16x8 a[RT], w[CT]; };
+  auto read = [&](uint32_t plane, Frags& f) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) f.w[c] = *reinterpret_cast<const bf16x8*>(lds + plane + w_at + c * 1024);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) f.a[r] = *reinterpret_cast<const bf16x8*>(lds + plane + a_at + r * 1024);
+  };
+  auto product = [&](const Frags& w, const Frags& a, f32x4 (&sum)[RT][CT]) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) sum[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.w[c], a.a[r], sum[r][c], 0, 0, 0);
+  };
+  auto stage = [&](int s, Staged& staged, uint32_t buf) {
+    Frags h, m, l;
+    read(buf, h);
+    read(buf + PLANE, m);
+    read(buf + 2 * PLANE, l);
+    put(staged, BUF - buf);                          // its readers are past the last barrier
+    fetch(s + 3, staged);
+    product(h, h, big);
+    product(m, h, small);
+    product(h, m, small);
+    product(m, m, small);
+    product(l, h, small);
+    product(h, l, small);
+    __builtin_amdgcn_sched_group_barrier(0x100, RT + CT, 0);
+    spread_with<6 * RT * CT, 2 * (RT + CT), 3 * Q, Q>();
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+  };
+  Staged s0, s1;
+  fetch(0, s0);
+  fetch(1, s1);
+  put(s0, 0);
+  fetch(2, s0);
+  __syncthreads();
+  int s = 0;
+#pragma unroll 1
+  for (; s + 1 < stages; s += 2) {
+    stage(s, s1, 0);
+    stage(s + 1, s0, BUF);
+  }
+  if (s < stages) stage(s, s1, 0);
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int m = m0 + 16 * (wm * RT + r) + r16;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int n = n0 + 16 * (wn * CT + c) + 4 * kg;
+      if (m >= M || n >= N) continue;                // N is a multiple of 4
+      f32x4 v = big[r][c] + small[r][c];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!(fabsf(v[e]) <= 3.402823466e38f) || (v[e] != 0.f && fabsf(v[e]) < 0x1p-90f)) v[e] = plain_dot(A + static_cast<size_t>(m) * lda, W + static_cast<size_t>(n + e) * K, K);
+      f32x4* to = reinterpret_cast<f32x4*>(C + static_cast<size_t>(m) * ldc + n);
+      *to = MODE == 1 ? *to + v : v;
+    }
+  }
+}
+
 // MT rows per workgroup (1, 2, 4, 8 or 16); SN columns of W per wave, each read DEPTH steps
 // ahead, so that SN * DEPTH loads of 16 bytes are in flight per lane: narrow outputs (few
 // columns, hence few waves) take one column per wave and look far ahead, wide ones four columns.
@@ -488,6 +649,43 @@ int mfma32_row_tiles(int M, int N) {
   return best;
 }
 
+// Tiles of the split product, and what a round of them over the chip takes at K = 2,048 (us).
+struct SplitTile { int bm, bn; float us; };
+constexpr SplitTile SPLIT_TILES[] = {{128, 128, 73.f}, {128, 64, 46.f}};
+constexpr int SPLIT_COUNT = 2;
+int g_split_tile = -1;        // tests: which of SPLIT_TILES is taken whatever the size; SPLIT_COUNT: none
+// Which of SPLIT_TILES an fp32 product of many rows takes (both give the same bits), or -1: the fp32 instruction, whose tiles are smaller, where there are
+// not tiles of 128 x 64 for three quarters of the compute units, and for short K.  One line in the rows for every weight, so that a row has the
+// same bits among any number of rows on its side of it.  Both measured, us (fp32 / split): 777 rows of 16,384 x 2,048 414 / 310, of 2,048 x 2,048 70 /
+// 55, of 2,048 x 8,192 229 / 182, of 3,072 x 2,048 87 / 77, 2,048 rows of 16,384 x 2,048 1,016 / 655, 300 of them 186 / 143; on the other side 65 of them 50 /
+// 55, 300 rows of 2,048 x 8,192 119 / 173, 777 of 1,536 x 512 19.6 / 20.0.
+constexpr int SPLIT_MIN_K = 512;
+int split_tile(int M, int N, int K) {
+  if (g_split_tile >= 0) return g_split_tile < SPLIT_COUNT ? g_split_tile : -1;
+  const long cus = compute_units();
+  if (K < SPLIT_MIN_K || static_cast<long>(M) * N < cus * (128 * 64 * 3 / 4)) return -1;
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < SPLIT_COUNT; ++i) {
+    const SplitTile& t = SPLIT_TILES[i];
+    const long tiles = static_cast<long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const float cost = (tiles + cus - 1) / cus * t.us;
+    if (i == 0 || cost < least) {
+      best = i;
+      least = cost;
+    }
+  }
+  return best;
+}
+template <int MODE>
+int launch_split(int tile, const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldc, hipStream_t s) {
+  const SplitTile& t = SPLIT_TILES[tile];
+  const dim3 grid(static_cast<unsigned>((static_cast<long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) + 7) / 8 * 8));
+  if (tile == 0) hipLaunchKernelGGL((gemm_split_kernel<2, 4, 4, 2, MODE>), grid, dim3(512), 0, s, A, W, C, M, N, K, lda, ldc);
+  else hipLaunchKernelGGL((gemm_split_kernel<4, 2, 2, 2, MODE>), grid, dim3(512), 0, s, A, W, C, M, N, K, lda, ldc);
+  return kvf_last_error();
+}
+
 template <typename TA, typename TW, typename TO, int MODE>
 int launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldc,
            hipStream_t s) {
@@ -511,6 +709,13 @@ int launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, 
                        static_cast<const TA*>(A), static_cast<const TW*>(W), static_cast<TO*>(C), M,
                        N, K, lda, ldc);
     return kvf_last_error();
+  }
+  if constexpr (std::is_same_v<TA, float> && std::is_same_v<TW, float> && std::is_same_v<TO, float>) {
+    if (quads && K >= SPLIT_K && K % SPLIT_K == 0 && N % 4 == 0 && ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0 && !g_vector_alus_only) {
+      const int tile = split_tile(M, N, K);
+      if (tile >= 0)
+        return launch_split<MODE>(tile, static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N, K, lda, ldc, s);
+    }
   }
   // (its loads need an element of K to be clamped to, and a tile's rows within 32 bits of each other)
   if (quads && K > 0 && K < MFMA32_MAX_ROW && lda < MFMA32_MAX_ROW && !g_vector_alus_only) {
@@ -541,6 +746,14 @@ int launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, 
 KVF_EXPORT int kvf_gemm_generic_vector_alus_only(int on) {
   const int before = g_vector_alus_only;
   g_vector_alus_only = on;
+  return before;
+}
+
+// For tests: which tile of the split product fp32 products of many rows take (0, 1), none (2), or the one that their size asks
+// for (-1).  Returns the setting before.
+KVF_EXPORT int kvf_gemm_generic_split_tile(int tile) {
+  const int before = g_split_tile;
+  g_split_tile = tile;
   return before;
 }
 

@@ -1031,8 +1031,8 @@ def gemm(a: torch.Tensor, w, out: torch.Tensor, accumulate: bool = False,
 
     ``a: [M, K]`` (row stride may exceed K), ``w: [N, K]`` contiguous or a ``StreamedWeight``,
     ``out: [M, N]``.
-    bf16 x bf16 runs on MFMA with fp32 accumulation; any operand in fp32 runs the fp32
-    vector-ALU kernel (true 32-bit multiply and accumulate).
+    bf16 x bf16 runs on MFMA with fp32 accumulation; any operand in fp32 runs the 32-bit kernels (fp32 multiply and accumulate, or, for
+    many rows of fp32, exact products of operands split in three, with fp32 sums: no further from 64 bits).
     With ``accumulate``: ``owed`` (bf16, shape and row stride of ``out``) is a sum still owed to
     ``out`` and is added on the way; ``half_out`` (bf16, likewise, only where ``k_halves_pay``)
     receives the product over the second half of K *instead of* ``out``, which the caller then
@@ -1090,6 +1090,12 @@ def gemm_generic_vector_alus_only(on: bool) -> bool:
     Returns the setting before."""
     f = _fn("gemm_generic", "kvf_gemm_generic_vector_alus_only", [c_int])
     return bool(f(1 if on else 0))
+
+
+def gemm_generic_split_tile(tile: int) -> int:
+    """For tests: which tile 32-bit products of many rows take on split operands (0, 1), that they take the fp32 instruction (2), or what
+    their size asks for (-1).  Returns the setting before."""
+    return int(_fn("gemm_generic", "kvf_gemm_generic_split_tile", [c_int])(tile))
 
 
 def gemm_gated(a: torch.Tensor, w, out: torch.Tensor, activation: str = "silu",

@@ -752,6 +752,46 @@ def _tile_case(m, n, k, seed):
 TILE_SIZES = [(65, 64, 320), (129, 200, 384), (257, 328, 512), (66, 16 * 1030, 320), (700, 8 * 1200, 448), (2048, 4112, 320)]
 
 
+@pytest.mark.parametrize("tile", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(33, 4, 32), (128, 128, 64), (129, 132, 96), (300, 260, 2048), (65, 4100, 8192)])
+def test_fp32_products_of_split_operands(m, n, k, tile):
+    """One to many stages, odd and even, on either side of a tile's end: no further from 64 bits than the fp32 instruction (two roundings
+    apart on the smallest), elementwise within what one rounding a step of 32 and those of the parts allow; stored and added, with rows further apart than K.
+    Values that are not finite, too large for bf16 or tiny are as in plain fp32 sums."""
+    g = torch.Generator().manual_seed(m + n + k)
+    a, w = torch.randn(m, k + 4, generator=g).to(DEV)[:, :k], torch.randn(n, k, generator=g).to(DEV)
+    exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    res = torch.randn(m, n, generator=g).to(DEV)
+
+    def run(how, rows, into=None):
+        wide = torch.full((m + 1, n + 4), 7.0, device=DEV)
+        if into is not None:
+            wide[:m, :n] = into
+        before = ops().gemm_generic_split_tile(how)
+        try:
+            ops().gemm(rows, w, wide[:m, :n], accumulate=into is not None)
+        finally:
+            ops().gemm_generic_split_tile(before)
+        assert bool((wide[:, n:] == 7.0).all()) and bool((wide[m] == 7.0).all())
+        return wide[:m, :n].double()
+
+    got, fp32 = run(tile, a), run(2, a)
+    assert float((got - exact).norm()) <= float((fp32 - exact).norm()) + 2.0 ** -24 * float(exact.norm())
+    assert bool(((got - exact).abs() <= (k / 32 + 8) * 2.0 ** -24 * size).all())
+    added = run(tile, a, res)
+    assert bool(((added - res.double() - exact).abs() <= (k / 32 + 9) * 2.0 ** -24 * (size + res.double().abs())).all())
+    odd = a.clone()
+    odd[1, 3], odd[2, 0], odd[4, 1], odd[5] = float("inf"), float("nan"), 3.4e38, odd[5] * 1e-37
+    got, fp32 = run(tile, odd), run(2, odd)
+    assert torch.equal(got.isnan(), fp32.isnan()) and torch.equal(got.isinf(), fp32.isinf())
+    exact = odd.double() @ w.double().T
+    for row in (4, 5):
+        ok = exact[row].abs() < 3e38
+        # sums of k / 8 terms each there, of k / 8 as well in the fp32 instruction; the parts of 3.4e38 are split like any other
+        off, by = (float((x[row] - exact[row])[ok].norm()) for x in (got, fp32))
+        assert off <= 1.5 * by + 2.0 ** -22 * float(exact[row][ok].norm())
+
+
 @pytest.mark.parametrize("tile", range(7))
 @pytest.mark.parametrize("m,n,k", TILE_SIZES)
 def test_gemm_tiles(m, n, k, tile):
