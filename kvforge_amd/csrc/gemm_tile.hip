@@ -296,8 +296,10 @@ constexpr Tile TILES[] = {{256, 256, 1, -7.1f, 13.3f, 37.3f}, {192, 256, 1, -2.4
 constexpr Tile PLAIN_TILES[] = {{192, 256, 1, -3.6f, 8.7f, 29.0f}, {128, 256, 1, -2.2f, 6.3f, 23.3f}, {128, 128, 1, 0.1f, 3.3f, 16.6f},
                                 {64, 128, 1, 1.2f, 1.9f, 11.9f},   {192, 128, 1, -0.4f, 4.2f, 19.8f}, {256, 128, 1, -1.9f, 6.1f, 23.9f},
                                 {64, 64, 2, 2.4f, 0.8f, 12.6f}};
-constexpr Tile QKV_TILES[] = {{128, 192, 1, 0.f, 9.f, 24.f}, {192, 128, 1, 0.f, 5.f, 26.f},   {128, 128, 1, 0.f, 5.f, 19.f},
-                              {64, 192, 1, 0.f, 4.f, 20.f},  {64, 128, 1, 0.f, 7.f, 11.5f}, {64, 64, 2, 0.f, 4.f, 16.f}};
+// (with rotation and cache write; fitted to 72 sizes of 66 to 2,048 rows, 1,024 to 6,144 columns and K of 512 to 4,096, within 10%: the tile it
+// names takes at most 5% more than the best of the six, 0.2% in the mean)
+constexpr Tile QKV_TILES[] = {{128, 192, 1, -0.2f, 8.4f, 20.5f}, {192, 128, 1, -1.7f, 10.3f, 18.9f}, {128, 128, 1, 0.8f, 6.1f, 15.4f},
+                              {64, 192, 1, 1.1f, 4.6f, 14.7f},   {64, 128, 1, 2.3f, 2.9f, 11.0f},    {64, 64, 2, 5.0f, 0.5f, 11.7f}};
 
 template <int COUNT> int best_tile(const Tile (&tiles)[COUNT], int M, int N, int K, int cus, float& us) {
   int best = 0;
@@ -375,19 +377,19 @@ int launch_tile(int tile, int kind, const bf16_t* A, const bf16_t* W, int M, int
 }
 }  // namespace
 
-// Whether the fused projection takes M rows of [N, K]: where it is expected to be faster than the library's product and
-// rope_kvwrite, which take 9 us, K / 285, 5.3 TB/s over the weights, 1.5 PFLOP/s, and 3.5 TB/s over 4 M N bytes (within 10% of
-// what was measured at five widths and nine row counts).  Both measured, those two / this, at 3,072 x 2,048: 2,048 rows 41.6 / 32.6,
-// 1,024 31.3 / 23.5, 512 23.4 / 18.0, 100 18.4 / 16.2; 1,024 x 512: 2,048 rows 16.2 / 9.4, 66 10.5 / 6.9; 6,144 x 4,096: 1,024 rows 63.3 /
-// 55.6, 333 46.0 / 39.5.  Large ones with a part of a round of tiles left over stay there: 1,500 rows of 6,144 x 4,096 89 / 101,
-// 2,048 of 5,120 x 3,072 77 / 82.
+// Whether the fused projection takes M rows of [N, K]: where it is expected to be faster than a product of its own (the library's, or one in
+// tiles) and rope_kvwrite, which take 9 us, K / 285, 5.3 TB/s over the weights, 1.5 PFLOP/s, and 3.5 TB/s over 4 M N bytes (within 10% of
+// what was measured at six widths and twelve row counts).  Both measured, those two / this, at 3,072 x 2,048: 2,048 rows 39.6 / 32.6,
+// 1,024 30.6 / 21.0, 512 21.6 / 16.2, 100 18.1 / 12.2; 1,024 x 512: 2,048 rows 13.3 / 9.1, 66 8.6 / 6.5; 6,144 x 4,096: 1,024 rows 61.5 /
+// 55.0, 333 44.8 / 37.8.  Large ones with a part of a round of tiles left over stay there: 1,500 rows of 6,144 x 4,096 83 / 97,
+// 2,048 of 5,120 x 3,072 66 / 76.
 KVF_EXPORT int kvf_gemm_tile_qkv_takes(int M, int N, int K, int rot) {
   if (rot < 0 || rot % 8 != 0 || rot > MAX_ROT) return 0;
   if (M <= 0 || N <= 0 || N % 4 != 0 || K <= 0 || K % 64 != 0) return 0;
   float us;
   best_tile(QKV_TILES, M, N, K, compute_units(), us);
-  const double two = 9.0 + K / 285.0 + 2.0 * N * K / 5.3e6 + 2.0 * M * N * K / 1.5e9 + 4.0 * M * N / 3.5e6;
-  return us <= 0.97 * two;
+  const double two = 9.0 + K / 285.0 + 2.0 * N * K / 5.3e6 + 2.0 * M * N * K / 1.75e9 + 4.0 * M * N / 3.5e6;
+  return us <= 0.92 * two;
 }
 
 // Arguments as kvf_gemm_bf16_qkv_rope with bf16 rows and tiled weights; K % 64 == 0.  tile: which of TILES, or
