@@ -366,7 +366,7 @@ def products_of(part: Part, x: torch.Tensor, step: "Step", which: str = "input_p
 def add_product(step: "Step", a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
                 owed: torch.Tensor | None = None) -> None:
     """``residual += a @ w.T``, the last product of a mixer or feed-forward.  With few rows (or in
-    fp32) the product kernel adds in its epilogue.  Many bf16 rows go to the library, whose
+    fp32) the product kernel adds in its epilogue.  Many bf16 rows go to the library or to tiles, whose
     product is left owed to the stream (``step.owe``) so that the next norm adds it on its way
     instead of an add kernel of its own.  One tile of rows over a deep weight with few columns
     is cut into two halves of K so that every compute unit pulls on the weight: the first half

@@ -416,6 +416,13 @@ def test_matrix_memory_passes_at_the_edges_of_their_tiles(dtype, H, dk, dv, n):
     torch.testing.assert_close(state, by_token, atol=3e-4, rtol=3e-4)
 
 
+@pytest.mark.parametrize("dk,n", [(4, 960), (4, 1024), (4, 1025), (4, 1089), (4, 2049), (200, 512), (200, 545)])
+def test_matrix_memory_chunks_in_rounds_of_sixteen(dk, n):
+    """Runs of fifteen, sixteen and more chunks of 64 tokens (32 with keys of 200): the gates' pass takes sixteen at a time, a wave each, and
+    carries the maximum from one to the next."""
+    test_matrix_memory_passes_at_the_edges_of_their_tiles(torch.float32, 2, dk, 17, n)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,dk,dv", [(3, 37, 100), (2, 128, 65), (2, 200, 130), (1, 64, 256)])
 def test_matrix_memory_passes_whatever_the_columns_of_a_workgroup(dtype, H, dk, dv):
