@@ -416,21 +416,44 @@ KVF_EXPORT int kvf_gemm_tile_qkv_rope(const void* A, const void* W, void* q_out,
 
 constexpr int MIN_K = 320;   // ten stages: eight on their way and one pair more
 
+// What the library's product of M rows of [N, K] takes, in us, in two ways.  By its work: 5.5 us, 1.34 with 1,000 of K, 8 TB/s over the weights,
+// 1.57 PFLOP/s, 5 TB/s over what is stored; the pass behind it that joins pairs 1 us and 5 TB/s.
+double library_by_work(int M, int N, int K, bool pairs) {
+  const double mn = 1e-6 * M * N;
+  return 5.5 + 1.34e-3 * K + 0.25e-6 * N * K + 1.28e-3 * mn * K + 0.4 * mn + (pairs ? 1.0 + 0.6 * mn : 0.0);
+}
+// By the rounds of its tiles over the chip, which the first does not see: 2,048 rows of 8,192 x 4,096 are one round of 256 x 256.  Fitted to
+// 1,750 times of 66 to 8,192 rows, 512 to 33,000 columns, K of 320 to 14,336: within 11% in the mean.
+double library_by_rounds(int M, int N, int K, int cus, bool pairs) {
+  constexpr int tiles[][2] = {{256, 256}, {256, 128}, {128, 128}, {64, 64}};
+  const double k = K / 2048.0;
+  double best = 0.0;
+  for (const auto& t : tiles) {
+    const long of = static_cast<long>((M + t[0] - 1) / t[0]) * ((N + t[1] - 1) / t[1]), rounds = (of + cus - 1) / cus;
+    const double area = t[0] * t[1] / 65536.0, us = rounds * (6.4 * area + (40.2 * area + 1.25 * (t[0] + t[1]) / 512.0) * k);
+    if (best == 0.0 || us < best) best = us;
+  }
+  return 8.7 + 1.9 * k + 0.12e-6 * N * K + best + (pairs ? 3.3 + 0.4e-6 * M * N : 0.0);
+}
+
 // Whether kvf_gemm_tile takes M rows of [N, K]: where it is expected to be faster than the library's product, and, with `pairs`, a pass over
-// it that joins the pairs.  What those take was fitted to the same 244 sizes (11% in the mean): 5.5 us, 1.34 with 1,000 of
-// K, 8 TB/s over the weights, 1.57 PFLOP/s, 5 TB/s over what is stored; the pass 1 us and 5 TB/s.  Over those sizes gated products take
-// 0.73 of the time of the two (0.71 with the better of both chosen each time; none is slower), plain ones, of which about a half are
-// taken, 0.92 of the library's (0.90).  Both measured, library / this in us.  Gated: 2,048 rows of 16,384 x 2,048 120 / 107, 512
-// 41 / 34, 66 21 / 17; of 4,096 x 2,048 40 / 32; 2,048 of 28,672 x 4,096 378 / 376.  Plain: 2,048 rows of 3,072 x 2,048 30.0 / 29.1, 320 13.1 /
-// 11.6, of 2,048 x 1,024 13.3 / 12.8, of 1,024 x 512 8.8 / 6.8, 66 6.1 / 4.4; of 2,048 x 8,192 73 / 78 and of 6,144 x 4,096 80 / 93: the library's.
+// it that joins the pairs, by both of the above, and below MOST products of two elements.  Of 1,111 sizes of gated products that were
+// measured it takes 721, in 0.63 of the time of the two, two of them more than 5% slower; of 1,002 of plain ones 470, in 0.71 of the
+// library's, four more than 5% slower.  (By the first alone it took 17 and 57 such, up to 36% slower: plain products of one round of 256 x 256, 2,048 rows
+// of 8,192 x 2,048 52 -> 67 us, and gated ones of large weights, 1,013 rows of 28,672 x 4,096 193 -> 214.)  Both measured, library / this in us.
+// Gated: 2,048 rows of 16,384 x 2,048 120 / 107, 512 41 / 34, 66 21 / 17; of 4,096 x 2,048 40 / 32.  Plain: 2,048 rows of 2,048 x 1,024
+// 13.3 / 12.8, 320 of 3,072 x 2,048 13.1 / 11.6, of 1,024 x 512 8.8 / 6.8, 66 6.1 / 4.4.  The library's: 2,048 rows of 2,048 x 8,192 73 / 78, of
+// 6,144 x 4,096 80 / 93, gated ones of 28,672 x 4,096 377 / 391.
+// Above MOST the two take the same within some percent whichever is faster, and the library's is left alone.
 // (Tiles of 256 x 256 are not for plain products: of 22 sizes at which they would be the best, the library is faster at 17.)
+constexpr double MOST = 1.1e11;
 KVF_EXPORT int kvf_gemm_tile_takes(int M, int N, int K, int pairs) {
-  if (M <= 0 || N <= 0 || N % (pairs ? 16 : 8) != 0 || K < MIN_K || K % 64 != 0) return 0;
+  if (M <= 0 || N <= 0 || N % (pairs ? 16 : 8) != 0 || K < MIN_K || K % 64 != 0 || 1.0 * M * N * K > MOST) return 0;
+  const int cus = compute_units();
   float us;
-  if (pairs) best_tile(TILES, M, N, K, compute_units(), us);
-  else best_tile(PLAIN_TILES, M, N, K, compute_units(), us);
-  const double mn = 1e-6 * M * N, library = 5.5 + 1.34e-3 * K + 0.25e-6 * N * K + 1.28e-3 * mn * K + 0.4 * mn;
-  return us <= 0.95 * (library + (pairs ? 1.0 + 0.6 * mn : 0.0));
+  if (pairs) best_tile(TILES, M, N, K, cus, us);
+  else best_tile(PLAIN_TILES, M, N, K, cus, us);
+  return us <= 0.95 * library_by_work(M, N, K, pairs) && us <= 0.86 * library_by_rounds(M, N, K, cus, pairs);
 }
 
 // The product of many rows: arguments as kvf_gemm_bf16 with bf16 rows and tiled weights.  kind: what becomes of it (Kind), `form`, limit, scale

@@ -45,6 +45,19 @@ def test_routed_experts_change_kernels_where_tiles_of_many_rows_pay(experts, ff,
     assert [many(rows * experts, experts, ff, k) for rows in (2, few, more, 4096)] == [0, 0, 1, 1]
 
 
+@pytest.mark.parametrize("pairs,own,library_s", [
+    # what the library makes in whole rounds of large tiles, whatever K; many rows of large weights; either side of the most that is taken
+    (0, [(2048, 1024, 512), (2048, 2048, 2048), (2048, 4096, 2048), (66, 28672, 4096), (333, 1024, 512), (777, 6144, 1024)],
+     [(2048, 8192, 2048), (2048, 8192, 8192), (1013, 16384, 2048), (1013, 16384, 4096), (2048, 16384, 4096), (430, 28672, 2048), (512, 28672, 4096),
+      (2048, 28672, 4096), (2048, 2048, 8192)]),
+    (1, [(2048, 16384, 2048), (66, 16384, 2048), (2048, 4096, 2048), (100, 28672, 4096), (512, 1024, 512), (1300, 16384, 2048)],
+     [(1771, 28672, 4096), (1013, 28672, 4096), (2048, 28672, 4096), (2048, 8192, 8192), (2048, 6144, 14336), (1300, 28672, 4096)])])
+def test_products_of_many_rows_that_the_library_makes_as_fast_are_left_to_it(pairs, own, library_s):
+    """Sizes that were timed both ways, faster in tiles and not."""
+    takes = ctypes.CDLL(library.build_module("gemm_tile")).kvf_gemm_tile_takes
+    assert [size for size in own if not takes(*size, pairs)] == [] and [size for size in library_s if takes(*size, pairs)] == []
+
+
 @pytest.mark.parametrize("q_lens,H,KV,pairs", [([33], 16, 1, False), ([256, 1], 16, 1, False), ([512], 32, 1, False),
                                                ([513], 32, 1, True), ([200, 200, 200], 32, 8, True), ([64], 8, 8, False)])
 def test_items_of_wide_heads_go_in_pairs_where_they_are_more_than_the_compute_units(monkeypatch, q_lens, H, KV, pairs):
