@@ -353,13 +353,17 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma32_kernel(const TA* __restric
 
 // Many rows, both operands fp32: every element is the sum of three bf16 numbers (x = h + m + l, each the rest of the one before rounded to nearest: 24
 // bits but for |x| below 2^-110, whose last bits lie under the least number of the type), and the product is six products of such parts on the
-// bf16 matrix cores, exact each, with fp32 sums: h h in one accumulator, h m, m h, m m, h l and l h in another.  What is
-// left out (m l, l m, l l) is below 2^-25 of a product of two elements, less than the rounding of one fp32 product.
+// bf16 matrix cores, exact each, with fp32 sums: h h in one accumulator, h m, m h, m m, h l and l h in another (Henry, Tang and Heinecke, "Leveraging
+// the bfloat16 artificial intelligence datatype for higher-precision computations", 2019).  What is left out (m l, l m, l l) is below 2^-24 of a product of
+// two elements, as much as the rounding of one fp32 product at most.
 //
 // Against 64 bits (2-norm; this / the fp32 instruction it takes the place of): normal rows and weights, K 512 1.3e-7 / 2.9e-7, 2,048 2.7e-7 / 5.8e-7,
-// 8,192 5.7e-7 / 1.1e-6, 28,672 1.1e-6 / 2.2e-6; all positive 0.7 of it; rows as they leave a gate, 0.5.
-// A result that is not finite (an element that is none, or more than bf16 can round, makes its row or column NaN here), or so small that its
-// elements' last parts may have been lost, is summed anew in fp32 by its lane.
+// 8,192 5.7e-7 / 1.1e-6, 28,672 1.1e-6 / 2.2e-6; all positive 0.7 of it; rows as they leave a gate, 0.5; all elements 1 + 2^-8 - 2^-17, which leave
+// out the most, 5.9e-8 both.
+// A result is in doubt that is not finite (an element that is none, or more than bf16 can round, makes its row or column NaN here), or so small
+// that its elements' last parts may have been lost.  A wave that holds one walks along K once more with the fp32
+// instruction, and results in doubt take its sums: which they are follows from their own row and column alone.  777 rows of 16,384 x 2,048 360 us, 510
+// with one NaN, 960 all NaN (790 and 17,900 where lanes summed theirs one by one); of 2,048 x 8,192 200, 500 and 630.
 //
 // What bounds it: 777 rows of 16,384 x 2,048 take 310 us (fp32 instruction 414), 168 TFLOP/s; the matrix instructions of a stage of 128 x 128 are
 // 1,536 cycles a SIMD, what splits its elements 700, reads and writes of LDS 1,500 at 128 bytes a cycle, in 2,600.  Tried: three buffers
@@ -386,15 +390,6 @@ __device__ __forceinline__ void spread_with() {
     if (i >= PRODUCTS - LOADS) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
   }
 }
-// (not inlined: seldom needed, by lanes one by one.  Eight sums side by side round no more than the fp32 instruction's.)
-__device__ __attribute__((noinline)) float plain_dot(const float* a, const float* w, int K) {
-  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < K; k += 8)                     // K is a multiple of 32
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sum[i] = fmaf(a[k + i], w[k + i], sum[i]);
-  return ((sum[0] + sum[1]) + (sum[2] + sum[3])) + ((sum[4] + sum[5]) + (sum[6] + sum[7]));
-}
-
 template <int WM, int WN, int RT, int CT, int MODE>
 __global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
                                                             int M, int N, int K, int lda, int ldc) {
@@ -444,7 +439,7 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_ke
       }
     }
   };
-  const int a_at = place(16 * wm * RT + r16, kg), w_at = place(TM_ + 16 * wn * CT + r16, kg);
+  const int a_in = place(16 * wm * RT + r16, kg), w_in = place(TM_ + 16 * wn * CT + r16, kg);
   f32x4 big[RT][CT], small[RT][CT];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
@@ -453,9 +448,9 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_ke
   struct Frags { bf16x8 a[RT], w[CT]; };
   auto read = [&](uint32_t plane, Frags& f) {
 #pragma unroll
-    for (int c = 0; c < CT; ++c) f.w[c] = *reinterpret_cast<const bf16x8*>(lds + plane + w_at + c * 1024);
+    for (int c = 0; c < CT; ++c) f.w[c] = *reinterpret_cast<const bf16x8*>(lds + plane + w_in + c * 1024);
 #pragma unroll
-    for (int r = 0; r < RT; ++r) f.a[r] = *reinterpret_cast<const bf16x8*>(lds + plane + a_at + r * 1024);
+    for (int r = 0; r < RT; ++r) f.a[r] = *reinterpret_cast<const bf16x8*>(lds + plane + a_in + r * 1024);
   };
   auto product = [&](const Frags& w, const Frags& a, f32x4 (&sum)[RT][CT]) {
 #pragma unroll
@@ -494,6 +489,60 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_ke
     stage(s + 1, s0, BUF);
   }
   if (s < stages) stage(s, s1, 0);
+  uint32_t doubt = 0;
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      big[r][c] += small[r][c];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = fabsf(big[r][c][e]);
+        doubt |= static_cast<uint32_t>(!(v <= 3.402823466e38f) || (v != 0.f && v < 0x1p-90f)) << ((r * CT + c) * 4 + e);
+      }
+    }
+  }
+  if (__any(doubt != 0)) {
+    // as gemm_mfma32_kernel sums, to the bit, with operands straight from memory
+    const float *a_at[RT], *w_at[CT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) a_at[r] = A + static_cast<size_t>(min(m0 + 16 * (wm * RT + r) + r16, M - 1)) * lda + 4 * kg;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) w_at[c] = W + static_cast<size_t>(min(n0 + 16 * (wn * CT + c) + r16, N - 1)) * K + 4 * kg;
+    f32x4 sum[2][RT][CT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) sum[0][r][c] = sum[1][r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int k = 0; k < K; k += XK) {
+      f32x4 a[2][RT], w[2][CT];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) a[u][r] = *reinterpret_cast<const f32x4*>(a_at[r] + k + 16 * u);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) w[u][c] = *reinterpret_cast<const f32x4*>(w_at[c] + k + 16 * u);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) sum[u][r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][c][e], a[u][r][e], sum[u][r][c], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        const f32x4 v = sum[0][r][c] + sum[1][r][c];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (doubt >> ((r * CT + c) * 4 + e) & 1) big[r][c][e] = v[e];
+      }
+  }
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     const int m = m0 + 16 * (wm * RT + r) + r16;
@@ -501,12 +550,8 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_ke
     for (int c = 0; c < CT; ++c) {
       const int n = n0 + 16 * (wn * CT + c) + 4 * kg;
       if (m >= M || n >= N) continue;                // N is a multiple of 4
-      f32x4 v = big[r][c] + small[r][c];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (!(fabsf(v[e]) <= 3.402823466e38f) || (v[e] != 0.f && fabsf(v[e]) < 0x1p-90f)) v[e] = plain_dot(A + static_cast<size_t>(m) * lda, W + static_cast<size_t>(n + e) * K, K);
       f32x4* to = reinterpret_cast<f32x4*>(C + static_cast<size_t>(m) * ldc + n);
-      *to = MODE == 1 ? *to + v : v;
+      *to = MODE == 1 ? *to + big[r][c] : big[r][c];
     }
   }
 }

@@ -792,6 +792,35 @@ def test_fp32_products_of_split_operands(m, n, k, tile):
         assert off <= 1.5 * by + 2.0 ** -22 * float(exact[row][ok].norm())
 
 
+def _fp32_product(how, a, w):
+    """``a @ w.T`` by one of the tiles of split operands (0, 1) or by the fp32 instruction (2)."""
+    out, before = torch.full((a.shape[0], w.shape[0]), 7.0, device=DEV), ops().gemm_generic_split_tile(how)
+    try:
+        ops().gemm(a, w, out)
+    finally:
+        ops().gemm_generic_split_tile(before)
+    return out
+
+
+@pytest.mark.parametrize("tile", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(33, 36, 32), (300, 260, 480)])
+def test_fp32_results_in_doubt_have_the_bits_of_the_fp32_instruction(m, n, k, tile):
+    """Rows and columns that are not finite or tiny, stored and added; the others keep theirs."""
+    g = torch.Generator().manual_seed(m)
+    a, w = torch.randn(m, k, generator=g).to(DEV), torch.randn(n, k, generator=g).to(DEV)
+    odd, odd_w = a.clone(), w.clone()
+    odd[1, 3], odd[2, 0], odd[17], odd[m - 1] = float("inf"), float("nan"), odd[17] * 1e-37, -0.0
+    odd_w[3, k - 1], odd_w[n - 1], odd_w[5] = -float("inf"), odd_w[n - 1] * 1e-36, 0.0
+    got, fp32, plain_ = _fp32_product(tile, odd, odd_w), _fp32_product(2, odd, odd_w), _fp32_product(tile, a, w)
+
+    def bits(x):
+        return torch.where(x.isnan(), torch.full_like(x, float("nan")), x).view(torch.int32)
+    rows, columns = [1, 2, 17, m - 1], [3, 5, n - 1]
+    assert torch.equal(bits(got[rows]), bits(fp32[rows])) and torch.equal(bits(got[:, columns]), bits(fp32[:, columns]))
+    got[rows], plain_[rows], got[:, columns], plain_[:, columns] = 0.0, 0.0, 0.0, 0.0
+    assert torch.equal(got, plain_) and not torch.equal(got, _fp32_product(2, a, w))
+
+
 @pytest.mark.parametrize("tile", range(7))
 @pytest.mark.parametrize("m,n,k", TILE_SIZES)
 def test_gemm_tiles(m, n, k, tile):
