@@ -360,8 +360,8 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma32_kernel(const TA* __restric
 // Against 64 bits (2-norm; this / the fp32 instruction it takes the place of): normal rows and weights, K 512 1.3e-7 / 2.9e-7, 2,048 2.7e-7 / 5.8e-7,
 // 8,192 5.7e-7 / 1.1e-6, 28,672 1.1e-6 / 2.2e-6; all positive 0.7 of it; rows as they leave a gate, 0.5; all elements 1 + 2^-8 - 2^-17, which leave
 // out the most, 5.9e-8 both.
-// A result is in doubt that is not finite (an element that is none, or more than bf16 can round, makes its row or column NaN here), or so small
-// that its elements' last parts may have been lost.  A wave that holds one walks along K once more with the fp32
+// A result is in doubt that is not finite (an element that is none, or more than bf16 can round, makes its row or column NaN here), or that the
+// last parts of elements below 2^-110 might change, by the largest elements of its row and column.  A wave that holds one walks along K once more with the fp32
 // instruction, and results in doubt take its sums: which they are follows from their own row and column alone.  777 rows of 16,384 x 2,048 360 us, 510
 // with one NaN, 960 all NaN (790 and 17,900 where lanes summed theirs one by one); of 2,048 x 8,192 200, 500 and 630.
 //
@@ -390,8 +390,9 @@ __device__ __forceinline__ void spread_with() {
     if (i >= PRODUCTS - LOADS) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
   }
 }
+// (two workgroups of the smaller tile share a compute unit: 300 rows of 16,384 x 2,048 149 us, 174 with one)
 template <int WM, int WN, int RT, int CT, int MODE>
-__global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+__global__ __launch_bounds__(WM * WN * KVF_WAVE, RT * CT > 4 ? WM * WN / 4 : WM * WN / 2) void gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
                                                             int M, int N, int K, int lda, int ldc) {
   constexpr int TM_ = 16 * RT * WM, TN_ = 16 * CT * WN, ROWS = TM_ + TN_, PLANE = ROWS * 64, BUF = 3 * PLANE;
   constexpr int PASS = WM * WN * 8;                  // rows that are staged at a time
@@ -420,9 +421,14 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_ke
 #pragma unroll
     for (int i = 0; i < Q; ++i) f.v[i] = *reinterpret_cast<const float4*>(src[i] + k);
   };
+  float top[Q], top2[Q];                             // of the thread's elements of each row, the largest magnitude; in two chains: one is 1 to 5% slower
+#pragma unroll
+  for (int i = 0; i < Q; ++i) top[i] = top2[i] = 0.f;
   auto put = [&](const Staged& f, uint32_t buf) {
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
+      top[i] = fmaxf(fmaxf(top[i], fabsf(f.v[i].x)), fabsf(f.v[i].y));
+      top2[i] = fmaxf(fmaxf(top2[i], fabsf(f.v[i].z)), fabsf(f.v[i].w));
       f32x2 x[2] = {{f.v[i].x, f.v[i].y}, {f.v[i].z, f.v[i].w}};
 #pragma unroll
       for (int part = 0; part < 3; ++part) {
@@ -489,20 +495,54 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, WM * WN / 4) void gemm_split_ke
     stage(s + 1, s0, BUF);
   }
   if (s < stages) stage(s, s1, 0);
-  uint32_t doubt = 0;
+  float* tops = reinterpret_cast<float*>(lds);       // nobody reads a stage any more
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    top[i] = fmaxf(top[i], top2[i]);
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) top[i] = fmaxf(top[i], __shfl_xor(top[i], o, KVF_WAVE));
+    if (sq == 0) tops[srow + PASS * i] = top[i];
+  }
+  __syncthreads();
+  // What the parts cannot hold of an element is less than 3 * 2^-126, and so is what a product of parts loses: results below 2^24 of the sum of
+  // these are in doubt.  (A row or column of zeros loses nothing.)
+  const float least = 0x1p-100f * K;
+  f32x4 col[CT];
+  float row[RT], most = 1.f, lowest = INFINITY, all = 0.f;
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    col[c] = *reinterpret_cast<const f32x4*>(tops + TM_ + 16 * (wn * CT + c) + 4 * kg);
+    most = fmaxf(fmaxf(fmaxf(most, col[c][0]), col[c][1]), fmaxf(col[c][2], col[c][3]));
+  }
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
+    row[r] = tops[16 * (wm * RT + r) + r16];
+    most = fmaxf(most, row[r]);
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
       big[r][c] += small[r][c];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float v = fabsf(big[r][c][e]);
-        doubt |= static_cast<uint32_t>(!(v <= 3.402823466e38f) || (v != 0.f && v < 0x1p-90f)) << ((r * CT + c) * 4 + e);
+        all += fabsf(big[r][c][e]);
+        lowest = fminf(lowest, fabsf(big[r][c][e]));
       }
     }
   }
-  if (__any(doubt != 0)) {
+  // (a launch fetches its code anew: what is seldom needed stands apart, and what asks for it is short; a prompt of 777 rows 11,740 us, 12,020 where
+  // every lane tested its 32 results one by one)
+  uint32_t doubt = 0;
+  if (__builtin_expect(__any(!(lowest >= 3.f * least * most && all <= 3.402823466e38f)), 0)) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = fabsf(big[r][c][e]), lost = row[r] > 0.f && col[c][e] > 0.f ? least * (row[r] + col[c][e] + 1.f) : 0.f;
+          doubt |= static_cast<uint32_t>(!(v <= 3.402823466e38f) || v < lost) << ((r * CT + c) * 4 + e);
+        }
+  }
+  if (__builtin_expect(__any(doubt != 0), 0)) {
     // as gemm_mfma32_kernel sums, to the bit, with operands straight from memory
     const float *a_at[RT], *w_at[CT];
 #pragma unroll

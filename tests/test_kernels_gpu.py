@@ -821,6 +821,21 @@ def test_fp32_results_in_doubt_have_the_bits_of_the_fp32_instruction(m, n, k, ti
     assert torch.equal(got, plain_) and not torch.equal(got, _fp32_product(2, a, w))
 
 
+@pytest.mark.parametrize("tile", [0, 1])
+@pytest.mark.parametrize("small", [-100, -105, -110, -116, -122, -126, -140])
+@pytest.mark.parametrize("small_rows", [True, False])
+def test_fp32_products_of_small_by_large_operands(small_rows, small, tile):
+    """Elements whose last parts lie below the least bf16 number, against large ones: no result is small for that, and none is further from 64 bits
+    than the fp32 instruction's, whose bits those in doubt have (two roundings apart on the others)."""
+    g = torch.Generator().manual_seed(small)
+    x, y = (torch.randn(130, 512, generator=g).to(DEV).double() for _ in range(2))
+    x, y = (x * 2.0 ** small).float(), (y * 2.0 ** 60).float()
+    a, w = (x, y[:100]) if small_rows else (y, x[:100])
+    exact = a.double() @ w.double().T
+    got, fp32 = _fp32_product(tile, a, w).double(), _fp32_product(2, a, w).double()
+    assert float((got - exact).norm()) <= float((fp32 - exact).norm()) + 2.0 ** -24 * float(exact.norm())
+
+
 @pytest.mark.parametrize("tile", range(7))
 @pytest.mark.parametrize("m,n,k", TILE_SIZES)
 def test_gemm_tiles(m, n, k, tile):
