@@ -1162,8 +1162,8 @@ def gemm_tiles(a: torch.Tensor, w: "StreamedWeight", out: torch.Tensor, tile: in
 def gemm_gated_tiles(a: torch.Tensor, w: "StreamedWeight", out: torch.Tensor, activation: str = "silu",
                      gate_bias: torch.Tensor | None = None, up_bias: torch.Tensor | None = None, limit: float | None = None,
                      scale: float = 1.0, tile: int = -1) -> None:
-    """``gemm_gated`` for many rows (callers ask ``tiles_take`` with ``pairs``): the product is rounded to bf16 before it is joined, so this is
-    ``gemm_tiles`` and ``gated_act``, but for the last bit of a few quotients.  K in whole 64s from 320.  ``tile``: which of its ``TILES_PAIRS``
+    """``gemm_gated`` for many rows (callers ask ``tiles_take`` with ``pairs``): the product is rounded to bf16 before it is joined, so this has
+    the bits of ``gemm_tiles`` and ``gated_act``.  K in whole 64s from 320.  ``tile``: which of its ``TILES_PAIRS``
     tiles."""
     m, n, k, lda, ldc = _gemm_operands(a, w, out, _halves)
     if not isinstance(w, StreamedWeight) or a.dtype != BF16 or out.dtype != BF16 or n % 16:
