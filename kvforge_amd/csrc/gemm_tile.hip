@@ -289,10 +289,12 @@ constexpr Tile TILES[] = {{256, 256, 1, -7.1f, 13.3f, 37.3f}, {192, 256, 1, -2.4
 constexpr Tile PLAIN_TILES[] = {{192, 256, 1, -3.6f, 8.7f, 29.0f}, {128, 256, 1, -2.2f, 6.3f, 23.3f}, {128, 128, 1, 0.1f, 3.3f, 16.6f},
                                 {64, 128, 1, 1.2f, 1.9f, 11.9f},   {192, 128, 1, -0.4f, 4.2f, 19.8f}, {256, 128, 1, -1.9f, 6.1f, 23.9f},
                                 {64, 64, 2, 2.4f, 0.8f, 12.6f}};
-// (with rotation and cache write; fitted to 72 sizes of 66 to 2,048 rows, 1,024 to 6,144 columns and K of 512 to 4,096, within 10%: the tile it
-// names takes at most 5% more than the best of the six, 0.2% in the mean)
+// (with rotation and cache write; fitted to 72 sizes of 66 to 2,048 rows, 1,024 to 6,144 columns and K of 512 to 4,096, the two smallest anew with 231 of
+// 65 to 2,100 rows, 192 to 10,240 columns and K from 64: over those the tile it names takes at most 3% more than the best of the six, 0.05% in the mean.
+// With a round of 64 x 64 at 0.5 us as the larger K asked for, many rounds of short ones took that tile: 1,434 rows of 4,096 x 192 18.5 us,
+// 13.2 in tiles of 192 x 128, 1,705 of 6,144 x 512 37.5 and 27.9)
 constexpr Tile QKV_TILES[] = {{128, 192, 1, -0.2f, 8.4f, 20.5f}, {192, 128, 1, -1.7f, 10.3f, 18.9f}, {128, 128, 1, 0.8f, 6.1f, 15.4f},
-                              {64, 192, 1, 1.1f, 4.6f, 14.7f},   {64, 128, 1, 2.3f, 2.9f, 11.0f},    {64, 64, 2, 5.0f, 0.5f, 11.7f}};
+                              {64, 192, 1, 1.1f, 4.6f, 14.7f},   {64, 128, 1, 1.7f, 2.9f, 11.0f},    {64, 64, 2, 3.0f, 2.5f, 11.7f}};
 
 template <int COUNT> int best_tile(const Tile (&tiles)[COUNT], int M, int N, int K, int cus, float& us) {
   int best = 0;
@@ -371,7 +373,7 @@ int launch_tile(int tile, int kind, const bf16_t* A, const bf16_t* W, int M, int
 }  // namespace
 
 // Whether the fused projection takes M rows of [N, K]: where it is expected to be faster than a product of its own (the library's, or one in
-// tiles) and rope_kvwrite, which take 9 us, K / 285, 5.3 TB/s over the weights, 1.5 PFLOP/s, and 3.5 TB/s over 4 M N bytes (within 10% of
+// tiles) and rope_kvwrite, which take 9 us, K / 285, 5.3 TB/s over the weights, 1.75 PFLOP/s, and 3.5 TB/s over 4 M N bytes (within 10% of
 // what was measured at six widths and twelve row counts).  Both measured, those two / this, at 3,072 x 2,048: 2,048 rows 39.6 / 32.6,
 // 1,024 30.6 / 21.0, 512 21.6 / 16.2, 100 18.1 / 12.2; 1,024 x 512: 2,048 rows 13.3 / 9.1, 66 8.6 / 6.5; 6,144 x 4,096: 1,024 rows 61.5 /
 // 55.0, 333 44.8 / 37.8.  Large ones with a part of a round of tiles left over stay there: 1,500 rows of 6,144 x 4,096 83 / 97,
@@ -382,11 +384,17 @@ KVF_EXPORT int kvf_gemm_tile_qkv_takes(int M, int N, int K, int rot) {
   float us;
   best_tile(QKV_TILES, M, N, K, compute_units(), us);
   const double two = 9.0 + K / 285.0 + 2.0 * N * K / 5.3e6 + 2.0 * M * N * K / 1.75e9 + 4.0 * M * N / 3.5e6;
-  return us <= 0.92 * two;
+  return K <= 512 || us <= 0.92 * two;   // (short K: what the two store and read again is most of it, 2,091 rows of 8,192 x 256 50 / 35)
 }
 
-// Arguments as kvf_gemm_bf16_qkv_rope with bf16 rows and tiled weights; K % 64 == 0.  tile: which of TILES, or
-// -1 for the one that the rule takes.
+// Which of QKV_TILES M rows of [N, K] take.
+KVF_EXPORT int kvf_gemm_tile_qkv_tile(int M, int N, int K) {
+  float us;
+  return best_tile(QKV_TILES, M, N, K, compute_units(), us);
+}
+
+// Arguments as kvf_gemm_bf16_qkv_rope with bf16 rows and tiled weights; K % 64 == 0.  tile: which of QKV_TILES,
+// or -1 for the one that the rule takes.
 KVF_EXPORT int kvf_gemm_tile_qkv_rope(const void* A, const void* W, void* q_out, int M, int K, int lda, int ldq, const int* positions,
                                       const int* seq_of_token, const float* cos_t, const float* sin_t, const int* block_table,
                                       void* k_pages, void* v_pages, int H, int KV, int d, int rot, int table_len, int block_size,

@@ -58,6 +58,13 @@ def test_products_of_many_rows_that_the_library_makes_as_fast_are_left_to_it(pai
     assert [size for size in own if not takes(*size, pairs)] == [] and [size for size in library_s if takes(*size, pairs)] == []
 
 
+@pytest.mark.parametrize("m,n,k,best", [(1434, 4096, 192, 1), (893, 6144, 128, 0), (1518, 3072, 64, 0), (1705, 6144, 512, 0), (1638, 5120, 256, 3),
+                                        (2072, 1536, 64, 2), (343, 1536, 64, 5), (423, 5120, 128, 3)])
+def test_tiles_of_the_fused_projection_where_k_is_short(m, n, k, best):
+    """The tile that was timed the fastest of the six is taken."""
+    assert ctypes.CDLL(library.build_module("gemm_tile")).kvf_gemm_tile_qkv_tile(m, n, k) == best
+
+
 @pytest.mark.parametrize("q_lens,H,KV,pairs", [([33], 16, 1, False), ([256, 1], 16, 1, False), ([512], 32, 1, False),
                                                ([513], 32, 1, True), ([200, 200, 200], 32, 8, True), ([64], 8, 8, False)])
 def test_items_of_wide_heads_go_in_pairs_where_they_are_more_than_the_compute_units(monkeypatch, q_lens, H, KV, pairs):
