@@ -739,16 +739,18 @@ struct SplitTile { int bm, bn; float us; };
 constexpr SplitTile SPLIT_TILES[] = {{128, 128, 73.f}, {128, 64, 46.f}};
 constexpr int SPLIT_COUNT = 2;
 int g_split_tile = -1;        // tests: which of SPLIT_TILES is taken whatever the size; SPLIT_COUNT: none
-// Which of SPLIT_TILES an fp32 product of many rows takes (both give the same bits), or -1: the fp32 instruction, whose tiles are smaller, where there are
-// not tiles of 128 x 64 for three quarters of the compute units, and for short K.  One line in the rows for every weight, so that a row has the
+// Which of SPLIT_TILES an fp32 product of many rows takes (both give the same bits), or -1: the fp32 instruction, whose tiles are smaller, up to 64 rows, where
+// there are not tiles of 128 x 64 for three quarters of the compute units, and for short K.  One line in the rows for every weight, so that a row has the
 // same bits among any number of rows on its side of it.  Both measured, us (fp32 / split): 777 rows of 16,384 x 2,048 414 / 310, of 2,048 x 2,048 70 /
-// 55, of 2,048 x 8,192 229 / 182, of 3,072 x 2,048 87 / 77, 2,048 rows of 16,384 x 2,048 1,016 / 655, 300 of them 186 / 143; on the other side 65 of them 50 /
-// 55, 300 rows of 2,048 x 8,192 119 / 173, 777 of 1,536 x 512 19.6 / 20.0.
-constexpr int SPLIT_MIN_K = 512;
+// 55, of 2,048 x 8,192 229 / 182, of 3,072 x 2,048 87 / 77, 2,048 rows of 16,384 x 2,048 1,016 / 655, 300 of them 186 / 143, 65 rows of 128,256 x 2,048 381 /
+// 343; on the other side 65 rows of 16,384 x 2,048 44 / 50, 300 rows of 2,048 x 8,192 111 / 165, 777 of 1,536 x 512 14.4 / 15.4, 48 and 64 rows of 128,256 x
+// 2,048 248 and 307 / 355.  (Tiles of 32 or 64 rows and 64 columns do not move the line: 64 rows of 16,384 x 2,048 37 / 45, 300 of 2,048 x 8,192 111 / 160:
+// a stage has its waits whatever the tile.)
+constexpr int SPLIT_MIN_K = 512, SPLIT_MIN_M = 65;
 int split_tile(int M, int N, int K) {
   if (g_split_tile >= 0) return g_split_tile < SPLIT_COUNT ? g_split_tile : -1;
   const long cus = compute_units();
-  if (K < SPLIT_MIN_K || static_cast<long>(M) * N < cus * (128 * 64 * 3 / 4)) return -1;
+  if (M < SPLIT_MIN_M || K < SPLIT_MIN_K || static_cast<long>(M) * N < cus * (128 * 64 * 3 / 4)) return -1;
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < SPLIT_COUNT; ++i) {
@@ -841,6 +843,9 @@ KVF_EXPORT int kvf_gemm_generic_split_tile(int tile) {
   g_split_tile = tile;
   return before;
 }
+
+// Which tile of the split product M fp32 rows of [N, K] take, or -1.
+KVF_EXPORT int kvf_gemm_generic_split_takes(int M, int N, int K) { return split_tile(M, N, K); }
 
 // a_type / w_type: 0 = fp32, 1 = bf16.  out_mode: 0 = store in a_type... see table below.
 //   out_kind 0: store fp32      out_kind 1: store bf16      out_kind 2: add into fp32

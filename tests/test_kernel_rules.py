@@ -58,6 +58,14 @@ def test_products_of_many_rows_that_the_library_makes_as_fast_are_left_to_it(pai
     assert [size for size in own if not takes(*size, pairs)] == [] and [size for size in library_s if takes(*size, pairs)] == []
 
 
+@pytest.mark.parametrize("m,n,k,split", [(33, 128256, 2048, False), (64, 128256, 2048, False), (65, 128256, 2048, True), (64, 25016, 704, False),
+                                         (95, 16384, 2048, False), (96, 16384, 2048, True), (767, 2048, 8192, False), (768, 2048, 8192, True),
+                                         (768, 2048, 511, False), (768, 2048, 512, True), (33, 16, 64, False)])
+def test_32_bit_products_on_split_operands_take_enough_rows(m, n, k, split):
+    """Either side of every line of the rule: 64 rows, 6,144 outputs a compute unit (of 256), K of 512."""
+    assert (ctypes.CDLL(library.build_module("gemm_generic")).kvf_gemm_generic_split_takes(m, n, k) >= 0) == split
+
+
 @pytest.mark.parametrize("m,n,k,best", [(1434, 4096, 192, 1), (893, 6144, 128, 0), (1518, 3072, 64, 0), (1705, 6144, 512, 0), (1638, 5120, 256, 3),
                                         (2072, 1536, 64, 2), (343, 1536, 64, 5), (423, 5120, 128, 3)])
 def test_tiles_of_the_fused_projection_where_k_is_short(m, n, k, best):
