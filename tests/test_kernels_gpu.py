@@ -747,9 +747,16 @@ def _tile_case(m, n, k, seed):
     return a, w, rows, exact, slack
 
 
-# the smallest K that is taken and the next (ten and twelve stages), rows and columns on either side of a tile's end, and several tiles a
-# workgroup (a launch has at most as many workgroups as there are compute units, in eighths)
-TILE_SIZES = [(65, 64, 320), (129, 200, 384), (257, 328, 512), (66, 16 * 1030, 320), (700, 8 * 1200, 448), (2048, 4112, 320)]
+# the smallest K that is taken and the next (ten and twelve stages), rows and columns on either side of a tile's end, and, last, several
+# tiles a workgroup for every tile, unevenly (a launch has at most as many workgroups as fit the compute units, in eighths)
+TILE_SIZES = [(65, 64, 320), (129, 200, 384), (257, 328, 512), (66, 16 * 1030, 320), (700, 8 * 1200, 448), (2048, 4112, 320), (2047, 16 * 1101, 320)]
+
+
+def test_the_last_of_these_sizes_gives_every_tile_workgroups_of_several():
+    m, n, _ = TILE_SIZES[-1]
+    for bm, bn, at_once in ((256, 256, 1), (192, 256, 1), (128, 256, 1), (128, 128, 1), (64, 128, 1), (192, 128, 1), (256, 128, 1), (64, 64, 2)):
+        tiles, room = -(-m // bm) * -(-n // bn), ops().compute_units(DEV) * at_once
+        assert tiles > 2 * room and tiles % room and m % bm and n % bn
 
 
 @pytest.mark.parametrize("tile", [0, 1])
@@ -836,6 +843,45 @@ def test_fp32_products_of_small_by_large_operands(small_rows, small, tile):
     assert float((got - exact).norm()) <= float((fp32 - exact).norm()) + 2.0 ** -24 * float(exact.norm())
 
 
+@pytest.mark.parametrize("k", [512, 2048, 8192])
+def test_fp32_products_of_the_elements_that_leave_out_the_most(k):
+    """1 + 2^-8 - 2^-17 throughout: the products of parts that are left out come to 2^-24 of the result, all of one sign; a result is rounded by as much."""
+    a, w = (torch.full((rows, k), 1 + 2.0 ** -8 - 2.0 ** -17, device=DEV) for rows in (130, 68))
+    exact = a[:1].double() @ w[:1].double().T
+    for tile in (0, 1):
+        assert bool(((_fp32_product(tile, a, w).double() - exact).abs() <= 2 * 2.0 ** -24 * exact).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 36, 32), (129, 132, 96), (300, 260, 2048), (1000, 1000, 512)])
+def test_fp32_products_have_the_same_bits_on_either_tile(m, n, k):
+    """Which of the two a row takes depends on the rows beside it."""
+    g = torch.Generator().manual_seed(m)
+    a, w = torch.randn(m, k, generator=g).to(DEV), torch.randn(n, k, generator=g).to(DEV)
+    first = _fp32_product(0, a, w)
+    assert torch.equal(first, _fp32_product(1, a, w)) and not torch.equal(first, _fp32_product(2, a, w))
+    for rows in (slice(0, 33), slice(m - 33, m)):
+        assert torch.equal(_fp32_product(1, a[rows], w), first[rows])
+
+
+@pytest.mark.parametrize("n,k", [(2048, 512), (16384, 544)])
+def test_fp32_products_on_both_sides_of_the_lines_in_their_rows(n, k):
+    """A weight's products change from lanes side by side to the fp32 instruction behind 32 rows and to split operands behind 64 rows and
+    6,144 outputs a compute unit.  Among any rows on one side of a line a row has the same bits, on every side it lies as near to 64 bits as fp32 sums
+    do."""
+    line = max(65, -(-6144 * ops().compute_units(DEV) // n))
+    g = torch.Generator().manual_seed(n)
+    a, w = torch.randn(line + 40, k, generator=g).to(DEV), torch.randn(n, k, generator=g).to(DEV)
+    size = a[:32].double().abs() @ w.double().abs().T
+    exact, seen = a[:32].double() @ w.double().T, []
+    for rows, way in ((32, None), (33, 2), (line - 1, 2), (line, 0), (line + 40, 0)):
+        out = torch.empty(rows, n, device=DEV)
+        ops().gemm(a[:rows], w, out)
+        assert way is None or torch.equal(out, _fp32_product(way, a[:rows], w))
+        assert bool(((out[:32] - exact).abs() <= (k / 8 + 8) * 2.0 ** -24 * size).all())
+        seen.append(out[:32])
+    assert torch.equal(seen[1], seen[2]) and torch.equal(seen[3], seen[4]) and not torch.equal(seen[2], seen[3])
+
+
 @pytest.mark.parametrize("tile", range(7))
 @pytest.mark.parametrize("m,n,k", TILE_SIZES)
 def test_gemm_tiles(m, n, k, tile):
@@ -902,6 +948,52 @@ def test_products_of_many_rows_go_in_tiles_where_they_fit():
             ops().gemm_tiles(rows, other, into)
         ops().gemm(rows, other, into)
         assert not into.any()
+
+
+@pytest.mark.parametrize("m,n,k,own", [(128, 1024, 512, True), (70, 256, 320, True), (130, 1008, 512, True), (2048, 8192, 512, True),
+                                       (70, 512, 2048, False), (200, 1024, 2048, False), (128, 1020, 512, False), (128, 1024, 544, False),
+                                       (2048, 2048, 4096, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_products_of_many_rows_take_the_route_that_their_size_names(m, n, k, own, dtype):
+    """``gemm`` has the bits of the tiles or of the library's product, and either is as near to 64 bits as sums of ``k`` rounded terms are."""
+    a, w, rows, exact, slack = _tile_case(m, n, k, m + n + k)
+    assert ops().tiles_take(a, w, torch.empty(m, n, dtype=dtype, device=DEV)) == own
+    got, want = (torch.full((m, n), 7.0, dtype=dtype, device=DEV) for _ in range(2))
+    ops().gemm(a, w, got)
+    if own:
+        ops().gemm_tiles(a, w, want)
+    else:
+        ops()._library_product(a, w.plain, want, False, m, n, k, a.stride(0), n)
+    assert torch.equal(got[rows], want[rows])
+    assert bool(((got[rows].double() - exact).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * exact.abs() + slack).all())
+
+
+@pytest.mark.parametrize("m,inter,hidden,own", [(128, 512, 512, True), (70, 128, 320, True), (65, 512, 512, True), (64, 512, 512, False),
+                                                (70, 256, 2048, False), (128, 516, 512, False), (128, 512, 544, False)])
+@pytest.mark.parametrize("kind", ["swiglu", "limited", "gelu_tanh"])
+def test_gate_and_up_of_many_rows_take_the_route_that_their_size_names(monkeypatch, m, inter, hidden, own, kind):
+    """What a feed-forward hands to its down projection: joined in the product's kernel or behind the stored product, with the same bits."""
+    from kvforge_amd.engine.batch import Step, Workspace
+    from kvforge_amd.parts import feedforward
+    part = (feedforward.SwiGLU("m", hidden, inter) if kind == "swiglu" else
+            feedforward.GatedFeedForward("m", hidden, inter, activation=kind, limit=1.5 if kind == "limited" else None))
+    g = torch.Generator().manual_seed(m + inter)
+    w = {name: (torch.randn(spec.shape, generator=g) / hidden ** 0.5).to(torch.bfloat16).to(DEV) for name, spec in part.weight_specs().items()}
+    part.load(w)
+    part.seal()
+    x = torch.randn(m, hidden, generator=g).to(torch.bfloat16).to(DEV)
+    calls, real, take = [], ops().gemm_gated_tiles, ops().tiles_take
+    monkeypatch.setattr(ops(), "gemm_gated_tiles", lambda *a, **k: (calls.append(1), real(*a, **k)))
+    outs = []
+    for tiles in (True, False):
+        step, residual = Step(), torch.zeros(m, hidden, device=DEV)
+        step.ws, step.act_dtype = Workspace(DEV), torch.bfloat16
+        if not tiles:
+            monkeypatch.setattr(ops(), "tiles_take", lambda *a, pairs=False: not pairs and take(*a))
+        part.forward(x, step, residual)
+        step.settle()
+        outs.append(residual)
+    assert len(calls) == own and torch.equal(*outs)
 
 
 @pytest.mark.parametrize("n,k", [(3072, 2048), (6144, 4096), (1024, 512), (2048, 2048)])
