@@ -16,7 +16,7 @@ tokens.  A step is one decode step of the whole engine (scheduler, batch buildin
 sampling, bookkeeping).  One JSON line is printed; besides the decode figure it carries a
 2,048-token prefill, the decode step's share of the HBM roofline, and decode at batch 1 and 64.
 ``points`` also holds (unless ``--no-points``) the same model over contexts of 4,096 and 8,192
-tokens (decode at batch 8 and 64, one prompt of 8,192 tokens), the same model in true 32-bit (decode at batch 1
+tokens (decode at batch 8 and 64, one prompt of 8,192 tokens), the same model in 32 bits (decode at batch 1
 and 8, prefill of 2,048 tokens, with their shares of the fp32 bounds), the mixed workload at the
 Llama 3.2 3B shape (32 requests, prompts of 128 to 4,096 tokens, chunked prefill under a
 2,048-token budget beside decode steps, 256 new tokens each) and long-context decoding at the
@@ -33,8 +33,8 @@ what a Rudorax token uses.
 ``--phase ludelix`` measures the Ludelix design (gated linear attention, attention whose values
 are its keys, chunked attention beside a retention, experts chosen by a table) beside Rudorax,
 the closest existing model, at equal sizes.
-Peaks are the published MI355X ones: HBM 8 TB/s; dense MFMA 2.5 PFLOP/s for bf16, 157.3 TFLOP/s
-for fp32.
+Peaks are the published MI355X ones: HBM 8 TB/s; dense MFMA 2.5 PFLOP/s for bf16.  Large 32-bit products are six
+bf16 products of split operands, so their peak is a sixth of that (the fp32 instruction's is 157.3 TFLOP/s).
 """
 
 from __future__ import annotations
@@ -51,7 +51,7 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-MFMA_PEAK = {"bfloat16": 2.5e15, "float32": 157.3e12}
+MFMA_PEAK = {"bfloat16": 2.5e15, "float32": 2.5e15 / 6}
 CONTEXT_CAP = 8192
 BLOCK_SIZE = 16
 PREFILL_TOKENS = 2048
@@ -235,7 +235,7 @@ def prefill_flops(nums, n):
 
 
 def fp32_points(cfg, vocab, nums, steps=48, warmup=8):
-    """The 1B shape in true 32-bit, weights drawn and held in 32-bit on the device: decode at
+    """The 1B shape in 32 bits, weights drawn and held in 32-bit on the device: decode at
     batch 1 and 8, prefill of 2,048 tokens."""
     import torch
     out = {}

@@ -1,4 +1,4 @@
-// Paged attention of the true 32-bit path: every product and sum in fp32.  It takes bf16
+// Paged attention of the 32-bit path: every product and sum in fp32.  It takes bf16
 // operands as well (widened exactly), for caches whose pages the bf16 kernels do not take and for
 // heads of more than 256 elements (up to 640: one latent row of a wide latent attention).
 //

@@ -1,5 +1,5 @@
 // C[M, N] = A[M, K] * W[N, K]^T with fp32 multiply and fp32 accumulate.
-// This is the matrix product of the true 32-bit path and the fallback for operand types the
+// This is the matrix product of the 32-bit path and the fallback for operand types the
 // bf16 MFMA kernels do not take (for instance a weight that the checkpoint stores in fp32 while
 // activations are bf16).  Operands stored in bf16 are widened (exactly) before they are multiplied.
 //

@@ -3,8 +3,9 @@
 // rotary and the cache write in its epilogue (qkv_tile_kernel, RopeEpi).
 //
 // Sums run along K in steps of 32 on one accumulator, and are rounded to bf16 before they are rotated or joined, as a stored product
-// is.  The library's product does the same at most sizes, to the bit; it cuts K at some (14 of 306 that were compared, of 65 to 128 rows), where 3 in
-// 100,000 of the result turn a rounding.
+// is.  The library's product does the same at most sizes, to the bit; it cuts K at some, where 3 to 7 in 100,000 of the result turn a rounding: of 713 sizes of
+// plain and gated products that were compared, of 66 to 2,048 rows, at three (1,771 rows of 28,672 columns), of 306 of the fused projection at 14
+// (65 to 128 rows).
 #include <type_traits>
 
 #include "tile_walk.h"
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_tile_kernel(const bf16_t* 
   walk.template start<false>(lds, K / 32, src);
   char* own = lds + T::BYTES + walk.wave * OWN;
   const auto tile = [&](auto is_last, bool first) {
-    walk.template run<T::RT, decltype(is_last)::value>(K / 32, first, src);
+    walk.template run<decltype(is_last)::value>(K / 32, first, src);
     int row_tile, col_tile;
     place_of(item, tm, tn, row_tile, col_tile);
     store_tile<T, KIND>(walk, e, own, row_tile * T::BM, col_tile * T::BN, M, N);
@@ -218,8 +219,8 @@ __global__ __launch_bounds__(T::THREADS, 2) void qkv_tile_kernel(const bf16_t* _
     const bool has = pos[r] >= 0 && pos[r] < rp.table_len && page[r] >= 0 && page[r] < rp.n_seqs && blk < rp.table_stride;
     page[r] = has ? rp.block_table[static_cast<size_t>(page[r]) * rp.table_stride + blk] : -1;
   }
-  if constexpr (FEW) walk.template run_few<RT>(K / 32);
-  else walk.template run<RT, true>(K / 32, true, src);
+  if constexpr (FEW) walk.run_few(K / 32);
+  else walk.template run<true>(K / 32, true, src);
   const auto& acc = walk.acc;
   // The angles of the tile's tokens go through LDS, a cosine and a sine side by side: a lane would read them 4 bytes at
   // a time from 16 rows of the tables otherwise, for every head anew (10 of 42 us at 2,048 x 3,072).
@@ -442,7 +443,7 @@ double library_by_rounds(int M, int N, int K, int cus, bool pairs) {
 // measured it takes 721, in 0.63 of the time of the two, two of them more than 5% slower; of 1,002 of plain ones 470, in 0.71 of the
 // library's, four more than 5% slower.  (By the first alone it took 17 and 57 such, up to 36% slower: plain products of one round of 256 x 256, 2,048 rows
 // of 8,192 x 2,048 52 -> 67 us, and gated ones of large weights, 1,013 rows of 28,672 x 4,096 193 -> 214.)  Both measured, library / this in us.
-// Gated: 2,048 rows of 16,384 x 2,048 120 / 107, 512 41 / 34, 66 21 / 17; of 4,096 x 2,048 40 / 32.  Plain: 2,048 rows of 2,048 x 1,024
+// Gated: 2,048 rows of 16,384 x 2,048 120 / 115, 512 42 / 36, 66 20 / 17; of 4,096 x 2,048 38 / 32.  Plain: 2,048 rows of 2,048 x 1,024
 // 13.3 / 12.8, 320 of 3,072 x 2,048 13.1 / 11.6, of 1,024 x 512 8.8 / 6.8, 66 6.1 / 4.4.  The library's: 2,048 rows of 2,048 x 8,192 73 / 78, of
 // 6,144 x 4,096 80 / 93, gated ones of 28,672 x 4,096 377 / 391.
 // Above MOST the two take the same within some percent whichever is faster, and the library's is left alone.

@@ -1,4 +1,4 @@
-// Products of many rows in tiles: how a workgroup walks along K.  Shared by gemm_tile.hip and moe.hip.
+// Products of many rows in tiles: how a workgroup of gemm_tile.hip walks along K.
 //
 // A workgroup of WM x WN waves takes tiles of BM = 16 RT WM rows by BN = 16 CT WN columns (rows of a weight in the tiled form of
 // gemm_bf16.hip), 32 of K a stage.  Rows and weights go from memory straight into LDS without passing through
@@ -10,8 +10,8 @@
 //
 // A workgroup that takes several tiles does not stop between them: the loads run on into the next tile (Source says
 // where it lies) while the last stages of one are multiplied and while its results are stored, and the first stages of a tile do
-// not wait for the stores before them.  No load stands under a condition: behind the last tile its first stages are
-// asked for once more, for nobody.
+// not wait for the stores before them.  No load stands under a condition: the last stages of the last tile, behind which nothing is
+// asked for, are code of their own.
 //
 // What bounds it: 2,048 x 16,384 x 2,048 in tiles of 256 x 256 takes 107 us (1.28 PFLOP/s).  Its matrix instructions alone are 65 at the 2.0
 // GHz that the chip holds under them; with the loads left out it took 18 us less, with the reads of LDS left out 8, with
@@ -147,11 +147,10 @@ struct Walk {
     read_on(0);
   }
 
-  // Stage h of a tile, H its parity: the products of its first R row fragments, from f; the next stage's operands go to g (READ), and
-  // later ones are asked for (ASK).
-  template <int R, int H, bool READ, bool ASK>
+  // Stage h of a tile, H its parity: its products, from f; the next stage's operands go to g (READ), and later ones are asked for (ASK).
+  template <int H, bool READ, bool ASK>
   __device__ __forceinline__ void products(const Frags& f, Frags& g) {
-    constexpr int PR = R * CT, RD = READ ? RT + CT : 0, LOADS = !ASK ? 0 : H == 1 ? AL + WL : WL;
+    constexpr int PR = RT * CT, RD = READ ? RT + CT : 0, LOADS = !ASK ? 0 : H == 1 ? AL + WL : WL;
     __builtin_amdgcn_sched_barrier(0);
     int rd = 0, ld = 0;
 #pragma unroll
@@ -171,11 +170,11 @@ struct Walk {
     if (READ) read_on(1 - H);
   }
   // `arrived`: the next stage's operands are known to be in LDS (this wave's part of them).
-  template <int R, int H, bool LAST, class Source>
+  template <int H, bool LAST, class Source>
   __device__ __forceinline__ void stage(const Frags& f, Frags& g, bool arrived, Source& src) {
     if (arrived) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     else loads_left<in_flight(H == 1)>();
-    products<R, H, true, true>(f, g);
+    products<H, true, true>(f, g);
     if (H == 1) {
       rows_asked();
       if (!LAST && --left_a == 0) src.rows(*this);
@@ -184,13 +183,13 @@ struct Walk {
     if (!LAST && --left_w == 0) src.weights(*this);
   }
   // The last NW stages of the last tile, behind which nothing is asked for.
-  template <int R, int J>
+  template <int J>
   __device__ __forceinline__ void last_stages() {
     if constexpr (J < NW) {
       constexpr bool odd = J % 2 == 1, more = J + 1 < NW;
       if constexpr (more) loads_left<in_flight(odd, 64 + odd - 1 - J)>();
-      products<R, J % 2, more, false>(odd ? f1 : f0, odd ? f0 : f1);
-      last_stages<R, J + 1>();
+      products<J % 2, more, false>(odd ? f1 : f0, odd ? f0 : f1);
+      last_stages<J + 1>();
     }
   }
 
@@ -202,26 +201,26 @@ struct Walk {
   }
   // A tile: S stages, an even number of at least NW + 2.  LAST: no tile comes behind it (a constant: where both ways meet, registers
   // are copied or spilled).  `first`: nothing was stored since start().
-  template <int R, bool LAST, class Source>
+  template <bool LAST, class Source>
   __device__ __forceinline__ void run(int S, bool first, Source& src) {
     clear();
     const int arrived = first ? 0 : ARRIVED;   // settle() has seen them arrive
     const int asks = LAST ? S - NW : S;
 #pragma unroll 1
     for (int s = 0; s < asks; s += 2) {
-      stage<R, 0, LAST>(f0, f1, s < arrived, src);
-      stage<R, 1, LAST>(f1, f0, s + 1 < arrived, src);
+      stage<0, LAST>(f0, f1, s < arrived, src);
+      stage<1, LAST>(f1, f0, s + 1 < arrived, src);
     }
-    if constexpr (LAST) last_stages<R, 0>();
+    if constexpr (LAST) last_stages<0>();
     else settle();
   }
   // The only tile, of fewer stages, all of which have arrived (start<true>).
-  template <int R> __device__ __forceinline__ void run_few(int S) {
+  __device__ __forceinline__ void run_few(int S) {
     clear();
 #pragma unroll 1
     for (int s = 0; s < S; s += 2) {
-      products<R, 0, true, false>(f0, f1);
-      products<R, 1, true, false>(f1, f0);
+      products<0, true, false>(f0, f1);
+      products<1, true, false>(f1, f0);
     }
   }
 
@@ -230,11 +229,11 @@ struct Walk {
 };
 
 // A wave's own place in LDS where 16 rows of PIECES pieces of 16 bytes are turned from fragments into rows.  A row's
-// pieces are mixed by its number where they are a power of two, and the rows a piece longer where not, against bank conflicts.
+// pieces are mixed by its number against bank conflicts.
 template <int PIECES> struct OwnRows {
-  static constexpr bool POW2 = (PIECES & (PIECES - 1)) == 0;
-  static constexpr int PITCH = (POW2 ? PIECES : PIECES + 1) * 16, BYTES = 16 * PITCH;
-  __device__ __forceinline__ static int place(int row, int piece) { return row * PITCH + (POW2 ? piece ^ (row & (PIECES - 1)) : piece) * 16; }
+  static_assert((PIECES & (PIECES - 1)) == 0, "pieces are mixed by the bits of a row's number");
+  static constexpr int PITCH = PIECES * 16, BYTES = 16 * PITCH;
+  __device__ __forceinline__ static int place(int row, int piece) { return row * PITCH + (piece ^ (row & (PIECES - 1))) * 16; }
   // go(row, piece, its 16 bytes) for all of them, 64 at a time
   template <class Go> __device__ __forceinline__ static void each(const char* own, int lane, const Go& go) {
 #pragma unroll

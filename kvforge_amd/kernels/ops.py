@@ -1532,7 +1532,7 @@ def _gate_args(gate, q: torch.Tensor, cols: int):
 
 def attention_on_matrix_cores(dtype: torch.dtype, block_size: int, head_dim: int) -> bool:
     """The bf16 MFMA attention kernels take bf16, pages of a multiple of 8 tokens and heads of up to
-    256 elements; everything else (the true 32-bit path above all) runs the fp32 kernels."""
+    256 elements; everything else (the 32-bit path above all) runs the fp32 kernels."""
     return dtype == BF16 and block_size % 8 == 0 and head_dim <= 256
 
 
