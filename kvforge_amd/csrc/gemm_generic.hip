@@ -3,7 +3,7 @@
 // bf16 MFMA kernels do not take (for instance a weight that the checkpoint stores in fp32 while
 // activations are bf16).  Operands stored in bf16 are widened (exactly) before they are multiplied.
 //
-// Many rows of fp32 by fp32 where there are enough of them: the bf16 matrix cores over operands split without loss
+// Many rows of fp32 by fp32 where there are enough of them: the bf16 matrix cores over operands split in three
 // (gemm_split_kernel below), whose sums are nearer to 64 bits than those of fp32 instructions.
 // Many rows (a portion of a prompt) otherwise, rows of K that start on 16 bytes: tiles of 16 to 128 rows x 64
 // outputs on the matrix cores with v_mfma_f32_16x16x4_f32, which multiplies and adds in fp32
@@ -421,14 +421,17 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, RT * CT > 4 ? WM * WN / 4 : WM 
 #pragma unroll
     for (int i = 0; i < Q; ++i) f.v[i] = *reinterpret_cast<const float4*>(src[i] + k);
   };
-  float top[Q], top2[Q];                             // of the thread's elements of each row, the largest magnitude; in two chains: one is 1 to 5% slower
+  // of the thread's elements of each row, the largest magnitude; of A's in two chains (one: 1% slower at 777 rows of 16,384 x 2,048; two for both:
+  // a register too many for two workgroups a compute unit)
+  float top[Q], top2[AQ];
 #pragma unroll
-  for (int i = 0; i < Q; ++i) top[i] = top2[i] = 0.f;
+  for (int i = 0; i < Q; ++i) top[i] = top2[min(i, AQ - 1)] = 0.f;
   auto put = [&](const Staged& f, uint32_t buf) {
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
       top[i] = fmaxf(fmaxf(top[i], fabsf(f.v[i].x)), fabsf(f.v[i].y));
-      top2[i] = fmaxf(fmaxf(top2[i], fabsf(f.v[i].z)), fabsf(f.v[i].w));
+      float& other = i < AQ ? top2[min(i, AQ - 1)] : top[i];
+      other = fmaxf(fmaxf(other, fabsf(f.v[i].z)), fabsf(f.v[i].w));
       f32x2 x[2] = {{f.v[i].x, f.v[i].y}, {f.v[i].z, f.v[i].w}};
 #pragma unroll
       for (int part = 0; part < 3; ++part) {
@@ -498,7 +501,7 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, RT * CT > 4 ? WM * WN / 4 : WM 
   float* tops = reinterpret_cast<float*>(lds);       // nobody reads a stage any more
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
-    top[i] = fmaxf(top[i], top2[i]);
+    if (i < AQ) top[i] = fmaxf(top[i], top2[min(i, AQ - 1)]);
 #pragma unroll
     for (int o = 1; o < 8; o <<= 1) top[i] = fmaxf(top[i], __shfl_xor(top[i], o, KVF_WAVE));
     if (sq == 0) tops[srow + PASS * i] = top[i];
@@ -507,17 +510,16 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, RT * CT > 4 ? WM * WN / 4 : WM 
   // What the parts cannot hold of an element is less than 3 * 2^-126, and so is what a product of parts loses: results below 2^24 of the sum of
   // these are in doubt.  (A row or column of zeros loses nothing.)
   const float least = 0x1p-100f * K;
-  f32x4 col[CT];
-  float row[RT], most = 1.f, lowest = INFINITY, all = 0.f;
+  const float *row_tops = tops + 16 * wm * RT + r16, *col_tops = tops + TM_ + 16 * wn * CT + 4 * kg;
+  float most = 1.f, lowest = INFINITY, all = 0.f;
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
-    col[c] = *reinterpret_cast<const f32x4*>(tops + TM_ + 16 * (wn * CT + c) + 4 * kg);
-    most = fmaxf(fmaxf(fmaxf(most, col[c][0]), col[c][1]), fmaxf(col[c][2], col[c][3]));
+    const f32x4 col = *reinterpret_cast<const f32x4*>(col_tops + 16 * c);
+    most = fmaxf(fmaxf(fmaxf(most, col[0]), col[1]), fmaxf(col[2], col[3]));
   }
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    row[r] = tops[16 * (wm * RT + r) + r16];
-    most = fmaxf(most, row[r]);
+    most = fmaxf(most, row_tops[16 * r]);
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
       big[r][c] += small[r][c];
@@ -538,7 +540,8 @@ __global__ __launch_bounds__(WM * WN * KVF_WAVE, RT * CT > 4 ? WM * WN / 4 : WM 
       for (int c = 0; c < CT; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float v = fabsf(big[r][c][e]), lost = row[r] > 0.f && col[c][e] > 0.f ? least * (row[r] + col[c][e] + 1.f) : 0.f;
+          const float v = fabsf(big[r][c][e]), row = row_tops[16 * r], col = col_tops[16 * c + e];
+          const float lost = row > 0.f && col > 0.f ? least * (row + col + 1.f) : 0.f;
           doubt |= static_cast<uint32_t>(!(v <= 3.402823466e38f) || v < lost) << ((r * CT + c) * 4 + e);
         }
   }
