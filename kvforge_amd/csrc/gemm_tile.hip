@@ -425,7 +425,7 @@ double library_by_work(int M, int N, int K, bool pairs) {
   return 5.5 + 1.34e-3 * K + 0.25e-6 * N * K + 1.28e-3 * mn * K + 0.4 * mn + (pairs ? 1.0 + 0.6 * mn : 0.0);
 }
 // By the rounds of its tiles over the chip, which the first does not see: 2,048 rows of 8,192 x 4,096 are one round of 256 x 256.  Fitted to
-// 1,750 times of 66 to 8,192 rows, 512 to 33,000 columns, K of 320 to 14,336: within 11% in the mean.
+// 2,113 times of 66 to 8,192 rows, 512 to 33,000 columns, K of 320 to 14,336: within 11% in the mean.
 double library_by_rounds(int M, int N, int K, int cus, bool pairs) {
   constexpr int tiles[][2] = {{256, 256}, {256, 128}, {128, 128}, {64, 64}};
   const double k = K / 2048.0;
